@@ -11,7 +11,8 @@
 #include "fe_internal.h"
 
 namespace {
-constexpr uint32_t kGemmLds = 2 * (256 + 256) * 64 * 2;  // GM_LDS_TILES
+constexpr uint32_t kGemmLds = 160 * 1024;                // two k tiles of A and three of W, 256 rows each
+constexpr uint32_t kGemmThreads = 512;
 constexpr uint32_t kTileM = 256, kTileN = 256;           // GM_BM, GM_BN
 constexpr uint32_t kGemvRows = 8;                        // rows of one GEMV pass (model.rs:326)
 constexpr uint32_t kSmallBatch = 16;                     // X3_ROWS: batches up to here are decode rows (model.rs:172)
@@ -141,7 +142,7 @@ int fe_bf16_gemm(const fe_bf16_kernels *kern, fe_stream_t s, fe_devptr_t y, uint
     uint32_t full = gs.full, splits = gs.splits;
     fe_devptr_t part = kern->part.p;
     void *args[] = {&y, &x, &w, &res, &m, &n, &k, &lda, &ldy, &group, &full, &splits, &part};
-    FE_TRY(fe_hip_launch(kern->gemm, gs.programs(), 1, 1, 256, 1, 1, kGemmLds, s, args));
+    FE_TRY(fe_hip_launch(kern->gemm, gs.programs(), 1, 1, kGemmThreads, 1, 1, kGemmLds, s, args));
     if (!gs.cut()) return 0;
     void *rargs[] = {&y, &part, &res, &m, &n, &ldy, &group, &full, &splits};
     return fe_hip_launch(kern->reduce, gs.cut() * 64, 1, 1, 256, 1, 1, 0, s, rargs);
@@ -175,7 +176,7 @@ int fe_bf16_gemm_swiglu(const fe_bf16_kernels *kern, fe_stream_t s, fe_devptr_t 
     uint32_t full = gs.full, splits = gs.splits;
     fe_devptr_t part = kern->part.p;
     void *args[] = {&act, &x, &w, &m, &n, &k, &lda, &group, &full, &splits, &part};
-    FE_TRY(fe_hip_launch(kern->swiglu, gs.programs(), 1, 1, 256, 1, 1, kGemmLds, s, args));
+    FE_TRY(fe_hip_launch(kern->swiglu, gs.programs(), 1, 1, kGemmThreads, 1, 1, kGemmLds, s, args));
     if (!gs.cut()) return 0;
     void *rargs[] = {&act, &part, &m, &n, &group, &full, &splits};
     return fe_hip_launch(kern->swiglu_reduce, gs.cut() * 64, 1, 1, 256, 1, 1, 0, s, rargs);

@@ -1,0 +1,250 @@
+// MFMA GEMM core for prefill-sized M: C[BM x BN tile] = A[M][K] (16-bit, row-major, from global) times a weight tile W[N][K].
+//
+// 512 threads = 8 wavefronts, two a SIMD, in a WM x WN grid; a wavefront owns 16 TM rows x 16 TN columns as TM x TN
+// v_mfma_f32_16x16x32 accumulators (128 registers a lane at 256 x 256). Both operands go from global memory straight into
+// LDS (buffer_load ... lds, 16 bytes a lane): no staging registers and no LDS write instructions, which cost the LDS pipe
+// about 17 cycles a kilobyte where the direct path costs 8. The loads of a k tile are spread evenly over the tile's MFMAs:
+// the address unit takes 16 cycles for each, and a burst of them holds the wavefront's next MFMA back.
+//
+// What the tile loop is bound by is the board's power: the matrix pipe is busy 81 % of the time and the clock settles where
+// the power limit puts it (1.75..1.95 GHz on random operands). So the choices are those that take the least energy a flop:
+// the 16x16x32 instruction (half the accumulator traffic a flop of 32x32x16: at the same schedule 98 against 104 us for
+// 4096^3), every operand byte once through LDS. 2048 x 16384 x 5120 bf16: 225 us (1526 TFLOP/s) against 266 us for four
+// wavefronts of 128 x 128 with 32x32x16 and operands staged through registers.
+//
+// LDS: NA stages of A (BM rows of 128 bytes) and NW stages of the weight operand; the loads run NA - 1 and NW - 1 k tiles
+// ahead. A row of 128 bytes is 8 chunks of 16; chunk c of row r lies at position perm(c) ^ (r & 7). A fragment read takes
+// row lane & 15, one chunk per group of 16 lanes; a 16-byte read serves the lanes {0-3, 12-15, 20-27} or {4-11, 16-19,
+// 28-31} of a half wavefront in a cycle (64 banks), and those 16 need 16 different (r & 1, position) pairs: with neighbouring
+// chunks in neighbouring lane groups (perm = identity) the XOR gives them; where lane group g takes chunks 2 g and 2 g + 1
+// (weights expanded from packed codes, 16 codes a lane), perm swaps the two low bits of c.
+#pragma once
+#include "gemm_core.h"
+
+#define G8_BK 64
+
+template <int WM_, int WN_, int TM_, int TN_>
+struct G8Tile {
+    static constexpr int WM = WM_, WN = WN_, TM = TM_, TN = TN_, NW = WM * WN, THREADS = 64 * NW;
+    static constexpr int BM = 16 * TM * WM, BN = 16 * TN * WN;
+    static constexpr int PART_FLOATS = BM * BN;
+    static_assert(NW == 8, "eight wavefronts");
+};
+
+// One wavefront moves 64 x 16 (4) bytes, lane l's from rs + voff + soff to LDS byte dst + 16 (4) l; dst and soff are uniform.
+// Not counted by the compiler's own waits: callers wait with g8_loads_wait.
+__device__ __forceinline__ void g8_load_lds16(u32x4 rs, uint32_t dst, uint32_t voff, uint32_t soff) {
+    asm volatile("s_mov_b32 m0, %0\n\ts_nop 0\n\tbuffer_load_dwordx4 %1, %2, %3 offen lds" ::"s"(__builtin_amdgcn_readfirstlane(dst)), "v"(voff), "s"(rs),
+                 "s"(__builtin_amdgcn_readfirstlane(soff))
+                 : "memory");
+}
+__device__ __forceinline__ void g8_load_lds4(u32x4 rs, uint32_t dst, uint32_t voff, uint32_t soff) {
+    asm volatile("s_mov_b32 m0, %0\n\ts_nop 0\n\tbuffer_load_dword %1, %2, %3 offen lds" ::"s"(__builtin_amdgcn_readfirstlane(dst)), "v"(voff), "s"(rs),
+                 "s"(__builtin_amdgcn_readfirstlane(soff))
+                 : "memory");
+}
+// All but the N youngest of the wavefront's vector memory operations are done, and its LDS operations are.
+template <int N>
+__device__ __forceinline__ void g8_loads_wait() {
+    asm volatile("s_waitcnt vmcnt(%0) lgkmcnt(0)" ::"n"(N) : "memory");
+}
+// Workgroup barrier without the compiler's wait for every load in flight.
+__device__ __forceinline__ void g8_barrier() {
+    __builtin_amdgcn_s_barrier();
+    asm volatile("" ::: "memory");
+}
+__device__ __forceinline__ u32x4 g8_rsrc(const void* p, uint32_t bytes) {
+    const uint64_t a = (uint64_t)p;
+    return (u32x4){(uint32_t)a, (uint32_t)(a >> 32) & 0xffffu, bytes, 0x00020000u};
+}
+__device__ __forceinline__ uint32_t g8_lds_addr(const void* p) {
+    return (uint32_t)(uintptr_t)(const __attribute__((address_space(3))) void*)p;
+}
+// chunk position <-> chunk (its own inverse): identity, or the two low bits swapped
+template <bool PERM>
+__device__ __forceinline__ constexpr uint32_t g8_perm(uint32_t c) {
+    return PERM ? (c & 4) | ((c & 1) << 1) | ((c >> 1) & 1) : c;
+}
+
+// Weight operand already in 16-bit form: rows of 64 values a k tile. voff[j]: byte offset of the lane's 16-byte piece j (row
+// 8 (wave + 8 j) + lane / 8, position lane & 7) at k tile 0; k tiles are kstep bytes apart. (dense_setup_rows / _image.)
+template <class T>
+struct G8Dense {
+    static constexpr bool kRaw = false, kPerm = false;
+    static constexpr int STAGE = T::BN * 128, LOADS = T::BN / 64;
+    u32x4 rs;
+    uint32_t voff[LOADS], kstep;
+    // row-major weights [n][k]: rows past n repeat row n - 1 (their columns are never stored)
+    __device__ __forceinline__ void rows(const void* w, uint32_t n, uint32_t k, uint32_t n0) {
+        const uint32_t lane = threadIdx.x & 63, wave = threadIdx.x >> 6;
+        rs = g8_rsrc(w, n * k * 2);
+        kstep = 128;
+#pragma unroll
+        for (int j = 0; j < LOADS; j++) {
+            const uint32_t r = 8 * (wave + 8 * j) + (lane >> 3), g = n0 + r < n ? n0 + r : n - 1;
+            voff[j] = (g * k + ((lane & 7) ^ (r & 7)) * 8) * 2;
+        }
+    }
+    __device__ __forceinline__ void issue(uint32_t kt, uint32_t dst, int j) const { g8_load_lds16(rs, dst + j * 8192, voff[j], kt * kstep); }
+};
+
+// acc[i][j]: weight rows (output columns) 16 (wn TN + j) + 4 (lane >> 4) + e, activation row 16 (wm TM + i) + (lane & 15).
+// k tiles kt0 .. kt0 + ktiles - 1. a: 16-bit values [m][lda]; rows past m repeat row m - 1. lds: the start of the dynamic LDS.
+//
+// One k tile is two slices of 32 k. A slice walks the TN columns of fragments (outer), TM MFMAs each; the outer fragment's
+// register is refilled for the next slice as soon as its MFMAs are issued, the TM inner fragments are double-buffered. The
+// barrier sits between the slices: by then every wavefront has this tile's fragments in registers (this tile's LDS stages
+// are free for the k tiles NA / NW ahead) and the loads of tile kt + 1 have been waited for. Slice 0 issues the weight loads,
+// slice 1 those of A.
+template <class T, int NA, int NW, bool BF16, class W>
+__device__ __forceinline__ void g8_mainloop(const void* a, uint32_t lda, uint32_t m, uint32_t kt0, uint32_t ktiles, uint32_t m0,
+                                            const W& wo, unsigned char* lds, f32x4 (&acc)[T::TM][T::TN]) {
+    constexpr int TM = T::TM, TN = T::TN, LA = T::BM / 64, LB = W::LOADS, A_STAGE = T::BM * 128, W_AT = NA * A_STAGE;
+    static_assert(NW == NA || NW == NA + 1, "the waits below");
+    static_assert(W_AT + NW * W::STAGE <= 160 * 1024, "LDS");
+    const uint32_t lane = threadIdx.x & 63, wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
+    const uint32_t wm = wave / T::WN, wn = wave % T::WN;
+    const u32x4 ra = g8_rsrc(a, m * lda * 2);
+    uint32_t va[LA];
+#pragma unroll
+    for (int j = 0; j < LA; j++) {
+        const uint32_t r = 8 * (wave + 8 * j) + (lane >> 3), g = m0 + r < m ? m0 + r : m - 1;
+        va[j] = (g * lda + (g8_perm<W::kPerm>((lane & 7) ^ (r & 7))) * 8) * 2;
+    }
+    const uint32_t base = g8_lds_addr(lds) + wave * 1024;
+    auto ktc = [&](uint32_t kt) { return kt0 + (kt < ktiles ? kt : ktiles - 1); };  // past the end: the last tile again, never used
+    auto load_a = [&](uint32_t kt, uint32_t st, int j) { g8_load_lds16(ra, base + st * A_STAGE + j * 8192, va[j], ktc(kt) * 128); };
+    auto load_w = [&](uint32_t kt, uint32_t st, int j) { wo.issue(ktc(kt), base + W_AT + st * W::STAGE, j); };
+    auto next = [](uint32_t st, uint32_t n) { return st + 1 == n ? 0u : st + 1; };
+
+    const uint32_t fr = lane & 15, fc = lane >> 4;
+    uint32_t foff[2];
+#pragma unroll
+    for (int kk = 0; kk < 2; kk++) foff[kk] = fr * 128 + (((4 * kk + fc) ^ (fr & 7)) << 4);
+    const unsigned char* pa = lds + wm * TM * 2048;
+    const unsigned char* pw = lds + W_AT + wn * TN * 2048;
+    f16x8 fa[2][TM], fw[TN];
+    auto rd_a = [&](int set, uint32_t st, int kk, int i) { fa[set][i] = *(const f16x8*)(pa + st * A_STAGE + 2048 * i + foff[kk]); };
+    auto rd_w = [&](uint32_t st, int kk, int j) { fw[j] = *(const f16x8*)(pw + st * W::STAGE + 2048 * j + foff[kk]); };
+    auto mfma = [&](int set, int i, int j) {
+        if constexpr (BF16)
+            acc[i][j] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(__builtin_bit_cast(bf16x8, fw[j]), __builtin_bit_cast(bf16x8, fa[set][i]),
+                                                                 acc[i][j], 0, 0, 0);
+        else
+            acc[i][j] = __builtin_amdgcn_mfma_f32_16x16x32_f16(fw[j], fa[set][i], acc[i][j], 0, 0, 0);
+    };
+#pragma unroll
+    for (int i = 0; i < TM; i++)
+#pragma unroll
+        for (int j = 0; j < TN; j++) acc[i][j] = (f32x4){0.f, 0.f, 0.f, 0.f};
+
+    // prologue: the loads in the order of the loop's own ([W of a slice 0, A of a slice 1] a tile), up to A of tile NA - 1
+#pragma unroll
+    for (int t = 0; t < NA; t++) {
+        if (NW - 1 - NA + t >= 0) {
+#pragma unroll
+            for (int j = 0; j < LB; j++) load_w(NW - 1 - NA + t, NW - 1 - NA + t, j);
+        }
+#pragma unroll
+        for (int j = 0; j < LA; j++) load_a(t, t, j);
+    }
+    g8_loads_wait<(NW > NA ? (NA - 1) * (LA + LB) : (NA - 1) * LA + (NA > 1 ? (NA - 2) * LB : 0))>();
+    g8_barrier();
+#pragma unroll
+    for (int i = 0; i < TM; i++) rd_a(0, 0, 0, i);
+#pragma unroll
+    for (int j = 0; j < TN; j++) rd_w(0, 0, j);
+
+    uint32_t sa = 0, sw = 0, sw_in = NW - 1;  // stages of tile kt; the weight stage that slice 0 of tile kt fills
+    for (uint32_t kt = 0; kt < ktiles; kt++) {
+        const uint32_t sa1 = next(sa, NA), sw1 = next(sw, NW);
+#pragma unroll
+        for (int kk = 0; kk < 2; kk++) {
+            if (kk == 1) {
+                g8_loads_wait<(NW > NA ? (NA - 1) * LB + (NA - 2) * LA : (NA - 2) * (LA + LB))>();
+                g8_barrier();
+            }
+            const uint32_t ra_st = kk ? sa1 : sa, rw_st = kk ? sw1 : sw;
+#pragma unroll
+            for (int j = 0; j < TN; j++) {
+#pragma unroll
+                for (int i = 0; i < TM; i++) mfma(kk, j & 1 ? TM - 1 - i : i, j);
+                rd_w(rw_st, kk ^ 1, j);
+                // the inner fragments of the next slice: in the first rows, TM of them
+                constexpr int PER = (2 * TM + TN - 1) / TN;
+#pragma unroll
+                for (int q = 0; q < PER; q++)
+                    if (j * PER + q < TM) rd_a(kk ^ 1, ra_st, kk ^ 1, j * PER + q);
+                const int n = kk ? LA : LB;
+#pragma unroll
+                for (int q = j * n / TN; q < (j + 1) * n / TN; q++) {
+                    if (kk == 0)
+                        load_w(kt + NW - 1, sw_in, q);
+                    else
+                        load_a(kt + NA, sa, q);
+                }
+                __builtin_amdgcn_sched_barrier(0);
+            }
+        }
+        sa = sa1, sw_in = sw, sw = sw1;
+    }
+    asm volatile("s_waitcnt vmcnt(0)" ::: "memory");
+    __syncthreads();  // the stages are free for the epilogue
+}
+
+// Hands the wavefront's accumulators out row by row: 16 rows at a time pass through the wavefront's own LDS slab so that
+// LPR = 4 TN consecutive lanes hold the wavefront's 16 TN columns of one row, 4 a lane. U passes of 64 / LPR rows are in
+// flight together: transform(v[U][4], lane in row) works on all of them at once (no branches), then
+// store(row in 0 .. 16 TM - 1, lane in row, v[4]) is called for each. No workgroup barrier: a slab belongs to its wavefront.
+template <class T, class Transform, class Store>
+__device__ __forceinline__ void g8_epilogue(f32x4 (&acc)[T::TM][T::TN], unsigned char* lds, Transform transform, Store store) {
+    constexpr int LPR = 4 * T::TN, RP = 64 / LPR, PITCH = 16 * T::TN + 4, U = 16 / RP < 4 ? 16 / RP : 4;
+    const uint32_t lane = threadIdx.x & 63, wave = threadIdx.x >> 6, fr = lane & 15, fc = lane >> 4;
+    float* slab = (float*)(lds + wave * (16 * PITCH * 4));
+    const uint32_t lr = lane / LPR, lc = lane % LPR;
+#pragma unroll
+    for (int i = 0; i < T::TM; i++) {
+#pragma unroll
+        for (int j = 0; j < T::TN; j++) *(f32x4*)(slab + fr * PITCH + 16 * j + 4 * fc) = acc[i][j];
+        gm_slab_sync();
+#pragma unroll
+        for (int r0 = 0; r0 < 16; r0 += RP * U) {
+            float v[U][4];
+#pragma unroll
+            for (int u = 0; u < U; u++) {
+                const f32x4 t = *(const f32x4*)(slab + (r0 + RP * u + lr) * PITCH + 4 * lc);
+                v[u][0] = t[0], v[u][1] = t[1], v[u][2] = t[2], v[u][3] = t[3];
+            }
+            transform(v, lc);
+#pragma unroll
+            for (int u = 0; u < U; u++) store(16 * i + r0 + RP * u + lr, lc, v[u]);
+        }
+        gm_slab_sync();
+    }
+}
+
+// A program's accumulators in its partial slot, as the lanes hold them: piece (i, j) of thread t at ((i TN + j) 512 + t) 16.
+template <class T>
+__device__ __forceinline__ void g8_store_partial(f32x4 (&acc)[T::TM][T::TN], float* slot) {
+#pragma unroll
+    for (int i = 0; i < T::TM; i++)
+#pragma unroll
+        for (int j = 0; j < T::TN; j++) *(f32x4*)(slot + ((i * T::TN + j) * T::THREADS + threadIdx.x) * 4) = acc[i][j];
+}
+
+// Body of a reduce kernel: grid = cut tiles * (BM / 8) * (BN / 128), 256 threads. Each half wavefront sums the `splits` slots
+// of one row of one 128-column block of a tile, 4 columns a lane, in split order, and hands them to fn(t, row in 0 .. BM - 1,
+// column block, l32, v[4]) with t the tile's index among the cut tiles. The 8 rows of a block are neighbours in the slots.
+template <class T, class RowFn>
+__device__ __forceinline__ void g8_reduce_rows(const float* __restrict__ part, uint32_t splits, RowFn fn) {
+    constexpr uint32_t CB = T::BN / 128, PER_TILE = T::BM / 8 * CB;
+    const uint32_t t = blockIdx.x / PER_TILE, b = blockIdx.x % PER_TILE, l32 = threadIdx.x & 31;
+    const uint32_t row = (b / CB) * 8 + (threadIdx.x >> 5), cb = b % CB;
+    const uint32_t c4 = cb * 32 + l32, wn = c4 / (4 * T::TN), j = (c4 / 4) % T::TN, fc = c4 % 4;
+    const uint32_t wm = row / (16 * T::TM), i = (row / 16) % T::TM, fr = row % 16;
+    const float* p = part + (size_t)t * splits * T::PART_FLOATS + ((i * T::TN + j) * T::THREADS + (wm * T::WN + wn) * 64 + fc * 16 + fr) * 4;
+    f32x4 sum = *(const f32x4*)p;
+    for (uint32_t sp = 1; sp < splits; sp++) sum += *(const f32x4*)(p + (size_t)sp * T::PART_FLOATS);
+    float v[4] = {sum[0], sum[1], sum[2], sum[3]};
+    fn(t, row, cb, l32, v);
+}

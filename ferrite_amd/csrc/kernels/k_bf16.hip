@@ -1,6 +1,6 @@
 // The plain bf16 weight form of the caller's linear: y[M][N] = x[M][K] . W[N][K]^T (+ residual), W row-major bf16, f32
 // sums, bf16 out. A GEMM on the shared 256 x 256 MFMA tile loop and two decode-sized GEMVs (kernels/k-core/src/gemm.rs).
-#include "gemm_core.h"
+#include "gemm8.h"
 
 // 4 sums of columns at.. of one row -> bf16; with res: bf16(bf16(sum) + res) (gemm.rs:152-158).
 __device__ __forceinline__ void bf16_store4(uint16_t* c, const uint16_t* res, size_t at, const float (&v)[4]) {
@@ -17,83 +17,53 @@ __device__ __forceinline__ void bf16_store4(uint16_t* c, const uint16_t* res, si
 
 // ---- GEMM ------------------------------------------------------------------------------------------------------------
 
-// A weight k tile is already what the LDS tile holds: thread t copies 16-byte chunk t & 7 of rows (t >> 3) + 32 j of each
-// 128-row half. Rows past n re-read row n - 1 (their columns are never stored).
-struct Bf16Producer {
-    const unsigned char* w;
-    uint32_t off[2][4];  // byte offset of row (t >> 3) + 32 j of half b, chunk t & 7, k tile 0
-    uint32_t st;
-    struct Raw {
-        u32x4 c[2][4];
-    };
-    static constexpr int kStoreValu = 0;
-    static constexpr bool kQuarters = false;
-    __device__ __forceinline__ void load(uint32_t kt, Raw& r, int half) const {
-#pragma unroll
-        for (int b = 0; b < 2; b++) {
-            if (b != half) continue;
-            const unsigned char* p = w + (size_t)kt * (GM_BK * 2);
-#pragma unroll
-            for (int j = 0; j < 4; j++) r.c[b][j] = *(const u32x4*)(p + off[b][j]);
-        }
+typedef G8Tile<4, 2, 4, 8> Bf16Tile;  // 256 x 256
+#define BF16_GEMM_STAGES 2, 3         // k tiles of A and of W in LDS: all 160 KB
+
+// One program's share of A . W^T: main loop, then the partial slot (a tile cut along K) or done(row, col, v[4]) for every
+// row piece of the tile, all lanes of a row calling (row >= m and col >= n included).
+template <class T, class Done>
+__device__ __forceinline__ void bf16_gemm_program(const uint16_t* a, const uint16_t* w, uint32_t m, uint32_t n, uint32_t k, uint32_t lda,
+                                                  uint32_t group_m, uint32_t full_tiles, uint32_t splits, float* part, Done done) {
+    extern __shared__ __attribute__((aligned(1024))) unsigned char lds[];
+    const uint32_t wave = threadIdx.x >> 6, wm = wave / T::WN, wn = wave % T::WN;
+    const GemmWork wk = gemm_work(blockIdx.x, (m + T::BM - 1) / T::BM, (n + T::BN - 1) / T::BN, group_m, k / G8_BK, full_tiles, splits);
+    G8Dense<T> wo;
+    wo.rows(w, n, k, wk.tn * T::BN);
+    f32x4 acc[T::TM][T::TN];
+    g8_mainloop<T, BF16_GEMM_STAGES, true>(a, lda, m, wk.kt0, wk.ktn, wk.tm * T::BM, wo, lds, acc);
+    if (wk.partial) {
+        g8_store_partial<T>(acc, part + (size_t)wk.slot * T::PART_FLOATS);
+        return;
     }
-    __device__ __forceinline__ void store(const Raw& r, unsigned char* Bs, int part) const {
-#pragma unroll
-        for (int b = 0; b < 2; b++) {
-            if (b != part) continue;
-#pragma unroll
-            for (int j = 0; j < 4; j++) *(u32x4*)(Bs + 16384 * b + st + 4096 * j) = r.c[b][j];
-        }
-    }
-};
+    const uint32_t m0 = wk.tm * T::BM + wm * 16 * T::TM, n0 = wk.tn * T::BN + wn * 16 * T::TN;
+    g8_epilogue<T>(
+        acc, lds, [](auto&, uint32_t) {}, [&](uint32_t row, uint32_t lc, float (&v)[4]) { done(m0 + row, n0 + 4 * lc, lc, v); });
+}
 
 // C[M][ldc] = bf16(A . W^T) (+ res); A bf16 [M][lda], W bf16 [N][K]. grid full_tiles + (tiles - full_tiles) * splits with
-// tiles = ceil(M / 256) * ceil(N / 256), 256 threads, dynamic LDS GM_LDS_TILES; tiles past full_tiles leave partials in
+// tiles = ceil(M / 256) * ceil(N / 256), 512 threads, dynamic LDS 160 KB; tiles past full_tiles leave partials in
 // `part` for fe_gemm_bf16_reduce. K % 64 == 0, N % 8 == 0, lda % 8 == 0, ldc % 4 == 0, operands under 4 GB.
 // (kernels/k-core/src/gemm.rs:128-167: fe_gemm_bf16, tile 128 x 128 x 32 on mma.m16n8k16 there)
-extern "C" __global__ __launch_bounds__(256, 1) void fe_gemm_bf16(uint16_t* c, const uint16_t* a, const uint16_t* w,
+extern "C" __global__ __launch_bounds__(512, 2) void fe_gemm_bf16(uint16_t* c, const uint16_t* a, const uint16_t* w,
                                                                   const uint16_t* res, uint32_t m, uint32_t n, uint32_t k,
                                                                   uint32_t lda, uint32_t ldc, uint32_t group_m,
                                                                   uint32_t full_tiles, uint32_t splits, float* part) {
-    extern __shared__ __attribute__((aligned(16))) unsigned char lds[];
-    const uint32_t tid = threadIdx.x, wave = tid >> 6, wm = wave >> 1, wn = wave & 1;
-    const GemmWork wk = gemm_work(blockIdx.x, (m + GM_BM - 1) / GM_BM, (n + GM_BN - 1) / GM_BN, group_m, k / GM_BK, full_tiles, splits);
-    const uint32_t m0 = wk.tm * GM_BM, n0 = wk.tn * GM_BN;
-    Bf16Producer prod;
-    const uint32_t chunk = tid & 7, row = tid >> 3;
-    prod.w = (const unsigned char*)w;
-#pragma unroll
-    for (int b = 0; b < 2; b++)
-#pragma unroll
-        for (int j = 0; j < 4; j++) {
-            uint32_t r = n0 + 128 * b + row + 32 * j;
-            r = r < n ? r : n - 1;
-            prod.off[b][j] = (r * k + chunk * 8) * 2;
-        }
-    prod.st = gm_swz(row, chunk);
-    f32x16 acc[4][4];
-    gemm_mainloop<Bf16Producer, true>((const _Float16*)a, lda, m, wk.kt0, wk.ktn, m0, prod, lds, acc);
-    if (wk.partial) {
-        gemm_store_partial(acc, lds, part + (size_t)wk.slot * GM_PART_FLOATS);
-        return;
-    }
-    const uint32_t col = n0 + wn * 128 + 4 * (tid & 31);
-    gemm_epilogue(
-        acc, lds, [](float (&)[4][4], uint32_t) {},
-        [&](uint32_t r, uint32_t, float (&v)[4]) {
-            const uint32_t grow = m0 + wm * 128 + r;
-            if (grow < m && col < n) bf16_store4(c, res, (size_t)grow * ldc + col, v);
-        });
+    bf16_gemm_program<Bf16Tile>(a, w, m, n, k, lda, group_m, full_tiles, splits, part,
+                                [&](uint32_t row, uint32_t col, uint32_t, float (&v)[4]) {
+                                    if (row < m && col < n) bf16_store4(c, res, (size_t)row * ldc + col, v);
+                                });
 }
 
 // Finishes the tiles fe_gemm_bf16 cut along K. grid (tiles - full_tiles) * 64, 256 threads.
 extern "C" __global__ __launch_bounds__(256) void fe_gemm_bf16_reduce(uint16_t* c, const float* part, const uint16_t* res,
                                                                       uint32_t m, uint32_t n, uint32_t ldc, uint32_t group_m,
                                                                       uint32_t full_tiles, uint32_t splits) {
-    gemm_reduce_rows(part, splits, [&](uint32_t t, uint32_t row, uint32_t cb, uint32_t l32, float (&v)[4]) {
+    typedef Bf16Tile T;
+    g8_reduce_rows<T>(part, splits, [&](uint32_t t, uint32_t row, uint32_t cb, uint32_t l32, float (&v)[4]) {
         uint32_t tm, tn;
-        gemm_raster(full_tiles + t, (m + GM_BM - 1) / GM_BM, (n + GM_BN - 1) / GM_BN, group_m, tm, tn);
-        const uint32_t grow = tm * GM_BM + row, col = tn * GM_BN + cb * 128 + 4 * l32;
+        gemm_raster(full_tiles + t, (m + T::BM - 1) / T::BM, (n + T::BN - 1) / T::BN, group_m, tm, tn);
+        const uint32_t grow = tm * T::BM + row, col = tn * T::BN + cb * 128 + 4 * l32;
         if (grow < m && col < n) bf16_store4(c, res, (size_t)grow * ldc + col, v);
     });
 }
@@ -116,48 +86,24 @@ __device__ __forceinline__ void bf16_swiglu_store4(uint16_t* act, const float (&
 
 // act[M][N / 2] = SwiGLU(A . W^T) for interleaved gate|up weights W [N][K], N % 16 == 0: fe_gemm_bf16 with the epilogue
 // above (and fe_gemm_bf16_swiglu_reduce for the tiles cut along K). (kernels/k-core/src/gemm.rs:264-279: fe_gemm_swiglu)
-extern "C" __global__ __launch_bounds__(256, 1) void fe_gemm_bf16_swiglu(uint16_t* act, const uint16_t* a, const uint16_t* w,
+extern "C" __global__ __launch_bounds__(512, 2) void fe_gemm_bf16_swiglu(uint16_t* act, const uint16_t* a, const uint16_t* w,
                                                                          uint32_t m, uint32_t n, uint32_t k, uint32_t lda,
                                                                          uint32_t group_m, uint32_t full_tiles,
                                                                          uint32_t splits, float* part) {
-    extern __shared__ __attribute__((aligned(16))) unsigned char lds[];
-    const uint32_t tid = threadIdx.x, wave = tid >> 6, wm = wave >> 1, wn = wave & 1;
-    const GemmWork wk = gemm_work(blockIdx.x, (m + GM_BM - 1) / GM_BM, (n + GM_BN - 1) / GM_BN, group_m, k / GM_BK, full_tiles, splits);
-    const uint32_t m0 = wk.tm * GM_BM, n0 = wk.tn * GM_BN;
-    Bf16Producer prod;
-    const uint32_t chunk = tid & 7, row = tid >> 3;
-    prod.w = (const unsigned char*)w;
-#pragma unroll
-    for (int b = 0; b < 2; b++)
-#pragma unroll
-        for (int j = 0; j < 4; j++) {
-            uint32_t r = n0 + 128 * b + row + 32 * j;
-            r = r < n ? r : n - 1;
-            prod.off[b][j] = (r * k + chunk * 8) * 2;
-        }
-    prod.st = gm_swz(row, chunk);
-    f32x16 acc[4][4];
-    gemm_mainloop<Bf16Producer, true>((const _Float16*)a, lda, m, wk.kt0, wk.ktn, m0, prod, lds, acc);
-    if (wk.partial) {
-        gemm_store_partial(acc, lds, part + (size_t)wk.slot * GM_PART_FLOATS);
-        return;
-    }
-    const uint32_t col = n0 + wn * 128 + 4 * (tid & 31);
-    gemm_epilogue(
-        acc, lds, [](float (&)[4][4], uint32_t) {},
-        [&](uint32_t r, uint32_t l32, float (&v)[4]) {
-            const uint32_t grow = m0 + wm * 128 + r;
-            bf16_swiglu_store4(act, v, l32, grow < m, grow, col, n);
-        });
+    bf16_gemm_program<Bf16Tile>(a, w, m, n, k, lda, group_m, full_tiles, splits, part,
+                                [&](uint32_t row, uint32_t col, uint32_t lc, float (&v)[4]) {
+                                    bf16_swiglu_store4(act, v, lc, row < m, row, col, n);
+                                });
 }
 
 extern "C" __global__ __launch_bounds__(256) void fe_gemm_bf16_swiglu_reduce(uint16_t* act, const float* part, uint32_t m,
                                                                              uint32_t n, uint32_t group_m,
                                                                              uint32_t full_tiles, uint32_t splits) {
-    gemm_reduce_rows(part, splits, [&](uint32_t t, uint32_t row, uint32_t cb, uint32_t l32, float (&v)[4]) {
+    typedef Bf16Tile T;
+    g8_reduce_rows<T>(part, splits, [&](uint32_t t, uint32_t row, uint32_t cb, uint32_t l32, float (&v)[4]) {
         uint32_t tm, tn;
-        gemm_raster(full_tiles + t, (m + GM_BM - 1) / GM_BM, (n + GM_BN - 1) / GM_BN, group_m, tm, tn);
-        const uint32_t grow = tm * GM_BM + row, col = tn * GM_BN + cb * 128 + 4 * l32;
+        gemm_raster(full_tiles + t, (m + T::BM - 1) / T::BM, (n + T::BN - 1) / T::BN, group_m, tm, tn);
+        const uint32_t grow = tm * T::BM + row, col = tn * T::BN + cb * 128 + 4 * l32;
         bf16_swiglu_store4(act, v, l32, grow < m, grow, col, n);
     });
 }
