@@ -14,14 +14,15 @@
 
 namespace {
 constexpr uint32_t kTile = 128;                 // crates/fe-fp4/src/lib.rs:28
-constexpr uint32_t kGemmLds = 2 * (256 + 256) * 64 * 2;  // GM_LDS_TILES: two k tiles of A and W, 256 rows each
+constexpr uint32_t kGemmLds = 160 * 1024;               // k tiles of A and W in flight
+constexpr uint32_t kGemmThreads = 512;
 constexpr uint32_t kTileM = 256;                        // GM_BM
 constexpr uint32_t kTileN = 256;                        // GM_BN
 }  // namespace
 
 struct fe_fp4_kernels {
     fe_module_t module = nullptr;
-    fe_function_t quant4 = nullptr, gemm4 = nullptr, reduce4 = nullptr, gemv4[3] = {nullptr, nullptr, nullptr};
+    fe_function_t quant4 = nullptr, gemm4 = nullptr, reduce4 = nullptr, reduce8c = nullptr, gemv4[3] = {nullptr, nullptr, nullptr};
     fe_function_t strip4 = nullptr;  // the GEMV over strips of 16 weight rows, up to 16 activation rows (no hand-off)
     fe_function_t strip_once[5] = {};  // ... with every load of a workgroup issued before anything waits: 1..5 groups of K a wavefront
     fe_function_t quant8 = nullptr, gemm8 = nullptr, swiglu4 = nullptr, swiglu_reduce4 = nullptr;
@@ -70,6 +71,7 @@ int fe_fp4_kernels_load(fe_fp4_kernels **out) {
     if (!c) c = fe_hip_module_get_function(&k->gemm4, k->module, "fe_gemm_nvfp4");
     if (!c) c = fe_hip_func_set_max_dyn_lds(k->gemm4, kGemmLds);
     if (!c) c = fe_hip_module_get_function(&k->reduce4, k->module, "fe_gemm_nvfp4_reduce");
+    if (!c) c = fe_hip_module_get_function(&k->reduce8c, k->module, "fe_gemm_fp8_codes_reduce");
     for (int xr = 1; xr <= 3 && !c; xr++) {
         char nm[32];
         snprintf(nm, sizeof nm, "fe_gemv_nvfp4_x%d", xr);
@@ -417,24 +419,24 @@ int fe_fp4_linear_gemm(const fe_fp4_linear *l, const fe_fp4_kernels *kern, fe_st
     // stream-K programs sit at different depths of K: one row tile at a time (column tiles fastest) keeps those that are
     // in step on one panel of activations
     if (sch.stream_k && kern->xcd < 0) group = 1;
-    float scale = l->fp8 ? 1.0f : 0.0625f;  // what the fp16 expansions of the two operands carry (FP4_OPERAND_SCALE)
+    float scale = l->fp8 ? 1.0f : 0.5f;  // 1 / what the fp16 operands carry (FP4_GEMM_SCALE)
     if (codes8) {
         fe_devptr_t codes = ws->codes.p;
         void *args8[] = {&y, &codes, &w, &alpha, &res, &m, &n, &k, &ldy, &group, &w_snt, &w_skt, &w_sr, &sch.args};
-        FE_TRY(fe_hip_launch(sch.stream_k ? kern->gemm8c_sk : kern->gemm8c, sch.programs, 1, 1, 256, 1, 1, kGemmLds, s, args8));
+        FE_TRY(fe_hip_launch(sch.stream_k ? kern->gemm8c_sk : kern->gemm8c, sch.programs, 1, 1, kGemmThreads, 1, 1, kGemmLds, s, args8));
     } else if (l->fp8) {
         void *args8[] = {&y, &aq, &w, &alpha, &res, &m, &n, &k, &ldy, &group, &w_snt, &w_skt, &w_sr, &sch.args};
-        FE_TRY(fe_hip_launch(sch.stream_k ? kern->gemm8_sk : kern->gemm8, sch.programs, 1, 1, 256, 1, 1, kGemmLds, s, args8));
+        FE_TRY(fe_hip_launch(sch.stream_k ? kern->gemm8_sk : kern->gemm8, sch.programs, 1, 1, kGemmThreads, 1, 1, kGemmLds, s, args8));
     } else {
         void *args[] = {&y,     &aq,    &w,     &sw,   &alpha, &res,   &m,    &n,       &k,
                         &ldy,   &group, &w_snt, &w_skt, &w_sr, &s_snt, &s_skt, &s_sr, &sch.args};
-        FE_TRY(fe_hip_launch(sch.stream_k ? kern->gemm4_sk : kern->gemm4, sch.programs, 1, 1, 256, 1, 1, kGemmLds, s, args));
+        FE_TRY(fe_hip_launch(sch.stream_k ? kern->gemm4_sk : kern->gemm4, sch.programs, 1, 1, kGemmThreads, 1, 1, kGemmLds, s, args));
     }
     if (sch.stream_k || !sch.split.cut()) return 0;
     uint32_t full = sch.split.full, splits = sch.split.splits;
     fe_devptr_t part = ws->part.p;
     void *rargs[] = {&y, &part, &alpha, &res, &m, &n, &ldy, &group, &full, &splits, &scale};
-    return fe_hip_launch(kern->reduce4, sch.split.cut() * 64, 1, 1, 256, 1, 1, 0, s, rargs);
+    return fe_hip_launch(codes8 ? kern->reduce8c : kern->reduce4, sch.split.cut() * 64, 1, 1, 256, 1, 1, 0, s, rargs);
 }
 
 int fe_fp4_linear_forward(const fe_fp4_linear *l, const fe_fp4_kernels *kern, fe_stream_t s, const fe_fp4_workspace *ws,
@@ -471,7 +473,7 @@ int fe_fp4_linear_forward_swiglu(const fe_fp4_linear *l, const fe_fp4_kernels *k
     if (sch.stream_k && kern->xcd < 0) group = 1;
     void *args[] = {&aq,    &w,     &sw,    &alpha, &m,       &n,       &k,    &group, &w_snt, &w_skt,
                     &w_sr,  &s_snt, &s_skt, &s_sr,  &sch.args, &q_codes, &q_sf, &q_aq,  &down_g};
-    FE_TRY(fe_hip_launch(sch.stream_k ? kern->swiglu4_sk : kern->swiglu4, sch.programs, 1, 1, 256, 1, 1, kGemmLds, s, args));
+    FE_TRY(fe_hip_launch(sch.stream_k ? kern->swiglu4_sk : kern->swiglu4, sch.programs, 1, 1, kGemmThreads, 1, 1, kGemmLds, s, args));
     if (sch.stream_k || !sch.split.cut()) return 0;
     const FeGemmSplit &gs = sch.split;
     uint32_t full = gs.full, splits = gs.splits;

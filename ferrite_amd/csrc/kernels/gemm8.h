@@ -248,3 +248,318 @@ __device__ __forceinline__ void g8_reduce_rows(const float* __restrict__ part, u
     float v[4] = {sum[0], sum[1], sum[2], sum[3]};
     fn(t, row, cb, l32, v);
 }
+
+// The same loop for a weight operand that is packed in memory and expanded to 16-bit values as it becomes a fragment: the
+// packed k tile goes into LDS as it is (a fraction of the 16-bit form: less LDS traffic, and three stages of it are small),
+// a wavefront reads its TN fragments' codes once a k tile and expands each slice's half while the matrix instructions of
+// the slice before run. Lane group g = lane >> 4 expands the 16 consecutive k 16 g .. 16 g + 15 of its row: slice kk multiplies k
+// 16 g + 8 kk .. + 7, so A's fragments take chunk 2 g + kk (kPerm). Outer loop: A's fragments, in place; inner: the expanded
+// weights, double-buffered.
+// W: kPerm = true, STAGE bytes and LOADS loads a stage, issue(kt, dst of the stage, j, wave), Raw, read(stage in LDS, row of
+// the tile, lane group) -> Raw, expand(Raw, kk) -> f16x8.
+template <class T, int NA, int NW, class W>
+__device__ __forceinline__ void g8_mainloop_packed(const _Float16* a, uint32_t lda, uint32_t m, uint32_t kt0, uint32_t ktiles, uint32_t m0,
+                                                   const W& wo, unsigned char* lds, f32x4 (&acc)[T::TM][T::TN]) {
+    constexpr int TM = T::TM, TN = T::TN, LA = T::BM / 64, LB = W::LOADS, A_STAGE = T::BM * 128, W_AT = NA * A_STAGE;
+    static_assert(NW == NA || NW == NA + 1, "the waits below");
+    static_assert(W_AT + NW * W::STAGE <= 160 * 1024, "LDS");
+    static_assert(W::kPerm, "A's chunks");
+    const uint32_t lane = threadIdx.x & 63, wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
+    const uint32_t wm = wave / T::WN, wn = wave % T::WN;
+    const u32x4 ra = g8_rsrc(a, m * lda * 2);
+    uint32_t va[LA];
+#pragma unroll
+    for (int j = 0; j < LA; j++) {
+        const uint32_t r = 8 * (wave + 8 * j) + (lane >> 3), g = m0 + r < m ? m0 + r : m - 1;
+        va[j] = (g * lda + (g8_perm<true>((lane & 7) ^ (r & 7))) * 8) * 2;
+    }
+    const uint32_t base = g8_lds_addr(lds);
+    auto ktc = [&](uint32_t kt) { return kt0 + (kt < ktiles ? kt : ktiles - 1); };
+    auto load_a = [&](uint32_t kt, uint32_t st, int j) {
+        g8_load_lds16(ra, base + wave * 1024 + st * A_STAGE + j * 8192, va[j], ktc(kt) * 128);
+    };
+    auto load_w = [&](uint32_t kt, uint32_t st, int j) { wo.issue(ktc(kt), base + W_AT + st * W::STAGE, j, wave); };
+    auto next = [](uint32_t st, uint32_t n) { return st + 1 == n ? 0u : st + 1; };
+
+    const uint32_t fr = lane & 15, fc = lane >> 4;
+    uint32_t foff[2];
+#pragma unroll
+    for (int kk = 0; kk < 2; kk++) foff[kk] = fr * 128 + ((g8_perm<true>(2 * fc + kk) ^ (fr & 7)) << 4);
+    const unsigned char* pa = lds + wm * TM * 2048;
+    f16x8 fa[TM], fw[2][TN];
+    typename W::Raw raw[TN];
+    auto rd_a = [&](uint32_t st, int kk, int i) { fa[i] = *(const f16x8*)(pa + st * A_STAGE + 2048 * i + foff[kk]); };
+    auto rd_raw = [&](uint32_t st, int j) { raw[j] = wo.read(lds + W_AT + st * W::STAGE, (wn * TN + j) * 16 + fr, fc); };
+#pragma unroll
+    for (int i = 0; i < TM; i++)
+#pragma unroll
+        for (int j = 0; j < TN; j++) acc[i][j] = (f32x4){0.f, 0.f, 0.f, 0.f};
+#pragma unroll
+    for (int t = 0; t < NA; t++) {
+        if (NW - 1 - NA + t >= 0) {
+#pragma unroll
+            for (int j = 0; j < LB; j++) load_w(NW - 1 - NA + t, NW - 1 - NA + t, j);
+        }
+#pragma unroll
+        for (int j = 0; j < LA; j++) load_a(t, t, j);
+    }
+    g8_loads_wait<(NW > NA ? (NA - 1) * (LA + LB) : (NA - 1) * LA + (NA > 1 ? (NA - 2) * LB : 0))>();
+    g8_barrier();
+#pragma unroll
+    for (int j = 0; j < TN; j++) rd_raw(0, j);
+#pragma unroll
+    for (int i = 0; i < TM; i++) rd_a(0, 0, i);
+#pragma unroll
+    for (int j = 0; j < TN; j++) fw[0][j] = wo.expand(raw[j], 0);
+
+    uint32_t sa = 0, sw = 0, sw_in = NW - 1;
+    for (uint32_t kt = 0; kt < ktiles; kt++) {
+        const uint32_t sa1 = next(sa, NA), sw1 = next(sw, NW);
+#pragma unroll
+        for (int kk = 0; kk < 2; kk++) {
+            if (kk == 1) {
+                g8_loads_wait<(NW > NA ? (NA - 1) * LB + (NA - 2) * LA : (NA - 2) * (LA + LB))>();
+                g8_barrier();
+            }
+            const uint32_t ra_st = kk ? sa1 : sa;
+#pragma unroll
+            for (int i = 0; i < TM; i++) {
+#pragma unroll
+                for (int j = 0; j < TN; j++) {
+                    const int jj = i & 1 ? TN - 1 - j : j;
+                    acc[i][jj] = __builtin_amdgcn_mfma_f32_16x16x32_f16(fw[kk][jj], fa[i], acc[i][jj], 0, 0, 0);
+                }
+                rd_a(ra_st, kk ^ 1, i);
+                if (kk == 0) {  // the second half of this tile's codes, spread over the slice
+#pragma unroll
+                    for (int j = i * TN / TM; j < (i + 1) * TN / TM; j++) fw[1][j] = wo.expand(raw[j], 1);
+                } else {  // the next tile's codes, then their first half in the slice's second half
+                    if (i == 0) {
+#pragma unroll
+                        for (int j = 0; j < TN; j++) rd_raw(sw1, j);
+                    }
+                    constexpr int H = TM / 2;
+                    if (i >= H) {
+#pragma unroll
+                        for (int j = (i - H) * TN / (TM - H); j < (i - H + 1) * TN / (TM - H); j++) fw[0][j] = wo.expand(raw[j], 0);
+                    }
+                }
+                const int n = kk ? LA : LB;
+#pragma unroll
+                for (int q = i * n / TM; q < (i + 1) * n / TM; q++) {
+                    if (kk == 0)
+                        load_w(kt + NW - 1, sw_in, q);
+                    else
+                        load_a(kt + NA, sa, q);
+                }
+                __builtin_amdgcn_sched_barrier(0);
+            }
+        }
+        sa = sa1, sw_in = sw, sw = sw1;
+    }
+    asm volatile("s_waitcnt vmcnt(0)" ::: "memory");
+    __syncthreads();
+}
+
+// The loop for 8-bit operands (e4m3 codes on both sides) on v_mfma_f32_16x16x128_f8f6f4: a k tile is 128 codes, so rows are again
+// 128 bytes and stages, chunk positions and loads are those of g8_mainloop; a lane's operand of the one MFMA step of a k
+// tile is chunks fc and 4 + fc of its row (both operands alike: k is a summation index only). A fragment takes 8 registers,
+// so the weight fragments pass through a ring of four, each refilled four columns ahead, and the A fragments are refilled in
+// place behind the last column. The barrier comes after the fifth column, the first that makes room for the next tile's.
+// a: codes [m][lda] (bytes).
+typedef int g8_i32x8 __attribute__((ext_vector_type(8)));
+template <class T, int NA, int NW>
+__device__ __forceinline__ void g8_mainloop_f8(const uint8_t* a, uint32_t lda, uint32_t m, uint32_t kt0, uint32_t ktiles, uint32_t m0,
+                                               const G8Dense<T>& wo, unsigned char* lds, f32x4 (&acc)[T::TM][T::TN]) {
+    constexpr int TM = T::TM, TN = T::TN, R = 4, LA = T::BM / 64, LB = G8Dense<T>::LOADS, A_STAGE = T::BM * 128, W_AT = NA * A_STAGE;
+    constexpr int W_STAGE = G8Dense<T>::STAGE, BAR = TN - R;  // the barrier follows column BAR
+    static_assert(TN >= 2 * R || TN == R, "columns 0 .. TN - R - 1 refill from this tile");
+    static_assert(NW == NA || NW == NA + 1, "the waits below");
+    static_assert(W_AT + NW * W_STAGE <= 160 * 1024, "LDS");
+    const uint32_t lane = threadIdx.x & 63, wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
+    const uint32_t wm = wave / T::WN, wn = wave % T::WN;
+    const u32x4 ra = g8_rsrc(a, m * lda);
+    uint32_t va[LA];
+#pragma unroll
+    for (int j = 0; j < LA; j++) {
+        const uint32_t r = 8 * (wave + 8 * j) + (lane >> 3), g = m0 + r < m ? m0 + r : m - 1;
+        va[j] = g * lda + ((lane & 7) ^ (r & 7)) * 16;
+    }
+    const uint32_t base = g8_lds_addr(lds) + wave * 1024;
+    auto ktc = [&](uint32_t kt) { return kt0 + (kt < ktiles ? kt : ktiles - 1); };
+    auto load_a = [&](uint32_t kt, uint32_t st, int j) { g8_load_lds16(ra, base + st * A_STAGE + j * 8192, va[j], ktc(kt) * 128); };
+    auto load_w = [&](uint32_t kt, uint32_t st, int j) { wo.issue(ktc(kt), base + W_AT + st * W_STAGE, j); };
+    auto next = [](uint32_t st, uint32_t n) { return st + 1 == n ? 0u : st + 1; };
+    const uint32_t fr = lane & 15, fc = lane >> 4;
+    uint32_t foff[2];
+#pragma unroll
+    for (int h = 0; h < 2; h++) foff[h] = fr * 128 + (((4 * h + fc) ^ (fr & 7)) << 4);
+    const unsigned char* pa = lds + wm * TM * 2048;
+    const unsigned char* pw = lds + W_AT + wn * TN * 2048;
+    auto read = [&](const unsigned char* p) {
+        const u32x4 lo = *(const u32x4*)(p + foff[0]), hi = *(const u32x4*)(p + foff[1]);
+        return (g8_i32x8){(int)lo[0], (int)lo[1], (int)lo[2], (int)lo[3], (int)hi[0], (int)hi[1], (int)hi[2], (int)hi[3]};
+    };
+    g8_i32x8 fa[TM], fw[R];
+    auto rd_a = [&](uint32_t st, int i) { fa[i] = read(pa + st * A_STAGE + 2048 * i); };
+    auto rd_w = [&](uint32_t st, int j) { fw[j % R] = read(pw + st * W_STAGE + 2048 * j); };
+#pragma unroll
+    for (int i = 0; i < TM; i++)
+#pragma unroll
+        for (int j = 0; j < TN; j++) acc[i][j] = (f32x4){0.f, 0.f, 0.f, 0.f};
+#pragma unroll
+    for (int t = 0; t < NA; t++) {
+        if (NW - 1 - NA + t >= 0) {
+#pragma unroll
+            for (int j = 0; j < LB; j++) load_w(NW - 1 - NA + t, NW - 1 - NA + t, j);
+        }
+#pragma unroll
+        for (int j = 0; j < LA; j++) load_a(t, t, j);
+    }
+    g8_loads_wait<(NW > NA ? (NA - 1) * (LA + LB) : (NA - 1) * LA + (NA > 1 ? (NA - 2) * LB : 0))>();
+    g8_barrier();
+#pragma unroll
+    for (int i = 0; i < TM; i++) rd_a(0, i);
+#pragma unroll
+    for (int j = 0; j < R; j++) rd_w(0, j);
+    uint32_t sa = 0, sw = 0, sw_in = NW - 1;
+    for (uint32_t kt = 0; kt < ktiles; kt++) {
+        const uint32_t sa1 = next(sa, NA), sw1 = next(sw, NW);
+#pragma unroll
+        for (int j = 0; j < TN; j++) {
+#pragma unroll
+            for (int x = 0; x < TM; x++) {
+                const int i = j & 1 ? TM - 1 - x : x;  // formats 0, 0: e4m3 x e4m3; zero scale operands select the unscaled instruction
+                acc[i][j] = __builtin_amdgcn_mfma_scale_f32_16x16x128_f8f6f4(fw[j % R], fa[i], acc[i][j], 0, 0, 0, 0, 0, 0);
+            }
+            if (j == BAR) {
+                g8_loads_wait<(NW > NA ? (NA - 1) * LB + (NA - 2) * LA : (NA - 2) * (LA + LB))>();
+                g8_barrier();
+            }
+            rd_w(j < BAR ? sw : sw1, (j + R) % TN);
+            if (j == TN - 1) {
+#pragma unroll
+                for (int x = 0; x < TM; x++) rd_a(sa1, j & 1 ? TM - 1 - x : x);
+            }
+            // loads: W in the columns before the barrier, A after it
+            if (j < BAR) {
+#pragma unroll
+                for (int q = j * LB / BAR; q < (j + 1) * LB / BAR; q++) load_w(kt + NW - 1, sw_in, q);
+            } else {
+#pragma unroll
+                for (int q = (j - BAR) * LA / R; q < (j - BAR + 1) * LA / R; q++) load_a(kt + NA, sa, q);
+            }
+            __builtin_amdgcn_sched_barrier(0);
+        }
+        sa = sa1, sw_in = sw, sw = sw1;
+    }
+    asm volatile("s_waitcnt vmcnt(0)" ::: "memory");
+    __syncthreads();
+}
+
+// ---- schedules -------------------------------------------------------------------------------------------------------------
+// (stream-K: see gemm_core.h's account of the runs, the slots and the arrival counters; here a piece is stored and read as the
+// lanes hold it, 512 threads x 16 bytes at a time)
+
+template <class T>
+__device__ __forceinline__ bool g8_sk_meet(f32x4 (&acc)[T::TM][T::TN], uint32_t p, uint32_t tile, uint32_t t0, uint32_t ktiles,
+                                           uint32_t base, uint32_t rem, float* part, uint32_t part_bytes, uint32_t* counters,
+                                           unsigned char* lds) {
+    constexpr int TM = T::TM, TN = T::TN;
+    constexpr uint32_t PIECE = T::THREADS * 16, SLOT = T::PART_FLOATS * 4;
+    const uint32_t tid = threadIdx.x;
+    const uint32_t first = sk_owner(t0, base, rem), last = sk_owner(t0 + ktiles - 1, base, rem);
+    const uint32_t n = last - first + 1, me = p - first;
+    const __amdgpu_buffer_rsrc_t rs = __builtin_amdgcn_make_buffer_rsrc((void*)part, 0, part_bytes, 0x00020000);
+    volatile uint32_t* flag = (volatile uint32_t*)lds;
+    uint32_t* cnt = counters + tile;
+    // a run's piece of a tile in which the run does not begin is the run's last segment
+    auto slot_of = [&](uint32_t q) { return 2 * q + (sk_start(q, base, rem) < t0 ? 1u : 0u); };
+    // (a read-modify-write, which is performed where all XCDs meet: no stale copy of the counter can answer it)
+    if (tid == 0) *flag = __hip_atomic_fetch_add(cnt, 0u, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+    __syncthreads();
+    uint32_t seen = *flag;
+    __syncthreads();
+    if (seen != n - 1) {  // someone is still at work: leave the piece
+        const uint32_t so = slot_of(p) * SLOT;
+#pragma unroll
+        for (int i = 0; i < TM; i++)
+#pragma unroll
+            for (int j = 0; j < TN; j++)
+                __builtin_amdgcn_raw_buffer_store_b128(__builtin_bit_cast(u32x4, acc[i][j]), rs, tid * 16, so + (i * TN + j) * PIECE, 16);
+        agent_stores_wait();
+        __syncthreads();
+        if (tid == 0) *flag = __hip_atomic_fetch_add(cnt, 1u, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+        __syncthreads();
+        seen = *flag;
+        __syncthreads();
+        if (seen != n - 1) return false;
+    }
+    // the pieces in piece order, starting from zero, this program's accumulators in their place
+#pragma unroll
+    for (int i = 0; i < TM; i++) {
+        f32x4 t[TN];
+#pragma unroll
+        for (int j = 0; j < TN; j++) t[j] = (f32x4){0.f, 0.f, 0.f, 0.f};
+        for (uint32_t q = 0; q < n; q++) {
+            if (q == me) {
+#pragma unroll
+                for (int j = 0; j < TN; j++) t[j] += acc[i][j];
+            } else {
+                const uint32_t so = slot_of(first + q) * SLOT + i * TN * PIECE;
+                f32x4 ld[TN];
+#pragma unroll
+                for (int j = 0; j < TN; j++) ld[j] = load_agent_f32x4(rs, tid * 16, so + j * PIECE);
+#pragma unroll
+                for (int j = 0; j < TN; j++) t[j] += ld[j];
+            }
+        }
+#pragma unroll
+        for (int j = 0; j < TN; j++) acc[i][j] = t[j];
+    }
+    if (tid == 0) __hip_atomic_store(cnt, 0u, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+    return true;
+}
+
+// Runs the program's share of the schedule: main(tm, tn, kt0, ktn, acc) is one pass of the main loop over k tiles
+// kt0 .. kt0 + ktn - 1 of tile (tm, tn), finish(tm, tn, acc) the tile's epilogue. sc.sk_base is nonzero exactly when SK.
+template <class T, bool SK, class Main, class Finish>
+__device__ __forceinline__ void g8_schedule(const GemmSched& sc, uint32_t tiles_m, uint32_t tiles_n, uint32_t group, uint32_t ktiles,
+                                            unsigned char* lds, Main main, Finish finish) {
+    const uint32_t p = blockIdx.x;
+    f32x4 acc[T::TM][T::TN];
+    if constexpr (!SK) {
+        const GemmWork wk = gemm_work(p, tiles_m, tiles_n, group, ktiles, sc.full_tiles, sc.splits);
+        main(wk.tm, wk.tn, wk.kt0, wk.ktn, acc);
+        if (wk.partial)
+            g8_store_partial<T>(acc, sc.part + (size_t)wk.slot * T::PART_FLOATS);
+        else
+            finish(wk.tm, wk.tn, acc);
+    } else {
+        const uint32_t whole = sc.full_tiles;  // taken whole, program p those p, p + grid, ...; the runs lie over the tiles after them
+        uint32_t next_whole = p;
+        uint32_t u = sk_start(p, sc.sk_base, sc.sk_rem);
+        const uint32_t uend = sk_start(p + 1, sc.sk_base, sc.sk_rem);
+        while (next_whole < whole || u < uend) {
+            uint32_t tile, t0 = 0, kt0 = 0, ktn = ktiles;
+            if (next_whole < whole) {
+                tile = next_whole;
+                next_whole += gridDim.x;
+            } else {
+                const uint32_t rel = u / ktiles;
+                t0 = rel * ktiles, kt0 = u - t0;
+                ktn = ktiles - kt0 < uend - u ? ktiles - kt0 : uend - u;
+                tile = whole + rel;
+                u += ktn;
+            }
+            uint32_t tm, tn;
+            gemm_raster(tile, tiles_m, tiles_n, group, tm, tn);
+            __syncthreads();  // the epilogue of the segment before is done with the LDS
+            main(tm, tn, kt0, ktn, acc);
+            bool fin = true;
+            if (ktn != ktiles)
+                fin = g8_sk_meet<T>(acc, p, tile, t0, ktiles, sc.sk_base, sc.sk_rem, sc.part, sc.part_bytes, sc.counters, lds);
+            if (fin) finish(tm, tn, acc);
+        }
+    }
+}

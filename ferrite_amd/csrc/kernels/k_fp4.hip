@@ -7,7 +7,7 @@
 // exact, normal fp16 number: both operands are expanded to fp16 (activations as 2 * code value * block scale, weights
 // as 8 * ...) and multiplied on the f16 MFMA with fp32 accumulation, which reproduces the block-scaled dot product up
 // to summation order; the factor 16 comes off in the epilogue.
-#include "gemm_core.h"
+#include "gemm8.h"
 
 // ---- number formats ----------------------------------------------------------------------------------------------------
 
@@ -183,38 +183,64 @@ extern "C" __global__ __launch_bounds__(256) void fe_fp4_quant(uint8_t* codes, u
 
 // ---- GEMM --------------------------------------------------------------------------------------------------------------
 
-// Weight tile producer: thread t expands the 64 codes of row t of the 256-row weight tile. Codes and scales are
-// addressed through strides, base + kt * skt for the thread's row, so both the row-major layout of the format and the
-// k-tile-major layout of an uploaded linear ([n / 128][k / 64][128 rows][32 bytes of codes | 4 scales], one contiguous
-// 4.5 KB read per 128 rows and k tile) are read by the same kernel.
-struct Fp4Producer {
-    const uint8_t* w;   // codes of this thread's row, k tile 0
-    const uint8_t* sw;  // scales of this thread's row, k tile 0
-    uint32_t w_skt, s_skt, row;
+// An e4m3 scale (sign bit clear) as packed fp16, both halves, times 2^-8: the code's bits shifted to fp16's place, exact
+// for normal and subnormal codes alike. The weight's conversion carries the 2^8.
+__device__ __forceinline__ f16x2 fp4_scale_2m8(uint32_t b) { return __builtin_bit_cast(f16x2, b * 0x00800080u); }
+// 8 codes of one u32 -> 8 fp16 (code * scale), elements in order: one instruction a weight
+__device__ __forceinline__ f16x8 fp4x8_scaled(uint32_t w, f16x2 s) {
+    u32x4 o;
+    o[0] = __builtin_bit_cast(uint32_t, (f16x2)(__builtin_amdgcn_cvt_scalef32_pk_f16_fp4(w, 256.0f, 0) * s));
+    o[1] = __builtin_bit_cast(uint32_t, (f16x2)(__builtin_amdgcn_cvt_scalef32_pk_f16_fp4(w, 256.0f, 1) * s));
+    o[2] = __builtin_bit_cast(uint32_t, (f16x2)(__builtin_amdgcn_cvt_scalef32_pk_f16_fp4(w, 256.0f, 2) * s));
+    o[3] = __builtin_bit_cast(uint32_t, (f16x2)(__builtin_amdgcn_cvt_scalef32_pk_f16_fp4(w, 256.0f, 3) * s));
+    return __builtin_bit_cast(f16x8, o);
+}
+
+// Weight operand of the GEMM: codes and scales of a k tile as they lie in memory, [BN rows][32 bytes of codes] and then [BN
+// rows][4 scales] in LDS. Addressed through strides, so both the row-major layout of the format and the k-tile-major layout
+// of an uploaded linear ([n / 128][k / 64][128 rows][32 bytes of codes | 4 scales], one contiguous 4.5 KB read per 128 rows
+// and k tile) are read by the same kernel. An odd count of 128-row tiles: the last program reads its first tile twice.
+template <class T>
+struct Fp4Packed {
+    static constexpr bool kPerm = true;
+    static constexpr int STAGE = T::BN * 36, LOADS = 2;
+    u32x4 rw, rs;
+    uint32_t wv, sv, w_skt, s_skt;
     struct Raw {
-        u32x4 c[2];
-        uint32_t s2[2];
+        u32x2 c;
+        f16x2 s;
     };
-    static constexpr int kStoreValu = 96;  // about the VALU instructions of store()
-    static constexpr bool kQuarters = false;
-    __device__ __forceinline__ void load(uint32_t kt, Raw& r, int half) const {
-        r.c[half] = *(const u32x4*)(w + (size_t)kt * w_skt + 16 * half);
-        r.s2[half] = *(const uint16_t*)(sw + (size_t)kt * s_skt + 2 * half);
+    __device__ __forceinline__ void setup(const uint8_t* w, const uint8_t* sw, uint32_t n, uint32_t k, uint32_t n0, uint32_t w_snt,
+                                          uint32_t w_skt_, uint32_t w_sr, uint32_t s_snt, uint32_t s_skt_, uint32_t s_sr) {
+        const uint32_t lane = threadIdx.x & 63, wave = threadIdx.x >> 6, nts = n / 128;
+        auto at = [&](uint32_t row, uint32_t snt, uint32_t sr) {
+            uint32_t nt = (n0 + row) / 128;
+            nt = nt < nts ? nt : nts - 1;
+            return nt * snt + (row & 127) * sr;
+        };
+        rw = g8_rsrc(w, n * (k / 2)), rs = g8_rsrc(sw, n * (k / 16));
+        wv = at((wave % (T::BN / 32)) * 32 + lane / 2, w_snt, w_sr) + (lane & 1) * 16;
+        sv = at((wave % (T::BN / 64)) * 64 + lane, s_snt, s_sr);
+        w_skt = w_skt_, s_skt = s_skt_;
     }
-    // part 0: chunks 0..3 of the row, part 1: 4..7
-    __device__ __forceinline__ void store(const Raw& r, unsigned char* Bs, int part) const {
-#pragma unroll
-        for (int d = 0; d < 8; d++) {
-            if (d / 4 != part) continue;
-            // (computed: looked up in an LDS table as the GEMV does, the reads queue behind the fragment reads of the
-            // k tile in flight and the GEMM is 5 % slower)
-            Fp4Scale sc = fp4_scale((r.s2[d >> 2] >> (8 * ((d >> 1) & 1))) & 0xff);
-            *(u32x4*)(Bs + gm_swz(row, d)) = fp4x8_to_f16(r.c[d >> 2][d & 3], sc);
-        }
+    // (fewer pieces than wavefronts: the others move one again)
+    __device__ __forceinline__ void issue(uint32_t kt, uint32_t dst, int j, uint32_t wave) const {
+        if (j == 0)
+            g8_load_lds16(rw, dst + (wave % (T::BN / 32)) * 1024, wv, kt * w_skt);
+        else
+            g8_load_lds4(rs, dst + T::BN * 32 + (wave % (T::BN / 64)) * 256, sv, kt * s_skt);
     }
+    __device__ __forceinline__ Raw read(const unsigned char* st, uint32_t row, uint32_t g) const {
+        Raw r;
+        r.c = *(const u32x2*)(st + row * 32 + 8 * g);
+        r.s = fp4_scale_2m8(__builtin_amdgcn_ubfe(*(const uint32_t*)(st + T::BN * 32 + row * 4), 8 * g, 8));
+        return r;
+    }
+    __device__ __forceinline__ f16x8 expand(const Raw& r, int kk) const { return fp4x8_scaled(kk ? r.c[1] : r.c[0], r.s); }
 };
 
-// The fp16 operands are 2 x the quantized activation and 8 x the quantized weight.
+// The fp16 operands of the GEMM are 2 x the quantized activation and the quantized weight; the GEMV's carry 8 x the weight.
+#define FP4_GEMM_SCALE 0.5f
 #define FP4_OPERAND_SCALE 0.0625f
 
 // One row piece of the output: 4 columns from `col` of row `grow`, bf16((sum) * alpha) (+ res: bf16(bf16(.) + res)).
@@ -267,32 +293,40 @@ extern "C" __global__ __launch_bounds__(256) void fe_fp8_quant(uint8_t* codes, _
     *(u32x4*)(aq + (size_t)row * k + c) = o;
 }
 
-// Weight tile producer for e4m3 weights: thread t expands the 64 codes (64 bytes) of row t of the 256-row weight tile
-// with the hardware conversion (exact). Addressing as Fp4Producer, 64 bytes a row and k tile.
-struct Fp8Producer {
-    const uint8_t* w;
-    uint32_t w_skt, row;
+// Weight operand of the fp16 form of the FP8 GEMM: e4m3 codes, [BN rows][64 bytes] in LDS, expanded with the hardware
+// conversion (exact). Addressing as Fp4Packed.
+template <class T>
+struct Fp8Packed {
+    static constexpr bool kPerm = true;
+    static constexpr int STAGE = T::BN * 64, LOADS = T::BN / 128;
+    u32x4 rw;
+    uint32_t wv[LOADS], w_skt;
     struct Raw {
-        u32x4 c[4];
+        u32x4 c;
     };
-    static constexpr int kStoreValu = 40;
-    static constexpr bool kQuarters = false;
-    __device__ __forceinline__ void load(uint32_t kt, Raw& r, int half) const {
-        const uint8_t* p = w + (size_t)kt * w_skt + 32 * half;
-        r.c[2 * half] = *(const u32x4*)p;
-        r.c[2 * half + 1] = *(const u32x4*)(p + 16);
-    }
-    // part 0: chunks 0..3 of the row (bytes 0..31), part 1: 4..7
-    __device__ __forceinline__ void store(const Raw& r, unsigned char* Bs, int part) const {
+    __device__ __forceinline__ void setup(const uint8_t* w, uint32_t n, uint32_t k, uint32_t n0, uint32_t w_snt, uint32_t w_skt_, uint32_t w_sr) {
+        const uint32_t lane = threadIdx.x & 63, wave = threadIdx.x >> 6, nts = n / 128;
+        rw = g8_rsrc(w, n * k);
 #pragma unroll
-        for (int d = 0; d < 8; d++) {
-            if (d / 4 != part) continue;
-            u32x4 o;
-#pragma unroll
-            for (int e = 0; e < 4; e++)
-                o[e] = e4m3x2_to_f16(r.c[d >> 1][2 * (d & 1) + (e >> 1)], e & 1);
-            *(u32x4*)(Bs + gm_swz(row, d)) = o;
+        for (int j = 0; j < LOADS; j++) {
+            const uint32_t row = (wave + 8 * j) * 16 + lane / 4;
+            uint32_t nt = (n0 + row) / 128;
+            nt = nt < nts ? nt : nts - 1;
+            wv[j] = nt * w_snt + (row & 127) * w_sr + (lane & 3) * 16;
         }
+        w_skt = w_skt_;
+    }
+    __device__ __forceinline__ void issue(uint32_t kt, uint32_t dst, int j, uint32_t wave) const {
+        g8_load_lds16(rw, dst + (wave + 8 * j) * 1024, wv[j], kt * w_skt);
+    }
+    __device__ __forceinline__ Raw read(const unsigned char* st, uint32_t row, uint32_t g) const {
+        return Raw{*(const u32x4*)(st + row * 64 + 16 * g)};
+    }
+    __device__ __forceinline__ f16x8 expand(const Raw& r, int kk) const {
+        u32x4 o;
+#pragma unroll
+        for (int e = 0; e < 4; e++) o[e] = e4m3x2_to_f16(r.c[2 * kk + (e >> 1)], e & 1);
+        return __builtin_bit_cast(f16x8, o);
     }
 };
 
@@ -377,63 +411,51 @@ __device__ __forceinline__ void fp_store_piece(const FpOut& o, const float (&v)[
     }
 }
 
+typedef G8Tile<4, 2, 4, 8> Fp8Tile;  // the GEMM over FP8 codes: 256 x 256
+typedef G8Tile<2, 4, 8, 4> FpTile;  // 256 x 256; a wavefront's 128 x 64 keeps the codes it expands to a quarter of the tile's
+
 // C[M][ldc] = bf16((A_q . W_q^T) * alpha[n]) (+ res: bf16(bf16(.) + res)); A_q = the fp16 operand of the quantizer,
-// W_q expanded by the producer make_prod(tn) of 256-column tile tn; `scale` = 1 / (the factors the two fp16 expansions
-// carry). Tiles = ceil(M / 256) * ceil(N / 256) (grouped raster), spread over the grid as sc says (gemm_schedule): one
-// piece a program, the cut tiles finished by the reduce kernel, or stream-K. 256 threads, dynamic LDS GM_LDS_TILES.
+// W_q expanded by the packed operand make_packed(tn) of 256-column tile tn; `scale` = 1 / (the factors the two fp16 operands
+// carry). Tiles = ceil(M / 256) * ceil(N / 256) (grouped raster), spread over the grid as sc says (g8_schedule): one
+// piece a program, the cut tiles finished by the reduce kernel, or stream-K. 512 threads, dynamic LDS 160 KB.
 // N % 128 == 0, K % 128 == 0. (kernels/k-fp4/src/lib.rs:285-470)
-template <bool SWIGLU, bool SK, class MakeProd>
-__device__ __forceinline__ void fp_gemm_body(MakeProd make_prod, const FpOut& out, const _Float16* aq, const float* alpha,
+template <bool SWIGLU, bool SK, class MakePacked>
+__device__ __forceinline__ void fp_gemm_body(MakePacked make_packed, const FpOut& out, const _Float16* aq, const float* alpha,
                                              float scale, uint32_t m, uint32_t n, uint32_t k, uint32_t group_m,
                                              const GemmSched& sc) {
-    extern __shared__ __attribute__((aligned(16))) unsigned char lds[];
-    const uint32_t tid = threadIdx.x, wave = tid >> 6, wm = wave >> 1, wn = wave & 1;
-    gemm_schedule<SK>(
-        sc, (m + GM_BM - 1) / GM_BM, (n / 128 + 1) / 2, group_m, k / GM_BK, lds,
-        [&](uint32_t tm, uint32_t tn, uint32_t kt0, uint32_t ktn, f32x16(&acc)[4][4]) {
-            auto prod = make_prod(tn);
-            gemm_mainloop(aq, k, m, kt0, ktn, tm * GM_BM, prod, lds, acc);
+    typedef FpTile T;
+    extern __shared__ __attribute__((aligned(1024))) unsigned char lds[];
+    const uint32_t lane = threadIdx.x & 63, wave = threadIdx.x >> 6, wm = wave / T::WN, wn = wave % T::WN;
+    g8_schedule<T, SK>(
+        sc, (m + T::BM - 1) / T::BM, (n / 128 + 1) / 2, group_m, k / G8_BK, lds,
+        [&](uint32_t tm, uint32_t tn, uint32_t kt0, uint32_t ktn, f32x4(&acc)[T::TM][T::TN]) {
+            auto w = make_packed(tn);
+            g8_mainloop_packed<T, 3, 3>(aq, k, m, kt0, ktn, tm * T::BM, w, lds, acc);
         },
-        [&](uint32_t tm, uint32_t tn, f32x16(&acc)[4][4]) {
-            const uint32_t m0 = tm * GM_BM, colb = tn * GM_BN + wn * 128;
+        [&](uint32_t tm, uint32_t tn, f32x4(&acc)[T::TM][T::TN]) {
+            const uint32_t m0 = tm * T::BM + wm * 16 * T::TM, colb = tn * T::BN + wn * 16 * T::TN;
             if (colb >= n) return;
-            const uint32_t col = colb + 4 * (tid & 31);
+            const uint32_t col = colb + 4 * (lane % (4 * T::TN));
             const f32x4 al = *(const f32x4*)(alpha + col) * scale;
-            gemm_epilogue(
-                acc, lds, [](float (&)[4][4], uint32_t) {},
-                [&](uint32_t row, uint32_t l32, float (&v)[4]) {
-                    fp_store_piece<SWIGLU>(out, v, al, l32, m0 + wm * 128 + row, m, col, n);
-                });
+            g8_epilogue<T>(
+                acc, lds, [](auto&, uint32_t) {},
+                [&](uint32_t row, uint32_t lc, float (&v)[4]) { fp_store_piece<SWIGLU>(out, v, al, lc, m0 + row, m, col, n); });
         });
 }
 
 // Finishes the tiles that a GEMM kernel cut along K. grid (tiles - full_tiles) * 64, 256 threads.
-template <bool SWIGLU>
+template <class T, bool SWIGLU>
 __device__ __forceinline__ void fp_reduce_body(const FpOut& out, const float* part, const float* alpha, float scale,
                                                uint32_t m, uint32_t n, uint32_t group_m, uint32_t full_tiles,
                                                uint32_t splits) {
     const uint32_t nts = n / 128;
-    gemm_reduce_rows(part, splits, [&](uint32_t t, uint32_t row, uint32_t cb, uint32_t l32, float (&v)[4]) {
+    g8_reduce_rows<T>(part, splits, [&](uint32_t t, uint32_t row, uint32_t cb, uint32_t l32, float (&v)[4]) {
         uint32_t tm, tn;
-        gemm_raster(full_tiles + t, (m + GM_BM - 1) / GM_BM, (nts + 1) / 2, group_m, tm, tn);
-        uint32_t grow = tm * GM_BM + row, col = tn * GM_BN + cb * 128 + 4 * l32;
-        if (tn * GM_BN + cb * 128 >= n) return;  // the absent half of an odd last tile (uniform over the half wavefront)
+        gemm_raster(full_tiles + t, (m + T::BM - 1) / T::BM, (nts + 1) / 2, group_m, tm, tn);
+        uint32_t grow = tm * T::BM + row, col = tn * T::BN + cb * 128 + 4 * l32;
+        if (tn * T::BN + cb * 128 >= n) return;  // the absent half of an odd last tile (uniform over the half wavefront)
         fp_store_piece<SWIGLU>(out, v, *(const f32x4*)(alpha + col) * scale, l32, grow, m, col, n);
     });
-}
-
-__device__ __forceinline__ Fp4Producer fp4_producer(const uint8_t* w, const uint8_t* sw, uint32_t tn, uint32_t nts,
-                                                    uint32_t w_snt, uint32_t w_skt, uint32_t w_sr, uint32_t s_snt,
-                                                    uint32_t s_skt, uint32_t s_sr) {
-    const uint32_t tid = threadIdx.x;
-    uint32_t nt = 2 * tn + (tid >> 7);
-    nt = nt < nts ? nt : nts - 1;  // an odd count of 128-row tiles: the last program expands its first tile twice
-    Fp4Producer prod;
-    prod.row = tid;
-    prod.w = w + (size_t)nt * w_snt + (size_t)(tid & 127) * w_sr;
-    prod.sw = sw + (size_t)nt * s_snt + (size_t)(tid & 127) * s_sr;
-    prod.w_skt = w_skt, prod.s_skt = s_skt;
-    return prod;
 }
 
 // NVFP4: the codes of row r = 128 nt + i, k tile kt are 32 bytes at w + nt * w_snt + kt * w_skt + i * w_sr, its 4 scales
@@ -447,13 +469,17 @@ template <bool SK>
 __device__ __forceinline__ void gemm_nvfp4_kernel(FP4_GEMM_PARAMS) {
     FpOut out = {c, res, ldc, nullptr, nullptr, nullptr, 0.f};
     fp_gemm_body<false, SK>(
-        [&](uint32_t tn) { return fp4_producer(w, sw, tn, n / 128, w_snt, w_skt, w_sr, s_snt, s_skt, s_sr); }, out, aq, alpha,
-        FP4_OPERAND_SCALE, m, n, k, group_m, sc);
+        [&](uint32_t tn) {
+            Fp4Packed<FpTile> p;
+            p.setup(w, sw, n, k, tn * FpTile::BN, w_snt, w_skt, w_sr, s_snt, s_skt, s_sr);
+            return p;
+        },
+        out, aq, alpha, FP4_GEMM_SCALE, m, n, k, group_m, sc);
 }
-extern "C" __global__ __launch_bounds__(256, 1) void fe_gemm_nvfp4(FP4_GEMM_PARAMS) {
+extern "C" __global__ __launch_bounds__(512, 2) void fe_gemm_nvfp4(FP4_GEMM_PARAMS) {
     gemm_nvfp4_kernel<false>(c, aq, w, sw, alpha, res, m, n, k, ldc, group_m, w_snt, w_skt, w_sr, s_snt, s_skt, s_sr, sc);
 }
-extern "C" __global__ __launch_bounds__(256, 1) void fe_gemm_nvfp4_sk(FP4_GEMM_PARAMS) {
+extern "C" __global__ __launch_bounds__(512, 2) void fe_gemm_nvfp4_sk(FP4_GEMM_PARAMS) {
     gemm_nvfp4_kernel<true>(c, aq, w, sw, alpha, res, m, n, k, ldc, group_m, w_snt, w_skt, w_sr, s_snt, s_skt, s_sr, sc);
 }
 
@@ -462,7 +488,7 @@ extern "C" __global__ __launch_bounds__(256) void fe_gemm_nvfp4_reduce(uint16_t*
                                                                        uint32_t ldc, uint32_t group_m, uint32_t full_tiles,
                                                                        uint32_t splits, float scale) {
     FpOut out = {c, res, ldc, nullptr, nullptr, nullptr, 0.f};
-    fp_reduce_body<false>(out, part, alpha, scale, m, n, group_m, full_tiles, splits);
+    fp_reduce_body<FpTile, false>(out, part, alpha, scale, m, n, group_m, full_tiles, splits);
 }
 
 // Fused MLP front: act = SwiGLU(x . [gate|up]^T), NVFP4-quantized with global scale qg (1 / input_scale of the down
@@ -476,14 +502,18 @@ template <bool SK>
 __device__ __forceinline__ void gemm_nvfp4_swiglu_kernel(FP4_SWIGLU_PARAMS) {
     FpOut out = {nullptr, nullptr, 0, q_codes, q_sf, q_aq, qg};
     fp_gemm_body<true, SK>(
-        [&](uint32_t tn) { return fp4_producer(w, sw, tn, n / 128, w_snt, w_skt, w_sr, s_snt, s_skt, s_sr); }, out, aq, alpha,
-        FP4_OPERAND_SCALE, m, n, k, group_m, sc);
+        [&](uint32_t tn) {
+            Fp4Packed<FpTile> p;
+            p.setup(w, sw, n, k, tn * FpTile::BN, w_snt, w_skt, w_sr, s_snt, s_skt, s_sr);
+            return p;
+        },
+        out, aq, alpha, FP4_GEMM_SCALE, m, n, k, group_m, sc);
 }
-extern "C" __global__ __launch_bounds__(256, 1) void fe_gemm_nvfp4_swiglu(FP4_SWIGLU_PARAMS) {
+extern "C" __global__ __launch_bounds__(512, 2) void fe_gemm_nvfp4_swiglu(FP4_SWIGLU_PARAMS) {
     gemm_nvfp4_swiglu_kernel<false>(aq, w, sw, alpha, m, n, k, group_m, w_snt, w_skt, w_sr, s_snt, s_skt, s_sr, sc, q_codes, q_sf,
                                     q_aq, qg);
 }
-extern "C" __global__ __launch_bounds__(256, 1) void fe_gemm_nvfp4_swiglu_sk(FP4_SWIGLU_PARAMS) {
+extern "C" __global__ __launch_bounds__(512, 2) void fe_gemm_nvfp4_swiglu_sk(FP4_SWIGLU_PARAMS) {
     gemm_nvfp4_swiglu_kernel<true>(aq, w, sw, alpha, m, n, k, group_m, w_snt, w_skt, w_sr, s_snt, s_skt, s_sr, sc, q_codes, q_sf,
                                    q_aq, qg);
 }
@@ -493,7 +523,16 @@ extern "C" __global__ __launch_bounds__(256) void fe_gemm_nvfp4_swiglu_reduce(co
                                                                               uint32_t splits, uint8_t* q_codes, uint8_t* q_sf,
                                                                               _Float16* q_aq, float qg) {
     FpOut out = {nullptr, nullptr, 0, q_codes, q_sf, q_aq, qg};
-    fp_reduce_body<true>(out, part, alpha, FP4_OPERAND_SCALE, m, n, group_m, full_tiles, splits);
+    fp_reduce_body<FpTile, true>(out, part, alpha, FP4_GEMM_SCALE, m, n, group_m, full_tiles, splits);
+}
+
+// The same for the GEMM over FP8 codes.
+extern "C" __global__ __launch_bounds__(256) void fe_gemm_fp8_codes_reduce(uint16_t* c, const float* part, const float* alpha,
+                                                                           const uint16_t* res, uint32_t m, uint32_t n,
+                                                                           uint32_t ldc, uint32_t group_m, uint32_t full_tiles,
+                                                                           uint32_t splits, float scale) {
+    FpOut out = {c, res, ldc, nullptr, nullptr, nullptr, 0.f};
+    fp_reduce_body<Fp8Tile, false>(out, part, alpha, scale, m, n, group_m, full_tiles, splits);
 }
 
 // FP8: the 64 codes of row r = 128 nt + i, k tile kt are at w + nt * w_snt + kt * w_skt + i * w_sr; both fp16 expansions
@@ -503,97 +542,63 @@ extern "C" __global__ __launch_bounds__(256) void fe_gemm_nvfp4_swiglu_reduce(co
         uint32_t ldc, uint32_t group_m, uint32_t w_snt, uint32_t w_skt, uint32_t w_sr, GemmSched sc
 template <bool SK>
 __device__ __forceinline__ void gemm_fp8_kernel(FP8_GEMM_PARAMS) {
-    const uint32_t nts = n / 128, tid = threadIdx.x;
     FpOut out = {c, res, ldc, nullptr, nullptr, nullptr, 0.f};
     fp_gemm_body<false, SK>(
         [&](uint32_t tn) {
-            uint32_t nt = 2 * tn + (tid >> 7);
-            nt = nt < nts ? nt : nts - 1;
-            Fp8Producer prod;
-            prod.row = tid;
-            prod.w = w + (size_t)nt * w_snt + (size_t)(tid & 127) * w_sr;
-            prod.w_skt = w_skt;
-            return prod;
+            Fp8Packed<FpTile> p;
+            p.setup(w, n, k, tn * FpTile::BN, w_snt, w_skt, w_sr);
+            return p;
         },
         out, aq, alpha, 1.0f, m, n, k, group_m, sc);
 }
-extern "C" __global__ __launch_bounds__(256, 1) void fe_gemm_fp8(FP8_GEMM_PARAMS) {
+extern "C" __global__ __launch_bounds__(512, 2) void fe_gemm_fp8(FP8_GEMM_PARAMS) {
     gemm_fp8_kernel<false>(c, aq, w, alpha, res, m, n, k, ldc, group_m, w_snt, w_skt, w_sr, sc);
 }
-extern "C" __global__ __launch_bounds__(256, 1) void fe_gemm_fp8_sk(FP8_GEMM_PARAMS) {
+extern "C" __global__ __launch_bounds__(512, 2) void fe_gemm_fp8_sk(FP8_GEMM_PARAMS) {
     gemm_fp8_kernel<true>(c, aq, w, alpha, res, m, n, k, ldc, group_m, w_snt, w_skt, w_sr, sc);
 }
 
 // The same linear on the 8-bit matrix instruction: activations are the quantizer's e4m3 codes [M][K], weights stay codes
 // in LDS, a k tile is 128 wide (two of the 64-wide weight tiles of the layout above). Same products (an e4m3 x e4m3
 // product is exact in f32) and f32 sums as fe_gemm_fp8, at twice the MFMA rate and half the LDS bytes per flop.
-struct Fp8CodeProducer {
-    const uint8_t* w[2];  // the two 128-row weight tiles + this thread's (row, chunk) offset
-    uint32_t w_skt, w_sr, st;
-    struct Raw {
-        u32x4 c[2][4];
-    };
-    static constexpr int kStoreValu = 0;
-    static constexpr bool kQuarters = false;
-    // thread t: 16-byte chunk t & 7 of rows (t >> 3) + 32 j of each 128-row half; chunks 0..3 come from 64-wide weight
-    // tile 2 kt, chunks 4..7 from 2 kt + 1
-    __device__ __forceinline__ void load(uint32_t kt, Raw& r, int half) const {
-#pragma unroll
-        for (int b = 0; b < 2; b++) {
-            if (b != half) continue;
-            const uint8_t* p = w[b] + (size_t)(2 * kt) * w_skt;
-#pragma unroll
-            for (int j = 0; j < 4; j++) r.c[b][j] = *(const u32x4*)(p + (size_t)(32 * j) * w_sr);
-        }
-    }
-    __device__ __forceinline__ void store(const Raw& r, unsigned char* Bs, int part) const {
-#pragma unroll
-        for (int b = 0; b < 2; b++) {
-            if (b != part) continue;
-#pragma unroll
-            for (int j = 0; j < 4; j++) *(u32x4*)(Bs + 16384 * b + st + 4096 * j) = r.c[b][j];
-        }
-    }
-};
-
 #define FP8C_GEMM_PARAMS                                                                                                   \
     uint16_t *c, const uint8_t *aq, const uint8_t *w, const float *alpha, const uint16_t *res, uint32_t m, uint32_t n, uint32_t k, \
         uint32_t ldc, uint32_t group_m, uint32_t w_snt, uint32_t w_skt, uint32_t w_sr, GemmSched sc
 template <bool SK>
 __device__ __forceinline__ void gemm_fp8_codes_kernel(FP8C_GEMM_PARAMS) {
-    extern __shared__ __attribute__((aligned(16))) unsigned char lds[];
-    const uint32_t nts = n / 128, tid = threadIdx.x, wave = tid >> 6, wm = wave >> 1, wn = wave & 1;
+    typedef Fp8Tile T;
+    extern __shared__ __attribute__((aligned(1024))) unsigned char lds[];
+    const uint32_t nts = n / 128, lane = threadIdx.x & 63, wave = threadIdx.x >> 6, wm = wave / T::WN, wn = wave % T::WN;
     FpOut out = {c, res, ldc, nullptr, nullptr, nullptr, 0.f};
-    gemm_schedule<SK>(
-        sc, (m + GM_BM - 1) / GM_BM, (nts + 1) / 2, group_m, k / 128, lds,
-        [&](uint32_t tm, uint32_t tn, uint32_t kt0, uint32_t ktn, f32x16(&acc)[4][4]) {
-            Fp8CodeProducer prod;
-            const uint32_t chunk = tid & 7, row = tid >> 3;
+    g8_schedule<T, SK>(
+        sc, (m + T::BM - 1) / T::BM, (nts + 1) / 2, group_m, k / 128, lds,
+        [&](uint32_t tm, uint32_t tn, uint32_t kt0, uint32_t ktn, f32x4(&acc)[T::TM][T::TN]) {
+            // a k tile of 128 codes is two of the layout's 64-wide ones: chunks 0..3 of a row from the first, 4..7 from the second
+            G8Dense<T> wo;
+            wo.rs = g8_rsrc(w, n * k), wo.kstep = 2 * w_skt;
 #pragma unroll
-            for (int b = 0; b < 2; b++) {
-                uint32_t nt = 2 * tn + b;
-                nt = nt < nts ? nt : nts - 1;  // an odd count of 128-row tiles: the last program copies its first tile twice
-                prod.w[b] = w + (size_t)nt * w_snt + (size_t)(chunk >> 2) * w_skt + (size_t)row * w_sr + (chunk & 3) * 16;
+            for (int j = 0; j < G8Dense<T>::LOADS; j++) {
+                const uint32_t r = 8 * (wave + 8 * j) + (lane >> 3), ch = (lane & 7) ^ (r & 7);
+                uint32_t nt = 2 * tn + r / 128;
+                nt = nt < nts ? nt : nts - 1;  // an odd count of 128-row tiles: the last program reads its first tile twice
+                wo.voff[j] = nt * w_snt + (ch >> 2) * w_skt + (r & 127) * w_sr + (ch & 3) * 16;
             }
-            prod.w_skt = w_skt, prod.w_sr = w_sr, prod.st = gm_swz(row, chunk);
-            gemm_mainloop_f8(aq, k, m, kt0, ktn, tm * GM_BM, prod, lds, acc);
+            g8_mainloop_f8<T, 2, 3>(aq, k, m, kt0, ktn, tm * T::BM, wo, lds, acc);
         },
-        [&](uint32_t tm, uint32_t tn, f32x16(&acc)[4][4]) {
-            const uint32_t m0 = tm * GM_BM, colb = tn * GM_BN + wn * 128;
+        [&](uint32_t tm, uint32_t tn, f32x4(&acc)[T::TM][T::TN]) {
+            const uint32_t m0 = tm * T::BM + wm * 16 * T::TM, colb = tn * T::BN + wn * 16 * T::TN;
             if (colb >= n) return;
-            const uint32_t col = colb + 4 * (tid & 31);
+            const uint32_t col = colb + 4 * (lane % (4 * T::TN));
             const f32x4 al = *(const f32x4*)(alpha + col);
-            gemm_epilogue(
-                acc, lds, [](float (&)[4][4], uint32_t) {},
-                [&](uint32_t r, uint32_t l32, float (&v)[4]) {
-                    fp_store_piece<false>(out, v, al, l32, m0 + wm * 128 + r, m, col, n);
-                });
+            g8_epilogue<T>(
+                acc, lds, [](auto&, uint32_t) {},
+                [&](uint32_t r, uint32_t lc, float (&v)[4]) { fp_store_piece<false>(out, v, al, lc, m0 + r, m, col, n); });
         });
 }
-extern "C" __global__ __launch_bounds__(256, 1) void fe_gemm_fp8_codes(FP8C_GEMM_PARAMS) {
+extern "C" __global__ __launch_bounds__(512, 2) void fe_gemm_fp8_codes(FP8C_GEMM_PARAMS) {
     gemm_fp8_codes_kernel<false>(c, aq, w, alpha, res, m, n, k, ldc, group_m, w_snt, w_skt, w_sr, sc);
 }
-extern "C" __global__ __launch_bounds__(256, 1) void fe_gemm_fp8_codes_sk(FP8C_GEMM_PARAMS) {
+extern "C" __global__ __launch_bounds__(512, 2) void fe_gemm_fp8_codes_sk(FP8C_GEMM_PARAMS) {
     gemm_fp8_codes_kernel<true>(c, aq, w, alpha, res, m, n, k, ldc, group_m, w_snt, w_skt, w_sr, sc);
 }
 
