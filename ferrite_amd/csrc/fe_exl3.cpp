@@ -25,7 +25,8 @@ constexpr uint32_t kGroupMax = 4;              // FE_EXL3_GROUP_MAX: linears of 
 // buffer holds 32 rows at a time
 constexpr uint32_t kJobLdsBudget = 53 * 1024;
 constexpr uint32_t kRedPitch = 132;            // GEMV_RED_PITCH
-constexpr uint32_t kGemmLds = 2 * (256 + 256) * 64 * 2;  // two k tiles of A and W, 256 rows each; the epilogue reuses it
+constexpr uint32_t kGemmLds = 160 * 1024;      // k tiles of A and W in flight; the epilogue reuses it
+constexpr uint32_t kGemmThreads = 512;
 constexpr uint32_t kCuLds = 160 * 1024;        // LDS of a CU
 constexpr size_t kChainStride = 64;            // FE_CHAIN_STRIDE: u32 words between two ready words of the one-launch MLP
 
@@ -554,11 +555,11 @@ static int launch_gemm(const fe_exl3_linear *l, fe_stream_t s, fe_devptr_t xh, f
         if (!kept) FE_TRY(launch_decode(l, s, hat));
         group = 0;  // the raster that deals column tiles to the XCDs: each decoded weight panel goes through one L2
         void *args[] = {&xh, &hat, &svh, &y, &n, &k, &rows, &mode, &group, &sch.args};
-        FE_TRY(fe_hip_launch(sch.stream_k ? kern->gemm_hat_sk : kern->gemm_hat, sch.programs, 1, 1, 256, 1, 1, kGemmLds, s, args));
+        FE_TRY(fe_hip_launch(sch.stream_k ? kern->gemm_hat_sk : kern->gemm_hat, sch.programs, 1, 1, kGemmThreads, 1, 1, kGemmLds, s, args));
     } else {
         if (sch.stream_k) group = 1;  // column tiles fastest: the programs that are in step share a panel of inputs
         void *args[] = {&xh, &tr, &svh, &y, &n, &k, &rows, &mode, &stride_k, &stride_nb, &group, &sch.args};
-        FE_TRY(fe_hip_launch((sch.stream_k ? kern->gemm_sk : kern->gemm)[bits_slot(l->bits)], sch.programs, 1, 1, 256, 1, 1, kGemmLds, s, args));
+        FE_TRY(fe_hip_launch((sch.stream_k ? kern->gemm_sk : kern->gemm)[bits_slot(l->bits)], sch.programs, 1, 1, kGemmThreads, 1, 1, kGemmLds, s, args));
     }
     if (sch.stream_k || !sch.split.cut()) return 0;
     uint32_t full = sch.split.full, splits = sch.split.splits;

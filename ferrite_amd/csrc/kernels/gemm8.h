@@ -361,6 +361,118 @@ __device__ __forceinline__ void g8_mainloop_packed(const _Float16* a, uint32_t l
     __syncthreads();
 }
 
+// The loop for a weight operand that is decoded by more arithmetic than a wavefront should repeat: every weight of the tile is
+// decoded once, by the thread that has its words, and written into LDS as 16-bit rows (as G8Dense's). The packed words of a k tile go
+// into LDS as they are (NR stages); a thread reads its words of tile t + 2 in slice 1 of tile t, decodes and writes their
+// first half there and their second half in slice 0 of tile t + 1, always into the weight stage the barrier before has freed.
+// Two stages of A, two of decoded weights.
+// W: RAW_STAGE bytes and LOADS loads a packed stage, issue(kt, dst of the stage, j, wave), Words, read(stage in LDS) -> Words,
+// store(words, half 0 or 1, weight stage).
+template <class T, int NR, class W>
+__device__ __forceinline__ void g8_mainloop_decode(const _Float16* a, uint32_t lda, uint32_t m, uint32_t kt0, uint32_t ktiles, uint32_t m0,
+                                                   const W& wo, unsigned char* lds, f32x4 (&acc)[T::TM][T::TN]) {
+    constexpr int TM = T::TM, TN = T::TN, LA = T::BM / 64, LR = W::LOADS, A_STAGE = T::BM * 128, W_STAGE = T::BN * 128;
+    constexpr int W_AT = 2 * A_STAGE, R_AT = W_AT + 2 * W_STAGE;
+    static_assert(R_AT + NR * W::RAW_STAGE <= 160 * 1024, "LDS");
+    static_assert(NR == 2 || NR == 3, "the waits below");
+    const uint32_t lane = threadIdx.x & 63, wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
+    const uint32_t wm = wave / T::WN, wn = wave % T::WN;
+    const u32x4 ra = g8_rsrc(a, m * lda * 2);
+    uint32_t va[LA];
+#pragma unroll
+    for (int j = 0; j < LA; j++) {
+        const uint32_t r = 8 * (wave + 8 * j) + (lane >> 3), g = m0 + r < m ? m0 + r : m - 1;
+        va[j] = (g * lda + ((lane & 7) ^ (r & 7)) * 8) * 2;
+    }
+    const uint32_t base = g8_lds_addr(lds);
+    auto ktc = [&](uint32_t kt) { return kt0 + (kt < ktiles ? kt : ktiles - 1); };
+    auto load_a = [&](uint32_t kt, uint32_t st, int j) { g8_load_lds16(ra, base + wave * 1024 + st * A_STAGE + j * 8192, va[j], ktc(kt) * 128); };
+    auto load_r = [&](uint32_t kt, uint32_t st, int j) { wo.issue(ktc(kt), base + R_AT + st * W::RAW_STAGE, j, wave); };
+    auto next = [](uint32_t st, uint32_t n) { return st + 1 == n ? 0u : st + 1; };
+
+    const uint32_t fr = lane & 15, fc = lane >> 4;
+    uint32_t foff[2];
+#pragma unroll
+    for (int kk = 0; kk < 2; kk++) foff[kk] = fr * 128 + (((4 * kk + fc) ^ (fr & 7)) << 4);
+    const unsigned char* pa = lds + wm * TM * 2048;
+    const unsigned char* pw = lds + W_AT + wn * TN * 2048;
+    f16x8 fa[2][TM], fw[TN];
+    auto rd_a = [&](int set, uint32_t st, int kk, int i) { fa[set][i] = *(const f16x8*)(pa + st * A_STAGE + 2048 * i + foff[kk]); };
+    auto rd_w = [&](uint32_t st, int kk, int j) { fw[j] = *(const f16x8*)(pw + st * W_STAGE + 2048 * j + foff[kk]); };
+    auto words = [&](uint32_t st) { return wo.read(lds + R_AT + st * W::RAW_STAGE); };
+    auto put = [&](const typename W::Words& w, int half, uint32_t st) { wo.store(w, half, lds + W_AT + st * W_STAGE); };
+#pragma unroll
+    for (int i = 0; i < TM; i++)
+#pragma unroll
+        for (int j = 0; j < TN; j++) acc[i][j] = (f32x4){0.f, 0.f, 0.f, 0.f};
+
+#pragma unroll
+    for (int t = 0; t < NR; t++)
+#pragma unroll
+        for (int j = 0; j < LR; j++) load_r(t, t, j);
+#pragma unroll
+    for (int t = 0; t < 2; t++)
+#pragma unroll
+        for (int j = 0; j < LA; j++) load_a(t, t, j);
+    g8_loads_wait<2 * LA>();  // the packed tiles
+    g8_barrier();
+    typename W::Words w = words(0);
+    put(w, 0, 0);
+    put(w, 1, 0);
+    w = words(1);
+    put(w, 0, 1);
+    g8_loads_wait<LA>();  // A of tile 0
+    g8_barrier();
+#pragma unroll
+    for (int j = 0; j < LR; j++) load_r(NR, 0, j);
+#pragma unroll
+    for (int i = 0; i < TM; i++) rd_a(0, 0, 0, i);
+#pragma unroll
+    for (int j = 0; j < TN; j++) rd_w(0, 0, j);
+
+    uint32_t sr = NR == 2 ? 0 : 2, sr_in = 1;  // the packed stage of tile kt + 2; the one that slice 1 of tile kt fills (tile kt + 1 + NR)
+    for (uint32_t kt = 0; kt < ktiles; kt++) {
+        const uint32_t s = kt & 1;
+#pragma unroll
+        for (int kk = 0; kk < 2; kk++) {
+            if (kk == 1) {
+                g8_loads_wait<(NR == 3 ? LR : 0)>();
+                g8_barrier();
+            }
+            const uint32_t st = kk ? s ^ 1 : s;
+#pragma unroll
+            for (int j = 0; j < TN; j++) {
+#pragma unroll
+                for (int i = 0; i < TM; i++) {
+                    const int ii = j & 1 ? TM - 1 - i : i;
+                    acc[ii][j] = __builtin_amdgcn_mfma_f32_16x16x32_f16(fw[j], fa[kk][ii], acc[ii][j], 0, 0, 0);
+                }
+                rd_w(st, kk ^ 1, j);
+                constexpr int PER = (2 * TM + TN - 1) / TN;
+#pragma unroll
+                for (int q = 0; q < PER; q++)
+                    if (j * PER + q < TM) rd_a(kk ^ 1, st, kk ^ 1, j * PER + q);
+                if (kk == 0) {  // second half of tile kt + 1
+                    if (j == 1) put(w, 1, s ^ 1);
+                } else {  // words and first half of tile kt + 2
+                    if (j == 0) w = words(sr);
+                    if (j == TN - 2) put(w, 0, s);
+#pragma unroll
+                    for (int q = j * LA / TN; q < (j + 1) * LA / TN; q++) load_a(kt + 2, s, q);
+                    if (j == TN - 1) {
+#pragma unroll
+                        for (int q = 0; q < LR; q++) load_r(kt + 1 + NR, sr_in, q);
+                    }
+                }
+                __builtin_amdgcn_sched_barrier(0);
+            }
+        }
+        sr = next(sr, NR), sr_in = next(sr_in, NR);
+    }
+    asm volatile("s_waitcnt vmcnt(0)" ::: "memory");
+    __syncthreads();
+}
+
 // The loop for 8-bit operands (e4m3 codes on both sides) on v_mfma_f32_16x16x128_f8f6f4: a k tile is 128 codes, so rows are again
 // 128 bytes and stages, chunk positions and loads are those of g8_mainloop; a lane's operand of the one MFMA step of a k
 // tile is chunks fc and 4 + fc of its row (both operands alike: k is a summation index only). A fragment takes 8 registers,

@@ -8,7 +8,7 @@
 // (crates/fe-exl3/src/cpu.rs:25-43, kernels/k-exl3/src/util.rs:76-85).
 #include <type_traits>
 
-#include "gemm_core.h"
+#include "gemm8.h"
 
 // ---- the mul1 codebook ------------------------------------------------------------------------------------------
 
@@ -1039,68 +1039,84 @@ GEMVB_FAMILY(8)
 
 // ---- prefill GEMM ----------------------------------------------------------------------------------------------------
 
-// Weight tile producer of the prefill GEMM: a 64-wide k tile of a 128-column block is 4 k steps x 8 tiles; wavefront w
-// takes k step w, lane L tile L >> 3, rows n = (L & 7) and (L & 7) + 8 of it (the same run of words as in the GEMV),
-// in both 128-column blocks of the 256-column output tile.
+typedef G8Tile<4, 2, 4, 8> Exl3Tile;  // 256 x 256; a wavefront's 128 columns are one Hadamard block
+
+// Weight operand of the prefill GEMM: a 64-wide k tile of a 128-column block is 4 k steps x 8 tiles; wavefront w takes block
+// w >> 2 of the 256-column output tile and k step w & 3, lane L tile L >> 3, rows n = (L & 7) and (L & 7) + 8 of it (the same
+// run of words as in the GEMV). A packed stage is [2 blocks][4 k steps][8 tiles][8 BITS words]: 2 BITS pieces of 1 KB.
 template <int BITS>
-struct Exl3Producer {
-    const uint32_t* base[2];  // the two blocks' trellis + this lane's tile
-    uint32_t stride_k, run_off, prev_off, brow, ks;
-    struct Raw {
-        LaneWords<BITS> w[2];
-    };
-    static constexpr int kStoreValu = 240;  // about the VALU instructions of the four quarters together
-    static constexpr bool kQuarters = true;  // the main loop spreads the decode over its four slices
-    __device__ __forceinline__ void load(uint32_t kt, Raw& r, int half) const {
+struct Exl3Packed {
+    static constexpr int RAW_STAGE = 2048 * BITS, LOADS = (2 * BITS + 7) / 8;
+    typedef LaneWords<BITS> Words;
+    u32x4 rs;
+    uint32_t voff[LOADS], step;
+    __device__ __forceinline__ void setup(const uint32_t* trellis, uint32_t n, uint32_t k, uint32_t tn, uint32_t stride_k, uint32_t stride_nb) {
+        const uint32_t lane = threadIdx.x & 63, wave = threadIdx.x >> 6, nbs = n / 128;
+        rs = g8_rsrc(trellis, (k / 16) * (n / 16) * 32 * BITS);
+        step = 16 * stride_k;
 #pragma unroll
-        for (int b = 0; b < 2; b++) {
-            if (b != half) continue;
-            const uint32_t* p = base[b] + (size_t)(kt * 4 + ks) * stride_k;
-            r.w[b] = load_lane_words<BITS>(p + run_off, p + prev_off);
+        for (int j = 0; j < LOADS; j++) {
+            const uint32_t at = (wave + 8 * j) % (2 * BITS) * 1024 + lane * 16;  // (fewer pieces than wavefronts: some are moved twice)
+            const uint32_t ks = at / (256 * BITS) % 4;
+            uint32_t nb = 2 * tn + at / (1024 * BITS);
+            nb = nb < nbs ? nb : nbs - 1;  // an odd block count: the last tile decodes its first block twice
+            voff[j] = 4 * (nb * stride_nb + ks * stride_k) + at % (256 * BITS);
         }
     }
-    // quarter q: row half q & 1 (rows n = brow + 8 (q & 1) of the lane's tile) of column block q >> 1
-    __device__ __forceinline__ void store_quarter(const Raw& r, unsigned char* Bs, int q) const {
+    __device__ __forceinline__ void issue(uint32_t kt, uint32_t dst, int j, uint32_t wave) const {
+        g8_load_lds16(rs, dst + (wave + 8 * j) % (2 * BITS) * 1024, voff[j], kt * step);
+    }
+    __device__ __forceinline__ Words read(const unsigned char* st) const {
+        const uint32_t* p = (const uint32_t*)st + (threadIdx.x >> 3) * (8 * BITS) + (threadIdx.x & 7) * BITS;
+        Words w;
+        if constexpr (BITS % 4 == 0) {
 #pragma unroll
-        for (int b = 0; b < 2; b++)
-#pragma unroll
-            for (int h = 0; h < 2; h++) {
-                if (2 * b + h != q) continue;
-                f16x8 op[2];
-                decode_lane_half<BITS>(r.w[b], h, op);
-#pragma unroll
-                for (int kh = 0; kh < 2; kh++) *(f16x8*)(Bs + gm_swz(128 * b + brow + 8 * h, 2 * ks + kh)) = op[kh];
+            for (int i = 0; i < BITS; i += 4) {
+                const u32x4 t = *(const u32x4*)(p + i);
+                w.w[i + 1] = t[0], w.w[i + 2] = t[1], w.w[i + 3] = t[2], w.w[i + 4] = t[3];
             }
+        } else {
+#pragma unroll
+            for (int i = 0; i < BITS; i++) w.w[i + 1] = p[i];
+        }
+        w.w[0] = 0;
+        return w;
+    }
+    // row half `half` (rows n = brow + 8 half of the lane's tile)
+    __device__ __forceinline__ void store(Words w, int half, unsigned char* ws) const {
+        const uint32_t lane = threadIdx.x & 63, wave = threadIdx.x >> 6, row = 128 * (wave >> 2) + (lane >> 3) * 16 + (lane & 7) + 8 * half;
+        f16x8 op[2];
+        w.w[0] = lane_prev_word(w.w[BITS]);
+        decode_lane_half<BITS>(w, half, op);
+#pragma unroll
+        for (int kh = 0; kh < 2; kh++) *(f16x8*)(ws + row * 128 + (((2 * (wave & 3) + kh) ^ (row & 7)) << 4)) = op[kh];
     }
 };
 
 // y[m][n] (+)= H(xh @ W_hat) * svh / sqrt(128) for prefill-sized m: xh fp16 [m][k] (rotated inputs), 256 x 256 output
 // tiles; a wavefront's 128 columns are exactly one Hadamard block, so the output rotation is local to the wavefront.
-// Tiles = ceil(m / 256) * ceil(n / 256) (grouped raster), spread over the grid as sc says (gemm_schedule): one piece a
-// program, the cut tiles finished by exl3_gemm_reduce, or stream-K. 256 threads, dynamic LDS GM_LDS_TILES (the epilogue
-// reuses it). make_producer(tn) builds the weight producer of 256-column tile tn.
-template <bool SK, class MakeProducer>
-__device__ __forceinline__ void exl3_gemm_tile(const _Float16* __restrict__ xh, const uint16_t* __restrict__ svh, void* y,
-                                               uint32_t n, uint32_t k, uint32_t m, uint32_t y_mode, uint32_t group_m,
-                                               const GemmSched& sched, MakeProducer make_producer) {
-    extern __shared__ __attribute__((aligned(16))) unsigned char lds[];
+// Tiles = ceil(m / 256) * ceil(n / 256) (grouped raster), spread over the grid as sc says (g8_schedule): one piece a
+// program, the cut tiles finished by exl3_gemm_reduce, or stream-K. 512 threads, dynamic LDS 160 KB (the epilogue
+// reuses it). loop(tm, tn, kt0, ktn, lds, acc) is a pass of the main loop.
+template <bool SK, class Loop>
+__device__ __forceinline__ void exl3_gemm_tile(const uint16_t* __restrict__ svh, void* y, uint32_t n, uint32_t k, uint32_t m,
+                                               uint32_t y_mode, uint32_t group_m, const GemmSched& sched, Loop loop) {
+    typedef Exl3Tile T;
+    extern __shared__ __attribute__((aligned(1024))) unsigned char lds[];
     const uint32_t nbs = n / 128;
-    const uint32_t tid = threadIdx.x, lane = tid & 63, wave = tid >> 6, wm = wave >> 1, wn = wave & 1;
-    gemm_schedule<SK>(
-        sched, (m + GM_BM - 1) / GM_BM, (nbs + 1) / 2, group_m, k / GM_BK, lds,
-        [&](uint32_t tm, uint32_t tn, uint32_t kt0, uint32_t ktn, f32x16(&acc)[4][4]) {
-            auto prod = make_producer(tn);
-            gemm_mainloop(xh, k, m, kt0, ktn, tm * GM_BM, prod, lds, acc);
-        },
-        [&](uint32_t tm, uint32_t tn, f32x16(&acc)[4][4]) {
-            const uint32_t m0 = tm * GM_BM, nb = 2 * tn + wn;
+    const uint32_t lane = threadIdx.x & 63, wave = threadIdx.x >> 6, wm = wave / T::WN, wn = wave % T::WN;
+    g8_schedule<T, SK>(
+        sched, (m + T::BM - 1) / T::BM, (nbs + 1) / 2, group_m, k / G8_BK, lds,
+        [&](uint32_t tm, uint32_t tn, uint32_t kt0, uint32_t ktn, f32x4(&acc)[T::TM][T::TN]) { loop(tm, tn, kt0, ktn, lds, acc); },
+        [&](uint32_t tm, uint32_t tn, f32x4(&acc)[T::TM][T::TN]) {
+            const uint32_t m0 = tm * T::BM + wm * 16 * T::TM, nb = 2 * tn + wn;
             if (nb >= nbs) return;
             const uint32_t col = nb * 128 + 4 * (lane & 31);
             const f32x4 sc = row_scales(svh, col);
             // one copy of the epilogue per output mode, so that the row loop has no mode branches
             auto run = [&](auto mode_tag) {
                 constexpr uint32_t MODE = decltype(mode_tag)::value;
-                gemm_epilogue(
+                g8_epilogue<T>(
                     acc, lds,
                     [&](float (&v)[4][4], uint32_t l32) {
                         fwht128_half_wave_rows(v, l32);
@@ -1110,8 +1126,7 @@ __device__ __forceinline__ void exl3_gemm_tile(const _Float16* __restrict__ xh, 
                             for (int e = 0; e < 4; e++) v[u][e] = v[u][e] * FE_HAD_SCALE * sc[e];  // finish_row's products
                     },
                     [&](uint32_t row, uint32_t, float (&v)[4]) {
-                        uint32_t grow = m0 + wm * 128 + row;
-                        if (grow < m) store4(y, MODE, (size_t)grow * n + col, v);
+                        if (m0 + row < m) store4(y, MODE, (size_t)(m0 + row) * n + col, v);
                     });
             };
             if (y_mode == 0)
@@ -1131,21 +1146,12 @@ __device__ __forceinline__ void exl3_gemm_body(const _Float16* __restrict__ xh, 
                                                const uint16_t* __restrict__ svh, void* y, uint32_t n, uint32_t k, uint32_t m,
                                                uint32_t y_mode, uint32_t stride_k, uint32_t stride_nb, uint32_t group_m,
                                                const GemmSched& sched) {
-    exl3_gemm_tile<SK>(xh, svh, y, n, k, m, y_mode, group_m, sched, [&](uint32_t tn) {
-        constexpr uint32_t tw = 8 * BITS;
-        const uint32_t lane = threadIdx.x & 63, nbs = n / 128;
-        Exl3Producer<BITS> prod;
-        uint32_t tj = lane >> 3, q = lane & 7;
-        uint32_t nb1 = 2 * tn + 1 < nbs ? 2 * tn + 1 : 2 * tn;  // an odd block count: the last tile decodes block 2 tn twice
-        prod.base[0] = trellis + (size_t)(2 * tn) * stride_nb + tj * tw;
-        prod.base[1] = trellis + (size_t)nb1 * stride_nb + tj * tw;
-        prod.stride_k = stride_k;
-        prod.run_off = q * BITS;
-        prod.prev_off = (q * BITS + tw - 1) % tw;
-        prod.brow = tj * 16 + q;
-        prod.ks = threadIdx.x >> 6;
-        return prod;
-    });
+    exl3_gemm_tile<SK>(svh, y, n, k, m, y_mode, group_m, sched,
+                       [&](uint32_t tm, uint32_t tn, uint32_t kt0, uint32_t ktn, unsigned char* lds, f32x4(&acc)[Exl3Tile::TM][Exl3Tile::TN]) {
+                           Exl3Packed<BITS> w;
+                           w.setup(trellis, n, k, tn, stride_k, stride_nb);
+                           g8_mainloop_decode<Exl3Tile, BITS <= 5 ? 3 : 2>(xh, k, m, kt0, ktn, tm * Exl3Tile::BM, w, lds, acc);
+                       });
 }
 
 // ---- prefill over decoded weights -----------------------------------------------------------------------------------
@@ -1192,50 +1198,32 @@ __device__ __forceinline__ void exl3_hat_tiles_body(const uint32_t* __restrict__
     }
 }
 
-// Weight producer over `hat`: a k tile of the 256-column tile is one 32 KB block, copied as it is; thread t moves chunks
-// t + 256 j (j < 4) of each 16 KB half.
-struct HatProducer {
-    const unsigned char* base;  // the tile's blocks + 16 * thread
-    struct Raw {
-        u32x4 c[2][4];
-    };
-    static constexpr int kStoreValu = 0;
-    static constexpr bool kQuarters = false;
-    __device__ __forceinline__ void load(uint32_t kt, Raw& r, int half) const {
-#pragma unroll
-        for (int b = 0; b < 2; b++) {
-            if (b != half) continue;
-            const unsigned char* p = base + (size_t)kt * GM_B_BYTES + b * (GM_B_BYTES / 2);
-#pragma unroll
-            for (int j = 0; j < 4; j++) r.c[b][j] = *(const u32x4*)(p + 4096 * j);
-        }
-    }
-    __device__ __forceinline__ void store(const Raw& r, unsigned char* Bs, int part) const {
-#pragma unroll
-        for (int b = 0; b < 2; b++) {
-            if (b != part) continue;
-#pragma unroll
-            for (int j = 0; j < 4; j++) *(u32x4*)(Bs + b * (GM_B_BYTES / 2) + 16 * threadIdx.x + 4096 * j) = r.c[b][j];
-        }
-    }
-};
-
 // (every GEMM kernel comes as NAME, one piece a program, and NAME_sk, stream-K, with the same parameters)
 #define HAT_GEMM_PARAMS                                                                                                  \
     const _Float16 *xh, const unsigned char *hat, const uint16_t *svh, void *y, uint32_t n, uint32_t k, uint32_t m, uint32_t y_mode, \
         uint32_t group_m, GemmSched sched
 template <bool SK>
 __device__ __forceinline__ void exl3_gemm_hat_kernel(HAT_GEMM_PARAMS) {
-    exl3_gemm_tile<SK>(xh, svh, y, n, k, m, y_mode, group_m, sched, [&](uint32_t tn) {
-        HatProducer prod;
-        prod.base = hat + (size_t)tn * (k / GM_BK) * GM_B_BYTES + 16 * threadIdx.x;
-        return prod;
-    });
+    typedef Exl3Tile T;
+    exl3_gemm_tile<SK>(svh, y, n, k, m, y_mode, group_m, sched,
+                       [&](uint32_t tm, uint32_t tn, uint32_t kt0, uint32_t ktn, unsigned char* lds, f32x4(&acc)[T::TM][T::TN]) {
+                           // the tile's blocks of 32 KB; a row's chunks lie where gm_swz puts them: the core's position, its low
+                           // bit flipped in every second group of 8 rows
+                           const uint32_t lane = threadIdx.x & 63, wave = threadIdx.x >> 6, bytes = (k / G8_BK) * GM_B_BYTES;
+                           G8Dense<T> w;
+                           w.rs = g8_rsrc(hat + (size_t)tn * bytes, bytes), w.kstep = GM_B_BYTES;
+#pragma unroll
+                           for (int j = 0; j < G8Dense<T>::LOADS; j++) {
+                               const uint32_t r = 8 * (wave + 8 * j) + (lane >> 3);
+                               w.voff[j] = r * 128 + (((lane & 7) ^ ((r >> 3) & 1)) << 4);
+                           }
+                           g8_mainloop<T, 2, 3, false>(xh, k, m, kt0, ktn, tm * T::BM, w, lds, acc);
+                       });
 }
-extern "C" __global__ __launch_bounds__(256, 1) void exl3_gemm_hat(HAT_GEMM_PARAMS) {
+extern "C" __global__ __launch_bounds__(512, 2) void exl3_gemm_hat(HAT_GEMM_PARAMS) {
     exl3_gemm_hat_kernel<false>(xh, hat, svh, y, n, k, m, y_mode, group_m, sched);
 }
-extern "C" __global__ __launch_bounds__(256, 1) void exl3_gemm_hat_sk(HAT_GEMM_PARAMS) {
+extern "C" __global__ __launch_bounds__(512, 2) void exl3_gemm_hat_sk(HAT_GEMM_PARAMS) {
     exl3_gemm_hat_kernel<true>(xh, hat, svh, y, n, k, m, y_mode, group_m, sched);
 }
 
@@ -1244,17 +1232,18 @@ extern "C" __global__ __launch_bounds__(256, 1) void exl3_gemm_hat_sk(HAT_GEMM_P
 extern "C" __global__ __launch_bounds__(256) void exl3_gemm_reduce(const float* part, const uint16_t* svh, void* y, uint32_t n,
                                                                    uint32_t m, uint32_t y_mode, uint32_t group_m,
                                                                    uint32_t full_tiles, uint32_t splits) {
+    typedef Exl3Tile T;
     const uint32_t nbs = n / 128;
-    gemm_reduce_rows(part, splits, [&](uint32_t t, uint32_t row, uint32_t cb, uint32_t l32, float (&v)[4]) {
+    g8_reduce_rows<T>(part, splits, [&](uint32_t t, uint32_t row, uint32_t cb, uint32_t l32, float (&v)[4]) {
         uint32_t tm, tn;
-        gemm_raster(full_tiles + t, (m + GM_BM - 1) / GM_BM, (nbs + 1) / 2, group_m, tm, tn);
-        uint32_t grow = tm * GM_BM + row, nb = 2 * tn + cb;
+        gemm_raster(full_tiles + t, (m + T::BM - 1) / T::BM, (nbs + 1) / 2, group_m, tm, tn);
+        uint32_t grow = tm * T::BM + row, nb = 2 * tn + cb;
         if (grow < m && nb < nbs) finish_row(v, l32, svh, nb * 128 + 4 * l32, y, y_mode, (size_t)grow * n + nb * 128 + 4 * l32);
     });
 }
 
 #define GEMM_KERNEL_(NAME, BITS, SK)                                                                                   \
-    extern "C" __global__ __launch_bounds__(256, 1) void NAME(                                                         \
+    extern "C" __global__ __launch_bounds__(512, 2) void NAME(                                                         \
         const _Float16* xh, const uint32_t* trellis, const uint16_t* svh, void* y, uint32_t n, uint32_t k, uint32_t m,  \
         uint32_t y_mode, uint32_t stride_k, uint32_t stride_nb, uint32_t group_m, GemmSched sched) {                    \
         exl3_gemm_body<BITS, SK>(xh, trellis, svh, y, n, k, m, y_mode, stride_k, stride_nb, group_m, sched);           \
