@@ -11,7 +11,8 @@
 #include "fe_internal.h"
 
 namespace {
-constexpr uint32_t kGemmLds = 160 * 1024;                // two k tiles of A and three of W, 256 rows each
+// dynamic LDS by form (256 x 256, unused, 128 x 256, 128 x 128): the k tiles in flight, two or three of A and three of W
+constexpr uint32_t kGemmLds[4] = {160 * 1024, 0, 144 * 1024, 80 * 1024};
 constexpr uint32_t kGemmThreads = 512;
 constexpr uint32_t kTileM = 256, kTileN = 256;           // GM_BM, GM_BN
 constexpr uint32_t kGemvRows = 8;                        // rows of one GEMV pass (model.rs:326)
@@ -20,7 +21,8 @@ constexpr uint32_t kSmallBatch = 16;                     // X3_ROWS: batches up 
 
 struct fe_bf16_kernels {
     fe_module_t module = nullptr;
-    fe_function_t gemm = nullptr, reduce = nullptr, swiglu = nullptr, swiglu_reduce = nullptr, interleave = nullptr;
+    fe_function_t gemm[4] = {}, reduce[3] = {}, swiglu[4] = {}, swiglu_reduce[3] = {};  // by form; by tile (fe_gemm_launch)
+    fe_function_t interleave = nullptr;
     fe_function_t gemv[4][4] = {};  // [rows 1, 2, 4, 8][columns of a program 1, 2, 4, 8]
     uint32_t cus = 0;
     FeBuf part;
@@ -28,6 +30,7 @@ struct fe_bf16_kernels {
     int32_t nc = -1;           // columns a GEMV program takes (1, 2, 4, 8); -1 = by the shape (FE_BF16_NC)
     int32_t raster_group = -1; // raster group of the GEMM; -1 = by the shape (FE_BF16_GROUP)
     uint32_t gemm_splits = 8;  // most pieces a cut output tile takes (FE_GEMM_SPLITS; 1: never cut)
+    FeGemmTileOptions tile;    // "gemm_tile", "gemm_pieces"
 };
 
 // log2 of the columns a GEMV program takes. Measured on 5120 x 17408, 17408 x 5120 and 5120 x 5120: 4 columns are best
@@ -64,12 +67,17 @@ int fe_bf16_kernels_load(fe_bf16_kernels **out) {
     if (!out) return fe_set_error(FE_ERR_ARG, "fe_bf16_kernels_load", "null out");
     auto *k = new fe_bf16_kernels;
     int c = fe_load_module(&k->module, "FE_BF16_HSACO", fe_k_bf16_hsaco, fe_k_bf16_hsaco_end);
-    if (!c) c = fe_hip_module_get_function(&k->gemm, k->module, "fe_gemm_bf16");
-    if (!c) c = fe_hip_func_set_max_dyn_lds(k->gemm, kGemmLds);
-    if (!c) c = fe_hip_module_get_function(&k->reduce, k->module, "fe_gemm_bf16_reduce");
-    if (!c) c = fe_hip_module_get_function(&k->swiglu, k->module, "fe_gemm_bf16_swiglu");
-    if (!c) c = fe_hip_func_set_max_dyn_lds(k->swiglu, kGemmLds);
-    if (!c) c = fe_hip_module_get_function(&k->swiglu_reduce, k->module, "fe_gemm_bf16_swiglu_reduce");
+    for (int tile = 0; tile < 3 && !c; tile++) {
+        static const char *suffix[] = {"", "_s1", "_s2"};
+        const int form = tile ? tile + 1 : 0;
+        const std::string s = suffix[tile];
+        c = fe_hip_module_get_function(&k->gemm[form], k->module, ("fe_gemm_bf16" + s).c_str());
+        if (!c) c = fe_hip_func_set_max_dyn_lds(k->gemm[form], kGemmLds[form]);
+        if (!c) c = fe_hip_module_get_function(&k->swiglu[form], k->module, ("fe_gemm_bf16_swiglu" + s).c_str());
+        if (!c) c = fe_hip_func_set_max_dyn_lds(k->swiglu[form], kGemmLds[form]);
+        if (!c) c = fe_hip_module_get_function(&k->reduce[tile], k->module, ("fe_gemm_bf16_reduce" + s).c_str());
+        if (!c) c = fe_hip_module_get_function(&k->swiglu_reduce[tile], k->module, ("fe_gemm_bf16_swiglu_reduce" + s).c_str());
+    }
     if (!c) c = fe_hip_module_get_function(&k->interleave, k->module, "fe_interleave_gu");
     for (int i = 0; i < 4 && !c; i++)
         for (int j = 0; j < 4 && !c; j++) {
@@ -106,6 +114,8 @@ int fe_bf16_kernels_set_option(fe_bf16_kernels *k, const char *name, int32_t val
     if (nm == "nc") k->nc = value;
     else if (nm == "raster_group") k->raster_group = value;
     else if (nm == "gemm_splits") k->gemm_splits = (uint32_t)value;
+    else if (nm == "gemm_tile") k->tile.force_tile = (uint32_t)value;
+    else if (nm == "gemm_pieces") k->tile.force_pieces = (uint32_t)value;
     else return fe_set_error(FE_ERR_ARG, "fe_bf16_kernels_set_option", name);
     return 0;
 }
@@ -138,14 +148,19 @@ int fe_bf16_gemm(const fe_bf16_kernels *kern, fe_stream_t s, fe_devptr_t y, uint
     uint32_t group = bf16_raster_group(m, n, k, tiles_m);
     if (kern->raster_group >= 0) group = (uint32_t)kern->raster_group;
     if (group > tiles_m) group = tiles_m;
-    FeGemmSplit gs = fe_gemm_split(tiles_m * tiles_n, k / 64, kern->cus, (uint32_t)(kern->part.bytes / kFeGemmPartBytes), kern->gemm_splits);
-    uint32_t full = gs.full, splits = gs.splits;
-    fe_devptr_t part = kern->part.p;
-    void *args[] = {&y, &x, &w, &res, &m, &n, &k, &lda, &ldy, &group, &full, &splits, &part};
-    FE_TRY(fe_hip_launch(kern->gemm, gs.programs(), 1, 1, kGemmThreads, 1, 1, kGemmLds, s, args));
-    if (!gs.cut()) return 0;
-    void *rargs[] = {&y, &part, &res, &m, &n, &ldy, &group, &full, &splits};
-    return fe_hip_launch(kern->reduce, gs.cut() * 64, 1, 1, 256, 1, 1, 0, s, rargs);
+    const FeGemmPlan plan = fe_gemm_plan(m, n, k / 64, kern->cus, kern->part.p, kern->part.bytes, 0, 0, kern->gemm_splits, 0, false,
+                                         kFeCostBf16, kern->tile);
+    return fe_gemm_launch(
+        plan,
+        [&](uint32_t form, uint32_t programs, FeGemmSchedArgs sched) {
+            void *args[] = {&y, &x, &w, &res, &m, &n, &k, &lda, &ldy, &group, &sched};
+            return fe_hip_launch(kern->gemm[form], programs, 1, 1, kGemmThreads, 1, 1, kGemmLds[form], s, args);
+        },
+        [&](uint32_t tile, uint32_t grid, uint32_t first, uint32_t splits) {
+            fe_devptr_t part = kern->part.p;
+            void *args[] = {&y, &part, &res, &m, &n, &ldy, &group, &first, &splits};
+            return fe_hip_launch(kern->reduce[tile], grid, 1, 1, 256, 1, 1, 0, s, args);
+        });
 }
 
 int fe_bf16_interleave_gu(const fe_bf16_kernels *kern, fe_stream_t s, fe_devptr_t dst, fe_devptr_t gate, fe_devptr_t up,
@@ -172,14 +187,19 @@ int fe_bf16_gemm_swiglu(const fe_bf16_kernels *kern, fe_stream_t s, fe_devptr_t 
     uint32_t group = bf16_raster_group(m, n, k, tiles_m);
     if (kern->raster_group >= 0) group = (uint32_t)kern->raster_group;
     if (group > tiles_m) group = tiles_m;
-    FeGemmSplit gs = fe_gemm_split(tiles_m * tiles_n, k / 64, kern->cus, (uint32_t)(kern->part.bytes / kFeGemmPartBytes), kern->gemm_splits);
-    uint32_t full = gs.full, splits = gs.splits;
-    fe_devptr_t part = kern->part.p;
-    void *args[] = {&act, &x, &w, &m, &n, &k, &lda, &group, &full, &splits, &part};
-    FE_TRY(fe_hip_launch(kern->swiglu, gs.programs(), 1, 1, kGemmThreads, 1, 1, kGemmLds, s, args));
-    if (!gs.cut()) return 0;
-    void *rargs[] = {&act, &part, &m, &n, &group, &full, &splits};
-    return fe_hip_launch(kern->swiglu_reduce, gs.cut() * 64, 1, 1, 256, 1, 1, 0, s, rargs);
+    const FeGemmPlan plan = fe_gemm_plan(m, n, k / 64, kern->cus, kern->part.p, kern->part.bytes, 0, 0, kern->gemm_splits, 0, false,
+                                         kFeCostBf16, kern->tile);
+    return fe_gemm_launch(
+        plan,
+        [&](uint32_t form, uint32_t programs, FeGemmSchedArgs sched) {
+            void *args[] = {&act, &x, &w, &m, &n, &k, &lda, &group, &sched};
+            return fe_hip_launch(kern->swiglu[form], programs, 1, 1, kGemmThreads, 1, 1, kGemmLds[form], s, args);
+        },
+        [&](uint32_t tile, uint32_t grid, uint32_t first, uint32_t splits) {
+            fe_devptr_t part = kern->part.p;
+            void *args[] = {&act, &part, &m, &n, &group, &first, &splits};
+            return fe_hip_launch(kern->swiglu_reduce[tile], grid, 1, 1, 256, 1, 1, 0, s, args);
+        });
 }
 
 int fe_bf16_linear_forward(const fe_bf16_kernels *kern, fe_stream_t s, fe_devptr_t y, uint32_t ldy, fe_devptr_t x,

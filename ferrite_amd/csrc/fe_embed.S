@@ -8,6 +8,12 @@ fe_k_exl3_hsaco:
     .global fe_k_exl3_hsaco_end
 fe_k_exl3_hsaco_end:
     .balign 4096
+    .global fe_k_exl3_gemm_hsaco
+fe_k_exl3_gemm_hsaco:
+    .incbin "k_exl3_gemm.hsaco"
+    .global fe_k_exl3_gemm_hsaco_end
+fe_k_exl3_gemm_hsaco_end:
+    .balign 4096
     .global fe_k_fp4_hsaco
 fe_k_fp4_hsaco:
     .incbin "k_fp4.hsaco"

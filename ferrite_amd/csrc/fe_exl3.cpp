@@ -25,7 +25,15 @@ constexpr uint32_t kGroupMax = 4;              // FE_EXL3_GROUP_MAX: linears of 
 // buffer holds 32 rows at a time
 constexpr uint32_t kJobLdsBudget = 53 * 1024;
 constexpr uint32_t kRedPitch = 132;            // GEMV_RED_PITCH
-constexpr uint32_t kGemmLds = 160 * 1024;      // k tiles of A and W in flight; the epilogue reuses it
+// Dynamic LDS of the prefill GEMMs by form (256 x 256, its stream-K form, 128 x 256, 128 x 128): the k tiles in flight, two of A and of
+// decoded weights (128 bytes a row each) and two or three of packed words; over decoded tiles two or three of A, three of W.
+// The epilogue reuses it.
+constexpr uint32_t kHatLds[4] = {160 * 1024, 160 * 1024, 144 * 1024, 80 * 1024};
+uint32_t gemm_lds(uint32_t form, uint32_t bits) {
+    const uint32_t room = form == 3 ? 80 * 1024 : 160 * 1024, fixed = form == 3 ? 64 * 1024 : form == 2 ? 112 * 1024 : 128 * 1024;
+    const uint32_t stage = (form == 3 ? 1024 : 2048) * bits;
+    return std::max(fixed + std::min(6u, std::max(2u, (room - fixed) / stage)) * stage, 68u * 1024);
+}
 constexpr uint32_t kGemmThreads = 512;
 constexpr uint32_t kCuLds = 160 * 1024;        // LDS of a CU
 constexpr size_t kChainStride = 64;            // FE_CHAIN_STRIDE: u32 words between two ready words of the one-launch MLP
@@ -77,10 +85,12 @@ struct fe_exl3_kernels {
     fe_function_t gemvb_fenced[6] = {};                           // the same for 1..16 rows with the fenced hand-off
     fe_function_t mlp[6] = {};                                    // the decode MLP in one launch, [bits slot]
     uint32_t cus = 0;
-    fe_function_t gemm[6] = {}, gemm_sk[6] = {};  // decode inside the GEMM: one piece a program / stream-K
-    fe_function_t gemm_reduce = nullptr;
+    fe_module_t gemm_module = nullptr;
+    fe_function_t gemm[6][4] = {};        // decode inside the GEMM, by form: 256 x 256, stream-K, 128 x 256, 128 x 128
+    fe_function_t gemm_reduce[3] = {};    // by tile
     fe_function_t hat_tiles[6] = {};  // trellis -> fp16 weights as the GEMM's LDS images
-    fe_function_t gemm_hat = nullptr, gemm_hat_sk = nullptr;  // the GEMM over them
+    fe_function_t gemm_hat[4] = {};   // the GEMM over them, by form
+    FeGemmTileOptions tile;           // "gemm_tile", "gemm_pieces"
     fe_exl3_options opt;
 };
 
@@ -172,20 +182,20 @@ int fe_exl3_kernels_load(fe_exl3_kernels **out) {
         snprintf(nm, sizeof nm, "exl3_mlp_b%d", kBits[i]);
         get(&k->mlp[i], nm);
         if (!c) c = fe_hip_func_set_max_dyn_lds(k->mlp[i], 84 * 1024);
-        snprintf(nm, sizeof nm, "exl3_gemm_b%d", kBits[i]);
-        get(&k->gemm[i], nm);
-        if (!c) c = fe_hip_func_set_max_dyn_lds(k->gemm[i], kGemmLds);
-        snprintf(nm, sizeof nm, "exl3_gemm_b%d_sk", kBits[i]);
-        get(&k->gemm_sk[i], nm);
-        if (!c) c = fe_hip_func_set_max_dyn_lds(k->gemm_sk[i], kGemmLds);
-        snprintf(nm, sizeof nm, "exl3_hat_tiles_b%d", kBits[i]);
-        get(&k->hat_tiles[i], nm);
-        if (i == 0) get(&k->gemm_reduce, "exl3_gemm_reduce");
     }
-    get(&k->gemm_hat, "exl3_gemm_hat");
-    if (!c) c = fe_hip_func_set_max_dyn_lds(k->gemm_hat, kGemmLds);
-    get(&k->gemm_hat_sk, "exl3_gemm_hat_sk");
-    if (!c) c = fe_hip_func_set_max_dyn_lds(k->gemm_hat_sk, kGemmLds);
+    if (!c) c = fe_load_module(&k->gemm_module, "FE_EXL3_GEMM_HSACO", fe_k_exl3_gemm_hsaco, fe_k_exl3_gemm_hsaco_end);
+    auto get_gemm = [&](fe_function_t *f, const std::string &name, uint32_t lds) {
+        if (!c) c = fe_hip_module_get_function(f, k->gemm_module, name.c_str());
+        if (!c && lds) c = fe_hip_func_set_max_dyn_lds(*f, lds);
+    };
+    static const char *form_sfx[] = {"", "_sk", "_s1", "_s2"}, *tile_sfx[] = {"", "_s1", "_s2"};
+    for (int i = 0; i < 6; i++) {
+        const std::string b = std::to_string(kBits[i]);
+        for (uint32_t f = 0; f < 4; f++) get_gemm(&k->gemm[i][f], "exl3_gemm_b" + b + form_sfx[f], gemm_lds(f, (uint32_t)kBits[i]));
+        get_gemm(&k->hat_tiles[i], "exl3_hat_tiles_b" + b, 0);
+    }
+    for (int f = 0; f < 4; f++) get_gemm(&k->gemm_hat[f], std::string("exl3_gemm_hat") + form_sfx[f], kHatLds[f]);
+    for (int i = 0; i < 3; i++) get_gemm(&k->gemm_reduce[i], std::string("exl3_gemm_reduce") + tile_sfx[i], 0);
     fe_exl3_options &o = k->opt;
     o.fused_rot = env_u32("FE_EXL3_NO_FUSED_ROT", 0) ? 0 : 1;
     o.fused_rot_pairs = env_u32("FE_EXL3_FUSED_ROT_PAIRS", o.fused_rot_pairs);
@@ -217,6 +227,7 @@ int fe_exl3_kernels_load(fe_exl3_kernels **out) {
 int fe_exl3_kernels_destroy(fe_exl3_kernels *k) {
     if (!k) return 0;
     if (k->module) fe_hip_module_unload(k->module);
+    if (k->gemm_module) fe_hip_module_unload(k->gemm_module);
     delete k;
     return 0;
 }
@@ -235,6 +246,8 @@ int fe_exl3_kernels_set_option(fe_exl3_kernels *k, const char *name, uint32_t va
     else if (nm == "gemm_group_m") o.gemm_group_m = value;
     else if (nm == "gemm_splits") o.gemm_splits = value;
     else if (nm == "gemm_sk") o.gemm_sk = value;
+    else if (nm == "gemm_tile") k->tile.force_tile = value;
+    else if (nm == "gemm_pieces") k->tile.force_pieces = value;
     else if (nm == "mlp_chain") o.mlp_chain = value;
     else if (nm == "handoff_fenced") o.handoff_fenced = value;
     else if (nm == "chain_spin") o.chain_spin = value;
@@ -542,29 +555,36 @@ static int launch_gemm(const fe_exl3_linear *l, fe_stream_t s, fe_devptr_t xh, f
     view_strides(l->view, &stride_k, &stride_nb);
     if ((uint64_t)rows * k * 2 >= (1ull << 32))
         return fe_set_error(FE_ERR_UNSUPPORTED, "fe_exl3_linear_gemv_rotated", "rotated input of 4 GB or more");
-    const uint32_t tiles_m = (rows + 255) / 256, tiles_n = (n / 128 + 1) / 2;
+    const uint32_t tiles_m = (rows + 255) / 256;
     if (group == 0 || group > tiles_m) group = tiles_m;
     fe_devptr_t tr = l->view.trellis, svh = l->view.svh, part = ws->part.p;
     const bool kept = l->hat.bytes != 0;  // decoded once and kept: any row count above the GEMV's runs over it
     const bool over_hat = kept || (rows >= kern->opt.hat_rows && ws->hat.bytes >= hat_bytes(l));
     // (decoded tiles are a large weight operand: 32 KB a k tile against the trellis's 2 KB a bit)
-    FeGemmSchedule sch = fe_gemm_schedule(tiles_m * tiles_n, k / 64, kern->cus, ws->part.p, ws->part.bytes, ws->counters.p,
-                                          ws->counters_len, kern->opt.gemm_splits, kern->opt.gemm_sk, !over_hat);
+    const FeGemmPlan plan = fe_gemm_plan(rows, n, k / 64, kern->cus, part, ws->part.bytes, ws->counters.p, ws->counters_len, kern->opt.gemm_splits,
+                                         (int)kern->opt.gemm_sk, !over_hat, kFeCostTrellis, kern->tile);
+    const bool stream_k = !plan.tile && plan.big.stream_k;
+    fe_devptr_t hat = kept ? l->hat.p : ws->hat.p;
     if (over_hat) {
-        fe_devptr_t hat = kept ? l->hat.p : ws->hat.p;
         if (!kept) FE_TRY(launch_decode(l, s, hat));
         group = 0;  // the raster that deals column tiles to the XCDs: each decoded weight panel goes through one L2
-        void *args[] = {&xh, &hat, &svh, &y, &n, &k, &rows, &mode, &group, &sch.args};
-        FE_TRY(fe_hip_launch(sch.stream_k ? kern->gemm_hat_sk : kern->gemm_hat, sch.programs, 1, 1, kGemmThreads, 1, 1, kGemmLds, s, args));
-    } else {
-        if (sch.stream_k) group = 1;  // column tiles fastest: the programs that are in step share a panel of inputs
-        void *args[] = {&xh, &tr, &svh, &y, &n, &k, &rows, &mode, &stride_k, &stride_nb, &group, &sch.args};
-        FE_TRY(fe_hip_launch((sch.stream_k ? kern->gemm_sk : kern->gemm)[bits_slot(l->bits)], sch.programs, 1, 1, kGemmThreads, 1, 1, kGemmLds, s, args));
+    } else if (stream_k) {
+        group = 1;  // column tiles fastest: the programs that are in step share a panel of inputs
     }
-    if (sch.stream_k || !sch.split.cut()) return 0;
-    uint32_t full = sch.split.full, splits = sch.split.splits;
-    void *rargs[] = {&part, &svh, &y, &n, &rows, &mode, &group, &full, &splits};
-    return fe_hip_launch(kern->gemm_reduce, sch.split.cut() * 64, 1, 1, 256, 1, 1, 0, s, rargs);
+    return fe_gemm_launch(
+        plan,
+        [&](uint32_t form, uint32_t programs, FeGemmSchedArgs sched) {
+            if (over_hat) {
+                void *args[] = {&xh, &hat, &svh, &y, &n, &k, &rows, &mode, &group, &sched};
+                return fe_hip_launch(kern->gemm_hat[form], programs, 1, 1, kGemmThreads, 1, 1, kHatLds[form], s, args);
+            }
+            void *args[] = {&xh, &tr, &svh, &y, &n, &k, &rows, &mode, &stride_k, &stride_nb, &group, &sched};
+            return fe_hip_launch(kern->gemm[bits_slot(l->bits)][form], programs, 1, 1, kGemmThreads, 1, 1, gemm_lds(form, l->bits), s, args);
+        },
+        [&](uint32_t tile, uint32_t grid, uint32_t first, uint32_t splits) {
+            void *args[] = {&part, &svh, &y, &n, &rows, &mode, &group, &first, &splits};
+            return fe_hip_launch(kern->gemm_reduce[tile], grid, 1, 1, 256, 1, 1, 0, s, args);
+        });
 }
 
 // The GEMV can rotate its own input: every program rotates the channels of its own run, (row, 128-channel block) pairs,

@@ -14,20 +14,21 @@
 
 namespace {
 constexpr uint32_t kTile = 128;                 // crates/fe-fp4/src/lib.rs:28
-constexpr uint32_t kGemmLds = 160 * 1024;               // k tiles of A and W in flight
+// dynamic LDS by form (256 x 256, its stream-K form, 128 x 256, 128 x 128): the k tiles in flight. Packed weights: three of A (128
+// bytes a row) and three of W (36 bytes; 64 in the fp16 form of FP8). FP8 codes: two or three of A, three of W, 128 bytes a row.
+constexpr uint32_t kGemmLds[4] = {144 * 1024, 144 * 1024, 136 * 1024, 68 * 1024}, kGemmLds8[4] = {160 * 1024, 160 * 1024, 144 * 1024, 80 * 1024};
 constexpr uint32_t kGemmThreads = 512;
 constexpr uint32_t kTileM = 256;                        // GM_BM
-constexpr uint32_t kTileN = 256;                        // GM_BN
 }  // namespace
 
 struct fe_fp4_kernels {
     fe_module_t module = nullptr;
-    fe_function_t quant4 = nullptr, gemm4 = nullptr, reduce4 = nullptr, reduce8c = nullptr, gemv4[3] = {nullptr, nullptr, nullptr};
+    fe_function_t quant4 = nullptr, gemv4[3] = {nullptr, nullptr, nullptr};
+    // by form (256 x 256, stream-K, 128 x 256, 128 x 128) and by tile (fe_gemm_launch); gemm8: the fp16 form, 256 x 256 only
+    fe_function_t gemm4[4] = {}, swiglu4[4] = {}, gemm8c[4] = {}, gemm8[2] = {}, reduce4[3] = {}, swiglu_reduce4[3] = {}, reduce8c[3] = {};
     fe_function_t strip4 = nullptr;  // the GEMV over strips of 16 weight rows, up to 16 activation rows (no hand-off)
     fe_function_t strip_once[5] = {};  // ... with every load of a workgroup issued before anything waits: 1..5 groups of K a wavefront
-    fe_function_t quant8 = nullptr, gemm8 = nullptr, swiglu4 = nullptr, swiglu_reduce4 = nullptr;
-    fe_function_t gemm8c = nullptr;  // FP8 on the 8-bit matrix instruction, operands as codes
-    fe_function_t gemm4_sk = nullptr, gemm8_sk = nullptr, gemm8c_sk = nullptr, swiglu4_sk = nullptr;  // the same on the stream-K schedule
+    fe_function_t quant8 = nullptr;
     uint32_t cus = 0;
     // Switches of the launch paths: read from the environment once, at load; fe_fp4_kernels_set_option changes them
     // afterwards. No forward call reads the environment.
@@ -41,6 +42,7 @@ struct fe_fp4_kernels {
     uint32_t fp8_f16 = 0;      // FP8 linears as fp16 expansion on the 16-bit matrix instruction (FE_FP8_F16=1)
     uint32_t gemm_splits = 8;  // most pieces a cut output tile takes (FE_GEMM_SPLITS; 1: never cut)
     int32_t gemm_sk = 1;       // stream-K schedule of the GEMMs: 0 never, 1 where measured faster, 2 always (FE_GEMM_SK)
+    FeGemmTileOptions tile;    // "gemm_tile", "gemm_pieces"
 };
 
 struct fe_fp4_linear {
@@ -68,10 +70,22 @@ int fe_fp4_kernels_load(fe_fp4_kernels **out) {
     auto *k = new fe_fp4_kernels;
     int c = fe_load_module(&k->module, "FE_FP4_HSACO", fe_k_fp4_hsaco, fe_k_fp4_hsaco_end);
     if (!c) c = fe_hip_module_get_function(&k->quant4, k->module, "fe_fp4_quant");
-    if (!c) c = fe_hip_module_get_function(&k->gemm4, k->module, "fe_gemm_nvfp4");
-    if (!c) c = fe_hip_func_set_max_dyn_lds(k->gemm4, kGemmLds);
-    if (!c) c = fe_hip_module_get_function(&k->reduce4, k->module, "fe_gemm_nvfp4_reduce");
-    if (!c) c = fe_hip_module_get_function(&k->reduce8c, k->module, "fe_gemm_fp8_codes_reduce");
+    auto get = [&](fe_function_t *f, const std::string &nm, uint32_t lds) {
+        if (!c) c = fe_hip_module_get_function(f, k->module, nm.c_str());
+        if (!c && lds) c = fe_hip_func_set_max_dyn_lds(*f, lds);
+    };
+    static const char *form_sfx[] = {"", "_sk", "_s1", "_s2"}, *tile_sfx[] = {"", "_s1", "_s2"};
+    for (int i = 0; i < 4; i++) {
+        get(&k->gemm4[i], std::string("fe_gemm_nvfp4") + form_sfx[i], kGemmLds[i]);
+        get(&k->swiglu4[i], std::string("fe_gemm_nvfp4_swiglu") + form_sfx[i], kGemmLds[i]);
+        get(&k->gemm8c[i], std::string("fe_gemm_fp8_codes") + form_sfx[i], kGemmLds8[i]);
+        if (i < 2) get(&k->gemm8[i], std::string("fe_gemm_fp8") + form_sfx[i], kGemmLds[i]);
+    }
+    for (int i = 0; i < 3; i++) {
+        get(&k->reduce4[i], std::string("fe_gemm_nvfp4_reduce") + tile_sfx[i], 0);
+        get(&k->swiglu_reduce4[i], std::string("fe_gemm_nvfp4_swiglu_reduce") + tile_sfx[i], 0);
+        get(&k->reduce8c[i], std::string("fe_gemm_fp8_codes_reduce") + tile_sfx[i], 0);
+    }
     for (int xr = 1; xr <= 3 && !c; xr++) {
         char nm[32];
         snprintf(nm, sizeof nm, "fe_gemv_nvfp4_x%d", xr);
@@ -85,20 +99,6 @@ int fe_fp4_kernels_load(fe_fp4_kernels **out) {
         if (!c) c = fe_hip_func_set_max_dyn_lds(k->strip_once[g - 1], 48 * 1024);
     }
     if (!c) c = fe_hip_module_get_function(&k->quant8, k->module, "fe_fp8_quant");
-    if (!c) c = fe_hip_module_get_function(&k->gemm8, k->module, "fe_gemm_fp8");
-    if (!c) c = fe_hip_func_set_max_dyn_lds(k->gemm8, kGemmLds);
-    if (!c) c = fe_hip_module_get_function(&k->gemm8c, k->module, "fe_gemm_fp8_codes");
-    if (!c) c = fe_hip_func_set_max_dyn_lds(k->gemm8c, kGemmLds);
-    struct { fe_function_t *f; const char *nm; } sks[] = {
-        {&k->gemm4_sk, "fe_gemm_nvfp4_sk"}, {&k->gemm8_sk, "fe_gemm_fp8_sk"}, {&k->gemm8c_sk, "fe_gemm_fp8_codes_sk"},
-        {&k->swiglu4_sk, "fe_gemm_nvfp4_swiglu_sk"}};
-    for (auto &e : sks) {
-        if (!c) c = fe_hip_module_get_function(e.f, k->module, e.nm);
-        if (!c) c = fe_hip_func_set_max_dyn_lds(*e.f, kGemmLds);
-    }
-    if (!c) c = fe_hip_module_get_function(&k->swiglu4, k->module, "fe_gemm_nvfp4_swiglu");
-    if (!c) c = fe_hip_func_set_max_dyn_lds(k->swiglu4, kGemmLds);
-    if (!c) c = fe_hip_module_get_function(&k->swiglu_reduce4, k->module, "fe_gemm_nvfp4_swiglu_reduce");
     int cus = 0;
     if (!c) c = fe_hip_cu_count(&cus);
     k->cus = (uint32_t)cus;
@@ -140,6 +140,8 @@ int fe_fp4_kernels_set_option(fe_fp4_kernels *k, const char *name, int32_t value
     else if (nm == "fp8_f16") k->fp8_f16 = value ? 1 : 0;
     else if (nm == "gemm_splits") k->gemm_splits = (uint32_t)value;
     else if (nm == "gemm_sk") k->gemm_sk = value;
+    else if (nm == "gemm_tile") k->tile.force_tile = (uint32_t)value;
+    else if (nm == "gemm_pieces") k->tile.force_pieces = (uint32_t)value;
     else return fe_set_error(FE_ERR_ARG, "fe_fp4_kernels_set_option", name);
     return 0;
 }
@@ -403,7 +405,7 @@ int fe_fp4_linear_gemm(const fe_fp4_linear *l, const fe_fp4_kernels *kern, fe_st
     }
     if ((uint64_t)m * k * 2 >= (1ull << 32) || (uint64_t)n * k >= (1ull << 32))
         return fe_set_error(FE_ERR_UNSUPPORTED, "fe_fp4_linear_gemm", "operand of 4 GB or more");
-    const uint32_t tiles_m = (m + kTileM - 1) / kTileM, tiles_n = (n + kTileN - 1) / kTileN;
+    const uint32_t tiles_m = (m + kTileM - 1) / kTileM;
     uint32_t group = kern->group_m == 0 || kern->group_m > tiles_m ? tiles_m : kern->group_m;  // lib.rs:148-151
     // FP8 codes: the weights are the larger operand from n >= m on, and at the 8-bit instruction's rate their traffic
     // shows: column tiles are dealt to the XCDs (gemm_raster with group 0), each weight panel through one L2
@@ -414,29 +416,35 @@ int fe_fp4_linear_gemm(const fe_fp4_linear *l, const fe_fp4_kernels *kern, fe_st
     // FP8 runs on the 8-bit matrix instruction over the codes of both operands, k tiles of 128 (FE_FP8_F16=1: the fp16
     // expansion on the 16-bit instruction, k tiles of 64; same products, another order of the f32 sums)
     const bool codes8 = l->fp8 && !kern->fp8_f16;
-    FeGemmSchedule sch = fe_gemm_schedule(tiles_m * tiles_n, codes8 ? k / 128 : k / 64, kern->cus, ws->part.p, ws->part.bytes,
-                                          ws->counters.p, kGemvCounters, kern->gemm_splits, kern->gemm_sk, /*small_b=*/!l->fp8);
+    const FeGemmTileOptions f16_form{1, 0};  // (the fp16 form exists for 256 x 256 tiles only)
+    const FeGemmPlan plan = fe_gemm_plan(m, n, codes8 ? k / 128 : k / 64, kern->cus, ws->part.p, ws->part.bytes, ws->counters.p, kGemvCounters,
+                                         kern->gemm_splits, kern->gemm_sk, /*small_b=*/!l->fp8,
+                                         l->fp8 ? kFeCostFp8 : kFeCostNvfp4, l->fp8 && !codes8 ? f16_form : kern->tile);
     // stream-K programs sit at different depths of K: one row tile at a time (column tiles fastest) keeps those that are
     // in step on one panel of activations
-    if (sch.stream_k && kern->xcd < 0) group = 1;
-    float scale = l->fp8 ? 1.0f : 0.5f;  // 1 / what the fp16 operands carry (FP4_GEMM_SCALE)
-    if (codes8) {
-        fe_devptr_t codes = ws->codes.p;
-        void *args8[] = {&y, &codes, &w, &alpha, &res, &m, &n, &k, &ldy, &group, &w_snt, &w_skt, &w_sr, &sch.args};
-        FE_TRY(fe_hip_launch(sch.stream_k ? kern->gemm8c_sk : kern->gemm8c, sch.programs, 1, 1, kGemmThreads, 1, 1, kGemmLds, s, args8));
-    } else if (l->fp8) {
-        void *args8[] = {&y, &aq, &w, &alpha, &res, &m, &n, &k, &ldy, &group, &w_snt, &w_skt, &w_sr, &sch.args};
-        FE_TRY(fe_hip_launch(sch.stream_k ? kern->gemm8_sk : kern->gemm8, sch.programs, 1, 1, kGemmThreads, 1, 1, kGemmLds, s, args8));
-    } else {
-        void *args[] = {&y,     &aq,    &w,     &sw,   &alpha, &res,   &m,    &n,       &k,
-                        &ldy,   &group, &w_snt, &w_skt, &w_sr, &s_snt, &s_skt, &s_sr, &sch.args};
-        FE_TRY(fe_hip_launch(sch.stream_k ? kern->gemm4_sk : kern->gemm4, sch.programs, 1, 1, kGemmThreads, 1, 1, kGemmLds, s, args));
-    }
-    if (sch.stream_k || !sch.split.cut()) return 0;
-    uint32_t full = sch.split.full, splits = sch.split.splits;
-    fe_devptr_t part = ws->part.p;
-    void *rargs[] = {&y, &part, &alpha, &res, &m, &n, &ldy, &group, &full, &splits, &scale};
-    return fe_hip_launch(codes8 ? kern->reduce8c : kern->reduce4, sch.split.cut() * 64, 1, 1, 256, 1, 1, 0, s, rargs);
+    if (!plan.tile && plan.big.stream_k && kern->xcd < 0) group = 1;
+    return fe_gemm_launch(
+        plan,
+        [&](uint32_t form, uint32_t programs, FeGemmSchedArgs sched) {
+            if (codes8) {
+                fe_devptr_t codes = ws->codes.p;
+                void *args[] = {&y, &codes, &w, &alpha, &res, &m, &n, &k, &ldy, &group, &w_snt, &w_skt, &w_sr, &sched};
+                return fe_hip_launch(kern->gemm8c[form], programs, 1, 1, kGemmThreads, 1, 1, kGemmLds8[form], s, args);
+            }
+            if (l->fp8) {
+                void *args[] = {&y, &aq, &w, &alpha, &res, &m, &n, &k, &ldy, &group, &w_snt, &w_skt, &w_sr, &sched};
+                return fe_hip_launch(kern->gemm8[form], programs, 1, 1, kGemmThreads, 1, 1, kGemmLds[form], s, args);
+            }
+            void *args[] = {&y,     &aq,    &w,     &sw,    &alpha, &res,   &m,    &n,    &k,
+                            &ldy,   &group, &w_snt, &w_skt, &w_sr,  &s_snt, &s_skt, &s_sr, &sched};
+            return fe_hip_launch(kern->gemm4[form], programs, 1, 1, kGemmThreads, 1, 1, kGemmLds[form], s, args);
+        },
+        [&](uint32_t tile, uint32_t grid, uint32_t first, uint32_t splits) {
+            fe_devptr_t part = ws->part.p;
+            float scale = l->fp8 ? 1.0f : 0.5f;  // 1 / what the fp16 operands carry (FP4_GEMM_SCALE)
+            void *args[] = {&y, &part, &alpha, &res, &m, &n, &ldy, &group, &first, &splits, &scale};
+            return fe_hip_launch(codes8 ? kern->reduce8c[tile] : kern->reduce4[tile], grid, 1, 1, 256, 1, 1, 0, s, args);
+        });
 }
 
 int fe_fp4_linear_forward(const fe_fp4_linear *l, const fe_fp4_kernels *kern, fe_stream_t s, const fe_fp4_workspace *ws,
@@ -462,23 +470,26 @@ int fe_fp4_linear_forward_swiglu(const fe_fp4_linear *l, const fe_fp4_kernels *k
     FE_TRY(fe_fp4_linear_quantize(l, kern, s, ws, x, lda, m));
     if ((uint64_t)m * k * 2 >= (1ull << 32) || (uint64_t)n * k / 2 >= (1ull << 32))
         return fe_set_error(FE_ERR_UNSUPPORTED, "fe_fp4_linear_forward_swiglu", "operand of 4 GB or more");
-    const uint32_t tiles_m = (m + kTileM - 1) / kTileM, tiles_n = (n + kTileN - 1) / kTileN;
+    const uint32_t tiles_m = (m + kTileM - 1) / kTileM;
     uint32_t group = kern->group_m == 0 || kern->group_m > tiles_m ? tiles_m : kern->group_m;
     fe_devptr_t aq = ws->aq.p, w = l->w.p, sw = l->sw.p, alpha = l->alpha.p, part = ws->part.p;
     fe_devptr_t q_codes = act->codes.p, q_sf = act->sf.p, q_aq = act->aq.p;
     uint32_t w_snt = l->w_snt, w_skt = l->w_skt, w_sr = l->w_sr, s_snt = l->s_snt, s_skt = l->s_skt, s_sr = l->s_sr;
-    FeGemmSchedule sch = fe_gemm_schedule(tiles_m * tiles_n, k / 64, kern->cus, ws->part.p, ws->part.bytes, ws->counters.p,
-                                          kGemvCounters, kern->gemm_splits, kern->gemm_sk >= 2 ? kern->gemm_sk : 0, true);
     // (stream-K only when forced: this kernel's stream-K form was slower wherever measured, 688 -> 714 us on 5120 x 34816)
-    if (sch.stream_k && kern->xcd < 0) group = 1;
-    void *args[] = {&aq,    &w,     &sw,    &alpha, &m,       &n,       &k,    &group, &w_snt, &w_skt,
-                    &w_sr,  &s_snt, &s_skt, &s_sr,  &sch.args, &q_codes, &q_sf, &q_aq,  &down_g};
-    FE_TRY(fe_hip_launch(sch.stream_k ? kern->swiglu4_sk : kern->swiglu4, sch.programs, 1, 1, kGemmThreads, 1, 1, kGemmLds, s, args));
-    if (sch.stream_k || !sch.split.cut()) return 0;
-    const FeGemmSplit &gs = sch.split;
-    uint32_t full = gs.full, splits = gs.splits;
-    void *rargs[] = {&part, &alpha, &m, &n, &group, &full, &splits, &q_codes, &q_sf, &q_aq, &down_g};
-    return fe_hip_launch(kern->swiglu_reduce4, gs.cut() * 64, 1, 1, 256, 1, 1, 0, s, rargs);
+    const FeGemmPlan plan = fe_gemm_plan(m, n, k / 64, kern->cus, ws->part.p, ws->part.bytes, ws->counters.p, kGemvCounters, kern->gemm_splits,
+                                         kern->gemm_sk >= 2 ? kern->gemm_sk : 0, true, kFeCostNvfp4, kern->tile);
+    if (!plan.tile && plan.big.stream_k && kern->xcd < 0) group = 1;
+    return fe_gemm_launch(
+        plan,
+        [&](uint32_t form, uint32_t programs, FeGemmSchedArgs sched) {
+            void *args[] = {&aq,   &w,     &sw,    &alpha, &m,     &n,       &k,    &group, &w_snt, &w_skt,
+                            &w_sr, &s_snt, &s_skt, &s_sr,  &sched, &q_codes, &q_sf, &q_aq,  &down_g};
+            return fe_hip_launch(kern->swiglu4[form], programs, 1, 1, kGemmThreads, 1, 1, kGemmLds[form], s, args);
+        },
+        [&](uint32_t tile, uint32_t grid, uint32_t first, uint32_t splits) {
+            void *args[] = {&part, &alpha, &m, &n, &group, &first, &splits, &q_codes, &q_sf, &q_aq, &down_g};
+            return fe_hip_launch(kern->swiglu_reduce4[tile], grid, 1, 1, 256, 1, 1, 0, s, args);
+        });
 }
 
 }  // extern "C"

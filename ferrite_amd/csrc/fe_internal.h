@@ -19,6 +19,8 @@ int fe_check_hip(int code, const char *call);
 // gfx950 code objects linked into the library (fe_embed.S)
 extern "C" const unsigned char fe_k_exl3_hsaco[];
 extern "C" const unsigned char fe_k_exl3_hsaco_end[];
+extern "C" const unsigned char fe_k_exl3_gemm_hsaco[];
+extern "C" const unsigned char fe_k_exl3_gemm_hsaco_end[];
 extern "C" const unsigned char fe_k_fp4_hsaco[];
 extern "C" const unsigned char fe_k_fp4_hsaco_end[];
 extern "C" const unsigned char fe_k_route_hsaco[];
@@ -229,4 +231,107 @@ inline FeGemmSchedule fe_gemm_schedule(uint32_t tiles, uint32_t ktiles, uint32_t
     r.args.full_tiles = whole;
     r.args.sk_base = base, r.args.sk_rem = rem;
     return r;
+}
+
+// ---- which tiles a GEMM launch takes -------------------------------------------------------------------------------------------
+// Tile 0: 256 x 256, on one of the two schedules above. Tiles 1 (128 x 256) and 2 (128 x 128): a launch of small tiles, each cut
+// `splits` ways along K.
+constexpr uint32_t kFeGemmTileM[3] = {256, 128, 128}, kFeGemmTileN[3] = {256, 256, 128};
+
+struct FeGemmPlan {
+    FeGemmSchedule big;  // tile 0
+    uint32_t tile = 0, tiles = 0, splits = 1;
+};
+// Switches of the plan (options of the three kernels handles): force_tile 0 = by the rule, 1 = 256 x 256, 2, 3 = small tile 1, 2
+// with force_pieces pieces of K (0: one).
+struct FeGemmTileOptions {
+    uint32_t force_tile = 0, force_pieces = 0;
+};
+
+// What a program of each tile takes on one weight form: us a k tile (64; FP8: 128), `full` more of it when all CUs are busy (clock and
+// memory), us a program besides, and how much slower two programs that share a CU (tile 2) are than one alone. Fitted to 770
+// timings a form (MI355X, 80..1536 rows, 2048 x 2048 .. 17408 x 5120, 1..8 pieces; within 6 % for trellis and NVFP4 weights,
+// 10..13 % for bf16 and FP8, whose panels compete for memory). stream_k: what meeting through the workspace adds.
+struct FeGemmCost {
+    float ktile[3], full[3], fixed[3], shared, stream_k;
+};
+constexpr FeGemmCost kFeCostTrellis = {{1.38f, 1.02f, 0.71f}, {0.12f, 0.07f, 0.08f}, {1.0f, 3.0f, 1.9f}, 1.63f, 48.7f};
+constexpr FeGemmCost kFeCostNvfp4 = {{1.32f, 0.73f, 0.44f}, {-0.07f, 0.05f, 0.09f}, {0.0f, 2.2f, 2.3f}, 1.59f, 44.0f};
+constexpr FeGemmCost kFeCostFp8 = {{1.20f, 0.58f, 0.66f}, {0.09f, 0.46f, 0.21f}, {0.0f, 2.5f, 0.4f}, 1.21f, 36.4f};
+constexpr FeGemmCost kFeCostBf16 = {{1.10f, 0.64f, 0.45f}, {0.22f, 0.43f, 0.41f}, {0.0f, 1.5f, 0.3f}, 1.53f, 53.2f};
+
+// `programs` programs of `ktiles` k tiles each, in rounds of all CUs (tile 2: two a CU).
+inline float fe_gemm_cost(const FeGemmCost &c, uint32_t tile, uint32_t programs, uint32_t ktiles, uint32_t cus) {
+    const uint32_t round = tile == 2 ? 2 * cus : cus, last = programs % round;
+    const float whole = (float)ktiles * c.ktile[tile] * (1.0f + c.full[tile]) * (tile == 2 ? c.shared : 1.0f) + c.fixed[tile];
+    const float part = (float)ktiles * c.ktile[tile] * (1.0f + c.full[tile] * (float)last / (float)cus) + c.fixed[tile];
+    return (float)(programs / round) * whole + (last > cus ? whole : last ? part : 0.0f);
+}
+// The reduce launch: its start, and the partials written and read once.
+inline float fe_gemm_reduce_cost(uint32_t programs, uint32_t tile) {
+    return 4.0f + (float)programs * (float)(kFeGemmTileM[tile] * kFeGemmTileN[tile]) * 8.0f / 5e6f;
+}
+
+// The rule: with fewer than a few rounds of 256 x 256 tiles, most of the time is CUs without a tile or pieces of K that meet;
+// tiles of half and a quarter the size fill the chip with fewer pieces. They read more operand bytes and run fewer matrix
+// instructions between two barriers (a k tile of them costs more than its share), so they pay only where the fill gains more:
+// the estimate above decides, with 6 % against a small tile for its error. Pieces of at least 8 k tiles, at most as many
+// programs as run at once when K is cut. Up to 2048 rows, what the estimate was fitted on: beyond, whole rounds of 256 x 256
+// prevail. 5120 x 5120, us, before -> with small tiles: NVFP4 100 rows 31 -> 21, bf16 1000 rows 58 -> 56, FP8 1000 rows 42 -> 30.
+inline FeGemmPlan fe_gemm_plan(uint32_t m, uint32_t n, uint32_t ktiles, uint32_t cus, fe_devptr_t part, size_t part_bytes,
+                               fe_devptr_t counters, size_t counters_len, uint32_t cap, int mode, bool small_b,
+                               const FeGemmCost &cost, const FeGemmTileOptions &opt) {
+    FeGemmPlan p;
+    p.big = fe_gemm_schedule(((m + 255) / 256) * ((n + 255) / 256), ktiles, cus, part, part_bytes, counters, counters_len, cap, mode, small_b);
+    auto take = [&](uint32_t tile, uint32_t tiles, uint32_t pieces) { p.tile = tile, p.tiles = tiles, p.splits = pieces; };
+    auto tiles_of = [&](uint32_t tile) {
+        return ((m + kFeGemmTileM[tile] - 1) / kFeGemmTileM[tile]) * ((n + kFeGemmTileN[tile] - 1) / kFeGemmTileN[tile]);
+    };
+    auto most_pieces = [&](uint32_t tile, uint32_t want) {
+        const size_t slots = part_bytes / (kFeGemmTileM[tile] * kFeGemmTileN[tile] * 4);
+        return (uint32_t)std::max<size_t>(1, std::min<size_t>({want, ktiles, slots / tiles_of(tile)}));
+    };
+    if (opt.force_tile >= 2) {
+        take(opt.force_tile - 1, tiles_of(opt.force_tile - 1), most_pieces(opt.force_tile - 1, std::max(1u, opt.force_pieces)));
+        return p;
+    }
+    if (opt.force_tile == 1 || mode >= 2 || m > 2048 || !cus) return p;
+    float best;
+    if (p.big.stream_k) {
+        const FeGemmSchedArgs &a = p.big.args;
+        best = fe_gemm_cost(cost, 0, p.big.programs, a.full_tiles / p.big.programs * ktiles + a.sk_base + 1, cus) + cost.stream_k;
+    } else {
+        const FeGemmSplit &g = p.big.split;
+        best = fe_gemm_cost(cost, 0, g.full, ktiles, cus);
+        if (g.cut())
+            best += fe_gemm_cost(cost, 0, g.cut() * g.splits, (ktiles + g.splits - 1) / g.splits, cus) + fe_gemm_reduce_cost(g.cut() * g.splits, 0);
+    }
+    for (uint32_t tile = 1; tile <= 2; tile++) {
+        const uint32_t tiles = tiles_of(tile), most = most_pieces(tile, std::min(cap, ktiles / 8));
+        for (uint32_t pieces = 1; pieces <= most; pieces++) {
+            if (pieces > 1 && tiles * pieces > cus * tile) break;
+            float c = fe_gemm_cost(cost, tile, tiles * pieces, (ktiles + pieces - 1) / pieces, cus);
+            if (pieces > 1) c += fe_gemm_reduce_cost(tiles * pieces, tile);
+            if (1.06f * c < best) take(tile, tiles, pieces), best = 1.06f * c;
+        }
+    }
+    return p;
+}
+
+// Launches a plan. gemm(form, programs, sched): form 0 = 256 x 256 one piece a program, 1 = stream-K, 2, 3 = tile 1, 2;
+// reduce(tile, grid, first, splits): the reduce kernel of a tile, for the tiles from `first` on.
+template <class Gemm, class Reduce>
+int fe_gemm_launch(const FeGemmPlan &p, Gemm gemm, Reduce reduce) {
+    const uint32_t reduce_grid = kFeGemmTileM[p.tile] / 8 * (kFeGemmTileN[p.tile] / 128);  // workgroups a tile
+    if (p.tile) {
+        FeGemmSchedArgs a = p.big.args;
+        a.full_tiles = 0, a.splits = p.splits, a.sk_base = a.sk_rem = 0;
+        FE_TRY(gemm(p.tile + 1, p.tiles * p.splits, a));
+        if (p.splits > 1) FE_TRY(reduce(p.tile, p.tiles * reduce_grid, 0u, p.splits));
+        return 0;
+    }
+    FE_TRY(gemm(p.big.stream_k ? 1u : 0u, p.big.programs, p.big.args));
+    if (!p.big.stream_k && p.big.split.cut())
+        FE_TRY(reduce(0u, p.big.split.cut() * reduce_grid, p.big.split.full, p.big.split.splits));
+    return 0;
 }

@@ -21,13 +21,14 @@
 #pragma once
 #include "gemm_core.h"
 
-#define G8_BK 64
+#define G8_BK GM_BK
 
 template <int WM_, int WN_, int TM_, int TN_>
 struct G8Tile {
     static constexpr int WM = WM_, WN = WN_, TM = TM_, TN = TN_, NW = WM * WN, THREADS = 64 * NW;
     static constexpr int BM = 16 * TM * WM, BN = 16 * TN * WN;
     static constexpr int PART_FLOATS = BM * BN;
+    static constexpr int PARTS = 256 * 256 / (BM * BN);  // of a tile of 256 x 256: 1; 2, 4: the small tiles
     static_assert(NW == 8, "eight wavefronts");
 };
 
@@ -66,6 +67,17 @@ __device__ __forceinline__ constexpr uint32_t g8_perm(uint32_t c) {
     return PERM ? (c & 4) | ((c & 1) << 1) | ((c >> 1) & 1) : c;
 }
 
+// Where the q-th of n side operations goes among the matrix instructions x0 .. x1 - 1 of a slice: spread evenly. What is issued
+// between two matrix instructions of a wavefront runs in the pipe's shadow; in a lump it does not (both wavefronts of a SIMD pass the
+// same barrier and would reach the lump together).
+__device__ __forceinline__ constexpr int g8_at(int q, int n, int x0, int x1) { return x0 + q * (x1 - x0) / n; }
+
+// Loads that may still be in flight at the barrier of a tile, with LA loads of A (NA stages) issued behind the barrier and LB of W
+// (NW stages) in front of it each tile: those issued after the later one of the next tile's A and W. And at the start of the
+// loop, where the first tile's have to be there.
+constexpr int g8_flight(int LA, int NA, int LB, int NW) { return NW > NA ? (NA - 1) * LB + (NA - 2) * LA : (NW - 2) * (LA + LB); }
+constexpr int g8_flight0(int LA, int NA, int LB, int NW) { return NW > NA ? (NA - 1) * (LA + LB) : (NW - 1) * LA + (NW - 2) * LB; }
+
 // Weight operand already in 16-bit form: rows of 64 values a k tile. voff[j]: byte offset of the lane's 16-byte piece j (row
 // 8 (wave + 8 j) + lane / 8, position lane & 7) at k tile 0; k tiles are kstep bytes apart. (dense_setup_rows / _image.)
 template <class T>
@@ -100,7 +112,7 @@ template <class T, int NA, int NW, bool BF16, class W>
 __device__ __forceinline__ void g8_mainloop(const void* a, uint32_t lda, uint32_t m, uint32_t kt0, uint32_t ktiles, uint32_t m0,
                                             const W& wo, unsigned char* lds, f32x4 (&acc)[T::TM][T::TN]) {
     constexpr int TM = T::TM, TN = T::TN, LA = T::BM / 64, LB = W::LOADS, A_STAGE = T::BM * 128, W_AT = NA * A_STAGE;
-    static_assert(NW == NA || NW == NA + 1, "the waits below");
+    static_assert(NA >= 2 && NW >= 2 && g8_flight0(LA, NA, LB, NW) < 64, "loads in flight");
     static_assert(W_AT + NW * W::STAGE <= 160 * 1024, "LDS");
     const uint32_t lane = threadIdx.x & 63, wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
     const uint32_t wm = wave / T::WN, wn = wave % T::WN;
@@ -138,17 +150,19 @@ __device__ __forceinline__ void g8_mainloop(const void* a, uint32_t lda, uint32_
 #pragma unroll
         for (int j = 0; j < TN; j++) acc[i][j] = (f32x4){0.f, 0.f, 0.f, 0.f};
 
-    // prologue: the loads in the order of the loop's own ([W of a slice 0, A of a slice 1] a tile), up to A of tile NA - 1
+    // prologue: the loads in the order of the loop's own ([W in slice 0, A in slice 1] a tile), as of tiles before the first
 #pragma unroll
-    for (int t = 0; t < NA; t++) {
-        if (NW - 1 - NA + t >= 0) {
+    for (int t = -(NA > NW - 1 ? NA : NW - 1); t < 0; t++) {
+        if (t - 1 + NW >= 0) {
 #pragma unroll
-            for (int j = 0; j < LB; j++) load_w(NW - 1 - NA + t, NW - 1 - NA + t, j);
+            for (int j = 0; j < LB; j++) load_w(t - 1 + NW, t - 1 + NW, j);
         }
+        if (t + NA >= 0) {
 #pragma unroll
-        for (int j = 0; j < LA; j++) load_a(t, t, j);
+            for (int j = 0; j < LA; j++) load_a(t + NA, t + NA, j);
+        }
     }
-    g8_loads_wait<(NW > NA ? (NA - 1) * (LA + LB) : (NA - 1) * LA + (NA > 1 ? (NA - 2) * LB : 0))>();
+    g8_loads_wait<g8_flight0(LA, NA, LB, NW)>();
     g8_barrier();
 #pragma unroll
     for (int i = 0; i < TM; i++) rd_a(0, 0, 0, i);
@@ -161,29 +175,31 @@ __device__ __forceinline__ void g8_mainloop(const void* a, uint32_t lda, uint32_
 #pragma unroll
         for (int kk = 0; kk < 2; kk++) {
             if (kk == 1) {
-                g8_loads_wait<(NW > NA ? (NA - 1) * LB + (NA - 2) * LA : (NA - 2) * (LA + LB))>();
+                g8_loads_wait<g8_flight(LA, NA, LB, NW)>();
                 g8_barrier();
             }
             const uint32_t ra_st = kk ? sa1 : sa, rw_st = kk ? sw1 : sw;
+            constexpr int MF = TM * TN;
 #pragma unroll
-            for (int j = 0; j < TN; j++) {
+            for (int x = 0; x < MF; x++) {
+                const int j = x / TM, i = j & 1 ? TM - 1 - x % TM : x % TM;
+                mfma(kk, i, j);
+                bool side = x % TM == TM - 1;
+                if (side) rd_w(rw_st, kk ^ 1, j);
 #pragma unroll
-                for (int i = 0; i < TM; i++) mfma(kk, j & 1 ? TM - 1 - i : i, j);
-                rd_w(rw_st, kk ^ 1, j);
-                // the inner fragments of the next slice: in the first rows, TM of them
-                constexpr int PER = (2 * TM + TN - 1) / TN;
-#pragma unroll
-                for (int q = 0; q < PER; q++)
-                    if (j * PER + q < TM) rd_a(kk ^ 1, ra_st, kk ^ 1, j * PER + q);
+                for (int q = 0; q < TM; q++)
+                    if (g8_at(q, TM, 0, MF / 2) == x) rd_a(kk ^ 1, ra_st, kk ^ 1, q), side = true;
                 const int n = kk ? LA : LB;
 #pragma unroll
-                for (int q = j * n / TN; q < (j + 1) * n / TN; q++) {
-                    if (kk == 0)
-                        load_w(kt + NW - 1, sw_in, q);
-                    else
-                        load_a(kt + NA, sa, q);
-                }
-                __builtin_amdgcn_sched_barrier(0);
+                for (int q = 0; q < n; q++)
+                    if (g8_at(q, n, 1, MF) == x) {
+                        side = true;
+                        if (kk == 0)
+                            load_w(kt + NW - 1, sw_in, q);
+                        else
+                            load_a(kt + NA, sa, q);
+                    }
+                if (side) __builtin_amdgcn_sched_barrier(0);
             }
         }
         sa = sa1, sw_in = sw, sw = sw1;
@@ -233,20 +249,30 @@ __device__ __forceinline__ void g8_store_partial(f32x4 (&acc)[T::TM][T::TN], flo
 }
 
 // Body of a reduce kernel: grid = cut tiles * (BM / 8) * (BN / 128), 256 threads. Each half wavefront sums the `splits` slots
-// of one row of one 128-column block of a tile, 4 columns a lane, in split order, and hands them to fn(t, row in 0 .. BM - 1,
-// column block, l32, v[4]) with t the tile's index among the cut tiles. The 8 rows of a block are neighbours in the slots.
+// of one row of one 128-column block of a tile, 4 columns a lane, in split order, and hands them to fn(row, first column of
+// the block, l32, v[4]); blocks outside n are left out, rows are not. The 8 rows of a workgroup are neighbours in the slots.
 template <class T, class RowFn>
-__device__ __forceinline__ void g8_reduce_rows(const float* __restrict__ part, uint32_t splits, RowFn fn) {
+__device__ __forceinline__ void g8_reduce_rows(const float* __restrict__ part, uint32_t m, uint32_t n, uint32_t group, uint32_t first,
+                                               uint32_t splits, RowFn fn) {
     constexpr uint32_t CB = T::BN / 128, PER_TILE = T::BM / 8 * CB;
     const uint32_t t = blockIdx.x / PER_TILE, b = blockIdx.x % PER_TILE, l32 = threadIdx.x & 31;
     const uint32_t row = (b / CB) * 8 + (threadIdx.x >> 5), cb = b % CB;
+    uint32_t tm, tn;
+    if constexpr (T::PARTS > 1) {
+        const uint32_t tiles_m = (m + T::BM - 1) / T::BM;
+        tm = t % tiles_m, tn = t / tiles_m;
+    } else {
+        gemm_raster(first + t, (m + 255) / 256, (n + 255) / 256, group, tm, tn);
+    }
+    const uint32_t m0 = tm * T::BM, n0 = tn * T::BN + cb * 128;
+    if (m0 + (b / CB) * 8 >= m || n0 >= n) return;
     const uint32_t c4 = cb * 32 + l32, wn = c4 / (4 * T::TN), j = (c4 / 4) % T::TN, fc = c4 % 4;
     const uint32_t wm = row / (16 * T::TM), i = (row / 16) % T::TM, fr = row % 16;
     const float* p = part + (size_t)t * splits * T::PART_FLOATS + ((i * T::TN + j) * T::THREADS + (wm * T::WN + wn) * 64 + fc * 16 + fr) * 4;
     f32x4 sum = *(const f32x4*)p;
     for (uint32_t sp = 1; sp < splits; sp++) sum += *(const f32x4*)(p + (size_t)sp * T::PART_FLOATS);
     float v[4] = {sum[0], sum[1], sum[2], sum[3]};
-    fn(t, row, cb, l32, v);
+    fn(m0 + row, n0, l32, v);
 }
 
 // The same loop for a weight operand that is packed in memory and expanded to 16-bit values as it becomes a fragment: the
@@ -256,12 +282,12 @@ __device__ __forceinline__ void g8_reduce_rows(const float* __restrict__ part, u
 // 16 g + 8 kk .. + 7, so A's fragments take chunk 2 g + kk (kPerm). Outer loop: A's fragments, in place; inner: the expanded
 // weights, double-buffered.
 // W: kPerm = true, STAGE bytes and LOADS loads a stage, issue(kt, dst of the stage, j, wave), Raw, read(stage in LDS, row of
-// the tile, lane group) -> Raw, expand(Raw, kk) -> f16x8.
+// the tile, lane group) -> Raw, expand(Raw, kk) -> values 8 kk .. + 7.
 template <class T, int NA, int NW, class W>
 __device__ __forceinline__ void g8_mainloop_packed(const _Float16* a, uint32_t lda, uint32_t m, uint32_t kt0, uint32_t ktiles, uint32_t m0,
                                                    const W& wo, unsigned char* lds, f32x4 (&acc)[T::TM][T::TN]) {
     constexpr int TM = T::TM, TN = T::TN, LA = T::BM / 64, LB = W::LOADS, A_STAGE = T::BM * 128, W_AT = NA * A_STAGE;
-    static_assert(NW == NA || NW == NA + 1, "the waits below");
+    static_assert(NA >= 2 && NW >= 2 && g8_flight0(LA, NA, LB, NW) < 64, "loads in flight");
     static_assert(W_AT + NW * W::STAGE <= 160 * 1024, "LDS");
     static_assert(W::kPerm, "A's chunks");
     const uint32_t lane = threadIdx.x & 63, wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
@@ -295,15 +321,17 @@ __device__ __forceinline__ void g8_mainloop_packed(const _Float16* a, uint32_t l
 #pragma unroll
         for (int j = 0; j < TN; j++) acc[i][j] = (f32x4){0.f, 0.f, 0.f, 0.f};
 #pragma unroll
-    for (int t = 0; t < NA; t++) {
-        if (NW - 1 - NA + t >= 0) {
+    for (int t = -(NA > NW - 1 ? NA : NW - 1); t < 0; t++) {
+        if (t - 1 + NW >= 0) {
 #pragma unroll
-            for (int j = 0; j < LB; j++) load_w(NW - 1 - NA + t, NW - 1 - NA + t, j);
+            for (int j = 0; j < LB; j++) load_w(t - 1 + NW, t - 1 + NW, j);
         }
+        if (t + NA >= 0) {
 #pragma unroll
-        for (int j = 0; j < LA; j++) load_a(t, t, j);
+            for (int j = 0; j < LA; j++) load_a(t + NA, t + NA, j);
+        }
     }
-    g8_loads_wait<(NW > NA ? (NA - 1) * (LA + LB) : (NA - 1) * LA + (NA > 1 ? (NA - 2) * LB : 0))>();
+    g8_loads_wait<g8_flight0(LA, NA, LB, NW)>();
     g8_barrier();
 #pragma unroll
     for (int j = 0; j < TN; j++) rd_raw(0, j);
@@ -318,41 +346,37 @@ __device__ __forceinline__ void g8_mainloop_packed(const _Float16* a, uint32_t l
 #pragma unroll
         for (int kk = 0; kk < 2; kk++) {
             if (kk == 1) {
-                g8_loads_wait<(NW > NA ? (NA - 1) * LB + (NA - 2) * LA : (NA - 2) * (LA + LB))>();
+                g8_loads_wait<g8_flight(LA, NA, LB, NW)>();
                 g8_barrier();
             }
             const uint32_t ra_st = kk ? sa1 : sa;
+            constexpr int MF = TM * TN;
 #pragma unroll
-            for (int i = 0; i < TM; i++) {
+            for (int x = 0; x < MF; x++) {
+                const int i = x / TN, j = i & 1 ? TN - 1 - x % TN : x % TN;
+                acc[i][j] = __builtin_amdgcn_mfma_f32_16x16x32_f16(fw[kk][j], fa[i], acc[i][j], 0, 0, 0);
+                bool side = x % TN == TN - 1;
+                if (side) rd_a(ra_st, kk ^ 1, i);
+                // slice 0: the second half of this tile's codes; slice 1: the next tile's codes, then their first half
+                if (kk == 1) {
 #pragma unroll
-                for (int j = 0; j < TN; j++) {
-                    const int jj = i & 1 ? TN - 1 - j : j;
-                    acc[i][jj] = __builtin_amdgcn_mfma_f32_16x16x32_f16(fw[kk][jj], fa[i], acc[i][jj], 0, 0, 0);
+                    for (int q = 0; q < TN; q++)
+                        if (g8_at(q, TN, 0, MF / 4) == x) rd_raw(sw1, q), side = true;
                 }
-                rd_a(ra_st, kk ^ 1, i);
-                if (kk == 0) {  // the second half of this tile's codes, spread over the slice
 #pragma unroll
-                    for (int j = i * TN / TM; j < (i + 1) * TN / TM; j++) fw[1][j] = wo.expand(raw[j], 1);
-                } else {  // the next tile's codes, then their first half in the slice's second half
-                    if (i == 0) {
-#pragma unroll
-                        for (int j = 0; j < TN; j++) rd_raw(sw1, j);
-                    }
-                    constexpr int H = TM / 2;
-                    if (i >= H) {
-#pragma unroll
-                        for (int j = (i - H) * TN / (TM - H); j < (i - H + 1) * TN / (TM - H); j++) fw[0][j] = wo.expand(raw[j], 0);
-                    }
-                }
+                for (int q = 0; q < TN; q++)
+                    if (g8_at(q, TN, kk ? MF / 2 : 1, MF) == x) fw[kk ^ 1][q] = wo.expand(raw[q], kk ^ 1), side = true;
                 const int n = kk ? LA : LB;
 #pragma unroll
-                for (int q = i * n / TM; q < (i + 1) * n / TM; q++) {
-                    if (kk == 0)
-                        load_w(kt + NW - 1, sw_in, q);
-                    else
-                        load_a(kt + NA, sa, q);
-                }
-                __builtin_amdgcn_sched_barrier(0);
+                for (int q = 0; q < n; q++)
+                    if (g8_at(q, n, 1, MF) == x) {
+                        side = true;
+                        if (kk == 0)
+                            load_w(kt + NW - 1, sw_in, q);
+                        else
+                            load_a(kt + NA, sa, q);
+                    }
+                if (side) __builtin_amdgcn_sched_barrier(0);
             }
         }
         sa = sa1, sw_in = sw, sw = sw1;
@@ -365,16 +389,20 @@ __device__ __forceinline__ void g8_mainloop_packed(const _Float16* a, uint32_t l
 // decoded once, by the thread that has its words, and written into LDS as 16-bit rows (as G8Dense's). The packed words of a k tile go
 // into LDS as they are (NR stages); a thread reads its words of tile t + 2 in slice 1 of tile t, decodes and writes their
 // first half there and their second half in slice 0 of tile t + 1, always into the weight stage the barrier before has freed.
-// Two stages of A, two of decoded weights.
+// NA stages of A, two of decoded weights.
 // W: RAW_STAGE bytes and LOADS loads a packed stage, issue(kt, dst of the stage, j, wave), Words, read(stage in LDS) -> Words,
-// store(words, half 0 or 1, weight stage).
-template <class T, int NR, class W>
+// prepare(words), OPS 8-value chunks a thread, pair(words, chunk, p) -> values 2 p, 2 p + 1 of a chunk as packed fp16,
+// put(weight stage, chunk, 4 pairs).
+template <class T, int NA, int NR, class W>
 __device__ __forceinline__ void g8_mainloop_decode(const _Float16* a, uint32_t lda, uint32_t m, uint32_t kt0, uint32_t ktiles, uint32_t m0,
                                                    const W& wo, unsigned char* lds, f32x4 (&acc)[T::TM][T::TN]) {
     constexpr int TM = T::TM, TN = T::TN, LA = T::BM / 64, LR = W::LOADS, A_STAGE = T::BM * 128, W_STAGE = T::BN * 128;
-    constexpr int W_AT = 2 * A_STAGE, R_AT = W_AT + 2 * W_STAGE;
+    constexpr int W_AT = NA * A_STAGE, R_AT = W_AT + 2 * W_STAGE;
     static_assert(R_AT + NR * W::RAW_STAGE <= 160 * 1024, "LDS");
-    static_assert(NR == 2 || NR == 3, "the waits below");
+    static_assert(NA >= 2 && NR >= 2 && NA <= NR + 1, "stages");
+    // In slice 1 of tile t the loads of A of tile t + NA, then the packed ones of tile t + 1 + NR. At the barrier of tile t A of tile
+    // t + 1 and the packed tile t + 2 have to be there: issued in tiles t + 1 - NA and t + 1 - NR.
+    constexpr int FLIGHT = NR >= NA ? (NA - 2) * (LA + LR) + (NR > NA ? LR : 0) : (NR - 2) * (LA + LR);
     const uint32_t lane = threadIdx.x & 63, wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
     const uint32_t wm = wave / T::WN, wn = wave % T::WN;
     const u32x4 ra = g8_rsrc(a, m * lda * 2);
@@ -400,28 +428,42 @@ __device__ __forceinline__ void g8_mainloop_decode(const _Float16* a, uint32_t l
     auto rd_a = [&](int set, uint32_t st, int kk, int i) { fa[set][i] = *(const f16x8*)(pa + st * A_STAGE + 2048 * i + foff[kk]); };
     auto rd_w = [&](uint32_t st, int kk, int j) { fw[j] = *(const f16x8*)(pw + st * W_STAGE + 2048 * j + foff[kk]); };
     auto words = [&](uint32_t st) { return wo.read(lds + R_AT + st * W::RAW_STAGE); };
-    auto put = [&](const typename W::Words& w, int half, uint32_t st) { wo.store(w, half, lds + W_AT + st * W_STAGE); };
+    constexpr int OPS = W::OPS;
+    typename W::Words w;
+    u32x4 chunk;
+    // pair p of the thread's share of a tile; behind the last of a chunk the chunk goes to weight stage st
+    auto decode = [&](int p, uint32_t st) {
+        chunk[p % 4] = wo.pair(w, p / 4, p % 4);
+        if (p % 4 == 3) wo.put(lds + W_AT + st * W_STAGE, p / 4, chunk);
+    };
 #pragma unroll
     for (int i = 0; i < TM; i++)
 #pragma unroll
         for (int j = 0; j < TN; j++) acc[i][j] = (f32x4){0.f, 0.f, 0.f, 0.f};
 
+    // prologue: the loads in the order of the loop's own, as of tiles before the first, but for packed tile NR, whose stage is not free yet
 #pragma unroll
-    for (int t = 0; t < NR; t++)
+    for (int t = -(NR + 1); t < 0; t++) {
+        if (t + NA >= 0) {
 #pragma unroll
-        for (int j = 0; j < LR; j++) load_r(t, t, j);
+            for (int j = 0; j < LA; j++) load_a(t + NA, t + NA, j);
+        }
+        if (t < -1) {
 #pragma unroll
-    for (int t = 0; t < 2; t++)
-#pragma unroll
-        for (int j = 0; j < LA; j++) load_a(t, t, j);
-    g8_loads_wait<2 * LA>();  // the packed tiles
+            for (int j = 0; j < LR; j++) load_r(t + 1 + NR, t + 1 + NR, j);
+        }
+    }
+    g8_loads_wait<(NR - 2) * LR + (NR - 1 < NA ? NR - 1 : NA) * LA>();  // packed tiles 0 and 1
     g8_barrier();
-    typename W::Words w = words(0);
-    put(w, 0, 0);
-    put(w, 1, 0);
+    w = words(0);
+    wo.prepare(w);
+#pragma unroll
+    for (int p = 0; p < 4 * OPS; p++) decode(p, 0);
     w = words(1);
-    put(w, 0, 1);
-    g8_loads_wait<LA>();  // A of tile 0
+    wo.prepare(w);
+#pragma unroll
+    for (int p = 0; p < 2 * OPS; p++) decode(p, 1);
+    g8_loads_wait<(NA - 1) * LA + (NA - 1 < NR ? NA - 1 : NR) * LR>();  // A of tile 0
     g8_barrier();
 #pragma unroll
     for (int j = 0; j < LR; j++) load_r(NR, 0, j);
@@ -430,44 +472,49 @@ __device__ __forceinline__ void g8_mainloop_decode(const _Float16* a, uint32_t l
 #pragma unroll
     for (int j = 0; j < TN; j++) rd_w(0, 0, j);
 
-    uint32_t sr = NR == 2 ? 0 : 2, sr_in = 1;  // the packed stage of tile kt + 2; the one that slice 1 of tile kt fills (tile kt + 1 + NR)
+    uint32_t sa = 0, sr = 2 % NR, sr_in = 1;  // stage of A of tile kt; the packed stage of tile kt + 2; the one that slice 1 of tile kt fills (tile kt + 1 + NR)
     for (uint32_t kt = 0; kt < ktiles; kt++) {
-        const uint32_t s = kt & 1;
+        const uint32_t s = kt & 1, sa1 = next(sa, NA);  // (decoded weights: two stages)
 #pragma unroll
         for (int kk = 0; kk < 2; kk++) {
             if (kk == 1) {
-                g8_loads_wait<(NR == 3 ? LR : 0)>();
+                g8_loads_wait<FLIGHT>();
                 g8_barrier();
             }
             const uint32_t st = kk ? s ^ 1 : s;
+            constexpr int MF = TM * TN;
 #pragma unroll
-            for (int j = 0; j < TN; j++) {
+            for (int x = 0; x < MF; x++) {
+                const int j = x / TM, i = j & 1 ? TM - 1 - x % TM : x % TM;
+                acc[i][j] = __builtin_amdgcn_mfma_f32_16x16x32_f16(fw[j], fa[kk][i], acc[i][j], 0, 0, 0);
+                bool side = x % TM == TM - 1;
+                if (side) rd_w(st, kk ^ 1, j);
 #pragma unroll
-                for (int i = 0; i < TM; i++) {
-                    const int ii = j & 1 ? TM - 1 - i : i;
-                    acc[ii][j] = __builtin_amdgcn_mfma_f32_16x16x32_f16(fw[j], fa[kk][ii], acc[ii][j], 0, 0, 0);
+                for (int q = 0; q < TM; q++)
+                    if (g8_at(q, TM, 0, MF / 2) == x) rd_a(kk ^ 1, kk ? sa1 : sa, kk ^ 1, q), side = true;
+                // slice 0: the second half of tile kt + 1; slice 1: the words of tile kt + 2, then their first half
+                if (kk == 1) {
+                    if (x == 0) w = words(sr), side = true;
+                    if (x == MF / 4) wo.prepare(w), side = true;
                 }
-                rd_w(st, kk ^ 1, j);
-                constexpr int PER = (2 * TM + TN - 1) / TN;
 #pragma unroll
-                for (int q = 0; q < PER; q++)
-                    if (j * PER + q < TM) rd_a(kk ^ 1, st, kk ^ 1, j * PER + q);
-                if (kk == 0) {  // second half of tile kt + 1
-                    if (j == 1) put(w, 1, s ^ 1);
-                } else {  // words and first half of tile kt + 2
-                    if (j == 0) w = words(sr);
-                    if (j == TN - 2) put(w, 0, s);
+                for (int q = 0; q < 2 * OPS; q++)
+                    if (g8_at(q, 2 * OPS, kk ? MF / 4 : 0, kk ? MF : MF * 7 / 8) == x) decode(kk ? q : 2 * OPS + q, kk ? s : s ^ 1), side = true;
+                if (kk == 1) {
 #pragma unroll
-                    for (int q = j * LA / TN; q < (j + 1) * LA / TN; q++) load_a(kt + 2, s, q);
-                    if (j == TN - 1) {
-#pragma unroll
-                        for (int q = 0; q < LR; q++) load_r(kt + 1 + NR, sr_in, q);
-                    }
+                    for (int q = 0; q < LA + LR; q++)
+                        if (g8_at(q, LA + LR, 1, MF) == x) {
+                            side = true;
+                            if (q < LA)
+                                load_a(kt + NA, sa, q);
+                            else
+                                load_r(kt + 1 + NR, sr_in, q - LA);
+                        }
                 }
-                __builtin_amdgcn_sched_barrier(0);
+                if (side) __builtin_amdgcn_sched_barrier(0);
             }
         }
-        sr = next(sr, NR), sr_in = next(sr_in, NR);
+        sa = sa1, sr = next(sr, NR), sr_in = next(sr_in, NR);
     }
     asm volatile("s_waitcnt vmcnt(0)" ::: "memory");
     __syncthreads();
@@ -485,8 +532,8 @@ __device__ __forceinline__ void g8_mainloop_f8(const uint8_t* a, uint32_t lda, u
                                                const G8Dense<T>& wo, unsigned char* lds, f32x4 (&acc)[T::TM][T::TN]) {
     constexpr int TM = T::TM, TN = T::TN, R = 4, LA = T::BM / 64, LB = G8Dense<T>::LOADS, A_STAGE = T::BM * 128, W_AT = NA * A_STAGE;
     constexpr int W_STAGE = G8Dense<T>::STAGE, BAR = TN - R;  // the barrier follows column BAR
-    static_assert(TN >= 2 * R || TN == R, "columns 0 .. TN - R - 1 refill from this tile");
-    static_assert(NW == NA || NW == NA + 1, "the waits below");
+    static_assert(TN == 2 * R || TN == R, "a ring of half or of all the columns");
+    static_assert(NA >= 2 && NW >= 2 && g8_flight0(LA, NA, LB, NW) < 64, "loads in flight");
     static_assert(W_AT + NW * W_STAGE <= 160 * 1024, "LDS");
     const uint32_t lane = threadIdx.x & 63, wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
     const uint32_t wm = wave / T::WN, wn = wave % T::WN;
@@ -520,15 +567,17 @@ __device__ __forceinline__ void g8_mainloop_f8(const uint8_t* a, uint32_t lda, u
 #pragma unroll
         for (int j = 0; j < TN; j++) acc[i][j] = (f32x4){0.f, 0.f, 0.f, 0.f};
 #pragma unroll
-    for (int t = 0; t < NA; t++) {
-        if (NW - 1 - NA + t >= 0) {
+    for (int t = -(NA > NW - 1 ? NA : NW - 1); t < 0; t++) {
+        if (t - 1 + NW >= 0) {
 #pragma unroll
-            for (int j = 0; j < LB; j++) load_w(NW - 1 - NA + t, NW - 1 - NA + t, j);
+            for (int j = 0; j < LB; j++) load_w(t - 1 + NW, t - 1 + NW, j);
         }
+        if (t + NA >= 0) {
 #pragma unroll
-        for (int j = 0; j < LA; j++) load_a(t, t, j);
+            for (int j = 0; j < LA; j++) load_a(t + NA, t + NA, j);
+        }
     }
-    g8_loads_wait<(NW > NA ? (NA - 1) * (LA + LB) : (NA - 1) * LA + (NA > 1 ? (NA - 2) * LB : 0))>();
+    g8_loads_wait<g8_flight0(LA, NA, LB, NW)>();
     g8_barrier();
 #pragma unroll
     for (int i = 0; i < TM; i++) rd_a(0, i);
@@ -545,7 +594,11 @@ __device__ __forceinline__ void g8_mainloop_f8(const uint8_t* a, uint32_t lda, u
                 acc[i][j] = __builtin_amdgcn_mfma_scale_f32_16x16x128_f8f6f4(fw[j % R], fa[i], acc[i][j], 0, 0, 0, 0, 0, 0);
             }
             if (j == BAR) {
-                g8_loads_wait<(NW > NA ? (NA - 1) * LB + (NA - 2) * LA : (NA - 2) * (LA + LB))>();
+                if (BAR == 0) {  // no column before it: the weight loads come here
+#pragma unroll
+                    for (int q = 0; q < LB; q++) load_w(kt + NW - 1, sw_in, q);
+                }
+                g8_loads_wait<g8_flight(LA, NA, LB, NW)>();
                 g8_barrier();
             }
             rd_w(j < BAR ? sw : sw1, (j + R) % TN);
@@ -556,7 +609,7 @@ __device__ __forceinline__ void g8_mainloop_f8(const uint8_t* a, uint32_t lda, u
             // loads: W in the columns before the barrier, A after it
             if (j < BAR) {
 #pragma unroll
-                for (int q = j * LB / BAR; q < (j + 1) * LB / BAR; q++) load_w(kt + NW - 1, sw_in, q);
+                for (int q = j * LB / (BAR > 0 ? BAR : 1); q < (j + 1) * LB / (BAR > 0 ? BAR : 1); q++) load_w(kt + NW - 1, sw_in, q);
             } else {
 #pragma unroll
                 for (int q = (j - BAR) * LA / R; q < (j - BAR + 1) * LA / R; q++) load_a(kt + NA, sa, q);
@@ -633,20 +686,43 @@ __device__ __forceinline__ bool g8_sk_meet(f32x4 (&acc)[T::TM][T::TN], uint32_t 
     return true;
 }
 
-// Runs the program's share of the schedule: main(tm, tn, kt0, ktn, acc) is one pass of the main loop over k tiles
-// kt0 .. kt0 + ktn - 1 of tile (tm, tn), finish(tm, tn, acc) the tile's epilogue. sc.sk_base is nonzero exactly when SK.
+// The small tiles of a launch: tile t = column tile * row tiles + row tile, piece `piece` of its K, for the program `pid` of
+// `grid` = tiles * splits. Workgroups go to the 8 XCDs round-robin; the grid is dealt so that an XCD takes a contiguous range
+// of (column tile, piece, row tile), row tiles fastest: those of one column tile and piece read the same weights through one
+// L2, and no XCD has more than one program more than another.
+struct G8SmallWork {
+    uint32_t tm, tn, tile, piece;
+};
+__device__ __forceinline__ G8SmallWork g8_small_work(uint32_t pid, uint32_t grid, uint32_t tiles_m, uint32_t splits) {
+    const uint32_t x = pid % 8, per = grid / 8, rem = grid % 8;
+    const uint32_t l = x * per + (x < rem ? x : rem) + pid / 8;
+    const uint32_t tm = l % tiles_m, q = l / tiles_m;
+    return G8SmallWork{tm, q / splits, q / splits * tiles_m + tm, q % splits};
+}
+
+// Runs the program's share of the schedule: main(m0, n0, kt0, ktn, acc) is one pass of the main loop over k tiles
+// kt0 .. kt0 + ktn - 1 of the tile at row m0, column n0, finish(m0, n0, acc) the tile's epilogue. sc.sk_base is nonzero exactly
+// when SK.
 template <class T, bool SK, class Main, class Finish>
-__device__ __forceinline__ void g8_schedule(const GemmSched& sc, uint32_t tiles_m, uint32_t tiles_n, uint32_t group, uint32_t ktiles,
+__device__ __forceinline__ void g8_schedule(const GemmSched& sc, uint32_t m, uint32_t n, uint32_t group, uint32_t ktiles,
                                             unsigned char* lds, Main main, Finish finish) {
-    const uint32_t p = blockIdx.x;
+    const uint32_t p = blockIdx.x, tiles_m = (m + 255) / 256, tiles_n = (n + 255) / 256;
     f32x4 acc[T::TM][T::TN];
-    if constexpr (!SK) {
+    if constexpr (T::PARTS > 1) {
+        const G8SmallWork wk = g8_small_work(p, gridDim.x, (m + T::BM - 1) / T::BM, sc.splits);
+        const uint32_t kt0 = wk.piece * ktiles / sc.splits;
+        main(wk.tm * T::BM, wk.tn * T::BN, kt0, (wk.piece + 1) * ktiles / sc.splits - kt0, acc);
+        if (sc.splits > 1)
+            g8_store_partial<T>(acc, sc.part + (size_t)(wk.tile * sc.splits + wk.piece) * T::PART_FLOATS);
+        else
+            finish(wk.tm * T::BM, wk.tn * T::BN, acc);
+    } else if constexpr (!SK) {
         const GemmWork wk = gemm_work(p, tiles_m, tiles_n, group, ktiles, sc.full_tiles, sc.splits);
-        main(wk.tm, wk.tn, wk.kt0, wk.ktn, acc);
+        main(wk.tm * T::BM, wk.tn * T::BN, wk.kt0, wk.ktn, acc);
         if (wk.partial)
             g8_store_partial<T>(acc, sc.part + (size_t)wk.slot * T::PART_FLOATS);
         else
-            finish(wk.tm, wk.tn, acc);
+            finish(wk.tm * T::BM, wk.tn * T::BN, acc);
     } else {
         const uint32_t whole = sc.full_tiles;  // taken whole, program p those p, p + grid, ...; the runs lie over the tiles after them
         uint32_t next_whole = p;
@@ -667,11 +743,11 @@ __device__ __forceinline__ void g8_schedule(const GemmSched& sc, uint32_t tiles_
             uint32_t tm, tn;
             gemm_raster(tile, tiles_m, tiles_n, group, tm, tn);
             __syncthreads();  // the epilogue of the segment before is done with the LDS
-            main(tm, tn, kt0, ktn, acc);
+            main(tm * T::BM, tn * T::BN, kt0, ktn, acc);
             bool fin = true;
             if (ktn != ktiles)
                 fin = g8_sk_meet<T>(acc, p, tile, t0, ktiles, sc.sk_base, sc.sk_rem, sc.part, sc.part_bytes, sc.counters, lds);
-            if (fin) finish(tm, tn, acc);
+            if (fin) finish(tm * T::BM, tn * T::BN, acc);
         }
     }
 }

@@ -17,56 +17,60 @@ __device__ __forceinline__ void bf16_store4(uint16_t* c, const uint16_t* res, si
 
 // ---- GEMM ------------------------------------------------------------------------------------------------------------
 
-typedef G8Tile<4, 2, 4, 8> Bf16Tile;  // 256 x 256
-#define BF16_GEMM_STAGES 2, 3         // k tiles of A and of W in LDS: all 160 KB
+typedef G8Tile<4, 2, 4, 8> Bf16Tile;    // 256 x 256
+typedef G8Tile<4, 2, 2, 8> Bf16TileS1;  // 128 x 256
+typedef G8Tile<4, 2, 2, 4> Bf16TileS2;  // 128 x 128, two programs a CU
+// k tiles of A and of W in LDS: as many as the tile leaves room for
+template <class T>
+struct Bf16Stages {
+    static constexpr int NA = T::PARTS == 2 ? 3 : 2, NW = 3, MIN_WAVES = T::PARTS == 4 ? 4 : 2;
+};
 
-// One program's share of A . W^T: main loop, then the partial slot (a tile cut along K) or done(row, col, v[4]) for every
-// row piece of the tile, all lanes of a row calling (row >= m and col >= n included).
+// One program's share of A . W^T: main loop, then the partial slot (a tile cut along K) or done(row, col, lane in row, v[4]) for
+// every row piece of the tile, all lanes of a row calling (row >= m and col >= n included).
 template <class T, class Done>
 __device__ __forceinline__ void bf16_gemm_program(const uint16_t* a, const uint16_t* w, uint32_t m, uint32_t n, uint32_t k, uint32_t lda,
-                                                  uint32_t group_m, uint32_t full_tiles, uint32_t splits, float* part, Done done) {
+                                                  uint32_t group_m, const GemmSched& sc, Done done) {
     extern __shared__ __attribute__((aligned(1024))) unsigned char lds[];
     const uint32_t wave = threadIdx.x >> 6, wm = wave / T::WN, wn = wave % T::WN;
-    const GemmWork wk = gemm_work(blockIdx.x, (m + T::BM - 1) / T::BM, (n + T::BN - 1) / T::BN, group_m, k / G8_BK, full_tiles, splits);
-    G8Dense<T> wo;
-    wo.rows(w, n, k, wk.tn * T::BN);
-    f32x4 acc[T::TM][T::TN];
-    g8_mainloop<T, BF16_GEMM_STAGES, true>(a, lda, m, wk.kt0, wk.ktn, wk.tm * T::BM, wo, lds, acc);
-    if (wk.partial) {
-        g8_store_partial<T>(acc, part + (size_t)wk.slot * T::PART_FLOATS);
-        return;
+    g8_schedule<T, false>(
+        sc, m, n, group_m, k / G8_BK, lds,
+        [&](uint32_t m0, uint32_t n0, uint32_t kt0, uint32_t ktn, f32x4(&acc)[T::TM][T::TN]) {
+            G8Dense<T> wo;
+            wo.rows(w, n, k, n0);
+            g8_mainloop<T, Bf16Stages<T>::NA, Bf16Stages<T>::NW, true>(a, lda, m, kt0, ktn, m0, wo, lds, acc);
+        },
+        [&](uint32_t m0, uint32_t n0, f32x4(&acc)[T::TM][T::TN]) {
+            const uint32_t row0 = m0 + wm * 16 * T::TM, col0 = n0 + wn * 16 * T::TN;
+            g8_epilogue<T>(
+                acc, lds, [](auto&, uint32_t) {},
+                [&](uint32_t row, uint32_t lc, float (&v)[4]) { done(row0 + row, col0 + 4 * lc, lc, v); });
+        });
+}
+
+// C[M][ldc] = bf16(A . W^T) (+ res); A bf16 [M][lda], W bf16 [N][K]. The grid's programs share the tiles as sc says (g8_schedule);
+// 512 threads, dynamic LDS as the stages of the tile take; tiles cut along K leave partials for the reduce kernel.
+// K % 64 == 0, N % 8 == 0, lda % 8 == 0, ldc % 4 == 0, operands under 4 GB. NAME: 256 x 256 tiles; NAME_s1: 128 x 256;
+// NAME_s2: 128 x 128. (kernels/k-core/src/gemm.rs:128-167: fe_gemm_bf16, tile 128 x 128 x 32 on mma.m16n8k16 there)
+#define BF16_GEMM_KERNELS(SUFFIX, TILE)                                                                                    \
+    extern "C" __global__ __launch_bounds__(512, Bf16Stages<TILE>::MIN_WAVES) void fe_gemm_bf16##SUFFIX(                   \
+        uint16_t* c, const uint16_t* a, const uint16_t* w, const uint16_t* res, uint32_t m, uint32_t n, uint32_t k,        \
+        uint32_t lda, uint32_t ldc, uint32_t group_m, GemmSched sc) {                                                      \
+        bf16_gemm_program<TILE>(a, w, m, n, k, lda, group_m, sc, [&](uint32_t row, uint32_t col, uint32_t, float (&v)[4]) { \
+            if (row < m && col < n) bf16_store4(c, res, (size_t)row * ldc + col, v);                                       \
+        });                                                                                                                \
+    }                                                                                                                      \
+    extern "C" __global__ __launch_bounds__(256) void fe_gemm_bf16_reduce##SUFFIX(                                         \
+        uint16_t* c, const float* part, const uint16_t* res, uint32_t m, uint32_t n, uint32_t ldc, uint32_t group_m,       \
+        uint32_t first, uint32_t splits) {                                                                                 \
+        g8_reduce_rows<TILE>(part, m, n, group_m, first, splits, [&](uint32_t row, uint32_t n0, uint32_t l32, float (&v)[4]) { \
+            const uint32_t col = n0 + 4 * l32;                                                                             \
+            if (row < m && col < n) bf16_store4(c, res, (size_t)row * ldc + col, v);                                       \
+        });                                                                                                                \
     }
-    const uint32_t m0 = wk.tm * T::BM + wm * 16 * T::TM, n0 = wk.tn * T::BN + wn * 16 * T::TN;
-    g8_epilogue<T>(
-        acc, lds, [](auto&, uint32_t) {}, [&](uint32_t row, uint32_t lc, float (&v)[4]) { done(m0 + row, n0 + 4 * lc, lc, v); });
-}
-
-// C[M][ldc] = bf16(A . W^T) (+ res); A bf16 [M][lda], W bf16 [N][K]. grid full_tiles + (tiles - full_tiles) * splits with
-// tiles = ceil(M / 256) * ceil(N / 256), 512 threads, dynamic LDS 160 KB; tiles past full_tiles leave partials in
-// `part` for fe_gemm_bf16_reduce. K % 64 == 0, N % 8 == 0, lda % 8 == 0, ldc % 4 == 0, operands under 4 GB.
-// (kernels/k-core/src/gemm.rs:128-167: fe_gemm_bf16, tile 128 x 128 x 32 on mma.m16n8k16 there)
-extern "C" __global__ __launch_bounds__(512, 2) void fe_gemm_bf16(uint16_t* c, const uint16_t* a, const uint16_t* w,
-                                                                  const uint16_t* res, uint32_t m, uint32_t n, uint32_t k,
-                                                                  uint32_t lda, uint32_t ldc, uint32_t group_m,
-                                                                  uint32_t full_tiles, uint32_t splits, float* part) {
-    bf16_gemm_program<Bf16Tile>(a, w, m, n, k, lda, group_m, full_tiles, splits, part,
-                                [&](uint32_t row, uint32_t col, uint32_t, float (&v)[4]) {
-                                    if (row < m && col < n) bf16_store4(c, res, (size_t)row * ldc + col, v);
-                                });
-}
-
-// Finishes the tiles fe_gemm_bf16 cut along K. grid (tiles - full_tiles) * 64, 256 threads.
-extern "C" __global__ __launch_bounds__(256) void fe_gemm_bf16_reduce(uint16_t* c, const float* part, const uint16_t* res,
-                                                                      uint32_t m, uint32_t n, uint32_t ldc, uint32_t group_m,
-                                                                      uint32_t full_tiles, uint32_t splits) {
-    typedef Bf16Tile T;
-    g8_reduce_rows<T>(part, splits, [&](uint32_t t, uint32_t row, uint32_t cb, uint32_t l32, float (&v)[4]) {
-        uint32_t tm, tn;
-        gemm_raster(full_tiles + t, (m + T::BM - 1) / T::BM, (n + T::BN - 1) / T::BN, group_m, tm, tn);
-        const uint32_t grow = tm * T::BM + row, col = tn * T::BN + cb * 128 + 4 * l32;
-        if (grow < m && col < n) bf16_store4(c, res, (size_t)grow * ldc + col, v);
-    });
-}
+BF16_GEMM_KERNELS(, Bf16Tile)
+BF16_GEMM_KERNELS(_s1, Bf16TileS1)
+BF16_GEMM_KERNELS(_s2, Bf16TileS2)
 
 // SwiGLU over a gate|up linear whose weight rows are interleaved in blocks of 8 ([gate 0..8, up 0..8, gate 8..16, ...],
 // fe_interleave_gu): of the 4 lanes that hold one 16-column block of a row, lanes 0, 1 have the 8 gate sums and lanes 2, 3
@@ -85,28 +89,24 @@ __device__ __forceinline__ void bf16_swiglu_store4(uint16_t* act, const float (&
 }
 
 // act[M][N / 2] = SwiGLU(A . W^T) for interleaved gate|up weights W [N][K], N % 16 == 0: fe_gemm_bf16 with the epilogue
-// above (and fe_gemm_bf16_swiglu_reduce for the tiles cut along K). (kernels/k-core/src/gemm.rs:264-279: fe_gemm_swiglu)
-extern "C" __global__ __launch_bounds__(512, 2) void fe_gemm_bf16_swiglu(uint16_t* act, const uint16_t* a, const uint16_t* w,
-                                                                         uint32_t m, uint32_t n, uint32_t k, uint32_t lda,
-                                                                         uint32_t group_m, uint32_t full_tiles,
-                                                                         uint32_t splits, float* part) {
-    bf16_gemm_program<Bf16Tile>(a, w, m, n, k, lda, group_m, full_tiles, splits, part,
-                                [&](uint32_t row, uint32_t col, uint32_t lc, float (&v)[4]) {
-                                    bf16_swiglu_store4(act, v, lc, row < m, row, col, n);
-                                });
-}
-
-extern "C" __global__ __launch_bounds__(256) void fe_gemm_bf16_swiglu_reduce(uint16_t* act, const float* part, uint32_t m,
-                                                                             uint32_t n, uint32_t group_m,
-                                                                             uint32_t full_tiles, uint32_t splits) {
-    typedef Bf16Tile T;
-    g8_reduce_rows<T>(part, splits, [&](uint32_t t, uint32_t row, uint32_t cb, uint32_t l32, float (&v)[4]) {
-        uint32_t tm, tn;
-        gemm_raster(full_tiles + t, (m + T::BM - 1) / T::BM, (n + T::BN - 1) / T::BN, group_m, tm, tn);
-        const uint32_t grow = tm * T::BM + row, col = tn * T::BN + cb * 128 + 4 * l32;
-        bf16_swiglu_store4(act, v, l32, grow < m, grow, col, n);
-    });
-}
+// above, and its reduce kernels. (kernels/k-core/src/gemm.rs:264-279: fe_gemm_swiglu)
+#define BF16_SWIGLU_KERNELS(SUFFIX, TILE)                                                                                  \
+    extern "C" __global__ __launch_bounds__(512, Bf16Stages<TILE>::MIN_WAVES) void fe_gemm_bf16_swiglu##SUFFIX(            \
+        uint16_t* act, const uint16_t* a, const uint16_t* w, uint32_t m, uint32_t n, uint32_t k, uint32_t lda,             \
+        uint32_t group_m, GemmSched sc) {                                                                                  \
+        bf16_gemm_program<TILE>(a, w, m, n, k, lda, group_m, sc, [&](uint32_t row, uint32_t col, uint32_t lc, float (&v)[4]) { \
+            bf16_swiglu_store4(act, v, lc, row < m, row, col, n);                                                          \
+        });                                                                                                                \
+    }                                                                                                                      \
+    extern "C" __global__ __launch_bounds__(256) void fe_gemm_bf16_swiglu_reduce##SUFFIX(                                  \
+        uint16_t* act, const float* part, uint32_t m, uint32_t n, uint32_t group_m, uint32_t first, uint32_t splits) {      \
+        g8_reduce_rows<TILE>(part, m, n, group_m, first, splits, [&](uint32_t row, uint32_t n0, uint32_t l32, float (&v)[4]) { \
+            bf16_swiglu_store4(act, v, l32, row < m, row, n0 + 4 * l32, n);                                                \
+        });                                                                                                                \
+    }
+BF16_SWIGLU_KERNELS(, Bf16Tile)
+BF16_SWIGLU_KERNELS(_s1, Bf16TileS1)
+BF16_SWIGLU_KERNELS(_s2, Bf16TileS2)
 
 // dst row 16 b + i = gate row 8 b + i for i < 8, up row 8 b + i - 8 otherwise: the weight layout of fe_gemm_bf16_swiglu.
 // grid 2 inter, 256 threads; k % 8 == 0. (kernels/k-core/src/gemm.rs:281-296: fe_interleave_gu)

@@ -1,41 +1,8 @@
 // EXL3 (trellis-coded, Hadamard-rotated) linear for gfx950: input rotation, the decode GEMV for 1..64 rows,
-// whole-tensor reconstruct, and probes.
-//
-// The trellis of a 16x16 tile is a cyclic stream of 256 * BITS bits, most significant bit of each u32 first; position t
-// owns the 16-bit state ending at stream bit (t + 1) * BITS (crates/fe-exl3/src/cpu.rs:12-23). Position
-// t = 8 * f + i sits at row k = 2 (f & 3) + (i & 1) + 8 ((i >> 1) & 1), column n = (f >> 2) + 8 (i >> 2) of the tile
-// (crates/fe-exl3/src/format.rs:146-156). A state decodes to fp16 by the mul1 codebook
-// (crates/fe-exl3/src/cpu.rs:25-43, kernels/k-exl3/src/util.rs:76-85).
+// whole-tensor reconstruct, and probes. (The prefill GEMMs are in k_exl3_gemm.hip, the decode in exl3_trellis.h.)
 #include <type_traits>
 
-#include "gemm8.h"
-
-// ---- the mul1 codebook ------------------------------------------------------------------------------------------
-
-// x = state * 0x83DCD12D mod 2^32 for the 16-bit state in the low (HI = 0) or high (HI = 1) half of r; the other half
-// of r may hold anything. On gfx950 v_mul_lo_u32 issues at the same rate as the other 3-operand integer instructions,
-// while the shift or mask that isolates the state is one of the double-rate simple instructions.
-template <int HI>
-__device__ __forceinline__ uint32_t mul1_x(uint32_t r) {
-    uint32_t s = HI ? (r >> 16) : (r & 0xffffu);
-    return s * 0x83DCD12Du;
-}
-
-// Two codebook values as packed fp16 (x0's in the low half): 0x6400 + byte sum is fp16(1024 + sum); one fused
-// fp16 multiply-add by 0x1eee with 0xc931 added, a single rounding per value.
-__device__ __forceinline__ uint32_t mul1_finish2(uint32_t x0, uint32_t x1) {
-    uint32_t h = __builtin_amdgcn_sad_u8(x0, 0u, 0x64006400u);
-    h = __builtin_amdgcn_sad_hi_u8(x1, 0u, h);
-    f16x2 v = __builtin_bit_cast(f16x2, h);
-    const f16x2 c1 = __builtin_bit_cast(f16x2, 0x1eee1eeeu);
-    const f16x2 c2 = __builtin_bit_cast(f16x2, 0xc931c931u);
-    f16x2 o = __builtin_elementwise_fma(v, c1, c2);
-    return __builtin_bit_cast(uint32_t, o);
-}
-
-__device__ __forceinline__ uint32_t decode2_mul1(uint32_t s0, uint32_t s1) {
-    return mul1_finish2(mul1_x<0>(s0), mul1_x<0>(s1));
-}
+#include "exl3_trellis.h"
 
 // ---- whole-tensor reconstruct (bits at run time: load-time code) ---------------------------------------------------
 
@@ -227,163 +194,6 @@ extern "C" __global__ __launch_bounds__(128) void exl3_rot_in_group(RotGroup g, 
     rot_in_body(RotSrc{x, nullptr, x_mode, k}, g.suh[blockIdx.z], g.xh[blockIdx.z], k);
 }
 
-// ---- decode GEMV: the lane mapping and the decode ----------------------------------------------------------------------
-//
-// A program works on one 128-column block at a time; 256 threads = 4 wavefronts, wavefront w owning tiles 2w, 2w + 1 of
-// the block's 8. A wavefront's load step covers 4 consecutive k steps of its two tiles: lane L = 16 g + r reads k step g,
-// tile r >> 3, the BITS words of fragment lanes 4q .. 4q + 3 (q = r & 7) plus the word before them, which is all its 32
-// states need. Those states are rows n = q and n = q + 8 of the tile over all 16 k, so after decoding the lane holds, for
-// each of the two, the 16 values as two 8-value MFMA operands (k 0..7 and k 8..15) in k order. v_mfma_f32_16x16x32_f16
-// then sums over the 4 k steps: A = decoded weights (row r), B = 16 rotated input rows (column = input row), and the
-// accumulator of lane L holds output column 4 (L >> 4) + i of the 16 rows-of-A, input row L & 15.
-
-template <int BITS>
-struct LaneWords {
-    uint32_t w[BITS + 1];  // w[0] = the word before the lane's run
-};
-
-template <int BITS>
-__device__ __forceinline__ LaneWords<BITS> load_lane_words(const uint32_t* run, const uint32_t* prev) {
-    LaneWords<BITS> r;
-    r.w[0] = __builtin_nontemporal_load(prev);
-    if constexpr (BITS == 1) {
-        r.w[1] = __builtin_nontemporal_load(run);
-    } else if constexpr (BITS == 2) {
-        u32x2_a4 t = __builtin_nontemporal_load((const u32x2_a4*)run);
-        r.w[1] = t[0], r.w[2] = t[1];
-    } else if constexpr (BITS == 3) {
-        u32x3_a4 t = __builtin_nontemporal_load((const u32x3_a4*)run);
-        r.w[1] = t[0], r.w[2] = t[1], r.w[3] = t[2];
-    } else {
-        u32x4_a4 t = __builtin_nontemporal_load((const u32x4_a4*)run);
-        r.w[1] = t[0], r.w[2] = t[1], r.w[3] = t[2], r.w[4] = t[3];
-        if constexpr (BITS == 5) {
-            r.w[5] = __builtin_nontemporal_load(run + 4);
-        } else if constexpr (BITS == 6) {
-            u32x2_a4 u = __builtin_nontemporal_load((const u32x2_a4*)(run + 4));
-            r.w[5] = u[0], r.w[6] = u[1];
-        } else if constexpr (BITS == 7) {
-            u32x3_a4 u = __builtin_nontemporal_load((const u32x3_a4*)(run + 4));
-            r.w[5] = u[0], r.w[6] = u[1], r.w[7] = u[2];
-        } else if constexpr (BITS == 8) {
-            u32x4_a4 u = __builtin_nontemporal_load((const u32x4_a4*)(run + 4));
-            r.w[5] = u[0], r.w[6] = u[1], r.w[7] = u[2], r.w[8] = u[3];
-        }
-    }
-    return r;
-}
-
-// The lane's local stream: bit 0 = most significant bit of w[0]; local position U (0..31) owns the 16 bits ending at local
-// bit (U + 1) * BITS + 32. A state either lies inside one word (one extract), or straddles the boundary between w[i - 1]
-// and w[i]: all states that straddle one boundary are cut out of one 32-bit window over it (low half of w[i - 1], high
-// half of w[i]): BITS funnel shifts a load step instead of one per state or per pair of states.
-template <int BITS>
-struct LaneWindows {
-    uint32_t b[BITS + 1];  // b[i], i >= 1: the window over the boundary in front of w[i]
-};
-template <int BITS>
-__device__ __forceinline__ LaneWindows<BITS> lane_windows(const LaneWords<BITS>& lw) {
-    LaneWindows<BITS> win;
-    win.b[0] = 0;
-#pragma unroll
-    for (int i = 1; i <= BITS; i++) {
-        uint32_t r = __builtin_amdgcn_alignbit(lw.w[i - 1], lw.w[i], 16);
-        // opaque to the optimizer, which would otherwise fold window and extract into a funnel shift and a mask per state
-        asm("" : "+v"(r));
-        win.b[i] = r;
-    }
-    return win;
-}
-
-// x = state * MUL1 of local position U.
-template <int BITS, int U>
-__device__ __forceinline__ uint32_t lane_x(const LaneWords<BITS>& lw, const LaneWindows<BITS>& win) {
-    constexpr int end = (U + 1) * BITS + 32, wi = end / 32, r = end % 32;
-    uint32_t state;
-    if constexpr (r == 0)
-        state = lw.w[wi - 1] & 0xffffu;
-    else if constexpr (r == 16)
-        state = lw.w[wi] >> 16;
-    else if constexpr (r > 16)
-        state = __builtin_amdgcn_ubfe(lw.w[wi], 32 - r, 16);
-    else
-        state = __builtin_amdgcn_ubfe(win.b[wi], 16 - r, 16);
-    return state * 0x83DCD12Du;
-}
-
-// The lane's 32 values as MFMA operands op[h][kh]: rows n = q + 8 h of the tile, k = 8 kh .. 8 kh + 7 in order.
-// Local position u = 8 c + i (fragment lane 4q + c, value i) is k = 2c + (i & 1) + 8 ((i >> 1) & 1), n half i >> 2.
-template <int BITS>
-__device__ __forceinline__ void decode_lane(const LaneWords<BITS>& lw, f16x8 (&op)[2][2]) {
-    const LaneWindows<BITS> win = lane_windows<BITS>(lw);
-#define FE_PAIR(H, KH, C) mul1_finish2(lane_x<BITS, 8 * (C) + 2 * (KH) + 4 * (H)>(lw, win), lane_x<BITS, 8 * (C) + 2 * (KH) + 4 * (H) + 1>(lw, win))
-#define FE_OP(H, KH)                                                                             \
-    {                                                                                            \
-        u32x4 t = {FE_PAIR(H, KH, 0), FE_PAIR(H, KH, 1), FE_PAIR(H, KH, 2), FE_PAIR(H, KH, 3)};  \
-        op[H][KH] = __builtin_bit_cast(f16x8, t);                                                \
-    }
-    FE_OP(0, 0) FE_OP(0, 1) FE_OP(1, 0) FE_OP(1, 1)
-#undef FE_OP
-#undef FE_PAIR
-}
-
-// Row half H of the same: op[kh] = decode_lane's op[H][kh], with only the windows and extracts those 16 values need.
-template <int BITS>
-__device__ __forceinline__ void decode_lane_half(const LaneWords<BITS>& lw, int h, f16x8 (&op)[2]) {
-    const LaneWindows<BITS> win = lane_windows<BITS>(lw);
-#define FE_PAIR(H, KH, C) mul1_finish2(lane_x<BITS, 8 * (C) + 2 * (KH) + 4 * (H)>(lw, win), lane_x<BITS, 8 * (C) + 2 * (KH) + 4 * (H) + 1>(lw, win))
-#define FE_OP(H, KH)                                                                             \
-    {                                                                                            \
-        u32x4 t = {FE_PAIR(H, KH, 0), FE_PAIR(H, KH, 1), FE_PAIR(H, KH, 2), FE_PAIR(H, KH, 3)};  \
-        op[KH] = __builtin_bit_cast(f16x8, t);                                                   \
-    }
-    if (h == 0) {
-        FE_OP(0, 0) FE_OP(0, 1)
-    } else {
-        FE_OP(1, 0) FE_OP(1, 1)
-    }
-#undef FE_OP
-#undef FE_PAIR
-}
-
-// Store 4 consecutive outputs. mode: 0 bf16, 1 f32, 2 bf16 y += v (f32 add, one rounding), 3 f32 y += v.
-// (kernels/k-exl3/src/gemv.rs:122-145)
-__device__ __forceinline__ void store4(void* y, uint32_t mode, size_t i, float (&v)[4]) {
-    if (mode & 1) {
-        float* p = (float*)y + i;
-        f32x4 o = {v[0], v[1], v[2], v[3]};
-        if (mode & 2) o += *(const f32x4*)p;
-        *(f32x4*)p = o;
-    } else {
-        uint32_t* p = (uint32_t*)((uint16_t*)y + i);
-        if (mode & 2) {
-            uint32_t a = p[0], b = p[1];
-            v[0] += __uint_as_float(a << 16), v[1] += __uint_as_float(a & 0xffff0000u);
-            v[2] += __uint_as_float(b << 16), v[3] += __uint_as_float(b & 0xffff0000u);
-        }
-        u32x2 o = {pack_bf16x2(v[0], v[1]), pack_bf16x2(v[2], v[3])};
-        *(u32x2*)p = o;
-    }
-}
-
-// H over the 128 sums of a row (4 a lane of a half wavefront), * svh / sqrt(128), stored. (gemv.rs:172-180)
-__device__ __forceinline__ void finish_row(float (&v)[4], uint32_t l32, const uint16_t* svh, uint32_t col, void* y,
-                                           uint32_t mode, size_t at) {
-    fwht128_half_wave(v, l32);
-    u32x2 s = *(const u32x2*)(svh + col);
-    v[0] = v[0] * FE_HAD_SCALE * f16_bits_to_f32(s[0] & 0xffff);
-    v[1] = v[1] * FE_HAD_SCALE * f16_bits_to_f32(s[0] >> 16);
-    v[2] = v[2] * FE_HAD_SCALE * f16_bits_to_f32(s[1] & 0xffff);
-    v[3] = v[3] * FE_HAD_SCALE * f16_bits_to_f32(s[1] >> 16);
-    store4(y, mode, at, v);
-}
-
-// The lane's four output scales as finish_row applies them, for callers that finish many rows of the same columns.
-__device__ __forceinline__ f32x4 row_scales(const uint16_t* svh, uint32_t col) {
-    u32x2 s = *(const u32x2*)(svh + col);
-    return (f32x4){f16_bits_to_f32(s[0] & 0xffff), f16_bits_to_f32(s[0] >> 16), f16_bits_to_f32(s[1] & 0xffff),
-                   f16_bits_to_f32(s[1] >> 16)};
-}
 #ifndef FE_STAGE_NB1
 #define FE_STAGE_NB1 4
 #endif
@@ -440,15 +250,6 @@ __device__ __forceinline__ void ring_turn(LaneWords<BITS> (&ring)[DEPTH], uint32
         LaneWords<BITS> t = ring[3];
         ring[3] = ring[2], ring[2] = ring[1], ring[1] = ring[0], ring[0] = t;
     }
-}
-
-// The word before a lane's run is the last word of the run of lane q - 1 of the same tile (q = lane & 7; for q = 0 the
-// tile's last word, lane q = 7): a move across lanes instead of a second load per step. The 16 lanes of a DPP row are the
-// two tiles of one k step, so lane i takes lane i - 1 (row_shr:1) or, at q = 0, lane i + 7 (row_ror:9).
-__device__ __forceinline__ uint32_t lane_prev_word(uint32_t last) {
-    const uint32_t shr = (uint32_t)__builtin_amdgcn_update_dpp(0, (int)last, 0x111, 0xf, 0xf, false);
-    const uint32_t ror = (uint32_t)__builtin_amdgcn_update_dpp(0, (int)last, 0x129, 0xf, 0xf, false);
-    return (threadIdx.x & 7) ? shr : ror;
 }
 
 // A lane's words of one load step through a buffer resource over the whole trellis: the lane's byte offsets (run, word
@@ -1036,238 +837,6 @@ GEMVB_FAMILY(4)
 GEMVB_FAMILY(5)
 GEMVB_FAMILY(6)
 GEMVB_FAMILY(8)
-
-// ---- prefill GEMM ----------------------------------------------------------------------------------------------------
-
-typedef G8Tile<4, 2, 4, 8> Exl3Tile;  // 256 x 256; a wavefront's 128 columns are one Hadamard block
-
-// Weight operand of the prefill GEMM: a 64-wide k tile of a 128-column block is 4 k steps x 8 tiles; wavefront w takes block
-// w >> 2 of the 256-column output tile and k step w & 3, lane L tile L >> 3, rows n = (L & 7) and (L & 7) + 8 of it (the same
-// run of words as in the GEMV). A packed stage is [2 blocks][4 k steps][8 tiles][8 BITS words]: 2 BITS pieces of 1 KB.
-template <int BITS>
-struct Exl3Packed {
-    static constexpr int RAW_STAGE = 2048 * BITS, LOADS = (2 * BITS + 7) / 8;
-    typedef LaneWords<BITS> Words;
-    u32x4 rs;
-    uint32_t voff[LOADS], step;
-    __device__ __forceinline__ void setup(const uint32_t* trellis, uint32_t n, uint32_t k, uint32_t tn, uint32_t stride_k, uint32_t stride_nb) {
-        const uint32_t lane = threadIdx.x & 63, wave = threadIdx.x >> 6, nbs = n / 128;
-        rs = g8_rsrc(trellis, (k / 16) * (n / 16) * 32 * BITS);
-        step = 16 * stride_k;
-#pragma unroll
-        for (int j = 0; j < LOADS; j++) {
-            const uint32_t at = (wave + 8 * j) % (2 * BITS) * 1024 + lane * 16;  // (fewer pieces than wavefronts: some are moved twice)
-            const uint32_t ks = at / (256 * BITS) % 4;
-            uint32_t nb = 2 * tn + at / (1024 * BITS);
-            nb = nb < nbs ? nb : nbs - 1;  // an odd block count: the last tile decodes its first block twice
-            voff[j] = 4 * (nb * stride_nb + ks * stride_k) + at % (256 * BITS);
-        }
-    }
-    __device__ __forceinline__ void issue(uint32_t kt, uint32_t dst, int j, uint32_t wave) const {
-        g8_load_lds16(rs, dst + (wave + 8 * j) % (2 * BITS) * 1024, voff[j], kt * step);
-    }
-    __device__ __forceinline__ Words read(const unsigned char* st) const {
-        const uint32_t* p = (const uint32_t*)st + (threadIdx.x >> 3) * (8 * BITS) + (threadIdx.x & 7) * BITS;
-        Words w;
-        if constexpr (BITS % 4 == 0) {
-#pragma unroll
-            for (int i = 0; i < BITS; i += 4) {
-                const u32x4 t = *(const u32x4*)(p + i);
-                w.w[i + 1] = t[0], w.w[i + 2] = t[1], w.w[i + 3] = t[2], w.w[i + 4] = t[3];
-            }
-        } else {
-#pragma unroll
-            for (int i = 0; i < BITS; i++) w.w[i + 1] = p[i];
-        }
-        w.w[0] = 0;
-        return w;
-    }
-    // row half `half` (rows n = brow + 8 half of the lane's tile)
-    __device__ __forceinline__ void store(Words w, int half, unsigned char* ws) const {
-        const uint32_t lane = threadIdx.x & 63, wave = threadIdx.x >> 6, row = 128 * (wave >> 2) + (lane >> 3) * 16 + (lane & 7) + 8 * half;
-        f16x8 op[2];
-        w.w[0] = lane_prev_word(w.w[BITS]);
-        decode_lane_half<BITS>(w, half, op);
-#pragma unroll
-        for (int kh = 0; kh < 2; kh++) *(f16x8*)(ws + row * 128 + (((2 * (wave & 3) + kh) ^ (row & 7)) << 4)) = op[kh];
-    }
-};
-
-// y[m][n] (+)= H(xh @ W_hat) * svh / sqrt(128) for prefill-sized m: xh fp16 [m][k] (rotated inputs), 256 x 256 output
-// tiles; a wavefront's 128 columns are exactly one Hadamard block, so the output rotation is local to the wavefront.
-// Tiles = ceil(m / 256) * ceil(n / 256) (grouped raster), spread over the grid as sc says (g8_schedule): one piece a
-// program, the cut tiles finished by exl3_gemm_reduce, or stream-K. 512 threads, dynamic LDS 160 KB (the epilogue
-// reuses it). loop(tm, tn, kt0, ktn, lds, acc) is a pass of the main loop.
-template <bool SK, class Loop>
-__device__ __forceinline__ void exl3_gemm_tile(const uint16_t* __restrict__ svh, void* y, uint32_t n, uint32_t k, uint32_t m,
-                                               uint32_t y_mode, uint32_t group_m, const GemmSched& sched, Loop loop) {
-    typedef Exl3Tile T;
-    extern __shared__ __attribute__((aligned(1024))) unsigned char lds[];
-    const uint32_t nbs = n / 128;
-    const uint32_t lane = threadIdx.x & 63, wave = threadIdx.x >> 6, wm = wave / T::WN, wn = wave % T::WN;
-    g8_schedule<T, SK>(
-        sched, (m + T::BM - 1) / T::BM, (nbs + 1) / 2, group_m, k / G8_BK, lds,
-        [&](uint32_t tm, uint32_t tn, uint32_t kt0, uint32_t ktn, f32x4(&acc)[T::TM][T::TN]) { loop(tm, tn, kt0, ktn, lds, acc); },
-        [&](uint32_t tm, uint32_t tn, f32x4(&acc)[T::TM][T::TN]) {
-            const uint32_t m0 = tm * T::BM + wm * 16 * T::TM, nb = 2 * tn + wn;
-            if (nb >= nbs) return;
-            const uint32_t col = nb * 128 + 4 * (lane & 31);
-            const f32x4 sc = row_scales(svh, col);
-            // one copy of the epilogue per output mode, so that the row loop has no mode branches
-            auto run = [&](auto mode_tag) {
-                constexpr uint32_t MODE = decltype(mode_tag)::value;
-                g8_epilogue<T>(
-                    acc, lds,
-                    [&](float (&v)[4][4], uint32_t l32) {
-                        fwht128_half_wave_rows(v, l32);
-#pragma unroll
-                        for (int u = 0; u < 4; u++)
-#pragma unroll
-                            for (int e = 0; e < 4; e++) v[u][e] = v[u][e] * FE_HAD_SCALE * sc[e];  // finish_row's products
-                    },
-                    [&](uint32_t row, uint32_t, float (&v)[4]) {
-                        if (m0 + row < m) store4(y, MODE, (size_t)(m0 + row) * n + col, v);
-                    });
-            };
-            if (y_mode == 0)
-                run(std::integral_constant<uint32_t, 0>{});
-            else if (y_mode == 1)
-                run(std::integral_constant<uint32_t, 1>{});
-            else if (y_mode == 2)
-                run(std::integral_constant<uint32_t, 2>{});
-            else
-                run(std::integral_constant<uint32_t, 3>{});
-        });
-}
-
-// The GEMM decoding the trellis itself: every 256-row tile of the output decodes its weights again.
-template <int BITS, bool SK>
-__device__ __forceinline__ void exl3_gemm_body(const _Float16* __restrict__ xh, const uint32_t* __restrict__ trellis,
-                                               const uint16_t* __restrict__ svh, void* y, uint32_t n, uint32_t k, uint32_t m,
-                                               uint32_t y_mode, uint32_t stride_k, uint32_t stride_nb, uint32_t group_m,
-                                               const GemmSched& sched) {
-    exl3_gemm_tile<SK>(svh, y, n, k, m, y_mode, group_m, sched,
-                       [&](uint32_t tm, uint32_t tn, uint32_t kt0, uint32_t ktn, unsigned char* lds, f32x4(&acc)[Exl3Tile::TM][Exl3Tile::TN]) {
-                           Exl3Packed<BITS> w;
-                           w.setup(trellis, n, k, tn, stride_k, stride_nb);
-                           g8_mainloop_decode<Exl3Tile, BITS <= 5 ? 3 : 2>(xh, k, m, kt0, ktn, tm * Exl3Tile::BM, w, lds, acc);
-                       });
-}
-
-// ---- prefill over decoded weights -----------------------------------------------------------------------------------
-//
-// For many rows the trellis is decoded once per call into `hat`, fp16, as the very images the GEMM keeps in LDS: block
-// (tn, kt) of 32 KB = rows n = 256 tn .. + 255 of k tile kt, 128 bytes a row, 16-byte chunk c of row r at the position gm_swz
-// gives it. The GEMM over it then copies blocks instead of decoding, with the same fragments, the same MFMA order and
-// so the same bits as exl3_gemm_b*.
-
-// grid (n / 128, gy), 256 threads; program (nb, j) decodes k tiles j, j + gy, ... of column block nb with the lane
-// mapping of Exl3Producer. The 16 KB of a k tile pass through LDS (two buffers, one barrier a tile) so that they leave
-// as whole 1 KB runs per wavefront instead of scattered 16-byte pieces.
-template <int BITS>
-__device__ __forceinline__ void exl3_hat_tiles_body(const uint32_t* __restrict__ trellis, unsigned char* __restrict__ hat,
-                                                    uint32_t k, uint32_t stride_k, uint32_t stride_nb) {
-    __shared__ __attribute__((aligned(16))) unsigned char img[2][GM_B_BYTES / 2];
-    constexpr uint32_t tw = 8 * BITS;
-    const uint32_t lane = threadIdx.x & 63, ks = threadIdx.x >> 6, tj = lane >> 3, q = lane & 7;
-    const uint32_t nb = blockIdx.x, ktiles = k / GM_BK;
-    const uint32_t* base = trellis + (size_t)nb * stride_nb + tj * tw;
-    const uint32_t run_off = q * BITS, prev_off = (q * BITS + tw - 1) % tw;
-    const uint32_t row = tj * 16 + q;
-    unsigned char* out = hat + (size_t)(nb >> 1) * ktiles * GM_B_BYTES + (nb & 1) * (GM_B_BYTES / 2) + 16 * threadIdx.x;
-    uint32_t kt = blockIdx.y;
-    if (kt >= ktiles) return;
-    const uint32_t* p = base + (size_t)(kt * 4 + ks) * stride_k;
-    LaneWords<BITS> cur = load_lane_words<BITS>(p + run_off, p + prev_off);
-    for (uint32_t it = 0; kt < ktiles; kt += gridDim.y, it++) {
-        uint32_t nk = kt + gridDim.y < ktiles ? kt + gridDim.y : kt;
-        const uint32_t* pn = base + (size_t)(nk * 4 + ks) * stride_k;
-        LaneWords<BITS> nxt = load_lane_words<BITS>(pn + run_off, pn + prev_off);
-        f16x8 op[2][2];
-        decode_lane<BITS>(cur, op);
-        unsigned char* buf = img[it & 1];
-#pragma unroll
-        for (int h = 0; h < 2; h++)
-#pragma unroll
-            for (int kh = 0; kh < 2; kh++) *(f16x8*)(buf + gm_swz(row + 8 * h, 2 * ks + kh)) = op[h][kh];
-        __syncthreads();
-        unsigned char* blk = out + (size_t)kt * GM_B_BYTES;
-#pragma unroll
-        for (int j = 0; j < 4; j++) *(u32x4*)(blk + 4096 * j) = *(const u32x4*)(buf + 16 * threadIdx.x + 4096 * j);
-        cur = nxt;
-    }
-}
-
-// (every GEMM kernel comes as NAME, one piece a program, and NAME_sk, stream-K, with the same parameters)
-#define HAT_GEMM_PARAMS                                                                                                  \
-    const _Float16 *xh, const unsigned char *hat, const uint16_t *svh, void *y, uint32_t n, uint32_t k, uint32_t m, uint32_t y_mode, \
-        uint32_t group_m, GemmSched sched
-template <bool SK>
-__device__ __forceinline__ void exl3_gemm_hat_kernel(HAT_GEMM_PARAMS) {
-    typedef Exl3Tile T;
-    exl3_gemm_tile<SK>(svh, y, n, k, m, y_mode, group_m, sched,
-                       [&](uint32_t tm, uint32_t tn, uint32_t kt0, uint32_t ktn, unsigned char* lds, f32x4(&acc)[T::TM][T::TN]) {
-                           // the tile's blocks of 32 KB; a row's chunks lie where gm_swz puts them: the core's position, its low
-                           // bit flipped in every second group of 8 rows
-                           const uint32_t lane = threadIdx.x & 63, wave = threadIdx.x >> 6, bytes = (k / G8_BK) * GM_B_BYTES;
-                           G8Dense<T> w;
-                           w.rs = g8_rsrc(hat + (size_t)tn * bytes, bytes), w.kstep = GM_B_BYTES;
-#pragma unroll
-                           for (int j = 0; j < G8Dense<T>::LOADS; j++) {
-                               const uint32_t r = 8 * (wave + 8 * j) + (lane >> 3);
-                               w.voff[j] = r * 128 + (((lane & 7) ^ ((r >> 3) & 1)) << 4);
-                           }
-                           g8_mainloop<T, 2, 3, false>(xh, k, m, kt0, ktn, tm * T::BM, w, lds, acc);
-                       });
-}
-extern "C" __global__ __launch_bounds__(512, 2) void exl3_gemm_hat(HAT_GEMM_PARAMS) {
-    exl3_gemm_hat_kernel<false>(xh, hat, svh, y, n, k, m, y_mode, group_m, sched);
-}
-extern "C" __global__ __launch_bounds__(512, 2) void exl3_gemm_hat_sk(HAT_GEMM_PARAMS) {
-    exl3_gemm_hat_kernel<true>(xh, hat, svh, y, n, k, m, y_mode, group_m, sched);
-}
-
-// Finishes the tiles that exl3_gemm_b* cut along K: sums their partial slots and applies the output rotation and scale.
-// grid (tiles - full_tiles) * 64, 256 threads.
-extern "C" __global__ __launch_bounds__(256) void exl3_gemm_reduce(const float* part, const uint16_t* svh, void* y, uint32_t n,
-                                                                   uint32_t m, uint32_t y_mode, uint32_t group_m,
-                                                                   uint32_t full_tiles, uint32_t splits) {
-    typedef Exl3Tile T;
-    const uint32_t nbs = n / 128;
-    g8_reduce_rows<T>(part, splits, [&](uint32_t t, uint32_t row, uint32_t cb, uint32_t l32, float (&v)[4]) {
-        uint32_t tm, tn;
-        gemm_raster(full_tiles + t, (m + T::BM - 1) / T::BM, (nbs + 1) / 2, group_m, tm, tn);
-        uint32_t grow = tm * T::BM + row, nb = 2 * tn + cb;
-        if (grow < m && nb < nbs) finish_row(v, l32, svh, nb * 128 + 4 * l32, y, y_mode, (size_t)grow * n + nb * 128 + 4 * l32);
-    });
-}
-
-#define GEMM_KERNEL_(NAME, BITS, SK)                                                                                   \
-    extern "C" __global__ __launch_bounds__(512, 2) void NAME(                                                         \
-        const _Float16* xh, const uint32_t* trellis, const uint16_t* svh, void* y, uint32_t n, uint32_t k, uint32_t m,  \
-        uint32_t y_mode, uint32_t stride_k, uint32_t stride_nb, uint32_t group_m, GemmSched sched) {                    \
-        exl3_gemm_body<BITS, SK>(xh, trellis, svh, y, n, k, m, y_mode, stride_k, stride_nb, group_m, sched);           \
-    }
-#define GEMM_KERNEL(BITS)                       \
-    GEMM_KERNEL_(exl3_gemm_b##BITS, BITS, false) \
-    GEMM_KERNEL_(exl3_gemm_b##BITS##_sk, BITS, true)
-#define HAT_KERNEL(BITS)                                                                                      \
-    extern "C" __global__ __launch_bounds__(256) void exl3_hat_tiles_b##BITS(                                 \
-        const uint32_t* trellis, unsigned char* hat, uint32_t k, uint32_t stride_k, uint32_t stride_nb) {     \
-        exl3_hat_tiles_body<BITS>(trellis, hat, k, stride_k, stride_nb);                                      \
-    }
-HAT_KERNEL(2)
-HAT_KERNEL(3)
-HAT_KERNEL(4)
-HAT_KERNEL(5)
-HAT_KERNEL(6)
-HAT_KERNEL(8)
-GEMM_KERNEL(2)
-GEMM_KERNEL(3)
-GEMM_KERNEL(4)
-GEMM_KERNEL(5)
-GEMM_KERNEL(6)
-GEMM_KERNEL(8)
 
 // ---- probes ----------------------------------------------------------------------------------------------------------
 

@@ -411,50 +411,54 @@ __device__ __forceinline__ void fp_store_piece(const FpOut& o, const float (&v)[
     }
 }
 
-typedef G8Tile<4, 2, 4, 8> Fp8Tile;  // the GEMM over FP8 codes: 256 x 256
-typedef G8Tile<2, 4, 8, 4> FpTile;  // 256 x 256; a wavefront's 128 x 64 keeps the codes it expands to a quarter of the tile's
+// Tiles of 256 x 256, 128 x 256 (S1) and 128 x 128 (S2). Packed weights: a wavefront's columns are a quarter of the tile's, so
+// that a weight is expanded by two wavefronts only. The GEMM over FP8 codes expands nothing.
+typedef G8Tile<2, 4, 8, 4> FpTile;
+typedef G8Tile<2, 4, 4, 4> FpTileS1;
+typedef G8Tile<2, 4, 4, 2> FpTileS2;
+typedef G8Tile<4, 2, 4, 8> Fp8Tile;
+typedef G8Tile<4, 2, 2, 8> Fp8TileS1;
+typedef G8Tile<4, 2, 2, 4> Fp8TileS2;
+// wavefronts a SIMD: two programs of the smallest tile fit a CU; k tiles of A and of packed weights in LDS
+template <class T>
+struct FpWaves {
+    static constexpr int MIN = T::PARTS == 4 ? 4 : 2, NA = T::PARTS == 2 ? 5 : 3, NW = T::PARTS == 2 ? 6 : T::PARTS == 4 ? 4 : 3;
+};
 
 // C[M][ldc] = bf16((A_q . W_q^T) * alpha[n]) (+ res: bf16(bf16(.) + res)); A_q = the fp16 operand of the quantizer,
-// W_q expanded by the packed operand make_packed(tn) of 256-column tile tn; `scale` = 1 / (the factors the two fp16 operands
-// carry). Tiles = ceil(M / 256) * ceil(N / 256) (grouped raster), spread over the grid as sc says (g8_schedule): one
-// piece a program, the cut tiles finished by the reduce kernel, or stream-K. 512 threads, dynamic LDS 160 KB.
+// W_q expanded by the packed operand make_packed(n0) of the tile at column n0; `scale` = 1 / (the factors the two fp16 operands
+// carry). Tiles (grouped raster) spread over the grid as sc says (g8_schedule). 512 threads, dynamic LDS as the stages take.
 // N % 128 == 0, K % 128 == 0. (kernels/k-fp4/src/lib.rs:285-470)
-template <bool SWIGLU, bool SK, class MakePacked>
+template <class T, bool SWIGLU, bool SK, class MakePacked>
 __device__ __forceinline__ void fp_gemm_body(MakePacked make_packed, const FpOut& out, const _Float16* aq, const float* alpha,
                                              float scale, uint32_t m, uint32_t n, uint32_t k, uint32_t group_m,
                                              const GemmSched& sc) {
-    typedef FpTile T;
     extern __shared__ __attribute__((aligned(1024))) unsigned char lds[];
     const uint32_t lane = threadIdx.x & 63, wave = threadIdx.x >> 6, wm = wave / T::WN, wn = wave % T::WN;
     g8_schedule<T, SK>(
-        sc, (m + T::BM - 1) / T::BM, (n / 128 + 1) / 2, group_m, k / G8_BK, lds,
-        [&](uint32_t tm, uint32_t tn, uint32_t kt0, uint32_t ktn, f32x4(&acc)[T::TM][T::TN]) {
-            auto w = make_packed(tn);
-            g8_mainloop_packed<T, 3, 3>(aq, k, m, kt0, ktn, tm * T::BM, w, lds, acc);
+        sc, m, n, group_m, k / G8_BK, lds,
+        [&](uint32_t m0, uint32_t n0, uint32_t kt0, uint32_t ktn, f32x4(&acc)[T::TM][T::TN]) {
+            auto w = make_packed(n0);
+            g8_mainloop_packed<T, FpWaves<T>::NA, FpWaves<T>::NW>(aq, k, m, kt0, ktn, m0, w, lds, acc);
         },
-        [&](uint32_t tm, uint32_t tn, f32x4(&acc)[T::TM][T::TN]) {
-            const uint32_t m0 = tm * T::BM + wm * 16 * T::TM, colb = tn * T::BN + wn * 16 * T::TN;
+        [&](uint32_t m0, uint32_t n0, f32x4(&acc)[T::TM][T::TN]) {
+            const uint32_t row0 = m0 + wm * 16 * T::TM, colb = n0 + wn * 16 * T::TN;
             if (colb >= n) return;
             const uint32_t col = colb + 4 * (lane % (4 * T::TN));
             const f32x4 al = *(const f32x4*)(alpha + col) * scale;
             g8_epilogue<T>(
                 acc, lds, [](auto&, uint32_t) {},
-                [&](uint32_t row, uint32_t lc, float (&v)[4]) { fp_store_piece<SWIGLU>(out, v, al, lc, m0 + row, m, col, n); });
+                [&](uint32_t row, uint32_t lc, float (&v)[4]) { fp_store_piece<SWIGLU>(out, v, al, lc, row0 + row, m, col, n); });
         });
 }
 
-// Finishes the tiles that a GEMM kernel cut along K. grid (tiles - full_tiles) * 64, 256 threads.
+// Finishes the tiles that a GEMM kernel cut along K. grid: cut tiles * (BM / 8) * (BN / 128), 256 threads.
 template <class T, bool SWIGLU>
 __device__ __forceinline__ void fp_reduce_body(const FpOut& out, const float* part, const float* alpha, float scale,
-                                               uint32_t m, uint32_t n, uint32_t group_m, uint32_t full_tiles,
-                                               uint32_t splits) {
-    const uint32_t nts = n / 128;
-    g8_reduce_rows<T>(part, splits, [&](uint32_t t, uint32_t row, uint32_t cb, uint32_t l32, float (&v)[4]) {
-        uint32_t tm, tn;
-        gemm_raster(full_tiles + t, (m + T::BM - 1) / T::BM, (nts + 1) / 2, group_m, tm, tn);
-        uint32_t grow = tm * T::BM + row, col = tn * T::BN + cb * 128 + 4 * l32;
-        if (tn * T::BN + cb * 128 >= n) return;  // the absent half of an odd last tile (uniform over the half wavefront)
-        fp_store_piece<SWIGLU>(out, v, *(const f32x4*)(alpha + col) * scale, l32, grow, m, col, n);
+                                               uint32_t m, uint32_t n, uint32_t group_m, uint32_t first, uint32_t splits) {
+    g8_reduce_rows<T>(part, m, n, group_m, first, splits, [&](uint32_t row, uint32_t n0, uint32_t l32, float (&v)[4]) {
+        const uint32_t col = n0 + 4 * l32;
+        fp_store_piece<SWIGLU>(out, v, *(const f32x4*)(alpha + col) * scale, l32, row, m, col, n);
     });
 }
 
@@ -465,31 +469,39 @@ __device__ __forceinline__ void fp_reduce_body(const FpOut& out, const float* pa
     uint16_t *c, const _Float16 *aq, const uint8_t *w, const uint8_t *sw, const float *alpha, const uint16_t *res, uint32_t m, \
         uint32_t n, uint32_t k, uint32_t ldc, uint32_t group_m, uint32_t w_snt, uint32_t w_skt, uint32_t w_sr, uint32_t s_snt, \
         uint32_t s_skt, uint32_t s_sr, GemmSched sc
-template <bool SK>
+template <class T, bool SK>
 __device__ __forceinline__ void gemm_nvfp4_kernel(FP4_GEMM_PARAMS) {
     FpOut out = {c, res, ldc, nullptr, nullptr, nullptr, 0.f};
-    fp_gemm_body<false, SK>(
-        [&](uint32_t tn) {
-            Fp4Packed<FpTile> p;
-            p.setup(w, sw, n, k, tn * FpTile::BN, w_snt, w_skt, w_sr, s_snt, s_skt, s_sr);
+    fp_gemm_body<T, false, SK>(
+        [&](uint32_t n0) {
+            Fp4Packed<T> p;
+            p.setup(w, sw, n, k, n0, w_snt, w_skt, w_sr, s_snt, s_skt, s_sr);
             return p;
         },
         out, aq, alpha, FP4_GEMM_SCALE, m, n, k, group_m, sc);
 }
-extern "C" __global__ __launch_bounds__(512, 2) void fe_gemm_nvfp4(FP4_GEMM_PARAMS) {
-    gemm_nvfp4_kernel<false>(c, aq, w, sw, alpha, res, m, n, k, ldc, group_m, w_snt, w_skt, w_sr, s_snt, s_skt, s_sr, sc);
-}
-extern "C" __global__ __launch_bounds__(512, 2) void fe_gemm_nvfp4_sk(FP4_GEMM_PARAMS) {
-    gemm_nvfp4_kernel<true>(c, aq, w, sw, alpha, res, m, n, k, ldc, group_m, w_snt, w_skt, w_sr, s_snt, s_skt, s_sr, sc);
-}
+#define FP4_GEMM_KERNEL(SUFFIX, TILE, SK)                                                                                  \
+    extern "C" __global__ __launch_bounds__(512, FpWaves<TILE>::MIN) void fe_gemm_nvfp4##SUFFIX(FP4_GEMM_PARAMS) {         \
+        gemm_nvfp4_kernel<TILE, SK>(c, aq, w, sw, alpha, res, m, n, k, ldc, group_m, w_snt, w_skt, w_sr, s_snt, s_skt, s_sr, sc); \
+    }
+FP4_GEMM_KERNEL(, FpTile, false)
+FP4_GEMM_KERNEL(_sk, FpTile, true)
+FP4_GEMM_KERNEL(_s1, FpTileS1, false)
+FP4_GEMM_KERNEL(_s2, FpTileS2, false)
 
-extern "C" __global__ __launch_bounds__(256) void fe_gemm_nvfp4_reduce(uint16_t* c, const float* part, const float* alpha,
-                                                                       const uint16_t* res, uint32_t m, uint32_t n,
-                                                                       uint32_t ldc, uint32_t group_m, uint32_t full_tiles,
-                                                                       uint32_t splits, float scale) {
-    FpOut out = {c, res, ldc, nullptr, nullptr, nullptr, 0.f};
-    fp_reduce_body<FpTile, false>(out, part, alpha, scale, m, n, group_m, full_tiles, splits);
-}
+#define FP_REDUCE_KERNEL(NAME, TILE)                                                                                       \
+    extern "C" __global__ __launch_bounds__(256) void NAME(uint16_t* c, const float* part, const float* alpha,             \
+                                                           const uint16_t* res, uint32_t m, uint32_t n, uint32_t ldc,      \
+                                                           uint32_t group_m, uint32_t first, uint32_t splits, float scale) { \
+        FpOut out = {c, res, ldc, nullptr, nullptr, nullptr, 0.f};                                                         \
+        fp_reduce_body<TILE, false>(out, part, alpha, scale, m, n, group_m, first, splits);                                \
+    }
+FP_REDUCE_KERNEL(fe_gemm_nvfp4_reduce, FpTile)
+FP_REDUCE_KERNEL(fe_gemm_nvfp4_reduce_s1, FpTileS1)
+FP_REDUCE_KERNEL(fe_gemm_nvfp4_reduce_s2, FpTileS2)
+FP_REDUCE_KERNEL(fe_gemm_fp8_codes_reduce, Fp8Tile)
+FP_REDUCE_KERNEL(fe_gemm_fp8_codes_reduce_s1, Fp8TileS1)
+FP_REDUCE_KERNEL(fe_gemm_fp8_codes_reduce_s2, Fp8TileS2)
 
 // Fused MLP front: act = SwiGLU(x . [gate|up]^T), NVFP4-quantized with global scale qg (1 / input_scale of the down
 // projection) into q_codes [M][inter/2], q_sf (tiled, kb = inter/16) and the fp16 operand q_aq [M][inter]; w, sw, alpha =
@@ -498,42 +510,36 @@ extern "C" __global__ __launch_bounds__(256) void fe_gemm_nvfp4_reduce(uint16_t*
     const _Float16 *aq, const uint8_t *w, const uint8_t *sw, const float *alpha, uint32_t m, uint32_t n, uint32_t k,           \
         uint32_t group_m, uint32_t w_snt, uint32_t w_skt, uint32_t w_sr, uint32_t s_snt, uint32_t s_skt, uint32_t s_sr,        \
         GemmSched sc, uint8_t *q_codes, uint8_t *q_sf, _Float16 *q_aq, float qg
-template <bool SK>
+template <class T, bool SK>
 __device__ __forceinline__ void gemm_nvfp4_swiglu_kernel(FP4_SWIGLU_PARAMS) {
     FpOut out = {nullptr, nullptr, 0, q_codes, q_sf, q_aq, qg};
-    fp_gemm_body<true, SK>(
-        [&](uint32_t tn) {
-            Fp4Packed<FpTile> p;
-            p.setup(w, sw, n, k, tn * FpTile::BN, w_snt, w_skt, w_sr, s_snt, s_skt, s_sr);
+    fp_gemm_body<T, true, SK>(
+        [&](uint32_t n0) {
+            Fp4Packed<T> p;
+            p.setup(w, sw, n, k, n0, w_snt, w_skt, w_sr, s_snt, s_skt, s_sr);
             return p;
         },
         out, aq, alpha, FP4_GEMM_SCALE, m, n, k, group_m, sc);
 }
-extern "C" __global__ __launch_bounds__(512, 2) void fe_gemm_nvfp4_swiglu(FP4_SWIGLU_PARAMS) {
-    gemm_nvfp4_swiglu_kernel<false>(aq, w, sw, alpha, m, n, k, group_m, w_snt, w_skt, w_sr, s_snt, s_skt, s_sr, sc, q_codes, q_sf,
-                                    q_aq, qg);
-}
-extern "C" __global__ __launch_bounds__(512, 2) void fe_gemm_nvfp4_swiglu_sk(FP4_SWIGLU_PARAMS) {
-    gemm_nvfp4_swiglu_kernel<true>(aq, w, sw, alpha, m, n, k, group_m, w_snt, w_skt, w_sr, s_snt, s_skt, s_sr, sc, q_codes, q_sf,
-                                   q_aq, qg);
-}
-
-extern "C" __global__ __launch_bounds__(256) void fe_gemm_nvfp4_swiglu_reduce(const float* part, const float* alpha, uint32_t m,
-                                                                              uint32_t n, uint32_t group_m, uint32_t full_tiles,
-                                                                              uint32_t splits, uint8_t* q_codes, uint8_t* q_sf,
-                                                                              _Float16* q_aq, float qg) {
-    FpOut out = {nullptr, nullptr, 0, q_codes, q_sf, q_aq, qg};
-    fp_reduce_body<FpTile, true>(out, part, alpha, FP4_GEMM_SCALE, m, n, group_m, full_tiles, splits);
-}
-
-// The same for the GEMM over FP8 codes.
-extern "C" __global__ __launch_bounds__(256) void fe_gemm_fp8_codes_reduce(uint16_t* c, const float* part, const float* alpha,
-                                                                           const uint16_t* res, uint32_t m, uint32_t n,
-                                                                           uint32_t ldc, uint32_t group_m, uint32_t full_tiles,
-                                                                           uint32_t splits, float scale) {
-    FpOut out = {c, res, ldc, nullptr, nullptr, nullptr, 0.f};
-    fp_reduce_body<Fp8Tile, false>(out, part, alpha, scale, m, n, group_m, full_tiles, splits);
-}
+#define FP4_SWIGLU_KERNEL(SUFFIX, TILE, SK)                                                                                \
+    extern "C" __global__ __launch_bounds__(512, FpWaves<TILE>::MIN) void fe_gemm_nvfp4_swiglu##SUFFIX(FP4_SWIGLU_PARAMS) { \
+        gemm_nvfp4_swiglu_kernel<TILE, SK>(aq, w, sw, alpha, m, n, k, group_m, w_snt, w_skt, w_sr, s_snt, s_skt, s_sr, sc, q_codes, \
+                                           q_sf, q_aq, qg);                                                                \
+    }
+FP4_SWIGLU_KERNEL(, FpTile, false)
+FP4_SWIGLU_KERNEL(_sk, FpTile, true)
+FP4_SWIGLU_KERNEL(_s1, FpTileS1, false)
+FP4_SWIGLU_KERNEL(_s2, FpTileS2, false)
+#define FP4_SWIGLU_REDUCE_KERNEL(SUFFIX, TILE)                                                                             \
+    extern "C" __global__ __launch_bounds__(256) void fe_gemm_nvfp4_swiglu_reduce##SUFFIX(                                 \
+        const float* part, const float* alpha, uint32_t m, uint32_t n, uint32_t group_m, uint32_t first, uint32_t splits,  \
+        uint8_t* q_codes, uint8_t* q_sf, _Float16* q_aq, float qg) {                                                       \
+        FpOut out = {nullptr, nullptr, 0, q_codes, q_sf, q_aq, qg};                                                        \
+        fp_reduce_body<TILE, true>(out, part, alpha, FP4_GEMM_SCALE, m, n, group_m, first, splits);                        \
+    }
+FP4_SWIGLU_REDUCE_KERNEL(, FpTile)
+FP4_SWIGLU_REDUCE_KERNEL(_s1, FpTileS1)
+FP4_SWIGLU_REDUCE_KERNEL(_s2, FpTileS2)
 
 // FP8: the 64 codes of row r = 128 nt + i, k tile kt are at w + nt * w_snt + kt * w_skt + i * w_sr; both fp16 expansions
 // are the values themselves. Finished by fe_gemm_nvfp4_reduce with scale 1. (kernels/k-fp4/src/lib.rs:472-484)
@@ -543,10 +549,10 @@ extern "C" __global__ __launch_bounds__(256) void fe_gemm_fp8_codes_reduce(uint1
 template <bool SK>
 __device__ __forceinline__ void gemm_fp8_kernel(FP8_GEMM_PARAMS) {
     FpOut out = {c, res, ldc, nullptr, nullptr, nullptr, 0.f};
-    fp_gemm_body<false, SK>(
-        [&](uint32_t tn) {
+    fp_gemm_body<FpTile, false, SK>(
+        [&](uint32_t n0) {
             Fp8Packed<FpTile> p;
-            p.setup(w, n, k, tn * FpTile::BN, w_snt, w_skt, w_sr);
+            p.setup(w, n, k, n0, w_snt, w_skt, w_sr);
             return p;
         },
         out, aq, alpha, 1.0f, m, n, k, group_m, sc);
@@ -564,43 +570,45 @@ extern "C" __global__ __launch_bounds__(512, 2) void fe_gemm_fp8_sk(FP8_GEMM_PAR
 #define FP8C_GEMM_PARAMS                                                                                                   \
     uint16_t *c, const uint8_t *aq, const uint8_t *w, const float *alpha, const uint16_t *res, uint32_t m, uint32_t n, uint32_t k, \
         uint32_t ldc, uint32_t group_m, uint32_t w_snt, uint32_t w_skt, uint32_t w_sr, GemmSched sc
-template <bool SK>
+template <class T, bool SK>
 __device__ __forceinline__ void gemm_fp8_codes_kernel(FP8C_GEMM_PARAMS) {
-    typedef Fp8Tile T;
+    constexpr int NA = T::PARTS == 2 ? 3 : 2;
     extern __shared__ __attribute__((aligned(1024))) unsigned char lds[];
     const uint32_t nts = n / 128, lane = threadIdx.x & 63, wave = threadIdx.x >> 6, wm = wave / T::WN, wn = wave % T::WN;
     FpOut out = {c, res, ldc, nullptr, nullptr, nullptr, 0.f};
     g8_schedule<T, SK>(
-        sc, (m + T::BM - 1) / T::BM, (nts + 1) / 2, group_m, k / 128, lds,
-        [&](uint32_t tm, uint32_t tn, uint32_t kt0, uint32_t ktn, f32x4(&acc)[T::TM][T::TN]) {
+        sc, m, n, group_m, k / 128, lds,
+        [&](uint32_t m0, uint32_t n0, uint32_t kt0, uint32_t ktn, f32x4(&acc)[T::TM][T::TN]) {
             // a k tile of 128 codes is two of the layout's 64-wide ones: chunks 0..3 of a row from the first, 4..7 from the second
             G8Dense<T> wo;
             wo.rs = g8_rsrc(w, n * k), wo.kstep = 2 * w_skt;
 #pragma unroll
             for (int j = 0; j < G8Dense<T>::LOADS; j++) {
                 const uint32_t r = 8 * (wave + 8 * j) + (lane >> 3), ch = (lane & 7) ^ (r & 7);
-                uint32_t nt = 2 * tn + r / 128;
+                uint32_t nt = (n0 + r) / 128;
                 nt = nt < nts ? nt : nts - 1;  // an odd count of 128-row tiles: the last program reads its first tile twice
                 wo.voff[j] = nt * w_snt + (ch >> 2) * w_skt + (r & 127) * w_sr + (ch & 3) * 16;
             }
-            g8_mainloop_f8<T, 2, 3>(aq, k, m, kt0, ktn, tm * T::BM, wo, lds, acc);
+            g8_mainloop_f8<T, NA, 3>(aq, k, m, kt0, ktn, m0, wo, lds, acc);
         },
-        [&](uint32_t tm, uint32_t tn, f32x4(&acc)[T::TM][T::TN]) {
-            const uint32_t m0 = tm * T::BM + wm * 16 * T::TM, colb = tn * T::BN + wn * 16 * T::TN;
+        [&](uint32_t m0, uint32_t n0, f32x4(&acc)[T::TM][T::TN]) {
+            const uint32_t row0 = m0 + wm * 16 * T::TM, colb = n0 + wn * 16 * T::TN;
             if (colb >= n) return;
             const uint32_t col = colb + 4 * (lane % (4 * T::TN));
             const f32x4 al = *(const f32x4*)(alpha + col);
             g8_epilogue<T>(
                 acc, lds, [](auto&, uint32_t) {},
-                [&](uint32_t r, uint32_t lc, float (&v)[4]) { fp_store_piece<false>(out, v, al, lc, m0 + r, m, col, n); });
+                [&](uint32_t r, uint32_t lc, float (&v)[4]) { fp_store_piece<false>(out, v, al, lc, row0 + r, m, col, n); });
         });
 }
-extern "C" __global__ __launch_bounds__(512, 2) void fe_gemm_fp8_codes(FP8C_GEMM_PARAMS) {
-    gemm_fp8_codes_kernel<false>(c, aq, w, alpha, res, m, n, k, ldc, group_m, w_snt, w_skt, w_sr, sc);
-}
-extern "C" __global__ __launch_bounds__(512, 2) void fe_gemm_fp8_codes_sk(FP8C_GEMM_PARAMS) {
-    gemm_fp8_codes_kernel<true>(c, aq, w, alpha, res, m, n, k, ldc, group_m, w_snt, w_skt, w_sr, sc);
-}
+#define FP8C_GEMM_KERNEL(SUFFIX, TILE, SK)                                                                                 \
+    extern "C" __global__ __launch_bounds__(512, FpWaves<TILE>::MIN) void fe_gemm_fp8_codes##SUFFIX(FP8C_GEMM_PARAMS) {    \
+        gemm_fp8_codes_kernel<TILE, SK>(c, aq, w, alpha, res, m, n, k, ldc, group_m, w_snt, w_skt, w_sr, sc);              \
+    }
+FP8C_GEMM_KERNEL(, Fp8Tile, false)
+FP8C_GEMM_KERNEL(_sk, Fp8Tile, true)
+FP8C_GEMM_KERNEL(_s1, Fp8TileS1, false)
+FP8C_GEMM_KERNEL(_s2, Fp8TileS2, false)
 
 // ---- GEMV (1..48 rows) -------------------------------------------------------------------------------------------------
 
@@ -1024,13 +1032,13 @@ __device__ __forceinline__ void mfma_peak_body(float* out, uint32_t iters, uint3
     auto h = [&](uint32_t flip) { return ((rnd() & keep16) | base16) ^ flip; };
     auto c = [&](uint32_t flip) { return (int)(((rnd() & 0x8f8f8f8fu) | 0x30303030u) ^ flip); };
     u32x4 a16[4], b16[4];
-    gm_i32x8 a8[4], b8[4];
+    g8_i32x8 a8[4], b8[4];
 #pragma unroll
     for (int i = 0; i < 4; i++) {
         a16[i] = (u32x4){h(0), h((lane & 1) << 15), h(0), h((uint32_t)i << 31)};
         b16[i] = (u32x4){h((lane & 2) << 14), h(0), h((uint32_t)i << 15), h(0)};
-        a8[i] = (gm_i32x8){c(0), c((lane & 1) << 7), c((uint32_t)i << 31), c(0), c(0), c(0), c(0), c(0)};
-        b8[i] = (gm_i32x8){c(0), c((lane & 2) << 6), c(0), c(0), c(0), c((uint32_t)i << 15), c(0), c(0)};
+        a8[i] = (g8_i32x8){c(0), c((lane & 1) << 7), c((uint32_t)i << 31), c(0), c(0), c(0), c(0), c(0)};
+        b8[i] = (g8_i32x8){c(0), c((lane & 2) << 6), c(0), c(0), c(0), c((uint32_t)i << 15), c(0), c(0)};
     }
     for (uint32_t it = 0; it < iters; it++) {
 #pragma unroll
