@@ -60,7 +60,7 @@ struct fe_exl3_options {
     uint32_t fused_rot_pairs = 16; // ... up to this many (row, 128-channel block) pairs a program (FE_EXL3_FUSED_ROT_PAIRS)
     uint32_t group = 1;            // linears of one input share a launch (FE_EXL3_NO_GROUP=1: one launch each)
     uint32_t hat_rows = kHatRows;  // rows from which the prefill decodes once (FE_EXL3_HAT_ROWS; 0: never)
-    uint32_t lds_pad = 1;          // LDS request that pins the programs per CU to the plan's occ (FE_EXL3_NO_LDS_PAD=1: off)
+    uint32_t lds_pad = 1;          // LDS request that spreads a launch's programs over the CUs (FE_EXL3_NO_LDS_PAD=1: off)
     uint32_t fuse = 1;             // consecutive programs share a workgroup when a launch has more than the CUs hold (FE_EXL3_NO_FUSE=1: off)
     uint32_t gemm_group_m = 8;     // raster group of the prefill GEMM (FE_EXL3_GROUP)
     uint32_t gemm_splits = 8;      // most pieces a cut output tile of the prefill GEMM takes (FE_GEMM_SPLITS; 1: never cut)
@@ -71,7 +71,7 @@ struct fe_exl3_options {
     uint32_t chain_down_units = 0;
     uint32_t handoff_fenced = 0;   // 1..16 rows through the kernels whose hand-off uses release / acquire fences (a slow cross-check)
     uint32_t mlp_chain = 1;        // the decode MLP (gate, up, down) as one launch where it applies (FE_EXL3_NO_CHAIN=1: off)
-    uint32_t chain_rot_pairs = 32; // (row, 128-channel block) pairs a program rotates at most inside the one-launch MLP (FE_EXL3_CHAIN_ROT_PAIRS)
+    uint32_t chain_rot_pairs = 48; // (row, 128-channel block) pairs a program rotates at most inside the one-launch MLP (FE_EXL3_CHAIN_ROT_PAIRS)
     uint32_t chain_perm = 1;       // the down stage's workgroups in the order in which their inputs get ready (FE_EXL3_CHAIN_PERM)
     uint32_t chain_spin = 1u << 16;  // polls a program of the down stage waits for the front stage's outputs (FE_EXL3_CHAIN_SPIN)
 };
@@ -81,7 +81,8 @@ struct fe_exl3_kernels {
     fe_function_t recon_hat_f32 = nullptr, recon_hat_f16 = nullptr, had_rows = nullptr, had_cols_bf16 = nullptr;
     fe_function_t rot_in = nullptr, rot_in_group = nullptr, probe_v4 = nullptr;
     fe_function_t probe_decode[3] = {nullptr, nullptr, nullptr};  // 3, 4, 5 bits
-    fe_function_t gemvb[6][4] = {};                               // the decode GEMV, [bits slot][row groups - 1]
+    fe_function_t gemvb[6] = {};                                  // the decode GEMV for 1..16 rows, [bits slot]
+    fe_function_t gemvw[6][3] = {};                               // for 17..64 rows, [bits slot][row groups - 2]
     fe_function_t gemvb_fenced[6] = {};                           // the same for 1..16 rows with the fenced hand-off
     fe_function_t mlp[6] = {};                                    // the decode MLP in one launch, [bits slot]
     uint32_t cus = 0;
@@ -171,10 +172,13 @@ int fe_exl3_kernels_load(fe_exl3_kernels **out) {
     }
     for (int i = 0; i < 6; i++) {
         char nm[64];
-        for (int rg = 1; rg <= 4; rg++) {
-            snprintf(nm, sizeof nm, "exl3_gemvb_b%d_r%d", kBits[i], rg);
-            get(&k->gemvb[i][rg - 1], nm);
-            if (!c) c = fe_hip_func_set_max_dyn_lds(k->gemvb[i][rg - 1], 84 * 1024);
+        snprintf(nm, sizeof nm, "exl3_gemvb_b%d_r1", kBits[i]);
+        get(&k->gemvb[i], nm);
+        if (!c) c = fe_hip_func_set_max_dyn_lds(k->gemvb[i], 84 * 1024);
+        for (int rg = 2; rg <= 4; rg++) {
+            snprintf(nm, sizeof nm, "exl3_gemvw_b%d_r%d", kBits[i], rg);
+            get(&k->gemvw[i][rg - 2], nm);
+            if (!c) c = fe_hip_func_set_max_dyn_lds(k->gemvw[i][rg - 2], 84 * 1024);
         }
         snprintf(nm, sizeof nm, "exl3_gemvb_b%d_r1_fenced", kBits[i]);
         get(&k->gemvb_fenced[i], nm);
@@ -307,6 +311,11 @@ static uint32_t plan_programs(const fe_exl3_kernels *kern, const fe_exl3_plan &p
         progs = std::max(p.sk, 1u);
     else
         progs = (p.occ ? p.occ : 4) * std::max(kern->cus, 1u), progs = std::min(progs, units / std::max(p.wk, 1u));
+    // Wider than deep (gate, up): two programs a CU where a plan asks for four. Such linears come in pairs, whose programs
+    // fill the CUs together, and every program leaves its partial sums of every row in memory: 1024 programs of 64 rows wrote
+    // and read 38 MB beside 45 MB of weights. 5120 x 17408 at 4 bits, gate + up + down: 1..16 rows the same, 40 rows 95 -> 87 us,
+    // 64 rows 117 -> 104. (A down projection keeps its shorter runs: it is the tail of the one-launch MLP.)
+    if (p.ver == 3 && p.occ == 4 && n > k) progs = std::min(progs, 2 * std::max(kern->cus, 1u));
     return std::max(1u, std::min(progs, units));
 }
 
@@ -597,9 +606,24 @@ static uint32_t units_per_program(const fe_exl3_linear *l, uint32_t programs) {
 
 static bool fused_rotation_fits(const fe_exl3_linear *l, uint32_t rows) {
     const fe_exl3_options &o = l->kern->opt;
-    if (!o.fused_rot || rows < 1 || rows > kMaxRowsPerPass) return false;
+    if (!o.fused_rot || rows < 1 || rows > 16) return false;
     const uint32_t units = (l->k / 128) * (l->n / 128);
     return rows * ((units + l->programs - 1) / l->programs) <= o.fused_rot_pairs;
+}
+
+// GemvWide<bits, rg>::LDS of k_exl3.hip
+static uint32_t wide_lds(uint32_t bits, uint32_t rg) {
+    const uint32_t stage = rg * 2048 + bits * 1024, depth = 4 * stage <= 36 * 1024 ? 4 : 3;
+    return std::max(depth * stage, 32 * kRedPitch * 4) + 16;
+}
+
+// LDS for a launch of `programs` workgroups of which a CU can hold four: the dispatcher fills a CU as far as registers and
+// LDS allow before it moves on, which would leave CUs empty while others are full; a request that fits the CU's 160 KB as often
+// as the launch has programs for each CU, and not once more, makes the CUs take that many each. (Fewer programs than CUs spread
+// out by themselves.)
+static uint32_t spread_lds(const fe_exl3_kernels *kern, uint32_t programs, uint32_t lds) {
+    const uint32_t cus = std::max(kern->cus, 1u), each = programs <= cus ? 4 : std::min(4u, (programs + cus - 1) / cus);
+    return kern->opt.lds_pad ? std::max(lds, kCuLds / (each + 1) + 512) : lds;
 }
 
 // mirrors GemvJob of k_exl3.hip
@@ -625,9 +649,9 @@ static int launch_job(const fe_exl3_linear *const *ls, size_t count, fe_stream_t
     // Programs of the partition a workgroup runs one after the other (`fuse`): when the members' programs together are
     // more than the CUs hold at once, consecutive programs share a workgroup instead of waiting for a free place, which
     // saves the second one's start-up. The partition, and with it every sum, stays the member's own.
-    uint32_t occ = 0, total = 0;
-    for (size_t i = 0; i < count; i++) occ = std::max(occ, ls[i]->plan.occ), total += ls[i]->programs;
-    const uint32_t places = std::max(1u, (occ ? occ : 4) * std::max(kern->cus, 1u));
+    uint32_t total = 0;
+    for (size_t i = 0; i < count; i++) total += ls[i]->programs;
+    const uint32_t places = 4 * std::max(kern->cus, 1u);
     // (measured on gate + up, 4 bits: 34.1 against 35.6 us at 1 row, 36.8 / 38.2 at 4, even at 8, 44.8 / 41.9 at 16, where the
     // longer run's inputs no longer fit the staging buffer in one piece: up to 4 rows; 4-unit programs of 17408 x 5120 sharing a
     // workgroup at 8 / 16 rows: 61.6 / 77.1 us a block against 65.2 / 75.8 without)
@@ -656,21 +680,22 @@ static int launch_job(const fe_exl3_linear *const *ls, size_t count, fe_stream_t
         run_steps = std::max(run_steps, 2 * fuse * ((units + l->programs - 1) / l->programs));
     }
     for (size_t i = count; i <= kGroupMax; i++) g.first[i] = programs;
+    uint32_t k = ls[0]->k, mode = (uint32_t)y_dtype;
+    const uint32_t bits = ls[0]->bits;
+    if (rows > 16 && !in.x) {
+        const uint32_t rg = (rows + 15) / 16;
+        void *args[] = {&g, &k, &rows, &mode};
+        return fe_hip_launch(kern->gemvw[bits_slot(bits)][rg - 2], programs, 1, 1, 256, 1, 1, spread_lds(kern, programs, wide_lds(bits, rg)), s, args);
+    }
     // staged inputs: the whole run where the LDS budget holds it for `rows` rows, else chunks of a multiple of 4 load steps
-    const uint32_t red = std::min(rows, 32u) * kRedPitch * 4;  // (more than 32 rows pass through it in two halves)
-    uint32_t chunk = std::max(4u, ((std::max(kJobLdsBudget, red + rows * 528) - red) / rows - 16) / 128 / 4 * 4);
+    const uint32_t red = rows * kRedPitch * 4;
+    uint32_t chunk = std::max(4u, ((kJobLdsBudget - red) / rows - 16) / 128 / 4 * 4);
     chunk = std::min(chunk, (run_steps + 3) / 4 * 4);
-    uint32_t lds = red + rows * (chunk * 128 + 16);
-    // Exactly occ programs a CU: the dispatcher fills a CU as far as registers and LDS allow (5 programs) before it moves
-    // on, which would leave CUs empty while others hold 5; an LDS request that fits occ times into the CU's 160 KB, and
-    // not occ + 1 times, makes the CUs take occ each.
-    // (several linears: the most programs per CU any of them asks for)
-    if (occ && kern->opt.lds_pad) lds = std::max(lds, kCuLds / (occ + 1) + 512);
-    uint32_t k = ls[0]->k, mode = (uint32_t)y_dtype, x_mode = in.mode, ldx = in.ld, inv_spb = 0xffffffffu / (k / 64);
+    const uint32_t lds = spread_lds(kern, programs, red + rows * (chunk * 128 + 16));
+    uint32_t x_mode = in.mode, ldx = in.ld, inv_spb = 0xffffffffu / (k / 64);
     fe_devptr_t x = in.x, x2 = in.x2;
     void *args[] = {&g, &x, &x2, &x_mode, &ldx, &k, &rows, &mode, &chunk, &inv_spb, &fuse};
-    const fe_function_t f = kern->opt.handoff_fenced && rows <= 16 ? kern->gemvb_fenced[bits_slot(ls[0]->bits)]
-                                                                   : kern->gemvb[bits_slot(ls[0]->bits)][(rows + 15) / 16 - 1];
+    const fe_function_t f = kern->opt.handoff_fenced ? kern->gemvb_fenced[bits_slot(bits)] : kern->gemvb[bits_slot(bits)];
     return fe_hip_launch(f, programs, 1, 1, 256, 1, 1, lds, s, args);
 }
 
@@ -888,7 +913,7 @@ static bool mlp_chain_fits(const fe_exl3_linear *g, const fe_exl3_linear *u, con
     if (g->k != u->k || g->n != u->n || d->k != g->n) return false;
     if (rows < 1 || rows > 16 || rows > ws->max_rows || y_dtype < 0 || y_dtype > 3) return false;
     // every stage rotates its own input inside the launch: (row, 128-channel block) pairs a program. As separate launches
-    // that pays up to 16 pairs (fused_rotation_fits); inside the one launch up to 32, i.e. up to 4 rows on the 27B-shaped
+    // that pays up to 16 pairs (fused_rotation_fits); inside the one launch up to 48, i.e. up to 4 rows on the 27B-shaped
     // MLP (measured at 4 bits, cold weights: 4 rows 53.6 us against 56.8 us for rotation and GEMV launches; 8 rows 65.1 / 60.1)
     const fe_exl3_options &o = g->kern->opt;
     const uint32_t d_units = units_per_program(d, chain_part(d)->programs);
@@ -908,8 +933,7 @@ static int launch_mlp(const fe_exl3_linear *g, const fe_exl3_linear *u, const fe
     MlpChainArgs a{};
     const fe_exl3_linear *front[2] = {g, u};
     const fe_devptr_t ys[2] = {yg, yu};
-    const uint32_t occ = std::max({g->plan.occ, u->plan.occ, d->plan.occ});
-    const uint32_t places = std::max(1u, (occ ? occ : 4) * std::max(kern->cus, 1u));
+    const uint32_t places = 4 * std::max(kern->cus, 1u);
     // (as launch_job: consecutive programs of the front stage share a workgroup when they are more than the CUs hold)
     a.fuse1 = kern->opt.fuse && rows <= 4 ? std::min(4u, std::max(1u, (g->programs + u->programs + places - 1) / places)) : 1;
     a.fuse2 = 1;
@@ -934,13 +958,12 @@ static int launch_mlp(const fe_exl3_linear *g, const fe_exl3_linear *u, const fe
     a.inv_spb1 = 0xffffffffu / (a.k1 / 64), a.inv_spb2 = 0xffffffffu / (a.k2 / 64);
     const uint32_t red = rows * kRedPitch * 4;
     auto chunk_of = [&](uint32_t run_steps) {
-        const uint32_t c = std::max(4u, ((std::max(kJobLdsBudget, red + rows * 528) - red) / rows - 16) / 128 / 4 * 4);
+        const uint32_t c = std::max(4u, ((kJobLdsBudget - red) / rows - 16) / 128 / 4 * 4);
         return std::min(c, (run_steps + 3) / 4 * 4);
     };
     a.chunk1 = chunk_of(2 * a.fuse1 * std::max(units_per_program(g, g->programs), units_per_program(u, u->programs)));
     a.chunk2 = chunk_of(2 * a.fuse2 * units_per_program(d, dp->programs));
-    uint32_t lds = red + rows * (std::max(a.chunk1, a.chunk2) * 128 + 16);
-    if (occ && kern->opt.lds_pad) lds = std::max(lds, kCuLds / (occ + 1) + 512);
+    const uint32_t lds = spread_lds(kern, places, red + rows * (std::max(a.chunk1, a.chunk2) * 128 + 16));
     // the down stage's programs in the order in which their inputs get ready (the linear's table)
     a.perm = kern->opt.chain_perm ? dp->order.p : 0;
     a.spin_limit = kern->opt.chain_spin;

@@ -3,6 +3,7 @@
 #include <type_traits>
 
 #include "exl3_trellis.h"
+#include "gemm8.h"
 
 // ---- whole-tensor reconstruct (bits at run time: load-time code) ---------------------------------------------------
 
@@ -199,7 +200,7 @@ extern "C" __global__ __launch_bounds__(128) void exl3_rot_in_group(RotGroup g, 
 #endif
 #define GEMV_RED_PITCH 132  // floats a row of the 128-column partial sums (16-byte aligned, banks spread)
 
-// ---- decode GEMV, balanced over the CUs (1..64 rows) ------------------------------------------------------------------
+// ---- decode GEMV, balanced over the CUs (1..16 rows) ------------------------------------------------------------------
 //
 // Work unit = one 128-channel block of K of one 128-column block of N (two load steps); units are ordered column block
 // by column block and the member's `programs` programs each take one contiguous run of them, base + 1 units for the first
@@ -336,7 +337,7 @@ __device__ __forceinline__ uint32_t load_agent_u32(const uint32_t* p) {
 // FENCED: the hand-off written with the memory model's own means (plain stores, a release fence at agent scope, the
 // arrival, an acquire fence, plain loads) instead of write-through stores and loads that pass the L2: the slow form
 // (the release writes the whole L2 back), kept as a cross-check of the fast one (option "handoff_fenced").
-template <int BITS, int RG, int CHAIN = 0, bool FENCED = false>
+template <int BITS, int CHAIN = 0, bool FENCED = false>
 __device__ __forceinline__ void gemvb_body(const GemvMember& mb, uint32_t p0, uint32_t np, uint32_t k, uint32_t m, uint32_t y_mode,
                                            uint32_t chunk, uint32_t inv_spb, const RotSrc src, uint16_t* stamp_base,
                                            const ChainCtx ch = ChainCtx{}) {
@@ -370,11 +371,8 @@ __device__ __forceinline__ void gemvb_body(const GemvMember& mb, uint32_t p0, ui
     uint32_t nb = udiv_inv(2 * u0, spb, inv_spb), st = 2 * u0 - nb * spb;  // where the run stands: column block, load step
     const uint32_t nb_run0 = nb, st_run0 = st;
 
-    // [min(m, 32)][GEMV_RED_PITCH] sums of a finished segment: more than 32 rows pass through it in two halves, so that the
-    // programs of 33..64 rows still fit three to a CU
-    float* red = (float*)lds;
-    const uint32_t red_rows = RG > 2 ? 32 : m;
-    unsigned char* xs = (unsigned char*)(red + red_rows * GEMV_RED_PITCH);  // [m][xpitch] rotated inputs of a chunk of the run
+    float* red = (float*)lds;                                        // [m][GEMV_RED_PITCH] sums of a finished segment
+    unsigned char* xs = (unsigned char*)(red + m * GEMV_RED_PITCH);  // [m][xpitch] rotated inputs of a chunk of the run
     const uint32_t xpitch = chunk * 128 + 16;
 
     const uint32_t lane_word = g * mb.stride_k + (2 * wave + tau) * tw;
@@ -385,15 +383,9 @@ __device__ __forceinline__ void gemvb_body(const GemvMember& mb, uint32_t p0, ui
         __builtin_amdgcn_make_buffer_rsrc((void*)mb.trellis, 0, (k / 16) * (n / 16) * tw * 4, 0x00020000);
     uint32_t snext = nb * mb.stride_nb * 4 + st * step_bytes;  // byte offset of the next load step to request
 
-    uint32_t xrow[RG];
-#pragma unroll
-    for (int rg = 0; rg < RG; rg++) {
-        uint32_t row = 16 * rg + r;
-        xrow[rg] = (row < m ? row : m - 1) * xpitch + g * 32;
-    }
-    f32x4 acc[RG][2];
-#pragma unroll
-    for (int rg = 0; rg < RG; rg++) acc[rg][0] = acc[rg][1] = (f32x4){0.f, 0.f, 0.f, 0.f};
+    const uint32_t xrow = (r < m ? r : m - 1) * xpitch + g * 32;
+    f32x4 acc[2];
+    acc[0] = acc[1] = (f32x4){0.f, 0.f, 0.f, 0.f};
 
     const uint32_t hw = tid >> 5, l32 = tid & 31;
     // Rotating here: (row, 128-channel block) pairs of a chunk go to the half wavefronts: half wavefront hw takes blocks hw,
@@ -488,15 +480,12 @@ __device__ __forceinline__ void gemvb_body(const GemvMember& mb, uint32_t p0, ui
         // keep the refill where it is issued: left alone, the scheduler sinks the loads to the end of the group, right in
         // front of the wait for them
         __builtin_amdgcn_sched_barrier(0);
-#pragma unroll
-        for (int rg = 0; rg < RG; rg++) {
-            const unsigned char* xp = xs + xrow[rg] + t * 128;
-            f16x8 x0 = *(const f16x8*)xp, x1 = *(const f16x8*)(xp + 16);
-            acc[rg][0] = __builtin_amdgcn_mfma_f32_16x16x32_f16(op[0][0], x0, acc[rg][0], 0, 0, 0);
-            acc[rg][1] = __builtin_amdgcn_mfma_f32_16x16x32_f16(op[1][0], x0, acc[rg][1], 0, 0, 0);
-            acc[rg][0] = __builtin_amdgcn_mfma_f32_16x16x32_f16(op[0][1], x1, acc[rg][0], 0, 0, 0);
-            acc[rg][1] = __builtin_amdgcn_mfma_f32_16x16x32_f16(op[1][1], x1, acc[rg][1], 0, 0, 0);
-        }
+        const unsigned char* xp = xs + xrow + t * 128;
+        f16x8 x0 = *(const f16x8*)xp, x1 = *(const f16x8*)(xp + 16);
+        acc[0] = __builtin_amdgcn_mfma_f32_16x16x32_f16(op[0][0], x0, acc[0], 0, 0, 0);
+        acc[1] = __builtin_amdgcn_mfma_f32_16x16x32_f16(op[1][0], x0, acc[1], 0, 0, 0);
+        acc[0] = __builtin_amdgcn_mfma_f32_16x16x32_f16(op[0][1], x1, acc[0], 0, 0, 0);
+        acc[1] = __builtin_amdgcn_mfma_f32_16x16x32_f16(op[1][1], x1, acc[1], 0, 0, 0);
         __builtin_amdgcn_sched_barrier(0);
     };
 
@@ -539,46 +528,17 @@ __device__ __forceinline__ void gemvb_body(const GemvMember& mb, uint32_t p0, ui
 
     // The segment of column block fnb that ends here: its sums meet in LDS, and then either are the block's sums (the
     // block lies in this run alone) or go to z for the program that arrives last at the block.
-    // More than 32 rows (RG > 2): the sums of rows 0..31, then of rows 32.., meet in `red`; use(row, its sums) is called for
-    // each row by the half wavefront that takes it.
-    auto through_red_halves = [&](auto use) {
-        float* rp = red + 32 * wave + 16 * (g >> 1) + 4 * (g & 1);
-#pragma unroll
-        for (int h = 0; h < 2; h++) {
-            __syncthreads();  // the readers before are done with `red`
-#pragma unroll
-            for (int rg = 2 * h; rg < (2 * h + 2 < RG ? 2 * h + 2 : RG); rg++) {
-                const uint32_t row = 16 * rg + r;  // accumulator column = input row
-                if (row < m) {
-                    *(f32x4*)(rp + (row - 32 * h) * GEMV_RED_PITCH) = acc[rg][0];
-                    *(f32x4*)(rp + (row - 32 * h) * GEMV_RED_PITCH + 8) = acc[rg][1];
-                }
-                acc[rg][0] = acc[rg][1] = (f32x4){0.f, 0.f, 0.f, 0.f};
-            }
-            __syncthreads();
-            const uint32_t end = m < 32u * h + 32 ? m : 32u * h + 32;
-            for (uint32_t row = 32 * h + hw; row < end; row += 8)
-                use(row, *(const f32x4*)(red + (row - 32 * h) * GEMV_RED_PITCH + 4 * l32));
-        }
-    };
-
     auto flush = [&](uint32_t fnb, uint32_t p) {
-        if constexpr (RG <= 2) __syncthreads();  // the previous segment's readers are done with `red`
+        __syncthreads();  // the previous segment's readers are done with `red`
         // rows 4 g .. 4 g + 3 of A are columns 16 (g >> 1) + 4 (g & 1) + 8 h .. + 3 of the wavefront's 32 (tile g >> 1 of
         // its pair, n = 4 (g & 1) + i + 8 h): a lane's four sums of either half are four neighbouring columns
-        if constexpr (RG <= 2) {
-            float* rp = red + 32 * wave + 16 * (g >> 1) + 4 * (g & 1);
-#pragma unroll
-            for (int rg = 0; rg < RG; rg++) {
-                uint32_t row = 16 * rg + r;  // accumulator column = input row
-                if (row < m) {
-                    *(f32x4*)(rp + row * GEMV_RED_PITCH) = acc[rg][0];
-                    *(f32x4*)(rp + row * GEMV_RED_PITCH + 8) = acc[rg][1];
-                }
-                acc[rg][0] = acc[rg][1] = (f32x4){0.f, 0.f, 0.f, 0.f};
-            }
-            __syncthreads();
+        float* rp = red + 32 * wave + 16 * (g >> 1) + 4 * (g & 1);
+        if (r < m) {  // accumulator column = input row
+            *(f32x4*)(rp + r * GEMV_RED_PITCH) = acc[0];
+            *(f32x4*)(rp + r * GEMV_RED_PITCH + 8) = acc[1];
         }
+        acc[0] = acc[1] = (f32x4){0.f, 0.f, 0.f, 0.f};
+        __syncthreads();
         FE_STAMP(4);
         const uint32_t col0 = fnb * 128;
         // programs of the block's first and last unit
@@ -586,17 +546,10 @@ __device__ __forceinline__ void gemvb_body(const GemvMember& mb, uint32_t p0, ui
         const uint32_t first_prog = ua < cut ? udiv_inv(ua, base + 1, mb.inv_base1) : rem + udiv_inv(ua - cut, base, mb.inv_base);
         const uint32_t last_prog = ub < cut ? udiv_inv(ub, base + 1, mb.inv_base1) : rem + udiv_inv(ub - cut, base, mb.inv_base);
         if (first_prog == last_prog) {
-            if constexpr (RG > 2) {
-                through_red_halves([&](uint32_t row, f32x4 t) {
-                    float v[4] = {t[0], t[1], t[2], t[3]};
-                    finish(v, col0, row);
-                });
-            } else {
-                for (uint32_t row = hw; row < m; row += 8) {
-                    f32x4 t = *(const f32x4*)(red + row * GEMV_RED_PITCH + 4 * l32);
-                    float v[4] = {t[0], t[1], t[2], t[3]};
-                    finish(v, col0, row);
-                }
+            for (uint32_t row = hw; row < m; row += 8) {
+                f32x4 t = *(const f32x4*)(red + row * GEMV_RED_PITCH + 4 * l32);
+                float v[4] = {t[0], t[1], t[2], t[3]};
+                finish(v, col0, row);
             }
             block_done(fnb);
             return;
@@ -609,10 +562,7 @@ __device__ __forceinline__ void gemvb_body(const GemvMember& mb, uint32_t p0, ui
         //     after the barrier that publishes last_flag.
         // Every byte that crosses is written through and read through, so no cache write-back or invalidate is needed.
         float* zseg = mb.z + (size_t)(p + fnb) * m * 128;
-        if constexpr (RG > 2) {
-            through_red_halves([&](uint32_t row, f32x4 t) { store_agent_f32x4(zseg + row * 128 + 4 * l32, t); });
-            agent_stores_wait();
-        } else if constexpr (FENCED) {
+        if constexpr (FENCED) {
             for (uint32_t row = hw; row < m; row += 8)
                 *(f32x4*)(zseg + row * 128 + 4 * l32) = *(const f32x4*)(red + row * GEMV_RED_PITCH + 4 * l32);
             __builtin_amdgcn_fence(__ATOMIC_RELEASE, "agent");
@@ -639,7 +589,7 @@ __device__ __forceinline__ void gemvb_body(const GemvMember& mb, uint32_t p0, ui
             const __amdgpu_buffer_rsrc_t zrs = __builtin_amdgcn_make_buffer_rsrc(
                 (void*)(mb.z + (size_t)(first_prog + fnb) * m * 128), 0, nseg * m * 512, 0x00020000);
             auto rows_of = [&](auto rb_tag) {
-                constexpr int RB = decltype(rb_tag)::value, SB = (BITS <= 4 && RG == 1 ? 12 : 8) / RB;
+                constexpr int RB = decltype(rb_tag)::value, SB = (BITS <= 4 ? 12 : 8) / RB;
                 for (uint32_t row0 = hw; row0 < m; row0 += 8 * RB) {
                     float v[RB][4];
 #pragma unroll
@@ -705,7 +655,7 @@ __device__ __forceinline__ void gemvb_body(const GemvMember& mb, uint32_t p0, ui
                 }
             }
         } else {  // rotated inputs of the chunk's load steps -> xs [row][cs * 64 fp16], NB 16-byte pieces in flight a thread
-            constexpr int NB = RG == 1 ? FE_STAGE_NB1 : 8;
+            constexpr int NB = FE_STAGE_NB1;
             const uint32_t chunks16 = cs * 8, total = m * chunks16, inv16 = 0xffffffffu / chunks16;
             for (uint32_t i0 = tid; i0 < total; i0 += 256 * NB) {
                 u32x4 v[NB];
@@ -763,15 +713,15 @@ __device__ __forceinline__ void gemvb_body(const GemvMember& mb, uint32_t p0, ui
     FE_STAMP(8);
 }
 
-// (second launch bound: wavefronts per SIMD the registers must allow. Four programs a CU for up to 16 rows.)
-#define GEMVB_KERNEL(BITS, RG)                                                                                        \
-    extern "C" __global__ __launch_bounds__(256, RG == 1 ? 4 : 2) void exl3_gemvb_b##BITS##_r##RG(                    \
+// (second launch bound: wavefronts per SIMD the registers must allow: four programs a CU)
+#define GEMVB_KERNEL(BITS)                                                                                        \
+    extern "C" __global__ __launch_bounds__(256, 4) void exl3_gemvb_b##BITS##_r1(                                      \
         GemvJob job, const void* x, const void* x2, uint32_t x_mode, uint32_t ldx, uint32_t k, uint32_t m,             \
         uint32_t y_mode, uint32_t chunk, uint32_t inv_spb, uint32_t fuse) {                                            \
         uint32_t i = 0;                                                                                               \
         while (i + 1 < job.count && blockIdx.x >= job.first[i + 1]) i++;                                              \
         const uint32_t p0 = (blockIdx.x - job.first[i]) * fuse, left = job.m[i].programs - p0;                        \
-        gemvb_body<BITS, RG>(job.m[i], p0, left < fuse ? left : fuse, k, m, y_mode, chunk, inv_spb,                   \
+        gemvb_body<BITS>(job.m[i], p0, left < fuse ? left : fuse, k, m, y_mode, chunk, inv_spb,                   \
                              RotSrc{x, x2, x_mode, ldx}, job.m[0].xh);                                                \
     }
 #define GEMVB_FENCED_KERNEL(BITS)                                                                                     \
@@ -781,10 +731,10 @@ __device__ __forceinline__ void gemvb_body(const GemvMember& mb, uint32_t p0, ui
         uint32_t i = 0;                                                                                               \
         while (i + 1 < job.count && blockIdx.x >= job.first[i + 1]) i++;                                              \
         const uint32_t p0 = (blockIdx.x - job.first[i]) * fuse, left = job.m[i].programs - p0;                        \
-        gemvb_body<BITS, 1, 0, true>(job.m[i], p0, left < fuse ? left : fuse, k, m, y_mode, chunk, inv_spb,           \
+        gemvb_body<BITS, 0, true>(job.m[i], p0, left < fuse ? left : fuse, k, m, y_mode, chunk, inv_spb,           \
                                      RotSrc{x, x2, x_mode, ldx}, job.m[0].xh);                                        \
     }
-#define GEMVB_FAMILY(BITS) GEMVB_KERNEL(BITS, 1) GEMVB_KERNEL(BITS, 2) GEMVB_KERNEL(BITS, 3) GEMVB_KERNEL(BITS, 4) GEMVB_FENCED_KERNEL(BITS)
+#define GEMVB_FAMILY(BITS) GEMVB_KERNEL(BITS) GEMVB_FENCED_KERNEL(BITS)
 
 // The decode MLP in one launch, 1..16 rows: grid = the front stage's workgroups (gate and up, alternating when their
 // counts are equal, so that block b of both is finished at about the same time), then the down stage's. Down workgroup
@@ -813,14 +763,14 @@ struct MlpChain {
                 lw = w - c.front.first[i];                                                                            \
             }                                                                                                         \
             const uint32_t p0 = lw * c.fuse1, left = c.front.m[i].programs - p0;                                      \
-            gemvb_body<BITS, 1, 1>(c.front.m[i], p0, left < c.fuse1 ? left : c.fuse1, c.k1, m, 0, c.chunk1, c.inv_spb1, \
+            gemvb_body<BITS, 1>(c.front.m[i], p0, left < c.fuse1 ? left : c.fuse1, c.k1, m, 0, c.chunk1, c.inv_spb1, \
                                    RotSrc{x, nullptr, x_mode, ldx}, c.front.m[0].xh,                                  \
                                    ChainCtx{c.state, c.state + (1 + i * nbf) * FE_CHAIN_STRIDE, nbf, nbd, c.spin_limit}); \
         } else {                                                                                                      \
             uint32_t lw = w - c.front_wgs;                                                                            \
             if (c.perm) lw = c.perm[lw];                                                                              \
             const uint32_t p0 = lw * c.fuse2, left = c.down.programs - p0;                                            \
-            gemvb_body<BITS, 1, 2>(c.down, p0, left < c.fuse2 ? left : c.fuse2, c.k2, m, y_mode, c.chunk2, c.inv_spb2, \
+            gemvb_body<BITS, 2>(c.down, p0, left < c.fuse2 ? left : c.fuse2, c.k2, m, y_mode, c.chunk2, c.inv_spb2, \
                                    RotSrc{c.front.m[0].y, c.front.m[1].y, 2, c.front.m[0].n}, c.front.m[0].xh,        \
                                    ChainCtx{c.state, c.state + FE_CHAIN_STRIDE, nbf, nbd, c.spin_limit});             \
         }                                                                                                             \
@@ -837,6 +787,194 @@ GEMVB_FAMILY(4)
 GEMVB_FAMILY(5)
 GEMVB_FAMILY(6)
 GEMVB_FAMILY(8)
+
+// ---- the same GEMV for more rows ------------------------------------------------------------------------------------------
+//
+// 17..64 rows. The programs, their runs, the order of every sum and so the bits are gemvb_body's. What differs is how a program
+// gets its operands and hands its sums over: both grow with the rows while the decode does not. Staging a run's inputs
+// through registers before its first step kept a program of 40 rows waiting for 6 of its 18 us, in chunks of 4 steps, and its
+// sums took 3.5 us more to pass through LDS on their way to z. Here the rotated inputs and the trellis words of a load step go
+// straight from memory into LDS, DEPTH - 1 steps ahead, and the sums go to z as the accumulators hold them, whole wavefronts at a
+// time; only the program that finishes a block turns them into rows. Registers stay under 128, so that four programs share a
+// CU. Bound by the partial sums (programs x rows x 512 bytes, written and read once) and by the decode. us, 4 bits, before ->
+// after, 40 rows: 5120 x 5120 23.0 -> 18.5, 2 x (5120 x 17408) 70 -> 55, 17408 x 5120 42.7 -> 35.
+template <int BITS, int RG>
+struct GemvWide {
+    static constexpr int X_STAGE = RG * 2048, W_STAGE = 1024 * BITS;
+    static constexpr int DEPTH = 4 * (X_STAGE + W_STAGE) <= 36 * 1024 ? 4 : 3;  // (so that four programs fit a CU, up to 5 bits)
+    static constexpr int W_AT = DEPTH * X_STAGE, STAGES = W_AT + DEPTH * W_STAGE;
+    static constexpr int LX = (2 * RG + 3) / 4, LW = (BITS + 3) / 4;  // loads a wavefront issues a step: 1 KB pieces, some twice
+    static constexpr int RED = 32 * GEMV_RED_PITCH * 4, LDS = (STAGES > RED ? STAGES : RED) + 16;
+};
+template <int BITS, int RG>
+__device__ __forceinline__ void gemv_wide_body(const GemvMember& mb, uint32_t p, uint32_t k, uint32_t m, uint32_t y_mode) {
+    typedef GemvWide<BITS, RG> C;
+    extern __shared__ __attribute__((aligned(16))) unsigned char lds[];
+    uint32_t* last_flag = (uint32_t*)(lds + C::LDS - 16);
+    const uint32_t tid = threadIdx.x, lane = tid & 63, wave = __builtin_amdgcn_readfirstlane(tid >> 6), hw = tid >> 5, l32 = tid & 31;
+    const uint32_t r = lane & 15, g = lane >> 4;
+    const uint32_t n = mb.n, upb = k / 128, base = mb.base, rem = mb.rem;
+    const u32x4 xrs = g8_rsrc(mb.xh, m * k * 2), wrs = g8_rsrc(mb.trellis, (k / 16) * (n / 16) * 32 * BITS);
+    const uint32_t step_bytes = 16 * mb.stride_k, lds0 = g8_lds_addr(lds);
+    uint32_t vx[C::LX], vw[C::LW];
+#pragma unroll
+    for (int j = 0; j < C::LX; j++) {  // piece: 8 rows x 64 channels; 16-byte chunk c of a row at position c ^ (row & 7)
+        const uint32_t row = (wave + 4 * j) % (2 * RG) * 8 + (lane >> 3);
+        vx[j] = ((row < m ? row : m - 1) * k + ((lane & 7) ^ (row & 7)) * 8) * 2;
+    }
+#pragma unroll
+    for (int j = 0; j < C::LW; j++) {  // [4 k steps][8 tiles][8 BITS words]
+        const uint32_t at = (wave + 4 * j) % BITS * 1024 + lane * 16;
+        vw[j] = 4 * (at / (256 * BITS) * mb.stride_k) + at % (256 * BITS);
+    }
+    const unsigned char* xp = lds + r * 128;
+    const uint32_t xo0 = ((2 * g) ^ (r & 7)) << 4, xo1 = ((2 * g + 1) ^ (r & 7)) << 4;
+    const unsigned char* wp = lds + C::W_AT + (g * 8 + 2 * wave + (r >> 3)) * (32 * BITS) + (r & 7) * (4 * BITS);
+
+    f32x4 acc[RG][2];
+    // Rows 16 rg .. of the accumulators lie in z one after the other: of each half h, wavefront and g 4 columns of the rows that exist.
+    auto zoff = [&](int rg, int h) {
+        const uint32_t mr = m - 16 * rg < 16 ? m - 16 * rg : 16;
+        return (uint32_t)(16 * rg) * 512 + ((h * 16 + wave * 4 + g) * mr + r) * 16;
+    };
+    uint32_t u = p * base + (p < rem ? p : rem);
+    const uint32_t uend = u + base + (p < rem ? 1 : 0);
+    while (u < uend) {
+        const uint32_t nb = u / upb, in = u - nb * upb, units = uend - u < upb - in ? uend - u : upb - in, steps = 2 * units;
+        u += units;
+        const uint32_t w0 = nb * mb.stride_nb * 4 + 2 * in * step_bytes, x0 = 2 * in * 128;
+        auto issue = [&](uint32_t s, uint32_t slot) {  // past the end: the last step again, never used
+            s = s < steps ? s : steps - 1;
+#pragma unroll
+            for (int j = 0; j < C::LX; j++)
+                g8_load_lds16(xrs, lds0 + slot * C::X_STAGE + (wave + 4 * j) % (2 * RG) * 1024, vx[j], x0 + s * 128);
+#pragma unroll
+            for (int j = 0; j < C::LW; j++)
+                g8_load_lds16(wrs, lds0 + C::W_AT + slot * C::W_STAGE + (wave + 4 * j) % BITS * 1024, vw[j], w0 + s * step_bytes);
+        };
+#pragma unroll
+        for (int s = 0; s < C::DEPTH - 1; s++) issue(s, s);
+#pragma unroll
+        for (int rg = 0; rg < RG; rg++) acc[rg][0] = acc[rg][1] = (f32x4){0.f, 0.f, 0.f, 0.f};
+        uint32_t slot = 0;
+        for (uint32_t s = 0; s < steps; s++) {
+            g8_loads_wait<(C::DEPTH - 2) * (C::LX + C::LW)>();
+            g8_barrier();
+            issue(s + C::DEPTH - 1, slot ? slot - 1 : C::DEPTH - 1);
+            LaneWords<BITS> lw;
+            const uint32_t* words = (const uint32_t*)(wp + slot * C::W_STAGE);
+            if constexpr (BITS % 4 == 0) {
+#pragma unroll
+                for (int i = 0; i < BITS; i += 4) {
+                    const u32x4 t = *(const u32x4*)(words + i);
+                    lw.w[i + 1] = t[0], lw.w[i + 2] = t[1], lw.w[i + 3] = t[2], lw.w[i + 4] = t[3];
+                }
+            } else {
+#pragma unroll
+                for (int i = 0; i < BITS; i++) lw.w[i + 1] = words[i];
+            }
+            lw.w[0] = lane_prev_word(lw.w[BITS]);
+            f16x8 op[2][2];
+            decode_lane<BITS>(lw, op);
+            const unsigned char* xs = xp + slot * C::X_STAGE;
+#pragma unroll
+            for (int rg = 0; rg < RG; rg++) {
+                const f16x8 b0 = *(const f16x8*)(xs + rg * 2048 + xo0), b1 = *(const f16x8*)(xs + rg * 2048 + xo1);
+                acc[rg][0] = __builtin_amdgcn_mfma_f32_16x16x32_f16(op[0][0], b0, acc[rg][0], 0, 0, 0);
+                acc[rg][1] = __builtin_amdgcn_mfma_f32_16x16x32_f16(op[1][0], b0, acc[rg][1], 0, 0, 0);
+                acc[rg][0] = __builtin_amdgcn_mfma_f32_16x16x32_f16(op[0][1], b1, acc[rg][0], 0, 0, 0);
+                acc[rg][1] = __builtin_amdgcn_mfma_f32_16x16x32_f16(op[1][1], b1, acc[rg][1], 0, 0, 0);
+            }
+            slot = slot + 1 == C::DEPTH ? 0 : slot + 1;
+        }
+        // the programs of the block's first and last unit
+        const uint32_t cut = rem * (base + 1), ua = nb * upb, ub = ua + upb - 1;
+        const uint32_t first_prog = ua < cut ? udiv_inv(ua, base + 1, mb.inv_base1) : rem + udiv_inv(ua - cut, base, mb.inv_base);
+        const uint32_t last_prog = ub < cut ? udiv_inv(ub, base + 1, mb.inv_base1) : rem + udiv_inv(ub - cut, base, mb.inv_base);
+        bool mine = true;
+        if (first_prog != last_prog) {  // the hand-off of gemvb_body
+            const uint32_t nseg = last_prog - first_prog + 1;
+            unsigned char* zseg = (unsigned char*)(mb.z + (size_t)(p + nb) * m * 128);
+#pragma unroll
+            for (int rg = 0; rg < RG; rg++)
+                if (16 * rg + r < m) {
+                    store_agent_f32x4((float*)(zseg + zoff(rg, 0)), acc[rg][0]);
+                    store_agent_f32x4((float*)(zseg + zoff(rg, 1)), acc[rg][1]);
+                }
+            agent_stores_wait();
+            __syncthreads();
+            if (tid == 0)
+                *last_flag = __hip_atomic_fetch_add(&mb.counters[nb], 1u, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT) == nseg - 1;
+            __syncthreads();
+            mine = *last_flag;
+            if (mine) {
+                constexpr int SB = RG == 2 ? 2 : 1;  // segments read together (more take registers, and with them resident programs: slower)
+                const __amdgpu_buffer_rsrc_t zrs =
+                    __builtin_amdgcn_make_buffer_rsrc((void*)(mb.z + (size_t)(first_prog + nb) * m * 128), 0, nseg * m * 512, 0x00020000);
+                uint32_t z0[RG], z1[RG];
+#pragma unroll
+                for (int rg = 0; rg < RG; rg++) {
+                    z0[rg] = 16 * rg + r < m ? zoff(rg, 0) : 0, z1[rg] = 16 * rg + r < m ? zoff(rg, 1) : 0;
+                    acc[rg][0] = acc[rg][1] = (f32x4){0.f, 0.f, 0.f, 0.f};
+                }
+                for (uint32_t sp0 = 0; sp0 < nseg; sp0 += SB) {
+                    f32x4 t[SB][RG][2];
+#pragma unroll
+                    for (int b = 0; b < SB; b++)
+#pragma unroll
+                        for (int rg = 0; rg < RG; rg++) {  // (past the last segment: out of range, reads zero)
+                            t[b][rg][0] = load_agent_f32x4(zrs, z0[rg], (sp0 + b) * m * 512);
+                            t[b][rg][1] = load_agent_f32x4(zrs, z1[rg], (sp0 + b) * m * 512);
+                        }
+#pragma unroll
+                    for (int b = 0; b < SB; b++)
+                        if (sp0 + b < nseg) {
+#pragma unroll
+                            for (int rg = 0; rg < RG; rg++) acc[rg][0] += t[b][rg][0], acc[rg][1] += t[b][rg][1];
+                        }
+                }
+                if (tid == 0) __hip_atomic_store(&mb.counters[nb], 0u, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+            }
+        }
+        g8_loads_wait<0>();  // (the repeated last steps) the stages are free
+        __syncthreads();
+        if (mine) {  // the block's sums become rows, up to 32 at a time, and are finished
+            float* red = (float*)lds;
+            float* rp = red + 32 * wave + 16 * (g >> 1) + 4 * (g & 1);
+#pragma unroll
+            for (int r0 = 0; r0 < RG; r0 += 2) {
+#pragma unroll
+                for (int i = r0; i < (r0 + 2 < RG ? r0 + 2 : RG); i++)
+                    if (16 * i + r < m) {
+                        *(f32x4*)(rp + (16 * (i - r0) + r) * GEMV_RED_PITCH) = acc[i][0];
+                        *(f32x4*)(rp + (16 * (i - r0) + r) * GEMV_RED_PITCH + 8) = acc[i][1];
+                    }
+                __syncthreads();
+                const uint32_t end = m < 16u * r0 + 32 ? m : 16u * r0 + 32;
+                for (uint32_t row = 16 * r0 + hw; row < end; row += 8) {
+                    const f32x4 t = *(const f32x4*)(red + (row - 16 * r0) * GEMV_RED_PITCH + 4 * l32);
+                    float v[4] = {t[0], t[1], t[2], t[3]};
+                    finish_row(v, l32, mb.svh, nb * 128 + 4 * l32, mb.y, y_mode, (size_t)row * n + nb * 128 + 4 * l32);
+                }
+                __syncthreads();
+            }
+        }
+    }
+}
+#define GEMV_WIDE_KERNEL(BITS, RG)                                                                                    \
+    extern "C" __global__ __launch_bounds__(256, 4) void exl3_gemvw_b##BITS##_r##RG(                         \
+        GemvJob job, uint32_t k, uint32_t m, uint32_t y_mode) {                                                       \
+        uint32_t i = 0;                                                                                               \
+        while (i + 1 < job.count && blockIdx.x >= job.first[i + 1]) i++;                                              \
+        gemv_wide_body<BITS, RG>(job.m[i], blockIdx.x - job.first[i], k, m, y_mode);                                  \
+    }
+#define GEMV_WIDE_FAMILY(BITS) GEMV_WIDE_KERNEL(BITS, 2) GEMV_WIDE_KERNEL(BITS, 3) GEMV_WIDE_KERNEL(BITS, 4)
+GEMV_WIDE_FAMILY(2)
+GEMV_WIDE_FAMILY(3)
+GEMV_WIDE_FAMILY(4)
+GEMV_WIDE_FAMILY(5)
+GEMV_WIDE_FAMILY(6)
+GEMV_WIDE_FAMILY(8)
 
 // ---- probes ----------------------------------------------------------------------------------------------------------
 
