@@ -255,6 +255,32 @@ def test_gemv_long_k_streams_inputs_in_chunks(env, oracle):
     check_linear(env, oracle, t, exl3.Plan(1), strips=True, rows_list=[1, 16, 64])
 
 
+@pytest.mark.parametrize("bits,programs,strips", [(2, 7, True), (3, 13, False), (4, 5, True), (5, 24, False), (6, 1, True), (8, 13, True)])
+def test_gemv_of_17_to_64_rows_at_its_edges(env, bits, programs, strips):
+    """Row counts at the edges of the wide kernel's row groups, runs that cross column blocks, trellis words on a multiple of
+    4 bytes only (here and in the prefill): every row has the bits of the single-row call, rows past the last are untouched."""
+    torch, exl3, kern = env
+    from ferrite_amd import synth
+    t = synth.exl3_tensor(1024, 384, bits, 40 + bits)
+    d = exl3.DeviceExl3(t, strips)
+    words = torch.zeros(d.trellis.numel() * d.trellis.element_size() // 4 + 1, dtype=torch.int32, device="cuda")
+    words[1:] = d.trellis.view(torch.int32).flatten()
+    plan = exl3.Plan(programs, 4, 4, 0)
+    aligned = exl3.Linear.with_plan(kern, d, plan)
+    lin = exl3.Linear.from_view(kern, "shifted", exl3.Exl3View(t.k, t.n, bits, words[1:].data_ptr(), d.suh.data_ptr(), d.svh.data_ptr(), strips), plan)
+    ws = exl3.Workspace([lin, aligned], 100)
+    x = dev_u16(torch, synth.activations(100, t.k, bits))
+    one = torch.zeros((64, t.n), dtype=torch.float32, device="cuda")
+    for r in range(64):
+        aligned.forward(x[r:], exl3.Dtype.Bf16, one[r:], exl3.Dtype.F32, 1, ws)
+    for rows in (17, 31, 32, 33, 40, 47, 48, 49, 63, 64):
+        y = run_forward(torch, exl3, lin, ws, x, rows, exl3.Dtype.F32)
+        assert torch.equal(y[:rows].view(torch.int32), one[:rows].view(torch.int32)), rows
+        assert rows == 64 or torch.isnan(y[rows:]).all()
+    prompt = [run_forward(torch, exl3, l, ws, x, 100, exl3.Dtype.F32) for l in (lin, aligned)]
+    assert torch.equal(prompt[0].view(torch.int32), prompt[1].view(torch.int32))
+
+
 def test_plan_for_default_and_determinism_with_shared_workspace(env, oracle):
     """crates/fe-exl3/src/bin/exl3-detcheck.rs:36-70: repeated forwards interleaved with a second linear that shares the
     workspace give identical bits."""
