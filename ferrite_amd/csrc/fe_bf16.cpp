@@ -14,8 +14,16 @@ namespace {
 // dynamic LDS by form (256 x 256, unused, 128 x 256, 128 x 128): the k tiles in flight, two or three of A and three of W
 constexpr uint32_t kGemmLds[4] = {160 * 1024, 0, 144 * 1024, 80 * 1024};
 constexpr uint32_t kGemmThreads = 512;
-constexpr uint32_t kTileM = 256, kTileN = 256;           // GM_BM, GM_BN
-constexpr uint32_t kGemvRows = 8;                        // rows of one GEMV pass (model.rs:326)
+constexpr uint32_t kTileM = 256;                         // rows of the largest output tile
+constexpr uint32_t kGemvRows = 8;                        // rows of one fe_bf16_gemv call (model.rs:326)
+constexpr uint32_t kGemvPass = 64;                       // rows of one pass over the weights
+// The GEMV's forms: rows / 8, and columns / 8 of a program (those whose stages fit LDS)
+constexpr uint32_t kGemvRowForms[5] = {1, 2, 4, 6, 8}, kGemvColForms[7] = {1, 2, 3, 4, 5, 6, 9};
+constexpr bool gemv_form(uint32_t xo, uint32_t co) { return 12 * (co + xo) <= 160; }
+// Bf16Gemv<XO, CO>::LDS of k_bf16.hip
+uint32_t gemv_lds(uint32_t xo, uint32_t co) {
+    return 4 * std::max(3u, std::min(20 / (co + xo), 8u)) * (co + xo) * 1024;
+}
 constexpr uint32_t kSmallBatch = 16;                     // X3_ROWS: batches up to here are decode rows (model.rs:172)
 }  // namespace
 
@@ -23,21 +31,39 @@ struct fe_bf16_kernels {
     fe_module_t module = nullptr;
     fe_function_t gemm[4] = {}, reduce[3] = {}, swiglu[4] = {}, swiglu_reduce[3] = {};  // by form; by tile (fe_gemm_launch)
     fe_function_t interleave = nullptr;
-    fe_function_t gemv[4][4] = {};  // [rows 1, 2, 4, 8][columns of a program 1, 2, 4, 8]
+    fe_function_t gemv[5][7] = {};  // [kGemvRowForms][kGemvColForms]
     uint32_t cus = 0;
     FeBuf part;
     // Switches, read from the environment once at load (fe_bf16_kernels_set_option changes them afterwards)
-    int32_t nc = -1;           // columns a GEMV program takes (1, 2, 4, 8); -1 = by the shape (FE_BF16_NC)
+    int32_t nc = -1;           // columns a GEMV program takes, rounded up to 8, 16, .. 48, 72; -1 = by the shape (FE_BF16_NC)
     int32_t raster_group = -1; // raster group of the GEMM; -1 = by the shape (FE_BF16_GROUP)
     uint32_t gemm_splits = 8;  // most pieces a cut output tile takes (FE_GEMM_SPLITS; 1: never cut)
     FeGemmTileOptions tile;    // "gemm_tile", "gemm_pieces"
 };
 
-// log2 of the columns a GEMV program takes. Measured on 5120 x 17408, 17408 x 5120 and 5120 x 5120: 4 columns are best
-// for 1 and 2 rows (5120 x 17408: 29 us at 1 row), 8 for 3..8 rows of a wide linear (31.7 against 33.8 us at 4 rows,
-// 42.6 against 43.8 at 8; one column: 83 us at 8 rows); narrow linears take fewer so that the grid still has a few
-// programs a CU.
-static int gemv_cols(uint32_t n, int form) { return n >= 8192 && form >= 2 ? 3 : n >= 4096 ? 2 : n >= 1024 ? 1 : 0; }
+// Which of kGemvColForms a GEMV takes. Time goes by the CU with the most columns, so the form is the one with the least of
+// rounds of one program a CU times a program's loads (columns, and half the weight for the x rows, which come from L2). us, 5120
+// columns of 17408 at 1 / 16 rows (640 octets of columns on 256 CUs): 2 octets 33.8 / 47.9, 3 octets 27.1 / 33.7, 4 octets
+// 30.0 / 39.4; 8704 columns of 5120 at 1 / 64 rows: 4 octets 20.9 / 43, 5 octets 15.2 / 27. With one or two rows a linear
+// of several octets a CU is better off with programs that start while others run: 17408 columns 27.1 us at 3 octets, 27.7 at 9.
+static uint32_t gemv_cols(uint32_t m, uint32_t n, uint32_t k, uint32_t xo, uint32_t cus, int32_t nc) {
+    const uint32_t octets = n / 8;
+    uint32_t best = 0;
+    uint64_t least = ~0ull;
+    for (uint32_t i = 0; i < 7; i++) {
+        const uint32_t co = kGemvColForms[i];
+        if (i && (!gemv_form(xo, co) || 16ull * co * k >= (1ull << 32))) break;
+        if (nc > 0) {
+            best = i;
+            if (8 * co >= (uint32_t)nc) break;
+            continue;
+        }
+        const uint64_t rounds = (octets + co * cus - 1) / (co * cus), cost = rounds * (2 * co + xo);
+        if (cost <= least) best = i, least = cost;
+    }
+    if (nc <= 0 && m <= 2 && best > 4) best = 2;
+    return best;
+}
 
 // Raster of the GEMM's output tiles (gemm_raster). Weights at least as large as the activations: column tiles are dealt
 // to the XCDs (group 0), each weight panel through one L2, the smaller activations through all of them; else row tiles
@@ -79,11 +105,14 @@ int fe_bf16_kernels_load(fe_bf16_kernels **out) {
         if (!c) c = fe_hip_module_get_function(&k->swiglu_reduce[tile], k->module, ("fe_gemm_bf16_swiglu_reduce" + s).c_str());
     }
     if (!c) c = fe_hip_module_get_function(&k->interleave, k->module, "fe_interleave_gu");
-    for (int i = 0; i < 4 && !c; i++)
-        for (int j = 0; j < 4 && !c; j++) {
+    for (uint32_t i = 0; i < 5 && !c; i++)
+        for (uint32_t j = 0; j < 7 && !c; j++) {
+            const uint32_t xo = kGemvRowForms[i], co = kGemvColForms[j];
+            if (!gemv_form(xo, co)) continue;
             char nm[32];
-            snprintf(nm, sizeof nm, "fe_gemv_bf16_r%d_c%d", 1 << i, 1 << j);
+            snprintf(nm, sizeof nm, "fe_gemv_bf16_r%u_c%u", xo, co);
             c = fe_hip_module_get_function(&k->gemv[i][j], k->module, nm);
+            if (!c) c = fe_hip_func_set_max_dyn_lds(k->gemv[i][j], gemv_lds(xo, co));
         }
     int cus = 0;
     if (!c) c = fe_hip_cu_count(&cus);
@@ -120,6 +149,20 @@ int fe_bf16_kernels_set_option(fe_bf16_kernels *k, const char *name, int32_t val
     return 0;
 }
 
+// One pass over the weights, operands checked, m in 1..kGemvPass.
+static int launch_gemv(const fe_bf16_kernels *kern, fe_stream_t s, fe_devptr_t y, uint32_t ldy, fe_devptr_t x, uint32_t lda,
+                       fe_devptr_t w, fe_devptr_t res, uint32_t m, uint32_t n, uint32_t k) {
+    if (m > 1 && (uint64_t)m * lda * 2 >= (1ull << 32)) {  // rows that lie further apart than an offset reaches
+        for (uint32_t r = 0; r < m; r++)
+            FE_TRY(launch_gemv(kern, s, y + (size_t)r * ldy * 2, ldy, x + (size_t)r * lda * 2, lda, w, res ? res + (size_t)r * ldy * 2 : 0, 1, n, k));
+        return 0;
+    }
+    const uint32_t form = m <= 8 ? 0 : (m + 15) / 16, xo = kGemvRowForms[form];
+    const uint32_t cols = gemv_cols(m, n, k, xo, std::max(kern->cus, 1u), kern->nc), co = kGemvColForms[cols];
+    void *args[] = {&y, &x, &w, &res, &m, &n, &k, &lda, &ldy};
+    return fe_hip_launch(kern->gemv[form][cols], (n / 8 + co - 1) / co, 1, 1, 256, 1, 1, gemv_lds(xo, co), s, args);
+}
+
 int fe_bf16_gemv(const fe_bf16_kernels *kern, fe_stream_t s, fe_devptr_t y, uint32_t ldy, fe_devptr_t x, uint32_t lda,
                  fe_devptr_t w, fe_devptr_t res, uint32_t m, uint32_t n, uint32_t k) {
     const char *fn = "fe_bf16_gemv";
@@ -127,13 +170,7 @@ int fe_bf16_gemv(const fe_bf16_kernels *kern, fe_stream_t s, fe_devptr_t y, uint
     if (m == 0) return 0;
     if (m > kGemvRows) return fe_set_error(FE_ERR_ARG, fn, "at most 8 rows a call");
     FE_TRY(check(fn, y, ldy, x, lda, w, res, n, k));
-    const int form = m <= 1 ? 0 : m <= 2 ? 1 : m <= 4 ? 2 : 3;
-    // columns of a program: the results do not depend on it. More columns read x less often (x is read once per program
-    // and step, the weights once in all), fewer give more programs
-    int cols = gemv_cols(n, form);
-    if (kern->nc > 0) cols = kern->nc >= 8 ? 3 : kern->nc >= 4 ? 2 : kern->nc >= 2 ? 1 : 0;
-    void *args[] = {&y, &x, &w, &res, &m, &n, &k, &lda, &ldy};
-    return fe_hip_launch(kern->gemv[form][cols], n >> cols, 1, 1, 256, 1, 1, 0, s, args);
+    return launch_gemv(kern, s, y, ldy, x, lda, w, res, m, n, k);
 }
 
 int fe_bf16_gemm(const fe_bf16_kernels *kern, fe_stream_t s, fe_devptr_t y, uint32_t ldy, fe_devptr_t x, uint32_t lda,
@@ -144,7 +181,7 @@ int fe_bf16_gemm(const fe_bf16_kernels *kern, fe_stream_t s, fe_devptr_t y, uint
     FE_TRY(check(fn, y, ldy, x, lda, w, res, n, k));
     if ((uint64_t)m * lda * 2 >= (1ull << 32) || (uint64_t)n * k * 2 >= (1ull << 32))
         return fe_set_error(FE_ERR_UNSUPPORTED, fn, "operand of 4 GB or more");
-    const uint32_t tiles_m = (m + kTileM - 1) / kTileM, tiles_n = (n + kTileN - 1) / kTileN;
+    const uint32_t tiles_m = (m + kTileM - 1) / kTileM;
     uint32_t group = bf16_raster_group(m, n, k, tiles_m);
     if (kern->raster_group >= 0) group = (uint32_t)kern->raster_group;
     if (group > tiles_m) group = tiles_m;
@@ -183,7 +220,7 @@ int fe_bf16_gemm_swiglu(const fe_bf16_kernels *kern, fe_stream_t s, fe_devptr_t 
     if (n % 16) return fe_set_error(FE_ERR_SHAPE, fn, "inter % 8 == 0");
     if ((uint64_t)m * lda * 2 >= (1ull << 32) || (uint64_t)n * k * 2 >= (1ull << 32))
         return fe_set_error(FE_ERR_UNSUPPORTED, fn, "operand of 4 GB or more");
-    const uint32_t tiles_m = (m + kTileM - 1) / kTileM, tiles_n = (n + kTileN - 1) / kTileN;
+    const uint32_t tiles_m = (m + kTileM - 1) / kTileM;
     uint32_t group = bf16_raster_group(m, n, k, tiles_m);
     if (kern->raster_group >= 0) group = (uint32_t)kern->raster_group;
     if (group > tiles_m) group = tiles_m;
@@ -208,12 +245,12 @@ int fe_bf16_linear_forward(const fe_bf16_kernels *kern, fe_stream_t s, fe_devptr
     if (!kern) return fe_set_error(FE_ERR_ARG, fn, "null kernels");
     if (m == 0) return 0;
     FE_TRY(check(fn, y, ldy, x, lda, w, res, n, k));
-    // decode / verify rows: the GEMV in passes of up to 8 rows, so that a row's bits do not depend on the batch
+    // decode / verify rows: the GEMV, so that a row's bits do not depend on the batch
     uint32_t d = m <= kSmallBatch ? m : (dec < m ? dec : m);
     if (k % 256) d = 0;
-    for (uint32_t r = 0; r < d; r += kGemvRows) {
-        const uint32_t mr = d - r < kGemvRows ? d - r : kGemvRows;
-        FE_TRY(fe_bf16_gemv(kern, s, y + (size_t)r * ldy * 2, ldy, x + (size_t)r * lda * 2, lda, w,
+    for (uint32_t r = 0; r < d; r += kGemvPass) {
+        const uint32_t mr = d - r < kGemvPass ? d - r : kGemvPass;
+        FE_TRY(launch_gemv(kern, s, y + (size_t)r * ldy * 2, ldy, x + (size_t)r * lda * 2, lda, w,
                             res ? res + (size_t)r * ldy * 2 : 0, mr, n, k));
     }
     if (d == m) return 0;

@@ -39,6 +39,11 @@ __device__ __forceinline__ void g8_load_lds16(u32x4 rs, uint32_t dst, uint32_t v
                  "s"(__builtin_amdgcn_readfirstlane(soff))
                  : "memory");
 }
+__device__ __forceinline__ void g8_load_lds16_nt(u32x4 rs, uint32_t dst, uint32_t voff, uint32_t soff) {
+    asm volatile("s_mov_b32 m0, %0\n\ts_nop 0\n\tbuffer_load_dwordx4 %1, %2, %3 offen nt lds" ::"s"(__builtin_amdgcn_readfirstlane(dst)), "v"(voff), "s"(rs),
+                 "s"(__builtin_amdgcn_readfirstlane(soff))
+                 : "memory");
+}
 __device__ __forceinline__ void g8_load_lds4(u32x4 rs, uint32_t dst, uint32_t voff, uint32_t soff) {
     asm volatile("s_mov_b32 m0, %0\n\ts_nop 0\n\tbuffer_load_dword %1, %2, %3 offen lds" ::"s"(__builtin_amdgcn_readfirstlane(dst)), "v"(voff), "s"(rs),
                  "s"(__builtin_amdgcn_readfirstlane(soff))

@@ -1,5 +1,7 @@
 // The plain bf16 weight form of the caller's linear: y[M][N] = x[M][K] . W[N][K]^T (+ residual), W row-major bf16, f32
-// sums, bf16 out. A GEMM on the shared 256 x 256 MFMA tile loop and two decode-sized GEMVs (kernels/k-core/src/gemm.rs).
+// sums, bf16 out. A GEMM on the shared MFMA tile loop and a decode-sized GEMV (kernels/k-core/src/gemm.rs).
+#include <type_traits>
+
 #include "gemm8.h"
 
 // 4 sums of columns at.. of one row -> bf16; with res: bf16(bf16(sum) + res) (gemm.rs:152-158).
@@ -118,103 +120,142 @@ extern "C" __global__ __launch_bounds__(256) void fe_interleave_gu(uint16_t* dst
     for (uint32_t j = threadIdx.x; j < k / 8; j += 256) *((u32x4*)d + j) = *((const u32x4*)src + j);
 }
 
-// ---- GEMV (1..8 rows) ------------------------------------------------------------------------------------------------
+// ---- GEMV (1..64 rows) -----------------------------------------------------------------------------------------------
 
-__device__ __forceinline__ float dot8_bf16(u32x4 w, u32x4 x, float acc) {
-#pragma unroll
-    for (int p = 0; p < 4; p++) {
-        // the elements are copied out first: __builtin_bit_cast applied to a vector element reads element 0
-        const uint32_t wp = w[p], xp = x[p];
-        acc = __builtin_amdgcn_fdot2_f32_bf16(__builtin_bit_cast(bf16x2, wp), __builtin_bit_cast(bf16x2, xp), acc, false);
-    }
-    return acc;
-}
+// y[r][n] = bf16(x[r][:] . W[n][:]) (+ res) for r < m <= 8 XO. grid ceil(N / 8 CO), 256 threads: a program takes 8 CO columns over
+// all of K, its four wavefronts a quarter of K's steps of 64 each; a wavefront adds its products in v_mfma_f32_16x16x32_bf16 in
+// ascending k, the four sums are added in order. So a row's bits depend on K only, neither on the other rows nor on XO or
+// CO: the host picks them by the row count and the shape, where the reference picks between two kernels by the shape.
+// K % 64 == 0, N % 8 == 0, lda % 8 == 0. (kernels/k-core/src/gemm.rs:172-262: fe_gemv_bf16 and fe_gemv_bf16_kw)
+//
+// Bound by the weights' way from HBM, every row count up to 64 reading them once: the sums of dot products that this replaces
+// ran out of registers at 8 rows and took another pass over the weights for every 8. Weights and x rows go straight into LDS,
+// DEPTH - 1 steps ahead, 8 rows x 128 bytes a load into stages that belong to one wavefront (no barrier in the loop): whole cache
+// lines, which fragments loaded straight into registers (16 rows x 64 bytes) are not, at 42 us instead of 28. The weight loads
+// are non-temporal (31.5 -> 28.3 us at 1 row). x comes from L2 once a program, so wide programs (CO) matter with the rows.
+// 5120 x 17408, us, before -> now: 1 row 26.6 -> 27.1, 4 rows 29.6 -> 27.8, 8 rows 40.6 -> 28.1, 16 rows 80.8 -> 29.2, 40 rows
+// 202 -> 43, 64 rows 321 -> 52 (one or two rows on a few widths 2 to 5 % slower: 5120 x 5120 9.4 -> 9.8); 17408 x 5120: 27.3 -> 27.1, 32.3 -> 27.8, 41.7 -> 29.3, 83.3 -> 33.7, 209 -> 48, 334 -> 57.
+// Distance of the bf16 results from 64-bit sums: 1.66e-3 of their norm, the same to seven digits before and now.
+template <int XO, int CO>
+struct Bf16Gemv {
+    static constexpr int L = CO + XO, STAGE = L * 1024;  // loads of a step
+    // steps in LDS: 80 KB a program, so that two share a CU, but three at least (half or twice the room: the same within 1 %)
+    static constexpr int FIT = 20 * 1024 / STAGE, DEPTH = FIT < 3 ? 3 : FIT < 8 ? FIT : 8;
+    static constexpr int LDS = 4 * DEPTH * STAGE;
+    static_assert((DEPTH - 1) * L < 64 && LDS <= 160 * 1024, "stages");
+};
 
-// Sum over each row of 16 lanes, left in all 16 (four DPP adds: no LDS traffic, unlike a butterfly of ds_bpermute).
-__device__ __forceinline__ float row16_sum(float v) {
-    v += dpp_mov<DPP_QUAD_XOR1>(v);
-    v += dpp_mov<DPP_QUAD_XOR2>(v);
-    v += dpp_mov<DPP_HALF_MIRROR>(v);
-    v += dpp_mov<DPP_ROW_MIRROR>(v);
-    return v;
-}
-
-// One wavefront: the sums of x rows 0..MR-1 (rows >= m repeat row m - 1) with NC weight rows over the 16-byte chunks
-// [c0, c1) of K, lane L taking chunks c0 + L, c0 + L + 64, ... in ascending order, one v_dot2 per element pair; then
-// every 16 lanes add up (the sum of lanes 16 q .. 16 q + 15 is left in all of them).
-template <int MR, int NC>
-__device__ __forceinline__ void gemv_bf16_sums(const uint16_t* a, const uint16_t* const (&wr)[NC], uint32_t m, uint32_t lda,
-                                               uint32_t c0, uint32_t c1, float (&acc)[MR][NC]) {
-    const uint32_t lane = threadIdx.x & 63;
-    const uint16_t* xr[MR];
-#pragma unroll
-    for (int r = 0; r < MR; r++) {
-        xr[r] = a + (size_t)((uint32_t)r < m ? r : m - 1) * lda;
-#pragma unroll
-        for (int j = 0; j < NC; j++) acc[r][j] = 0.f;
-    }
-#pragma unroll 2
-    for (uint32_t i = c0 + lane; i < c1; i += 64) {
-        u32x4 wv[NC], xv[MR];
-#pragma unroll
-        for (int j = 0; j < NC; j++) wv[j] = __builtin_nontemporal_load((const u32x4*)wr[j] + i);
-#pragma unroll
-        for (int r = 0; r < MR; r++) xv[r] = *((const u32x4*)xr[r] + i);
-#pragma unroll
-        for (int r = 0; r < MR; r++)
-#pragma unroll
-            for (int j = 0; j < NC; j++) acc[r][j] = dot8_bf16(wv[j], xv[r], acc[r][j]);
-    }
-#pragma unroll
-    for (int r = 0; r < MR; r++)
-#pragma unroll
-        for (int j = 0; j < NC; j++) acc[r][j] = row16_sum(acc[r][j]);
-}
-
-// y[r][n] = bf16(x[r][:] . W[n][:]) (+ res) for r < m <= MR. grid N / NC, 256 threads: a program takes NC consecutive
-// columns; K is walked in steps of 64 chunks of 16 bytes (a 1 KB run of every weight row a step), wavefront w takes
-// steps [w S / 4, (w + 1) S / 4) of the S steps, and the sixteen sums (4 wavefronts x 4 rows of 16 lanes) are added in order. So a row's bits depend
-// on K only, neither on the other rows nor on NC: the host picks NC by the shape and the row count (more columns a program
-// read x less often, fewer columns give more programs), where the reference picks between two kernels by the shape.
-// K % 8 == 0, N % NC == 0, lda % 8 == 0. (kernels/k-core/src/gemm.rs:172-262: fe_gemv_bf16 and fe_gemv_bf16_kw)
-template <int MR, int NC>
+template <int XO, int CO>
 __device__ __forceinline__ void gemv_bf16_body(uint16_t* c, const uint16_t* a, const uint16_t* w, const uint16_t* res,
                                                uint32_t m, uint32_t n, uint32_t k, uint32_t lda, uint32_t ldc) {
-    __shared__ float red[16][MR][NC];
-    const uint32_t lane = threadIdx.x & 63, wave = threadIdx.x >> 6, col = blockIdx.x * NC;
-    const uint16_t* wr[NC];
+    typedef Bf16Gemv<XO, CO> C;
+    constexpr int RG = (XO + 1) / 2, CG = (CO + 1) / 2, AHEAD = C::DEPTH - 1, PITCH = 16 * CG + 4;
+    extern __shared__ __attribute__((aligned(1024))) unsigned char lds[];
+    const uint32_t tid = threadIdx.x, lane = tid & 63, wave = __builtin_amdgcn_readfirstlane(tid >> 6), r = lane & 15, g = lane >> 4;
+    const uint32_t col0 = blockIdx.x * 8 * CO, cols = n - col0 < 8 * CO ? n - col0 : 8 * CO;
+    const u32x4 wrs = g8_rsrc(w + (size_t)col0 * k, cols * k * 2), xrs = g8_rsrc(a, ((m - 1) * lda + k) * 2);
+    // a row's 16-byte chunk c of a step lies at position c ^ (row & 7); rows that do not exist repeat the last one
+    const uint32_t lr = lane >> 3, lc = ((lane & 7) ^ lr) << 4;
+    uint32_t vw[CO], vx[XO];
 #pragma unroll
-    for (int j = 0; j < NC; j++) wr[j] = w + (size_t)(col + j) * k;
-    const uint32_t chunks = k / 8, steps = (chunks + 63) / 64;
-    const uint32_t c0 = (wave * steps / 4) * 64, c1 = ((wave + 1) * steps / 4) * 64;
-    float acc[MR][NC];
-    gemv_bf16_sums<MR, NC>(a, wr, m, lda, c0, c1 < chunks ? c1 : chunks, acc);
-    if ((lane & 15) == 0) {
+    for (int j = 0; j < CO; j++) vw[j] = (8 * j + lr < cols ? 8 * j + lr : cols - 1) * k * 2 + lc;
 #pragma unroll
-        for (int r = 0; r < MR; r++)
+    for (int j = 0; j < XO; j++) vx[j] = (8 * j + lr < m ? 8 * j + lr : m - 1) * lda * 2 + lc;
+    unsigned char* stages = lds + wave * (C::DEPTH * C::STAGE);
+    const uint32_t stages0 = g8_lds_addr(stages);
+    const uint32_t steps = k / 64, s0 = wave * steps / 4, count = (wave + 1) * steps / 4 - s0;
+    auto issue = [&](uint32_t s, uint32_t slot) {
+        const uint32_t at = stages0 + slot * C::STAGE, off = (s0 + s) * 128;
 #pragma unroll
-            for (int j = 0; j < NC; j++) red[threadIdx.x >> 4][r][j] = acc[r][j];
+        for (int j = 0; j < CO; j++) g8_load_lds16_nt(wrs, at + j * 1024, vw[j], off);
+#pragma unroll
+        for (int j = 0; j < XO; j++) g8_load_lds16(xrs, at + (CO + j) * 1024, vx[j], off);
+    };
+    // where the lane's fragments lie in a stage (columns past the program's: the last one again, not stored)
+    uint32_t fw[CG][2], fx[RG][2];
+    auto frag = [&](uint32_t row, int h) { return row * 128 + (((4 * h + g) ^ (row & 7)) << 4); };
+#pragma unroll
+    for (int h = 0; h < 2; h++) {
+#pragma unroll
+        for (int j = 0; j < CG; j++) fw[j][h] = frag(16 * j + r < 8 * CO ? 16 * j + r : 8 * CO - 1, h);
+#pragma unroll
+        for (int i = 0; i < RG; i++) fx[i][h] = CO * 1024 + frag(16 * i + r < m ? 16 * i + r : m - 1, h);
     }
-    __syncthreads();
-    const uint32_t r = threadIdx.x / NC, j = threadIdx.x % NC;
-    if (r < m) {
-        float y = red[0][r][j];
-        for (int q = 1; q < 16; q++) y += red[q][r][j];
-        const size_t at = (size_t)r * ldc + col + j;
-        if (res) y = bf16_bits_to_f32(f32_to_bf16_bits(y)) + bf16_bits_to_f32(res[at]);
-        c[at] = (uint16_t)f32_to_bf16_bits(y);
+    f32x4 acc[RG][CG] = {};
+    uint32_t slot = 0;
+    auto add = [&]() {
+        const unsigned char* st = stages + slot * C::STAGE;
+#pragma unroll
+        for (int h = 0; h < 2; h++) {
+            bf16x8 wv[CG];
+#pragma unroll
+            for (int j = 0; j < CG; j++) wv[j] = *(const bf16x8*)(st + fw[j][h]);
+#pragma unroll
+            for (int i = 0; i < RG; i++) {
+                const bf16x8 xv = *(const bf16x8*)(st + fx[i][h]);
+#pragma unroll
+                for (int j = 0; j < CG; j++) acc[i][j] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(wv[j], xv, acc[i][j], 0, 0, 0);
+            }
+        }
+        slot = slot + 1 == C::DEPTH ? 0 : slot + 1;
+    };
+    if (count) {
+#pragma unroll
+        for (int u = 0; u < AHEAD; u++) issue((uint32_t)u < count ? u : count - 1, u);  // past the end: the last step again, not added
+        uint32_t s = 0;
+        for (; s + AHEAD < count; s++) {
+            g8_loads_wait<(AHEAD - 1) * C::L>();  // (the stage in front of this one has been read, too)
+            issue(s + AHEAD, slot ? slot - 1 : AHEAD);
+            add();
+        }
+        auto tail = [&](auto u_tag) {
+            constexpr int U = decltype(u_tag)::value;
+            if (s + U < count) {
+                g8_loads_wait<(AHEAD - 1 - U) * C::L>();
+                add();
+            }
+        };
+        tail(std::integral_constant<int, 0>{});
+        if constexpr (AHEAD > 1) tail(std::integral_constant<int, 1>{});
+        if constexpr (AHEAD > 2) tail(std::integral_constant<int, 2>{});
+        if constexpr (AHEAD > 3) tail(std::integral_constant<int, 3>{});
+        if constexpr (AHEAD > 4) tail(std::integral_constant<int, 4>{});
+        if constexpr (AHEAD > 5) tail(std::integral_constant<int, 5>{});
+        if constexpr (AHEAD > 6) tail(std::integral_constant<int, 6>{});
+        g8_loads_wait<0>();
+    }
+    float(*red)[16][PITCH] = (float(*)[16][PITCH])lds;
+#pragma unroll
+    for (int i = 0; i < RG; i++) {
+        __syncthreads();
+#pragma unroll
+        for (int j = 0; j < CG; j++) *(f32x4*)&red[wave][r][16 * j + 4 * g] = acc[i][j];
+        __syncthreads();
+#pragma unroll
+        for (int e = 0; e < CG; e++) {
+            const uint32_t row = (tid + 256 * e) / (8 * CO), j = (tid + 256 * e) % (8 * CO);
+            if (row < 16 && 16 * i + row < m && j < cols) {
+                float y = ((red[0][row][j] + red[1][row][j]) + red[2][row][j]) + red[3][row][j];
+                const size_t at = (size_t)(16 * i + row) * ldc + col0 + j;
+                if (res) y = bf16_bits_to_f32(f32_to_bf16_bits(y)) + bf16_bits_to_f32(res[at]);
+                c[at] = (uint16_t)f32_to_bf16_bits(y);
+            }
+        }
     }
 }
 
-#define BF16_GEMV_KERNEL(MR, NC)                                                                                           \
-    extern "C" __global__ __launch_bounds__(256) void fe_gemv_bf16_r##MR##_c##NC(uint16_t* c, const uint16_t* a,           \
-                                                                                 const uint16_t* w, const uint16_t* res,  \
-                                                                                 uint32_t m, uint32_t n, uint32_t k,      \
-                                                                                 uint32_t lda, uint32_t ldc) {            \
-        gemv_bf16_body<MR, NC>(c, a, w, res, m, n, k, lda, ldc);                                                           \
+#define BF16_GEMV_KERNEL(XO, CO)                                                                                             \
+    extern "C" __global__ __launch_bounds__(256) void fe_gemv_bf16_r##XO##_c##CO(                                            \
+        uint16_t* c, const uint16_t* a, const uint16_t* w, const uint16_t* res, uint32_t m, uint32_t n, uint32_t k, uint32_t lda, \
+        uint32_t ldc) {                                                                                                    \
+        gemv_bf16_body<XO, CO>(c, a, w, res, m, n, k, lda, ldc);                                                           \
     }
-#define BF16_GEMV_ROWS(MR) BF16_GEMV_KERNEL(MR, 1) BF16_GEMV_KERNEL(MR, 2) BF16_GEMV_KERNEL(MR, 4) BF16_GEMV_KERNEL(MR, 8)
+#define BF16_GEMV_ROWS(XO)                                                                                                  \
+    BF16_GEMV_KERNEL(XO, 1) BF16_GEMV_KERNEL(XO, 2) BF16_GEMV_KERNEL(XO, 3) BF16_GEMV_KERNEL(XO, 4) BF16_GEMV_KERNEL(XO, 5)
 BF16_GEMV_ROWS(1)
 BF16_GEMV_ROWS(2)
 BF16_GEMV_ROWS(4)
+BF16_GEMV_ROWS(6)
 BF16_GEMV_ROWS(8)
+BF16_GEMV_KERNEL(1, 6) BF16_GEMV_KERNEL(2, 6) BF16_GEMV_KERNEL(4, 6) BF16_GEMV_KERNEL(6, 6)
+BF16_GEMV_KERNEL(1, 9) BF16_GEMV_KERNEL(2, 9) BF16_GEMV_KERNEL(4, 9)

@@ -23,13 +23,13 @@ extern "C" {
 typedef struct fe_bf16_kernels fe_bf16_kernels;
 int fe_bf16_kernels_load(fe_bf16_kernels **out);
 int fe_bf16_kernels_destroy(fe_bf16_kernels *k);
-/* Switches by name: "nc" columns a GEMV program takes (FE_BF16_NC; -1 = by the shape), "raster_group" (FE_BF16_GROUP;
+/* Switches by name: "nc" columns a GEMV program takes (rounded up to 8, 16, .. 48, 72; FE_BF16_NC; -1 = by the shape), "raster_group" (FE_BF16_GROUP;
  * -1 = by the shape), "gemm_splits" (FE_GEMM_SPLITS); "gemm_tile" 0..3 (output tile of the GEMMs: by the shape,
  * 256 x 256, 128 x 256, 128 x 128) and "gemm_pieces" (pieces of K a forced small tile takes), both for tests. Read from the environment once, at load; no call reads it later. */
 int fe_bf16_kernels_set_option(fe_bf16_kernels *k, const char *name, int32_t value);
 
-/* fe_gemv_bf16 / fe_gemv_bf16_kw (gemm.rs:172-262): m <= 8 rows. One kernel family here: a program takes 1, 2, 4
- * or 8 columns by the width of the linear and the row count (model.rs:316-322 picks between the two kernels by the shape), and a row's bits
+/* fe_gemv_bf16 / fe_gemv_bf16_kw (gemm.rs:172-262): m <= 8 rows (fe_bf16_linear_forward takes up to 64 through
+ * the same kernels). One kernel family here: a program takes 8 to 72 columns by the width of the linear and the row count (model.rs:316-322 picks between the two kernels by the shape), and a row's bits
  * depend neither on that nor on m. res (stride ldy) may be 0; with it y = bf16(bf16(x . W) + res), res may be y. */
 int fe_bf16_gemv(const fe_bf16_kernels *kern, fe_stream_t s, fe_devptr_t y, uint32_t ldy, fe_devptr_t x, uint32_t lda,
                  fe_devptr_t w, fe_devptr_t res, uint32_t m, uint32_t n, uint32_t k);
@@ -45,7 +45,7 @@ int fe_bf16_interleave_gu(const fe_bf16_kernels *kern, fe_stream_t s, fe_devptr_
 int fe_bf16_gemm_swiglu(const fe_bf16_kernels *kern, fe_stream_t s, fe_devptr_t act, fe_devptr_t x, uint32_t lda,
                         fe_devptr_t w, uint32_t m, uint32_t inter, uint32_t k);
 /* The bf16 branch of Linear::forward (model.rs:310-345): all rows of a batch of <= 16, else the leading `dec` rows, go
- * through the GEMV in passes of 8 rows (when k % 256 == 0); the rows after them through the GEMM. */
+ * through the GEMV in passes of up to 64 rows (when k % 256 == 0); the rows after them through the GEMM. */
 int fe_bf16_linear_forward(const fe_bf16_kernels *kern, fe_stream_t s, fe_devptr_t y, uint32_t ldy, fe_devptr_t x,
                            uint32_t lda, fe_devptr_t w, fe_devptr_t res, uint32_t m, uint32_t n, uint32_t k, uint32_t dec);
 

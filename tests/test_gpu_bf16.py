@@ -89,6 +89,29 @@ def test_gemv(env, oracle, n, k, m):
     assert np.array_equal(with_res, bits(f32(got) + f32(rb[:m])))
 
 
+@pytest.mark.parametrize("n,k,lda", [(8, 64, 64), (72, 192, 200), (136, 256, 256), (264, 832, 832), (2568, 512, 520)])
+def test_rows_of_any_batch_have_the_bits_of_one_row(env, oracle, n, k, lda):
+    """Every row count at an edge of the GEMV's forms and every width of a program: the single row's bits, within the
+    oracle's bound, nothing written past the rows and columns."""
+    torch, bf16, kern = env
+    xb, wb = operands(n, k, 64, 31 + n, lda=lda)
+    x, w = dev_u16(torch, xb), dev_u16(torch, wb)
+    one = np.concatenate([call(torch, bf16.gemv, kern, x[r:r + 1].contiguous(), w, 1, n, lda=lda) for r in range(64)])
+    close(one, oracle.bf16_linear_ref(xb[:, :k], wb)[1])
+    if k % 256:  # only the GEMV's own call (up to 8 rows) takes such a K to the GEMV
+        rows_list, fn = (2, 7, 8), bf16.gemv
+    else:
+        rows_list, fn = (2, 8, 9, 16, 17, 32, 33, 48, 49, 64), lambda *a, **kw: bf16.forward(*a, dec=64, **kw)
+    try:
+        for nc in (-1, 8, 16, 24, 32, 40, 48, 72):
+            kern.set_option("nc", nc)
+            for rows in rows_list:
+                got = call(torch, fn, kern, x, w, rows, n, ldy=n + 12, lda=lda)
+                assert np.array_equal(got, one[:rows]), (nc, rows)
+    finally:
+        kern.set_option("nc", -1)
+
+
 @pytest.mark.parametrize("n,k,m,lda", [(256, 512, 200, 512), (520, 768, 300, 776), (1024, 1024, 700, 1024), (96, 256, 33, 256),
                                        (768, 2048, 1, 2048)])
 def test_gemm_whole_and_cut(env, oracle, n, k, m, lda):
