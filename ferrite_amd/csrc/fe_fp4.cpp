@@ -17,6 +17,13 @@ constexpr uint32_t kTile = 128;                 // crates/fe-fp4/src/lib.rs:28
 // dynamic LDS by form (256 x 256, its stream-K form, 128 x 256, 128 x 128): the k tiles in flight. Packed weights: three of A (128
 // bytes a row) and three of W (36 bytes; 64 in the fp16 form of FP8). FP8 codes: two or three of A, three of W, 128 bytes a row.
 constexpr uint32_t kGemmLds[4] = {144 * 1024, 144 * 1024, 136 * 1024, 68 * 1024}, kGemmLds8[4] = {160 * 1024, 160 * 1024, 144 * 1024, 80 * 1024};
+// Forms of the GEMV over programs of 8 CO columns: rows / 2 and CO
+constexpr uint32_t kWideRowForms[4] = {1, 2, 4, 8}, kWideColForms[7] = {1, 2, 3, 4, 5, 6, 9};
+// Fp4Wide<XP, CO>::LDS of k_fp4.hip
+uint32_t wide_lds(uint32_t xp, uint32_t co) {
+    const uint32_t cg = (co + 1) / 2, stage = (co + xp) * 1024 + cg * 256;
+    return std::max(4 * std::max(2u, std::min(20 * 1024 / stage, 6u)) * stage, 256 * (16 * cg + 4));
+}
 constexpr uint32_t kGemmThreads = 512;
 constexpr uint32_t kTileM = 256;                        // GM_BM
 }  // namespace
@@ -26,8 +33,7 @@ struct fe_fp4_kernels {
     fe_function_t quant4 = nullptr, gemv4[3] = {nullptr, nullptr, nullptr};
     // by form (256 x 256, stream-K, 128 x 256, 128 x 128) and by tile (fe_gemm_launch); gemm8: the fp16 form, 256 x 256 only
     fe_function_t gemm4[4] = {}, swiglu4[4] = {}, gemm8c[4] = {}, gemm8[2] = {}, reduce4[3] = {}, swiglu_reduce4[3] = {}, reduce8c[3] = {};
-    fe_function_t strip4 = nullptr;  // the GEMV over strips of 16 weight rows, up to 16 activation rows (no hand-off)
-    fe_function_t strip_once[5] = {};  // ... with every load of a workgroup issued before anything waits: 1..5 groups of K a wavefront
+    fe_function_t wide[4][7] = {};   // the GEMV over programs of 8 CO columns, [kWideRowForms][kWideColForms]
     fe_function_t quant8 = nullptr;
     uint32_t cus = 0;
     // Switches of the launch paths: read from the environment once, at load; fe_fp4_kernels_set_option changes them
@@ -35,9 +41,8 @@ struct fe_fp4_kernels {
     uint32_t group_m = 8;      // raster group height in row tiles; 0 = all (FE_FP4_GROUP, lib.rs:31-32, 68)
     uint32_t gemv = 1;         // up to 64 rows run the GEMV (FE_FP4_NO_GEMV=1: the GEMM's single tile row)
     uint32_t gemv_sk = 0;      // K splits of the GEMV over weight tiles; 0 = two programs a CU (FE_FP4_GEMV_SK)
-    uint32_t gemv_strips = 1;  // the GEMV runs over strips of 16 weight rows, K split inside the workgroup (FE_FP4_NO_STRIPS=1: over weight tiles and K splits)
-    uint32_t gemv_once = 1;    // strips whose loads all go out at once, where a wavefront's share of K allows (FE_FP4_NO_ONCE=1: never)
-    uint32_t gemv_waves = 0;   // wavefronts of a strip's workgroup: 4, 8 or 16; 0 = four or more wavefronts a SIMD (FE_FP4_GEMV_WAVES)
+    uint32_t gemv_strips = 1;  // up to 16 rows run programs of some columns over all of K; 0: weight tiles and K splits, as more rows do (FE_FP4_NO_STRIPS=1)
+    uint32_t gemv_cols = 0;    // columns a program of the GEMV for up to 16 rows takes, rounded up to 8, 16, .. 48, 72; 0 = by the shape (FE_FP4_GEMV_COLS)
     int32_t xcd = -1;          // column tiles dealt to the XCDs: -1 = where the weights are the larger operand (FE_FP4_XCD)
     uint32_t fp8_f16 = 0;      // FP8 linears as fp16 expansion on the 16-bit matrix instruction (FE_FP8_F16=1)
     uint32_t gemm_splits = 8;  // most pieces a cut output tile takes (FE_GEMM_SPLITS; 1: never cut)
@@ -91,13 +96,10 @@ int fe_fp4_kernels_load(fe_fp4_kernels **out) {
         snprintf(nm, sizeof nm, "fe_gemv_nvfp4_x%d", xr);
         c = fe_hip_module_get_function(&k->gemv4[xr - 1], k->module, nm);
     }
-    if (!c) c = fe_hip_module_get_function(&k->strip4, k->module, "fe_gemv_nvfp4_strips");
-    if (!c) c = fe_hip_func_set_max_dyn_lds(k->strip4, 48 * 1024);
-    for (int g = 1; g <= 5 && !c; g++) {
-        const std::string nm = "fe_gemv_nvfp4_strips_once_g" + std::to_string(g);
-        c = fe_hip_module_get_function(&k->strip_once[g - 1], k->module, nm.c_str());
-        if (!c) c = fe_hip_func_set_max_dyn_lds(k->strip_once[g - 1], 48 * 1024);
-    }
+    for (uint32_t i = 0; i < 4; i++)
+        for (uint32_t j = 0; j < 7; j++)
+            get(&k->wide[i][j], "fe_gemv_nvfp4_r" + std::to_string(kWideRowForms[i]) + "_c" + std::to_string(kWideColForms[j]),
+                wide_lds(kWideRowForms[i], kWideColForms[j]));
     if (!c) c = fe_hip_module_get_function(&k->quant8, k->module, "fe_fp8_quant");
     int cus = 0;
     if (!c) c = fe_hip_cu_count(&cus);
@@ -106,8 +108,7 @@ int fe_fp4_kernels_load(fe_fp4_kernels **out) {
     if (const char *e = getenv("FE_FP4_NO_GEMV")) k->gemv = atoi(e) ? 0 : 1;
     if (const char *e = getenv("FE_FP4_GEMV_SK")) k->gemv_sk = (uint32_t)atoi(e);
     if (const char *e = getenv("FE_FP4_NO_STRIPS")) k->gemv_strips = atoi(e) ? 0 : 1;
-    if (const char *e = getenv("FE_FP4_NO_ONCE")) k->gemv_once = atoi(e) ? 0 : 1;
-    if (const char *e = getenv("FE_FP4_GEMV_WAVES")) k->gemv_waves = (uint32_t)atoi(e);
+    if (const char *e = getenv("FE_FP4_GEMV_COLS")) k->gemv_cols = (uint32_t)atoi(e);
     if (const char *e = getenv("FE_FP4_XCD")) k->xcd = atoi(e) ? 1 : 0;
     if (const char *e = getenv("FE_FP8_F16")) k->fp8_f16 = atoi(e) ? 1 : 0;
     if (const char *e = getenv("FE_GEMM_SPLITS")) k->gemm_splits = (uint32_t)atoi(e);
@@ -133,9 +134,9 @@ int fe_fp4_kernels_set_option(fe_fp4_kernels *k, const char *name, int32_t value
     if (nm == "group_m") k->group_m = (uint32_t)value;
     else if (nm == "gemv") k->gemv = value ? 1 : 0;
     else if (nm == "gemv_sk") k->gemv_sk = (uint32_t)value;
+    else if (nm == "gemv_cols") k->gemv_cols = value;
     else if (nm == "gemv_strips") k->gemv_strips = (uint32_t)value;
-    else if (nm == "gemv_once") k->gemv_once = (uint32_t)value;
-    else if (nm == "gemv_waves") k->gemv_waves = (uint32_t)value;
+    else if (nm == "gemv_once" || nm == "gemv_waves") (void)value;  // of a kernel that is no more: accepted, without effect
     else if (nm == "xcd") k->xcd = value;
     else if (nm == "fp8_f16") k->fp8_f16 = value ? 1 : 0;
     else if (nm == "gemm_splits") k->gemm_splits = (uint32_t)value;
@@ -335,6 +336,30 @@ int fe_fp4_linear_quantize(const fe_fp4_linear *l, const fe_fp4_kernels *kern, f
     return fe_hip_launch(kern->quant4, (blocks16 + 255) / 256, 1, 1, 256, 1, 1, 0, s, args);
 }
 
+// Which of kWideColForms a GEMV takes: the least of the loads of the CU with the most programs (a program's codes and activations;
+// a quarter more where a CU holds one at a time and has several) and the starts of its rounds of programs. us at 1 row: 34816 columns
+// of 5120 at 1, 2, .. 6 octets a program 36.9, 24.7, 24.7, 22.1, 23.3, 21.7; 17408 columns 21.8, 15.5, 15.1, 15.4, 13.7, 14.0; 5120 columns
+// of 17408 21.0, 17.6, 14.3, 15.7, 18.9, 19.3. Programs of 72 columns pay where the activations weigh most: 34816 columns at 16 rows
+// 28.8 us against 29.8 at 48 columns; at 1 row 25.6.
+static uint32_t wide_cols(uint32_t n, uint32_t xp, uint32_t cus, uint32_t forced) {
+    uint32_t best = 0;
+    uint64_t least = ~0ull;
+    for (uint32_t i = 0; i < 7; i++) {
+        const uint32_t co = kWideColForms[i], programs = (n / 8 + co - 1) / co, room = wide_lds(xp, co) <= 80 * 1024 ? 2 : 1;
+        if (forced) {
+            best = i;
+            if (8 * co >= forced) break;
+            continue;
+        }
+        if (co == 9 && xp < 8) break;
+        uint64_t cost = 4ull * ((programs + cus - 1) / cus) * (4 * co + xp);
+        if (room == 1 && programs > cus) cost += cost / 4;
+        cost += 32ull * ((programs + room * cus - 1) / (room * cus));
+        if (cost <= least) best = i, least = cost;
+    }
+    return best;
+}
+
 int fe_fp4_linear_gemm(const fe_fp4_linear *l, const fe_fp4_kernels *kern, fe_stream_t s, const fe_fp4_workspace *ws,
                        fe_devptr_t y, uint32_t ldy, uint32_t m, fe_devptr_t res) {
     if (!l || !kern || !ws) return fe_set_error(FE_ERR_ARG, "fe_fp4_linear_gemm", "null argument");
@@ -348,44 +373,14 @@ int fe_fp4_linear_gemm(const fe_fp4_linear *l, const fe_fp4_kernels *kern, fe_st
         // decode-sized: the weight-read-bound GEMV, up to 48 rows a pass. Two programs fit a CU: as many programs as run
         // at once, not more (a second round of short programs costs more than idle CUs in the first).
         const uint32_t nts = n / kTile, kts = k / 64;
-        // Strips of 16 weight rows over all of K, one a workgroup, the activations staged in LDS: no hand-off between
-        // programs. Every program stages all m rows of activations, so it pays where that is small beside the weights:
-        // one or two rows, or up to four on narrow linears (measured, cold weights: 5120 x 17408 at 1 row 14.3 against 15.4 us for
-        // the weight tiles with K splits, 5120 x 5120 at 1..4 rows 7.2-7.8 against 9.7-10.0; at k = 17408 the staging
-        // costs more than the hand-off it saves: 17.0 against 15.8). gemv_strips 2 forces it wherever it fits.
-        const bool strips_fit = k % 256 == 0 && (size_t)m * k * 2 <= 48 * 1024 && m <= 16;
-        const bool strips_pay = k <= 8192 && (m <= 2 || (n <= 8192 && m <= 4));  // (5120 x 17408 at 2 rows: 14.3 against 15.3 us; at 4: 16.5)
-        if (kern->gemv_strips && strips_fit && (strips_pay || kern->gemv_strips == 2)) {
-            const uint32_t strips = n / 16;
-            uint32_t waves = 4;  // wavefronts of a workgroup: two or more a SIMD in all
-            while (waves < 16 && strips * waves < 8 * kern->cus) waves *= 2;
-            if (kern->gemv_waves && kern->gemv_waves <= 16 && !(kern->gemv_waves & (kern->gemv_waves - 1))) waves = kern->gemv_waves;
-            while (waves > 1 && waves > kts / 4) waves /= 2;
-            // Where a wavefront's share of K can be at most five groups of four k tiles and the activations at most four
-            // 16-byte pieces a thread, the kernel that issues every load at once, with the number of wavefronts (any, up to
-            // 16) that wastes the fewest loads: a wavefront with fewer groups than the others requests one again, and a
-            // load instruction costs the address unit the same either way (5120 x 5120: 8 wavefronts of 3 groups for 20
-            // groups 9.3 us, 10 of 2 groups measured faster).
-            fe_function_t strip_fn = kern->strip4;
-            if (kern->gemv_once) {
-                const uint32_t groups = k / 256, want = kern->gemv_waves ? waves : std::max(4u, (8 * kern->cus + strips - 1) / strips);
-                uint32_t best_w = 0, best_waste = ~0u;
-                for (uint32_t w1 = std::min(want, 16u); w1 <= (kern->gemv_waves ? want : 16u); w1++) {
-                    const uint32_t gpw = (groups + w1 - 1) / w1;
-                    if (gpw > 5 || w1 > groups || ((size_t)m * (k / 8) + 64 * w1 - 1) / (64 * w1) > 4) continue;
-                    if (w1 * gpw - groups < best_waste) best_waste = w1 * gpw - groups, best_w = w1;
-                }
-                if (best_w) waves = best_w, strip_fn = kern->strip_once[(groups + best_w - 1) / best_w - 1];
-            }
-            fe_devptr_t w = l->w.p, sw = l->sw.p, alpha = l->alpha.p;
+        // up to 16 rows: programs of some columns over all of K, nothing handed between them
+        if (kern->gemv_strips && !kern->gemv_sk && m <= 16 && k % 256 == 0) {
+            const uint32_t form = m <= 2 ? 0 : m <= 4 ? 1 : m <= 8 ? 2 : 3, xp = kWideRowForms[form];
+            const uint32_t cols = wide_cols(n, xp, std::max(kern->cus, 1u), kern->gemv_cols), co = kWideColForms[cols];
+            fe_devptr_t aq = ws->aq.p, w = l->w.p, sw = l->sw.p, alpha = l->alpha.p;
             uint32_t w_snt = l->w_snt, w_skt = l->w_skt, w_sr = l->w_sr, s_snt = l->s_snt, s_skt = l->s_skt, s_sr = l->s_sr;
-            for (uint32_t r0 = 0; r0 < m; r0 += kGemvRows) {
-                uint32_t rows = m - r0 < kGemvRows ? m - r0 : kGemvRows;
-                fe_devptr_t yy = y + (size_t)r0 * ldy * 2, aq = ws->aq.p + (size_t)r0 * k * 2, rr = res ? res + (size_t)r0 * ldy * 2 : 0;
-                void *args[] = {&yy, &aq, &w, &sw, &alpha, &rr, &rows, &n, &k, &ldy, &w_snt, &w_skt, &w_sr, &s_snt, &s_skt, &s_sr};
-                FE_TRY(fe_hip_launch(strip_fn, strips, 1, 1, 64 * waves, 1, 1, rows * k * 2, s, args));
-            }
-            return 0;
+            void *args[] = {&y, &aq, &w, &sw, &alpha, &res, &m, &n, &k, &ldy, &w_snt, &w_skt, &w_sr, &s_snt, &s_skt, &s_sr};
+            return fe_hip_launch(kern->wide[form][cols], (n / 8 + co - 1) / co, 1, 1, 256, 1, 1, wide_lds(xp, co), s, args);
         }
         uint32_t sk = 2 * kern->cus / nts;
         if (kern->gemv_sk) sk = kern->gemv_sk;

@@ -7,6 +7,8 @@
 // exact, normal fp16 number: both operands are expanded to fp16 (activations as 2 * code value * block scale, weights
 // as 8 * ...) and multiplied on the f16 MFMA with fp32 accumulation, which reproduces the block-scaled dot product up
 // to summation order; the factor 16 comes off in the epilogue.
+#include <type_traits>
+
 #include "gemm8.h"
 
 // ---- number formats ----------------------------------------------------------------------------------------------------
@@ -805,200 +807,163 @@ FP4_GEMV_KERNEL(1)
 FP4_GEMV_KERNEL(2)
 FP4_GEMV_KERNEL(3)  // (four groups of rows would not fit the registers of two programs a CU)
 
-// ---- GEMV over strips of 16 weight rows (1..16 rows): no hand-off between programs ------------------------------------------
+// ---- GEMV over programs of 8 CO columns (1..16 rows): no hand-off, every operand straight into LDS ---------------------------------
 //
-// A program takes one strip of 16 weight rows over all of K; its W wavefronts (blockDim.x / 64: 4, 8 or 16, the host's
-// choice, so that a launch has four or more wavefronts a SIMD) take groups of four k tiles in turn and their sums meet
-// in LDS. Nothing crosses between programs: no partial sums in memory, no arrival counters, no finisher.
+// y[r][n] for r < m <= 2 XP. grid ceil(N / 8 CO), 256 threads: a program takes 8 CO weight rows over all of K, its four wavefronts a
+// quarter of K's steps of 256 each (four k tiles); their sums are added in order. A row's bits depend on (k, W) only. K % 256 == 0.
+// Lane L = 16 g + r multiplies, for 16 weight rows, row r's k tile 4 s + g (64 codes, four block scales) with the activations of the
+// same k; the order of k inside a step does not matter.
+// Stages belong to one wavefront (no barrier in the loop). Codes: 8 weight rows a load, [4 k tiles][8 rows][32 bytes]; lanes of
+// odd g read the second half of a row's k tile first, so that 16 lanes that read together cover the 64 banks. Scales: 16 rows a load,
+// [4 k tiles][16 rows][4]. Activations: 2 rows a load, 512 bytes each, chunk c at position c ^ (row & 15) in its half.
 //
-// What bounds a kernel that reads 9/16 byte a weight is the address unit: a vector memory instruction occupies it for
-// 16 clocks whatever it fetches. So a load step of a wavefront is four k tiles at once: lane L = 16 g + r takes row r
-// of k tile kt0 + g whole, 32 bytes of codes as two 16-byte loads and its four scale bytes as one dword (three
-// instructions per 2 KB of codes, where a lane that takes 16 codes of one k tile needs two per 512 bytes); the MFMA's k
-// index is only a summation index, so step s of the group multiplies, in lane group g, the 16 codes of scale block s of
-// k tile kt0 + g with the same 16 activations. The activations (m rows of k fp16: the host takes this kernel only where
-// they fit in 48 KB) are staged in LDS once per program and read from there. A row's bits depend on (k, W) only.
-struct Fp4StripStage {
-    u32x4 c[2];   // the lane's row of k tile kt0 + g: 64 codes
-    uint32_t sc;  // its four scale bytes
+// Bound by the codes' way from HBM and the start of a launch at one row, by the activations' way from L2 from 8 rows on. It replaces programs of 16 weight rows with the activations
+// staged whole (one and two rows: too many programs, each waiting for its own staging) and, up to 16 rows, weight tiles cut
+// along K (whose partial sums meet through memory; 17 rows and more still run there). us with the quantizer's launch, before -> now:
+// 5120 x 34816 at 1 / 4 / 8 / 16 rows 25.6 -> 22.1, 32.2 -> 22.1, 32.4 -> 25.7, 34.4 -> 28.8; 17408 x 5120 19.0 -> 14.3, 17.8 -> 14.9,
+// 18.0 -> 18.4, 19.3 -> 20.7; 5120 x 5120 9.6 -> 9.0, 10.3 -> 9.0, 12.2 -> 9.1, 12.5 -> 10.1.
+template <int XP, int CO>
+struct Fp4Wide {
+    static constexpr int CG = (CO + 1) / 2, L = CO + CG + XP;
+    static constexpr int SC_AT = CO * 1024, X_AT = SC_AT + CG * 256, STAGE = X_AT + XP * 1024;
+    static constexpr int FIT = 20 * 1024 / STAGE, DEPTH = FIT < 2 ? 2 : FIT < 6 ? FIT : 6;  // two programs a CU where two steps allow it
+    static constexpr int RED = 4 * 16 * (16 * CG + 4) * 4, LDS = 4 * DEPTH * STAGE > RED ? 4 * DEPTH * STAGE : RED;
+    static_assert(DEPTH >= 2 && (DEPTH - 1) * L < 64 && LDS <= 160 * 1024, "stages");
 };
-#define FP4_STRIP_WAVES_MAX 16
 
-__device__ __forceinline__ void gemv_nvfp4_strip_body(uint16_t* c, const _Float16* aq, const uint8_t* w, const uint8_t* sw,
-                                                      const float* alpha, const uint16_t* res, uint32_t m, uint32_t n, uint32_t k,
-                                                      uint32_t ldc, uint32_t w_snt, uint32_t w_skt, uint32_t w_sr, uint32_t s_snt,
-                                                      uint32_t s_skt, uint32_t s_sr) {
-    constexpr int XR = 1;  // up to 16 activation rows
-    __shared__ f32x4 red[FP4_STRIP_WAVES_MAX][64];
-    __shared__ u32x2 scale_lut[128];
-    extern __shared__ __attribute__((aligned(16))) unsigned char xs[];
-    const uint32_t tid = threadIdx.x, lane = tid & 63, wave = tid >> 6, waves = blockDim.x >> 6, r = lane & 15, g = lane >> 4;
-    fp4_scale_lut_fill(scale_lut);
-    for (uint32_t i = tid; i < m * (k / 8); i += blockDim.x) ((u32x4*)xs)[i] = ((const u32x4*)aq)[i];
-    const uint32_t strip = blockIdx.x, nt = strip >> 3, rg = strip & 7;  // the strip: 16-row group rg of weight tile nt
-    const uint32_t groups = k / 256;                                      // groups of four k tiles
-    const uint8_t* wp = w + (size_t)nt * w_snt + (size_t)(16 * rg + r) * w_sr + (size_t)g * w_skt;
-    const uint8_t* sp = sw + (size_t)nt * s_snt + (size_t)(16 * rg + r) * s_sr + (size_t)g * s_skt;
-    uint32_t xo[XR];  // byte offset in xs of the lane's activation row at k tile g
-#pragma unroll
-    for (int xr = 0; xr < XR; xr++) xo[xr] = ((16 * xr + r < m ? 16 * xr + r : m - 1) * k + 64 * g) * 2;
-
-    auto load = [&](Fp4StripStage& st, uint32_t gi) {
-        const uint8_t* p = wp + (size_t)gi * 4 * w_skt;
-        st.c[0] = __builtin_nontemporal_load((const u32x4*)p);
-        st.c[1] = __builtin_nontemporal_load((const u32x4*)(p + 16));
-        st.sc = __builtin_nontemporal_load((const uint32_t*)(sp + (size_t)gi * 4 * s_skt));
+template <int XP, int CO>
+__device__ __forceinline__ void gemv_nvfp4_wide_body(uint16_t* c, const _Float16* aq, const uint8_t* w, const uint8_t* sw,
+                                                     const float* alpha, const uint16_t* res, uint32_t m, uint32_t n, uint32_t k,
+                                                     uint32_t ldc, uint32_t w_snt, uint32_t w_skt, uint32_t w_sr, uint32_t s_snt,
+                                                     uint32_t s_skt, uint32_t s_sr) {
+    typedef Fp4Wide<XP, CO> C;
+    constexpr int CG = C::CG, AHEAD = C::DEPTH - 1, PITCH = 16 * CG + 4;
+    extern __shared__ __attribute__((aligned(1024))) unsigned char lds[];
+    const uint32_t tid = threadIdx.x, lane = tid & 63, wave = __builtin_amdgcn_readfirstlane(tid >> 6), r = lane & 15, g = lane >> 4;
+    const uint32_t col0 = blockIdx.x * 8 * CO, nt0 = col0 / 128, nts = n / 128, span = nts - nt0 < 2 ? nts - nt0 : 2;
+    const u32x4 wrs = g8_rsrc(w + (size_t)nt0 * w_snt, span * 128 * (k / 2)), srs = g8_rsrc(sw + (size_t)nt0 * s_snt, span * 128 * (k / 16));
+    const u32x4 xrs = g8_rsrc(aq, m * k * 2);
+    // weight row `row` of the program (past n: the last one again, not stored), byte offset from weight tile nt0
+    auto at = [&](uint32_t row, uint32_t snt, uint32_t sr) {
+        const uint32_t i = (col0 + row < n ? col0 + row : n - 1) - 128 * nt0;
+        return (i >> 7) * snt + (i & 127) * sr;
     };
-    f32x4 acc[XR];
+    uint32_t vw[CO], vs[CG], vx[XP];
 #pragma unroll
-    for (int xr = 0; xr < XR; xr++) acc[xr] = (f32x4){0.f, 0.f, 0.f, 0.f};
-    auto compute = [&](const Fp4StripStage& st, uint32_t gi) {
+    for (int j = 0; j < CO; j++) vw[j] = at(8 * j + ((lane >> 1) & 7), w_snt, w_sr) + g * w_skt + (lane & 1) * 16;
 #pragma unroll
-        for (int blk = 0; blk < 4; blk++) {  // scale block blk of the lane's k tile: codes 16 blk .. 16 blk + 15
-            const Fp4Scale s = fp4_scale_lut(scale_lut, __builtin_amdgcn_ubfe(st.sc, 8 * blk, 8) << 3);
+    for (int j = 0; j < CG; j++) vs[j] = at(16 * j + r, s_snt, s_sr) + g * s_skt;
 #pragma unroll
-            for (int j = 0; j < 2; j++) {
-                u32x4 a = fp4x8_to_f16(st.c[blk >> 1][2 * (blk & 1) + j], s);
+    for (int j = 0; j < XP; j++) {
+        const uint32_t row = 2 * j + (lane >> 5), chunk = (lane & 16) | ((lane ^ row) & 15);
+        vx[j] = (row < m ? row : m - 1) * k * 2 + chunk * 16;
+    }
+    unsigned char* stages = lds + wave * (C::DEPTH * C::STAGE);
+    const uint32_t stages0 = g8_lds_addr(stages);
+    const uint32_t steps = k / 256, s0 = wave * steps / 4, count = (wave + 1) * steps / 4 - s0;
+    auto issue = [&](uint32_t s, uint32_t slot) {
+        const uint32_t to = stages0 + slot * C::STAGE;
 #pragma unroll
-                for (int xr = 0; xr < XR; xr++) {
-                    const f16x8 x = *(const f16x8*)(xs + xo[xr] + gi * 512 + 32 * blk + 16 * j);
-                    acc[xr] = __builtin_amdgcn_mfma_f32_16x16x32_f16(__builtin_bit_cast(f16x8, a), x, acc[xr], 0, 0, 0);
-                }
+        for (int j = 0; j < CO; j++) g8_load_lds16_nt(wrs, to + j * 1024, vw[j], (s0 + s) * 4 * w_skt);
+#pragma unroll
+        for (int j = 0; j < CG; j++) g8_load_lds4(srs, to + C::SC_AT + j * 256, vs[j], (s0 + s) * 4 * s_skt);
+#pragma unroll
+        for (int j = 0; j < XP; j++) g8_load_lds16(xrs, to + C::X_AT + j * 1024, vx[j], (s0 + s) * 512);
+    };
+    const uint32_t odd = g & 1, xr = r < m ? r : m - 1;
+    // half h of the lane's row and k tile; the 16-byte chunk of 8 activations that goes with code 32 (h ^ odd) + 8 e on
+    uint32_t fw[CG], fx[8];
+#pragma unroll
+    for (int j = 0; j < CG; j++) {
+        const uint32_t row = 16 * j + r < 8 * CO ? 16 * j + r : 8 * CO - 1;
+        fw[j] = (row >> 3) * 1024 + g * 256 + (row & 7) * 32;
+    }
+#pragma unroll
+    for (int h = 0; h < 2; h++)
+#pragma unroll
+        for (int e = 0; e < 4; e++) {
+            const uint32_t chunk = 8 * g + 4 * (h ^ odd) + e;
+            fx[4 * h + e] = C::X_AT + xr * 512 + (((chunk & 16) | ((chunk ^ xr) & 15)) << 4);
+        }
+    f32x4 acc[CG] = {};
+    uint32_t slot = 0;
+    auto add = [&]() {
+        const unsigned char* st = stages + slot * C::STAGE;
+        uint32_t sc[CG];
+#pragma unroll
+        for (int j = 0; j < CG; j++) {
+            const uint32_t b = *(const uint32_t*)(st + C::SC_AT + j * 256 + lane * 4);
+            sc[j] = __builtin_amdgcn_alignbit(b, b, 16 * odd);
+        }
+#pragma unroll
+        for (int h = 0; h < 2; h++) {
+            f16x8 x[4];
+#pragma unroll
+            for (int e = 0; e < 4; e++) x[e] = *(const f16x8*)(st + fx[4 * h + e]);
+#pragma unroll
+            for (int j = 0; j < CG; j++) {
+                const u32x4 codes = *(const u32x4*)(st + fw[j] + 16 * (h ^ odd));
+#pragma unroll
+                for (int e = 0; e < 4; e++)
+                    acc[j] = __builtin_amdgcn_mfma_f32_16x16x32_f16(
+                        fp4x8_scaled(codes[e], fp4_scale_2m8(__builtin_amdgcn_ubfe(sc[j], 16 * h + 8 * (e >> 1), 8))), x[e], acc[j], 0, 0, 0);
             }
         }
+        slot = slot + 1 == C::DEPTH ? 0 : slot + 1;
     };
-    constexpr int NS = 4;  // groups in flight a wavefront (16 k tiles)
-    Fp4StripStage st[NS];
-    uint32_t gi = wave;
+    if (count) {
 #pragma unroll
-    for (int i = 0; i < NS; i++)
-        if (gi + waves * i < groups) load(st[i], gi + waves * i);
-    __syncthreads();  // scale_lut, xs
-    for (; gi < groups; gi += waves * NS) {
-#pragma unroll
-        for (int i = 0; i < NS; i++) {
-            if (gi + waves * i < groups) compute(st[i], gi + waves * i);
-            __builtin_amdgcn_sched_barrier(0);
-            if (gi + waves * (i + NS) < groups) load(st[i], gi + waves * (i + NS));
-            __builtin_amdgcn_sched_barrier(0);
+        for (int u = 0; u < AHEAD; u++) issue((uint32_t)u < count ? u : count - 1, u);  // past the end: the last step again, not added
+        uint32_t s = 0;
+        for (; s + AHEAD < count; s++) {
+            g8_loads_wait<(AHEAD - 1) * C::L>();  // (the stage in front of this one has been read, too)
+            issue(s + AHEAD, slot ? slot - 1 : AHEAD);
+            add();
         }
-    }
-    // The wavefronts' sums meet in LDS, one group of activation rows at a time; wavefront 0 adds them in wavefront order.
-    // Lane (r, g) holds output row 16 xr + r, columns 16 strip + 4 g .. + 3.
-    const uint32_t col = 16 * strip + 4 * g;
-#pragma unroll
-    for (int xr = 0; xr < XR; xr++) {
-        if (xr) __syncthreads();
-        red[wave][lane] = acc[xr];
-        __syncthreads();
-        const uint32_t row = 16 * xr + r;
-        if (wave == 0 && row < m) {
-            f32x4 sum = red[0][lane];
-            for (uint32_t v = 1; v < waves; v++) sum += red[v][lane];
-            float o[4] = {sum[0], sum[1], sum[2], sum[3]};
-            fp4_store4(c, res, (size_t)row * ldc + col, o, *(const f32x4*)(alpha + col) * FP4_OPERAND_SCALE);
-        }
-    }
-}
-
-extern "C" __global__ __launch_bounds__(1024) void fe_gemv_nvfp4_strips(uint16_t* c, const _Float16* aq, const uint8_t* w,
-                                                                        const uint8_t* sw, const float* alpha, const uint16_t* res,
-                                                                        uint32_t m, uint32_t n, uint32_t k, uint32_t ldc, uint32_t w_snt,
-                                                                        uint32_t w_skt, uint32_t w_sr, uint32_t s_snt, uint32_t s_skt,
-                                                                        uint32_t s_sr) {
-    gemv_nvfp4_strip_body(c, aq, w, sw, alpha, res, m, n, k, ldc, w_snt, w_skt, w_sr, s_snt, s_skt, s_sr);
-}
-
-// The same strips when a wavefront's share of K is GPW <= 5 groups and the activations are at most four 16-byte pieces a
-// thread: every load of the workgroup goes out before anything waits. The activations' loads first (they
-// are few and mostly hit L2; loads return in order), then the wavefront's whole share of the strip, then the activations
-// go to LDS while the weights are on their way, and the groups are taken in the order they arrive. No load sits under a
-// condition (a wavefront with fewer groups than the others requests its last group again and does not use it; a thread
-// past the end of the activations requests the last piece again), so the compiler counts its waits exactly instead of
-// waiting for everything at the head of a loop. A vector memory instruction costs the address unit the same whether
-// its data is wanted or not, so the kernel exists per GPW and the host picks a number of wavefronts that divides the
-// groups where it can (any number up to 16, not only powers of two).
-template <int GPW>
-__device__ __forceinline__ void gemv_nvfp4_strip_once_body(uint16_t* c, const _Float16* aq, const uint8_t* w, const uint8_t* sw,
-                                                           const float* alpha, const uint16_t* res, uint32_t m, uint32_t k,
-                                                           uint32_t ldc, uint32_t w_snt, uint32_t w_skt, uint32_t w_sr,
-                                                           uint32_t s_snt, uint32_t s_skt, uint32_t s_sr) {
-    __shared__ f32x4 red[FP4_STRIP_WAVES_MAX][64];
-    __shared__ u32x2 scale_lut[128];
-    extern __shared__ __attribute__((aligned(16))) unsigned char xs[];
-    const uint32_t tid = threadIdx.x, lane = tid & 63, wave = tid >> 6, waves = blockDim.x >> 6, r = lane & 15, g = lane >> 4;
-    constexpr int XV = 4;
-    const uint32_t xn = m * (k / 8);  // 16-byte pieces of the activations
-    u32x4 xv[XV];
-    uint32_t xi[XV];
-#pragma unroll
-    for (int i = 0; i < XV; i++) {
-        xi[i] = tid + i * blockDim.x;
-        xi[i] = xi[i] < xn ? xi[i] : xn - 1;
-        xv[i] = ((const u32x4*)aq)[xi[i]];
-    }
-    const uint32_t strip = blockIdx.x, nt = strip >> 3, rg = strip & 7;  // the strip: 16-row group rg of weight tile nt
-    const uint32_t groups = k / 256;                                      // groups of four k tiles
-    const uint8_t* wp = w + (size_t)nt * w_snt + (size_t)(16 * rg + r) * w_sr + (size_t)g * w_skt;
-    const uint8_t* sp = sw + (size_t)nt * s_snt + (size_t)(16 * rg + r) * s_sr + (size_t)g * s_skt;
-    Fp4StripStage st[GPW];
-#pragma unroll
-    for (int i = 0; i < GPW; i++) {
-        uint32_t gi = wave + waves * i;
-        gi = gi < groups ? gi : groups - 1;
-        const uint8_t* p = wp + (size_t)gi * 4 * w_skt;
-        st[i].c[0] = __builtin_nontemporal_load((const u32x4*)p);
-        st[i].c[1] = __builtin_nontemporal_load((const u32x4*)(p + 16));
-        st[i].sc = __builtin_nontemporal_load((const uint32_t*)(sp + (size_t)gi * 4 * s_skt));
-    }
-    fp4_scale_lut_fill(scale_lut);
-#pragma unroll
-    for (int i = 0; i < XV; i++) ((u32x4*)xs)[xi[i]] = xv[i];
-    __syncthreads();  // scale_lut, xs
-    const uint32_t xo = ((r < m ? r : m - 1) * k + 64 * g) * 2;  // byte offset in xs of the lane's activation row at k tile g
-    f32x4 acc = (f32x4){0.f, 0.f, 0.f, 0.f};
-#pragma unroll
-    for (int i = 0; i < GPW; i++) {
-        const uint32_t gi = wave + waves * i;
-        if (gi < groups) {
-#pragma unroll
-            for (int blk = 0; blk < 4; blk++) {  // scale block blk of the lane's k tile: codes 16 blk .. 16 blk + 15
-                const Fp4Scale sc = fp4_scale_lut(scale_lut, __builtin_amdgcn_ubfe(st[i].sc, 8 * blk, 8) << 3);
-#pragma unroll
-                for (int j = 0; j < 2; j++) {
-                    u32x4 a = fp4x8_to_f16(st[i].c[blk >> 1][2 * (blk & 1) + j], sc);
-                    const f16x8 x = *(const f16x8*)(xs + xo + gi * 512 + 32 * blk + 16 * j);
-                    acc = __builtin_amdgcn_mfma_f32_16x16x32_f16(__builtin_bit_cast(f16x8, a), x, acc, 0, 0, 0);
+        auto tail = [&](auto u_tag) {
+            constexpr int U = decltype(u_tag)::value;
+            if constexpr (U < AHEAD)
+                if (s + U < count) {
+                    g8_loads_wait<(AHEAD - 1 - U) * C::L>();
+                    add();
                 }
-            }
-        }
+        };
+        tail(std::integral_constant<int, 0>{});
+        tail(std::integral_constant<int, 1>{});
+        tail(std::integral_constant<int, 2>{});
+        tail(std::integral_constant<int, 3>{});
+        tail(std::integral_constant<int, 4>{});
+        g8_loads_wait<0>();
     }
-    // The wavefronts' sums meet in LDS; wavefront 0 adds them in wavefront order. Lane (r, g) holds output row r, columns
-    // 16 strip + 4 g .. + 3. (The groups of a wavefront are added in the order of the kernel above: the same bits.)
-    const uint32_t col = 16 * strip + 4 * g;
-    red[wave][lane] = acc;
+    float(*red)[16][PITCH] = (float(*)[16][PITCH])lds;
     __syncthreads();
-    if (wave == 0 && r < m) {
-        f32x4 sum = red[0][lane];
-        for (uint32_t v = 1; v < waves; v++) sum += red[v][lane];
-        float o[4] = {sum[0], sum[1], sum[2], sum[3]};
-        fp4_store4(c, res, (size_t)r * ldc + col, o, *(const f32x4*)(alpha + col) * FP4_OPERAND_SCALE);
+#pragma unroll
+    for (int j = 0; j < CG; j++) *(f32x4*)&red[wave][r][16 * j + 4 * g] = acc[j];
+    __syncthreads();
+    for (uint32_t i = tid; i < m * 2 * CO; i += 256) {
+        const uint32_t row = i / (2 * CO), j = 4 * (i % (2 * CO)), col = col0 + j;
+        if (col >= n) continue;
+        const f32x4 sum = ((*(const f32x4*)&red[0][row][j] + *(const f32x4*)&red[1][row][j]) + *(const f32x4*)&red[2][row][j]) +
+                          *(const f32x4*)&red[3][row][j];
+        const float v[4] = {sum[0], sum[1], sum[2], sum[3]};
+        fp4_store4(c, res, (size_t)row * ldc + col, v, *(const f32x4*)(alpha + col) * FP4_GEMM_SCALE);
     }
 }
 
-#define FP4_STRIPS_ONCE_KERNEL(GPW)                                                                                       \
-    extern "C" __global__ __launch_bounds__(1024) void fe_gemv_nvfp4_strips_once_g##GPW(                                  \
+#define FP4_WIDE_KERNEL(XP, CO)                                                                                           \
+    extern "C" __global__ __launch_bounds__(256) void fe_gemv_nvfp4_r##XP##_c##CO(                                        \
         uint16_t* c, const _Float16* aq, const uint8_t* w, const uint8_t* sw, const float* alpha, const uint16_t* res,   \
         uint32_t m, uint32_t n, uint32_t k, uint32_t ldc, uint32_t w_snt, uint32_t w_skt, uint32_t w_sr, uint32_t s_snt, \
         uint32_t s_skt, uint32_t s_sr) {                                                                                  \
-        (void)n;                                                                                                          \
-        gemv_nvfp4_strip_once_body<GPW>(c, aq, w, sw, alpha, res, m, k, ldc, w_snt, w_skt, w_sr, s_snt, s_skt, s_sr);     \
+        gemv_nvfp4_wide_body<XP, CO>(c, aq, w, sw, alpha, res, m, n, k, ldc, w_snt, w_skt, w_sr, s_snt, s_skt, s_sr);     \
     }
-FP4_STRIPS_ONCE_KERNEL(1)
-FP4_STRIPS_ONCE_KERNEL(2)
-FP4_STRIPS_ONCE_KERNEL(3)
-FP4_STRIPS_ONCE_KERNEL(4)
-FP4_STRIPS_ONCE_KERNEL(5)
+#define FP4_WIDE_FAMILY(XP)                                                                                             \
+    FP4_WIDE_KERNEL(XP, 1) FP4_WIDE_KERNEL(XP, 2) FP4_WIDE_KERNEL(XP, 3) FP4_WIDE_KERNEL(XP, 4) FP4_WIDE_KERNEL(XP, 5)  \
+    FP4_WIDE_KERNEL(XP, 6) FP4_WIDE_KERNEL(XP, 9)
+FP4_WIDE_FAMILY(1)
+FP4_WIDE_FAMILY(2)
+FP4_WIDE_FAMILY(4)
+FP4_WIDE_FAMILY(8)
 
 // ---- matrix-unit peak probe ---------------------------------------------------------------------------------------------
 //

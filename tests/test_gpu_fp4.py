@@ -307,6 +307,43 @@ def test_fp4_gemv_over_strips_agrees_with_the_weight_tiles(env, oracle, n, k):
         kern.set_option("gemv_once", 1)
 
 
+@pytest.mark.parametrize("n,k", [(128, 256), (384, 768), (640, 1280), (256, 4352)])
+def test_fp4_gemv_up_to_16_rows_at_its_edges(env, oracle, n, k):
+    """Every row form and every width of a program, wavefronts without a step (k = 256), programs that cross weight tiles or end
+    past the last column, both weight layouts: a row's bits depend on nothing but k and the weights; against the GEMV over
+    weight tiles (the same exact products in another order); rows past m untouched."""
+    torch, fp4, kern = env
+    from ferrite_amd import synth
+    host = synth.fp4_linear(n, k, 53, input_scale=1.0)
+    host.alpha[:] = host.alpha * np.linspace(0.5, 2.0, n).astype(np.float32)
+    lin = host.upload()
+    view = fp4.PromptLinear.from_view("view", n, k, torch.from_numpy(host.codes).cuda(), torch.from_numpy(host.sf).cuda(),
+                                      torch.from_numpy(host.alpha).cuda(), host.g)
+    ws = fp4.Workspace(16, k)
+    xd = dev_u16(torch, fp4_check_activations(16, k, lin.g, 71))
+
+    def run(l, m, cols, strips=1):
+        kern.set_option("gemv_cols", cols)
+        kern.set_option("gemv_strips", strips)
+        y = torch.full((m + 1, n), -3.0, dtype=torch.bfloat16, device="cuda")
+        l.forward(kern, ws, y, n, xd, k, m)
+        torch.cuda.synchronize()
+        out = y.view(torch.int16).cpu().numpy().view(np.uint16)
+        assert (out[m:] == bf16_bits(np.float32([-3.0]))[0]).all()
+        return out[:m]
+
+    try:
+        want = run(lin, 16, 0)
+        a, b = bf16_to_f32(want).astype(np.float64), bf16_to_f32(run(lin, 16, 0, strips=0)).astype(np.float64)
+        assert (np.abs(a - b) <= np.abs(b) / 128.0 + 1e-30).all()
+        for m in (1, 2, 3, 4, 5, 8, 9, 15, 16):
+            for cols in (0, 8, 16, 24, 32, 40, 48, 72):
+                assert np.array_equal(run(lin, m, cols), want[:m]) and np.array_equal(run(view, m, cols), want[:m]), (m, cols)
+    finally:
+        kern.set_option("gemv_cols", 0)
+        kern.set_option("gemv_strips", 1)
+
+
 def test_quantizer_on_special_values(env, oracle):
     """Ties between codes, the saturation boundary, signed zeros, infinities and NaN (a NaN element has magnitude 0 and
     keeps its sign, format.rs:28-41, 66-69; it does not enter the block maximum, format.rs:76): codes and scales as the
