@@ -304,13 +304,18 @@ int fe_exl3_plan_parse(const char *s, fe_exl3_plan *out) {
 // partition). Never more programs than units.
 static uint32_t plan_programs(const fe_exl3_kernels *kern, const fe_exl3_plan &p, uint32_t k, uint32_t n) {
     const uint32_t units = (k / 128) * (n / 128);
+    // Runs of four units at least (plan_for): shorter ones leave more partial sums than they save time. With fewer units than CUs,
+    // where most CUs would have no program at all, runs of two instead: us at 1 / 16 / 64 rows, four -> two: 1024 x 1024 (64 units)
+    // 7.4 -> 6.6, 10.3 -> 9.1, 13.5 -> 12.2; 2816 x 1024 (176) 8.8 -> 7.2, 12.0 -> 10.5, 16.9 -> 17.3; 2048 x 2048 (256) 8.1 -> 7.8, 10.7 ->
+    // 10.8, 14.8 -> 17.4; 5120 x 1024 (320) 8.2 -> 8.6, 11.7 -> 12.5, 18.6 -> 22.5. The 1024 / 2816 MLP block at 1 row 16.8 -> 13.7.
+    const uint32_t wk = p.ver == 3 && p.wk == 4 && units < kern->cus ? 2 : std::max(p.wk, 1u);
     uint32_t progs;
     if (p.ver <= 1)
         progs = n / 128 * std::max(p.sk, 1u);
     else if (p.ver == 4)
         progs = std::max(p.sk, 1u);
     else
-        progs = (p.occ ? p.occ : 4) * std::max(kern->cus, 1u), progs = std::min(progs, units / std::max(p.wk, 1u));
+        progs = (p.occ ? p.occ : 4) * std::max(kern->cus, 1u), progs = std::min(progs, units / wk);
     // Wider than deep (gate, up): two programs a CU where a plan asks for four. Such linears come in pairs, whose programs
     // fill the CUs together, and every program leaves its partial sums of every row in memory: 1024 programs of 64 rows wrote
     // and read 38 MB beside 45 MB of weights. 5120 x 17408 at 4 bits, gate + up + down: 1..16 rows the same, 40 rows 95 -> 87 us,

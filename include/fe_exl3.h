@@ -39,8 +39,8 @@ typedef struct {
 /* Launch plan (Plan, crates/fe-exl3/src/linear.rs:33-43), the reference's plan strings "sk,wk[,ver[,occ]]". The gfx950
  * decode GEMV deals 128-channel x 128-column units of the tensor to its programs in equal contiguous runs; a plan says how
  * many programs. ver 1 (the reference's meaning): sk programs per 128-column block, i.e. sk K splits (needs k / 64
- * divisible by sk). ver 2, 3 (what fe_exl3_plan_for returns): occ programs per CU, each a run of at least wk units; sk then
- * records the K splits per column block this amounts to. ver 4: sk programs in all (any partition: tests and tuners). */
+ * divisible by sk). ver 2, 3 (what fe_exl3_plan_for returns): occ programs per CU, each a run of at least wk units (ver 3:
+ * of two for the default of four where a tensor has fewer units than the device CUs); sk then records the K splits per column block this amounts to. ver 4: sk programs in all (any partition: tests and tuners). */
 typedef struct {
     uint32_t sk, wk, ver, occ;
 } fe_exl3_plan;
