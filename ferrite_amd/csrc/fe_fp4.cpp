@@ -34,7 +34,7 @@ struct fe_fp4_kernels {
     // by form (256 x 256, stream-K, 128 x 256, 128 x 128) and by tile (fe_gemm_launch); gemm8: the fp16 form, 256 x 256 only
     fe_function_t gemm4[4] = {}, swiglu4[4] = {}, gemm8c[4] = {}, gemm8[2] = {}, reduce4[3] = {}, swiglu_reduce4[3] = {}, reduce8c[3] = {};
     fe_function_t wide[4][7] = {};   // the GEMV over programs of 8 CO columns, [kWideRowForms][kWideColForms]
-    fe_function_t quant8 = nullptr;
+    fe_function_t quant8 = nullptr, expand8 = nullptr;
     uint32_t cus = 0;
     // Switches of the launch paths: read from the environment once, at load; fe_fp4_kernels_set_option changes them
     // afterwards. No forward call reads the environment.
@@ -101,6 +101,7 @@ int fe_fp4_kernels_load(fe_fp4_kernels **out) {
             get(&k->wide[i][j], "fe_gemv_nvfp4_r" + std::to_string(kWideRowForms[i]) + "_c" + std::to_string(kWideColForms[j]),
                 wide_lds(kWideRowForms[i], kWideColForms[j]));
     if (!c) c = fe_hip_module_get_function(&k->quant8, k->module, "fe_fp8_quant");
+    if (!c) c = fe_hip_module_get_function(&k->expand8, k->module, "fe_fp8_expand");
     int cus = 0;
     if (!c) c = fe_hip_cu_count(&cus);
     k->cus = (uint32_t)cus;
@@ -328,8 +329,8 @@ int fe_fp4_linear_quantize(const fe_fp4_linear *l, const fe_fp4_kernels *kern, f
     float g = l->g;
     fe_devptr_t codes = ws->codes.p, sf = ws->sf.p, aq = ws->aq.p;
     if (l->fp8) {
-        void *args8[] = {&codes, &aq, &x, &m, &k, &lda, &g};
-        return fe_hip_launch(kern->quant8, (m * (k / 8) + 255) / 256, 1, 1, 256, 1, 1, 0, s, args8);
+        void *args8[] = {&codes, &x, &m, &k, &lda, &g};
+        return fe_hip_launch(kern->quant8, (m * (k / 16) + 255) / 256, 1, 1, 256, 1, 1, 0, s, args8);
     }
     void *args[] = {&codes, &sf, &aq, &x, &m, &k, &lda, &g};
     const uint32_t blocks16 = m * (k / 16);
@@ -415,6 +416,12 @@ int fe_fp4_linear_gemm(const fe_fp4_linear *l, const fe_fp4_kernels *kern, fe_st
     const FeGemmPlan plan = fe_gemm_plan(m, n, codes8 ? k / 128 : k / 64, kern->cus, ws->part.p, ws->part.bytes, ws->counters.p, kGemvCounters,
                                          kern->gemm_splits, kern->gemm_sk, /*small_b=*/!l->fp8,
                                          l->fp8 ? kFeCostFp8 : kFeCostNvfp4, l->fp8 && !codes8 ? f16_form : kern->tile);
+    if (l->fp8 && !codes8) {
+        uint32_t count = m * k;
+        fe_devptr_t codes = ws->codes.p;
+        void *args[] = {&aq, &codes, &count};
+        FE_TRY(fe_hip_launch(kern->expand8, (count / 8 + 255) / 256, 1, 1, 256, 1, 1, 0, s, args));
+    }
     // stream-K programs sit at different depths of K: one row tile at a time (column tiles fastest) keeps those that are
     // in step on one panel of activations
     if (!plan.tile && plan.big.stream_k && kern->xcd < 0) group = 1;

@@ -266,33 +266,45 @@ __device__ __forceinline__ uint32_t e4m3x2_to_f16(uint32_t w, int hi) {
     return __builtin_bit_cast(uint32_t, v);
 }
 
-// f32 -> e4m3 code of either sign, round to nearest even, saturating; NaN -> 0x7f. (crates/fe-fp4/src/format.rs:57-63)
-__device__ __forceinline__ uint32_t f32_to_e4m3(float x) {
-    if (x != x) return 0x7f;
-    return f32_to_e4m3_pos(__builtin_fabsf(x)) | ((__float_as_uint(x) >> 24) & 0x80u);
+// Two f32 -> two e4m3 codes in bytes 0, 1 (HI: 2, 3) of old: round to nearest even, saturating, either sign; NaN -> 0x7f. The hardware
+// conversion on clamped values (checked against the definition for every bf16 value). (crates/fe-fp4/src/format.rs:57-63)
+template <bool HI>
+__device__ __forceinline__ uint32_t f32x2_to_e4m3(uint32_t old, float a, float b) {
+    uint32_t q = (uint32_t)__builtin_amdgcn_cvt_pk_fp8_f32(__builtin_amdgcn_fmed3f(a, -448.f, 448.f), __builtin_amdgcn_fmed3f(b, -448.f, 448.f), (int)old, HI);
+    constexpr uint32_t S = HI ? 16 : 0;
+    if (a != a) q = (q & ~(0xffu << S)) | (0x7fu << S);
+    if (b != b) q = (q & ~(0xff00u << S)) | (0x7f00u << S);
+    return q;
 }
 
-// bf16 x[M][ldx] -> e4m3 codes [M][K], q = e4m3(x * g), and the fp16 operand the GEMM reads (an e4m3 value is an exact
-// fp16 number). One thread per 8 elements: grid ceil(M * K / 8 / 256), 256 threads. K % 8 == 0.
-// (kernels/k-fp4/src/lib.rs:199-214)
-extern "C" __global__ __launch_bounds__(256) void fe_fp8_quant(uint8_t* codes, _Float16* aq, const uint16_t* x, uint32_t m,
-                                                               uint32_t k, uint32_t ldx, float g) {
-    uint32_t i = blockIdx.x * 256 + threadIdx.x, k8 = k >> 3;
-    if (i >= m * k8) return;
-    uint32_t row = i / k8, c = (i - row * k8) * 8;
-    u32x4 r = *(const u32x4*)(x + (size_t)row * ldx + c);
-    uint32_t q[2] = {0, 0};
+// bf16 x[M][ldx] -> e4m3 codes [M][K], q = e4m3(x * g). One thread per 16 elements: grid ceil(M * K / 16 / 256), 256 threads. K % 16
+// == 0, rows 16-byte aligned. Bound by its 3 bytes an element. (kernels/k-fp4/src/lib.rs:199-214)
+extern "C" __global__ __launch_bounds__(256) void fe_fp8_quant(uint8_t* codes, const uint16_t* x, uint32_t m, uint32_t k, uint32_t ldx, float g) {
+    const uint32_t i = blockIdx.x * 256 + threadIdx.x, k16 = k >> 4;
+    if (i >= m * k16) return;
+    const uint32_t row = i / k16, c = (i - row * k16) * 16;
+    const u32x4* p = (const u32x4*)(x + (size_t)row * ldx + c);
+    const u32x4 r[2] = {p[0], p[1]};
+    u32x4 q;
 #pragma unroll
     for (int j = 0; j < 4; j++) {
-        uint32_t lo = f32_to_e4m3(__uint_as_float(r[j] << 16) * g), hi = f32_to_e4m3(__uint_as_float(r[j] & 0xffff0000u) * g);
-        q[j >> 1] |= (lo | (hi << 8)) << (16 * (j & 1));
+        const uint32_t lo = r[j >> 1][2 * (j & 1)], hi = r[j >> 1][2 * (j & 1) + 1];
+        const uint32_t t = f32x2_to_e4m3<false>(0, __uint_as_float(lo << 16) * g, __uint_as_float(lo & 0xffff0000u) * g);
+        q[j] = f32x2_to_e4m3<true>(t, __uint_as_float(hi << 16) * g, __uint_as_float(hi & 0xffff0000u) * g);
     }
-    *(u32x2*)(codes + (size_t)row * k + c) = (u32x2){q[0], q[1]};
+    *(u32x4*)(codes + (size_t)row * k + c) = q;
+}
+
+// e4m3 codes -> the fp16 operand of the fp16 form of the FP8 GEMM (an e4m3 value is an exact fp16 number). One thread per 8 of
+// `count` elements.
+extern "C" __global__ __launch_bounds__(256) void fe_fp8_expand(_Float16* aq, const uint8_t* codes, uint32_t count) {
+    const uint32_t i = (blockIdx.x * 256 + threadIdx.x) * 8;
+    if (i >= count) return;
+    const u32x2 q = *(const u32x2*)(codes + i);
     u32x4 o;
 #pragma unroll
-    for (int j = 0; j < 4; j++)
-        o[j] = e4m3x2_to_f16(q[j >> 1], j & 1);
-    *(u32x4*)(aq + (size_t)row * k + c) = o;
+    for (int j = 0; j < 4; j++) o[j] = e4m3x2_to_f16(q[j >> 1], j & 1);
+    *(u32x4*)(aq + i) = o;
 }
 
 // Weight operand of the fp16 form of the FP8 GEMM: e4m3 codes, [BN rows][64 bytes] in LDS, expanded with the hardware

@@ -28,6 +28,21 @@ def bf16_bits(x):
     return ((b + 0x7FFF + ((b >> 16) & 1)) >> 16).astype(np.uint16)
 
 
+@pytest.mark.parametrize("input_scale", [1.0, 0.3, 1e-3, 77.0])
+def test_fp8_quantizer_on_every_bf16_value(env, oracle, input_scale):
+    """Codes of all 65536 bf16 values (subnormals, infinities, NaN of either sign) at four scales, byte for byte."""
+    torch, fp4, kern = env
+    from ferrite_amd import synth
+    m, k = 64, 1024
+    lin = synth.fp8_linear(128, k, 3, input_scale=input_scale).upload()
+    ws = fp4.Workspace(m, k)
+    xb = np.random.default_rng(1).permutation(np.arange(1 << 16, dtype=np.uint32)).astype(np.uint16).reshape(m, k)
+    y = torch.zeros((m, 128), dtype=torch.bfloat16, device="cuda")
+    lin.forward(kern, ws, y, 128, dev_u16(torch, xb), k, m)
+    torch.cuda.synchronize()
+    assert np.array_equal(ws.read_fp8(m, k), np.stack([oracle.quant_fp8_row(r, lin.g) for r in xb]))
+
+
 @pytest.mark.parametrize("n,k,m,input_scale", [(256, 512, 200, 0.05), (128, 1024, 1, 0.02), (640, 256, 300, 0.1),
                                                (384, 1152, 520, 0.05)])
 def test_fp8_linear(env, oracle, n, k, m, input_scale):
