@@ -358,3 +358,26 @@ def test_mlp_block_routes_as_the_reference(env, oracle):
     rms = np.sqrt((ref ** 2).mean())
     assert np.abs(gotf - ref).max() / rms < 3e-2  # three bf16 roundings on the way (gate/up, silu, act) and the fp16 rotation
     c.dec = 0
+
+
+@pytest.mark.parametrize("rows", [65, 203, 320])
+def test_mlp_block_of_a_prompt_through_the_trellis_alone(env, rows):
+    """No prompt weights: down reads SwiGLU of gate and up as it rotates its input; the bits of the steps by hand
+    (gate, up, fe_silu_mul, down with the residual), rows past the prompt untouched."""
+    e = env
+    torch, route, exl3 = e.torch, e.route, e.exl3
+    c = route.LinCtx((e.xk, e.xws), None, None)
+    gate_up = route.Proj([(route.Linear("gate", INTER, HIDDEN, q=e.q_gate), [INTER]), (route.Linear("up", INTER, HIDDEN, q=e.q_up), [INTER])])
+    down = route.Linear("down", HIDDEN, INTER, q=e.q_down)
+    xn = dev_u16(torch, e.synth.activations(rows, HIDDEN, 21))
+    x_b = bf16_bits(np.random.default_rng(22).normal(size=(rows + 1, HIDDEN)).astype(np.float32))
+    new = lambda n: torch.zeros((rows, n), dtype=torch.bfloat16, device="cuda")
+    yg, yu, a, want = new(INTER), new(INTER), new(INTER), dev_u16(torch, x_b).view(torch.bfloat16)
+    for lin, y in ((e.q_gate, yg), (e.q_up, yu)):
+        lin.forward(xn, exl3.Dtype.Bf16, y, exl3.Dtype.Bf16, rows, e.xws)
+    route.silu_mul(a, yg.data_ptr(), yu.data_ptr(), INTER, INTER, rows)
+    e.q_down.forward(a, exl3.Dtype.Bf16, want, exl3.Dtype.Bf16Add, rows, e.xws)
+    x = dev_u16(torch, x_b).view(torch.bfloat16)
+    route.mlp_forward(c, gate_up, down, x, xn, new(2 * INTER), new(INTER), rows, HIDDEN, INTER)
+    torch.cuda.synchronize()
+    assert np.array_equal(bits(x), bits(want)) and not np.array_equal(bits(x)[:rows], x_b[:rows])
