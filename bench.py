@@ -869,7 +869,7 @@ def prefill(torch, np, exl3, fp4, synth, kern, ev, stream, m=2048, k=5120, n=174
     y8 = torch.zeros((m, n), dtype=torch.bfloat16, device="cuda")
     f8.forward(fk, fws, y8, n, xf, k, m)
     ms = timed(lambda: f8.gemm(fk, fws, y8, n, m), 5)
-    res["fp8_5120x17408"] = {"gemm_ms": round(ms, 4), "TFLOP/s": round(flops / ms / 1e9, 1), "mfma": "f32_32x32x64_f8f6f4 (e4m3 x e4m3)",
+    res["fp8_5120x17408"] = {"gemm_ms": round(ms, 4), "TFLOP/s": round(flops / ms / 1e9, 1), "mfma": "f32_16x16x128_f8f6f4 (e4m3 x e4m3)",
                              "frac_mfma_fp8_peak": round(flops / ms / 1e9 / MFMA_FP8_PEAK_TFLOPS, 4)}
     del f8, y8
     # the plain bf16 weight form of the same linear (the caller's third form): GEMM at M = 2048 on the bf16 MFMA, GEMV

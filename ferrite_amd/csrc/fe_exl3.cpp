@@ -319,7 +319,8 @@ static uint32_t plan_programs(const fe_exl3_kernels *kern, const fe_exl3_plan &p
     // Wider than deep (gate, up): two programs a CU where a plan asks for four. Such linears come in pairs, whose programs
     // fill the CUs together, and every program leaves its partial sums of every row in memory: 1024 programs of 64 rows wrote
     // and read 38 MB beside 45 MB of weights. 5120 x 17408 at 4 bits, gate + up + down: 1..16 rows the same, 40 rows 95 -> 87 us,
-    // 64 rows 117 -> 104. (A down projection keeps its shorter runs: it is the tail of the one-launch MLP.)
+    // 64 rows 117 -> 104. One such linear launched alone pays at few rows: 1 row 19.3 -> 20.4, 16 rows 25.3 -> 26.6, 40 rows 33.6 -> 31.1, 64 rows
+    // 40.8 -> 35.1 (65536 columns: 48.3 -> 47.7 .. 81.8 -> 78.5). (A down projection keeps its shorter runs: it is the tail of the one-launch MLP.)
     if (p.ver == 3 && p.occ == 4 && n > k) progs = std::min(progs, 2 * std::max(kern->cus, 1u));
     return std::max(1u, std::min(progs, units));
 }
