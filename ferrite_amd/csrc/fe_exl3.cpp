@@ -645,6 +645,10 @@ struct RotGroupArgs {  // RotGroup
     fe_devptr_t suh[kGroupMax], xh[kGroupMax];
 };
 
+// The decode GEMV addresses a trellis as one buffer by 32-bit offsets; the prefill GEMM and the decode into tiles do not, and take
+// any size.
+static bool gemv_reaches(const fe_exl3_linear *l) { return fe_exl3_linear_weight_bytes(l) < (1ull << 32); }
+
 // The decode GEMV for 1..4 linears of one input in one launch, 1..64 rows: member i reads its rotated input at xhs[i]
 // (in.x == 0) or rotates in.x itself and leaves the result at xhs[i]. The caller has checked rows, k and bits.
 static int launch_job(const fe_exl3_linear *const *ls, size_t count, fe_stream_t s, const fe_devptr_t *xhs, const fe_devptr_t *ys,
@@ -668,6 +672,11 @@ static int launch_job(const fe_exl3_linear *const *ls, size_t count, fe_stream_t
     for (size_t i = 0; i < count; i++) {
         const fe_exl3_linear *l = ls[i];
         GemvJobArgs::Member &m = g.m[i];
+        if (!gemv_reaches(l)) {
+            snprintf(msg, sizeof msg, "%s: trellis of 4 GB or more at %u rows (only calls of more than %u rows take it)", l->name.c_str(), rows,
+                     kMaxRowsPerPass);
+            return fe_set_error(FE_ERR_UNSUPPORTED, fn, msg);
+        }
         if (z_at + job_z(l, rows) > ws->z_len || cnt_at + l->n / 128 > ws->counters_len) {
             snprintf(msg, sizeof msg, "%s: %u rows do not fit the workspace (partial sums %zu of %zu floats, counters %zu of %zu)",
                      l->name.c_str(), rows, z_at + job_z(l, rows), ws->z_len, cnt_at + l->n / 128, ws->counters_len);
@@ -917,6 +926,7 @@ static bool mlp_chain_fits(const fe_exl3_linear *g, const fe_exl3_linear *u, con
     if (!g || !u || !d || !ws || ws->chain_off || !g->kern->opt.mlp_chain || g->kern->opt.handoff_fenced) return false;
     if (g->kern != u->kern || g->kern != d->kern || g->bits != u->bits || g->bits != d->bits) return false;
     if (g->k != u->k || g->n != u->n || d->k != g->n) return false;
+    if (!gemv_reaches(g) || !gemv_reaches(u) || !gemv_reaches(d)) return false;
     if (rows < 1 || rows > 16 || rows > ws->max_rows || y_dtype < 0 || y_dtype > 3) return false;
     // every stage rotates its own input inside the launch: (row, 128-channel block) pairs a program. As separate launches
     // that pays up to 16 pairs (fused_rotation_fits); inside the one launch up to 48, i.e. up to 4 rows on the 27B-shaped

@@ -24,23 +24,27 @@ struct Exl3Packed {
         LaneWords<BITS> w;
         LaneWindows<BITS> win;
     };
-    u32x4 rs;
-    uint32_t voff[LOADS], step;
+    // A trellis may hold 4 GB and more (its row of tiles of a k tile or its column block is far below that): the resource starts at the
+    // k tile that is loaded, with a 64-bit address, and ends where that k tile's last run of words does.
+    uint64_t base;
+    uint32_t voff[LOADS], step, span;
     __device__ __forceinline__ void setup(const uint32_t* trellis, uint32_t n, uint32_t k, uint32_t n0, uint32_t stride_k, uint32_t stride_nb) {
-        const uint32_t lane = threadIdx.x & 63, wave = threadIdx.x >> 6, nbs = n / 128;
-        rs = g8_rsrc(trellis, (k / 16) * (n / 16) * 32 * BITS);
-        step = 16 * stride_k;
+        const uint32_t lane = threadIdx.x & 63, wave = threadIdx.x >> 6;
+        const uint32_t nb0 = n0 / 128, blocks = n / 128 - nb0 < BLOCKS ? n / 128 - nb0 : BLOCKS;  // (an odd block count: the last tile holds one)
+        const uint64_t b = (uint64_t)(trellis + (size_t)nb0 * stride_nb);
+        base = (uint64_t)(uint32_t)__builtin_amdgcn_readfirstlane((uint32_t)(b >> 32)) << 32 | (uint32_t)__builtin_amdgcn_readfirstlane((uint32_t)b);
+        step = 16 * stride_k, span = __builtin_amdgcn_readfirstlane(4 * ((blocks - 1) * stride_nb + 3 * stride_k + 64 * BITS));
 #pragma unroll
         for (int j = 0; j < LOADS; j++) {
             const uint32_t at = (wave + 8 * j) % PIECES * 1024 + lane * 16;  // (fewer pieces than wavefronts: some are moved twice)
             const uint32_t ks = at / (256 * BITS) % 4;
-            uint32_t nb = n0 / 128 + at / (1024 * BITS);
-            nb = nb < nbs ? nb : nbs - 1;  // an odd block count: the last tile decodes its first block twice
+            uint32_t nb = at / (1024 * BITS);
+            nb = nb < blocks ? nb : blocks - 1;  // the last tile of an odd block count decodes its first block twice
             voff[j] = 4 * (nb * stride_nb + ks * stride_k) + at % (256 * BITS);
         }
     }
     __device__ __forceinline__ void issue(uint32_t kt, uint32_t dst, int j, uint32_t wave) const {
-        g8_load_lds16(rs, dst + (wave + 8 * j) % PIECES * 1024, voff[j], kt * step);
+        g8_load_lds16(g8_rsrc((const void*)(base + (uint64_t)(uint32_t)__builtin_amdgcn_readfirstlane(kt) * step), span), dst + (wave + 8 * j) % PIECES * 1024, voff[j], 0);
     }
     __device__ __forceinline__ Words read(const unsigned char* st) const {
         const uint32_t lane = threadIdx.x & 63, wave = threadIdx.x >> 6, tile = (BLOCKS == 2 ? wave : wave & 3) * 8 + (lane >> 3);

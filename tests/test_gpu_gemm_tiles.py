@@ -98,3 +98,63 @@ def test_small_tiles_of_the_nvfp4_swiglu_front(inter, k, m):
         kern.set_option("gemm_splits", 8)
         kern.set_option("gemm_tile", 0)
         kern.set_option("gemm_pieces", 0)
+
+
+@pytest.mark.parametrize("strips", [True, False])
+def test_trellis_of_4_gb_and_more(strips):
+    """Byte offsets into a trellis of 2^32 bytes and a few column blocks: every tile of the prefill GEMM, both schedules, and the decode into
+    tiles give the first, a middle and the last column blocks the bits of linears that hold these blocks alone. The decode GEMV, which
+    addresses a trellis by 32 bits, refuses it, one linear, a group or an MLP block."""
+    import torch
+    from ferrite_amd import exl3
+    from ferrite_amd._lib import FeError
+    k, n, bits, m = 16384, 262144 + 384, 8, 70
+    kt, nb, tile = k // 16, n // 128, 8 * 8 * bits  # words of the 8 tiles of a column block and k step
+    gen = torch.Generator(device="cuda")
+    gen.manual_seed(7)
+    words = torch.empty(k * n // 32 * bits, dtype=torch.int32, device="cuda")
+    for part in words.chunk(8):
+        part.random_(-(1 << 31), 1 << 31, generator=gen)
+    assert words.numel() * 4 > 1 << 32
+    suh = torch.ones(k, dtype=torch.float16, device="cuda")
+    svh = (torch.rand(n, generator=gen, device="cuda") + 0.5).to(torch.float16) / 128
+    x = torch.randn(m, k, generator=gen, device="cuda").to(torch.bfloat16)
+    kern = exl3.Kernels.load()
+
+    def linear(w, cols, sv):
+        view = exl3.Exl3View(k, cols, bits, w.data_ptr(), suh.data_ptr(), sv.data_ptr(), strips)
+        lin = exl3.Linear.from_view(kern, "w", view, exl3.Linear.plan_for(k, cols, bits, exl3.default_blocks(exl3.cu_count())))
+        lin.keep = (w, sv)
+        return lin
+
+    def forward(lin, out=exl3.Dtype.Bf16):
+        y = torch.zeros((m, lin.n), dtype=torch.bfloat16, device="cuda")
+        lin.forward(x, exl3.Dtype.Bf16, y, out, m, exl3.Workspace([lin], m))
+        torch.cuda.synchronize()
+        return y
+
+    whole = linear(words, n, svh)
+    try:
+        for option, value in (("gemm_tile", 1), ("gemm_tile", 2), ("gemm_tile", 3), ("hat_rows", 65)):
+            kern.set_option("gemm_splits", 1)
+            kern.set_option("gemm_sk", 0)
+            kern.set_option(option, value)
+            y = forward(whole)
+            for b0, b1 in ((0, 2), (1024, 1026), (nb - 3, nb)):
+                w = words.view(nb, kt * tile)[b0:b1] if strips else words.view(kt, nb, tile)[:, b0:b1]
+                want = forward(linear(w.contiguous(), 128 * (b1 - b0), svh[128 * b0:128 * b1].contiguous()))
+                assert want.float().abs().amax(dim=0).min() > 0  # (no column of zeros: what reads past a wrapped size give)
+                assert torch.equal(y[:, 128 * b0:128 * b1], want), (option, value, b0)
+    finally:
+        for option, value in (("gemm_tile", 0), ("hat_rows", 3072), ("gemm_splits", 8), ("gemm_sk", 1)):
+            kern.set_option(option, value)
+    down = linear(words, n, svh)
+    ws = exl3.Workspace([whole, down], m)
+    y = torch.full((m, n), 2.0, dtype=torch.bfloat16, device="cuda")
+    for rows in (1, 8, 17, 64):
+        with pytest.raises(FeError, match="4 GB"):
+            whole.forward(x, exl3.Dtype.Bf16, y, exl3.Dtype.Bf16, rows, ws)
+        with pytest.raises(FeError, match="4 GB"):
+            exl3.forward_group([whole, down], x, exl3.Dtype.Bf16, [y, y], exl3.Dtype.Bf16, rows, ws)
+    torch.cuda.synchronize()
+    assert (y == 2.0).all()
