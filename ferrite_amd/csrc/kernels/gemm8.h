@@ -33,20 +33,30 @@ struct G8Tile {
 };
 
 // One wavefront moves 64 x 16 (4) bytes, lane l's from rs + voff + soff to LDS byte dst + 16 (4) l; dst and soff are uniform.
-// Not counted by the compiler's own waits: callers wait with g8_loads_wait.
+// Not counted by the compiler's own waits: callers wait with g8_loads_wait. What the compiler does not see inside such a statement is
+// its hazards: a buffer load needs five wait states after a vector instruction (a v_readfirstlane) has written a scalar register
+// that it reads, and one after m0. So the offset passes through a scalar move, which waits for it and is m0's wait state, and the
+// LDS byte goes into m0 as an operand: the compiler writes that register and knows what it holds. (The resource comes from scalar code
+// or stands long before the load; tests/test_code_objects.py checks the built code.)
 __device__ __forceinline__ void g8_load_lds16(u32x4 rs, uint32_t dst, uint32_t voff, uint32_t soff) {
-    asm volatile("s_mov_b32 m0, %0\n\ts_nop 0\n\tbuffer_load_dwordx4 %1, %2, %3 offen lds" ::"s"(__builtin_amdgcn_readfirstlane(dst)), "v"(voff), "s"(rs),
-                 "s"(__builtin_amdgcn_readfirstlane(soff))
+    uint32_t at;
+    asm volatile("s_mov_b32 %0, %4\n\tbuffer_load_dwordx4 %2, %3, %0 offen lds"
+                 : "=&s"(at)
+                 : "{m0}"(__builtin_amdgcn_readfirstlane(dst)), "v"(voff), "s"(rs), "s"(__builtin_amdgcn_readfirstlane(soff))
                  : "memory");
 }
 __device__ __forceinline__ void g8_load_lds16_nt(u32x4 rs, uint32_t dst, uint32_t voff, uint32_t soff) {
-    asm volatile("s_mov_b32 m0, %0\n\ts_nop 0\n\tbuffer_load_dwordx4 %1, %2, %3 offen nt lds" ::"s"(__builtin_amdgcn_readfirstlane(dst)), "v"(voff), "s"(rs),
-                 "s"(__builtin_amdgcn_readfirstlane(soff))
+    uint32_t at;
+    asm volatile("s_mov_b32 %0, %4\n\tbuffer_load_dwordx4 %2, %3, %0 offen nt lds"
+                 : "=&s"(at)
+                 : "{m0}"(__builtin_amdgcn_readfirstlane(dst)), "v"(voff), "s"(rs), "s"(__builtin_amdgcn_readfirstlane(soff))
                  : "memory");
 }
 __device__ __forceinline__ void g8_load_lds4(u32x4 rs, uint32_t dst, uint32_t voff, uint32_t soff) {
-    asm volatile("s_mov_b32 m0, %0\n\ts_nop 0\n\tbuffer_load_dword %1, %2, %3 offen lds" ::"s"(__builtin_amdgcn_readfirstlane(dst)), "v"(voff), "s"(rs),
-                 "s"(__builtin_amdgcn_readfirstlane(soff))
+    uint32_t at;
+    asm volatile("s_mov_b32 %0, %4\n\tbuffer_load_dword %2, %3, %0 offen lds"
+                 : "=&s"(at)
+                 : "{m0}"(__builtin_amdgcn_readfirstlane(dst)), "v"(voff), "s"(rs), "s"(__builtin_amdgcn_readfirstlane(soff))
                  : "memory");
 }
 // All but the N youngest of the wavefront's vector memory operations are done, and its LDS operations are.

@@ -31,12 +31,29 @@ def test_library_exports_every_declared_symbol():
     assert sorted(_lib.SYMBOLS) == names
 
 
+def test_inline_assembly_tells_the_compiler_about_m0():
+    """A load into LDS takes its LDS byte from m0. The statement names m0 as an operand, so that the compiler writes it; none writes it in
+    its text, behind the compiler's back."""
+    kernels = os.path.join(ROOT, "ferrite_amd", "csrc", "kernels")
+    loads = 0
+    for f in sorted(os.listdir(kernels)):
+        text = open(os.path.join(kernels, f)).read()
+        for a in re.findall(r"\basm\b(?: volatile)?\((.*?)\);", text, flags=re.S):
+            leading = re.match(r'\s*((?:"(?:[^"\\]|\\.)*"\s*)*)', a)
+            template = leading.group(1) if leading else ""
+            assert "m0" not in template, (f, a)
+            if " lds" in template:
+                loads += 1
+                assert '"{m0}"(' in a, (f, a)
+    assert loads >= 3
+
+
 def test_embedded_code_objects_are_gfx950_elf():
     import subprocess
     out = subprocess.run(["nm", "-D", "--defined-only", os.path.join(ROOT, "ferrite_amd", "libferrite_amd.so")],
                          stdout=subprocess.PIPE, text=True).stdout
     # the code objects are private data of the library; check them through the build directory instead
-    for k in ("k_exl3", "k_fp4", "k_route", "k_bf16"):
+    for k in ("k_exl3", "k_exl3_gemm", "k_fp4", "k_route", "k_bf16"):
         p = os.path.join(ROOT, "ferrite_amd", "_build", k + ".hsaco")
         if os.path.exists(p):
             head = open(p, "rb").read(20)
