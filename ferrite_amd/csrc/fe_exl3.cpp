@@ -69,6 +69,7 @@ struct fe_exl3_options {
     // linear's own partition; 2, 4, 8 shorter programs, which end the one launch sooner at one row and cost the two-launch
     // form of the call time from 8 rows on (FE_EXL3_CHAIN_DOWN_UNITS)
     uint32_t chain_down_units = 0;
+    uint32_t gemv_pairs = 1;       // 17..64 rows: two programs a workgroup: 0 never, 1 by the rule, 2 always (tests)
     uint32_t handoff_fenced = 0;   // 1..16 rows through the kernels whose hand-off uses release / acquire fences (a slow cross-check)
     uint32_t mlp_chain = 1;        // the decode MLP (gate, up, down) as one launch where it applies (FE_EXL3_NO_CHAIN=1: off)
     uint32_t chain_rot_pairs = 48; // (row, 128-channel block) pairs a program rotates at most inside the one-launch MLP (FE_EXL3_CHAIN_ROT_PAIRS)
@@ -82,7 +83,7 @@ struct fe_exl3_kernels {
     fe_function_t rot_in = nullptr, rot_in_group = nullptr, probe_v4 = nullptr;
     fe_function_t probe_decode[3] = {nullptr, nullptr, nullptr};  // 3, 4, 5 bits
     fe_function_t gemvb[6] = {};                                  // the decode GEMV for 1..16 rows, [bits slot]
-    fe_function_t gemvw[6][3] = {};                               // for 17..64 rows, [bits slot][row groups - 2]
+    fe_function_t gemvw[6][3][2] = {};                            // for 17..64 rows, [bits slot][row groups - 2][programs a workgroup - 1]
     fe_function_t gemvb_fenced[6] = {};                           // the same for 1..16 rows with the fenced hand-off
     fe_function_t mlp[6] = {};                                    // the decode MLP in one launch, [bits slot]
     uint32_t cus = 0;
@@ -176,9 +177,11 @@ int fe_exl3_kernels_load(fe_exl3_kernels **out) {
         get(&k->gemvb[i], nm);
         if (!c) c = fe_hip_func_set_max_dyn_lds(k->gemvb[i], 84 * 1024);
         for (int rg = 2; rg <= 4; rg++) {
-            snprintf(nm, sizeof nm, "exl3_gemvw_b%d_r%d", kBits[i], rg);
-            get(&k->gemvw[i][rg - 2], nm);
-            if (!c) c = fe_hip_func_set_max_dyn_lds(k->gemvw[i][rg - 2], 84 * 1024);
+            for (int per = 1; per <= 2; per++) {
+                snprintf(nm, sizeof nm, "exl3_gemvw_b%d_r%d%s", kBits[i], rg, per == 2 ? "_pairs" : "");
+                get(&k->gemvw[i][rg - 2][per - 1], nm);
+                if (!c) c = fe_hip_func_set_max_dyn_lds(k->gemvw[i][rg - 2][per - 1], 84 * 1024);
+            }
         }
         snprintf(nm, sizeof nm, "exl3_gemvb_b%d_r1_fenced", kBits[i]);
         get(&k->gemvb_fenced[i], nm);
@@ -253,6 +256,7 @@ int fe_exl3_kernels_set_option(fe_exl3_kernels *k, const char *name, uint32_t va
     else if (nm == "gemm_tile") k->tile.force_tile = value;
     else if (nm == "gemm_pieces") k->tile.force_pieces = value;
     else if (nm == "mlp_chain") o.mlp_chain = value;
+    else if (nm == "gemv_pairs") o.gemv_pairs = value;
     else if (nm == "handoff_fenced") o.handoff_fenced = value;
     else if (nm == "chain_spin") o.chain_spin = value;
     else if (nm == "chain_perm") o.chain_perm = value;
@@ -277,12 +281,26 @@ int fe_exl3_plan_for(uint32_t k, uint32_t n, uint32_t bits, uint32_t blocks, fe_
     int cus = 0;
     if (fe_hip_cu_count(&cus) || cus <= 0) cus = 256;  // planning without a device: the MI355X count
     uint32_t occ = blocks ? std::min(5u, std::max(1u, (blocks + (uint32_t)cus / 2) / (uint32_t)cus)) : 4, wk = 4;
+    const uint32_t units = (k / 128) * (n / 128), nb = n / 128;
     if (!env_is("FE_EXL3_UNTUNED", "1")) {
+        bool tuned = false;
         for (const FeTunedPlan &t : kFeTunedPlans)
-            if (t.k == k && t.n == n && t.bits == bits && t.cus == (uint32_t)cus) occ = t.occ, wk = t.min_units;
+            if (t.k == k && t.n == n && t.bits == bits && t.cus == (uint32_t)cus) occ = t.occ, wk = t.min_units, tuned = true;
+        // Fewer units than CUs, where most CUs would have no program at all: runs of two. us at 1 / 16 / 64 rows, four -> two: 1024 x
+        // 1024 (64 units) 7.4 -> 6.6, 10.3 -> 9.1, 13.5 -> 12.2; 2816 x 1024 (176) 8.8 -> 7.2, 12.0 -> 10.5, 16.9 -> 17.3; 2048 x 2048
+        // (256) 8.1 -> 7.8, 10.7 -> 10.8, 14.8 -> 17.4; 5120 x 1024 (320) 8.2 -> 8.6, 11.7 -> 12.5, 18.6 -> 22.5. The 1024 / 2816 MLP
+        // block at 1 row 16.8 -> 13.7.
+        if (!tuned && units < (uint32_t)cus) wk = 2;
+        // Wider than deep (gate, up) with more than two but fewer than four programs a CU: two. Such linears come in pairs, whose
+        // programs then fill the CUs once. us, 4 bits, one linear / gate and up at 1 and at 40 rows: 5120 x 8704, 680 programs 13.3 / 20.5, 25.0 / 36.3,
+        // 512 programs 12.5 / 18.3, 22.2 / 34.3; 5120 x 7168, 560: 12.8 / 20.2, 25.2 / 33.4, 512: 12.0 / 16.4, 22.6 / 32.1; 4096 x 11008, 688: 13.2 / 20.5, 23.8 / 36.4, 512:
+        // 13.8 / 19.6, 23.4 / 33.7 (one such linear alone is the loser, 0.6 us up to 8 rows). Of four programs a CU and more all four, which
+        // hide each other's loads where one linear runs alone (5120 x 17408, 512 -> 1024 programs: 1, 2, 16 rows 20.5 -> 18.2, 21.9 -> 19.1, 26.9 -> 25.0; gate
+        // and up 30.9 -> 30.7, 33.3 -> 32.3, 42.2 -> 41.8) and from 17 rows on run in pairs (programs_per); at 8 bits, with twice the bytes in flight,
+        // they gain nothing: 1, 5, 16 rows 23.9 -> 24.3, 26.6 -> 28.8, 32.4 -> 32.8.
+        if (!tuned && n > k && occ == 4 && units / wk > 2 * (uint32_t)cus && (bits == 8 || units / wk < 4 * (uint32_t)cus)) occ = 2;
     }
     occ = env_u32("FE_EXL3_OCC", occ), wk = std::max(1u, env_u32("FE_EXL3_MIN_UNITS", wk));  // tuning runs
-    const uint32_t units = (k / 128) * (n / 128), nb = n / 128;
     const uint32_t programs = std::max(1u, std::min(occ * (uint32_t)cus, units / wk));
     *out = fe_exl3_plan{(programs + nb - 1) / nb, wk, 3, occ};
     return 0;
@@ -304,11 +322,7 @@ int fe_exl3_plan_parse(const char *s, fe_exl3_plan *out) {
 // partition). Never more programs than units.
 static uint32_t plan_programs(const fe_exl3_kernels *kern, const fe_exl3_plan &p, uint32_t k, uint32_t n) {
     const uint32_t units = (k / 128) * (n / 128);
-    // Runs of four units at least (plan_for): shorter ones leave more partial sums than they save time. With fewer units than CUs,
-    // where most CUs would have no program at all, runs of two instead: us at 1 / 16 / 64 rows, four -> two: 1024 x 1024 (64 units)
-    // 7.4 -> 6.6, 10.3 -> 9.1, 13.5 -> 12.2; 2816 x 1024 (176) 8.8 -> 7.2, 12.0 -> 10.5, 16.9 -> 17.3; 2048 x 2048 (256) 8.1 -> 7.8, 10.7 ->
-    // 10.8, 14.8 -> 17.4; 5120 x 1024 (320) 8.2 -> 8.6, 11.7 -> 12.5, 18.6 -> 22.5. The 1024 / 2816 MLP block at 1 row 16.8 -> 13.7.
-    const uint32_t wk = p.ver == 3 && p.wk == 4 && units < kern->cus ? 2 : std::max(p.wk, 1u);
+    const uint32_t wk = std::max(p.wk, 1u);
     uint32_t progs;
     if (p.ver <= 1)
         progs = n / 128 * std::max(p.sk, 1u);
@@ -316,12 +330,6 @@ static uint32_t plan_programs(const fe_exl3_kernels *kern, const fe_exl3_plan &p
         progs = std::max(p.sk, 1u);
     else
         progs = (p.occ ? p.occ : 4) * std::max(kern->cus, 1u), progs = std::min(progs, units / wk);
-    // Wider than deep (gate, up): two programs a CU where a plan asks for four. Such linears come in pairs, whose programs
-    // fill the CUs together, and every program leaves its partial sums of every row in memory: 1024 programs of 64 rows wrote
-    // and read 38 MB beside 45 MB of weights. 5120 x 17408 at 4 bits, gate + up + down: 1..16 rows the same, 40 rows 95 -> 87 us,
-    // 64 rows 117 -> 104. One such linear launched alone pays at few rows: 1 row 19.3 -> 20.4, 16 rows 25.3 -> 26.6, 40 rows 33.6 -> 31.1, 64 rows
-    // 40.8 -> 35.1 (65536 columns: 48.3 -> 47.7 .. 81.8 -> 78.5). (A down projection keeps its shorter runs: it is the tail of the one-launch MLP.)
-    if (p.ver == 3 && p.occ == 4 && n > k) progs = std::min(progs, 2 * std::max(kern->cus, 1u));
     return std::max(1u, std::min(progs, units));
 }
 
@@ -602,19 +610,21 @@ static int launch_gemm(const fe_exl3_linear *l, fe_stream_t s, fe_devptr_t xh, f
         });
 }
 
-// The GEMV can rotate its own input: every program rotates the channels of its own run, (row, 128-channel block) pairs,
-// 8 at a time, so every column block repeats the rotation of its K range. Measured on 5120 x 17408: one launch wins up
-// to a few rows, the separate rotation launch from about 8 rows on.
 static uint32_t units_per_program(const fe_exl3_linear *l, uint32_t programs) {
     const uint32_t units = (l->k / 128) * (l->n / 128);
     return (units + programs - 1) / programs;
 }
 
+// The GEMV can rotate its own input: every program rotates the channels of its own run, (row, 128-channel block) pairs, 8 at a time,
+// in front of its loop, so every column block repeats the rotation of its K range. A launch for the rotation costs about 2 us at any
+// of these row counts, a row of the rotation inside the GEMV about 0.4 us: one launch against two, us, 1 / 4 / 5 / 6 / 8 rows: 5120 x 5120 (runs of
+// 4 units) 10.6 / 12.3 / 13.1 / 13.7 / 15.0 against 12.6 / 13.1 / 13.6 / 13.6 / 13.9; 17408 x 5120 (8) 19.0 / 21.6 / 22.5 / 23.5 / 25.8 against
+// 21.6 / 22.1 / 22.6 / 22.7 / 23.3; gate and up of 5120 x 17408 (6) 30.5, 32.0, 33.5, 35.1 at 1 .. 4 rows against 32.5, 32.9, 33.2, 33.4. Up to 16
+// pairs every one of them gains.
 static bool fused_rotation_fits(const fe_exl3_linear *l, uint32_t rows) {
     const fe_exl3_options &o = l->kern->opt;
     if (!o.fused_rot || rows < 1 || rows > 16) return false;
-    const uint32_t units = (l->k / 128) * (l->n / 128);
-    return rows * ((units + l->programs - 1) / l->programs) <= o.fused_rot_pairs;
+    return rows * units_per_program(l, l->programs) <= o.fused_rot_pairs;
 }
 
 // GemvWide<bits, rg>::LDS of k_exl3.hip
@@ -649,6 +659,18 @@ struct RotGroupArgs {  // RotGroup
 // any size.
 static bool gemv_reaches(const fe_exl3_linear *l) { return fe_exl3_linear_weight_bytes(l) < (1ull << 32); }
 
+// Programs that a workgroup of the GEMV for 17..64 rows runs as one: two where every linear of the launch has four programs a CU. Every
+// segment leaves its sums of all rows in memory, so from 17 rows on half as many segments pay, while up to 16 rows the programs as
+// they are hide each other's loads (the bits are the same). 5120 x 17408 at 4 bits (1024 programs, 2 x 20 KB of sums each at 40 rows), one linear / gate and up,
+// us, single programs -> pairs: 32 rows 30.1 / 49.2 -> 25.3 / 40.4, 40 rows 35.0 / 57.5 -> 28.0 / 45.8, 64 rows 41.9 / 69.3 -> 34.1 / 54.2; 17408 x 5120 at 6 bits 24 / 40 / 64
+// rows 39.0 / 53.0 / 66.1 -> 32.9 / 40.4 / 48.9.
+static uint32_t programs_per(const fe_exl3_linear *const *ls, size_t count) {
+    const uint32_t opt = ls[0]->kern->opt.gemv_pairs;
+    for (size_t i = 0; i < count; i++)
+        if (!opt || (opt == 1 && ls[i]->programs < 4 * std::max(ls[i]->kern->cus, 1u))) return 1;
+    return 2;
+}
+
 // The decode GEMV for 1..4 linears of one input in one launch, 1..64 rows: member i reads its rotated input at xhs[i]
 // (in.x == 0) or rotates in.x itself and leaves the result at xhs[i]. The caller has checked rows, k and bits.
 static int launch_job(const fe_exl3_linear *const *ls, size_t count, fe_stream_t s, const fe_devptr_t *xhs, const fe_devptr_t *ys,
@@ -665,7 +687,9 @@ static int launch_job(const fe_exl3_linear *const *ls, size_t count, fe_stream_t
     // (measured on gate + up, 4 bits: 34.1 against 35.6 us at 1 row, 36.8 / 38.2 at 4, even at 8, 44.8 / 41.9 at 16, where the
     // longer run's inputs no longer fit the staging buffer in one piece: up to 4 rows; 4-unit programs of 17408 x 5120 sharing a
     // workgroup at 8 / 16 rows: 61.6 / 77.1 us a block against 65.2 / 75.8 without)
+    const bool wide = rows > 16 && !in.x;
     uint32_t fuse = kern->opt.fuse && rows <= 4 ? std::min(4u, std::max(1u, (total + places - 1) / places)) : 1;
+    const uint32_t per = wide ? programs_per(ls, count) : 1;
     uint32_t programs = 0, run_steps = 0;  // (programs: workgroups of the launch)
     size_t z_at = 0, cnt_at = 0;
     char msg[200];
@@ -687,7 +711,7 @@ static int launch_job(const fe_exl3_linear *const *ls, size_t count, fe_stream_t
         m.n = l->n, m.programs = l->programs;
         view_strides(l->view, &m.stride_k, &m.stride_nb);
         g.first[i] = programs;
-        programs += (l->programs + fuse - 1) / fuse;
+        programs += (l->programs + fuse * per - 1) / (fuse * per);
         z_at += job_z(l, rows), cnt_at += l->n / 128;
         const uint32_t units = (l->k / 128) * (l->n / 128);
         m.base = units / l->programs, m.rem = units % l->programs;
@@ -697,10 +721,10 @@ static int launch_job(const fe_exl3_linear *const *ls, size_t count, fe_stream_t
     for (size_t i = count; i <= kGroupMax; i++) g.first[i] = programs;
     uint32_t k = ls[0]->k, mode = (uint32_t)y_dtype;
     const uint32_t bits = ls[0]->bits;
-    if (rows > 16 && !in.x) {
+    if (wide) {
         const uint32_t rg = (rows + 15) / 16;
         void *args[] = {&g, &k, &rows, &mode};
-        return fe_hip_launch(kern->gemvw[bits_slot(bits)][rg - 2], programs, 1, 1, 256, 1, 1, spread_lds(kern, programs, wide_lds(bits, rg)), s, args);
+        return fe_hip_launch(kern->gemvw[bits_slot(bits)][rg - 2][per - 1], programs, 1, 1, 256, 1, 1, spread_lds(kern, programs, wide_lds(bits, rg)), s, args);
     }
     // staged inputs: the whole run where the LDS budget holds it for `rows` rows, else chunks of a multiple of 4 load steps
     const uint32_t red = rows * kRedPitch * 4;

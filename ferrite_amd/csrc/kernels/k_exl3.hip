@@ -208,8 +208,8 @@ extern "C" __global__ __launch_bounds__(128) void exl3_rot_in_group(RotGroup g, 
 // round by round, the CUs' shares differ by at most one unit. (Spreading the longer runs evenly over the program numbers
 // is worse: their period can divide the CU count, and then a CU gets only long runs or only short ones.) A run may start and end inside a column block, so a block's sum is assembled from segments: each program
 // leaves the partial sums of its segment of block nb in z[program + nb] and bumps the block's arrival counter; the
-// program that arrives last adds the segments in program order (the order does not depend on who is last: deterministic),
-// applies the output rotation and re-arms the counter. The partition depends on (k, n, programs) only, never on the
+// program that arrives last adds the segments, those of programs 2 j and 2 j + 1 to each other first and the pairs in program order
+// (so that gemv_wide_body can run a pair as one workgroup; the order does not depend on who is last: deterministic), applies the output rotation and re-arms the counter. The partition depends on (k, n, programs) only, never on the
 // row count: row r of a batch has the bits of the single-row call. Inside a program: 4 wavefronts owning 2 of the
 // block's 8 tiles each, the rotated inputs of the run staged in LDS (rotated here when src.x is set), four load steps in
 // flight per lane. Several linears of one input share a launch: each member's programs are exactly those of its own
@@ -353,6 +353,7 @@ __device__ __forceinline__ void gemvb_body(const GemvMember& mb, uint32_t p0, ui
     (void)stamp_base;
 #endif
     constexpr uint32_t tw = 8 * BITS;
+    constexpr bool PAIRS = CHAIN == 1;  // (in the grouped launches: 0.2 us slower for one linear, 0.2 us faster for gate and up)
     constexpr int DEPTH = 4;  // load steps in flight per lane (5 and 6 measured 2..5 % slower, 8 10 %: 22.9 against 20.7 us)
     constexpr int GROUP = 8;  // steps of straight-line code per loop iteration (a multiple of DEPTH)
     const uint32_t tid = threadIdx.x, lane = tid & 63, wave = tid >> 6;
@@ -528,16 +529,27 @@ __device__ __forceinline__ void gemvb_body(const GemvMember& mb, uint32_t p0, ui
 
     // The segment of column block fnb that ends here: its sums meet in LDS, and then either are the block's sums (the
     // block lies in this run alone) or go to z for the program that arrives last at the block.
-    auto flush = [&](uint32_t fnb, uint32_t p) {
+    // PAIRS: where the workgroup also runs the other program of a pair in the same block, the first one's sums wait in LDS and leave
+    // with the second's as one segment, which saves a hand-off in the middle of the run (the MLP of 5120 x 17408 in one launch, 1 / 4 rows, us: 3 bits
+    // 45.0 / 51.8 -> 44.1 / 51.1, 4 bits 46.5 / 53.4 -> 45.8 / 52.6).
+    uint32_t pending = 0;
+    auto flush = [&](uint32_t fnb, uint32_t p, bool keep) {
         __syncthreads();  // the previous segment's readers are done with `red`
         // rows 4 g .. 4 g + 3 of A are columns 16 (g >> 1) + 4 (g & 1) + 8 h .. + 3 of the wavefront's 32 (tile g >> 1 of
         // its pair, n = 4 (g & 1) + i + 8 h): a lane's four sums of either half are four neighbouring columns
         float* rp = red + 32 * wave + 16 * (g >> 1) + 4 * (g & 1);
         if (r < m) {  // accumulator column = input row
-            *(f32x4*)(rp + r * GEMV_RED_PITCH) = acc[0];
-            *(f32x4*)(rp + r * GEMV_RED_PITCH + 8) = acc[1];
+            f32x4 *r0 = (f32x4*)(rp + r * GEMV_RED_PITCH), *r1 = (f32x4*)(rp + r * GEMV_RED_PITCH + 8);
+            if (PAIRS && pending) acc[0] = *r0 + acc[0], acc[1] = *r1 + acc[1];
+            *r0 = acc[0], *r1 = acc[1];
         }
         acc[0] = acc[1] = (f32x4){0.f, 0.f, 0.f, 0.f};
+        if (PAIRS && keep) {
+            pending = 1;
+            return;
+        }
+        const uint32_t two = PAIRS ? pending : 0;  // the segment is that of programs p - 1 and p
+        pending = 0;
         __syncthreads();
         FE_STAMP(4);
         const uint32_t col0 = fnb * 128;
@@ -545,7 +557,7 @@ __device__ __forceinline__ void gemvb_body(const GemvMember& mb, uint32_t p0, ui
         const uint32_t cut = rem * (base + 1), ua = fnb * upb, ub = ua + upb - 1;
         const uint32_t first_prog = ua < cut ? udiv_inv(ua, base + 1, mb.inv_base1) : rem + udiv_inv(ua - cut, base, mb.inv_base);
         const uint32_t last_prog = ub < cut ? udiv_inv(ub, base + 1, mb.inv_base1) : rem + udiv_inv(ub - cut, base, mb.inv_base);
-        if (first_prog == last_prog) {
+        if (first_prog + two == last_prog) {
             for (uint32_t row = hw; row < m; row += 8) {
                 f32x4 t = *(const f32x4*)(red + row * GEMV_RED_PITCH + 4 * l32);
                 float v[4] = {t[0], t[1], t[2], t[3]};
@@ -561,7 +573,7 @@ __device__ __forceinline__ void gemvb_body(const GemvMember& mb, uint32_t p0, ui
         //  3. the program whose arrival completes the count reads the segments with agent-scope loads (past its own L2)
         //     after the barrier that publishes last_flag.
         // Every byte that crosses is written through and read through, so no cache write-back or invalidate is needed.
-        float* zseg = mb.z + (size_t)(p + fnb) * m * 128;
+        float* zseg = mb.z + (size_t)(p - two + fnb) * m * 128;
         if constexpr (FENCED) {
             for (uint32_t row = hw; row < m; row += 8)
                 *(f32x4*)(zseg + row * 128 + 4 * l32) = *(const f32x4*)(red + row * GEMV_RED_PITCH + 4 * l32);
@@ -569,32 +581,36 @@ __device__ __forceinline__ void gemvb_body(const GemvMember& mb, uint32_t p0, ui
         } else {
             for (uint32_t row = hw; row < m; row += 8)
                 store_agent_f32x4(zseg + row * 128 + 4 * l32, *(const f32x4*)(red + row * GEMV_RED_PITCH + 4 * l32));
+            if (PAIRS && two)
+                for (uint32_t row = hw; row < m; row += 8) store_agent_f32x4(zseg + (m + row) * 128 + 4 * l32, (f32x4){0.f, 0.f, 0.f, 0.f});
             agent_stores_wait();
         }
         FE_STAMP(5);
         __syncthreads();
         if (tid == 0) {
-            uint32_t old = __hip_atomic_fetch_add(&mb.counters[fnb], 1u, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
-            last_flag = (old == last_prog - first_prog);
+            uint32_t old = __hip_atomic_fetch_add(&mb.counters[fnb], 1u + two, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+            last_flag = (old + two == last_prog - first_prog);
         }
         __syncthreads();
         FE_STAMP(6);
         if (last_flag) {
             if constexpr (FENCED) __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "agent");
             // A half wavefront finishes rows hw, hw + 8, ...: RB of them at a time with SB segments each, 8 or 12 agent-scope
-            // loads in flight (each takes a trip to memory: the trips overlap); every row's segments are added in program
-            // order (as many in flight as the registers hold without costing the kernel a resident wavefront). Up to 8 rows
-            // every half wavefront has at most one row and takes all of the batch from it.
-            const uint32_t nseg = last_prog - first_prog + 1;
+            // loads in flight (each takes a trip to memory: the trips overlap); every row's segments are added pair by pair, in
+            // program order (as many in flight as the registers hold without costing the kernel a resident wavefront). Up to 8 rows
+            // every half wavefront has at most one row and takes all of the batch from it. An odd first program is the second of its
+            // pair: slot 0 is then where its partner, which has no part in this block, would leave its sums, and counts as zero. (What lies
+            // past the last segment reads zero, so the sums need no conditions: 5120 x 5120 at 1 / 4 rows 10.9 / 12.7 -> 10.7 / 12.3 us.)
+            const uint32_t odd = first_prog & 1, slots = last_prog - first_prog + 1 + odd;
             const __amdgpu_buffer_rsrc_t zrs = __builtin_amdgcn_make_buffer_rsrc(
-                (void*)(mb.z + (size_t)(first_prog + fnb) * m * 128), 0, nseg * m * 512, 0x00020000);
+                (void*)(mb.z + (size_t)(first_prog - odd + fnb) * m * 128), 0, slots * m * 512, 0x00020000);
             auto rows_of = [&](auto rb_tag) {
                 constexpr int RB = decltype(rb_tag)::value, SB = (BITS <= 4 ? 12 : 8) / RB;
                 for (uint32_t row0 = hw; row0 < m; row0 += 8 * RB) {
                     float v[RB][4];
 #pragma unroll
                     for (int j = 0; j < RB; j++) v[j][0] = v[j][1] = v[j][2] = v[j][3] = 0.f;
-                    for (uint32_t sp0 = 0; sp0 < nseg; sp0 += SB) {
+                    for (uint32_t sp0 = 0; sp0 < slots; sp0 += SB) {
                         f32x4 t[RB * SB];
 #pragma unroll
                         for (int j = 0; j < RB; j++) {
@@ -604,15 +620,14 @@ __device__ __forceinline__ void gemvb_body(const GemvMember& mb, uint32_t p0, ui
                                 t[j * SB + b] = FENCED ? __builtin_bit_cast(f32x4, __builtin_amdgcn_raw_buffer_load_b128(
                                                              zrs, row * 512 + 16 * l32, (sp0 + b) * m * 512, 0))
                                                        : load_agent_f32x4(zrs, row * 512 + 16 * l32, (sp0 + b) * m * 512);
+                            if (odd > sp0) t[j * SB] = (f32x4){0.f, 0.f, 0.f, 0.f};
                         }
 #pragma unroll
                         for (int j = 0; j < RB; j++)
 #pragma unroll
-                            for (int b = 0; b < SB; b++)
-                                if (sp0 + b < nseg) {
+                            for (int b = 0; b < SB; b += 2)
 #pragma unroll
-                                    for (int e = 0; e < 4; e++) v[j][e] += t[j * SB + b][e];
-                                }
+                                for (int e = 0; e < 4; e++) v[j][e] += t[j * SB + b][e] + t[j * SB + b + 1][e];
                     }
 #pragma unroll
                     for (int j = 0; j < RB; j++) {
@@ -701,7 +716,7 @@ __device__ __forceinline__ void gemvb_body(const GemvMember& mb, uint32_t p0, ui
             i += seg, st += seg;
             const bool block_end = st == spb, run_end = c0 + i == lend;
             if (block_end || run_end) {
-                flush(nb, pl);
+                flush(nb, pl, PAIRS && !block_end && !(pl & 1) && pl + 1 < p0 + np);
                 if (block_end) {
                     nb++, st = 0;
                     if (c0 + i < S) sv = *(const u32x2*)(mb.svh + nb * 128 + 4 * l32);  // the next block's output scales
@@ -790,7 +805,9 @@ GEMVB_FAMILY(8)
 
 // ---- the same GEMV for more rows ------------------------------------------------------------------------------------------
 //
-// 17..64 rows. The programs, their runs, the order of every sum and so the bits are gemvb_body's. What differs is how a program
+// 17..64 rows. The programs, their runs, the order of every sum and so the bits are gemvb_body's. With PER 2 a
+// workgroup runs the programs 2 j and 2 j + 1 as one: where the first's run ends inside a column block its sums step aside, and are
+// added to the second's before they leave as one segment, as the finisher of gemvb_body adds them. What differs is how a program
 // gets its operands and hands its sums over: both grow with the rows while the decode does not. Staging a run's inputs
 // through registers before its first step kept a program of 40 rows waiting for 6 of its 18 us, in chunks of 4 steps, and its
 // sums took 3.5 us more to pass through LDS on their way to z. Here the rotated inputs and the trellis words of a load step go
@@ -806,7 +823,7 @@ struct GemvWide {
     static constexpr int LX = (2 * RG + 3) / 4, LW = (BITS + 3) / 4;  // loads a wavefront issues a step: 1 KB pieces, some twice
     static constexpr int RED = 32 * GEMV_RED_PITCH * 4, LDS = (STAGES > RED ? STAGES : RED) + 16;
 };
-template <int BITS, int RG>
+template <int BITS, int RG, int PER>
 __device__ __forceinline__ void gemv_wide_body(const GemvMember& mb, uint32_t p, uint32_t k, uint32_t m, uint32_t y_mode) {
     typedef GemvWide<BITS, RG> C;
     extern __shared__ __attribute__((aligned(16))) unsigned char lds[];
@@ -837,10 +854,12 @@ __device__ __forceinline__ void gemv_wide_body(const GemvMember& mb, uint32_t p,
         const uint32_t mr = m - 16 * rg < 16 ? m - 16 * rg : 16;
         return (uint32_t)(16 * rg) * 512 + ((h * 16 + wave * 4 + g) * mr + r) * 16;
     };
-    uint32_t u = p * base + (p < rem ? p : rem);
-    const uint32_t uend = u + base + (p < rem ? 1 : 0);
+    auto run_start = [&](uint32_t q) { return q * base + (q < rem ? q : rem); };
+    uint32_t u = run_start(PER * p);
+    const uint32_t uend = run_start(PER * p + PER < mb.programs ? PER * p + PER : mb.programs), mid = run_start(PER * p + 1);
     while (u < uend) {
         const uint32_t nb = u / upb, in = u - nb * upb, units = uend - u < upb - in ? uend - u : upb - in, steps = 2 * units;
+        const uint32_t aside = mid > u && mid < u + units ? 2 * (mid - u) : steps;  // the step at which the second program's run starts
         u += units;
         const uint32_t w0 = nb * mb.stride_nb * 4 + 2 * in * step_bytes, x0 = 2 * in * 128;
         auto issue = [&](uint32_t s, uint32_t slot) {  // past the end: the last step again, never used
@@ -857,7 +876,7 @@ __device__ __forceinline__ void gemv_wide_body(const GemvMember& mb, uint32_t p,
 #pragma unroll
         for (int rg = 0; rg < RG; rg++) acc[rg][0] = acc[rg][1] = (f32x4){0.f, 0.f, 0.f, 0.f};
         uint32_t slot = 0;
-        for (uint32_t s = 0; s < steps; s++) {
+        auto step = [&](uint32_t s) {
             g8_loads_wait<(C::DEPTH - 2) * (C::LX + C::LW)>();
             g8_barrier();
             issue(s + C::DEPTH - 1, slot ? slot - 1 : C::DEPTH - 1);
@@ -886,11 +905,33 @@ __device__ __forceinline__ void gemv_wide_body(const GemvMember& mb, uint32_t p,
                 acc[rg][1] = __builtin_amdgcn_mfma_f32_16x16x32_f16(op[1][1], b1, acc[rg][1], 0, 0, 0);
             }
             slot = slot + 1 == C::DEPTH ? 0 : slot + 1;
+        };
+        if constexpr (PER == 1) {
+            for (uint32_t s = 0; s < steps; s++) step(s);
+        } else {
+            f32x4 hold[RG][2] = {};
+            uint32_t s = 0, stop = aside;
+            for (;;) {
+                do step(s);
+                while (++s < stop);
+                if (s == steps) break;
+#pragma unroll
+                for (int rg = 0; rg < RG; rg++) {
+                    hold[rg][0] = acc[rg][0], hold[rg][1] = acc[rg][1];
+                    acc[rg][0] = acc[rg][1] = (f32x4){0.f, 0.f, 0.f, 0.f};
+                }
+                stop = steps;
+            }
+            if (aside != steps) {
+#pragma unroll
+                for (int rg = 0; rg < RG; rg++) acc[rg][0] = hold[rg][0] + acc[rg][0], acc[rg][1] = hold[rg][1] + acc[rg][1];
+            }
         }
-        // the programs of the block's first and last unit
+        // the programs (pairs) of the block's first and last unit
         const uint32_t cut = rem * (base + 1), ua = nb * upb, ub = ua + upb - 1;
-        const uint32_t first_prog = ua < cut ? udiv_inv(ua, base + 1, mb.inv_base1) : rem + udiv_inv(ua - cut, base, mb.inv_base);
-        const uint32_t last_prog = ub < cut ? udiv_inv(ub, base + 1, mb.inv_base1) : rem + udiv_inv(ub - cut, base, mb.inv_base);
+        uint32_t first_prog = ua < cut ? udiv_inv(ua, base + 1, mb.inv_base1) : rem + udiv_inv(ua - cut, base, mb.inv_base);
+        uint32_t last_prog = ub < cut ? udiv_inv(ub, base + 1, mb.inv_base1) : rem + udiv_inv(ub - cut, base, mb.inv_base);
+        if constexpr (PER == 2) first_prog >>= 1, last_prog >>= 1;
         bool mine = true;
         if (first_prog != last_prog) {  // the hand-off of gemvb_body
             const uint32_t nseg = last_prog - first_prog + 1;
@@ -908,31 +949,47 @@ __device__ __forceinline__ void gemv_wide_body(const GemvMember& mb, uint32_t p,
             __syncthreads();
             mine = *last_flag;
             if (mine) {
-                constexpr int SB = RG == 2 ? 2 : 1;  // segments read together (more take registers, and with them resident programs: slower)
+                // A pair's two segments are read together, up to three row groups at a time (12 loads in flight; more take registers,
+                // and with them resident programs). A program's segments are added in pairs, as in gemvb_body; a pair's own one after the other.
+                constexpr int SET = RG == 4 ? 2 : RG;
+                const uint32_t odd = PER == 2 ? 0 : first_prog & 1, slots = nseg + odd;
                 const __amdgpu_buffer_rsrc_t zrs =
-                    __builtin_amdgcn_make_buffer_rsrc((void*)(mb.z + (size_t)(first_prog + nb) * m * 128), 0, nseg * m * 512, 0x00020000);
-                uint32_t z0[RG], z1[RG];
+                    __builtin_amdgcn_make_buffer_rsrc((void*)(mb.z + (size_t)(first_prog - odd + nb) * m * 128), 0, slots * m * 512, 0x00020000);
 #pragma unroll
-                for (int rg = 0; rg < RG; rg++) {
-                    z0[rg] = 16 * rg + r < m ? zoff(rg, 0) : 0, z1[rg] = 16 * rg + r < m ? zoff(rg, 1) : 0;
-                    acc[rg][0] = acc[rg][1] = (f32x4){0.f, 0.f, 0.f, 0.f};
-                }
-                for (uint32_t sp0 = 0; sp0 < nseg; sp0 += SB) {
-                    f32x4 t[SB][RG][2];
+                for (int r0 = 0; r0 < RG; r0 += SET) {
+                    uint32_t z[SET][2];
 #pragma unroll
-                    for (int b = 0; b < SB; b++)
-#pragma unroll
-                        for (int rg = 0; rg < RG; rg++) {  // (past the last segment: out of range, reads zero)
-                            t[b][rg][0] = load_agent_f32x4(zrs, z0[rg], (sp0 + b) * m * 512);
-                            t[b][rg][1] = load_agent_f32x4(zrs, z1[rg], (sp0 + b) * m * 512);
+                    for (int i = 0; i < SET; i++)
+                        if (r0 + i < RG) {
+                            const bool there = 16 * (r0 + i) + r < m;
+                            z[i][0] = there ? zoff(r0 + i, 0) : 0, z[i][1] = there ? zoff(r0 + i, 1) : 0;
+                            acc[r0 + i][0] = acc[r0 + i][1] = (f32x4){0.f, 0.f, 0.f, 0.f};
                         }
+                    for (uint32_t sp0 = 0; sp0 < slots; sp0 += 2) {
+                        f32x4 t[2][SET][2];
 #pragma unroll
-                    for (int b = 0; b < SB; b++)
-                        if (sp0 + b < nseg) {
+                        for (int b = 0; b < 2; b++)
 #pragma unroll
-                            for (int rg = 0; rg < RG; rg++) acc[rg][0] += t[b][rg][0], acc[rg][1] += t[b][rg][1];
-                        }
+                            for (int i = 0; i < SET; i++)
+                                if (r0 + i < RG) {  // (past the last segment: out of range, reads zero)
+                                    t[b][i][0] = load_agent_f32x4(zrs, z[i][0], (sp0 + b) * m * 512);
+                                    t[b][i][1] = load_agent_f32x4(zrs, z[i][1], (sp0 + b) * m * 512);
+                                }
+#pragma unroll
+                        for (int i = 0; i < SET; i++)
+#pragma unroll
+                            for (int h = 0; h < 2; h++)
+                                if (r0 + i < RG) {
+                                    if (PER == 1 && odd > sp0) t[0][i][h] = (f32x4){0.f, 0.f, 0.f, 0.f};
+                                    if constexpr (PER == 2)
+                                        acc[r0 + i][h] = acc[r0 + i][h] + t[0][i][h] + t[1][i][h];
+                                    else
+                                        acc[r0 + i][h] += t[0][i][h] + t[1][i][h];
+                                }
+                    }
                 }
+                // (vmcnt(0), for the compiler: else it waits in every step of the next segment for the pieces that count as zero)
+                __builtin_amdgcn_s_waitcnt(0x0f70);
                 if (tid == 0) __hip_atomic_store(&mb.counters[nb], 0u, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
             }
         }
@@ -961,14 +1018,16 @@ __device__ __forceinline__ void gemv_wide_body(const GemvMember& mb, uint32_t p,
         }
     }
 }
-#define GEMV_WIDE_KERNEL(BITS, RG)                                                                                    \
-    extern "C" __global__ __launch_bounds__(256, 4) void exl3_gemvw_b##BITS##_r##RG(                         \
-        GemvJob job, uint32_t k, uint32_t m, uint32_t y_mode) {                                                       \
+#define GEMV_WIDE_KERNEL(NAME, BITS, RG, PER)                                                                         \
+    extern "C" __global__ __launch_bounds__(256, 4) void NAME(GemvJob job, uint32_t k, uint32_t m, uint32_t y_mode) { \
         uint32_t i = 0;                                                                                               \
         while (i + 1 < job.count && blockIdx.x >= job.first[i + 1]) i++;                                              \
-        gemv_wide_body<BITS, RG>(job.m[i], blockIdx.x - job.first[i], k, m, y_mode);                                  \
+        gemv_wide_body<BITS, RG, PER>(job.m[i], blockIdx.x - job.first[i], k, m, y_mode);                             \
     }
-#define GEMV_WIDE_FAMILY(BITS) GEMV_WIDE_KERNEL(BITS, 2) GEMV_WIDE_KERNEL(BITS, 3) GEMV_WIDE_KERNEL(BITS, 4)
+#define GEMV_WIDE_ROWS(BITS, RG)                                    \
+    GEMV_WIDE_KERNEL(exl3_gemvw_b##BITS##_r##RG, BITS, RG, 1)        \
+    GEMV_WIDE_KERNEL(exl3_gemvw_b##BITS##_r##RG##_pairs, BITS, RG, 2)
+#define GEMV_WIDE_FAMILY(BITS) GEMV_WIDE_ROWS(BITS, 2) GEMV_WIDE_ROWS(BITS, 3) GEMV_WIDE_ROWS(BITS, 4)
 GEMV_WIDE_FAMILY(2)
 GEMV_WIDE_FAMILY(3)
 GEMV_WIDE_FAMILY(4)

@@ -39,8 +39,8 @@ typedef struct {
 /* Launch plan (Plan, crates/fe-exl3/src/linear.rs:33-43), the reference's plan strings "sk,wk[,ver[,occ]]". The gfx950
  * decode GEMV deals 128-channel x 128-column units of the tensor to its programs in equal contiguous runs; a plan says how
  * many programs. ver 1 (the reference's meaning): sk programs per 128-column block, i.e. sk K splits (needs k / 64
- * divisible by sk). ver 2, 3 (what fe_exl3_plan_for returns): occ programs per CU, each a run of at least wk units (ver 3:
- * of two for the default of four where a tensor has fewer units than the device CUs); sk then records the K splits per column block this amounts to. ver 4: sk programs in all (any partition: tests and tuners). */
+ * divisible by sk). ver 2, 3 (what fe_exl3_plan_for returns): occ programs per CU, each a run of at least wk units; sk then
+ * records the K splits per column block this amounts to. ver 4: sk programs in all (any partition: tests and tuners). */
 typedef struct {
     uint32_t sk, wk, ver, occ;
 } fe_exl3_plan;
@@ -49,15 +49,17 @@ typedef struct fe_exl3_kernels fe_exl3_kernels;     /* Kernels, crates/fe-exl3/s
 typedef struct fe_exl3_linear fe_exl3_linear;       /* Linear, crates/fe-exl3/src/linear.rs:163-176 */
 typedef struct fe_exl3_workspace fe_exl3_workspace; /* Workspace, crates/fe-exl3/src/linear.rs:137-161 */
 
-/* Kernels::load: the embedded gfx950 code object, or the file named by FE_EXL3_HSACO (the reference's FE_EXL3_CUBIN,
- * crates/fe-exl3/src/gpu/mod.rs:88-93). */
+/* Kernels::load: the embedded gfx950 code objects, or the files named by FE_EXL3_HSACO (the decode kernels, rotations, reconstruction and
+ * probes; the reference's FE_EXL3_CUBIN, crates/fe-exl3/src/gpu/mod.rs:88-93) and FE_EXL3_GEMM_HSACO (the prefill GEMMs and the
+ * decode into tiles). */
 int fe_exl3_kernels_load(fe_exl3_kernels **out);
 int fe_exl3_kernels_destroy(fe_exl3_kernels *k);
 /* Switches of the launch paths, by name (the environment variable that sets the same switch when the kernels are loaded):
  * "fused_rot" 0/1 (FE_EXL3_NO_FUSED_ROT), "fused_rot_pairs" (FE_EXL3_FUSED_ROT_PAIRS), "group" 0/1 (FE_EXL3_NO_GROUP),
  * "hat_rows" (FE_EXL3_HAT_ROWS; 0 = never), "lds_pad" 0/1 (FE_EXL3_NO_LDS_PAD), "fuse" 0/1 (FE_EXL3_NO_FUSE), "gemm_group_m" (FE_EXL3_GROUP),
  * "gemm_splits" (FE_GEMM_SPLITS), "gemm_tile" 0..3 (output tile of the prefill GEMM: by the shape, 256 x 256, 128 x 256, 128 x 128) and
- * "gemm_pieces" (pieces of K a forced small tile takes), both for tests, "mlp_chain" 0/1 (FE_EXL3_NO_CHAIN), "chain_spin" (FE_EXL3_CHAIN_SPIN),
+ * "gemm_pieces" (pieces of K a forced small tile takes), both for tests, "gemv_pairs" 0..2 (two programs a workgroup of the decode GEMV for 17..64 rows
+ * never / where the linears have four programs a CU / always; same bits), "mlp_chain" 0/1 (FE_EXL3_NO_CHAIN), "chain_spin" (FE_EXL3_CHAIN_SPIN),
  * "handoff_fenced" 0/1 (the decode GEMV for 1..16 rows with its hand-off between programs written with release / acquire fences
  * at agent scope and plain accesses instead of write-through stores and loads that pass the L2: several times slower, a cross-check), "gemm_sk" 0..3 (FE_GEMM_SK: the stream-K schedule of the prefill GEMM never / where it
  * is the faster one / over all tiles / whole rounds then runs, the last two for tests). forward() reads no environment variable; tests and tuners flip a switch here. Not for
@@ -66,8 +68,10 @@ int fe_exl3_kernels_destroy(fe_exl3_kernels *k);
 int fe_exl3_kernels_set_option(fe_exl3_kernels *k, const char *name, uint32_t value);
 
 /* Linear::plan_for (crates/fe-exl3/src/linear.rs:217-233): the tuned plan of the shape where the table has one for this
- * CU count (plans::tuned; FE_EXL3_UNTUNED=1 skips the table), else the rule: `blocks` is the program target (4 per CU is the
- * default, default_blocks linear.rs:132-134), rounded to whole programs per CU. Honours FE_EXL3_NOSPLIT=1 / FE_EXL3_SPLIT=0. */
+ * CU count (plans::tuned), else the rule: `blocks` is the program target (4 per CU is the default, default_blocks
+ * linear.rs:132-134), rounded to whole programs per CU, with runs of at least four units; of two where a tensor has fewer
+ * units than the device CUs, and two programs a CU instead of four where a tensor wider than deep has fewer than four or 8 bits.
+ * FE_EXL3_UNTUNED=1 skips the table and these two exceptions. Honours FE_EXL3_NOSPLIT=1 / FE_EXL3_SPLIT=0. */
 int fe_exl3_plan_for(uint32_t k, uint32_t n, uint32_t bits, uint32_t blocks, fe_exl3_plan *out);
 /* Plan::parse "sk,wk[,ver[,occ]]" (linear.rs:47-55). */
 int fe_exl3_plan_parse(const char *s, fe_exl3_plan *out);
@@ -152,7 +156,7 @@ int fe_exl3_linear_forward_group_launches(const fe_exl3_linear *const *ls, size_
  * under the first. The wait is bounded ("chain_spin" polls, about a microsecond each): when it runs out the program sets
  * the workspace's chain error word and goes on, the launch still ends normally, and its results are void;
  * fe_exl3_workspace_chain_status reports and clears that. It applies where every program rotates at most
- * "chain_rot_pairs" (32) pairs of (row, 128-channel block) of its own input (up to 4 rows on a 5120 x 17408 MLP), with the
+ * "chain_rot_pairs" (48) pairs of (row, 128-channel block) of its own input (up to 4 rows on a 5120 x 17408 MLP), with the
  * same width, gate and up of one shape, and a workspace created from (at least) these three linears; "mlp_chain" 0
  * (FE_EXL3_NO_CHAIN=1) turns it off.
  * fe_exl3_mlp_forward_launches: 1 if the call is the one launch, else 0. */

@@ -155,6 +155,18 @@ def test_plans():
         Linear.plan_for(100, 128, 4, 1024)
 
 
+def test_plans_state_the_programs_they_run():
+    """occ programs a CU (256 where no device is bound) of at least wk units each is what a plan of version 3 means: the K splits it
+    records are those of that count, for the tuned shapes and for what the rule makes of small and of wide linears."""
+    from ferrite_amd.exl3 import Linear
+    for (k, n, bits), (occ, wk) in {(5120, 17408, 4): (4, 2), (5120, 17408, 5): (3, 8), (5120, 17408, 6): (4, 4), (5120, 17408, 8): (2, 4),
+                                    (5120, 8704, 4): (2, 4), (8704, 5120, 4): (4, 4), (4096, 14336, 4): (2, 4), (2048, 5632, 4): (4, 4),
+                                    (2816, 1024, 3): (4, 2), (1024, 256, 3): (4, 2), (5120, 65536, 3): (4, 4)}.items():
+        p, units, nb = Linear.plan_for(k, n, bits, 1024), (k // 128) * (n // 128), n // 128
+        programs = max(1, min(occ * 256, units // wk))
+        assert (p.ver, p.occ, p.wk, p.sk) == (3, occ, wk, -(-programs // nb)), (k, n, bits)
+
+
 def test_fused_host_linear(oracle):
     from ferrite_amd.fp4 import HostLinear
     rng = np.random.default_rng(0)

@@ -281,6 +281,37 @@ def test_gemv_of_17_to_64_rows_at_its_edges(env, bits, programs, strips):
     assert torch.equal(prompt[0].view(torch.int32), prompt[1].view(torch.int32))
 
 
+@pytest.mark.parametrize("bits,programs", [(2, 24), (3, 23), (4, 13), (5, 9), (6, 2), (8, 7)])
+def test_gemv_of_17_to_64_rows_in_pairs_of_programs(env, bits, programs):
+    """Workgroups of one or two programs (option gemv_pairs), a pair that lies in one column block, ends with it or crosses into the next, an
+    odd last program, pairs of which a block holds one half only: the bits of the single-row call, one linear and two of one input."""
+    torch, exl3, kern = env
+    from ferrite_amd import synth
+    ts = [synth.exl3_tensor(1024, n, bits, 60 + bits + n) for n in (384, 256)]
+    lins = [exl3.Linear.with_plan(kern, exl3.DeviceExl3.upload_strips(t), exl3.Plan(min(p, t.n // 16), 4, 4, 0)) for t, p in zip(ts, (programs, 11))]
+    x = dev_u16(torch, synth.activations(64, 1024, bits))
+    try:
+        kern.set_option("gemv_pairs", 0)
+        ws = exl3.Workspace(lins, 64)
+        one = [torch.zeros((64, l.n), dtype=torch.float32, device="cuda") for l in lins]
+        for l, y in zip(lins, one):
+            for r in range(64):
+                l.forward(x[r:], exl3.Dtype.Bf16, y[r:], exl3.Dtype.F32, 1, ws)
+        for pairs in (0, 2):
+            kern.set_option("gemv_pairs", pairs)
+            for rows in (16, 17, 32, 33, 48, 49, 64):
+                y = run_forward(torch, exl3, lins[0], ws, x, rows, exl3.Dtype.F32)
+                assert torch.equal(y[:rows].view(torch.int32), one[0][:rows].view(torch.int32)), (pairs, rows)
+                ys = [torch.full((64, l.n), float("nan"), dtype=torch.float32, device="cuda") for l in lins]
+                exl3.forward_group(lins, x, exl3.Dtype.Bf16, ys, exl3.Dtype.F32, rows, ws)
+                torch.cuda.synchronize()
+                for y, want in zip(ys, one):
+                    assert torch.equal(y[:rows].view(torch.int32), want[:rows].view(torch.int32)), (pairs, rows)
+                    assert rows == 64 or torch.isnan(y[rows:]).all()
+    finally:
+        kern.set_option("gemv_pairs", 1)
+
+
 def test_plan_for_default_and_determinism_with_shared_workspace(env, oracle):
     """crates/fe-exl3/src/bin/exl3-detcheck.rs:36-70: repeated forwards interleaved with a second linear that shares the
     workspace give identical bits."""

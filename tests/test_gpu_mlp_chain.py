@@ -65,6 +65,33 @@ def test_one_launch_has_the_bits_of_the_two_launches(bits, hidden, inter, rows, 
     assert ws.chain_status() == 0
 
 
+@pytest.mark.parametrize("programs", [576, 515])
+def test_one_launch_whose_front_workgroups_run_two_programs(programs):
+    """More front programs than the CUs hold at once: a workgroup runs two, and hands the sums of two that lie in one column block over as
+    one segment; runs of one and of one or two units, blocks that a pair finishes by itself, blocks of which it holds half."""
+    import torch
+    from ferrite_amd import exl3, synth
+    kern = exl3.Kernels.load()
+    hidden, inter, bits = 1024, 9216, 3
+    ts = [synth.exl3_tensor(hidden, inter, bits, 81), synth.exl3_tensor(hidden, inter, bits, 82), synth.exl3_tensor(inter, hidden, bits, 83)]
+    plans = [exl3.Plan(programs, 1, 4, 4)] * 2 + [exl3.Plan(72, 1, 4, 4)]
+    lins = [exl3.Linear.with_plan(kern, exl3.DeviceExl3.upload_strips(t), p) for t, p in zip(ts, plans)]
+    ws = exl3.Workspace(lins, 5)
+    for rows in (1, 3, 5):
+        x = dev_u16(torch, synth.activations(rows, hidden, rows))
+        kern.set_option("mlp_chain", 0)
+        kern.set_option("fuse", 0)
+        want = [t.clone() for t in run(torch, exl3, lins, x, rows, exl3.Dtype.Bf16, ws)]
+        kern.set_option("mlp_chain", 1)
+        kern.set_option("fuse", 1)
+        assert exl3.mlp_forward_launches(*lins, rows, exl3.Dtype.Bf16, ws) == 1
+        for _ in range(3):
+            got = run(torch, exl3, lins, x, rows, exl3.Dtype.Bf16, ws)
+            torch.cuda.synchronize()
+            assert all(torch.equal(a.view(torch.int16), b.view(torch.int16)) for a, b in zip(got, want)), rows
+    assert ws.chain_status() == 0
+
+
 def test_one_launch_against_the_oracle(oracle):
     """End to end against the CPU path: gate and up by linear_f64 on the bf16 input, SwiGLU in the reference's bf16
     arithmetic, down by linear_f64 on that activation."""
