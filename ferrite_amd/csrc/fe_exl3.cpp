@@ -18,6 +18,7 @@ namespace {
 
 constexpr uint32_t kMaxRowsPerPass = 64;       // 4 row groups of 16
 constexpr uint32_t kHatRows = 3072;            // rows from which the prefill decodes once into fp16 tiles (12 output tile rows)
+constexpr uint32_t kChainRows = 8;             // most rows of the one-launch MLP (mlp_chain_fits)
 constexpr uint32_t kGroupMax = 4;              // FE_EXL3_GROUP_MAX: linears of one launch
 // LDS of one GEMV program (sums of a segment + staged inputs of a chunk of the run): three programs fit a CU's 160 KB. Up
 // to 16 rows a whole run fits in far less; from 17 rows on a larger budget (76 KB: longer chunks, two programs a CU) was
@@ -72,7 +73,7 @@ struct fe_exl3_options {
     uint32_t gemv_pairs = 1;       // 17..64 rows: two programs a workgroup: 0 never, 1 by the rule, 2 always (tests)
     uint32_t handoff_fenced = 0;   // 1..16 rows through the kernels whose hand-off uses release / acquire fences (a slow cross-check)
     uint32_t mlp_chain = 1;        // the decode MLP (gate, up, down) as one launch where it applies (FE_EXL3_NO_CHAIN=1: off)
-    uint32_t chain_rot_pairs = 48; // (row, 128-channel block) pairs a program rotates at most inside the one-launch MLP (FE_EXL3_CHAIN_ROT_PAIRS)
+    uint32_t chain_rot_pairs = 48; // (row, 128-channel block) pairs a program and round rotates at most inside the one-launch MLP (FE_EXL3_CHAIN_ROT_PAIRS)
     uint32_t chain_perm = 1;       // the down stage's workgroups in the order in which their inputs get ready (FE_EXL3_CHAIN_PERM)
     uint32_t chain_spin = 1u << 16;  // polls a program of the down stage waits for the front stage's outputs (FE_EXL3_CHAIN_SPIN)
 };
@@ -614,6 +615,11 @@ static uint32_t units_per_program(const fe_exl3_linear *l, uint32_t programs) {
     const uint32_t units = (l->k / 128) * (l->n / 128);
     return (units + programs - 1) / programs;
 }
+// Programs that follow each other on a CU's places (four) in a launch of `programs`.
+static uint32_t launch_rounds(const fe_exl3_kernels *kern, uint32_t programs) {
+    const uint32_t places = 4 * std::max(kern->cus, 1u);
+    return (programs + places - 1) / places;
+}
 
 // The GEMV can rotate its own input: every program rotates the channels of its own run, (row, 128-channel block) pairs, 8 at a time,
 // in front of its loop, so every column block repeats the rotation of its K range. A launch for the rotation costs about 2 us at any
@@ -952,13 +958,15 @@ static bool mlp_chain_fits(const fe_exl3_linear *g, const fe_exl3_linear *u, con
     if (g->k != u->k || g->n != u->n || d->k != g->n) return false;
     if (!gemv_reaches(g) || !gemv_reaches(u) || !gemv_reaches(d)) return false;
     if (rows < 1 || rows > 16 || rows > ws->max_rows || y_dtype < 0 || y_dtype > 3) return false;
-    // every stage rotates its own input inside the launch: (row, 128-channel block) pairs a program. As separate launches
-    // that pays up to 16 pairs (fused_rotation_fits); inside the one launch up to 48, i.e. up to 4 rows on the 27B-shaped
-    // MLP (measured at 4 bits, cold weights: 4 rows 53.6 us against 56.8 us for rotation and GEMV launches; 8 rows 65.1 / 60.1)
+    // every stage rotates its own input inside the launch, (row, 128-channel block) pairs a program and round of the front stage (as
+    // fused_rotation_fits, but there are two rotations' launches to save). One launch against several, us: 5120 x 17408 at 4 bits (6 units, two rounds) 4 / 5 /
+    // 6 / 8 rows 52.6 / 56.3 / 58.9 / 64.4 against 55.5 / 57.2 / 57.6 / 59.8; 5120 x 8704 (6 units, one round) 6 / 8 / 10 rows 37.6 / 41.1 / 46.2 against 39.7 / 41.3 /
+    // 43.2; 2048 x 5632 (4 units) 6 / 8 / 10 / 12 rows 24.0 / 26.5 / 30.1 / 32.0 against 25.7 / 26.1 / 27.5 / 27.5; 1024 x 2816 (2 units) 8 / 10 rows 21.2 / 24.3 against
+    // 23.2 / 21.6. So up to 8 rows and 48 pairs.
     const fe_exl3_options &o = g->kern->opt;
-    const uint32_t d_units = units_per_program(d, chain_part(d)->programs);
-    if (!o.fused_rot || rows * std::max({units_per_program(g, g->programs), units_per_program(u, u->programs), d_units}) > o.chain_rot_pairs)
-        return false;
+    const uint32_t d_units = units_per_program(d, chain_part(d)->programs), rounds = launch_rounds(g->kern, g->programs + u->programs);
+    const uint32_t f_units = std::max(units_per_program(g, g->programs), units_per_program(u, u->programs));
+    if (!o.fused_rot || rows > kChainRows || rows * std::max(f_units * rounds, d_units) > o.chain_rot_pairs) return false;
     if (d_units > 32) return false;
     if (std::max(g->k, d->k) > ws->max_k || (size_t)2 * rows * g->k * 2 > ws->xh.bytes) return false;
     if (job_z(g, rows) + job_z(u, rows) + chain_z(d, rows) > ws->z_len) return false;

@@ -92,6 +92,27 @@ def test_one_launch_whose_front_workgroups_run_two_programs(programs):
     assert ws.chain_status() == 0
 
 
+def test_one_launch_only_where_its_rotations_cost_less_than_their_launches():
+    """Rows times the longest run up to 48 pairs, the front's once for each round of its programs, and up to 8 rows however short the runs."""
+    from ferrite_amd import exl3, synth
+    kern = exl3.Kernels.load()
+    _, lins = make(exl3, synth, kern, 1024, 2816, 3, 61)  # runs of two units
+    ws = exl3.Workspace(lins, 16)
+    assert [exl3.mlp_forward_launches(*lins, r, exl3.Dtype.Bf16, ws) for r in (1, 8, 9, 16)] == [1, 1, 0, 0]
+    t = [synth.exl3_tensor(2048, 8448, 3, 7), synth.exl3_tensor(2048, 8448, 3, 8), synth.exl3_tensor(8448, 2048, 3, 9)]
+    wide = [exl3.Linear.with_plan(kern, exl3.DeviceExl3.upload_strips(w), exl3.Plan(264, 1, 4, 4)) for w in t]  # runs of four units
+    front = [exl3.Linear.with_plan(kern, exl3.DeviceExl3.upload_strips(w), exl3.Plan(1056 // 4 * 2 + 1, 1, 4, 4)) for w in t[:2]]  # of two, in two rounds
+    ws = exl3.Workspace(wide + front, 16)
+    assert [exl3.mlp_forward_launches(*wide, r, exl3.Dtype.Bf16, ws) for r in (8, 9)] == [1, 0]
+    kern.set_option("chain_rot_pairs", 30)
+    try:  # 7 rows: 28 pairs of the down projection; of the front's runs 14, twice
+        assert [exl3.mlp_forward_launches(front[0], front[1], wide[2], r, exl3.Dtype.Bf16, ws) for r in (7, 8)] == [1, 0]
+        kern.set_option("chain_rot_pairs", 27)
+        assert exl3.mlp_forward_launches(front[0], front[1], wide[2], 7, exl3.Dtype.Bf16, ws) == 0
+    finally:
+        kern.set_option("chain_rot_pairs", 48)
+
+
 def test_one_launch_against_the_oracle(oracle):
     """End to end against the CPU path: gate and up by linear_f64 on the bf16 input, SwiGLU in the reference's bf16
     arithmetic, down by linear_f64 on that activation."""
