@@ -981,7 +981,11 @@ static int launch_mlp(const fe_exl3_linear *g, const fe_exl3_linear *u, const fe
     MlpChainArgs a{};
     const fe_exl3_linear *front[2] = {g, u};
     const fe_devptr_t ys[2] = {yg, yu};
-    const uint32_t places = 4 * std::max(kern->cus, 1u);
+    // Programs a CU: what the plans of the three ask for, of the four that fit. 5120 x 17408 at 5 bits (plans of 3 and 2): 1 / 2 / 3 rows 56.4 / 59.1 /
+    // 62.2 us with three, 57.6 / 60.7 / 63.8 with four; at 4 bits (4, 3) 47.7 / 50.5 / 53.7 and 45.6 / 47.9 / 50.4.
+    uint32_t occ = 0;
+    for (const fe_exl3_linear *l : {g, u, d}) occ = std::max(occ, l->plan.occ ? l->plan.occ : 4);
+    const uint32_t places = std::min(occ, 4u) * std::max(kern->cus, 1u);
     // (as launch_job: consecutive programs of the front stage share a workgroup when they are more than the CUs hold)
     a.fuse1 = kern->opt.fuse && rows <= 4 ? std::min(4u, std::max(1u, (g->programs + u->programs + places - 1) / places)) : 1;
     a.fuse2 = 1;
