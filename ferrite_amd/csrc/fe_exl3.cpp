@@ -690,11 +690,11 @@ static int launch_job(const fe_exl3_linear *const *ls, size_t count, fe_stream_t
     uint32_t total = 0;
     for (size_t i = 0; i < count; i++) total += ls[i]->programs;
     const uint32_t places = 4 * std::max(kern->cus, 1u);
-    // (measured on gate + up, 4 bits: 34.1 against 35.6 us at 1 row, 36.8 / 38.2 at 4, even at 8, 44.8 / 41.9 at 16, where the
-    // longer run's inputs no longer fit the staging buffer in one piece: up to 4 rows; 4-unit programs of 17408 x 5120 sharing a
-    // workgroup at 8 / 16 rows: 61.6 / 77.1 us a block against 65.2 / 75.8 without)
+    // (measured on gate + up, 5120 x 17408, two a workgroup against one: 3 bits 5 / 8 rows 33.3 / 35.3 us against 34.2 / 35.5, 4 bits
+    // 34.0 / 35.9 against 35.3 / 36.6, 6 bits 40.3 / 42.3 against 43.3 / 44.6; at 16 rows 44.8 against 41.9, where the longer run's
+    // inputs no longer fit the staging buffer in one piece: up to 8 rows)
     const bool wide = rows > 16 && !in.x;
-    uint32_t fuse = kern->opt.fuse && rows <= 4 ? std::min(4u, std::max(1u, (total + places - 1) / places)) : 1;
+    uint32_t fuse = kern->opt.fuse && rows <= 8 ? std::min(4u, std::max(1u, (total + places - 1) / places)) : 1;
     const uint32_t per = wide ? programs_per(ls, count) : 1;
     uint32_t programs = 0, run_steps = 0;  // (programs: workgroups of the launch)
     size_t z_at = 0, cnt_at = 0;
@@ -987,7 +987,7 @@ static int launch_mlp(const fe_exl3_linear *g, const fe_exl3_linear *u, const fe
     for (const fe_exl3_linear *l : {g, u, d}) occ = std::max(occ, l->plan.occ ? l->plan.occ : 4);
     const uint32_t places = std::min(occ, 4u) * std::max(kern->cus, 1u);
     // (as launch_job: consecutive programs of the front stage share a workgroup when they are more than the CUs hold)
-    a.fuse1 = kern->opt.fuse && rows <= 4 ? std::min(4u, std::max(1u, (g->programs + u->programs + places - 1) / places)) : 1;
+    a.fuse1 = kern->opt.fuse && rows <= 8 ? std::min(4u, std::max(1u, (g->programs + u->programs + places - 1) / places)) : 1;
     a.fuse2 = 1;
     size_t z_at = 0, cnt_at = 0;
     uint32_t wgs = 0;
