@@ -250,15 +250,17 @@ struct FeGemmTileOptions {
 
 // What a program of each tile takes on one weight form: us a k tile (64; FP8: 128), `full` more of it when all CUs are busy (clock and
 // memory), us a program besides, and how much slower two programs that share a CU (tile 2) are than one alone. Fitted to 770
-// timings a form (MI355X, 80..1536 rows, 2048 x 2048 .. 17408 x 5120, 1..8 pieces; within 6 % for trellis and NVFP4 weights,
-// 10..13 % for bf16 and FP8, whose panels compete for memory). stream_k: what meeting through the workspace adds.
+// timings a form (MI355X, 80..1536 rows, 2048 x 2048 .. 17408 x 5120, 1..8 pieces; most of them within 6 % for trellis and NVFP4 weights,
+// 10..13 % for bf16 and FP8, whose panels compete for memory). stream_k: what meeting through the workspace adds. again: what small
+// tiles in more than one round take more than their rounds add up to (trellis: the programs that come second decode alone; 528 tiles 128 x 128 of
+// 32 k tiles 80 us where the rounds add up to 67).
 struct FeGemmCost {
-    float ktile[3], full[3], fixed[3], shared, stream_k;
+    float ktile[3], full[3], fixed[3], shared, stream_k, again;
 };
-constexpr FeGemmCost kFeCostTrellis = {{1.38f, 1.02f, 0.71f}, {0.12f, 0.07f, 0.08f}, {1.0f, 3.0f, 1.9f}, 1.63f, 48.7f};
-constexpr FeGemmCost kFeCostNvfp4 = {{1.32f, 0.73f, 0.44f}, {-0.07f, 0.05f, 0.09f}, {0.0f, 2.2f, 2.3f}, 1.59f, 44.0f};
-constexpr FeGemmCost kFeCostFp8 = {{1.20f, 0.58f, 0.66f}, {0.09f, 0.46f, 0.21f}, {0.0f, 2.5f, 0.4f}, 1.21f, 36.4f};
-constexpr FeGemmCost kFeCostBf16 = {{1.10f, 0.64f, 0.45f}, {0.22f, 0.43f, 0.41f}, {0.0f, 1.5f, 0.3f}, 1.53f, 53.2f};
+constexpr FeGemmCost kFeCostTrellis = {{1.38f, 1.02f, 0.71f}, {0.12f, 0.07f, 0.08f}, {1.0f, 3.0f, 1.9f}, 1.63f, 48.7f, 1.12f};
+constexpr FeGemmCost kFeCostNvfp4 = {{1.32f, 0.73f, 0.44f}, {-0.07f, 0.05f, 0.09f}, {0.0f, 2.2f, 2.3f}, 1.59f, 44.0f, 1.0f};
+constexpr FeGemmCost kFeCostFp8 = {{1.20f, 0.58f, 0.66f}, {0.09f, 0.46f, 0.21f}, {0.0f, 2.5f, 0.4f}, 1.21f, 36.4f, 1.0f};
+constexpr FeGemmCost kFeCostBf16 = {{1.10f, 0.64f, 0.45f}, {0.22f, 0.43f, 0.41f}, {0.0f, 1.5f, 0.3f}, 1.53f, 53.2f, 1.0f};
 
 // `programs` programs of `ktiles` k tiles each, in rounds of all CUs (tile 2: two a CU).
 inline float fe_gemm_cost(const FeGemmCost &c, uint32_t tile, uint32_t programs, uint32_t ktiles, uint32_t cus) {
@@ -275,7 +277,10 @@ inline float fe_gemm_reduce_cost(uint32_t programs, uint32_t tile) {
 // The rule: with fewer than a few rounds of 256 x 256 tiles, most of the time is CUs without a tile or pieces of K that meet;
 // tiles of half and a quarter the size fill the chip with fewer pieces. They read more operand bytes and run fewer matrix
 // instructions between two barriers (a k tile of them costs more than its share), so they pay only where the fill gains more:
-// the estimate above decides, with 6 % against a small tile for its error. Pieces of at least 8 k tiles, at most as many
+// the estimate above decides, with 6 % against a small tile. The margin is the one that loses least over the estimate's errors, not a bound
+// of them: of 14 row counts on 10 layers in each form the rule took a tile more than 3 % slower than 256 x 256 once (NVFP4, 1536 rows of 8704 x 5120:
+// 133 us against 126); with the errors' 10..13 % as the margin bf16 and FP8 miss a dozen gains (bf16 192 rows of 17408 x 5120 59 -> 67, FP8 777 rows
+// of 5120 x 17408 80 -> 88) and avoid no loss. Pieces of at least 8 k tiles, at most as many
 // programs as run at once when K is cut. Up to 2048 rows, what the estimate was fitted on: beyond, whole rounds of 256 x 256
 // prevail. 5120 x 5120, us, before -> with small tiles: NVFP4 100 rows 31 -> 21, bf16 1000 rows 58 -> 56, FP8 1000 rows 42 -> 30.
 inline FeGemmPlan fe_gemm_plan(uint32_t m, uint32_t n, uint32_t ktiles, uint32_t cus, fe_devptr_t part, size_t part_bytes,
@@ -312,6 +317,7 @@ inline FeGemmPlan fe_gemm_plan(uint32_t m, uint32_t n, uint32_t ktiles, uint32_t
             if (pieces > 1 && tiles * pieces > cus * tile) break;
             float c = fe_gemm_cost(cost, tile, tiles * pieces, (ktiles + pieces - 1) / pieces, cus);
             if (pieces > 1) c += fe_gemm_reduce_cost(tiles * pieces, tile);
+            if (tiles * pieces > cus * tile) c *= cost.again;
             if (1.06f * c < best) take(tile, tiles, pieces), best = 1.06f * c;
         }
     }
