@@ -17,7 +17,10 @@
 namespace {
 
 constexpr uint32_t kMaxRowsPerPass = 64;       // 4 row groups of 16
-constexpr uint32_t kHatRows = 3072;            // rows from which the prefill decodes once into fp16 tiles (12 output tile rows)
+// Rows from which the prefill decodes once into fp16 tiles (9 output tile rows). Decoding in the GEMM against once, us, at 2048 / 2304 / 3072 rows: 5120 x
+// 17408 at 4 bits 377 / 435 / 548 against 364 / 432 / 522, at 8 bits 398 / 454 / 568 against 377 / 446 / 535, 17408 x 5120 387 / 453 / 546 against 394 / 438 / 515, 5120 x
+// 5120 143 / 143 / 172 against 146 / 139 / 165, 2048 x 5632 68.3 / 72.6 / 98.2 against 69.3 / 73.1 / 96.1.
+constexpr uint32_t kHatRows = 2304;
 constexpr uint32_t kChainRows = 8;             // most rows of the one-launch MLP (mlp_chain_fits)
 constexpr uint32_t kGroupMax = 4;              // FE_EXL3_GROUP_MAX: linears of one launch
 // LDS of one GEMV program (sums of a segment + staged inputs of a chunk of the run): three programs fit a CU's 160 KB. Up

@@ -146,7 +146,7 @@ def test_trellis_of_4_gb_and_more(strips):
                 assert want.float().abs().amax(dim=0).min() > 0  # (no column of zeros: what reads past a wrapped size give)
                 assert torch.equal(y[:, 128 * b0:128 * b1], want), (option, value, b0)
     finally:
-        for option, value in (("gemm_tile", 0), ("hat_rows", 3072), ("gemm_splits", 8), ("gemm_sk", 1)):
+        for option, value in (("gemm_tile", 0), ("hat_rows", 2304), ("gemm_splits", 8), ("gemm_sk", 1)):
             kern.set_option(option, value)
     down = linear(words, n, svh)
     ws = exl3.Workspace([whole, down], m)
