@@ -261,10 +261,11 @@ def test_fp4_gemv_agrees_with_the_gemm(env, oracle):
 
 @pytest.mark.parametrize("n,k", [(384, 2048), (128, 256), (1024, 5120)])
 def test_fp4_gemv_over_strips_agrees_with_the_weight_tiles(env, oracle, n, k):
-    """The GEMV over strips of 16 weight rows (a workgroup a strip over all of K, activations staged in LDS, nothing
-    handed between programs; option gemv_strips = 2 takes it wherever it fits, 0 never) against the GEMV over weight tiles
-    and K splits: the same exact products summed in another order; both weight layouts; the residual epilogue; rows past m
-    untouched; repeats bit-equal; and against the f64 reference over the dequantized operands (fp4-check.rs:134-144)."""
+    """The GEMV in programs of some columns over all of K (option gemv_strips nonzero; nothing handed between programs) against the GEMV over
+    weight tiles and K splits (gemv_strips 0): the same exact products summed in another order; both weight layouts; every width of a
+    program (gemv_cols) the same bits; the residual epilogue; rows past m untouched; repeats bit-equal; and against the f64
+    reference over the dequantized operands (fp4-check.rs:134-144). The options of a kernel that is no more, gemv_once and gemv_waves, are
+    accepted and change nothing."""
     torch, fp4, kern = env
     from ferrite_amd import synth
     host = synth.fp4_linear(n, k, 51, input_scale=1.0)
@@ -274,16 +275,14 @@ def test_fp4_gemv_over_strips_agrees_with_the_weight_tiles(env, oracle, n, k):
     wdq = oracle.dequant_fp4(host.codes, host.sf, 1.0)
     try:
         for m in (1, 2, 4, 9, 16):
-            if m * k * 2 > 48 * 1024:
-                continue
             ws = fp4.Workspace(m, k)
             xb = fp4_check_activations(m, k, lin.g, 60 + m)
             xd = dev_u16(torch, xb)
             res = dev_u16(torch, bf16_bits(np.random.default_rng(m).normal(size=(m + 1, n)).astype(np.float32)))
 
-            def run(l, strips, r=None, once=1):
+            def run(l, strips, r=None, cols=0):
                 kern.set_option("gemv_strips", strips)
-                kern.set_option("gemv_once", once)  # (1: every load of a workgroup issued at once, where K allows)
+                kern.set_option("gemv_cols", cols)
                 y = torch.full((m + 1, n), -3.0, dtype=torch.bfloat16, device="cuda")
                 l.forward(kern, ws, y, n, xd, k, m, res=r)
                 torch.cuda.synchronize()
@@ -295,8 +294,10 @@ def test_fp4_gemv_over_strips_agrees_with_the_weight_tiles(env, oracle, n, k):
             assert np.array_equal(strips, run(lin, 2)) and np.array_equal(strips, run(view, 2))
             a, b = bf16_to_f32(strips).astype(np.float64), bf16_to_f32(tiles).astype(np.float64)
             assert (np.abs(a - b) <= np.abs(b) / 128.0 + 1e-30).all(), m
-            looped = bf16_to_f32(run(lin, 2, once=0)).astype(np.float64)  # the looped form: other wavefront counts, other order
-            assert (np.abs(looped - b) <= np.abs(b) / 128.0 + 1e-30).all(), m
+            assert np.array_equal(strips, run(lin, 1, cols=8)) and np.array_equal(strips, run(view, 1, cols=72))
+            kern.set_option("gemv_once", 0)
+            kern.set_option("gemv_waves", 8)
+            assert np.array_equal(strips, run(lin, 1))
             with_res = run(lin, 2, res)
             assert np.array_equal(with_res, bf16_bits(bf16_to_f32(strips) + bf16_to_f32(res.cpu().numpy().view(np.uint16)[:m])))
             codes, sf = oracle.quant_fp4(xb, host.g)
@@ -304,6 +305,7 @@ def test_fp4_gemv_over_strips_agrees_with_the_weight_tiles(env, oracle, n, k):
             assert (np.abs(a - ref) / np.abs(ref).max(axis=1, keepdims=True)).max() < 8e-3, m
     finally:
         kern.set_option("gemv_strips", 1)
+        kern.set_option("gemv_cols", 0)
         kern.set_option("gemv_once", 1)
 
 
