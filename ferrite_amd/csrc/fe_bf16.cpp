@@ -46,6 +46,9 @@ struct fe_bf16_kernels {
 // columns of 17408 at 1 / 16 rows (640 octets of columns on 256 CUs): 2 octets 33.8 / 47.9, 3 octets 27.1 / 33.7, 4 octets
 // 30.0 / 39.4; 8704 columns of 5120 at 1 / 64 rows: 4 octets 20.9 / 43, 5 octets 15.2 / 27. With one or two rows a linear
 // of several octets a CU is better off with programs that start while others run: 17408 columns 27.1 us at 3 octets, 27.7 at 9.
+// (One and two rows as dot products on the vector ALUs would be up to 0.4 us faster at some widths: 5120 columns of 5120 9.7 / 10.1 us against
+// 10.0 / 10.2, 1024 of 5120 3.9 / 4.1 against 4.3 / 4.5; but a row's bits may not depend on the batch, and from three rows on the matrix
+// instruction is far ahead.)
 static uint32_t gemv_cols(uint32_t m, uint32_t n, uint32_t k, uint32_t xo, uint32_t cus, int32_t nc) {
     const uint32_t octets = n / 8;
     uint32_t best = 0;

@@ -23,10 +23,9 @@ constexpr uint32_t kMaxRowsPerPass = 64;       // 4 row groups of 16
 constexpr uint32_t kHatRows = 2304;
 constexpr uint32_t kChainRows = 8;             // most rows of the one-launch MLP (mlp_chain_fits)
 constexpr uint32_t kGroupMax = 4;              // FE_EXL3_GROUP_MAX: linears of one launch
-// LDS of one GEMV program (sums of a segment + staged inputs of a chunk of the run): three programs fit a CU's 160 KB. Up
-// to 16 rows a whole run fits in far less; from 17 rows on a larger budget (76 KB: longer chunks, two programs a CU) was
-// measured slower: 37.8 against 30.9 us a linear at 32 rows on 5120 x 17408; at 64 rows 52.7 against 45.2 once the sums'
-// buffer holds 32 rows at a time
+// LDS of one GEMV program of 1..16 rows and of one of the one-launch MLP (sums of a segment + staged inputs of a chunk of the
+// run): three programs fit a CU's 160 KB. A whole run mostly fits in far less; the budget cuts long runs of many rows into
+// chunks. The programs of 17..64 rows size their own (wide_lds).
 constexpr uint32_t kJobLdsBudget = 53 * 1024;
 constexpr uint32_t kRedPitch = 132;            // GEMV_RED_PITCH
 // Dynamic LDS of the prefill GEMMs by form (256 x 256, its stream-K form, 128 x 256, 128 x 128): the k tiles in flight, two of A and of

@@ -12,7 +12,7 @@ struct FeTunedPlan {
 // clang-format off
 static const FeTunedPlan kFeTunedPlans[] = {
     // MI355X, 256 CUs: us at 1 row / 16 rows of the best candidates (graph-replayed after 40 ms of the same replays, weights
-    // cycled past the caches)
+    // cycled past the caches). With occ 4 5120 x 17408 has 1024 programs; from 17 rows on two of them share a workgroup
     {5120, 17408, 3, 256, 4, 2},  // occ 4 wk 2: 17.6 / 24.2; occ 3..5 wk 8: 18.2 / 23.5
     {17408, 5120, 3, 256, 3, 8},  // occ 3..5 wk 8 (680 programs, 17 a column block): 19.1 / 26.4; occ 3 wk 2: 19.4 / 26.3
     // (gate + up in one launch: occ 4 wk 2 30.7 us at 1 row, 33.5 at 4, 36.0 at 8, 42.3 at 16; occ 3..5 wk 8 32.5 / 35.5 /

@@ -341,7 +341,9 @@ int fe_fp4_linear_quantize(const fe_fp4_linear *l, const fe_fp4_kernels *kern, f
 // a quarter more where a CU holds one at a time and has several) and the starts of its rounds of programs. us at 1 row: 34816 columns
 // of 5120 at 1, 2, .. 6 octets a program 36.9, 24.7, 24.7, 22.1, 23.3, 21.7; 17408 columns 21.8, 15.5, 15.1, 15.4, 13.7, 14.0; 5120 columns
 // of 17408 21.0, 17.6, 14.3, 15.7, 18.9, 19.3. Programs of 72 columns pay where the activations weigh most: 34816 columns at 16 rows
-// 28.8 us against 29.8 at 48 columns; at 1 row 25.6.
+// 28.8 us against 29.8 at 48 columns; at 1 row 25.6. Against the weight tiles (gemv_strips = 0), which are ahead at one width: 5120 columns of
+// 17408 at 8 / 9 / 12 / 16 rows 19.1 / 20.0 / 20.5 / 21.3 us against 18.4 / 18.8 / 19.2 / 19.9. They are not taken there because a row's bits are to
+// be the same at 1 to 16 rows, and at 1 row it is 15.4 against 18.3 (5120 columns of 8704: 1 / 12 rows 10.6 / 13.3 against 13.8 / 14.1).
 static uint32_t wide_cols(uint32_t n, uint32_t xp, uint32_t cus, uint32_t forced) {
     uint32_t best = 0;
     uint64_t least = ~0ull;

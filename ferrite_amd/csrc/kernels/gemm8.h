@@ -6,8 +6,9 @@
 // about 17 cycles a kilobyte where the direct path costs 8. The loads of a k tile are spread evenly over the tile's MFMAs:
 // the address unit takes 16 cycles for each, and a burst of them holds the wavefront's next MFMA back.
 //
-// What the tile loop is bound by is the board's power: the matrix pipe is busy 81 % of the time and the clock settles where
-// the power limit puts it (1.75..1.95 GHz on random operands). So the choices are those that take the least energy a flop:
+// What the tile loop is bound by is the board's power: the matrix pipe is busy 70 % of a bf16 launch of 2048 rows by the
+// counters (first loads, last tiles and the epilogue included) and the clock settles where the power limit puts it
+// (1.75..1.95 GHz on random operands). So the choices are those that take the least energy a flop:
 // the 16x16x32 instruction (half the accumulator traffic a flop of 32x32x16: at the same schedule 98 against 104 us for
 // 4096^3), every operand byte once through LDS. 2048 x 16384 x 5120 bf16: 225 us (1526 TFLOP/s) against 266 us for four
 // wavefronts of 128 x 128 with 32x32x16 and operands staged through registers.
