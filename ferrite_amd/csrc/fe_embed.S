@@ -14,6 +14,12 @@ fe_k_exl3_gemm_hsaco:
     .global fe_k_exl3_gemm_hsaco_end
 fe_k_exl3_gemm_hsaco_end:
     .balign 4096
+    .global fe_k_exl3_rgemm_hsaco
+fe_k_exl3_rgemm_hsaco:
+    .incbin "k_exl3_rgemm.hsaco"
+    .global fe_k_exl3_rgemm_hsaco_end
+fe_k_exl3_rgemm_hsaco_end:
+    .balign 4096
     .global fe_k_fp4_hsaco
 fe_k_fp4_hsaco:
     .incbin "k_fp4.hsaco"

@@ -38,6 +38,13 @@ uint32_t gemm_lds(uint32_t form, uint32_t bits) {
     return std::max(fixed + std::min(6u, std::max(2u, (room - fixed) / stage)) * stage, 68u * 1024);
 }
 constexpr uint32_t kGemmThreads = 512;
+// Dynamic LDS of the GEMM that decodes into registers (RgCfg::LDS): stages of A and of words, and the sums' rows behind the loop.
+uint32_t rgemm_lds(uint32_t bits, uint32_t rg, uint32_t blocks) {
+    const uint32_t bm = 16 * rg, loaders = 4 * blocks, a = (3 - blocks) * ((2 * rg + loaders - 1) / loaders * loaders * 1024);
+    const uint32_t w = 8 * ((bits + 3) / 4) * 1024, st = std::min(4u, 160 * 1024 / (a + w));
+    const uint32_t sw = st * a + (st + 1) * w <= 160 * 1024 ? st + 1 : st, red_rows = blocks == 2 && bm > 128 ? 128 : bm;
+    return std::max(st * a + sw * w, red_rows * blocks * 132 * 4);
+}
 constexpr uint32_t kCuLds = 160 * 1024;        // LDS of a CU
 constexpr size_t kChainStride = 64;            // FE_CHAIN_STRIDE: u32 words between two ready words of the one-launch MLP
 
@@ -72,6 +79,8 @@ struct fe_exl3_options {
     // linear's own partition; 2, 4, 8 shorter programs, which end the one launch sooner at one row and cost the two-launch
     // form of the call time from 8 rows on (FE_EXL3_CHAIN_DOWN_UNITS)
     uint32_t chain_down_units = 0;
+    uint32_t rgemm = 1;            // prompts through the GEMM that decodes into registers: 0 never, 1 by the rule (FE_EXL3_NO_RGEMM=1: never)
+    uint32_t rgemm_form = 0, rgemm_pieces = 0;  // ... column blocks a program (1, 2), pieces of K that every tile takes; 0: by the plan (tests)
     uint32_t gemv_pairs = 1;       // 17..64 rows: two programs a workgroup: 0 never, 1 by the rule, 2 always (tests)
     uint32_t handoff_fenced = 0;   // 1..16 rows through the kernels whose hand-off uses release / acquire fences (a slow cross-check)
     uint32_t mlp_chain = 1;        // the decode MLP (gate, up, down) as one launch where it applies (FE_EXL3_NO_CHAIN=1: off)
@@ -90,9 +99,10 @@ struct fe_exl3_kernels {
     fe_function_t gemvb_fenced[6] = {};                           // the same for 1..16 rows with the fenced hand-off
     fe_function_t mlp[6] = {};                                    // the decode MLP in one launch, [bits slot]
     uint32_t cus = 0;
-    fe_module_t gemm_module = nullptr;
+    fe_module_t gemm_module = nullptr, rgemm_module = nullptr;
     fe_function_t gemm[6][4] = {};        // decode inside the GEMM, by form: 256 x 256, stream-K, 128 x 256, 128 x 128
     fe_function_t gemm_reduce[3] = {};    // by tile
+    fe_function_t rgemm[6][2][6] = {}, rgemm_reduce = nullptr;  // decode into registers, [bits slot][column blocks - 1][row groups / 2 - 3]
     fe_function_t hat_tiles[6] = {};  // trellis -> fp16 weights as the GEMM's LDS images
     fe_function_t gemm_hat[4] = {};   // the GEMM over them, by form
     FeGemmTileOptions tile;           // "gemm_tile", "gemm_pieces"
@@ -204,6 +214,20 @@ int fe_exl3_kernels_load(fe_exl3_kernels **out) {
         for (uint32_t f = 0; f < 4; f++) get_gemm(&k->gemm[i][f], "exl3_gemm_b" + b + form_sfx[f], gemm_lds(f, (uint32_t)kBits[i]));
         get_gemm(&k->hat_tiles[i], "exl3_hat_tiles_b" + b, 0);
     }
+    if (!c) c = fe_load_module(&k->rgemm_module, "FE_EXL3_RGEMM_HSACO", fe_k_exl3_rgemm_hsaco, fe_k_exl3_rgemm_hsaco_end);
+    auto get_rgemm = [&](fe_function_t *f, const std::string &name, uint32_t lds) {
+        if (!c) c = fe_hip_module_get_function(f, k->rgemm_module, name.c_str());
+        if (!c && lds) c = fe_hip_func_set_max_dyn_lds(*f, lds);
+    };
+    for (int i = 0; i < 6; i++) {
+        const std::string b = "exl3_rgemm_b" + std::to_string(kBits[i]);
+        for (uint32_t j = 0; j < 6; j++) {
+            const uint32_t rg = 6 + 2 * j;
+            get_rgemm(&k->rgemm[i][0][j], b + "_r" + std::to_string(rg) + "_k2", rgemm_lds((uint32_t)kBits[i], rg, 1));
+            if (rg >= 10) get_rgemm(&k->rgemm[i][1][j], b + "_r" + std::to_string(rg) + "_k1", rgemm_lds((uint32_t)kBits[i], rg, 2));
+        }
+    }
+    get_rgemm(&k->rgemm_reduce, "exl3_rgemm_reduce", 0);
     for (int f = 0; f < 4; f++) get_gemm(&k->gemm_hat[f], std::string("exl3_gemm_hat") + form_sfx[f], kHatLds[f]);
     for (int i = 0; i < 3; i++) get_gemm(&k->gemm_reduce[i], std::string("exl3_gemm_reduce") + tile_sfx[i], 0);
     fe_exl3_options &o = k->opt;
@@ -216,6 +240,7 @@ int fe_exl3_kernels_load(fe_exl3_kernels **out) {
     o.gemm_group_m = env_u32("FE_EXL3_GROUP", o.gemm_group_m);
     o.gemm_splits = env_u32("FE_GEMM_SPLITS", o.gemm_splits);
     o.gemm_sk = env_u32("FE_GEMM_SK", o.gemm_sk);
+    o.rgemm = env_u32("FE_EXL3_NO_RGEMM", 0) ? 0 : 1;
     o.mlp_chain = env_u32("FE_EXL3_NO_CHAIN", 0) ? 0 : 1;
     o.chain_spin = env_u32("FE_EXL3_CHAIN_SPIN", o.chain_spin);
     o.chain_perm = env_u32("FE_EXL3_CHAIN_PERM", o.chain_perm);
@@ -238,6 +263,7 @@ int fe_exl3_kernels_destroy(fe_exl3_kernels *k) {
     if (!k) return 0;
     if (k->module) fe_hip_module_unload(k->module);
     if (k->gemm_module) fe_hip_module_unload(k->gemm_module);
+    if (k->rgemm_module) fe_hip_module_unload(k->rgemm_module);
     delete k;
     return 0;
 }
@@ -259,6 +285,9 @@ int fe_exl3_kernels_set_option(fe_exl3_kernels *k, const char *name, uint32_t va
     else if (nm == "gemm_tile") k->tile.force_tile = value;
     else if (nm == "gemm_pieces") k->tile.force_pieces = value;
     else if (nm == "mlp_chain") o.mlp_chain = value;
+    else if (nm == "rgemm") o.rgemm = value;
+    else if (nm == "rgemm_form") o.rgemm_form = value;
+    else if (nm == "rgemm_pieces") o.rgemm_pieces = value;
     else if (nm == "gemv_pairs") o.gemv_pairs = value;
     else if (nm == "handoff_fenced") o.handoff_fenced = value;
     else if (nm == "chain_spin") o.chain_spin = value;
@@ -574,9 +603,66 @@ static int launch_decode(const fe_exl3_linear *l, fe_stream_t s, fe_devptr_t hat
     return fe_hip_launch(kern->hat_tiles[bits_slot(l->bits)], nbs, gy, 1, 256, 1, 1, 0, s, dargs);
 }
 
+// mirrors RgJob of k_exl3_rgemm.hip
+struct RgJobArgs {
+    struct Member {
+        fe_devptr_t xh, trellis, svh, y;
+        uint32_t n, stride_k, stride_nb, first;
+    } m[kGroupMax];
+    uint32_t count, k, rows, y_mode, tiles_m, tiles_n, group, full, runs, base, rem, pad;
+    fe_devptr_t part;
+};
+static_assert(sizeof(RgJobArgs) == kGroupMax * 48 + 56, "RgJob layout");
+
+static bool gemv_reaches(const fe_exl3_linear *l);
+
+// Prompts up to kHatRows go through it under the default switches; those that pick the schedule or the tile of the GEMM that passes the
+// decoded weights through LDS (exl3_gemm_b*) pick that GEMM too. It also takes a trellis of 4 GB and more, which this one addresses by 32
+// bits, and what lies beyond kHatRows. Both, us, LDS / registers, 4 bits: an MLP block of 5120 x 17408 at 70 / 203 / 512 / 2048 rows 138 / 200 / 337 / 1060
+// against 99 / 158 / 302 / 1014, of 2048 x 5632 59 / 75 / 99 / 210 against 38 / 50 / 70 / 190; over 120 random single linears of 2 to 8 bits and 65..2048
+// rows the geometric mean is 0.86, the slowest one (16896 x 1920, 1501 rows) 1.16 of the LDS form's time.
+static bool rgemm_takes(const fe_exl3_linear *l, uint32_t rows) {
+    const fe_exl3_kernels *kern = l->kern;
+    const fe_exl3_options &o = kern->opt;
+    return o.rgemm && rows > kMaxRowsPerPass && rows < std::min(kHatRows, o.hat_rows) && !l->hat.bytes && gemv_reaches(l) && !kern->tile.force_tile &&
+           o.gemm_sk == 1 && o.gemm_splits == 8;
+}
+
+static int launch_rgemm(const fe_exl3_linear *const *ls, size_t count, fe_stream_t s, const fe_devptr_t *xhs, const fe_devptr_t *ys, int y_dtype,
+                        uint32_t rows, const fe_exl3_workspace *ws) {
+    const fe_exl3_kernels *kern = ls[0]->kern;
+    const uint32_t k = ls[0]->k, cus = std::max(kern->cus, 1u);
+    if ((uint64_t)rows * k * 2 >= (1ull << 32))
+        return fe_set_error(FE_ERR_UNSUPPORTED, "fe_exl3_linear_gemv_rotated", "rotated input of 4 GB or more");
+    uint32_t ns[kGroupMax];
+    for (size_t i = 0; i < count; i++) ns[i] = ls[i]->n;
+    const FeRgemmPlan p = fe_rgemm_plan(rows, k, ns, (uint32_t)count, cus, ws->part.bytes, kern->opt.rgemm_form, kern->opt.rgemm_pieces);
+    RgJobArgs j{};
+    uint32_t first = 0;
+    for (size_t i = 0; i < count; i++) {
+        const fe_exl3_linear *l = ls[i];
+        RgJobArgs::Member &m = j.m[i];
+        m.xh = xhs[i], m.trellis = l->view.trellis, m.svh = l->view.svh, m.y = ys[i], m.n = l->n, m.first = first;
+        view_strides(l->view, &m.stride_k, &m.stride_nb);
+        first += (l->n / 128 + p.blocks - 1) / p.blocks;
+    }
+    const uint32_t rest = p.tiles_m * p.tiles_n - p.full, steps = rest * p.steps();
+    j.count = (uint32_t)count, j.k = k, j.rows = rows, j.y_mode = (uint32_t)y_dtype, j.tiles_m = p.tiles_m, j.tiles_n = p.tiles_n;
+    j.group = std::min(p.tiles_m, 8u), j.full = p.full, j.runs = p.runs, j.part = ws->part.p;
+    j.base = p.runs ? steps / p.runs : 1, j.rem = p.runs ? steps % p.runs : 0;
+    const uint32_t slot_bits = (uint32_t)bits_slot(ls[0]->bits);
+    void *args[] = {&j};
+    FE_TRY(fe_hip_launch(kern->rgemm[slot_bits][p.blocks - 1][p.rg / 2 - 3], p.full + p.runs, 1, 1, kGemmThreads, 1, 1, rgemm_lds(ls[0]->bits, p.rg, p.blocks), s, args));
+    if (!p.reduce()) return 0;
+    uint32_t bm = 16 * p.rg, blocks = p.blocks, all = p.steps();
+    void *rargs[] = {&j, &bm, &blocks, &all};
+    return fe_hip_launch(kern->rgemm_reduce, rest * blocks * (bm / 8), 1, 1, 256, 1, 1, 0, s, rargs);
+}
+
 static int launch_gemm(const fe_exl3_linear *l, fe_stream_t s, fe_devptr_t xh, fe_devptr_t y, int y_dtype, uint32_t rows,
                        const fe_exl3_workspace *ws) {
     const fe_exl3_kernels *kern = l->kern;
+    if (rgemm_takes(l, rows)) return launch_rgemm(&l, 1, s, &xh, &y, y_dtype, rows, ws);
     uint32_t n = l->n, k = l->k, mode = (uint32_t)y_dtype, stride_k, stride_nb, group = kern->opt.gemm_group_m;
     view_strides(l->view, &stride_k, &stride_nb);
     if ((uint64_t)rows * k * 2 >= (1ull << 32))
@@ -925,6 +1011,25 @@ int fe_exl3_linear_forward_group(const fe_exl3_linear *const *ls, size_t count, 
 }
 
 }  // extern "C"
+
+int fe_exl3_forward_prompt_group(const fe_exl3_linear *const *ls, size_t count, const fe_exl3_kernels *kern, fe_stream_t s, fe_devptr_t x,
+                                 const fe_devptr_t *ys, uint32_t rows, const fe_exl3_workspace *ws, bool *taken) {
+    *taken = false;
+    if (count < 2 || count > kGroupMax || rows > ws->max_rows || !kern->opt.group || ls[0]->k > ws->max_k || count * (size_t)rows * ls[0]->k * 2 > ws->xh.bytes) return 0;
+    for (size_t i = 0; i < count; i++)
+        if (ls[i]->k != ls[0]->k || ls[i]->bits != ls[0]->bits || ls[i]->kern != ls[0]->kern || !rgemm_takes(ls[i], rows)) return 0;
+    *taken = true;
+    RotGroupArgs r{};
+    fe_devptr_t xhs[kGroupMax] = {};
+    for (size_t i = 0; i < count; i++) {
+        xhs[i] = ws->xh.p + i * (size_t)rows * ls[i]->k * 2;
+        r.suh[i] = ls[i]->view.suh, r.xh[i] = xhs[i];
+    }
+    uint32_t mode = 0, k = ls[0]->k;
+    void *args[] = {&r, &x, &mode, &k};
+    FE_TRY(fe_hip_launch(kern->rot_in_group, (k + 511) / 512, rows, (uint32_t)count, 128, 1, 1, 0, s, args));
+    return launch_rgemm(ls, count, s, xhs, ys, FE_DTYPE_BF16, rows, ws);
+}
 
 // mirrors MlpChain of k_exl3.hip
 struct MlpChainArgs {

@@ -21,6 +21,8 @@ extern "C" const unsigned char fe_k_exl3_hsaco[];
 extern "C" const unsigned char fe_k_exl3_hsaco_end[];
 extern "C" const unsigned char fe_k_exl3_gemm_hsaco[];
 extern "C" const unsigned char fe_k_exl3_gemm_hsaco_end[];
+extern "C" const unsigned char fe_k_exl3_rgemm_hsaco[];
+extern "C" const unsigned char fe_k_exl3_rgemm_hsaco_end[];
 extern "C" const unsigned char fe_k_fp4_hsaco[];
 extern "C" const unsigned char fe_k_fp4_hsaco_end[];
 extern "C" const unsigned char fe_k_route_hsaco[];
@@ -77,9 +79,15 @@ struct FeBuf {
 // Allocates nothing. (fe_exl3.cpp; used by fe_exl3_linear_forward_static.)
 struct fe_exl3_linear;
 struct fe_exl3_kernels;
+struct fe_exl3_workspace;
 int fe_exl3_forward_over(const fe_exl3_linear *l, const fe_exl3_kernels *kern, fe_stream_t s, fe_devptr_t x, int x_dtype,
                          fe_devptr_t y, int y_dtype, uint32_t rows, uint32_t max_rows, fe_devptr_t counters,
                          size_t counters_bytes, fe_devptr_t xh, size_t xh_bytes, fe_devptr_t z, size_t z_bytes, const char *fn);
+// Linears of one input (bf16, rows of k) over a prompt in one launch behind one rotation, bf16 out, where the GEMM that decodes into
+// registers takes all of them and the workspace holds their rotated inputs; *taken: whether it was. A member's sums may add in
+// another order than its own forward's (the launch's tiles are spread as one). For the routing layer.
+int fe_exl3_forward_prompt_group(const fe_exl3_linear *const *ls, size_t count, const fe_exl3_kernels *kern, fe_stream_t s, fe_devptr_t x,
+                                 const fe_devptr_t *ys, uint32_t rows, const fe_exl3_workspace *ws, bool *taken);
 // Looks up the static scratch array of fe_exl3_linear_forward_static on the current device and clears its counters
 // (fe_exl3_static.hip); fe_hip_init calls it for the device it binds.
 int fe_exl3_static_setup_current_device();
@@ -322,6 +330,71 @@ inline FeGemmPlan fe_gemm_plan(uint32_t m, uint32_t n, uint32_t ktiles, uint32_t
         }
     }
     return p;
+}
+
+// ---- the GEMM that decodes a trellis into registers (k_exl3_rgemm.hip): how a launch is spread --------------------------------
+// A program takes `blocks` column blocks of 128 and 16 rg rows. The first `full` tiles are computed whole, the steps of the others laid end
+// to end and dealt to `runs` programs in equal runs; pieces of a tile meet through the workspace and a reduce launch.
+struct FeRgemmPlan {
+    uint32_t blocks = 1, rg = 16, tiles_m = 0, tiles_n = 0, full = 0, runs = 0, k = 0;
+    float us = 0;
+    uint32_t steps() const { return k / (blocks == 1 ? 128 : 64); }  // of a tile
+    bool reduce() const { return runs && runs != tiles_m * tiles_n - full; }
+};
+// The rule: the cheapest by an estimate among one or two column blocks a program, the fewest row tiles of 256 rows at most or one more,
+// all tiles whole, or whole rounds of the CUs (or one round fewer) and the rest in one run a CU or in 2, 3, .. runs a tile. A step costs
+// its matrix instructions, or its decode where the rows are few, and more when the chip is full (clock). Fitted to 1400 timings (120 shapes, 2 to
+// 8 bits, 65..2048 rows, both block counts, 1 to 11 pieces a tile): half of them within 6 %, nine tenths within 17 %. What the fit leaves out
+// and the picks showed, they are its underestimates: runs behind whole rounds and runs that cross from one tile to the next take 4 us
+// more, and where several row tiles share their inputs through L2, runs that cross are at different depths of K and lose that. Forced block
+// counts and pieces: for tests.
+inline FeRgemmPlan fe_rgemm_plan(uint32_t rows, uint32_t k, const uint32_t *n, uint32_t count, uint32_t cus, size_t part_bytes, uint32_t force_blocks,
+                                 uint32_t force_pieces) {
+    FeRgemmPlan best;
+    best.us = 1e30f;
+    for (uint32_t blocks = 1; blocks <= 2; blocks++) {
+        if (force_blocks && blocks != force_blocks) continue;
+        for (uint32_t cut_m = (rows + 255) / 256; cut_m <= (rows + 255) / 256 + 1; cut_m++) {
+            FeRgemmPlan p;
+            p.k = k, p.blocks = blocks, p.rg = std::max(((rows + cut_m - 1) / cut_m + 31) / 32 * 2, blocks == 1 ? 6u : 10u);
+            p.tiles_m = (rows + 16 * p.rg - 1) / (16 * p.rg);
+            for (uint32_t i = 0; i < count; i++) p.tiles_n += (n[i] / 128 + blocks - 1) / blocks;
+            const size_t slot = (size_t)blocks * p.rg * 16 * 512;
+            const uint32_t tiles = p.tiles_m * p.tiles_n, all = p.steps(), slots = (uint32_t)(part_bytes / slot);
+            auto step_us = [&](uint32_t programs) {
+                const float fill = std::min(1.0f, (float)programs / (float)cus), rg = (float)p.rg;
+                const float c = std::max(0.74f, 0.325f + 0.075f * rg) * (blocks == 2 ? 0.87f : 1.0f);
+                return c * (1.0f + 0.22f * std::min(1.0f, rg / 13.0f) * std::max(0.0f, (fill - 0.45f) / 0.5f));
+            };
+            auto consider = [&](uint32_t full, uint32_t runs) {
+                const uint32_t rest = tiles - full;
+                if (rest && (!runs || runs > rest * all || runs + rest > slots)) return;
+                float t = (float)((full + cus - 1) / cus) * (2.0f + (float)all * step_us(full));
+                if (rest) {
+                    const uint32_t len = (rest * all + runs - 1) / runs, per = runs / rest;
+                    const bool aligned = per && runs % rest == 0 && all % per == 0;
+                    const uint32_t crossings = aligned ? 0 : (len + all - 2) / all;
+                    const float run = (float)len * step_us(runs);
+                    t += (full ? 6.0f : 2.0f) + run + (float)crossings * (6.0f + (p.tiles_m > 1 ? 0.08f * run : 0.0f));
+                    if (runs != rest) t += 3.0f + 0.28e-6f * (float)slot * (float)(aligned ? runs : runs + rest);
+                }
+                if (t < best.us) best = p, best.full = full, best.runs = rest ? runs : 0, best.us = t;
+            };
+            const uint32_t forced = std::min(tiles * std::min(force_pieces, all), slots > tiles ? slots - tiles : 0);
+            if (force_pieces > 1 && forced > tiles) {
+                consider(0, forced);
+                continue;
+            }
+            consider(tiles, 0);
+            for (uint32_t back = 0; back <= 1 && back <= tiles / cus && !force_pieces; back++) {
+                const uint32_t full = (tiles / cus - back) * cus, rest = tiles - full;
+                if (!rest) continue;
+                consider(full, cus);
+                for (uint32_t s = 2; s * rest <= cus; s++) consider(full, s * rest);
+            }
+        }
+    }
+    return best;
 }
 
 // Launches a plan. gemm(form, programs, sched): form 0 = 256 x 256 one piece a program, 1 = stream-K, 2, 3 = tile 1, 2;

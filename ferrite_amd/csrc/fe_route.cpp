@@ -306,20 +306,27 @@ static int proj_forward(const fe_route_proj *p, const fe_route_ctx *c, uint32_t 
     }
     for (size_t i = first; i < p->lins.size();) {
         // Trellis linears of this input, for a batch the GEMV takes whole in one pass: one grouped launch for up to four of them
-        // (the bits of each linear's own forward). The reference runs them one after the other (model.rs:384-392).
+        // (the bits of each linear's own forward); a prompt through the trellis alone likewise, where its GEMM takes them together. The
+        // reference runs them one after the other (model.rs:384-392).
         size_t j = i;
-        if ((m <= FE_X3_ROWS || (dec >= m && m <= FE_X3_PASS)) && c->x3())
-            while (j < p->lins.size() && j - i < 4 && p->lins[j].first->q && p->lins[j].first->k == lda) j++;
-        if (j - i >= 2) {
-            const fe_exl3_linear *qs[4];
-            fe_devptr_t ys[4];
-            size_t o = off;
-            for (size_t t = i; t < j; t++) {
-                qs[t - i] = p->lins[t].first->q, ys[t - i] = out + o * 2;
-                o += (size_t)m * p->lins[t].first->n;
-            }
+        const bool gemv = m <= FE_X3_ROWS || (dec >= m && m <= FE_X3_PASS);
+        if (c->x3())
+            while (j < p->lins.size() && j - i < 4 && p->lins[j].first->q && p->lins[j].first->k == lda &&
+                   (gemv || trellis_prompt(p->lins[j].first, c, dec, m)))
+                j++;
+        const fe_exl3_linear *qs[4];
+        fe_devptr_t ys[4];
+        size_t o = off;
+        for (size_t t = i; t < j; t++) {
+            qs[t - i] = p->lins[t].first->q, ys[t - i] = out + o * 2;
+            o += (size_t)m * p->lins[t].first->n;
+        }
+        bool together = j - i >= 2;
+        if (together && gemv)
             FE_TRY(fe_exl3_linear_forward_group(qs, j - i, c->xk, c->s, x, FE_DTYPE_BF16, ys, FE_DTYPE_BF16, m, c->xws));
-        } else {
+        else if (together)
+            FE_TRY(fe_exl3_forward_prompt_group(qs, j - i, c->xk, c->s, x, ys, m, c->xws, &together));
+        if (!together) {
             j = i + 1;
             FE_TRY(linear_forward(p->lins[i].first, c, dec, out + off * 2, p->lins[i].first->n, x, lda, m, 0));
         }

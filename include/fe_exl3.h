@@ -50,15 +50,17 @@ typedef struct fe_exl3_linear fe_exl3_linear;       /* Linear, crates/fe-exl3/sr
 typedef struct fe_exl3_workspace fe_exl3_workspace; /* Workspace, crates/fe-exl3/src/linear.rs:137-161 */
 
 /* Kernels::load: the embedded gfx950 code objects, or the files named by FE_EXL3_HSACO (the decode kernels, rotations, reconstruction and
- * probes; the reference's FE_EXL3_CUBIN, crates/fe-exl3/src/gpu/mod.rs:88-93) and FE_EXL3_GEMM_HSACO (the prefill GEMMs and the
- * decode into tiles). */
+ * probes; the reference's FE_EXL3_CUBIN, crates/fe-exl3/src/gpu/mod.rs:88-93), FE_EXL3_GEMM_HSACO (the prefill GEMMs and the
+ * decode into tiles) and FE_EXL3_RGEMM_HSACO (the prefill GEMM that decodes into registers). */
 int fe_exl3_kernels_load(fe_exl3_kernels **out);
 int fe_exl3_kernels_destroy(fe_exl3_kernels *k);
 /* Switches of the launch paths, by name (the environment variable that sets the same switch when the kernels are loaded):
  * "fused_rot" 0/1 (FE_EXL3_NO_FUSED_ROT), "fused_rot_pairs" (FE_EXL3_FUSED_ROT_PAIRS), "group" 0/1 (FE_EXL3_NO_GROUP),
  * "hat_rows" (FE_EXL3_HAT_ROWS; 0 = never), "lds_pad" 0/1 (FE_EXL3_NO_LDS_PAD), "fuse" 0/1 (FE_EXL3_NO_FUSE), "gemm_group_m" (FE_EXL3_GROUP),
  * "gemm_splits" (FE_GEMM_SPLITS), "gemm_tile" 0..3 (output tile of the prefill GEMM: by the shape, 256 x 256, 128 x 256, 128 x 128) and
- * "gemm_pieces" (pieces of K a forced small tile takes), both for tests, "gemv_pairs" 0..2 (two programs a workgroup of the decode GEMV for 17..64 rows
+ * "gemm_pieces" (pieces of K a forced small tile takes), both for tests, "rgemm" 0/1 (FE_EXL3_NO_RGEMM: prompts of 65..2303 rows through the
+ * GEMM that decodes into registers; a forced gemm_tile, another gemm_splits or gemm_sk than the default and kept tiles take the other one),
+ * "rgemm_form" 0..2 and "rgemm_pieces" (its column blocks a program and pieces of K a tile, 0: by its plan; for tests), "gemv_pairs" 0..2 (two programs a workgroup of the decode GEMV for 17..64 rows
  * never / where the linears have four programs a CU / always; same bits), "mlp_chain" 0/1 (FE_EXL3_NO_CHAIN), "chain_spin" (FE_EXL3_CHAIN_SPIN),
  * "handoff_fenced" 0/1 (the decode GEMV for 1..16 rows with its hand-off between programs written with release / acquire fences
  * at agent scope and plain accesses instead of write-through stores and loads that pass the L2: several times slower, a cross-check), "gemm_sk" 0..3 (FE_GEMM_SK: the stream-K schedule of the prefill GEMM never / where it

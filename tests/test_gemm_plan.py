@@ -50,3 +50,40 @@ def test_the_tile_that_was_timed_faster(tmp_path):
     got = [int(v) for v in subprocess.run([exe, *args], stdout=subprocess.PIPE, text=True, check=True).stdout.split()]
     for key, tile in zip(TIMED, got):
         assert tile == TIMED[key], key
+
+
+RGEMM = r"""
+#include <cstdio>
+#include "fe_internal.h"
+// every plan covers its tiles once, within the workspace, with the row groups that kernels exist for
+int main() {
+    unsigned seed = 1;
+    auto rnd = [&](unsigned lo, unsigned hi) { seed = seed * 1664525u + 1013904223u; return lo + (unsigned)((unsigned long long)(seed >> 8) * (hi - lo + 1) >> 24); };
+    for (int i = 0; i < 200000; i++) {
+        const uint32_t rows = rnd(0, 3) ? rnd(65, 2303) : rnd(65, 300), k = 128 * rnd(1, 140), count = rnd(1, 4), cus = rnd(0, 3) ? 256 : rnd(1, 304);
+        uint32_t n[4];
+        for (auto &v : n) v = 128 * rnd(1, 140);
+        const uint32_t form = rnd(0, 3) ? 0 : rnd(1, 2), pieces = rnd(0, 3) ? 0 : rnd(1, 12);
+        const size_t part = rnd(0, 9) ? (size_t)512 * 262144 : (size_t)rnd(0, 64) * 262144;
+        const FeRgemmPlan p = fe_rgemm_plan(rows, k, n, count, cus, part, form, pieces);
+        const uint32_t tiles = p.tiles_m * p.tiles_n, rest = tiles - p.full;
+        uint32_t tn = 0;
+        for (uint32_t j = 0; j < count; j++) tn += (n[j] / 128 + p.blocks - 1) / p.blocks;
+        bool ok = p.us < 1e29f && (p.blocks == 1 || p.blocks == 2) && (!form || p.blocks == form) && p.rg % 2 == 0 && p.rg <= 16 && p.rg >= (p.blocks == 1 ? 6u : 10u);
+        ok = ok && p.tiles_n == tn && p.tiles_m * 16 * p.rg >= rows && (p.tiles_m - 1) * 16 * p.rg < rows && p.full <= tiles && p.k == k;
+        ok = ok && (rest == 0) == (p.runs == 0) && p.runs <= rest * p.steps();
+        ok = ok && (!rest || (size_t)(p.runs + rest) * p.blocks * p.rg * 16 * 512 <= part);
+        if (!ok) return printf("%u x %u x %u: %u %u\n", rows, k, n[0], form, pieces), 1;
+    }
+    return 0;
+}
+"""
+
+
+def test_every_plan_of_the_register_gemm_covers_its_tiles(tmp_path):
+    src = tmp_path / "rgemm.cpp"
+    src.write_text(RGEMM)
+    exe = str(tmp_path / "rgemm")
+    subprocess.run(["g++", "-std=c++17", "-O1", "-I", os.path.join(ROOT, "ferrite_amd", "csrc"), "-I", os.path.join(ROOT, "include"), str(src), "-o", exe,
+                    "-Wl,--unresolved-symbols=ignore-all"], check=True)
+    subprocess.run([exe], check=True)
