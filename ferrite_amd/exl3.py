@@ -164,6 +164,9 @@ def _stream(s):
     """A stream argument: None = torch's current stream, a torch stream, a raw handle (int) or a ctypes pointer."""
     if s is None:
         import torch
+        raw = getattr(torch._C, "_cuda_getCurrentRawStream", None)  # the handle alone: 0.2 us, the Stream object around it takes 2.6
+        if raw is not None:
+            return C.c_void_p(raw(torch.cuda.current_device()))
         s = torch.cuda.current_stream()
     if isinstance(s, C.c_void_p):
         return s
