@@ -96,6 +96,7 @@ struct fe_exl3_kernels {
     fe_function_t probe_decode[3] = {nullptr, nullptr, nullptr};  // 3, 4, 5 bits
     fe_function_t gemvb[6] = {};                                  // the decode GEMV for 1..16 rows, [bits slot]
     fe_function_t gemvw[6][3][2] = {};                            // for 17..64 rows, [bits slot][row groups - 2][programs a workgroup - 1]
+    fe_function_t gemvw_finish[2] = {}, gemvw_finish_mlp[2] = {};  // their outputs, [programs a workgroup - 1]; gate's and up's with down's rotated input
     fe_function_t gemvb_fenced[6] = {};                           // the same for 1..16 rows with the fenced hand-off
     fe_function_t mlp[6] = {};                                    // the decode MLP in one launch, [bits slot]
     uint32_t cus = 0;
@@ -179,6 +180,10 @@ int fe_exl3_kernels_load(fe_exl3_kernels **out) {
     get(&k->rot_in, "exl3_rot_in");
     get(&k->rot_in_group, "exl3_rot_in_group");
     get(&k->probe_v4, "exl3_probe_v4");
+    for (int per = 0; per < 2; per++) {
+        get(&k->gemvw_finish[per], per ? "exl3_gemvw_finish_pairs" : "exl3_gemvw_finish");
+        get(&k->gemvw_finish_mlp[per], per ? "exl3_gemvw_finish_mlp_pairs" : "exl3_gemvw_finish_mlp");
+    }
     for (int b = 3; b <= 5; b++) {
         char nm[64];
         snprintf(nm, sizeof nm, "exl3_probe_decode_b%d", b);
@@ -721,10 +726,10 @@ static bool fused_rotation_fits(const fe_exl3_linear *l, uint32_t rows) {
     return rows * units_per_program(l, l->programs) <= o.fused_rot_pairs;
 }
 
-// GemvWide<bits, rg>::LDS of k_exl3.hip
+// The stages of GemvWide<bits, rg> of k_exl3.hip
 static uint32_t wide_lds(uint32_t bits, uint32_t rg) {
-    const uint32_t stage = rg * 2048 + bits * 1024, depth = 4 * stage <= 36 * 1024 ? 4 : 3;
-    return std::max(depth * stage, 32 * kRedPitch * 4) + 16;
+    const uint32_t stage = rg * 2048 + bits * 1024;
+    return (4 * stage <= 40 * 1024 ? 4 : 3) * stage;
 }
 
 // LDS for a launch of `programs` workgroups of which a CU can hold four: the dispatcher fills a CU as far as registers and
@@ -756,8 +761,8 @@ static bool gemv_reaches(const fe_exl3_linear *l) { return fe_exl3_linear_weight
 // Programs that a workgroup of the GEMV for 17..64 rows runs as one: two where every linear of the launch has four programs a CU. Every
 // segment leaves its sums of all rows in memory, so from 17 rows on half as many segments pay, while up to 16 rows the programs as
 // they are hide each other's loads (the bits are the same). 5120 x 17408 at 4 bits (1024 programs, 2 x 20 KB of sums each at 40 rows), one linear / gate and up,
-// us, single programs -> pairs: 32 rows 30.1 / 49.2 -> 25.3 / 40.4, 40 rows 35.0 / 57.5 -> 28.0 / 45.8, 64 rows 41.9 / 69.3 -> 34.1 / 54.2; 17408 x 5120 at 6 bits 24 / 40 / 64
-// rows 39.0 / 53.0 / 66.1 -> 32.9 / 40.4 / 48.9.
+// us, single programs -> pairs: 17 rows 25.6 / 41.2 -> 25.5 / 39.2, 40 rows 29.9 / 50.6 -> 28.8 / 45.6, 64 rows 35.0 / 57.9 -> 32.8 / 53.2; 17408 x 5120 at 6 bits 40 / 64
+// rows 34.2 / 43.2 -> 33.4 / 37.9.
 static uint32_t programs_per(const fe_exl3_linear *const *ls, size_t count) {
     const uint32_t opt = ls[0]->kern->opt.gemv_pairs;
     for (size_t i = 0; i < count; i++)
@@ -767,8 +772,9 @@ static uint32_t programs_per(const fe_exl3_linear *const *ls, size_t count) {
 
 // The decode GEMV for 1..4 linears of one input in one launch, 1..64 rows: member i reads its rotated input at xhs[i]
 // (in.x == 0) or rotates in.x itself and leaves the result at xhs[i]. The caller has checked rows, k and bits.
+// down: of a group of gate and up of 17..64 rows, the linear whose rotated input of SwiGLU(gate, up) is left at ws->xh, or null.
 static int launch_job(const fe_exl3_linear *const *ls, size_t count, fe_stream_t s, const fe_devptr_t *xhs, const fe_devptr_t *ys,
-                      int y_dtype, uint32_t rows, const fe_exl3_workspace *ws, const RotInput &in, const char *fn) {
+                      int y_dtype, uint32_t rows, const fe_exl3_workspace *ws, const RotInput &in, const char *fn, const fe_exl3_linear *down = nullptr) {
     GemvJobArgs g{};
     g.count = (uint32_t)count;
     const fe_exl3_kernels *kern = ls[0]->kern;
@@ -817,8 +823,15 @@ static int launch_job(const fe_exl3_linear *const *ls, size_t count, fe_stream_t
     const uint32_t bits = ls[0]->bits;
     if (wide) {
         const uint32_t rg = (rows + 15) / 16;
-        void *args[] = {&g, &k, &rows, &mode};
-        return fe_hip_launch(kern->gemvw[bits_slot(bits)][rg - 2][per - 1], programs, 1, 1, 256, 1, 1, spread_lds(kern, programs, wide_lds(bits, rg)), s, args);
+        void *args[] = {&g, &k, &rows};
+        FE_TRY(fe_hip_launch(kern->gemvw[bits_slot(bits)][rg - 2][per - 1], programs, 1, 1, 256, 1, 1, spread_lds(kern, programs, wide_lds(bits, rg)), s, args));
+        if (down) {
+            fe_devptr_t suh = down->view.suh, xh = ws->xh.p;
+            void *fargs[] = {&g, &k, &rows, &suh, &xh};
+            return fe_hip_launch(kern->gemvw_finish_mlp[per - 1], ls[0]->n / 128, (rows + 7) / 8, 1, 256, 1, 1, 0, s, fargs);
+        }
+        void *fargs[] = {&g, &k, &rows, &mode};
+        return fe_hip_launch(kern->gemvw_finish[per - 1], (uint32_t)cnt_at, (rows + 7) / 8, 1, 256, 1, 1, 0, s, fargs);
     }
     // staged inputs: the whole run where the LDS budget holds it for `rows` rows, else chunks of a multiple of 4 load steps
     const uint32_t red = rows * kRedPitch * 4;
@@ -971,6 +984,10 @@ static bool group_fits(const fe_exl3_linear *const *ls, size_t count, uint32_t r
     return z <= ws->z_len && nb <= ws->counters_len && ls[0]->k <= ws->max_k;
 }
 
+static int forward_group(const fe_exl3_linear *const *ls, size_t count, const fe_exl3_kernels *kern, fe_stream_t s, fe_devptr_t x, int x_dtype,
+                         const fe_devptr_t *ys, int y_dtype, uint32_t rows, const fe_exl3_workspace *ws, bool fused, const fe_exl3_linear *down,
+                         const char *fn);
+
 extern "C" {
 
 int fe_exl3_linear_forward_group_launches(const fe_exl3_linear *const *ls, size_t count, uint32_t rows,
@@ -990,6 +1007,15 @@ int fe_exl3_linear_forward_group(const fe_exl3_linear *const *ls, size_t count, 
         for (size_t i = 0; i < count; i++) FE_TRY(fe_exl3_linear_forward(ls[i], kern, s, x, x_dtype, ys[i], y_dtype, rows, ws));
         return 0;
     }
+    return forward_group(ls, count, kern, s, x, x_dtype, ys, y_dtype, rows, ws, fused, nullptr, fn);
+}
+
+}  // extern "C"
+
+// A group that fits; down: see launch_job.
+static int forward_group(const fe_exl3_linear *const *ls, size_t count, const fe_exl3_kernels *kern, fe_stream_t s, fe_devptr_t x, int x_dtype,
+                         const fe_devptr_t *ys, int y_dtype, uint32_t rows, const fe_exl3_workspace *ws, bool fused, const fe_exl3_linear *down,
+                         const char *fn) {
     if (x_dtype != FE_DTYPE_BF16 && x_dtype != FE_DTYPE_F32) return fe_set_error(FE_ERR_ARG, fn, "x is bf16 or f32");
     if (y_dtype < 0 || y_dtype > 3) return fe_set_error(FE_ERR_ARG, fn, "bad y dtype");
     RotGroupArgs r{};
@@ -1007,10 +1033,8 @@ int fe_exl3_linear_forward_group(const fe_exl3_linear *const *ls, size_t count, 
         void *rargs[] = {&r, &x, &x_mode, &k};
         FE_TRY(fe_hip_launch(kern->rot_in_group, (k + 511) / 512, rows, (uint32_t)count, 128, 1, 1, 0, s, rargs));
     }
-    return launch_job(ls, count, s, xhs, ys, y_dtype, rows, ws, in, fn);
+    return launch_job(ls, count, s, xhs, ys, y_dtype, rows, ws, in, fn, down);
 }
-
-}  // extern "C"
 
 int fe_exl3_forward_prompt_group(const fe_exl3_linear *const *ls, size_t count, const fe_exl3_kernels *kern, fe_stream_t s, fe_devptr_t x,
                                  const fe_devptr_t *ys, uint32_t rows, const fe_exl3_workspace *ws, bool *taken) {
@@ -1151,7 +1175,6 @@ int fe_exl3_mlp_forward(const fe_exl3_linear *gate, const fe_exl3_linear *up, co
         return launch_mlp(gate, up, down, s, x, x_dtype, yg, yu, y, y_dtype, rows, ws);
     const fe_exl3_linear *front[2] = {gate, up};
     const fe_devptr_t ys[2] = {yg, yu};
-    FE_TRY(fe_exl3_linear_forward_group(front, 2, kern, s, x, x_dtype, ys, FE_DTYPE_BF16, rows, ws));
     // down in the partition it has in the one launch (where the GEMV runs and the workspace has the room), so that a row's
     // bits are the same at every row count of this call
     const fe_exl3_linear *dl = down;
@@ -1159,6 +1182,12 @@ int fe_exl3_mlp_forward(const fe_exl3_linear *gate, const fe_exl3_linear *up, co
         const fe_exl3_linear::ChainPart *part = chain_part(down);
         if (part->as_linear && job_z(part->as_linear.get(), rows) <= ws->z_len) dl = part->as_linear.get();
     }
+    bool fused = false;
+    if (rows > 16 && group_fits(front, 2, rows, ws, &fused) && down->k <= ws->max_k) {  // down's input is rotated where gate and up are finished
+        FE_TRY(forward_group(front, 2, kern, s, x, x_dtype, ys, FE_DTYPE_BF16, rows, ws, false, dl, fn));
+        return launch_rows(dl, s, ws->xh.p, y, y_dtype, rows, ws, RotInput{});
+    }
+    FE_TRY(fe_exl3_linear_forward_group(front, 2, kern, s, x, x_dtype, ys, FE_DTYPE_BF16, rows, ws));
     return fe_exl3_linear_forward_swiglu(dl, kern, s, yg, yu, gate->n, y, y_dtype, rows, ws);
 }
 

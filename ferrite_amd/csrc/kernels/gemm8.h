@@ -20,6 +20,9 @@
 // chunks in neighbouring lane groups (perm = identity) the XOR gives them; where lane group g takes chunks 2 g and 2 g + 1
 // (weights expanded from packed codes, 16 codes a lane), perm swaps the two low bits of c.
 #pragma once
+#include <type_traits>
+#include <utility>
+
 #include "gemm_core.h"
 
 #define G8_BK GM_BK
@@ -87,6 +90,16 @@ __device__ __forceinline__ constexpr uint32_t g8_perm(uint32_t c) {
 // between two matrix instructions of a wavefront runs in the pipe's shadow; in a lump it does not (both wavefronts of a SIMD pass the
 // same barrier and would reach the lump together).
 __device__ __forceinline__ constexpr int g8_at(int q, int n, int x0, int x1) { return x0 + q * (x1 - x0) / n; }
+
+// f(0) .. f(N - 1) with constant arguments (the compiler gives up unrolling the largest of these loops by itself)
+template <class F, int... I>
+__device__ __forceinline__ void g8_for_(F f, std::integer_sequence<int, I...>) {
+    (f(std::integral_constant<int, I>{}), ...);
+}
+template <int N, class F>
+__device__ __forceinline__ void g8_for(F f) {
+    g8_for_(f, std::make_integer_sequence<int, N>{});
+}
 
 // Loads that may still be in flight at the barrier of a tile, with LA loads of A (NA stages) issued behind the barrier and LB of W
 // (NW stages) in front of it each tile: those issued after the later one of the next tile's A and W. And at the start of the

@@ -808,27 +808,27 @@ GEMVB_FAMILY(8)
 // 17..64 rows. The programs, their runs, the order of every sum and so the bits are gemvb_body's. With PER 2 a
 // workgroup runs the programs 2 j and 2 j + 1 as one: where the first's run ends inside a column block its sums step aside, and are
 // added to the second's before they leave as one segment, as the finisher of gemvb_body adds them. What differs is how a program
-// gets its operands and hands its sums over: both grow with the rows while the decode does not. Staging a run's inputs
-// through registers before its first step kept a program of 40 rows waiting for 6 of its 18 us, in chunks of 4 steps, and its
-// sums took 3.5 us more to pass through LDS on their way to z. Here the rotated inputs and the trellis words of a load step go
-// straight from memory into LDS, DEPTH - 1 steps ahead, and the sums go to z as the accumulators hold them, whole wavefronts at a
-// time; only the program that finishes a block turns them into rows. Registers stay under 128, so that four programs share a
-// CU. Bound by the partial sums (programs x rows x 512 bytes, written and read once) and by the decode. us, 4 bits, before ->
-// after, 40 rows: 5120 x 5120 23.0 -> 18.5, 2 x (5120 x 17408) 70 -> 55, 17408 x 5120 42.7 -> 35.
+// gets its operands and hands its sums over: both grow with the rows while the decode does not. The rotated inputs and the trellis words of a
+// load step go straight from memory into LDS, DEPTH - 1 steps ahead. Every segment's sums go to z as the accumulators hold them, whole
+// wavefronts at a time, and a launch behind this one (exl3_gemvw_finish*) adds and finishes them with all CUs. (In gemvb_body's hand-off the
+// program that arrives last at a block reads its segments alone, 12 loads in flight: at 40 rows and 4 bits 10.4 of 22.2 us for q + k + v of the
+// 5120 / 17408 layer, 8.0 of 17.6 for o, 7.6 of 42.8 for gate and up, 14.2 of 34.9 for down; now 13.7 + 4.6, 11.3 + 4.7, 36.4 + 6.1, 21.8 + 5, and the launch
+// behind gate and up leaves down's rotated input as well, which took a launch of 5 us.) A layer at 17 / 40 / 64 rows 107 / 138 / 173 -> 99 / 116 / 140 us. Written through
+// (a plain store leaves the launch's end to write 14 MB back: 1 to 2 us more). Registers stay under 128, so that four programs share a
+// CU. Bound by the decode (gate and up: 22 us at the vector ALUs' rate), each program's start, and the products; decoding the next step between the
+// products of this one was measured and changes nothing, the other programs of the CU already fill that time.
 template <int BITS, int RG>
 struct GemvWide {
     static constexpr int X_STAGE = RG * 2048, W_STAGE = 1024 * BITS;
-    static constexpr int DEPTH = 4 * (X_STAGE + W_STAGE) <= 36 * 1024 ? 4 : 3;  // (so that four programs fit a CU, up to 5 bits)
-    static constexpr int W_AT = DEPTH * X_STAGE, STAGES = W_AT + DEPTH * W_STAGE;
+    static constexpr int DEPTH = 4 * (X_STAGE + W_STAGE) <= 40 * 1024 ? 4 : 3;  // (so that four programs fit a CU, up to 5 bits)
+    static constexpr int W_AT = DEPTH * X_STAGE;
     static constexpr int LX = (2 * RG + 3) / 4, LW = (BITS + 3) / 4;  // loads a wavefront issues a step: 1 KB pieces, some twice
-    static constexpr int RED = 32 * GEMV_RED_PITCH * 4, LDS = (STAGES > RED ? STAGES : RED) + 16;
 };
 template <int BITS, int RG, int PER>
-__device__ __forceinline__ void gemv_wide_body(const GemvMember& mb, uint32_t p, uint32_t k, uint32_t m, uint32_t y_mode) {
+__device__ __forceinline__ void gemv_wide_body(const GemvMember& mb, uint32_t p, uint32_t k, uint32_t m) {
     typedef GemvWide<BITS, RG> C;
     extern __shared__ __attribute__((aligned(16))) unsigned char lds[];
-    uint32_t* last_flag = (uint32_t*)(lds + C::LDS - 16);
-    const uint32_t tid = threadIdx.x, lane = tid & 63, wave = __builtin_amdgcn_readfirstlane(tid >> 6), hw = tid >> 5, l32 = tid & 31;
+    const uint32_t tid = threadIdx.x, lane = tid & 63, wave = __builtin_amdgcn_readfirstlane(tid >> 6);
     const uint32_t r = lane & 15, g = lane >> 4;
     const uint32_t n = mb.n, upb = k / 128, base = mb.base, rem = mb.rem;
     const u32x4 xrs = g8_rsrc(mb.xh, m * k * 2), wrs = g8_rsrc(mb.trellis, (k / 16) * (n / 16) * 32 * BITS);
@@ -927,102 +927,104 @@ __device__ __forceinline__ void gemv_wide_body(const GemvMember& mb, uint32_t p,
                 for (int rg = 0; rg < RG; rg++) acc[rg][0] = hold[rg][0] + acc[rg][0], acc[rg][1] = hold[rg][1] + acc[rg][1];
             }
         }
-        // the programs (pairs) of the block's first and last unit
-        const uint32_t cut = rem * (base + 1), ua = nb * upb, ub = ua + upb - 1;
-        uint32_t first_prog = ua < cut ? udiv_inv(ua, base + 1, mb.inv_base1) : rem + udiv_inv(ua - cut, base, mb.inv_base);
-        uint32_t last_prog = ub < cut ? udiv_inv(ub, base + 1, mb.inv_base1) : rem + udiv_inv(ub - cut, base, mb.inv_base);
-        if constexpr (PER == 2) first_prog >>= 1, last_prog >>= 1;
-        bool mine = true;
-        if (first_prog != last_prog) {  // the hand-off of gemvb_body
-            const uint32_t nseg = last_prog - first_prog + 1;
-            unsigned char* zseg = (unsigned char*)(mb.z + (size_t)(p + nb) * m * 128);
+        unsigned char* zseg = (unsigned char*)(mb.z + (size_t)(p + nb) * m * 128);
 #pragma unroll
-            for (int rg = 0; rg < RG; rg++)
-                if (16 * rg + r < m) {
-                    store_agent_f32x4((float*)(zseg + zoff(rg, 0)), acc[rg][0]);
-                    store_agent_f32x4((float*)(zseg + zoff(rg, 1)), acc[rg][1]);
-                }
-            agent_stores_wait();
-            __syncthreads();
-            if (tid == 0)
-                *last_flag = __hip_atomic_fetch_add(&mb.counters[nb], 1u, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT) == nseg - 1;
-            __syncthreads();
-            mine = *last_flag;
-            if (mine) {
-                // A pair's two segments are read together, up to three row groups at a time (12 loads in flight; more take registers,
-                // and with them resident programs). A program's segments are added in pairs, as in gemvb_body; a pair's own one after the other.
-                constexpr int SET = RG == 4 ? 2 : RG;
-                const uint32_t odd = PER == 2 ? 0 : first_prog & 1, slots = nseg + odd;
-                const __amdgpu_buffer_rsrc_t zrs =
-                    __builtin_amdgcn_make_buffer_rsrc((void*)(mb.z + (size_t)(first_prog - odd + nb) * m * 128), 0, slots * m * 512, 0x00020000);
+        for (int rg = 0; rg < RG; rg++) asm volatile("" : "+v"(acc[rg][0]), "+v"(acc[rg][1]));
+        asm volatile("s_nop 15\n\ts_nop 3");  // the last product's wait states, which the compiler does not know of in front of stores in inline assembly
 #pragma unroll
-                for (int r0 = 0; r0 < RG; r0 += SET) {
-                    uint32_t z[SET][2];
-#pragma unroll
-                    for (int i = 0; i < SET; i++)
-                        if (r0 + i < RG) {
-                            const bool there = 16 * (r0 + i) + r < m;
-                            z[i][0] = there ? zoff(r0 + i, 0) : 0, z[i][1] = there ? zoff(r0 + i, 1) : 0;
-                            acc[r0 + i][0] = acc[r0 + i][1] = (f32x4){0.f, 0.f, 0.f, 0.f};
-                        }
-                    for (uint32_t sp0 = 0; sp0 < slots; sp0 += 2) {
-                        f32x4 t[2][SET][2];
-#pragma unroll
-                        for (int b = 0; b < 2; b++)
-#pragma unroll
-                            for (int i = 0; i < SET; i++)
-                                if (r0 + i < RG) {  // (past the last segment: out of range, reads zero)
-                                    t[b][i][0] = load_agent_f32x4(zrs, z[i][0], (sp0 + b) * m * 512);
-                                    t[b][i][1] = load_agent_f32x4(zrs, z[i][1], (sp0 + b) * m * 512);
-                                }
-#pragma unroll
-                        for (int i = 0; i < SET; i++)
-#pragma unroll
-                            for (int h = 0; h < 2; h++)
-                                if (r0 + i < RG) {
-                                    if (PER == 1 && odd > sp0) t[0][i][h] = (f32x4){0.f, 0.f, 0.f, 0.f};
-                                    if constexpr (PER == 2)
-                                        acc[r0 + i][h] = acc[r0 + i][h] + t[0][i][h] + t[1][i][h];
-                                    else
-                                        acc[r0 + i][h] += t[0][i][h] + t[1][i][h];
-                                }
-                    }
-                }
-                // (vmcnt(0), for the compiler: else it waits in every step of the next segment for the pieces that count as zero)
-                __builtin_amdgcn_s_waitcnt(0x0f70);
-                if (tid == 0) __hip_atomic_store(&mb.counters[nb], 0u, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+        for (int rg = 0; rg < RG; rg++)
+            if (16 * rg + r < m) {
+                store_agent_f32x4((float*)(zseg + zoff(rg, 0)), acc[rg][0]);
+                store_agent_f32x4((float*)(zseg + zoff(rg, 1)), acc[rg][1]);
             }
-        }
-        g8_loads_wait<0>();  // (the repeated last steps) the stages are free
-        __syncthreads();
-        if (mine) {  // the block's sums become rows, up to 32 at a time, and are finished
-            float* red = (float*)lds;
-            float* rp = red + 32 * wave + 16 * (g >> 1) + 4 * (g & 1);
-#pragma unroll
-            for (int r0 = 0; r0 < RG; r0 += 2) {
-#pragma unroll
-                for (int i = r0; i < (r0 + 2 < RG ? r0 + 2 : RG); i++)
-                    if (16 * i + r < m) {
-                        *(f32x4*)(rp + (16 * (i - r0) + r) * GEMV_RED_PITCH) = acc[i][0];
-                        *(f32x4*)(rp + (16 * (i - r0) + r) * GEMV_RED_PITCH + 8) = acc[i][1];
-                    }
-                __syncthreads();
-                const uint32_t end = m < 16u * r0 + 32 ? m : 16u * r0 + 32;
-                for (uint32_t row = 16 * r0 + hw; row < end; row += 8) {
-                    const f32x4 t = *(const f32x4*)(red + (row - 16 * r0) * GEMV_RED_PITCH + 4 * l32);
-                    float v[4] = {t[0], t[1], t[2], t[3]};
-                    finish_row(v, l32, mb.svh, nb * 128 + 4 * l32, mb.y, y_mode, (size_t)row * n + nb * 128 + 4 * l32);
-                }
-                __syncthreads();
-            }
-        }
+        g8_loads_wait<2 * RG>();  // the repeated last steps (the stores, 2 RG of every wavefront, may be in flight)
+        g8_barrier();             // the stages are free
     }
 }
+// The sums of row `row`, column block nb: what gemv_wide_body's programs left of them, added in gemvb_body's order (programs 2 j and 2 j + 1 to
+// each other, the pairs in order; PER 2: a segment is a pair's). A lane of the half wavefront gets columns 4 l32 .. + 3.
+template <int PER>
+__device__ __forceinline__ f32x4 wide_row_sums(const GemvMember& mb, uint32_t nb, uint32_t upb, uint32_t m, uint32_t row, uint32_t l32) {
+    const uint32_t base = mb.base, rem = mb.rem, cut = rem * (base + 1), ua = nb * upb, ub = ua + upb - 1;
+    uint32_t first = ua < cut ? udiv_inv(ua, base + 1, mb.inv_base1) : rem + udiv_inv(ua - cut, base, mb.inv_base);
+    uint32_t last = ub < cut ? udiv_inv(ub, base + 1, mb.inv_base1) : rem + udiv_inv(ub - cut, base, mb.inv_base);
+    if constexpr (PER == 2) first >>= 1, last >>= 1;
+    const uint32_t odd = PER == 2 ? 0 : first & 1, slots = last - first + 1 + odd;
+    const __amdgpu_buffer_rsrc_t zrs =
+        __builtin_amdgcn_make_buffer_rsrc((void*)(mb.z + (size_t)(first - odd + nb) * m * 128), 0, slots * m * 512, 0x00020000);
+    // (zoff of gemv_wide_body: column 32 wave + 16 (g >> 1) + 8 h + 4 (g & 1))
+    const uint32_t rg = row / 16, r = row % 16, mr = m - 16 * rg < 16 ? m - 16 * rg : 16, c = l32 & 7;
+    const uint32_t piece = ((c >> 1) & 1) * 16 + (l32 >> 3) * 4 + 2 * (c >> 2) + (c & 1), at = 16 * rg * 512 + (piece * mr + r) * 16;
+    constexpr uint32_t SB = 4;  // segments in flight a lane (8: 0.4 us slower, 18: 2 us at gate and up; a whole wave of rows hides the trips)
+    f32x4 sum = {0.f, 0.f, 0.f, 0.f};
+    for (uint32_t s0 = 0; s0 < slots; s0 += SB) {
+        f32x4 t[SB];
+#pragma unroll
+        for (uint32_t b = 0; b < SB; b++)  // (past the last segment: out of range, reads zero)
+            t[b] = __builtin_bit_cast(f32x4, __builtin_amdgcn_raw_buffer_load_b128(zrs, at, (s0 + b) * m * 512, 0));
+        if (PER == 1 && odd > s0) t[0] = (f32x4){0.f, 0.f, 0.f, 0.f};  // where the first segment's partner, which has no part in the block, would leave its sums
+#pragma unroll
+        for (uint32_t b = 0; b < SB; b += 2) {
+            if constexpr (PER == 2)
+                sum = sum + t[b] + t[b + 1];
+            else
+                sum += t[b] + t[b + 1];
+        }
+    }
+    return sum;
+}
+// Finishes the outputs of a launch of gemv_wide_body: grid (column blocks of all members, ceil(m / 8)), 256 threads, a half wavefront a
+// row. Bound by its one read of the segments, which other XCDs have just written (14 MB for down of 40 rows: 5 us).
+template <int PER>
+__device__ __forceinline__ void wide_finish_body(const GemvJob& job, uint32_t k, uint32_t m, uint32_t y_mode) {
+    const uint32_t l32 = threadIdx.x & 31, row = blockIdx.y * 8 + (threadIdx.x >> 5);
+    uint32_t i = 0, nb = blockIdx.x;
+    while (nb >= job.m[i].n / 128) nb -= job.m[i++].n / 128;
+    const GemvMember& mb = job.m[i];
+    if (row >= m) return;
+    const f32x4 s = wide_row_sums<PER>(mb, nb, k / 128, m, row, l32);
+    float v[4] = {s[0], s[1], s[2], s[3]};
+    finish_row(v, l32, mb.svh, nb * 128 + 4 * l32, mb.y, y_mode, (size_t)row * mb.n + nb * 128 + 4 * l32);
+}
+// The same for gate and up in front of down: both outputs (bf16), and down's rotated input of SwiGLU(gate, up), a 128-channel block of which
+// is a column block of the two. grid (column blocks of one of them, ceil(m / 8)).
+template <int PER>
+__device__ __forceinline__ void wide_finish_mlp_body(const GemvJob& job, uint32_t k, uint32_t m, const uint16_t* suh, uint16_t* xh) {
+    const uint32_t l32 = threadIdx.x & 31, row = blockIdx.y * 8 + (threadIdx.x >> 5), nb = blockIdx.x, c = nb * 128 + 4 * l32, n = job.m[0].n;
+    if (row >= m) return;
+    u32x2 y[2];
+#pragma unroll
+    for (int i = 0; i < 2; i++) {
+        const f32x4 s = wide_row_sums<PER>(job.m[i], nb, k / 128, m, row, l32);
+        float v[4] = {s[0], s[1], s[2], s[3]};
+        fwht128_half_wave(v, l32);
+        const u32x2 sv = *(const u32x2*)(job.m[i].svh + c);
+        v[0] = v[0] * FE_HAD_SCALE * f16_bits_to_f32(sv[0] & 0xffff);  // finish_row's products
+        v[1] = v[1] * FE_HAD_SCALE * f16_bits_to_f32(sv[0] >> 16);
+        v[2] = v[2] * FE_HAD_SCALE * f16_bits_to_f32(sv[1] & 0xffff);
+        v[3] = v[3] * FE_HAD_SCALE * f16_bits_to_f32(sv[1] >> 16);
+        y[i] = (u32x2){pack_bf16x2(v[0], v[1]), pack_bf16x2(v[2], v[3])};
+        *(u32x2*)((uint16_t*)job.m[i].y + (size_t)row * n + c) = y[i];
+    }
+    RotRaw raw = {};
+    raw.xb = y[0], raw.ub = y[1], raw.s = *(const u32x2*)(suh + c);
+    *(u32x2*)(xh + (size_t)row * n + c) = rot_finish(raw, 2, l32);
+}
+#define WIDE_FINISH_KERNELS(SUFFIX, PER)                                                                                         \
+    extern "C" __global__ __launch_bounds__(256) void exl3_gemvw_finish##SUFFIX(GemvJob job, uint32_t k, uint32_t m, uint32_t y_mode) { \
+        wide_finish_body<PER>(job, k, m, y_mode);                                                                                \
+    }                                                                                                                            \
+    extern "C" __global__ __launch_bounds__(256) void exl3_gemvw_finish_mlp##SUFFIX(GemvJob job, uint32_t k, uint32_t m,          \
+                                                                                     const uint16_t* suh, uint16_t* xh) {         \
+        wide_finish_mlp_body<PER>(job, k, m, suh, xh);                                                                           \
+    }
+WIDE_FINISH_KERNELS(, 1)
+WIDE_FINISH_KERNELS(_pairs, 2)
 #define GEMV_WIDE_KERNEL(NAME, BITS, RG, PER)                                                                         \
-    extern "C" __global__ __launch_bounds__(256, 4) void NAME(GemvJob job, uint32_t k, uint32_t m, uint32_t y_mode) { \
+    extern "C" __global__ __launch_bounds__(256, 4) void NAME(GemvJob job, uint32_t k, uint32_t m) {                  \
         uint32_t i = 0;                                                                                               \
         while (i + 1 < job.count && blockIdx.x >= job.first[i + 1]) i++;                                              \
-        gemv_wide_body<BITS, RG, PER>(job.m[i], blockIdx.x - job.first[i], k, m, y_mode);                             \
+        gemv_wide_body<BITS, RG, PER>(job.m[i], blockIdx.x - job.first[i], k, m);                             \
     }
 #define GEMV_WIDE_ROWS(BITS, RG)                                    \
     GEMV_WIDE_KERNEL(exl3_gemvw_b##BITS##_r##RG, BITS, RG, 1)        \

@@ -17,9 +17,6 @@
 // and up in one launch. Loads are issued early in a step (at two stages the wait at the next step's start has to find them done: 17408 x
 // 5120, 224 rows 47.5 -> 43.0 us), words a step earlier than A. us, the GEMM that goes through LDS -> this one, 4 bits, with rotation and reduce
 // launches: 5120 x 17408 at 180 / 480 / 1300 rows 73.7 / 124 / 294 -> 61.5 / 114 / 253, 4096 x 11008 at 330 rows 80 -> 50, MLP blocks at rgemm_takes.
-#include <type_traits>
-#include <utility>
-
 #include "exl3_trellis.h"
 #include "gemm8.h"
 
@@ -40,16 +37,6 @@ struct RgJob {
     uint32_t count, k, rows, y_mode, tiles_m, tiles_n, group, full, runs, base, rem, pad;
     float* part;  // [slot][column block][BM rows][128]
 };
-
-// f(0) .. f(N - 1) with constant arguments (the compiler gives up unrolling the largest of these loops by itself)
-template <class F, int... I>
-__device__ __forceinline__ void rg_for_(F f, std::integer_sequence<int, I...>) {
-    (f(std::integral_constant<int, I>{}), ...);
-}
-template <int N, class F>
-__device__ __forceinline__ void rg_for(F f) {
-    rg_for_(f, std::make_integer_sequence<int, N>{});
-}
 
 template <int BITS, int RG, int KG>
 struct RgCfg {
@@ -178,15 +165,15 @@ __device__ __forceinline__ void rgemm_segment(const RgJob& job, uint32_t tile, u
 #pragma unroll
         for (int i = 0; i < AHEAD; i++) rd(i);
         prepare();
-        rg_for<MF>([&](auto f_tag) {
+        g8_for<MF>([&](auto f_tag) {
             constexpr int f = decltype(f_tag)::value, i = f / 4, h = f & 1, kh = (f >> 1) & 1, LOADS = C::LA + C::LW;
             if constexpr (f % 4 == 0 && i + AHEAD < RG) rd(i + AHEAD);
             acc[i][h] = __builtin_amdgcn_mfma_f32_16x16x32_f16(__builtin_bit_cast(f16x8, op[SET][h][kh]), x[i % (AHEAD + 1)][kh], acc[i][h], 0, 0, 0);
             asm volatile("" : "+v"(acc[i][h]));
-            rg_for<16>([&](auto q) {
+            g8_for<16>([&](auto q) {
                 if constexpr (g8_at(decltype(q)::value, 16, 0, MF) == f) decode(SET ^ 1, decltype(q)::value);
             });
-            rg_for<LOADS>([&](auto q_tag) {
+            g8_for<LOADS>([&](auto q_tag) {
                 constexpr int q = decltype(q_tag)::value;
                 if constexpr (g8_at(q, LOADS, 1, C::ST == 2 ? MF / 2 : MF) == f) {
                     if constexpr (q < C::LA)
