@@ -95,7 +95,7 @@ struct fe_exl3_kernels {
     fe_function_t rot_in = nullptr, rot_in_group = nullptr, probe_v4 = nullptr;
     fe_function_t probe_decode[3] = {nullptr, nullptr, nullptr};  // 3, 4, 5 bits
     fe_function_t gemvb[6] = {};                                  // the decode GEMV for 1..16 rows, [bits slot]
-    fe_function_t gemvw[6][3][2] = {};                            // for 17..64 rows, [bits slot][row groups - 2][programs a workgroup - 1]
+    fe_function_t gemvw[6][4][2] = {};                            // for 17..64 rows (gate and up of an MLP block: any), [bits slot][row groups - 1][programs a workgroup - 1]
     fe_function_t gemvw_finish[2] = {}, gemvw_finish_mlp[2] = {};  // their outputs, [programs a workgroup - 1]; gate's and up's with down's rotated input
     fe_function_t gemvb_fenced[6] = {};                           // the same for 1..16 rows with the fenced hand-off
     fe_function_t mlp[6] = {};                                    // the decode MLP in one launch, [bits slot]
@@ -194,11 +194,11 @@ int fe_exl3_kernels_load(fe_exl3_kernels **out) {
         snprintf(nm, sizeof nm, "exl3_gemvb_b%d_r1", kBits[i]);
         get(&k->gemvb[i], nm);
         if (!c) c = fe_hip_func_set_max_dyn_lds(k->gemvb[i], 84 * 1024);
-        for (int rg = 2; rg <= 4; rg++) {
+        for (int rg = 1; rg <= 4; rg++) {
             for (int per = 1; per <= 2; per++) {
                 snprintf(nm, sizeof nm, "exl3_gemvw_b%d_r%d%s", kBits[i], rg, per == 2 ? "_pairs" : "");
-                get(&k->gemvw[i][rg - 2][per - 1], nm);
-                if (!c) c = fe_hip_func_set_max_dyn_lds(k->gemvw[i][rg - 2][per - 1], 84 * 1024);
+                get(&k->gemvw[i][rg - 1][per - 1], nm);
+                if (!c) c = fe_hip_func_set_max_dyn_lds(k->gemvw[i][rg - 1][per - 1], 84 * 1024);
             }
         }
         snprintf(nm, sizeof nm, "exl3_gemvb_b%d_r1_fenced", kBits[i]);
@@ -772,7 +772,7 @@ static uint32_t programs_per(const fe_exl3_linear *const *ls, size_t count) {
 
 // The decode GEMV for 1..4 linears of one input in one launch, 1..64 rows: member i reads its rotated input at xhs[i]
 // (in.x == 0) or rotates in.x itself and leaves the result at xhs[i]. The caller has checked rows, k and bits.
-// down: of a group of gate and up of 17..64 rows, the linear whose rotated input of SwiGLU(gate, up) is left at ws->xh, or null.
+// down: of a group of gate and up, the linear whose rotated input of SwiGLU(gate, up) is left at ws->xh, or null.
 static int launch_job(const fe_exl3_linear *const *ls, size_t count, fe_stream_t s, const fe_devptr_t *xhs, const fe_devptr_t *ys,
                       int y_dtype, uint32_t rows, const fe_exl3_workspace *ws, const RotInput &in, const char *fn, const fe_exl3_linear *down = nullptr) {
     GemvJobArgs g{};
@@ -787,8 +787,8 @@ static int launch_job(const fe_exl3_linear *const *ls, size_t count, fe_stream_t
     // (measured on gate + up, 5120 x 17408, two a workgroup against one: 3 bits 5 / 8 rows 33.3 / 35.3 us against 34.2 / 35.5, 4 bits
     // 34.0 / 35.9 against 35.3 / 36.6, 6 bits 40.3 / 42.3 against 43.3 / 44.6; at 16 rows 44.8 against 41.9, where the longer run's
     // inputs no longer fit the staging buffer in one piece: up to 8 rows)
-    const bool wide = rows > 16 && !in.x;
-    uint32_t fuse = kern->opt.fuse && rows <= 8 ? std::min(4u, std::max(1u, (total + places - 1) / places)) : 1;
+    const bool wide = (rows > 16 || down) && !in.x;
+    uint32_t fuse = kern->opt.fuse && !wide && rows <= 8 ? std::min(4u, std::max(1u, (total + places - 1) / places)) : 1;
     const uint32_t per = wide ? programs_per(ls, count) : 1;
     uint32_t programs = 0, run_steps = 0;  // (programs: workgroups of the launch)
     size_t z_at = 0, cnt_at = 0;
@@ -824,7 +824,7 @@ static int launch_job(const fe_exl3_linear *const *ls, size_t count, fe_stream_t
     if (wide) {
         const uint32_t rg = (rows + 15) / 16;
         void *args[] = {&g, &k, &rows};
-        FE_TRY(fe_hip_launch(kern->gemvw[bits_slot(bits)][rg - 2][per - 1], programs, 1, 1, 256, 1, 1, spread_lds(kern, programs, wide_lds(bits, rg)), s, args));
+        FE_TRY(fe_hip_launch(kern->gemvw[bits_slot(bits)][rg - 1][per - 1], programs, 1, 1, 256, 1, 1, spread_lds(kern, programs, wide_lds(bits, rg)), s, args));
         if (down) {
             fe_devptr_t suh = down->view.suh, xh = ws->xh.p;
             void *fargs[] = {&g, &k, &rows, &suh, &xh};
@@ -1183,7 +1183,10 @@ int fe_exl3_mlp_forward(const fe_exl3_linear *gate, const fe_exl3_linear *up, co
         if (part->as_linear && job_z(part->as_linear.get(), rows) <= ws->z_len) dl = part->as_linear.get();
     }
     bool fused = false;
-    if (rows > 16 && group_fits(front, 2, rows, ws, &fused) && down->k <= ws->max_k) {  // down's input is rotated where gate and up are finished
+    // From 9 rows on gate and up leave their sums to a launch that finishes them with all CUs and rotates down's input too, in the place of the
+    // rotation's launch. A layer, 4 / 5 / 8 bits, at 5 / 8 / 11 / 16 rows, with the finisher inside the GEMV and a rotation / this way: 5120 x 17408 84.7 / 96.4 /
+    // 96.9 / 130.0 us against 85.9 / 97.0 / 93.1 / 123.8, 2560 x 6912 59.3 / 67.6 against 57.5 / 64.8 at 11 / 16.
+    if (rows > 8 && group_fits(front, 2, rows, ws, &fused) && !fused && down->k <= ws->max_k && (rows > 16 || !kern->opt.handoff_fenced)) {
         FE_TRY(forward_group(front, 2, kern, s, x, x_dtype, ys, FE_DTYPE_BF16, rows, ws, false, dl, fn));
         return launch_rows(dl, s, ws->xh.p, y, y_dtype, rows, ws, RotInput{});
     }

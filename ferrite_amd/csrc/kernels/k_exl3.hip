@@ -805,7 +805,7 @@ GEMVB_FAMILY(8)
 
 // ---- the same GEMV for more rows ------------------------------------------------------------------------------------------
 //
-// 17..64 rows. The programs, their runs, the order of every sum and so the bits are gemvb_body's. With PER 2 a
+// 17..64 rows, and gate and up of an MLP block from 9 rows on. The programs, their runs, the order of every sum and so the bits are gemvb_body's. With PER 2 a
 // workgroup runs the programs 2 j and 2 j + 1 as one: where the first's run ends inside a column block its sums step aside, and are
 // added to the second's before they leave as one segment, as the finisher of gemvb_body adds them. What differs is how a program
 // gets its operands and hands its sums over: both grow with the rows while the decode does not. The rotated inputs and the trellis words of a
@@ -1029,7 +1029,7 @@ WIDE_FINISH_KERNELS(_pairs, 2)
 #define GEMV_WIDE_ROWS(BITS, RG)                                    \
     GEMV_WIDE_KERNEL(exl3_gemvw_b##BITS##_r##RG, BITS, RG, 1)        \
     GEMV_WIDE_KERNEL(exl3_gemvw_b##BITS##_r##RG##_pairs, BITS, RG, 2)
-#define GEMV_WIDE_FAMILY(BITS) GEMV_WIDE_ROWS(BITS, 2) GEMV_WIDE_ROWS(BITS, 3) GEMV_WIDE_ROWS(BITS, 4)
+#define GEMV_WIDE_FAMILY(BITS) GEMV_WIDE_ROWS(BITS, 1) GEMV_WIDE_ROWS(BITS, 2) GEMV_WIDE_ROWS(BITS, 3) GEMV_WIDE_ROWS(BITS, 4)
 GEMV_WIDE_FAMILY(2)
 GEMV_WIDE_FAMILY(3)
 GEMV_WIDE_FAMILY(4)

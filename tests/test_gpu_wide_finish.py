@@ -1,4 +1,4 @@
-"""17..64 rows: the launch that finishes gate and up also forms down's rotated input. The MLP block against its parts, bit for bit: the
+"""9..64 rows: the launch that finishes gate and up also forms down's rotated input. The MLP block against its parts, bit for bit: the
 grouped launch of gate and up, fe_silu_mul, down's own forward; programs singly and in pairs (option gemv_pairs)."""
 import numpy as np
 import pytest
@@ -18,7 +18,7 @@ def test_mlp_block_has_the_bits_of_its_parts(bits, hidden, inter, strips):
     bf = lambda *shape: torch.full(shape, 1.5, dtype=torch.bfloat16, device="cuda")
     B = exl3.Dtype.Bf16
     try:
-        for rows in (17, 32, 33, 47, 48, 64):
+        for rows in (9, 15, 16, 17, 32, 33, 47, 48, 64):
             yg, yu, act, want = bf(rows, inter), bf(rows, inter), bf(rows, inter), bf(rows, hidden)
             kern.set_option("gemv_pairs", 0)
             exl3.forward_group([g, u], x, B, [yg, yu], B, rows, ws)
