@@ -353,7 +353,9 @@ inline FeRgemmPlan fe_rgemm_plan(uint32_t rows, uint32_t k, const uint32_t *n, u
     FeRgemmPlan best;
     best.us = 1e30f;
     for (uint32_t blocks = 1; blocks <= 2; blocks++) {
-        if (force_blocks && blocks != force_blocks) continue;
+        // Two column blocks from 129 rows on: their lowest tile is 160 rows, whose last pieces lie, by the scalar offset alone, past the end of fewer
+        // rows, and the range check is only stated for scalar offsets inside the buffer. (Every other tile has more than rg - 2 row groups.)
+        if (blocks != (rows <= 128 ? 1 : force_blocks ? force_blocks : blocks)) continue;
         for (uint32_t cut_m = (rows + 255) / 256; cut_m <= (rows + 255) / 256 + 1; cut_m++) {
             FeRgemmPlan p;
             p.k = k, p.blocks = blocks, p.rg = std::max(((rows + cut_m - 1) / cut_m + 31) / 32 * 2, blocks == 1 ? 6u : 10u);

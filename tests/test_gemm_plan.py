@@ -69,8 +69,11 @@ int main() {
         const uint32_t tiles = p.tiles_m * p.tiles_n, rest = tiles - p.full;
         uint32_t tn = 0;
         for (uint32_t j = 0; j < count; j++) tn += (n[j] / 128 + p.blocks - 1) / p.blocks;
-        bool ok = p.us < 1e29f && (p.blocks == 1 || p.blocks == 2) && (!form || p.blocks == form) && p.rg % 2 == 0 && p.rg <= 16 && p.rg >= (p.blocks == 1 ? 6u : 10u);
+        bool ok = p.us < 1e29f && (p.blocks == 1 || p.blocks == 2) && (rows <= 128 ? p.blocks == 1 : !form || p.blocks == form) && p.rg % 2 == 0 && p.rg <= 16 && p.rg >= (p.blocks == 1 ? 6u : 10u);
         ok = ok && p.tiles_n == tn && p.tiles_m * 16 * p.rg >= rows && (p.tiles_m - 1) * 16 * p.rg < rows && p.full <= tiles && p.k == k;
+        ok = ok && 16 * (p.rg - 2) < rows;  // no piece of A lies past the end of the rows by its scalar offset alone
+        const uint32_t loaders = 4 * p.blocks, pieces_a = (2 * p.rg + loaders - 1) / loaders;
+        ok = ok && (uint64_t)(pieces_a - 1) * 16 * loaders * k + 2 * k - 128 < (uint64_t)rows * k * 2;
         ok = ok && (rest == 0) == (p.runs == 0) && p.runs <= rest * p.steps();
         ok = ok && (!rest || (size_t)(p.runs + rest) * p.blocks * p.rg * 16 * 512 <= part);
         if (!ok) return printf("%u x %u x %u: %u %u\n", rows, k, n[0], form, pieces), 1;
