@@ -960,8 +960,8 @@ __device__ __forceinline__ f32x4 wide_row_sums(const GemvMember& mb, uint32_t nb
     for (uint32_t s0 = 0; s0 < slots; s0 += SB) {
         f32x4 t[SB];
 #pragma unroll
-        for (uint32_t b = 0; b < SB; b++)  // (past the last segment: out of range, reads zero)
-            t[b] = __builtin_bit_cast(f32x4, __builtin_amdgcn_raw_buffer_load_b128(zrs, at, (s0 + b) * m * 512, 0));
+        for (uint32_t b = 0; b < SB; b++)  // (past the last segment: out of range by the vector offset, reads zero)
+            t[b] = __builtin_bit_cast(f32x4, __builtin_amdgcn_raw_buffer_load_b128(zrs, at + (s0 + b) * m * 512, 0, 0));
         if (PER == 1 && odd > s0) t[0] = (f32x4){0.f, 0.f, 0.f, 0.f};  // where the first segment's partner, which has no part in the block, would leave its sums
 #pragma unroll
         for (uint32_t b = 0; b < SB; b += 2) {
