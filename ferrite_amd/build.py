@@ -20,7 +20,10 @@ HIPCC = os.path.join(ROCM, "bin", "hipcc")
 # -packed-fp32-ops off: the compiler must not form v_pk_*_f32 from the float code in these kernels
 DEVICE_FLAGS = ["--offload-arch=gfx950", "-O3", "-std=c++17", "-mcode-object-version=5",
                 "-Xclang", "-target-feature", "-Xclang", "-packed-fp32-ops"]
-KERNELS = ["k_exl3_gemm", "k_exl3_rgemm", "k_exl3", "k_fp4", "k_route", "k_bf16"]
+# code objects: name, source, defines; the ones that take longest first
+KERNELS = [("k_exl3_gemm", "k_exl3_gemm.hip", [])]
+KERNELS += [(f"k_exl3_rgemm_b{b}", "k_exl3_rgemm.hip", [f"-DRG_BITS={b}"]) for b in (8, 6, 5, 4, 3, 2)]
+KERNELS += [(k, k + ".hip", []) for k in ("k_exl3", "k_fp4", "k_bf16", "k_route")]
 HOST = ["fe_hip.cpp", "fe_exl3.cpp", "fe_fp4.cpp", "fe_bf16.cpp", "fe_route.cpp"]
 # host sources that also hold device code (a file-scope __device__ array): compiled by hipcc as one unit
 HOST_HIP = ["fe_exl3_static.hip"]
@@ -39,10 +42,10 @@ def build(verbose: bool = False) -> str:
     only = [k for k in os.environ.get("FE_BUILD_ONLY", "").split(",") if k]  # e.g. k_exl3: the others are kept as built
     inc = ["-I", os.path.join(os.path.dirname(HERE), "include"), "-I", CSRC, "-I", os.path.join(ROCM, "include")]
     jobs = []
-    for k in KERNELS:
-        if only and k not in only and os.path.exists(os.path.join(OUT, k + ".hsaco")):
+    for k, src, defines in KERNELS:
+        if only and not {k, src[:-4]} & set(only) and os.path.exists(os.path.join(OUT, k + ".hsaco")):
             continue
-        jobs.append([HIPCC, "--genco", "--no-gpu-bundle-output", *DEVICE_FLAGS, "-I", KERN, os.path.join(KERN, k + ".hip"),
+        jobs.append([HIPCC, "--genco", "--no-gpu-bundle-output", *DEVICE_FLAGS, *defines, "-I", KERN, os.path.join(KERN, src),
                      "-o", os.path.join(OUT, k + ".hsaco")])
     for src in HOST_HIP:
         jobs.append([HIPCC, "-c", "-fPIC", *DEVICE_FLAGS, *inc, os.path.join(CSRC, src), "-o",

@@ -14,11 +14,41 @@ fe_k_exl3_gemm_hsaco:
     .global fe_k_exl3_gemm_hsaco_end
 fe_k_exl3_gemm_hsaco_end:
     .balign 4096
-    .global fe_k_exl3_rgemm_hsaco
-fe_k_exl3_rgemm_hsaco:
-    .incbin "k_exl3_rgemm.hsaco"
-    .global fe_k_exl3_rgemm_hsaco_end
-fe_k_exl3_rgemm_hsaco_end:
+    .global fe_k_exl3_rgemm_b2_hsaco
+fe_k_exl3_rgemm_b2_hsaco:
+    .incbin "k_exl3_rgemm_b2.hsaco"
+    .global fe_k_exl3_rgemm_b2_hsaco_end
+fe_k_exl3_rgemm_b2_hsaco_end:
+    .balign 4096
+    .global fe_k_exl3_rgemm_b3_hsaco
+fe_k_exl3_rgemm_b3_hsaco:
+    .incbin "k_exl3_rgemm_b3.hsaco"
+    .global fe_k_exl3_rgemm_b3_hsaco_end
+fe_k_exl3_rgemm_b3_hsaco_end:
+    .balign 4096
+    .global fe_k_exl3_rgemm_b4_hsaco
+fe_k_exl3_rgemm_b4_hsaco:
+    .incbin "k_exl3_rgemm_b4.hsaco"
+    .global fe_k_exl3_rgemm_b4_hsaco_end
+fe_k_exl3_rgemm_b4_hsaco_end:
+    .balign 4096
+    .global fe_k_exl3_rgemm_b5_hsaco
+fe_k_exl3_rgemm_b5_hsaco:
+    .incbin "k_exl3_rgemm_b5.hsaco"
+    .global fe_k_exl3_rgemm_b5_hsaco_end
+fe_k_exl3_rgemm_b5_hsaco_end:
+    .balign 4096
+    .global fe_k_exl3_rgemm_b6_hsaco
+fe_k_exl3_rgemm_b6_hsaco:
+    .incbin "k_exl3_rgemm_b6.hsaco"
+    .global fe_k_exl3_rgemm_b6_hsaco_end
+fe_k_exl3_rgemm_b6_hsaco_end:
+    .balign 4096
+    .global fe_k_exl3_rgemm_b8_hsaco
+fe_k_exl3_rgemm_b8_hsaco:
+    .incbin "k_exl3_rgemm_b8.hsaco"
+    .global fe_k_exl3_rgemm_b8_hsaco_end
+fe_k_exl3_rgemm_b8_hsaco_end:
     .balign 4096
     .global fe_k_fp4_hsaco
 fe_k_fp4_hsaco:

@@ -100,10 +100,10 @@ struct fe_exl3_kernels {
     fe_function_t gemvb_fenced[6] = {};                           // the same for 1..16 rows with the fenced hand-off
     fe_function_t mlp[6] = {};                                    // the decode MLP in one launch, [bits slot]
     uint32_t cus = 0;
-    fe_module_t gemm_module = nullptr, rgemm_module = nullptr;
+    fe_module_t gemm_module = nullptr, rgemm_module[6] = {};  // [bits slot]; a file that FE_EXL3_RGEMM_HSACO names holds every width: the first alone
     fe_function_t gemm[6][4] = {};        // decode inside the GEMM, by form: 256 x 256, stream-K, 128 x 256, 128 x 128
     fe_function_t gemm_reduce[3] = {};    // by tile
-    fe_function_t rgemm[6][2][6] = {}, rgemm_reduce = nullptr;  // decode into registers, [bits slot][column blocks - 1][row groups / 2 - 3]
+    fe_function_t rgemm[6][2][6] = {}, rgemm_reduce[6] = {};  // decode into registers, [bits slot][column blocks - 1][row groups / 2 - 3]
     fe_function_t hat_tiles[6] = {};  // trellis -> fp16 weights as the GEMM's LDS images
     fe_function_t gemm_hat[4] = {};   // the GEMM over them, by form
     FeGemmTileOptions tile;           // "gemm_tile", "gemm_pieces"
@@ -219,20 +219,25 @@ int fe_exl3_kernels_load(fe_exl3_kernels **out) {
         for (uint32_t f = 0; f < 4; f++) get_gemm(&k->gemm[i][f], "exl3_gemm_b" + b + form_sfx[f], gemm_lds(f, (uint32_t)kBits[i]));
         get_gemm(&k->hat_tiles[i], "exl3_hat_tiles_b" + b, 0);
     }
-    if (!c) c = fe_load_module(&k->rgemm_module, "FE_EXL3_RGEMM_HSACO", fe_k_exl3_rgemm_hsaco, fe_k_exl3_rgemm_hsaco_end);
-    auto get_rgemm = [&](fe_function_t *f, const std::string &name, uint32_t lds) {
-        if (!c) c = fe_hip_module_get_function(f, k->rgemm_module, name.c_str());
-        if (!c && lds) c = fe_hip_func_set_max_dyn_lds(*f, lds);
-    };
+    static const unsigned char *const rgemm_image[6][2] = {{fe_k_exl3_rgemm_b2_hsaco, fe_k_exl3_rgemm_b2_hsaco_end}, {fe_k_exl3_rgemm_b3_hsaco, fe_k_exl3_rgemm_b3_hsaco_end},
+                                                           {fe_k_exl3_rgemm_b4_hsaco, fe_k_exl3_rgemm_b4_hsaco_end}, {fe_k_exl3_rgemm_b5_hsaco, fe_k_exl3_rgemm_b5_hsaco_end},
+                                                           {fe_k_exl3_rgemm_b6_hsaco, fe_k_exl3_rgemm_b6_hsaco_end}, {fe_k_exl3_rgemm_b8_hsaco, fe_k_exl3_rgemm_b8_hsaco_end}};
+    const char *rgemm_file = getenv("FE_EXL3_RGEMM_HSACO");
+    const bool one_rgemm = rgemm_file && *rgemm_file;
     for (int i = 0; i < 6; i++) {
+        if (!c && (i == 0 || !one_rgemm)) c = fe_load_module(&k->rgemm_module[i], "FE_EXL3_RGEMM_HSACO", rgemm_image[i][0], rgemm_image[i][1]);
+        auto get_rgemm = [&](fe_function_t *f, const std::string &name, uint32_t lds) {
+            if (!c) c = fe_hip_module_get_function(f, k->rgemm_module[one_rgemm ? 0 : i], name.c_str());
+            if (!c && lds) c = fe_hip_func_set_max_dyn_lds(*f, lds);
+        };
         const std::string b = "exl3_rgemm_b" + std::to_string(kBits[i]);
         for (uint32_t j = 0; j < 6; j++) {
             const uint32_t rg = 6 + 2 * j;
             get_rgemm(&k->rgemm[i][0][j], b + "_r" + std::to_string(rg) + "_k2", rgemm_lds((uint32_t)kBits[i], rg, 1));
             if (rg >= 10) get_rgemm(&k->rgemm[i][1][j], b + "_r" + std::to_string(rg) + "_k1", rgemm_lds((uint32_t)kBits[i], rg, 2));
         }
+        get_rgemm(&k->rgemm_reduce[i], "exl3_rgemm_reduce", 0);
     }
-    get_rgemm(&k->rgemm_reduce, "exl3_rgemm_reduce", 0);
     for (int f = 0; f < 4; f++) get_gemm(&k->gemm_hat[f], std::string("exl3_gemm_hat") + form_sfx[f], kHatLds[f]);
     for (int i = 0; i < 3; i++) get_gemm(&k->gemm_reduce[i], std::string("exl3_gemm_reduce") + tile_sfx[i], 0);
     fe_exl3_options &o = k->opt;
@@ -268,7 +273,8 @@ int fe_exl3_kernels_destroy(fe_exl3_kernels *k) {
     if (!k) return 0;
     if (k->module) fe_hip_module_unload(k->module);
     if (k->gemm_module) fe_hip_module_unload(k->gemm_module);
-    if (k->rgemm_module) fe_hip_module_unload(k->rgemm_module);
+    for (fe_module_t m : k->rgemm_module)
+        if (m) fe_hip_module_unload(m);
     delete k;
     return 0;
 }
@@ -661,7 +667,7 @@ static int launch_rgemm(const fe_exl3_linear *const *ls, size_t count, fe_stream
     if (!p.reduce()) return 0;
     uint32_t bm = 16 * p.rg, blocks = p.blocks, all = p.steps();
     void *rargs[] = {&j, &bm, &blocks, &all};
-    return fe_hip_launch(kern->rgemm_reduce, rest * blocks * (bm / 8), 1, 1, 256, 1, 1, 0, s, rargs);
+    return fe_hip_launch(kern->rgemm_reduce[slot_bits], rest * blocks * (bm / 8), 1, 1, 256, 1, 1, 0, s, rargs);
 }
 
 static int launch_gemm(const fe_exl3_linear *l, fe_stream_t s, fe_devptr_t xh, fe_devptr_t y, int y_dtype, uint32_t rows,

@@ -21,8 +21,15 @@ extern "C" const unsigned char fe_k_exl3_hsaco[];
 extern "C" const unsigned char fe_k_exl3_hsaco_end[];
 extern "C" const unsigned char fe_k_exl3_gemm_hsaco[];
 extern "C" const unsigned char fe_k_exl3_gemm_hsaco_end[];
-extern "C" const unsigned char fe_k_exl3_rgemm_hsaco[];
-extern "C" const unsigned char fe_k_exl3_rgemm_hsaco_end[];
+#define FE_RGEMM_OBJECT(B)                                             \
+    extern "C" const unsigned char fe_k_exl3_rgemm_b##B##_hsaco[];     \
+    extern "C" const unsigned char fe_k_exl3_rgemm_b##B##_hsaco_end[];
+FE_RGEMM_OBJECT(2)
+FE_RGEMM_OBJECT(3)
+FE_RGEMM_OBJECT(4)
+FE_RGEMM_OBJECT(5)
+FE_RGEMM_OBJECT(6)
+FE_RGEMM_OBJECT(8)
 extern "C" const unsigned char fe_k_fp4_hsaco[];
 extern "C" const unsigned char fe_k_fp4_hsaco_end[];
 extern "C" const unsigned char fe_k_route_hsaco[];

@@ -315,8 +315,10 @@ extern "C" __global__ __launch_bounds__(256) void exl3_rgemm_reduce(RgJob job, u
     RGEMM_KERNEL(BITS, 6, 2) RGEMM_KERNEL(BITS, 8, 2) RGEMM_KERNEL(BITS, 10, 2) RGEMM_KERNEL(BITS, 12, 2)         \
     RGEMM_KERNEL(BITS, 14, 2) RGEMM_KERNEL(BITS, 16, 2)                                                           \
     RGEMM_KERNEL(BITS, 10, 1) RGEMM_KERNEL(BITS, 12, 1) RGEMM_KERNEL(BITS, 14, 1) RGEMM_KERNEL(BITS, 16, 1)
-#ifdef RG_ONLY4
-RGEMM_ROWS(4)
+// One code object a width in bits (RG_BITS): sixty unrolled kernels in one take a compiler eight times as long as the next largest source.
+// Without RG_BITS the file compiles to one that holds them all.
+#ifdef RG_BITS
+RGEMM_ROWS(RG_BITS)
 #else
 RGEMM_ROWS(2)
 RGEMM_ROWS(3)

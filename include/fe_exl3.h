@@ -51,7 +51,7 @@ typedef struct fe_exl3_workspace fe_exl3_workspace; /* Workspace, crates/fe-exl3
 
 /* Kernels::load: the embedded gfx950 code objects, or the files named by FE_EXL3_HSACO (the decode kernels, rotations, reconstruction and
  * probes; the reference's FE_EXL3_CUBIN, crates/fe-exl3/src/gpu/mod.rs:88-93), FE_EXL3_GEMM_HSACO (the prefill GEMMs and the
- * decode into tiles) and FE_EXL3_RGEMM_HSACO (the prefill GEMM that decodes into registers). */
+ * decode into tiles) and FE_EXL3_RGEMM_HSACO (the prefill GEMM that decodes into registers, every width in one file). */
 int fe_exl3_kernels_load(fe_exl3_kernels **out);
 int fe_exl3_kernels_destroy(fe_exl3_kernels *k);
 /* Switches of the launch paths, by name (the environment variable that sets the same switch when the kernels are loaded):

@@ -123,7 +123,7 @@ def store_hazards(body):
     return found
 
 
-@pytest.mark.parametrize("name", ["k_exl3", "k_exl3_gemm", "k_exl3_rgemm", "k_fp4", "k_bf16", "k_route"])
+@pytest.mark.parametrize("name", ["k_exl3", "k_exl3_gemm", *(f"k_exl3_rgemm_b{b}" for b in (2, 3, 4, 5, 6, 8)), "k_fp4", "k_bf16", "k_route"])
 def test_wait_states(name):
     path = os.path.join(ROOT, "ferrite_amd", "_build", name + ".hsaco")
     assert os.path.exists(path), "build the library first"
