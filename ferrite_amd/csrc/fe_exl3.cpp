@@ -1000,7 +1000,7 @@ int fe_exl3_linear_forward_group_launches(const fe_exl3_linear *const *ls, size_
                                           const fe_exl3_workspace *ws) {
     bool fused = false;
     if (!group_fits(ls, count, rows, ws, &fused)) return 0;
-    return fused ? 1 : 2;
+    return fused ? 1 : rows > 16 ? 3 : 2;
 }
 
 int fe_exl3_linear_forward_group(const fe_exl3_linear *const *ls, size_t count, const fe_exl3_kernels *kern, fe_stream_t s,

@@ -1,0 +1,39 @@
+"""What the queries say about the launches of a call, against the kernels that a capture of the call records."""
+import ctypes as C
+
+import numpy as np
+import pytest
+
+pytestmark = pytest.mark.gpu
+
+
+def kernels_recorded(torch, call):
+    """Kernel nodes of a captured call."""
+    hip = C.CDLL("libamdhip64.so")
+    call()
+    torch.cuda.synchronize()
+    graph = torch.cuda.CUDAGraph(keep_graph=True)
+    with torch.cuda.graph(graph, stream=torch.cuda.Stream()):
+        call()
+    raw, n = C.c_void_p(graph.raw_cuda_graph()), C.c_size_t(0)
+    assert hip.hipGraphGetNodes(raw, None, C.byref(n)) == 0
+    nodes, kind, kernels = (C.c_void_p * n.value)(), C.c_int(0), 0
+    assert hip.hipGraphGetNodes(raw, nodes, C.byref(n)) == 0
+    for node in nodes:
+        assert hip.hipGraphNodeGetType(C.c_void_p(node), C.byref(kind)) == 0
+        kernels += kind.value == 0  # hipGraphNodeTypeKernel
+    return kernels
+
+
+@pytest.mark.parametrize("rows", [1, 8, 16, 17, 40, 64])
+def test_group_launches(rows):
+    import torch
+    from ferrite_amd import exl3, synth
+    kern = exl3.Kernels.load()
+    k = 1024
+    lins = [exl3.Linear.new(kern, exl3.DeviceExl3.upload_strips(synth.exl3_tensor(k, n, 4, n)), 256) for n in (384, 256)]
+    ws = exl3.Workspace(lins, 64)
+    x = torch.from_numpy(synth.activations(rows, k, 3).view(np.int16)).cuda()
+    ys = [torch.zeros((rows, l.n), dtype=torch.bfloat16, device="cuda") for l in lins]
+    call = lambda: exl3.forward_group(lins, x, exl3.Dtype.Bf16, ys, exl3.Dtype.Bf16, rows, ws)
+    assert exl3.forward_group_launches(lins, rows, ws) == kernels_recorded(torch, call)
