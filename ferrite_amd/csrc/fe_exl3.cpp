@@ -22,6 +22,7 @@ constexpr uint32_t kMaxRowsPerPass = 64;       // 4 row groups of 16
 // 5120 143 / 143 / 172 against 146 / 139 / 165, 2048 x 5632 68.3 / 72.6 / 98.2 against 69.3 / 73.1 / 96.1.
 constexpr uint32_t kHatRows = 2304;
 constexpr uint32_t kChainRows = 8;             // most rows of the one-launch MLP (mlp_chain_fits)
+constexpr uint32_t kWideWhole = 4;             // WIDE_WHOLE of k_exl3.hip
 constexpr uint32_t kGroupMax = 4;              // FE_EXL3_GROUP_MAX: linears of one launch
 // LDS of one GEMV program of 1..16 rows and of one of the one-launch MLP (sums of a segment + staged inputs of a chunk of the
 // run): three programs fit a CU's 160 KB. A whole run mostly fits in far less; the budget cuts long runs of many rows into
@@ -95,7 +96,7 @@ struct fe_exl3_kernels {
     fe_function_t rot_in = nullptr, rot_in_group = nullptr, probe_v4 = nullptr;
     fe_function_t probe_decode[3] = {nullptr, nullptr, nullptr};  // 3, 4, 5 bits
     fe_function_t gemvb[6] = {};                                  // the decode GEMV for 1..16 rows, [bits slot]
-    fe_function_t gemvw[6][4][2] = {};                            // for 17..64 rows (gate and up of an MLP block: any), [bits slot][row groups - 1][programs a workgroup - 1]
+    fe_function_t gemvw[6][4][2][2] = {};                         // for 17..64 rows (gate and up of an MLP block: any), [bits slot][row groups - 1][programs a workgroup - 1][finishes whole blocks]
     fe_function_t gemvw_finish[2] = {}, gemvw_finish_mlp[2] = {};  // their outputs, [programs a workgroup - 1]; gate's and up's with down's rotated input
     fe_function_t gemvb_fenced[6] = {};                           // the same for 1..16 rows with the fenced hand-off
     fe_function_t mlp[6] = {};                                    // the decode MLP in one launch, [bits slot]
@@ -115,6 +116,7 @@ struct fe_exl3_linear {
     uint32_t k = 0, n = 0, bits = 0;
     fe_exl3_plan plan{};
     uint32_t programs = 0;  // grid of the decode GEMV under this plan
+    uint32_t cut_blocks[2] = {};  // column blocks that it cuts, [programs a workgroup - 1] (17..64 rows)
     fe_exl3_view view{};
     FeBuf trellis, suh, svh;  // owned copies (upload), empty for from_view
     FeBuf hat;                // decoded fp16 tiles kept with the linear (fe_exl3_linear_keep_decoded), else empty
@@ -196,9 +198,11 @@ int fe_exl3_kernels_load(fe_exl3_kernels **out) {
         if (!c) c = fe_hip_func_set_max_dyn_lds(k->gemvb[i], 84 * 1024);
         for (int rg = 1; rg <= 4; rg++) {
             for (int per = 1; per <= 2; per++) {
-                snprintf(nm, sizeof nm, "exl3_gemvw_b%d_r%d%s", kBits[i], rg, per == 2 ? "_pairs" : "");
-                get(&k->gemvw[i][rg - 1][per - 1], nm);
-                if (!c) c = fe_hip_func_set_max_dyn_lds(k->gemvw[i][rg - 1][per - 1], 84 * 1024);
+                for (int ends = 0; ends < 2; ends++) {
+                    snprintf(nm, sizeof nm, "exl3_gemvw_b%d_r%d%s%s", kBits[i], rg, per == 2 ? "_pairs" : "", ends ? "_ends" : "");
+                    get(&k->gemvw[i][rg - 1][per - 1][ends], nm);
+                    if (!c) c = fe_hip_func_set_max_dyn_lds(k->gemvw[i][rg - 1][per - 1][ends], 84 * 1024);
+                }
             }
         }
         snprintf(nm, sizeof nm, "exl3_gemvb_b%d_r1_fenced", kBits[i]);
@@ -376,6 +380,10 @@ static uint32_t plan_programs(const fe_exl3_kernels *kern, const fe_exl3_plan &p
     return std::max(1u, std::min(progs, units));
 }
 
+static void count_cut_blocks(fe_exl3_linear *l) {
+    for (uint32_t per = 1; per <= 2; per++) l->cut_blocks[per - 1] = fe_gemv_cut_blocks((l->k / 128) * (l->n / 128), l->programs, l->k / 128, per);
+}
+
 // The programs of a partition of the linear in the order in which, as the down projection of a one-launch MLP, their
 // inputs get ready: sorted by the last 128-channel block their run reads (a run that crosses into the next column block
 // reads the last block of all), then by program number. A program of the down stage waits for lower-numbered programs'
@@ -397,12 +405,14 @@ static int make_chain_part(fe_exl3_linear *l, uint32_t unit_len, uint32_t progra
         fe_exl3_linear &sh = *part->as_linear;
         sh.name = l->name, sh.k = l->k, sh.n = l->n, sh.bits = l->bits, sh.plan = l->plan, sh.programs = programs;
         sh.view = l->view, sh.kern = l->kern;
+        count_cut_blocks(&sh);
     }
     l->chain_parts.push_back(std::move(part));
     return 0;
 }
 
 static int make_chain_order(fe_exl3_linear *l) {
+    count_cut_blocks(l);
     if (int c = make_chain_part(l, 0, l->programs)) return c;
     const uint32_t upb = l->k / 128, units = upb * (l->n / 128);
     for (uint32_t len : {2u, 4u, 8u})
@@ -776,6 +786,23 @@ static uint32_t programs_per(const fe_exl3_linear *const *ls, size_t count) {
     return 2;
 }
 
+// Who finishes the column blocks of 17..64 rows: the GEMV's programs, where no block is cut (wide linears of a short K: the launch behind would only carry
+// sums to memory and back); from 33 rows on the programs and the launch each their own, where half the blocks are whole and there are programs enough
+// to finish them side by side; else the launch all of them. us, 4 bits, all by the launch -> by this rule, 17 / 33 / 64 rows: whole: 512 x 65536 15.1 / - / 21.4 -> 12.4 / - / 15.7,
+// 768 x 65536 18.4 / 21.3 / 25.1 -> 15.4 / 17.4 / 19.8, 2560 x 131072 66.5 / 77.8 / 89.6 -> 63.8 / 71.4 / 82.7, 5120 x 131072 124.7 / 145.0 / 162.3 -> 121.0 / 137.4 / 157.4;
+// both: 512 x 99968 25.3 / 32.3 -> 24.1 / 29.3 at 33 / 64, 1024 x 151936 50.3 / 59.6 -> 48.6 / 56.9 (at 17 rows both lose 0 to 4 % to the launch). Few programs finish
+// slowly: 256 x 32896, 128 of them, 40 / 64 rows 16.0 / 18.9 by the launch, 17.4 / 20.5 by both.
+enum class WideEnd { Launch, Both, Programs };
+static WideEnd wide_end(const fe_exl3_linear *const *ls, size_t count, uint32_t per, uint32_t rows) {
+    bool whole = true, half = rows > 32;
+    for (size_t i = 0; i < count; i++) {
+        const uint32_t cut = ls[i]->cut_blocks[per - 1];
+        whole = whole && !cut;
+        half = half && 2 * cut <= ls[i]->n / 128 && ls[i]->programs >= 2 * std::max(ls[i]->kern->cus, 1u);
+    }
+    return whole ? WideEnd::Programs : half ? WideEnd::Both : WideEnd::Launch;
+}
+
 // The decode GEMV for 1..4 linears of one input in one launch, 1..64 rows: member i reads its rotated input at xhs[i]
 // (in.x == 0) or rotates in.x itself and leaves the result at xhs[i]. The caller has checked rows, k and bits.
 // down: of a group of gate and up, the linear whose rotated input of SwiGLU(gate, up) is left at ws->xh, or null.
@@ -829,14 +856,17 @@ static int launch_job(const fe_exl3_linear *const *ls, size_t count, fe_stream_t
     const uint32_t bits = ls[0]->bits;
     if (wide) {
         const uint32_t rg = (rows + 15) / 16;
-        void *args[] = {&g, &k, &rows};
-        FE_TRY(fe_hip_launch(kern->gemvw[bits_slot(bits)][rg - 1][per - 1], programs, 1, 1, 256, 1, 1, spread_lds(kern, programs, wide_lds(bits, rg)), s, args));
+        const WideEnd end = down ? WideEnd::Launch : wide_end(ls, count, per, rows);
+        uint32_t finish_mode = end == WideEnd::Both ? mode | kWideWhole : mode;
+        void *args[] = {&g, &k, &rows, &mode};
+        FE_TRY(fe_hip_launch(kern->gemvw[bits_slot(bits)][rg - 1][per - 1][end != WideEnd::Launch], programs, 1, 1, 256, 1, 1, spread_lds(kern, programs, wide_lds(bits, rg)), s, args));
         if (down) {
             fe_devptr_t suh = down->view.suh, xh = ws->xh.p;
             void *fargs[] = {&g, &k, &rows, &suh, &xh};
             return fe_hip_launch(kern->gemvw_finish_mlp[per - 1], ls[0]->n / 128, (rows + 7) / 8, 1, 256, 1, 1, 0, s, fargs);
         }
-        void *fargs[] = {&g, &k, &rows, &mode};
+        if (end == WideEnd::Programs) return 0;
+        void *fargs[] = {&g, &k, &rows, &finish_mode};
         return fe_hip_launch(kern->gemvw_finish[per - 1], (uint32_t)cnt_at, (rows + 7) / 8, 1, 256, 1, 1, 0, s, fargs);
     }
     // staged inputs: the whole run where the LDS budget holds it for `rows` rows, else chunks of a multiple of 4 load steps
@@ -1000,7 +1030,7 @@ int fe_exl3_linear_forward_group_launches(const fe_exl3_linear *const *ls, size_
                                           const fe_exl3_workspace *ws) {
     bool fused = false;
     if (!group_fits(ls, count, rows, ws, &fused)) return 0;
-    return fused ? 1 : rows > 16 ? 3 : 2;
+    return fused ? 1 : rows > 16 && wide_end(ls, count, programs_per(ls, count), rows) != WideEnd::Programs ? 3 : 2;
 }
 
 int fe_exl3_linear_forward_group(const fe_exl3_linear *const *ls, size_t count, const fe_exl3_kernels *kern, fe_stream_t s,

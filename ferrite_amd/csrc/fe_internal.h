@@ -99,6 +99,18 @@ int fe_exl3_forward_prompt_group(const fe_exl3_linear *const *ls, size_t count, 
 // (fe_exl3_static.hip); fe_hip_init calls it for the device it binds.
 int fe_exl3_static_setup_current_device();
 
+// Column blocks of upb units that the decode GEMV of `programs` runs (run q starts at unit q base + min(q, rem)), `per` of them a workgroup, cuts: those inside
+// which a workgroup's run starts.
+inline uint32_t fe_gemv_cut_blocks(uint32_t units, uint32_t programs, uint32_t upb, uint32_t per) {
+    const uint32_t base = units / programs, rem = units % programs;
+    uint32_t cut = 0, last = 0xffffffffu;
+    for (uint32_t q = per; q < programs; q += per) {
+        const uint32_t u = q * base + std::min(q, rem), nb = u / upb;
+        if (u % upb && nb != last) cut++, last = nb;
+    }
+    return cut;
+}
+
 // How the prefill GEMM's output tiles (256 x 256) are spread over the CUs: `full` tiles are computed whole, one per
 // program; the `tiles - full` tiles of a last, mostly empty round are each cut `splits` ways along K (partials in a
 // workspace, then a reduce kernel). splits == 1 means nothing is cut (full == tiles).

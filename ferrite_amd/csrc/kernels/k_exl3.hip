@@ -810,7 +810,8 @@ GEMVB_FAMILY(8)
 // added to the second's before they leave as one segment, as the finisher of gemvb_body adds them. What differs is how a program
 // gets its operands and hands its sums over: both grow with the rows while the decode does not. The rotated inputs and the trellis words of a
 // load step go straight from memory into LDS, DEPTH - 1 steps ahead. Every segment's sums go to z as the accumulators hold them, whole
-// wavefronts at a time, and a launch behind this one (exl3_gemvw_finish*) adds and finishes them with all CUs. (In gemvb_body's hand-off the
+// wavefronts at a time, and a launch behind this one (exl3_gemvw_finish*) adds and finishes them with all CUs, unless the host has the programs finish
+// the column blocks that lie in one run (wide_end). (In gemvb_body's hand-off the
 // program that arrives last at a block reads its segments alone, 12 loads in flight: at 40 rows and 4 bits 10.4 of 22.2 us for q + k + v of the
 // 5120 / 17408 layer, 8.0 of 17.6 for o, 7.6 of 42.8 for gate and up, 14.2 of 34.9 for down; now 13.7 + 4.6, 11.3 + 4.7, 36.4 + 6.1, 21.8 + 5, and the launch
 // behind gate and up leaves down's rotated input as well, which took a launch of 5 us.) A layer at 17 / 40 / 64 rows 107 / 138 / 173 -> 99 / 116 / 140 us. Written through
@@ -823,9 +824,12 @@ struct GemvWide {
     static constexpr int DEPTH = 4 * (X_STAGE + W_STAGE) <= 40 * 1024 ? 4 : 3;  // (so that four programs fit a CU, up to 5 bits)
     static constexpr int W_AT = DEPTH * X_STAGE;
     static constexpr int LX = (2 * RG + 3) / 4, LW = (BITS + 3) / 4;  // loads a wavefront issues a step: 1 KB pieces, some twice
+    static_assert(16 * RG * GEMV_RED_PITCH * 4 <= DEPTH * (X_STAGE + W_STAGE), "a finished block's sums take the stages' place");
 };
-template <int BITS, int RG, int PER>
-__device__ __forceinline__ void gemv_wide_body(const GemvMember& mb, uint32_t p, uint32_t k, uint32_t m) {
+// ENDS: a column block that lies in one run is finished here, from LDS: its sums would travel to memory and back for nothing. (Kernels of their own: beside
+// the code for it the loop takes 1 % longer, decode of 40 rows.)
+template <int BITS, int RG, int PER, bool ENDS>
+__device__ __forceinline__ void gemv_wide_body(const GemvMember& mb, uint32_t p, uint32_t k, uint32_t m, uint32_t y_mode) {
     typedef GemvWide<BITS, RG> C;
     extern __shared__ __attribute__((aligned(16))) unsigned char lds[];
     const uint32_t tid = threadIdx.x, lane = tid & 63, wave = __builtin_amdgcn_readfirstlane(tid >> 6);
@@ -927,6 +931,24 @@ __device__ __forceinline__ void gemv_wide_body(const GemvMember& mb, uint32_t p,
                 for (int rg = 0; rg < RG; rg++) acc[rg][0] = hold[rg][0] + acc[rg][0], acc[rg][1] = hold[rg][1] + acc[rg][1];
             }
         }
+        if (ENDS && units == upb) {
+            g8_loads_wait<0>();  // (the repeated last steps' too)
+            g8_barrier();        // the stages are free for the sums, rows of GEMV_RED_PITCH
+            float* red = (float*)lds + 32 * wave + 16 * (g >> 1) + 4 * (g & 1);
+#pragma unroll
+            for (int rg = 0; rg < RG; rg++)
+#pragma unroll
+                for (int h = 0; h < 2; h++) *(f32x4*)(red + (16 * rg + r) * GEMV_RED_PITCH + 8 * h) = acc[rg][h];
+            __syncthreads();
+            const uint32_t l32 = tid & 31, col = nb * 128 + 4 * l32;
+            for (uint32_t row = tid >> 5; row < m; row += 8) {
+                const f32x4 t = *(const f32x4*)((const float*)lds + row * GEMV_RED_PITCH + 4 * l32);
+                float v[4] = {t[0], t[1], t[2], t[3]};
+                finish_row(v, l32, mb.svh, col, mb.y, y_mode, (size_t)row * n + col);
+            }
+            __syncthreads();
+            continue;
+        }
         unsigned char* zseg = (unsigned char*)(mb.z + (size_t)(p + nb) * m * 128);
 #pragma unroll
         for (int rg = 0; rg < RG; rg++) asm volatile("" : "+v"(acc[rg][0]), "+v"(acc[rg][1]));
@@ -941,17 +963,25 @@ __device__ __forceinline__ void gemv_wide_body(const GemvMember& mb, uint32_t p,
         g8_barrier();             // the stages are free
     }
 }
+// The workgroups whose runs have part in a column block: first .. last (PER programs each).
+struct WideSpan {
+    uint32_t first, last, odd;  // odd: PER 1, the first one is the second of its pair of programs
+};
+template <int PER>
+__device__ __forceinline__ WideSpan wide_span(const GemvMember& mb, uint32_t nb, uint32_t upb) {
+    const uint32_t base = mb.base, rem = mb.rem, cut = rem * (base + 1), ua = nb * upb, ub = ua + upb - 1;
+    const uint32_t first = ua < cut ? udiv_inv(ua, base + 1, mb.inv_base1) : rem + udiv_inv(ua - cut, base, mb.inv_base);
+    const uint32_t last = ub < cut ? udiv_inv(ub, base + 1, mb.inv_base1) : rem + udiv_inv(ub - cut, base, mb.inv_base);
+    if constexpr (PER == 2) return {first >> 1, last >> 1, 0};
+    return {first, last, first & 1};
+}
 // The sums of row `row`, column block nb: what gemv_wide_body's programs left of them, added in gemvb_body's order (programs 2 j and 2 j + 1 to
 // each other, the pairs in order; PER 2: a segment is a pair's). A lane of the half wavefront gets columns 4 l32 .. + 3.
 template <int PER>
-__device__ __forceinline__ f32x4 wide_row_sums(const GemvMember& mb, uint32_t nb, uint32_t upb, uint32_t m, uint32_t row, uint32_t l32) {
-    const uint32_t base = mb.base, rem = mb.rem, cut = rem * (base + 1), ua = nb * upb, ub = ua + upb - 1;
-    uint32_t first = ua < cut ? udiv_inv(ua, base + 1, mb.inv_base1) : rem + udiv_inv(ua - cut, base, mb.inv_base);
-    uint32_t last = ub < cut ? udiv_inv(ub, base + 1, mb.inv_base1) : rem + udiv_inv(ub - cut, base, mb.inv_base);
-    if constexpr (PER == 2) first >>= 1, last >>= 1;
-    const uint32_t odd = PER == 2 ? 0 : first & 1, slots = last - first + 1 + odd;
+__device__ __forceinline__ f32x4 wide_row_sums(const GemvMember& mb, uint32_t nb, const WideSpan& sp, uint32_t m, uint32_t row, uint32_t l32) {
+    const uint32_t odd = sp.odd, slots = sp.last - sp.first + 1 + odd;
     const __amdgpu_buffer_rsrc_t zrs =
-        __builtin_amdgcn_make_buffer_rsrc((void*)(mb.z + (size_t)(first - odd + nb) * m * 128), 0, slots * m * 512, 0x00020000);
+        __builtin_amdgcn_make_buffer_rsrc((void*)(mb.z + (size_t)(sp.first - odd + nb) * m * 128), 0, slots * m * 512, 0x00020000);
     // (zoff of gemv_wide_body: column 32 wave + 16 (g >> 1) + 8 h + 4 (g & 1))
     const uint32_t rg = row / 16, r = row % 16, mr = m - 16 * rg < 16 ? m - 16 * rg : 16, c = l32 & 7;
     const uint32_t piece = ((c >> 1) & 1) * 16 + (l32 >> 3) * 4 + 2 * (c >> 2) + (c & 1), at = 16 * rg * 512 + (piece * mr + r) * 16;
@@ -974,17 +1004,20 @@ __device__ __forceinline__ f32x4 wide_row_sums(const GemvMember& mb, uint32_t nb
     return sum;
 }
 // Finishes the outputs of a launch of gemv_wide_body: grid (column blocks of all members, ceil(m / 8)), 256 threads, a half wavefront a
-// row. Bound by its one read of the segments, which other XCDs have just written (14 MB for down of 40 rows: 5 us).
+// row. Bound by its one read of the segments, which other XCDs have just written (14 MB for down of 40 rows: 5 us). y_mode + WIDE_WHOLE: blocks
+// that lie in one run are finished already.
+#define WIDE_WHOLE 4u
 template <int PER>
 __device__ __forceinline__ void wide_finish_body(const GemvJob& job, uint32_t k, uint32_t m, uint32_t y_mode) {
     const uint32_t l32 = threadIdx.x & 31, row = blockIdx.y * 8 + (threadIdx.x >> 5);
     uint32_t i = 0, nb = blockIdx.x;
     while (nb >= job.m[i].n / 128) nb -= job.m[i++].n / 128;
     const GemvMember& mb = job.m[i];
-    if (row >= m) return;
-    const f32x4 s = wide_row_sums<PER>(mb, nb, k / 128, m, row, l32);
+    const WideSpan sp = wide_span<PER>(mb, nb, k / 128);
+    if (row >= m || ((y_mode & WIDE_WHOLE) && sp.first == sp.last)) return;
+    const f32x4 s = wide_row_sums<PER>(mb, nb, sp, m, row, l32);
     float v[4] = {s[0], s[1], s[2], s[3]};
-    finish_row(v, l32, mb.svh, nb * 128 + 4 * l32, mb.y, y_mode, (size_t)row * mb.n + nb * 128 + 4 * l32);
+    finish_row(v, l32, mb.svh, nb * 128 + 4 * l32, mb.y, y_mode & 3, (size_t)row * mb.n + nb * 128 + 4 * l32);
 }
 // The same for gate and up in front of down: both outputs (bf16), and down's rotated input of SwiGLU(gate, up), a 128-channel block of which
 // is a column block of the two. grid (column blocks of one of them, ceil(m / 8)).
@@ -995,7 +1028,7 @@ __device__ __forceinline__ void wide_finish_mlp_body(const GemvJob& job, uint32_
     u32x2 y[2];
 #pragma unroll
     for (int i = 0; i < 2; i++) {
-        const f32x4 s = wide_row_sums<PER>(job.m[i], nb, k / 128, m, row, l32);
+        const f32x4 s = wide_row_sums<PER>(job.m[i], nb, wide_span<PER>(job.m[i], nb, k / 128), m, row, l32);
         float v[4] = {s[0], s[1], s[2], s[3]};
         fwht128_half_wave(v, l32);
         const u32x2 sv = *(const u32x2*)(job.m[i].svh + c);
@@ -1020,15 +1053,17 @@ __device__ __forceinline__ void wide_finish_mlp_body(const GemvJob& job, uint32_
     }
 WIDE_FINISH_KERNELS(, 1)
 WIDE_FINISH_KERNELS(_pairs, 2)
-#define GEMV_WIDE_KERNEL(NAME, BITS, RG, PER)                                                                         \
-    extern "C" __global__ __launch_bounds__(256, 4) void NAME(GemvJob job, uint32_t k, uint32_t m) {                  \
+#define GEMV_WIDE_KERNEL(NAME, BITS, RG, PER, ENDS)                                                                   \
+    extern "C" __global__ __launch_bounds__(256, 4) void NAME(GemvJob job, uint32_t k, uint32_t m, uint32_t y_mode) { \
         uint32_t i = 0;                                                                                               \
         while (i + 1 < job.count && blockIdx.x >= job.first[i + 1]) i++;                                              \
-        gemv_wide_body<BITS, RG, PER>(job.m[i], blockIdx.x - job.first[i], k, m);                             \
+        gemv_wide_body<BITS, RG, PER, ENDS>(job.m[i], blockIdx.x - job.first[i], k, m, y_mode);               \
     }
 #define GEMV_WIDE_ROWS(BITS, RG)                                    \
-    GEMV_WIDE_KERNEL(exl3_gemvw_b##BITS##_r##RG, BITS, RG, 1)        \
-    GEMV_WIDE_KERNEL(exl3_gemvw_b##BITS##_r##RG##_pairs, BITS, RG, 2)
+    GEMV_WIDE_KERNEL(exl3_gemvw_b##BITS##_r##RG, BITS, RG, 1, false)        \
+    GEMV_WIDE_KERNEL(exl3_gemvw_b##BITS##_r##RG##_ends, BITS, RG, 1, true) \
+    GEMV_WIDE_KERNEL(exl3_gemvw_b##BITS##_r##RG##_pairs, BITS, RG, 2, false) \
+    GEMV_WIDE_KERNEL(exl3_gemvw_b##BITS##_r##RG##_pairs_ends, BITS, RG, 2, true)
 #define GEMV_WIDE_FAMILY(BITS) GEMV_WIDE_ROWS(BITS, 1) GEMV_WIDE_ROWS(BITS, 2) GEMV_WIDE_ROWS(BITS, 3) GEMV_WIDE_ROWS(BITS, 4)
 GEMV_WIDE_FAMILY(2)
 GEMV_WIDE_FAMILY(3)

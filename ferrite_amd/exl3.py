@@ -340,8 +340,8 @@ def forward_group(linears, x, x_dtype: Dtype, ys, y_dtype: Dtype, rows: int, ws:
 
 
 def forward_group_launches(linears, rows: int, ws: "Workspace") -> int:
-    """Launches of forward_group: 1 (the GEMV rotates its input), 2 (a rotation for all members, then the GEMV), 3 (17..64 rows: and
-    the launch that finishes the outputs), 0 (the members run one after the other)."""
+    """Launches of forward_group: 1 (the GEMV rotates its input), 2 (a rotation for all members, then the GEMV), 3 (17..64 rows, unless
+    every column block lies in one program's run: and the launch that finishes the outputs), 0 (the members run one after the other)."""
     return _lib.lib().fe_exl3_linear_forward_group_launches(_group_handles(linears), len(linears), rows, ws.h)
 
 

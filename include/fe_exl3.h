@@ -137,8 +137,8 @@ int fe_exl3_linear_forward_swiglu(const fe_exl3_linear *l, const fe_exl3_kernels
 int fe_exl3_linear_forward_group(const fe_exl3_linear *const *ls, size_t count, const fe_exl3_kernels *kern, fe_stream_t s,
                                  fe_devptr_t x, int x_dtype, const fe_devptr_t *ys, int y_dtype, uint32_t rows,
                                  const fe_exl3_workspace *ws);
-/* Launches of that call: 1, 2 with the rotation's, 3 with the one that finishes the outputs as well (17..64 rows), or 0 when the members
- * run one after the other. */
+/* Launches of that call: 1, 2 with the rotation's, 3 with the one that finishes the outputs as well (17..64 rows, unless every column block
+ * lies in one program's run), or 0 when the members run one after the other. */
 int fe_exl3_linear_forward_group_launches(const fe_exl3_linear *const *ls, size_t count, uint32_t rows,
                                           const fe_exl3_workspace *ws);
 /* The decode MLP block in one launch: yg = x @ W_gate, yu = x @ W_up (bf16 [rows][n]), y (+)= SwiGLU(yg, yu) @ W_down.

@@ -90,3 +90,36 @@ def test_every_plan_of_the_register_gemm_covers_its_tiles(tmp_path):
     subprocess.run(["g++", "-std=c++17", "-O1", "-I", os.path.join(ROOT, "ferrite_amd", "csrc"), "-I", os.path.join(ROOT, "include"), str(src), "-o", exe,
                     "-Wl,--unresolved-symbols=ignore-all"], check=True)
     subprocess.run([exe], check=True)
+
+
+WHOLE = r"""
+#include <cstdio>
+#include "fe_internal.h"
+int main() {
+    for (uint32_t upb = 1; upb <= 9; upb++)
+        for (uint32_t nb = 1; nb <= 24; nb++)
+            for (uint32_t programs = 1; programs <= upb * nb; programs++)
+                for (uint32_t per = 1; per <= 2; per++) {
+                    const uint32_t units = upb * nb, base = units / programs, rem = units % programs;
+                    bool start[9 * 24 + 1] = {};
+                    for (uint32_t q = 0; q < programs; q += per) start[q * base + (q < rem ? q : rem)] = true;
+                    uint32_t cut = 0;
+                    for (uint32_t b = 0; b < nb; b++) {
+                        bool c = false;
+                        for (uint32_t u = 1; u < upb; u++) c = c || start[b * upb + u];
+                        cut += c;
+                    }
+                    if (cut != fe_gemv_cut_blocks(units, programs, upb, per)) return printf("%u %u %u %u\n", upb, nb, programs, per), 1;
+                }
+    return 0;
+}
+"""
+
+
+def test_which_column_blocks_are_cut(tmp_path):
+    src = tmp_path / "whole.cpp"
+    src.write_text(WHOLE)
+    exe = str(tmp_path / "whole")
+    subprocess.run(["g++", "-std=c++17", "-O1", "-I", os.path.join(ROOT, "ferrite_amd", "csrc"), "-I", os.path.join(ROOT, "include"), str(src), "-o", exe,
+                    "-Wl,--unresolved-symbols=ignore-all"], check=True)
+    subprocess.run([exe], check=True)
