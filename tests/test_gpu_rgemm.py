@@ -63,6 +63,29 @@ def test_against_the_oracle(oracle, bits, k, n, m, strips):
         options(kern)
 
 
+@pytest.mark.parametrize("bits,k,n,m,form,pieces", [(4, 2560, 256, 70, 1, 9), (3, 2560, 128, 130, 1, 10), (5, 2560, 384, 200, 2, 17), (4, 2560, 256, 66, 1, 20), (8, 2432, 128, 129, 2, 38)])
+def test_many_pieces_of_a_tile(oracle, bits, k, n, m, form, pieces):
+    """Tiles cut into more pieces than the reduce launch loads at once, a step each at most."""
+    torch, exl3, kern, t, lin, x = setup(k, n, bits, m)
+    ws = exl3.Workspace([lin], m)
+    got = []
+    try:
+        for _ in range(2):
+            options(kern, rgemm_form=form, rgemm_pieces=pieces)
+            y = torch.full((m + 1, n), 3.0, dtype=torch.float32, device="cuda")
+            lin.forward(x, exl3.Dtype.Bf16, y, exl3.Dtype.F32, m, ws)
+            torch.cuda.synchronize()
+            assert (y[m] == 3.0).all()
+            got.append(y[:m].cpu().numpy().astype(np.float64))
+    finally:
+        options(kern)
+    o = oracle.Exl3(t.k, t.n, t.bits, t.trellis, t.suh, t.svh)
+    rows = sorted({0, 1, 15, 16, 63, m // 2, m - 2, m - 1})
+    ref = oracle.gemv_ref(o, oracle.w_hat_f16(o), ws.xh(m, k)[rows])
+    assert np.abs(got[0][rows] - ref).max() < 1e-4 * np.sqrt((ref ** 2).mean())
+    assert np.array_equal(got[0], got[1])
+
+
 @pytest.mark.parametrize("m", [70, 300])
 def test_gate_and_up_in_one_launch(m):
     """The routing layer's prompt over two trellis linears of one input: one launch, the members' own results up to the order of the sums,
