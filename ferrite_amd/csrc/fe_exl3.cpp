@@ -630,7 +630,7 @@ struct RgJobArgs {
         fe_devptr_t xh, trellis, svh, y;
         uint32_t n, stride_k, stride_nb, first;
     } m[kGroupMax];
-    uint32_t count, k, rows, y_mode, tiles_m, tiles_n, group, full, runs, base, rem, pad;
+    uint32_t count, k, rows, y_mode, tiles_m, tiles_n, group, full, runs, base, rem, per;
     fe_devptr_t part;
 };
 static_assert(sizeof(RgJobArgs) == kGroupMax * 48 + 56, "RgJob layout");
@@ -670,7 +670,7 @@ static int launch_rgemm(const fe_exl3_linear *const *ls, size_t count, fe_stream
     const uint32_t rest = p.tiles_m * p.tiles_n - p.full, steps = rest * p.steps();
     j.count = (uint32_t)count, j.k = k, j.rows = rows, j.y_mode = (uint32_t)y_dtype, j.tiles_m = p.tiles_m, j.tiles_n = p.tiles_n;
     j.group = std::min(p.tiles_m, 8u), j.full = p.full, j.runs = p.runs, j.part = ws->part.p;
-    j.base = p.runs ? steps / p.runs : 1, j.rem = p.runs ? steps % p.runs : 0;
+    j.base = p.runs ? steps / p.runs : 1, j.rem = p.runs ? steps % p.runs : 0, j.per = p.runs && p.runs % rest == 0 ? p.runs / rest : 0;
     const uint32_t slot_bits = (uint32_t)bits_slot(ls[0]->bits);
     void *args[] = {&j};
     FE_TRY(fe_hip_launch(kern->rgemm[slot_bits][p.blocks - 1][p.rg / 2 - 3], p.full + p.runs, 1, 1, kGemmThreads, 1, 1, rgemm_lds(ls[0]->bits, p.rg, p.blocks), s, args));

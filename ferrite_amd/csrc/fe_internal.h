@@ -352,8 +352,9 @@ inline FeGemmPlan fe_gemm_plan(uint32_t m, uint32_t n, uint32_t ktiles, uint32_t
 }
 
 // ---- the GEMM that decodes a trellis into registers (k_exl3_rgemm.hip): how a launch is spread --------------------------------
-// A program takes `blocks` column blocks of 128 and 16 rg rows. The first `full` tiles are computed whole, the steps of the others laid end
-// to end and dealt to `runs` programs in equal runs; pieces of a tile meet through the workspace and a reduce launch.
+// A program takes `blocks` column blocks of 128 and 16 rg rows. The first `full` tiles are computed whole, the others by `runs` programs: as many a tile, each
+// an equal part of its steps, where that comes out even, else the tiles' steps laid end to end and dealt in equal runs. Pieces of a tile meet through the
+// workspace and a reduce launch.
 struct FeRgemmPlan {
     uint32_t blocks = 1, rg = 16, tiles_m = 0, tiles_n = 0, full = 0, runs = 0, k = 0;
     float us = 0;
@@ -393,7 +394,7 @@ inline FeRgemmPlan fe_rgemm_plan(uint32_t rows, uint32_t k, const uint32_t *n, u
                 float t = (float)((full + cus - 1) / cus) * (2.0f + (float)all * step_us(full));
                 if (rest) {
                     const uint32_t len = (rest * all + runs - 1) / runs, per = runs / rest;
-                    const bool aligned = per && runs % rest == 0 && all % per == 0;
+                    const bool aligned = per && runs % rest == 0;
                     const uint32_t crossings = aligned ? 0 : (len + all - 2) / all;
                     const float run = (float)len * step_us(runs);
                     t += (full ? 6.0f : 2.0f) + run + (float)crossings * (6.0f + (p.tiles_m > 1 ? 0.08f * run : 0.0f));

@@ -29,12 +29,13 @@ struct RgMember {
     uint32_t n, stride_k, stride_nb, first;  // first: its first column tile among those of the launch
 };
 // The tiles: the members' column tiles, one member after the other, times tiles_m row tiles of BM rows. Programs 0 .. full - 1 take
-// one tile each over all of K. The steps of the tiles after them, laid end to end, are dealt to `runs` programs in equal runs (base
-// steps, the first rem programs one more); a tile that is cut leaves the sums of its pieces, the one of run q in slot q + (tile -
-// full), for the reduce kernel, which adds them in the order of K.
+// one tile each over all of K. The tiles after them are dealt to `runs` programs: `per` a tile, each a per-th of its steps, or (per 0) the tiles' steps laid
+// end to end in equal runs (base steps, the first rem programs one more). Runs that end inside a tile start the next one's products over, and meet
+// the other programs' inputs at another depth of K: where pieces come out even a tile, 3 % of the time of the best plan (589 linears). A tile that is cut leaves the sums of its pieces, the one of run q in slot
+// q + (tile - full), for the reduce kernel, which adds them in the order of K.
 struct RgJob {
     RgMember m[RG_MEMBERS];
-    uint32_t count, k, rows, y_mode, tiles_m, tiles_n, group, full, runs, base, rem, pad;
+    uint32_t count, k, rows, y_mode, tiles_m, tiles_n, group, full, runs, base, rem, per;
     float* part;  // [slot][column block][BM rows][128]
 };
 
@@ -272,12 +273,17 @@ __device__ __forceinline__ void rgemm_segment(const RgJob& job, uint32_t tile, u
         run(std::integral_constant<uint32_t, 3>{});
 }
 
+// The first step of run q, counted from the first tile that is not a program's own
+__device__ __forceinline__ uint32_t rg_start(const RgJob& job, uint32_t q, uint32_t all) {
+    return job.per ? q / job.per * all + q % job.per * all / job.per : sk_start(q, job.base, job.rem);
+}
+
 template <int BITS, int RG, int KG>
 __device__ __forceinline__ void rgemm_body(const RgJob& job) {
     const uint32_t p = blockIdx.x, all = job.k / (64 * KG);
     // a whole tile is a run of its own
-    uint32_t u = p < job.full ? p * all : job.full * all + sk_start(p - job.full, job.base, job.rem);
-    const uint32_t end = p < job.full ? u + all : job.full * all + sk_start(p - job.full + 1, job.base, job.rem);
+    uint32_t u = p < job.full ? p * all : job.full * all + rg_start(job, p - job.full, all);
+    const uint32_t end = p < job.full ? u + all : job.full * all + rg_start(job, p - job.full + 1, all);
     while (u < end) {
         const uint32_t tile = u / all, s0 = u - tile * all, steps = all - s0 < end - u ? all - s0 : end - u;
         rgemm_segment<BITS, RG, KG>(job, tile, s0, steps, p + tile - 2 * job.full, steps == all);
@@ -297,7 +303,8 @@ extern "C" __global__ __launch_bounds__(256) void exl3_rgemm_reduce(RgJob job, u
     while (mi + 1 < job.count && tn >= job.m[mi + 1].first) mi++;
     const RgMember& mb = job.m[mi];
     const uint32_t nb = (tn - mb.first) * blocks + b, at = tm * bm + row;
-    const uint32_t first = sk_owner(t * all, job.base, job.rem), last = sk_owner(t * all + all - 1, job.base, job.rem);
+    const uint32_t first = job.per ? t * job.per : sk_owner(t * all, job.base, job.rem);
+    const uint32_t last = job.per ? first + job.per - 1 : sk_owner(t * all + all - 1, job.base, job.rem);
     if (first == last || nb >= mb.n / 128 || tm * bm + blockIdx.x % per * 8 >= job.rows) return;  // (one run's: finished there)
     const uint32_t slot = blocks * bm * 128;
     const float* p = job.part + (size_t)(first + t) * slot + ((size_t)b * bm + row) * 128 + 4 * l32;
