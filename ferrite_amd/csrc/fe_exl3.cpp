@@ -637,27 +637,42 @@ static_assert(sizeof(RgJobArgs) == kGroupMax * 48 + 56, "RgJob layout");
 
 static bool gemv_reaches(const fe_exl3_linear *l);
 
-// Prompts up to kHatRows go through it under the default switches; those that pick the schedule or the tile of the GEMM that passes the
-// decoded weights through LDS (exl3_gemm_b*) pick that GEMM too. It also takes a trellis of 4 GB and more, which this one addresses by 32
-// bits, and what lies beyond kHatRows. Both, us, LDS / registers, 4 bits: an MLP block of 5120 x 17408 at 70 / 203 / 512 / 2048 rows 138 / 200 / 337 / 1060
-// against 99 / 158 / 302 / 1014, of 2048 x 5632 59 / 75 / 99 / 210 against 38 / 50 / 70 / 190; over 120 random single linears of 2 to 8 bits and 65..2048
-// rows the geometric mean is 0.86, the slowest one (16896 x 1920, 1501 rows) 1.16 of the LDS form's time.
-static bool rgemm_takes(const fe_exl3_linear *l, uint32_t rows) {
+// Whether prompts may go through the GEMM that decodes into registers. Switches that pick the schedule or the tile of the GEMM that passes the
+// decoded weights through LDS (exl3_gemm_b*) pick that GEMM too; it also takes a trellis of 4 GB and more, which this one addresses by 32 bits.
+static bool rgemm_reaches(const fe_exl3_linear *l, uint32_t rows) {
     const fe_exl3_kernels *kern = l->kern;
     const fe_exl3_options &o = kern->opt;
     return o.rgemm && rows > kMaxRowsPerPass && rows < std::min(kHatRows, o.hat_rows) && !l->hat.bytes && gemv_reaches(l) && !kern->tile.force_tile &&
            o.gemm_sk == 1 && o.gemm_splits == 8;
 }
 
-static int launch_rgemm(const fe_exl3_linear *const *ls, size_t count, fe_stream_t s, const fe_devptr_t *xhs, const fe_devptr_t *ys, int y_dtype,
-                        uint32_t rows, const fe_exl3_workspace *ws) {
+// ... and whether they do, by the estimates of both (fe_rgemm_takes): the other one is the faster on some narrow linears, where its smaller tiles
+// need fewer pieces of K. us with the rotation, 4 bits, LDS / the registers alone, by the plan before this estimate / by this rule: 16896 x 1920 at 1501 rows 131 / 136 /
+// 131, 3328 x 1024 at 387 rows 23.1 / 27.7 / 23.0, 2816 x 1024 at 512 rows 22.8 / 27.8 / 23.1 (through LDS), 5120 x 1024 at 128 rows 21.1 / 23.6 / 17.3, 17408 x 5120 at 203, 512
+// and 2048 rows 69.5 / 61.9 / 55.4, 110 / 118 / 105, 370 / 355 / 354, 5120 x 17408 at 203 rows 65.8 / 64.2 / 60.9. MLP blocks: 110 drawn ones take 0.77 of their time through LDS and 0.97 of
+// their time by the plan before (slowest: 1.00 and 1.05).
+static bool rgemm_takes(const fe_exl3_linear *const *ls, size_t count, uint32_t rows, const fe_exl3_workspace *ws, FeRgemmPlan *p) {
     const fe_exl3_kernels *kern = ls[0]->kern;
+    const fe_exl3_options &o = kern->opt;
     const uint32_t k = ls[0]->k, cus = std::max(kern->cus, 1u);
+    uint32_t ns[kGroupMax];
+    float other_us = 0;
+    for (size_t i = 0; i < count; i++) {
+        if (!rgemm_reaches(ls[i], rows)) return false;
+        ns[i] = ls[i]->n;
+        other_us += fe_rgemm_other_us(fe_gemm_plan(rows, ns[i], k / 64, cus, ws->part.p, ws->part.bytes, ws->counters.p, ws->counters_len, 8, 1, true,
+                                                   kFeCostTrellis, FeGemmTileOptions{}), cus);
+    }
+    *p = fe_rgemm_plan(rows, k, ns, (uint32_t)count, cus, ws->part.bytes, o.rgemm_form, o.rgemm_pieces);
+    return o.rgemm_form || o.rgemm_pieces || fe_rgemm_takes(*p, other_us, (uint32_t)count);
+}
+
+static int launch_rgemm(const fe_exl3_linear *const *ls, size_t count, fe_stream_t s, const fe_devptr_t *xhs, const fe_devptr_t *ys, int y_dtype,
+                        uint32_t rows, const fe_exl3_workspace *ws, const FeRgemmPlan &p) {
+    const fe_exl3_kernels *kern = ls[0]->kern;
+    const uint32_t k = ls[0]->k;
     if ((uint64_t)rows * k * 2 >= (1ull << 32))
         return fe_set_error(FE_ERR_UNSUPPORTED, "fe_exl3_linear_gemv_rotated", "rotated input of 4 GB or more");
-    uint32_t ns[kGroupMax];
-    for (size_t i = 0; i < count; i++) ns[i] = ls[i]->n;
-    const FeRgemmPlan p = fe_rgemm_plan(rows, k, ns, (uint32_t)count, cus, ws->part.bytes, kern->opt.rgemm_form, kern->opt.rgemm_pieces);
     RgJobArgs j{};
     uint32_t first = 0;
     for (size_t i = 0; i < count; i++) {
@@ -683,7 +698,8 @@ static int launch_rgemm(const fe_exl3_linear *const *ls, size_t count, fe_stream
 static int launch_gemm(const fe_exl3_linear *l, fe_stream_t s, fe_devptr_t xh, fe_devptr_t y, int y_dtype, uint32_t rows,
                        const fe_exl3_workspace *ws) {
     const fe_exl3_kernels *kern = l->kern;
-    if (rgemm_takes(l, rows)) return launch_rgemm(&l, 1, s, &xh, &y, y_dtype, rows, ws);
+    FeRgemmPlan in_registers;
+    if (rgemm_takes(&l, 1, rows, ws, &in_registers)) return launch_rgemm(&l, 1, s, &xh, &y, y_dtype, rows, ws, in_registers);
     uint32_t n = l->n, k = l->k, mode = (uint32_t)y_dtype, stride_k, stride_nb, group = kern->opt.gemm_group_m;
     view_strides(l->view, &stride_k, &stride_nb);
     if ((uint64_t)rows * k * 2 >= (1ull << 32))
@@ -1077,7 +1093,9 @@ int fe_exl3_forward_prompt_group(const fe_exl3_linear *const *ls, size_t count, 
     *taken = false;
     if (count < 2 || count > kGroupMax || rows > ws->max_rows || !kern->opt.group || ls[0]->k > ws->max_k || count * (size_t)rows * ls[0]->k * 2 > ws->xh.bytes) return 0;
     for (size_t i = 0; i < count; i++)
-        if (ls[i]->k != ls[0]->k || ls[i]->bits != ls[0]->bits || ls[i]->kern != ls[0]->kern || !rgemm_takes(ls[i], rows)) return 0;
+        if (ls[i]->k != ls[0]->k || ls[i]->bits != ls[0]->bits || ls[i]->kern != ls[0]->kern) return 0;
+    FeRgemmPlan p;
+    if (!rgemm_takes(ls, count, rows, ws, &p)) return 0;
     *taken = true;
     RotGroupArgs r{};
     fe_devptr_t xhs[kGroupMax] = {};
@@ -1088,7 +1106,7 @@ int fe_exl3_forward_prompt_group(const fe_exl3_linear *const *ls, size_t count, 
     uint32_t mode = 0, k = ls[0]->k;
     void *args[] = {&r, &x, &mode, &k};
     FE_TRY(fe_hip_launch(kern->rot_in_group, (k + 511) / 512, rows, (uint32_t)count, 128, 1, 1, 0, s, args));
-    return launch_rgemm(ls, count, s, xhs, ys, FE_DTYPE_BF16, rows, ws);
+    return launch_rgemm(ls, count, s, xhs, ys, FE_DTYPE_BF16, rows, ws, p);
 }
 
 // mirrors MlpChain of k_exl3.hip

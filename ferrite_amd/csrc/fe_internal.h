@@ -268,6 +268,7 @@ constexpr uint32_t kFeGemmTileM[3] = {256, 128, 128}, kFeGemmTileN[3] = {256, 25
 struct FeGemmPlan {
     FeGemmSchedule big;  // tile 0
     uint32_t tile = 0, tiles = 0, splits = 1;
+    float us = 0;  // the estimate (0: a tile was forced)
 };
 // Switches of the plan (options of the three kernels handles): force_tile 0 = by the rule, 1 = 256 x 256, 2, 3 = small tile 1, 2
 // with force_pieces pieces of K (0: one).
@@ -327,7 +328,7 @@ inline FeGemmPlan fe_gemm_plan(uint32_t m, uint32_t n, uint32_t ktiles, uint32_t
         take(opt.force_tile - 1, tiles_of(opt.force_tile - 1), most_pieces(opt.force_tile - 1, std::max(1u, opt.force_pieces)));
         return p;
     }
-    if (opt.force_tile == 1 || mode >= 2 || m > 2048 || !cus) return p;
+    if (opt.force_tile == 1 || mode >= 2 || !cus) return p;
     float best;
     if (p.big.stream_k) {
         const FeGemmSchedArgs &a = p.big.args;
@@ -338,14 +339,15 @@ inline FeGemmPlan fe_gemm_plan(uint32_t m, uint32_t n, uint32_t ktiles, uint32_t
         if (g.cut())
             best += fe_gemm_cost(cost, 0, g.cut() * g.splits, (ktiles + g.splits - 1) / g.splits, cus) + fe_gemm_reduce_cost(g.cut() * g.splits, 0);
     }
-    for (uint32_t tile = 1; tile <= 2; tile++) {
+    p.us = best;
+    for (uint32_t tile = 1; tile <= 2 && m <= 2048; tile++) {
         const uint32_t tiles = tiles_of(tile), most = most_pieces(tile, std::min(cap, ktiles / 8));
         for (uint32_t pieces = 1; pieces <= most; pieces++) {
             if (pieces > 1 && tiles * pieces > cus * tile) break;
             float c = fe_gemm_cost(cost, tile, tiles * pieces, (ktiles + pieces - 1) / pieces, cus);
             if (pieces > 1) c += fe_gemm_reduce_cost(tiles * pieces, tile);
             if (tiles * pieces > cus * tile) c *= cost.again;
-            if (1.06f * c < best) take(tile, tiles, pieces), best = 1.06f * c;
+            if (1.06f * c < best) take(tile, tiles, pieces), p.us = c, best = 1.06f * c;
         }
     }
     return p;
@@ -362,12 +364,13 @@ struct FeRgemmPlan {
     bool reduce() const { return runs && runs != tiles_m * tiles_n - full; }
 };
 // The rule: the cheapest by an estimate among one or two column blocks a program, the fewest row tiles of 256 rows at most or one more,
-// all tiles whole, or whole rounds of the CUs (or one round fewer) and the rest in one run a CU or in 2, 3, .. runs a tile. A step costs
-// its matrix instructions, or its decode where the rows are few, and more when the chip is full (clock). Fitted to 1400 timings (120 shapes, 2 to
-// 8 bits, 65..2048 rows, both block counts, 1 to 11 pieces a tile): half of them within 6 %, nine tenths within 17 %. What the fit leaves out
-// and the picks showed, they are its underestimates: runs behind whole rounds and runs that cross from one tile to the next take 4 us
-// more, and where several row tiles share their inputs through L2, runs that cross are at different depths of K and lose that. Forced block
-// counts and pieces: for tests.
+// all tiles whole, or whole rounds of the CUs (or one round fewer) and the rest in one run a CU or in 2, 3, .. runs a tile. Fitted to 10600 timings
+// of 589 single linears (2 to 8 bits, 65..2303 rows, every plan that looked near the best; launches replayed from a graph, without the rotation): half of them
+// within 7 %, nine tenths within 19 %. The plan it picks takes 1.2 % more than the fastest one timed (geometric mean; 5 of 589 more than 10 %, at most 17 %).
+// Its terms: a step's matrix instructions and decode; a program's start, and its output rotation or piece by the tile's size; runs that end inside a tile,
+// which meet their neighbours' inputs at another depth of K, so that with several row tiles each reads them past L2, the more the larger they are; the
+// reduce launch by the pieces' bytes (more a byte where short runs leave them all at once) and by its rounds of eight. Forced block counts and pieces: for
+// tests.
 inline FeRgemmPlan fe_rgemm_plan(uint32_t rows, uint32_t k, const uint32_t *n, uint32_t count, uint32_t cus, size_t part_bytes, uint32_t force_blocks,
                                  uint32_t force_pieces) {
     FeRgemmPlan best;
@@ -383,22 +386,19 @@ inline FeRgemmPlan fe_rgemm_plan(uint32_t rows, uint32_t k, const uint32_t *n, u
             for (uint32_t i = 0; i < count; i++) p.tiles_n += (n[i] / 128 + blocks - 1) / blocks;
             const size_t slot = (size_t)blocks * p.rg * 16 * 512;
             const uint32_t tiles = p.tiles_m * p.tiles_n, all = p.steps(), slots = (uint32_t)(part_bytes / slot);
-            auto step_us = [&](uint32_t programs) {
-                const float fill = std::min(1.0f, (float)programs / (float)cus), rg = (float)p.rg;
-                const float c = std::max(0.74f, 0.325f + 0.075f * rg) * (blocks == 2 ? 0.87f : 1.0f);
-                return c * (1.0f + 0.22f * std::min(1.0f, rg / 13.0f) * std::max(0.0f, (fill - 0.45f) / 0.5f));
-            };
+            const float step = (0.63f + 0.06f * (float)p.rg) * (blocks == 2 ? 0.91f : 1.0f), ends = 0.24f * (float)(p.rg * blocks);
+            const float apart = p.tiles_m > 1 ? 0.35f * (0.3f + std::min(1.0f, (float)rows * (float)k * 2.0f / 32e6f)) : 0.0f;
             auto consider = [&](uint32_t full, uint32_t runs) {
-                const uint32_t rest = tiles - full;
+                const uint32_t rest = tiles - full, rounds = (full + cus - 1) / cus;
                 if (rest && (!runs || runs > rest * all || runs + rest > slots)) return;
-                float t = (float)((full + cus - 1) / cus) * (2.0f + (float)all * step_us(full));
+                float t = full ? 2.7f + 12.0f * (float)(rounds - 1) + (float)rounds * (ends + (float)all * step) : -2.6f;
                 if (rest) {
-                    const uint32_t len = (rest * all + runs - 1) / runs, per = runs / rest;
-                    const bool aligned = per && runs % rest == 0;
-                    const uint32_t crossings = aligned ? 0 : (len + all - 2) / all;
-                    const float run = (float)len * step_us(runs);
-                    t += (full ? 6.0f : 2.0f) + run + (float)crossings * (6.0f + (p.tiles_m > 1 ? 0.08f * run : 0.0f));
-                    if (runs != rest) t += 3.0f + 0.28e-6f * (float)slot * (float)(aligned ? runs : runs + rest);
+                    const uint32_t len = (rest * all + runs - 1) / runs, pieces = (runs + rest - 1) / rest;
+                    const bool even = runs % rest == 0;
+                    t += 5.3f + ends + (float)len * step;
+                    if (!even) t += 6.3f * (float)((len + all - 2) / all) + (float)len * step * apart;
+                    if (runs != rest)
+                        t += 1e-6f * (float)slot * (float)(even ? runs : runs + rest) * (0.2f + 0.45f / (1.0f + (float)len / 3.0f)) + 2.2f * (float)((pieces + 6) / 8);
                 }
                 if (t < best.us) best = p, best.full = full, best.runs = rest ? runs : 0, best.us = t;
             };
@@ -418,6 +418,16 @@ inline FeRgemmPlan fe_rgemm_plan(uint32_t rows, uint32_t k, const uint32_t *n, u
     }
     return best;
 }
+
+// Of the two GEMMs that decode a trellis, whether the one that decodes into registers takes `count` linears in one launch: both estimates, the other GEMM's
+// (its launches together) with what the comparison of 589 single linears showed it to leave out, 12 us a round of programs after the first, and to count twice,
+// 3 us of the reduce launch of cut small tiles. On those linears the rule's pick takes 0.3 % more than the faster of the two (geometric mean); 6 of them take
+// more than 5 % longer than through the other GEMM (at most 15 %), 7 more than 5 % longer than through this one (at most 13 %).
+inline float fe_rgemm_other_us(const FeGemmPlan &p, uint32_t cus) {
+    const uint32_t programs = p.tile ? p.tiles * p.splits : p.big.programs, round = p.tile == 2 ? 2 * cus : cus;
+    return p.us + 12.0f * (float)((std::max(programs, 1u) - 1) / round) - (p.tile && p.splits > 1 ? 3.0f : 0.0f);
+}
+inline bool fe_rgemm_takes(const FeRgemmPlan &p, float other_us, uint32_t count) { return p.us <= other_us + 3.0f * (float)count; }
 
 // Launches a plan. gemm(form, programs, sched): form 0 = 256 x 256 one piece a program, 1 = stream-K, 2, 3 = tile 1, 2;
 // reduce(tile, grid, first, splits): the reduce kernel of a tile, for the tiles from `first` on.

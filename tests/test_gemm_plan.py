@@ -52,6 +52,45 @@ def test_the_tile_that_was_timed_faster(tmp_path):
         assert tile == TIMED[key], key
 
 
+FORM = r"""
+#include <cstdio>
+#include <cstdlib>
+#include "fe_internal.h"
+int main(int argc, char **argv) {
+    for (int i = 1; i + 2 < argc; i += 3) {
+        const uint32_t rows = atoi(argv[i]), n = atoi(argv[i + 1]), k = atoi(argv[i + 2]);
+        const FeRgemmPlan p = fe_rgemm_plan(rows, k, &n, 1, 256, (size_t)512 * kFeGemmPartBytes, 0, 0);
+        const FeGemmPlan g = fe_gemm_plan(rows, n, k / 64, 256, 1, (size_t)512 * kFeGemmPartBytes, 1, 8192, 8, 1, true, kFeCostTrellis, FeGemmTileOptions{});
+        printf("%d\n", (int)fe_rgemm_takes(p, fe_rgemm_other_us(g, 256), 1));
+    }
+}
+"""
+# (rows, columns, K): whether a trellis prompt takes the GEMM that decodes into registers; us of the one that decodes through LDS and of this one
+FORMS = {
+    (507, 2048, 2048): 0,    # 20.2, 23.7
+    (512, 1024, 2816): 0,    # 19.2, 22.2
+    (1416, 896, 1664): 0,    # 21.2, 23.5
+    (915, 2176, 640): 0,     # 14.8, 17.0
+    (65, 2048, 5632): 1,     # 20.1, 14.8
+    (309, 512, 8448): 1,     # 26.3, 19.5
+    (128, 1024, 5120): 1,    # 18.4, 14.3
+    (203, 5120, 17408): 1,   # 66.4, 52.3
+    (512, 5120, 17408): 1,   # 105, 100
+    (2048, 17408, 5120): 1,  # 339, 336
+}
+
+
+def test_the_trellis_gemm_that_was_timed_faster(tmp_path):
+    src = tmp_path / "form.cpp"
+    src.write_text(FORM)
+    exe = str(tmp_path / "form")
+    subprocess.run(["g++", "-std=c++17", "-O1", "-I", os.path.join(ROOT, "ferrite_amd", "csrc"), "-I", os.path.join(ROOT, "include"), str(src), "-o", exe,
+                    "-Wl,--unresolved-symbols=ignore-all"], check=True)
+    args = [str(v) for key in FORMS for v in key]
+    got = [int(v) for v in subprocess.run([exe, *args], stdout=subprocess.PIPE, text=True, check=True).stdout.split()]
+    assert dict(zip(FORMS, got)) == FORMS
+
+
 RGEMM = r"""
 #include <cstdio>
 #include "fe_internal.h"
