@@ -17,9 +17,11 @@
 namespace {
 
 constexpr uint32_t kMaxRowsPerPass = 64;       // 4 row groups of 16
-// Rows from which the prefill decodes once into fp16 tiles (9 output tile rows). Decoding in the GEMM against once, us, at 2048 / 2304 / 3072 rows: 5120 x
-// 17408 at 4 bits 377 / 435 / 548 against 364 / 432 / 522, at 8 bits 398 / 454 / 568 against 377 / 446 / 535, 17408 x 5120 387 / 453 / 546 against 394 / 438 / 515, 5120 x
-// 5120 143 / 143 / 172 against 146 / 139 / 165, 2048 x 5632 68.3 / 72.6 / 98.2 against 69.3 / 73.1 / 96.1.
+// Rows from which the prefill decodes once into fp16 tiles (9 output tile rows). Decoding in the registers (exl3_rgemm_b*) against once, us, at 2048 (or 2100) / 2304 / 2560 (2600) /
+// 3072 / 4096 rows, 4 bits: 5120 x 17408 345 / 388 / 431 / 507 / 667 against 341 / 400 / 434 / 484 / 638, 17408 x 5120 353 / 401 / 449 / 497 / 663 against 374 / 406 / 435 / 479 / 646, 5120 x 5120 126 /
+// 136 / 141 / 158 / 220 against 139 / 132 / 138 / 152 / 210, 4096 x 14336 244 / 251 / 315 / 355 / 461 against 241 / 244 / 308 / 357 / 432, 11008 x 4096 203 / 211 / 248 / 275 / 335 against 243 / 245 / 258 / 272 /
+// 327; at 2 and 8 bits alike. So they meet between 2304 and 2600 rows. Linears below about 16 million weights stay faster in the registers up to 4000 rows (2048 x 2048 39 / 42 / 42 / 47 / 50 against
+// 47 / 50 / 74 / 79 / 64), which this line does not tell apart.
 constexpr uint32_t kHatRows = 2304;
 constexpr uint32_t kChainRows = 8;             // most rows of the one-launch MLP (mlp_chain_fits)
 constexpr uint32_t kWideWhole = 4;             // WIDE_WHOLE of k_exl3.hip

@@ -26,7 +26,7 @@ def options(kern, **o):
 # shortest K, K of an odd count of steps; trellis layouts
 @pytest.mark.parametrize("bits,k,n,m,strips", [(2, 256, 128, 65, True), (3, 384, 384, 96, False), (4, 1024, 384, 97, True), (5, 640, 640, 160, True),
                                                (6, 512, 256, 255, False), (8, 1152, 384, 256, True), (4, 512, 640, 257, False),
-                                               (3, 1024, 256, 449, True), (8, 384, 384, 513, True), (4, 256, 384, 1100, True)])
+                                               (3, 1024, 256, 449, True), (8, 384, 384, 513, True), (4, 256, 384, 1100, True), (3, 256, 256, 2303, True)])
 def test_against_the_oracle(oracle, bits, k, n, m, strips):
     torch, exl3, kern, t, lin, x = setup(k, n, bits, m, strips)
     ws = exl3.Workspace([lin], m)
