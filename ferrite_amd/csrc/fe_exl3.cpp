@@ -1241,7 +1241,8 @@ int fe_exl3_mlp_forward(const fe_exl3_linear *gate, const fe_exl3_linear *up, co
     bool fused = false;
     // From 9 rows on gate and up leave their sums to a launch that finishes them with all CUs and rotates down's input too, in the place of the
     // rotation's launch. A layer, 4 / 5 / 8 bits, at 5 / 8 / 11 / 16 rows, with the finisher inside the GEMV and a rotation / this way: 5120 x 17408 84.7 / 96.4 /
-    // 96.9 / 130.0 us against 85.9 / 97.0 / 93.1 / 123.8, 2560 x 6912 59.3 / 67.6 against 57.5 / 64.8 at 11 / 16.
+    // 96.9 / 130.0 us against 85.9 / 97.0 / 93.1 / 123.8, 2560 x 6912 59.3 / 67.6 against 57.5 / 64.8 at 11 / 16. Over 271 MLP blocks of 9..16 rows (2 to 8 bits, 512 .. 6144 wide) 0.95 of the
+    // time (geometric mean; slowest 1.03: 2560 x 6912 at 9 rows and 2 bits, 31.5 against 32.5 us).
     if (rows > 8 && group_fits(front, 2, rows, ws, &fused) && !fused && down->k <= ws->max_k && (rows > 16 || !kern->opt.handoff_fenced)) {
         FE_TRY(forward_group(front, 2, kern, s, x, x_dtype, ys, FE_DTYPE_BF16, rows, ws, false, dl, fn));
         return launch_rows(dl, s, ws->xh.p, y, y_dtype, rows, ws, RotInput{});

@@ -306,8 +306,9 @@ static int proj_forward(const fe_route_proj *p, const fe_route_ctx *c, uint32_t 
     }
     for (size_t i = first; i < p->lins.size();) {
         // Trellis linears of this input, for a batch the GEMV takes whole in one pass: one grouped launch for up to four of them
-        // (the bits of each linear's own forward); a prompt through the trellis alone likewise, where its GEMM takes them together. The
-        // reference runs them one after the other (model.rs:384-392).
+        // (the bits of each linear's own forward); a prompt through the trellis alone too, where its GEMM takes them together (its tiles are spread as
+        // one launch's, so sums may add in another order than in each linear's own forward). The reference runs them one after the other
+        // (model.rs:384-392).
         size_t j = i;
         const bool gemv = m <= FE_X3_ROWS || (dec >= m && m <= FE_X3_PASS);
         if (c->x3())

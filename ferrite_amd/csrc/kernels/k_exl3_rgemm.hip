@@ -10,13 +10,14 @@
 // instructions of this one; both are pinned there (empty asm statements), since the compiler's scheduler moves all of the decode to the
 // front of the loop, where it runs with the matrix pipe idle.
 //
-// What bounds it: with few rows the decode (330 vector instructions of the two wavefronts of a SIMD a step: 0.70 us at 96 rows), from 160 rows on
-// the board's power: 208 rows of 17408 x 5120 run at 1.76 GHz with the matrix pipe 44 % busy, and the same cycles take a third less time when
-// few CUs work. So what counts beside the balance of the programs is to move and multiply little: row tiles as even and as low as the rows
+// What bounds it: with few rows the decode (96 rows: 156 vector instructions a wavefront and step, 24 of them products; a step of the two wavefronts of a SIMD
+// takes 1980 cycles, the matrix pipe busy 38 %), from 160 rows on the board's power: 208 rows of 17408 x 5120 run at 1.76 GHz with the matrix pipe 47 % busy, and
+// 256 programs of whole tiles take the cycles of 130 of them (399 000) and 22 % more time, 1.73 GHz against 2.14. So what counts beside the balance of the
+// programs is to move and multiply little: row tiles as even and as low as the rows
 // need (203 rows: 224, not 256), rows that do not exist read as zeros, tiles whole where possible (the sums of a cut one travel twice), gate
 // and up in one launch. Loads are issued early in a step (at two stages the wait at the next step's start has to find them done: 17408 x
 // 5120, 224 rows 47.5 -> 43.0 us), words a step earlier than A. us, the GEMM that goes through LDS -> this one, 4 bits, with rotation and reduce
-// launches: 5120 x 17408 at 180 / 480 / 1300 rows 73.7 / 124 / 294 -> 61.5 / 114 / 253, 4096 x 11008 at 330 rows 80 -> 50, MLP blocks at rgemm_takes.
+// launches: 5120 x 17408 at 203 / 512 / 2048 rows 65.8 / 112 / 350 -> 60.9 / 107 / 347, 17408 x 5120 69.5 / 110 / 370 -> 55.4 / 105 / 354, 5120 x 1024 at 128 rows 21.1 -> 17.3.
 #include "exl3_trellis.h"
 #include "gemm8.h"
 

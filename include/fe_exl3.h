@@ -98,7 +98,8 @@ int fe_exl3_workspace_destroy(fe_exl3_workspace *ws);
 int fe_exl3_workspace_xh(const fe_exl3_workspace *ws, fe_devptr_t *xh, uint32_t *max_rows, uint32_t *max_k);
 
 /* Linear::forward (linear.rs:274-287): y[rows][n] = x[rows][k] @ W; x bf16 or f32, y bf16 or f32 (+ the add forms),
- * both row-major and contiguous. rows <= 64 run the decode GEMV (HBM-bound); more rows run the LDS-staged MFMA GEMM.
+ * both row-major and contiguous. rows <= 64 run the decode GEMV (HBM-bound); more rows run an MFMA GEMM: one that decodes the trellis into
+ * registers or one that stages decoded weights in LDS, and from 2304 rows on one over weights decoded once, where the workspace holds them.
  * The workspace's xh holds the rotated input afterwards, as after rotate_input. */
 int fe_exl3_linear_forward(const fe_exl3_linear *l, const fe_exl3_kernels *kern, fe_stream_t s, fe_devptr_t x, int x_dtype,
                            fe_devptr_t y, int y_dtype, uint32_t rows, const fe_exl3_workspace *ws);
@@ -143,7 +144,8 @@ int fe_exl3_linear_forward_group_launches(const fe_exl3_linear *const *ls, size_
                                           const fe_exl3_workspace *ws);
 /* The decode MLP block in one launch: yg = x @ W_gate, yu = x @ W_up (bf16 [rows][n]), y (+)= SwiGLU(yg, yu) @ W_down.
  * Whenever the one launch does not apply the call is fe_exl3_linear_forward_group on {gate, up} followed by
- * fe_exl3_linear_forward_swiglu on down (two launches), with the same bits: a row's result does not depend on the row
+ * fe_exl3_linear_forward_swiglu on down (two launches and their rotations'), and from 9 rows on the rotation, the GEMV of gate and up, a launch that
+ * finishes them and leaves down's rotated input, and down's GEMV (with its finishing launch from 17), with the same bits: a row's result does not depend on the row
  * count of the call (1..64 rows), and every output has the bits of the linear's own forward. Option "chain_down_units"
  * (FE_EXL3_CHAIN_DOWN_UNITS; 2, 4 or 8; default 0 = off; set before the workspace is made) partitions down, in this call
  * only, into programs of that many units of 128 channels x 128 columns where that divides its column blocks, at every row

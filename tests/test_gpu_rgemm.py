@@ -86,6 +86,31 @@ def test_many_pieces_of_a_tile(oracle, bits, k, n, m, form, pieces):
     assert np.array_equal(got[0], got[1])
 
 
+@pytest.mark.parametrize("m,form", [(70, 1), (203, 1), (203, 2), (203, -1), (40, 0)])
+def test_infinities_and_nans_stay_in_their_rows(m, form):
+    """Rows that hold infinities and NaN among ordinary rows of one tile: the others keep their bits (through both GEMMs, form -1 the one
+    that decodes into LDS, and the decode GEMV)."""
+    torch, exl3, kern, t, lin, x = setup(640, 384, 4, m)
+    ws = exl3.Workspace([lin], m)
+    bad = [0, 5, 17, 31, m // 2, m - 1]
+    x2 = x.clone().view(torch.bfloat16)
+    for i, r in enumerate(bad):
+        x2[r, 7 * i + 3] = (float("inf"), float("-inf"), float("nan"))[i % 3]
+    got = []
+    try:
+        options(kern, rgemm=0 if form < 0 else 1, rgemm_form=max(form, 0), rgemm_pieces=3 if form > 0 else 0)
+        for inp in (x, x2):
+            y = torch.zeros((m, 384), dtype=torch.float32, device="cuda")
+            lin.forward(inp, exl3.Dtype.Bf16, y, exl3.Dtype.F32, m, ws)
+            torch.cuda.synchronize()
+            got.append(y)
+    finally:
+        options(kern)
+    fine = [r for r in range(m) if r not in bad]
+    assert torch.equal(got[0][fine], got[1][fine]) and torch.isfinite(got[0]).all()
+    assert not torch.isfinite(got[1][bad]).all(dim=1).any()
+
+
 @pytest.mark.parametrize("m", [70, 300])
 def test_gate_and_up_in_one_launch(m):
     """The routing layer's prompt over two trellis linears of one input: one launch, the members' own results up to the order of the sums,
