@@ -382,10 +382,6 @@ static uint32_t plan_programs(const fe_exl3_kernels *kern, const fe_exl3_plan &p
     return std::max(1u, std::min(progs, units));
 }
 
-static void count_cut_blocks(fe_exl3_linear *l) {
-    for (uint32_t per = 1; per <= 2; per++) l->cut_blocks[per - 1] = fe_gemv_cut_blocks((l->k / 128) * (l->n / 128), l->programs, l->k / 128, per);
-}
-
 // The programs of a partition of the linear in the order in which, as the down projection of a one-launch MLP, their
 // inputs get ready: sorted by the last 128-channel block their run reads (a run that crosses into the next column block
 // reads the last block of all), then by program number. A program of the down stage waits for lower-numbered programs'
@@ -407,16 +403,16 @@ static int make_chain_part(fe_exl3_linear *l, uint32_t unit_len, uint32_t progra
         fe_exl3_linear &sh = *part->as_linear;
         sh.name = l->name, sh.k = l->k, sh.n = l->n, sh.bits = l->bits, sh.plan = l->plan, sh.programs = programs;
         sh.view = l->view, sh.kern = l->kern;
-        count_cut_blocks(&sh);
+        sh.cut_blocks[0] = sh.cut_blocks[1] = sh.n / 128;  // (short runs: taken as cut, so that 17..64 rows are finished by the launch behind)
     }
     l->chain_parts.push_back(std::move(part));
     return 0;
 }
 
 static int make_chain_order(fe_exl3_linear *l) {
-    count_cut_blocks(l);
-    if (int c = make_chain_part(l, 0, l->programs)) return c;
     const uint32_t upb = l->k / 128, units = upb * (l->n / 128);
+    for (uint32_t per = 1; per <= 2; per++) l->cut_blocks[per - 1] = fe_gemv_cut_blocks(units, l->programs, upb, per);
+    if (int c = make_chain_part(l, 0, l->programs)) return c;
     for (uint32_t len : {2u, 4u, 8u})
         if (upb % len == 0 && units / len <= 8192 && units / len != l->programs)
             if (int c = make_chain_part(l, len, units / len)) return c;

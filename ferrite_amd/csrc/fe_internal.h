@@ -103,10 +103,10 @@ int fe_exl3_static_setup_current_device();
 // which a workgroup's run starts.
 inline uint32_t fe_gemv_cut_blocks(uint32_t units, uint32_t programs, uint32_t upb, uint32_t per) {
     const uint32_t base = units / programs, rem = units % programs;
-    uint32_t cut = 0, last = 0xffffffffu;
+    uint32_t cut = 0, nb = 0, in = 0, last = 0xffffffffu;  // the start: unit `in` of block nb
     for (uint32_t q = per; q < programs; q += per) {
-        const uint32_t u = q * base + std::min(q, rem), nb = u / upb;
-        if (u % upb && nb != last) cut++, last = nb;
+        for (in += per * base + std::min(q, rem) - std::min(q - per, rem); in >= upb; in -= upb) nb++;
+        if (in && nb != last) cut++, last = nb;
     }
     return cut;
 }
