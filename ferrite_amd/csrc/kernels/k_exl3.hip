@@ -230,6 +230,28 @@ struct GemvJob {
     GemvMember m[FE_EXL3_GROUP_MAX];
 };
 
+// A launch's arguments lie in memory that no cache of the XCD holds when the launch begins, so the first scalar load of each of their lines is a trip to
+// memory, and left to itself the compiler loads an argument where it is first used: seven such waits, one behind the other, in front of a program's
+// first weights. As inputs of one empty statement (which needs them in registers) every scalar and a word of every line of the members are asked for at
+// once, and then the program's member whole, out of the cache that now holds it. 0.4 us a launch (nothing in launches of few arguments, the rotations): a decode layer of the 5120 / 17408 model at 1 row 69.7 ->
+// 68.5 us, of 7 rows at 5 bits 97.0 -> 94.4, of 40 rows 113.1 -> 109.2; 1024 / 2816 at 1 row (three launches) 27.9 -> 26.7.
+#define GEMV_JOB_LINES(job)                                                                                                              \
+    "s"((job).count), "s"((job).first[1]), "s"((job).first[2]), "s"((job).first[3]), "s"((job).first[4]), "s"((job).m[0].n), "s"((job).m[1].n), \
+        "s"((job).m[2].trellis), "s"((job).m[2].n), "s"((job).m[3].n)
+// the member that workgroup wg belongs to, and that member's first workgroup
+__device__ __forceinline__ uint32_t gemv_member_of(const GemvJob& job, uint32_t wg, uint32_t& first) {
+    uint32_t i = 0;
+    first = 0;
+#pragma unroll
+    for (uint32_t j = 1; j < FE_EXL3_GROUP_MAX; j++)
+        if (j < job.count && wg >= job.first[j]) i = j, first = job.first[j];
+    return i;
+}
+__device__ __forceinline__ void gemv_member_now(const GemvMember& mb) {
+    asm volatile("" ::"s"(mb.trellis), "s"(mb.svh), "s"(mb.suh), "s"(mb.xh), "s"(mb.y), "s"(mb.z), "s"(mb.counters), "s"(mb.n), "s"(mb.programs),
+                 "s"(mb.stride_k), "s"(mb.stride_nb), "s"(mb.base), "s"(mb.rem), "s"(mb.inv_base), "s"(mb.inv_base1));
+}
+
 // x / d for x < 2^31 with inv = floor((2^32 - 1) / d): a multiply-high and one correction (uniform operands: scalar code).
 __device__ __forceinline__ uint32_t udiv_inv(uint32_t x, uint32_t d, uint32_t inv) {
     uint32_t q = __umulhi(x, inv);
@@ -338,7 +360,7 @@ __device__ __forceinline__ uint32_t load_agent_u32(const uint32_t* p) {
 // arrival, an acquire fence, plain loads) instead of write-through stores and loads that pass the L2: the slow form
 // (the release writes the whole L2 back), kept as a cross-check of the fast one (option "handoff_fenced").
 template <int BITS, int CHAIN = 0, bool FENCED = false>
-__device__ __forceinline__ void gemvb_body(const GemvMember& mb, uint32_t p0, uint32_t np, uint32_t k, uint32_t m, uint32_t y_mode,
+__device__ __forceinline__ void gemvb_body(const GemvMember mb, uint32_t p0, uint32_t np, uint32_t k, uint32_t m, uint32_t y_mode,
                                            uint32_t chunk, uint32_t inv_spb, const RotSrc src, uint16_t* stamp_base,
                                            const ChainCtx ch = ChainCtx{}) {
     extern __shared__ __attribute__((aligned(16))) unsigned char lds[];
@@ -729,27 +751,20 @@ __device__ __forceinline__ void gemvb_body(const GemvMember& mb, uint32_t p0, ui
 }
 
 // (second launch bound: wavefronts per SIMD the registers must allow: four programs a CU)
-#define GEMVB_KERNEL(BITS)                                                                                        \
-    extern "C" __global__ __launch_bounds__(256, 4) void exl3_gemvb_b##BITS##_r1(                                      \
+#define GEMVB_KERNEL(NAME, BITS, FENCED)                                                                          \
+    extern "C" __global__ __launch_bounds__(256, 4) void NAME(                                                        \
         GemvJob job, const void* x, const void* x2, uint32_t x_mode, uint32_t ldx, uint32_t k, uint32_t m,             \
         uint32_t y_mode, uint32_t chunk, uint32_t inv_spb, uint32_t fuse) {                                            \
-        uint32_t i = 0;                                                                                               \
-        while (i + 1 < job.count && blockIdx.x >= job.first[i + 1]) i++;                                              \
-        const uint32_t p0 = (blockIdx.x - job.first[i]) * fuse, left = job.m[i].programs - p0;                        \
-        gemvb_body<BITS>(job.m[i], p0, left < fuse ? left : fuse, k, m, y_mode, chunk, inv_spb,                   \
-                             RotSrc{x, x2, x_mode, ldx}, job.m[0].xh);                                                \
+        asm volatile("" ::GEMV_JOB_LINES(job), "s"(x), "s"(x2), "s"(x_mode), "s"(ldx), "s"(k), "s"(m), "s"(y_mode), "s"(chunk), "s"(inv_spb), "s"(fuse)); \
+        uint32_t first;                                                                                               \
+        const GemvMember mb = job.m[gemv_member_of(job, blockIdx.x, first)];                                          \
+        gemv_member_now(mb);                                                                                          \
+        const uint32_t p0 = (blockIdx.x - first) * fuse;                                                              \
+        const uint32_t left = mb.programs - p0;                                                                       \
+        gemvb_body<BITS, 0, FENCED>(mb, p0, left < fuse ? left : fuse, k, m, y_mode, chunk, inv_spb,                  \
+                                    RotSrc{x, x2, x_mode, ldx}, job.m[0].xh);                                         \
     }
-#define GEMVB_FENCED_KERNEL(BITS)                                                                                     \
-    extern "C" __global__ __launch_bounds__(256, 4) void exl3_gemvb_b##BITS##_r1_fenced(                              \
-        GemvJob job, const void* x, const void* x2, uint32_t x_mode, uint32_t ldx, uint32_t k, uint32_t m,             \
-        uint32_t y_mode, uint32_t chunk, uint32_t inv_spb, uint32_t fuse) {                                            \
-        uint32_t i = 0;                                                                                               \
-        while (i + 1 < job.count && blockIdx.x >= job.first[i + 1]) i++;                                              \
-        const uint32_t p0 = (blockIdx.x - job.first[i]) * fuse, left = job.m[i].programs - p0;                        \
-        gemvb_body<BITS, 0, true>(job.m[i], p0, left < fuse ? left : fuse, k, m, y_mode, chunk, inv_spb,           \
-                                     RotSrc{x, x2, x_mode, ldx}, job.m[0].xh);                                        \
-    }
-#define GEMVB_FAMILY(BITS) GEMVB_KERNEL(BITS) GEMVB_FENCED_KERNEL(BITS)
+#define GEMVB_FAMILY(BITS) GEMVB_KERNEL(exl3_gemvb_b##BITS##_r1, BITS, false) GEMVB_KERNEL(exl3_gemvb_b##BITS##_r1_fenced, BITS, true)
 
 // The decode MLP in one launch, 1..16 rows: grid = the front stage's workgroups (gate and up, alternating when their
 // counts are equal, so that block b of both is finished at about the same time), then the down stage's. Down workgroup
@@ -768,24 +783,27 @@ struct MlpChain {
 #define MLP_KERNEL(BITS)                                                                                              \
     extern "C" __global__ __launch_bounds__(256, 4) void exl3_mlp_b##BITS(MlpChain c, const void* x, uint32_t x_mode,  \
                                                                           uint32_t ldx, uint32_t m, uint32_t y_mode) { \
+        asm volatile("" ::"s"(c.front.count), "s"(c.front.first[1]), "s"(c.front.m[0].n), "s"(c.front.m[1].trellis), "s"(c.front.m[1].n),        \
+                     "s"(c.front.m[1].inv_base1), "s"(c.down.trellis), "s"(c.down.n), "s"(c.state), "s"(c.perm), "s"(c.front_wgs), "s"(c.interleave), \
+                     "s"(c.k1), "s"(c.chunk1), "s"(c.inv_spb1), "s"(c.fuse1), "s"(c.k2), "s"(c.chunk2), "s"(c.inv_spb2), "s"(c.fuse2),   \
+                     "s"(c.spin_limit), "s"(x), "s"(x_mode), "s"(ldx), "s"(m), "s"(y_mode));                                          \
         const uint32_t w = blockIdx.x, nbf = c.front.m[0].n / 128, nbd = c.down.n / 128;                              \
         if (w < c.front_wgs) {                                                                                        \
-            uint32_t i = 0, lw = w;                                                                                   \
-            if (c.interleave) {                                                                                       \
-                i = w & 1, lw = w >> 1;                                                                               \
-            } else {                                                                                                  \
-                while (i + 1 < c.front.count && w >= c.front.first[i + 1]) i++;                                       \
-                lw = w - c.front.first[i];                                                                            \
-            }                                                                                                         \
-            const uint32_t p0 = lw * c.fuse1, left = c.front.m[i].programs - p0;                                      \
-            gemvb_body<BITS, 1>(c.front.m[i], p0, left < c.fuse1 ? left : c.fuse1, c.k1, m, 0, c.chunk1, c.inv_spb1, \
+            const uint32_t i = c.interleave ? w & 1 : c.front.count > 1 && w >= c.front.first[1];                     \
+            const uint32_t lw = c.interleave ? w >> 1 : i ? w - c.front.first[1] : w;                                 \
+            const GemvMember mb = c.front.m[i];                                                                       \
+            gemv_member_now(mb);                                                                                      \
+            const uint32_t p0 = lw * c.fuse1, left = mb.programs - p0;                                                \
+            gemvb_body<BITS, 1>(mb, p0, left < c.fuse1 ? left : c.fuse1, c.k1, m, 0, c.chunk1, c.inv_spb1,            \
                                    RotSrc{x, nullptr, x_mode, ldx}, c.front.m[0].xh,                                  \
                                    ChainCtx{c.state, c.state + (1 + i * nbf) * FE_CHAIN_STRIDE, nbf, nbd, c.spin_limit}); \
         } else {                                                                                                      \
             uint32_t lw = w - c.front_wgs;                                                                            \
             if (c.perm) lw = c.perm[lw];                                                                              \
-            const uint32_t p0 = lw * c.fuse2, left = c.down.programs - p0;                                            \
-            gemvb_body<BITS, 2>(c.down, p0, left < c.fuse2 ? left : c.fuse2, c.k2, m, y_mode, c.chunk2, c.inv_spb2, \
+            const GemvMember mb = c.down;                                                                             \
+            gemv_member_now(mb);                                                                                      \
+            const uint32_t p0 = lw * c.fuse2, left = mb.programs - p0;                                                \
+            gemvb_body<BITS, 2>(mb, p0, left < c.fuse2 ? left : c.fuse2, c.k2, m, y_mode, c.chunk2, c.inv_spb2,       \
                                    RotSrc{c.front.m[0].y, c.front.m[1].y, 2, c.front.m[0].n}, c.front.m[0].xh,        \
                                    ChainCtx{c.state, c.state + FE_CHAIN_STRIDE, nbf, nbd, c.spin_limit});             \
         }                                                                                                             \
@@ -829,7 +847,7 @@ struct GemvWide {
 // ENDS: a column block that lies in one run is finished here, from LDS: its sums would travel to memory and back for nothing. (Kernels of their own: beside
 // the code for it the loop takes 1 % longer, decode of 40 rows.)
 template <int BITS, int RG, int PER, bool ENDS>
-__device__ __forceinline__ void gemv_wide_body(const GemvMember& mb, uint32_t p, uint32_t k, uint32_t m, uint32_t y_mode) {
+__device__ __forceinline__ void gemv_wide_body(const GemvMember mb, uint32_t p, uint32_t k, uint32_t m, uint32_t y_mode) {
     typedef GemvWide<BITS, RG> C;
     extern __shared__ __attribute__((aligned(16))) unsigned char lds[];
     const uint32_t tid = threadIdx.x, lane = tid & 63, wave = __builtin_amdgcn_readfirstlane(tid >> 6);
@@ -1009,10 +1027,16 @@ __device__ __forceinline__ f32x4 wide_row_sums(const GemvMember& mb, uint32_t nb
 #define WIDE_WHOLE 4u
 template <int PER>
 __device__ __forceinline__ void wide_finish_body(const GemvJob& job, uint32_t k, uint32_t m, uint32_t y_mode) {
+    asm volatile("" ::GEMV_JOB_LINES(job), "s"(k), "s"(m), "s"(y_mode));
     const uint32_t l32 = threadIdx.x & 31, row = blockIdx.y * 8 + (threadIdx.x >> 5);
-    uint32_t i = 0, nb = blockIdx.x;
-    while (nb >= job.m[i].n / 128) nb -= job.m[i++].n / 128;
-    const GemvMember& mb = job.m[i];
+    uint32_t i = 0, nb = blockIdx.x, before = 0;
+#pragma unroll
+    for (uint32_t j = 1; j < FE_EXL3_GROUP_MAX; j++) {
+        before += job.m[j - 1].n / 128;
+        if (j < job.count && blockIdx.x >= before) i = j, nb = blockIdx.x - before;
+    }
+    const GemvMember mb = job.m[i];
+    gemv_member_now(mb);
     const WideSpan sp = wide_span<PER>(mb, nb, k / 128);
     if (row >= m || ((y_mode & WIDE_WHOLE) && sp.first == sp.last)) return;
     const f32x4 s = wide_row_sums<PER>(mb, nb, sp, m, row, l32);
@@ -1024,7 +1048,9 @@ __device__ __forceinline__ void wide_finish_body(const GemvJob& job, uint32_t k,
 template <int PER>
 __device__ __forceinline__ void wide_finish_mlp_body(const GemvJob& job, uint32_t k, uint32_t m, const uint16_t* suh, uint16_t* xh) {
     const uint32_t l32 = threadIdx.x & 31, row = blockIdx.y * 8 + (threadIdx.x >> 5), nb = blockIdx.x, c = nb * 128 + 4 * l32, n = job.m[0].n;
+    gemv_member_now(job.m[0]);
     if (row >= m) return;
+    gemv_member_now(job.m[1]);
     u32x2 y[2];
 #pragma unroll
     for (int i = 0; i < 2; i++) {
@@ -1055,9 +1081,11 @@ WIDE_FINISH_KERNELS(, 1)
 WIDE_FINISH_KERNELS(_pairs, 2)
 #define GEMV_WIDE_KERNEL(NAME, BITS, RG, PER, ENDS)                                                                   \
     extern "C" __global__ __launch_bounds__(256, 4) void NAME(GemvJob job, uint32_t k, uint32_t m, uint32_t y_mode) { \
-        uint32_t i = 0;                                                                                               \
-        while (i + 1 < job.count && blockIdx.x >= job.first[i + 1]) i++;                                              \
-        gemv_wide_body<BITS, RG, PER, ENDS>(job.m[i], blockIdx.x - job.first[i], k, m, y_mode);               \
+        asm volatile("" ::GEMV_JOB_LINES(job), "s"(k), "s"(m), "s"(y_mode));                                          \
+        uint32_t first;                                                                                               \
+        const GemvMember mb = job.m[gemv_member_of(job, blockIdx.x, first)];                                          \
+        gemv_member_now(mb);                                                                                          \
+        gemv_wide_body<BITS, RG, PER, ENDS>(mb, blockIdx.x - first, k, m, y_mode);                                    \
     }
 #define GEMV_WIDE_ROWS(BITS, RG)                                    \
     GEMV_WIDE_KERNEL(exl3_gemvw_b##BITS##_r##RG, BITS, RG, 1, false)        \
