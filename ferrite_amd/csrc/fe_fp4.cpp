@@ -19,11 +19,12 @@ constexpr uint32_t kTile = 128;                 // crates/fe-fp4/src/lib.rs:28
 constexpr uint32_t kGemmLds[4] = {144 * 1024, 144 * 1024, 136 * 1024, 68 * 1024}, kGemmLds8[4] = {160 * 1024, 160 * 1024, 144 * 1024, 80 * 1024};
 // Forms of the GEMV over programs of 8 CO columns: rows / 2 and CO
 constexpr uint32_t kWideRowForms[4] = {1, 2, 4, 8}, kWideColForms[7] = {1, 2, 3, 4, 5, 6, 9};
-// Fp4Wide<XP, CO>::LDS of k_fp4.hip
-uint32_t wide_lds(uint32_t xp, uint32_t co) {
-    const uint32_t cg = (co + 1) / 2, stage = (co + xp) * 1024 + cg * 256;
-    return std::max(4 * std::max(2u, std::min(20 * 1024 / stage, 6u)) * stage, 256 * (16 * cg + 4));
+// Fp4Wide<XP, CO, Q>::LDS of k_fp4.hip; Q (rows m of k quantized by the program itself): with its four wavefronts' activations in the place of a stage's
+uint32_t wide_lds(uint32_t xp, uint32_t co, bool q = false, uint32_t m = 0, uint32_t k = 0) {
+    const uint32_t cg = (co + 1) / 2, stage = (co + (q ? 0 : xp)) * 1024 + cg * 256, x = q ? ((k / 256 + 3) / 4 * m + 1) / 2 * 4096 : 0;
+    return std::max(4 * std::max(2u, std::min((q ? 15 : 20) * 1024 / stage, 6u)) * stage + x, 256 * (16 * cg + 4));
 }
+constexpr uint32_t kCuLds = 160 * 1024;
 constexpr uint32_t kGemmThreads = 512;
 constexpr uint32_t kTileM = 256;                        // GM_BM
 }  // namespace
@@ -34,6 +35,7 @@ struct fe_fp4_kernels {
     // by form (256 x 256, stream-K, 128 x 256, 128 x 128) and by tile (fe_gemm_launch); gemm8: the fp16 form, 256 x 256 only
     fe_function_t gemm4[4] = {}, swiglu4[4] = {}, gemm8c[4] = {}, gemm8[2] = {}, reduce4[3] = {}, swiglu_reduce4[3] = {}, reduce8c[3] = {};
     fe_function_t wide[4][7] = {};   // the GEMV over programs of 8 CO columns, [kWideRowForms][kWideColForms]
+    fe_function_t wide_q[3][7] = {};  // the same, quantizing its activations itself
     fe_function_t quant8 = nullptr, expand8 = nullptr;
     uint32_t cus = 0;
     // Switches of the launch paths: read from the environment once, at load; fe_fp4_kernels_set_option changes them
@@ -42,6 +44,7 @@ struct fe_fp4_kernels {
     uint32_t gemv = 1;         // up to 64 rows run the GEMV (FE_FP4_NO_GEMV=1: the GEMM's single tile row)
     uint32_t gemv_sk = 0;      // K splits of the GEMV over weight tiles; 0 = two programs a CU (FE_FP4_GEMV_SK)
     uint32_t gemv_strips = 1;  // up to 16 rows run programs of some columns over all of K; 0: weight tiles and K splits, as more rows do (FE_FP4_NO_STRIPS=1)
+    uint32_t gemv_quant = 10240;  // most values (rows x k) that the GEMV for up to 16 rows quantizes itself, in every program (FE_FP4_GEMV_QUANT)
     uint32_t gemv_cols = 0;    // columns a program of the GEMV for up to 16 rows takes, rounded up to 8, 16, .. 48, 72; 0 = by the shape (FE_FP4_GEMV_COLS)
     int32_t xcd = -1;          // column tiles dealt to the XCDs: -1 = where the weights are the larger operand (FE_FP4_XCD)
     uint32_t fp8_f16 = 0;      // FP8 linears as fp16 expansion on the 16-bit matrix instruction (FE_FP8_F16=1)
@@ -100,6 +103,9 @@ int fe_fp4_kernels_load(fe_fp4_kernels **out) {
         for (uint32_t j = 0; j < 7; j++)
             get(&k->wide[i][j], "fe_gemv_nvfp4_r" + std::to_string(kWideRowForms[i]) + "_c" + std::to_string(kWideColForms[j]),
                 wide_lds(kWideRowForms[i], kWideColForms[j]));
+    for (uint32_t i = 0; i < 3; i++)
+        for (uint32_t j = 0; j < 7; j++)
+            get(&k->wide_q[i][j], "fe_gemv_nvfp4_q" + std::to_string(kWideRowForms[i]) + "_c" + std::to_string(kWideColForms[j]), kCuLds);
     if (!c) c = fe_hip_module_get_function(&k->quant8, k->module, "fe_fp8_quant");
     if (!c) c = fe_hip_module_get_function(&k->expand8, k->module, "fe_fp8_expand");
     int cus = 0;
@@ -109,6 +115,7 @@ int fe_fp4_kernels_load(fe_fp4_kernels **out) {
     if (const char *e = getenv("FE_FP4_NO_GEMV")) k->gemv = atoi(e) ? 0 : 1;
     if (const char *e = getenv("FE_FP4_GEMV_SK")) k->gemv_sk = (uint32_t)atoi(e);
     if (const char *e = getenv("FE_FP4_NO_STRIPS")) k->gemv_strips = atoi(e) ? 0 : 1;
+    if (const char *e = getenv("FE_FP4_GEMV_QUANT")) k->gemv_quant = (uint32_t)atoi(e);
     if (const char *e = getenv("FE_FP4_GEMV_COLS")) k->gemv_cols = (uint32_t)atoi(e);
     if (const char *e = getenv("FE_FP4_XCD")) k->xcd = atoi(e) ? 1 : 0;
     if (const char *e = getenv("FE_FP8_F16")) k->fp8_f16 = atoi(e) ? 1 : 0;
@@ -135,6 +142,7 @@ int fe_fp4_kernels_set_option(fe_fp4_kernels *k, const char *name, int32_t value
     if (nm == "group_m") k->group_m = (uint32_t)value;
     else if (nm == "gemv") k->gemv = value ? 1 : 0;
     else if (nm == "gemv_sk") k->gemv_sk = (uint32_t)value;
+    else if (nm == "gemv_quant") k->gemv_quant = (uint32_t)value;
     else if (nm == "gemv_cols") k->gemv_cols = value;
     else if (nm == "gemv_strips") k->gemv_strips = (uint32_t)value;
     else if (nm == "gemv_once" || nm == "gemv_waves") (void)value;  // of a kernel that is no more: accepted, without effect
@@ -315,16 +323,22 @@ int fe_fp4_workspace_operand(const fe_fp4_workspace *ws, fe_devptr_t *aq) {
     return 0;
 }
 
-int fe_fp4_linear_quantize(const fe_fp4_linear *l, const fe_fp4_kernels *kern, fe_stream_t s, const fe_fp4_workspace *ws,
-                           fe_devptr_t x, uint32_t lda, uint32_t m) {
+static int check_quantize(const fe_fp4_linear *l, const fe_fp4_kernels *kern, const fe_fp4_workspace *ws, fe_devptr_t x, uint32_t lda, uint32_t m) {
     if (!l || !kern || !ws) return fe_set_error(FE_ERR_ARG, "fe_fp4_linear_quantize", "null argument");
     if (m > ws->max_rows || l->k > ws->max_k) {  // lib.rs:521-522
         char msg[200];
         snprintf(msg, sizeof msg, "%s: workspace %ux%u < %ux%u", l->name.c_str(), ws->max_rows, ws->max_k, m, l->k);
         return fe_set_error(FE_ERR_WORKSPACE, "fe_fp4_linear_quantize", msg);
     }
+    if (m && (!x || lda < l->k || lda % 8 || x % 16))
+        return fe_set_error(FE_ERR_ARG, "fe_fp4_linear_quantize", "x must be 16-byte aligned rows of >= k");
+    return 0;
+}
+
+int fe_fp4_linear_quantize(const fe_fp4_linear *l, const fe_fp4_kernels *kern, fe_stream_t s, const fe_fp4_workspace *ws,
+                           fe_devptr_t x, uint32_t lda, uint32_t m) {
+    FE_TRY(check_quantize(l, kern, ws, x, lda, m));
     if (m == 0) return 0;
-    if (!x || lda < l->k || lda % 8 || x % 16) return fe_set_error(FE_ERR_ARG, "fe_fp4_linear_quantize", "x must be 16-byte aligned rows of >= k");
     uint32_t k = l->k;
     float g = l->g;
     fe_devptr_t codes = ws->codes.p, sf = ws->sf.p, aq = ws->aq.p;
@@ -344,11 +358,11 @@ int fe_fp4_linear_quantize(const fe_fp4_linear *l, const fe_fp4_kernels *kern, f
 // 28.8 us against 29.8 at 48 columns; at 1 row 25.6. Against the weight tiles (gemv_strips = 0), which are ahead at one width: 5120 columns of
 // 17408 at 8 / 9 / 12 / 16 rows 19.1 / 20.0 / 20.5 / 21.3 us against 18.4 / 18.8 / 19.2 / 19.9. They are not taken there because a row's bits are to
 // be the same at 1 to 16 rows, and at 1 row it is 15.4 against 18.3 (5120 columns of 8704: 1 / 12 rows 10.6 / 13.3 against 13.8 / 14.1).
-static uint32_t wide_cols(uint32_t n, uint32_t xp, uint32_t cus, uint32_t forced) {
+static uint32_t wide_cols(uint32_t n, uint32_t xp, uint32_t cus, uint32_t forced, bool q = false, uint32_t m = 0, uint32_t k = 0) {
     uint32_t best = 0;
     uint64_t least = ~0ull;
     for (uint32_t i = 0; i < 7; i++) {
-        const uint32_t co = kWideColForms[i], programs = (n / 8 + co - 1) / co, room = wide_lds(xp, co) <= 80 * 1024 ? 2 : 1;
+        const uint32_t co = kWideColForms[i], programs = (n / 8 + co - 1) / co, room = wide_lds(xp, co, q, m, k) <= 80 * 1024 ? 2 : 1;
         if (forced) {
             best = i;
             if (8 * co >= forced) break;
@@ -363,9 +377,13 @@ static uint32_t wide_cols(uint32_t n, uint32_t xp, uint32_t cus, uint32_t forced
     return best;
 }
 
-int fe_fp4_linear_gemm(const fe_fp4_linear *l, const fe_fp4_kernels *kern, fe_stream_t s, const fe_fp4_workspace *ws,
-                       fe_devptr_t y, uint32_t ldy, uint32_t m, fe_devptr_t res) {
-    if (!l || !kern || !ws) return fe_set_error(FE_ERR_ARG, "fe_fp4_linear_gemm", "null argument");
+// Whether fe_fp4_linear_gemm takes the GEMV of up to 16 rows over programs of some columns and all of K, nothing handed between them.
+static bool takes_wide(const fe_fp4_linear *l, const fe_fp4_kernels *kern, uint32_t m) {
+    return !l->fp8 && m <= 16 && l->n / kTile <= kGemvCounters && kern->gemv && kern->gemv_strips && !kern->gemv_sk && l->k % 256 == 0;
+}
+// x: null, or the activations (bf16 rows of lda) which that GEMV quantizes itself
+static int linear_gemm(const fe_fp4_linear *l, const fe_fp4_kernels *kern, fe_stream_t s, const fe_fp4_workspace *ws, fe_devptr_t y, uint32_t ldy,
+                       uint32_t m, fe_devptr_t res, fe_devptr_t x, uint32_t lda) {
     if (m == 0) return 0;  // lib.rs:535-537
     if (m > ws->max_rows || l->k > ws->max_k) return fe_set_error(FE_ERR_WORKSPACE, "fe_fp4_linear_gemm", "rows or k exceed the workspace");
     // lib.rs:156-157
@@ -376,14 +394,18 @@ int fe_fp4_linear_gemm(const fe_fp4_linear *l, const fe_fp4_kernels *kern, fe_st
         // decode-sized: the weight-read-bound GEMV, up to 48 rows a pass. Two programs fit a CU: as many programs as run
         // at once, not more (a second round of short programs costs more than idle CUs in the first).
         const uint32_t nts = n / kTile, kts = k / 64;
-        // up to 16 rows: programs of some columns over all of K, nothing handed between them
-        if (kern->gemv_strips && !kern->gemv_sk && m <= 16 && k % 256 == 0) {
+        if (takes_wide(l, kern, m)) {
             const uint32_t form = m <= 2 ? 0 : m <= 4 ? 1 : m <= 8 ? 2 : 3, xp = kWideRowForms[form];
-            const uint32_t cols = wide_cols(n, xp, std::max(kern->cus, 1u), kern->gemv_cols), co = kWideColForms[cols];
-            fe_devptr_t aq = ws->aq.p, w = l->w.p, sw = l->sw.p, alpha = l->alpha.p;
+            const uint32_t cols = wide_cols(n, xp, std::max(kern->cus, 1u), kern->gemv_cols, x != 0, m, k), co = kWideColForms[cols];
+            struct {  // Fp4QuantTo
+                fe_devptr_t codes, sf, aq;
+                uint32_t ldx;
+                float g;
+            } to = {ws->codes.p, ws->sf.p, ws->aq.p, lda, l->g};
+            fe_devptr_t aq = x ? x : ws->aq.p, w = l->w.p, sw = l->sw.p, alpha = l->alpha.p;
             uint32_t w_snt = l->w_snt, w_skt = l->w_skt, w_sr = l->w_sr, s_snt = l->s_snt, s_skt = l->s_skt, s_sr = l->s_sr;
-            void *args[] = {&y, &aq, &w, &sw, &alpha, &res, &m, &n, &k, &ldy, &w_snt, &w_skt, &w_sr, &s_snt, &s_skt, &s_sr};
-            return fe_hip_launch(kern->wide[form][cols], (n / 8 + co - 1) / co, 1, 1, 256, 1, 1, wide_lds(xp, co), s, args);
+            void *args[] = {&y, &aq, &w, &sw, &alpha, &res, &m, &n, &k, &ldy, &w_snt, &w_skt, &w_sr, &s_snt, &s_skt, &s_sr, &to};
+            return fe_hip_launch(x ? kern->wide_q[form][cols] : kern->wide[form][cols], (n / 8 + co - 1) / co, 1, 1, 256, 1, 1, wide_lds(xp, co, x != 0, m, k), s, args);
         }
         uint32_t sk = 2 * kern->cus / nts;
         if (kern->gemv_sk) sk = kern->gemv_sk;
@@ -451,8 +473,29 @@ int fe_fp4_linear_gemm(const fe_fp4_linear *l, const fe_fp4_kernels *kern, fe_st
         });
 }
 
+int fe_fp4_linear_gemm(const fe_fp4_linear *l, const fe_fp4_kernels *kern, fe_stream_t s, const fe_fp4_workspace *ws,
+                       fe_devptr_t y, uint32_t ldy, uint32_t m, fe_devptr_t res) {
+    if (!l || !kern || !ws) return fe_set_error(FE_ERR_ARG, "fe_fp4_linear_gemm", "null argument");
+    return linear_gemm(l, kern, s, ws, y, ldy, m, res, 0, 0);
+}
+
+// Whether the GEMV's programs each quantize all of the activations: few values, since a program waits for all of them before its first product. us, with the
+// quantizer's launch -> without: 1024 x 1024 at 1 / 8 rows 6.9 -> 3.8, 7.1 -> 4.1; 5120 x 5120 at 1 / 2 rows 8.7 -> 7.3, 8.9 -> 8.0; 17408 x 5120 at 1 / 2 15.8 -> 14.0,
+// 16.2 -> 14.5; 34816 x 5120 at 2 24.7 -> 23.7; 16384 x 2560 at 4 9.3 -> 8.3; 5120 x 8704 at 1 11.5 -> 10.0. Beyond 10240 values it turns: 34816 x 5120 at 3 rows
+// 25.2 -> 27.0, 5120 x 8704 at 3 11.7 -> 12.6, 16384 x 2560 at 6 10.2 -> 14.3 (one program a CU). Up to 8 rows, what the LDS holds and 32 bits address. Not where the output or the
+// workspace lies in the activations' memory: programs that have finished would write over what others have yet to read.
+static bool fp4_quants_itself(const fe_fp4_linear *l, const fe_fp4_kernels *kern, const fe_fp4_workspace *ws, fe_devptr_t y, uint32_t ldy, fe_devptr_t x,
+                              uint32_t lda, uint32_t m) {
+    if (!m || m > 8 || !takes_wide(l, kern, m) || (uint64_t)m * l->k > std::min(kern->gemv_quant, 32768u) || (uint64_t)m * lda >= (1u << 30)) return false;
+    const fe_devptr_t xe = x + ((size_t)(m - 1) * lda + l->k) * 2;
+    auto apart = [&](fe_devptr_t p, size_t bytes) { return p + bytes <= x || p >= xe; };
+    return apart(y, ((size_t)(m - 1) * ldy + l->n) * 2) && apart(ws->codes.p, ws->codes.bytes) && apart(ws->sf.p, ws->sf.bytes) && apart(ws->aq.p, ws->aq.bytes);
+}
+
 int fe_fp4_linear_forward(const fe_fp4_linear *l, const fe_fp4_kernels *kern, fe_stream_t s, const fe_fp4_workspace *ws,
                           fe_devptr_t y, uint32_t ldy, fe_devptr_t x, uint32_t lda, uint32_t m, fe_devptr_t res) {
+    FE_TRY(check_quantize(l, kern, ws, x, lda, m));
+    if (fp4_quants_itself(l, kern, ws, y, ldy, x, lda, m)) return linear_gemm(l, kern, s, ws, y, ldy, m, res, x, lda);
     FE_TRY(fe_fp4_linear_quantize(l, kern, s, ws, x, lda, m));
     return fe_fp4_linear_gemm(l, kern, s, ws, y, ldy, m, res);
 }

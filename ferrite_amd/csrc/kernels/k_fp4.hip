@@ -132,9 +132,73 @@ __device__ __forceinline__ uint32_t sf_tiled(uint32_t row, uint32_t b, uint32_t 
     return ((row >> 7) * (kb >> 3) + (b >> 3)) * 1024 + (row & 127) * 8 + (b & 7);
 }
 
+// A block of 16 bf16 values (r0: 0..7, r1: 8..15): sf = e4m3(amax * (1/6) * g), q = e2m1(x * (g / sf)), and o = 2 * code value * block scale as fp16.
+struct Fp4Block {
+    u32x2 q;
+    uint32_t s8;
+    u32x4 o[2];
+};
+// Without a NaN among the values: their magnitudes as bf16 bits are in order, so the largest is a maximum of 16-bit integers, and the conversions are the
+// hardware's; a block with a NaN (a magnitude above infinity's) goes through e2m1_nan_to_zero.
+__device__ __forceinline__ Fp4Block fp4_quant_block(u32x4 r0, u32x4 r1, float g) {
+    typedef uint16_t u16x2 __attribute__((ext_vector_type(2)));
+    u16x2 top = {0, 0};
+#pragma unroll
+    for (int j = 0; j < 4; j++) {
+        top = __builtin_elementwise_max(top, __builtin_bit_cast(u16x2, r0[j] & 0x7fff7fffu));
+        top = __builtin_elementwise_max(top, __builtin_bit_cast(u16x2, r1[j] & 0x7fff7fffu));
+    }
+    uint32_t amax = top[0] > top[1] ? top[0] : top[1];
+    const bool nan = amax > 0x7f80u;
+    if (nan) {  // the largest of the others
+        amax = 0;
+#pragma unroll
+        for (int j = 0; j < 8; j++) {
+            const uint32_t w = j < 4 ? r0[j & 3] : r1[j & 3], lo = w & 0x7fffu, hi = (w >> 16) & 0x7fffu;
+            if (lo <= 0x7f80u && lo > amax) amax = lo;
+            if (hi <= 0x7f80u && hi > amax) amax = hi;
+        }
+    }
+    Fp4Block out;
+    out.s8 = f32_to_e4m3_pos(__uint_as_float(amax << 16) * (1.0f / 6.0f) * g);
+    float sv = e4m3_to_f32(out.s8);
+    float mul = sv > 0.f ? g / sv : 0.f;
+    const f16x2 sc = e4m3_to_f16x2(out.s8);
+    const bool careful = nan || !(mul <= 3.402823466e38f);  // (0 times infinity)
+#pragma unroll
+    for (int w = 0; w < 2; w++) {
+        float f[8];
+#pragma unroll
+        for (int j = 0; j < 4; j++) {
+            const uint32_t v = w ? r1[j] : r0[j];
+            f[2 * j] = __uint_as_float(v << 16) * mul, f[2 * j + 1] = __uint_as_float(v & 0xffff0000u) * mul;
+        }
+        if (careful) {
+#pragma unroll
+            for (int j = 0; j < 8; j++) f[j] = e2m1_nan_to_zero(f[j]);
+        }
+        uint32_t q = 0;
+        q = __builtin_amdgcn_cvt_scalef32_pk_fp4_f32(q, f[0], f[1], 1.0f, 0);
+        q = __builtin_amdgcn_cvt_scalef32_pk_fp4_f32(q, f[2], f[3], 1.0f, 1);
+        q = __builtin_amdgcn_cvt_scalef32_pk_fp4_f32(q, f[4], f[5], 1.0f, 2);
+        q = __builtin_amdgcn_cvt_scalef32_pk_fp4_f32(q, f[6], f[7], 1.0f, 3);
+        out.q[w] = q;
+        const f16x2 v0 = __builtin_amdgcn_cvt_scalef32_pk_f16_fp4(q, 2.0f, 0) * sc, v1 = __builtin_amdgcn_cvt_scalef32_pk_f16_fp4(q, 2.0f, 1) * sc;
+        const f16x2 v2 = __builtin_amdgcn_cvt_scalef32_pk_f16_fp4(q, 2.0f, 2) * sc, v3 = __builtin_amdgcn_cvt_scalef32_pk_f16_fp4(q, 2.0f, 3) * sc;
+        out.o[w] = (u32x4){__builtin_bit_cast(uint32_t, v0), __builtin_bit_cast(uint32_t, v1), __builtin_bit_cast(uint32_t, v2), __builtin_bit_cast(uint32_t, v3)};
+    }
+    return out;
+}
+// Block b of row `row` where fe_fp4_quant leaves it.
+__device__ __forceinline__ void fp4_store_block(const Fp4Block& v, uint8_t* codes, uint8_t* sf, _Float16* aq, uint32_t row, uint32_t b, uint32_t k) {
+    *(u32x2*)(codes + (size_t)row * (k >> 1) + b * 8) = v.q;
+    sf[sf_tiled(row, b, k >> 4)] = (uint8_t)v.s8;
+    u32x4* ap = (u32x4*)(aq + (size_t)row * k + b * 16);
+    ap[0] = v.o[0], ap[1] = v.o[1];
+}
+
 // bf16 x[M][ldx] -> codes [M][K/2], e4m3 block scales (tiled layout), and the dequantized operand the GEMM reads:
-// aq[M][K] fp16 = 2 * code value * block scale. sf = e4m3(amax16 * (1/6) * g), q = e2m1(x * (g / sf)).
-// One thread per 16-element block: grid ceil(M * K / 16 / 256), 256 threads.
+// aq[M][K] fp16 = 2 * code value * block scale. One thread per 16-element block: grid ceil(M * K / 16 / 256), 256 threads.
 // (kernels/k-fp4/src/lib.rs:162-197; CPU form crates/fe-fp4/src/format.rs:72-90)
 extern "C" __global__ __launch_bounds__(256) void fe_fp4_quant(uint8_t* codes, uint8_t* sf, _Float16* aq, const uint16_t* x,
                                                                uint32_t m, uint32_t k, uint32_t ldx, float g) {
@@ -143,44 +207,7 @@ extern "C" __global__ __launch_bounds__(256) void fe_fp4_quant(uint8_t* codes, u
     if (i >= m * kb) return;
     uint32_t row = i / kb, b = i - row * kb;
     const u32x4* p = (const u32x4*)(x + (size_t)row * ldx + b * 16);
-    u32x4 r0 = p[0], r1 = p[1];
-    float f[16];
-#pragma unroll
-    for (int j = 0; j < 4; j++) {
-        f[2 * j] = __uint_as_float(r0[j] << 16), f[2 * j + 1] = __uint_as_float(r0[j] & 0xffff0000u);
-        f[8 + 2 * j] = __uint_as_float(r1[j] << 16), f[9 + 2 * j] = __uint_as_float(r1[j] & 0xffff0000u);
-    }
-    float amax = 0.f;
-#pragma unroll
-    for (int j = 0; j < 16; j++) amax = __builtin_fmaxf(amax, __builtin_fabsf(f[j]));
-    uint32_t s8 = f32_to_e4m3_pos(amax * (1.0f / 6.0f) * g);
-    float sv = e4m3_to_f32(s8);
-    float mul = sv > 0.f ? g / sv : 0.f;
-    uint32_t q[2] = {0, 0};
-#pragma unroll
-    for (int w = 0; w < 2; w++) {
-        q[w] = f32x2_to_e2m1_byte<0>(q[w], f[8 * w + 0] * mul, f[8 * w + 1] * mul);
-        q[w] = f32x2_to_e2m1_byte<1>(q[w], f[8 * w + 2] * mul, f[8 * w + 3] * mul);
-        q[w] = f32x2_to_e2m1_byte<2>(q[w], f[8 * w + 4] * mul, f[8 * w + 5] * mul);
-        q[w] = f32x2_to_e2m1_byte<3>(q[w], f[8 * w + 6] * mul, f[8 * w + 7] * mul);
-    }
-    u32x2 qv = {q[0], q[1]};
-    *(u32x2*)(codes + (size_t)row * (k >> 1) + b * 8) = qv;
-    sf[sf_tiled(row, b, kb)] = (uint8_t)s8;
-    f16x2 sc = e4m3_to_f16x2(s8);
-    uint32_t o[8];
-    {
-        uint32_t t[4];
-        e2m1x8_to_f16(q[0], t);
-#pragma unroll
-        for (int j = 0; j < 4; j++) o[j] = __builtin_bit_cast(uint32_t, (f16x2)(__builtin_bit_cast(f16x2, t[j]) * sc));
-        e2m1x8_to_f16(q[1], t);
-#pragma unroll
-        for (int j = 0; j < 4; j++) o[4 + j] = __builtin_bit_cast(uint32_t, (f16x2)(__builtin_bit_cast(f16x2, t[j]) * sc));
-    }
-    u32x4* ap = (u32x4*)(aq + (size_t)row * k + b * 16);
-    ap[0] = (u32x4){o[0], o[1], o[2], o[3]};
-    ap[1] = (u32x4){o[4], o[5], o[6], o[7]};
+    fp4_store_block(fp4_quant_block(p[0], p[1], g), codes, sf, aq, row, b, k);
 }
 
 // ---- GEMM --------------------------------------------------------------------------------------------------------------
@@ -834,39 +861,50 @@ FP4_GEMV_KERNEL(3)  // (four groups of rows would not fit the registers of two p
 // along K (whose partial sums meet through memory; 17 rows and more still run there). us with the quantizer's launch, before -> now:
 // 5120 x 34816 at 1 / 4 / 8 / 16 rows 25.6 -> 22.1, 32.2 -> 22.1, 32.4 -> 25.7, 34.4 -> 28.8; 17408 x 5120 19.0 -> 14.3, 17.8 -> 14.9,
 // 18.0 -> 18.4, 19.3 -> 20.7; 5120 x 5120 9.6 -> 9.0, 10.3 -> 9.0, 12.2 -> 9.1, 12.5 -> 10.1.
-template <int XP, int CO>
+//
+// Q: the program quantizes the activations itself, in front of its first step. aq is then bf16 rows [m][ldx]: a wavefront moves its quarter of K into LDS as
+// it is, in front of the first weights, makes fe_fp4_quant's values of it in their places (a block of 16 a lane) while the weights are on their way, and every
+// step reads them there; program 0 leaves codes, scales and operand in memory as that kernel does. The same bits, and a launch less: for few values
+// (fp4_quants_itself of fe_fp4.cpp), since every program quantizes all of them.
+struct Fp4QuantTo {
+    uint8_t *codes, *sf;
+    _Float16* aq;
+    uint32_t ldx;
+    float g;
+};
+template <int XP, int CO, bool Q>
 struct Fp4Wide {
-    static constexpr int CG = (CO + 1) / 2, L = CO + CG + XP;
-    static constexpr int SC_AT = CO * 1024, X_AT = SC_AT + CG * 256, STAGE = X_AT + XP * 1024;
-    static constexpr int FIT = 20 * 1024 / STAGE, DEPTH = FIT < 2 ? 2 : FIT < 6 ? FIT : 6;  // two programs a CU where two steps allow it
+    static constexpr int CG = (CO + 1) / 2, XL = Q ? 0 : XP, L = CO + CG + XL;
+    static constexpr int SC_AT = CO * 1024, X_AT = SC_AT + CG * 256, STAGE = X_AT + XL * 1024;
+    static constexpr int FIT = (Q ? 15 : 20) * 1024 / STAGE, DEPTH = FIT < 2 ? 2 : FIT < 6 ? FIT : 6;  // two programs a CU where two steps allow it
     static constexpr int RED = 4 * 16 * (16 * CG + 4) * 4, LDS = 4 * DEPTH * STAGE > RED ? 4 * DEPTH * STAGE : RED;
-    static_assert(DEPTH >= 2 && (DEPTH - 1) * L < 64 && LDS <= 160 * 1024, "stages");
+    static_assert(DEPTH >= 2 && (DEPTH - 1) * L < (Q ? 48 : 64) && LDS <= 160 * 1024, "stages");
 };
 
-template <int XP, int CO>
+template <int XP, int CO, bool Q>
 __device__ __forceinline__ void gemv_nvfp4_wide_body(uint16_t* c, const _Float16* aq, const uint8_t* w, const uint8_t* sw,
                                                      const float* alpha, const uint16_t* res, uint32_t m, uint32_t n, uint32_t k,
                                                      uint32_t ldc, uint32_t w_snt, uint32_t w_skt, uint32_t w_sr, uint32_t s_snt,
-                                                     uint32_t s_skt, uint32_t s_sr) {
-    typedef Fp4Wide<XP, CO> C;
+                                                     uint32_t s_skt, uint32_t s_sr, const Fp4QuantTo qt) {
+    typedef Fp4Wide<XP, CO, Q> C;
     constexpr int CG = C::CG, AHEAD = C::DEPTH - 1, PITCH = 16 * CG + 4;
     extern __shared__ __attribute__((aligned(1024))) unsigned char lds[];
     const uint32_t tid = threadIdx.x, lane = tid & 63, wave = __builtin_amdgcn_readfirstlane(tid >> 6), r = lane & 15, g = lane >> 4;
     const uint32_t col0 = blockIdx.x * 8 * CO, nt0 = col0 / 128, nts = n / 128, span = nts - nt0 < 2 ? nts - nt0 : 2;
     const u32x4 wrs = g8_rsrc(w + (size_t)nt0 * w_snt, span * 128 * (k / 2)), srs = g8_rsrc(sw + (size_t)nt0 * s_snt, span * 128 * (k / 16));
-    const u32x4 xrs = g8_rsrc(aq, m * k * 2);
+    const u32x4 xrs = g8_rsrc(aq, Q ? ((m - 1) * qt.ldx + k) * 2 : m * k * 2);
     // weight row `row` of the program (past n: the last one again, not stored), byte offset from weight tile nt0
     auto at = [&](uint32_t row, uint32_t snt, uint32_t sr) {
         const uint32_t i = (col0 + row < n ? col0 + row : n - 1) - 128 * nt0;
         return (i >> 7) * snt + (i & 127) * sr;
     };
-    uint32_t vw[CO], vs[CG], vx[XP];
+    uint32_t vw[CO], vs[CG], vx[C::XL + 1];
 #pragma unroll
     for (int j = 0; j < CO; j++) vw[j] = at(8 * j + ((lane >> 1) & 7), w_snt, w_sr) + g * w_skt + (lane & 1) * 16;
 #pragma unroll
     for (int j = 0; j < CG; j++) vs[j] = at(16 * j + r, s_snt, s_sr) + g * s_skt;
 #pragma unroll
-    for (int j = 0; j < XP; j++) {
+    for (int j = 0; j < C::XL; j++) {
         const uint32_t row = 2 * j + (lane >> 5), chunk = (lane & 16) | ((lane ^ row) & 15);
         vx[j] = (row < m ? row : m - 1) * k * 2 + chunk * 16;
     }
@@ -880,9 +918,11 @@ __device__ __forceinline__ void gemv_nvfp4_wide_body(uint16_t* c, const _Float16
 #pragma unroll
         for (int j = 0; j < CG; j++) g8_load_lds4(srs, to + C::SC_AT + j * 256, vs[j], (s0 + s) * 4 * s_skt);
 #pragma unroll
-        for (int j = 0; j < XP; j++) g8_load_lds16(xrs, to + C::X_AT + j * 1024, vx[j], (s0 + s) * 512);
+        for (int j = 0; j < C::XL; j++) g8_load_lds16(xrs, to + C::X_AT + j * 1024, vx[j], (s0 + s) * 512);
     };
     const uint32_t odd = g & 1, xr = r < m ? r : m - 1;
+    // Q: the wavefront's activations, [its steps][m rows][512 bytes] (a whole number of loads), chunks placed as in a stage
+    unsigned char* xq = lds + 4 * C::DEPTH * C::STAGE + wave * (((steps + 3) / 4 * m + 1) / 2 * 1024);
     // half h of the lane's row and k tile; the 16-byte chunk of 8 activations that goes with code 32 (h ^ odd) + 8 e on
     uint32_t fw[CG], fx[8];
 #pragma unroll
@@ -895,12 +935,12 @@ __device__ __forceinline__ void gemv_nvfp4_wide_body(uint16_t* c, const _Float16
 #pragma unroll
         for (int e = 0; e < 4; e++) {
             const uint32_t chunk = 8 * g + 4 * (h ^ odd) + e;
-            fx[4 * h + e] = C::X_AT + xr * 512 + (((chunk & 16) | ((chunk ^ xr) & 15)) << 4);
+            fx[4 * h + e] = (Q ? 0 : C::X_AT) + xr * 512 + (((chunk & 16) | ((chunk ^ xr) & 15)) << 4);
         }
     f32x4 acc[CG] = {};
     uint32_t slot = 0;
-    auto add = [&]() {
-        const unsigned char* st = stages + slot * C::STAGE;
+    auto add = [&](uint32_t s) {
+        const unsigned char *st = stages + slot * C::STAGE, *xst = Q ? xq + s * (m * 512) : st;
         uint32_t sc[CG];
 #pragma unroll
         for (int j = 0; j < CG; j++) {
@@ -911,7 +951,7 @@ __device__ __forceinline__ void gemv_nvfp4_wide_body(uint16_t* c, const _Float16
         for (int h = 0; h < 2; h++) {
             f16x8 x[4];
 #pragma unroll
-            for (int e = 0; e < 4; e++) x[e] = *(const f16x8*)(st + fx[4 * h + e]);
+            for (int e = 0; e < 4; e++) x[e] = *(const f16x8*)(xst + fx[4 * h + e]);
 #pragma unroll
             for (int j = 0; j < CG; j++) {
                 const u32x4 codes = *(const u32x4*)(st + fw[j] + 16 * (h ^ odd));
@@ -924,20 +964,38 @@ __device__ __forceinline__ void gemv_nvfp4_wide_body(uint16_t* c, const _Float16
         slot = slot + 1 == C::DEPTH ? 0 : slot + 1;
     };
     if (count) {
+        if constexpr (Q) {
+            const uint32_t xq0 = g8_lds_addr(xq), units = count * m;  // a unit: 256 values of a row, half a load
+            for (uint32_t u0 = 0; u0 < units; u0 += 2) {
+                const uint32_t u = u0 + (lane >> 5) < units ? u0 + (lane >> 5) : u0, s = u / m, row = u - s * m;
+                g8_load_lds16(xrs, xq0 + u0 * 512, (row * qt.ldx + (s0 + s) * 256) * 2 + ((lane & 16) | ((lane ^ row) & 15)) * 16, 0);
+            }
+        }
 #pragma unroll
         for (int u = 0; u < AHEAD; u++) issue((uint32_t)u < count ? u : count - 1, u);  // past the end: the last step again, not added
+        if constexpr (Q) {
+            g8_loads_wait<AHEAD * C::L>();
+            for (uint32_t i = lane; i < count * m * 16; i += 64) {
+                const uint32_t u = i >> 4, b = i & 15, s = u / m, row = u - s * m, c = 2 * b;
+                u32x4 *p0 = (u32x4*)(xq + u * 512 + (((c & 16) | ((c ^ row) & 15)) << 4)), *p1 = (u32x4*)(xq + u * 512 + ((((c + 1) & 16) | (((c + 1) ^ row) & 15)) << 4));
+                const Fp4Block v = fp4_quant_block(*p0, *p1, qt.g);
+                *p0 = v.o[0], *p1 = v.o[1];
+                if (blockIdx.x == 0) fp4_store_block(v, qt.codes, qt.sf, qt.aq, row, (s0 + s) * 16 + b, k);
+            }
+            asm volatile("" ::: "memory");
+        }
         uint32_t s = 0;
         for (; s + AHEAD < count; s++) {
             g8_loads_wait<(AHEAD - 1) * C::L>();  // (the stage in front of this one has been read, too)
             issue(s + AHEAD, slot ? slot - 1 : AHEAD);
-            add();
+            add(s);
         }
         auto tail = [&](auto u_tag) {
             constexpr int U = decltype(u_tag)::value;
             if constexpr (U < AHEAD)
                 if (s + U < count) {
                     g8_loads_wait<(AHEAD - 1 - U) * C::L>();
-                    add();
+                    add(s + U);
                 }
         };
         tail(std::integral_constant<int, 0>{});
@@ -967,15 +1025,24 @@ __device__ __forceinline__ void gemv_nvfp4_wide_body(uint16_t* c, const _Float16
         uint16_t* c, const _Float16* aq, const uint8_t* w, const uint8_t* sw, const float* alpha, const uint16_t* res,   \
         uint32_t m, uint32_t n, uint32_t k, uint32_t ldc, uint32_t w_snt, uint32_t w_skt, uint32_t w_sr, uint32_t s_snt, \
         uint32_t s_skt, uint32_t s_sr) {                                                                                  \
-        gemv_nvfp4_wide_body<XP, CO>(c, aq, w, sw, alpha, res, m, n, k, ldc, w_snt, w_skt, w_sr, s_snt, s_skt, s_sr);     \
+        gemv_nvfp4_wide_body<XP, CO, false>(c, aq, w, sw, alpha, res, m, n, k, ldc, w_snt, w_skt, w_sr, s_snt, s_skt, s_sr, Fp4QuantTo{}); \
     }
-#define FP4_WIDE_FAMILY(XP)                                                                                             \
-    FP4_WIDE_KERNEL(XP, 1) FP4_WIDE_KERNEL(XP, 2) FP4_WIDE_KERNEL(XP, 3) FP4_WIDE_KERNEL(XP, 4) FP4_WIDE_KERNEL(XP, 5)  \
-    FP4_WIDE_KERNEL(XP, 6) FP4_WIDE_KERNEL(XP, 9)
-FP4_WIDE_FAMILY(1)
-FP4_WIDE_FAMILY(2)
-FP4_WIDE_FAMILY(4)
-FP4_WIDE_FAMILY(8)
+#define FP4_WIDE_QUANT_KERNEL(XP, CO)                                                                                     \
+    extern "C" __global__ __launch_bounds__(256) void fe_gemv_nvfp4_q##XP##_c##CO(                                        \
+        uint16_t* c, const _Float16* x, const uint8_t* w, const uint8_t* sw, const float* alpha, const uint16_t* res,    \
+        uint32_t m, uint32_t n, uint32_t k, uint32_t ldc, uint32_t w_snt, uint32_t w_skt, uint32_t w_sr, uint32_t s_snt, \
+        uint32_t s_skt, uint32_t s_sr, Fp4QuantTo qt) {                                                                   \
+        gemv_nvfp4_wide_body<XP, CO, true>(c, x, w, sw, alpha, res, m, n, k, ldc, w_snt, w_skt, w_sr, s_snt, s_skt, s_sr, qt); \
+    }
+#define FP4_WIDE_FAMILY(KERNEL, XP) \
+    KERNEL(XP, 1) KERNEL(XP, 2) KERNEL(XP, 3) KERNEL(XP, 4) KERNEL(XP, 5) KERNEL(XP, 6) KERNEL(XP, 9)
+FP4_WIDE_FAMILY(FP4_WIDE_KERNEL, 1)
+FP4_WIDE_FAMILY(FP4_WIDE_KERNEL, 2)
+FP4_WIDE_FAMILY(FP4_WIDE_KERNEL, 4)
+FP4_WIDE_FAMILY(FP4_WIDE_KERNEL, 8)
+FP4_WIDE_FAMILY(FP4_WIDE_QUANT_KERNEL, 1)
+FP4_WIDE_FAMILY(FP4_WIDE_QUANT_KERNEL, 2)
+FP4_WIDE_FAMILY(FP4_WIDE_QUANT_KERNEL, 4)
 
 // ---- matrix-unit peak probe ---------------------------------------------------------------------------------------------
 //
