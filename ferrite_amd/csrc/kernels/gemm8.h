@@ -80,6 +80,12 @@ __device__ __forceinline__ u32x4 g8_rsrc(const void* p, uint32_t bytes) {
 __device__ __forceinline__ uint32_t g8_lds_addr(const void* p) {
     return (uint32_t)(uintptr_t)(const __attribute__((address_space(3))) void*)p;
 }
+// Byte offset of row `row` of an operand of m rows of `pitch` bytes. Rows past m lie out of the resource's range and read zero: what they would multiply is never
+// stored, and zeros take less of the board's power, which is what bounds the loop. (Operands of 2 GB and more, whose range such an offset could meet: row m - 1 again.)
+__device__ __forceinline__ uint32_t g8_row(uint32_t row, uint32_t m, uint32_t pitch) {
+    const uint32_t past = m * pitch <= 0x7fff0000u ? 0x80000000u : (m - 1) * pitch;
+    return row < m ? row * pitch : past;
+}
 // chunk position <-> chunk (its own inverse): identity, or the two low bits swapped
 template <bool PERM>
 __device__ __forceinline__ constexpr uint32_t g8_perm(uint32_t c) {
@@ -149,8 +155,8 @@ __device__ __forceinline__ void g8_mainloop(const void* a, uint32_t lda, uint32_
     uint32_t va[LA];
 #pragma unroll
     for (int j = 0; j < LA; j++) {
-        const uint32_t r = 8 * (wave + 8 * j) + (lane >> 3), g = m0 + r < m ? m0 + r : m - 1;
-        va[j] = (g * lda + (g8_perm<W::kPerm>((lane & 7) ^ (r & 7))) * 8) * 2;
+        const uint32_t r = 8 * (wave + 8 * j) + (lane >> 3);
+        va[j] = g8_row(m0 + r, m, lda * 2) + (g8_perm<W::kPerm>((lane & 7) ^ (r & 7))) * 16;
     }
     const uint32_t base = g8_lds_addr(lds) + wave * 1024;
     auto ktc = [&](uint32_t kt) { return kt0 + (kt < ktiles ? kt : ktiles - 1); };  // past the end: the last tile again, never used
@@ -268,13 +274,16 @@ __device__ __forceinline__ void g8_epilogue(f32x4 (&acc)[T::TM][T::TN], unsigned
     }
 }
 
-// A program's accumulators in its partial slot, as the lanes hold them: piece (i, j) of thread t at ((i TN + j) 512 + t) 16.
+// A program's accumulators in its partial slot, as the lanes hold them: piece (i, j) of thread t at ((i TN + j) 512 + t) 16. rows: those of the tile that
+// exist; groups of 16 past them are left out.
 template <class T>
-__device__ __forceinline__ void g8_store_partial(f32x4 (&acc)[T::TM][T::TN], float* slot) {
+__device__ __forceinline__ void g8_store_partial(f32x4 (&acc)[T::TM][T::TN], float* slot, uint32_t rows) {
+    const uint32_t row0 = (threadIdx.x >> 6) / T::WN * (16 * T::TM);
 #pragma unroll
     for (int i = 0; i < T::TM; i++)
+        if (row0 + 16 * i < rows)
 #pragma unroll
-        for (int j = 0; j < T::TN; j++) *(f32x4*)(slot + ((i * T::TN + j) * T::THREADS + threadIdx.x) * 4) = acc[i][j];
+            for (int j = 0; j < T::TN; j++) *(f32x4*)(slot + ((i * T::TN + j) * T::THREADS + threadIdx.x) * 4) = acc[i][j];
 }
 
 // Body of a reduce kernel: grid = cut tiles * (BM / 8) * (BN / 128), 256 threads. Each half wavefront sums the `splits` slots
@@ -299,7 +308,18 @@ __device__ __forceinline__ void g8_reduce_rows(const float* __restrict__ part, u
     const uint32_t wm = row / (16 * T::TM), i = (row / 16) % T::TM, fr = row % 16;
     const float* p = part + (size_t)t * splits * T::PART_FLOATS + ((i * T::TN + j) * T::THREADS + (wm * T::WN + wn) * 64 + fc * 16 + fr) * 4;
     f32x4 sum = *(const f32x4*)p;
-    for (uint32_t sp = 1; sp < splits; sp++) sum += *(const f32x4*)(p + (size_t)sp * T::PART_FLOATS);
+    auto add = [&](auto n_tag, uint32_t sp) {  // so many pieces in flight a lane
+        constexpr uint32_t N = decltype(n_tag)::value;
+        f32x4 piece[N];
+#pragma unroll
+        for (uint32_t q = 0; q < N; q++) piece[q] = *(const f32x4*)(p + (size_t)(sp + q) * T::PART_FLOATS);
+#pragma unroll
+        for (uint32_t q = 0; q < N; q++) sum += piece[q];
+    };
+    uint32_t sp = 1;
+    for (; sp + 4 <= splits; sp += 4) add(std::integral_constant<uint32_t, 4>{}, sp);
+    if (sp + 2 <= splits) add(std::integral_constant<uint32_t, 2>{}, sp), sp += 2;
+    if (sp < splits) add(std::integral_constant<uint32_t, 1>{}, sp);
     float v[4] = {sum[0], sum[1], sum[2], sum[3]};
     fn(m0 + row, n0, l32, v);
 }
@@ -325,8 +345,8 @@ __device__ __forceinline__ void g8_mainloop_packed(const _Float16* a, uint32_t l
     uint32_t va[LA];
 #pragma unroll
     for (int j = 0; j < LA; j++) {
-        const uint32_t r = 8 * (wave + 8 * j) + (lane >> 3), g = m0 + r < m ? m0 + r : m - 1;
-        va[j] = (g * lda + (g8_perm<true>((lane & 7) ^ (r & 7))) * 8) * 2;
+        const uint32_t r = 8 * (wave + 8 * j) + (lane >> 3);
+        va[j] = g8_row(m0 + r, m, lda * 2) + (g8_perm<true>((lane & 7) ^ (r & 7))) * 16;
     }
     const uint32_t base = g8_lds_addr(lds);
     auto ktc = [&](uint32_t kt) { return kt0 + (kt < ktiles ? kt : ktiles - 1); };
@@ -438,8 +458,8 @@ __device__ __forceinline__ void g8_mainloop_decode(const _Float16* a, uint32_t l
     uint32_t va[LA];
 #pragma unroll
     for (int j = 0; j < LA; j++) {
-        const uint32_t r = 8 * (wave + 8 * j) + (lane >> 3), g = m0 + r < m ? m0 + r : m - 1;
-        va[j] = (g * lda + ((lane & 7) ^ (r & 7)) * 8) * 2;
+        const uint32_t r = 8 * (wave + 8 * j) + (lane >> 3);
+        va[j] = g8_row(m0 + r, m, lda * 2) + ((lane & 7) ^ (r & 7)) * 16;
     }
     const uint32_t base = g8_lds_addr(lds);
     auto ktc = [&](uint32_t kt) { return kt0 + (kt < ktiles ? kt : ktiles - 1); };
@@ -570,8 +590,8 @@ __device__ __forceinline__ void g8_mainloop_f8(const uint8_t* a, uint32_t lda, u
     uint32_t va[LA];
 #pragma unroll
     for (int j = 0; j < LA; j++) {
-        const uint32_t r = 8 * (wave + 8 * j) + (lane >> 3), g = m0 + r < m ? m0 + r : m - 1;
-        va[j] = g * lda + ((lane & 7) ^ (r & 7)) * 16;
+        const uint32_t r = 8 * (wave + 8 * j) + (lane >> 3);
+        va[j] = g8_row(m0 + r, m, lda) + ((lane & 7) ^ (r & 7)) * 16;
     }
     const uint32_t base = g8_lds_addr(lds) + wave * 1024;
     auto ktc = [&](uint32_t kt) { return kt0 + (kt < ktiles ? kt : ktiles - 1); };
@@ -742,14 +762,14 @@ __device__ __forceinline__ void g8_schedule(const GemmSched& sc, uint32_t m, uin
         const uint32_t kt0 = wk.piece * ktiles / sc.splits;
         main(wk.tm * T::BM, wk.tn * T::BN, kt0, (wk.piece + 1) * ktiles / sc.splits - kt0, acc);
         if (sc.splits > 1)
-            g8_store_partial<T>(acc, sc.part + (size_t)(wk.tile * sc.splits + wk.piece) * T::PART_FLOATS);
+            g8_store_partial<T>(acc, sc.part + (size_t)(wk.tile * sc.splits + wk.piece) * T::PART_FLOATS, m - wk.tm * T::BM);
         else
             finish(wk.tm * T::BM, wk.tn * T::BN, acc);
     } else if constexpr (!SK) {
         const GemmWork wk = gemm_work(p, tiles_m, tiles_n, group, ktiles, sc.full_tiles, sc.splits);
         main(wk.tm * T::BM, wk.tn * T::BN, wk.kt0, wk.ktn, acc);
         if (wk.partial)
-            g8_store_partial<T>(acc, sc.part + (size_t)wk.slot * T::PART_FLOATS);
+            g8_store_partial<T>(acc, sc.part + (size_t)wk.slot * T::PART_FLOATS, m - wk.tm * T::BM);
         else
             finish(wk.tm * T::BM, wk.tn * T::BN, acc);
     } else {
