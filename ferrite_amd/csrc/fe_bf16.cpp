@@ -12,7 +12,7 @@
 
 namespace {
 // dynamic LDS by form (256 x 256, unused, 128 x 256, 128 x 128): the k tiles in flight, two or three of A and three of W
-constexpr uint32_t kGemmLds[4] = {160 * 1024, 0, 144 * 1024, 80 * 1024};
+constexpr uint32_t kGemmLds[kFeGemmForms] = {160 * 1024, 0, 144 * 1024, 80 * 1024, 160 * 1024, 144 * 1024, 144 * 1024};
 constexpr uint32_t kGemmThreads = 512;
 constexpr uint32_t kTileM = 256;                         // rows of the largest output tile
 constexpr uint32_t kGemvRows = 8;                        // rows of one fe_bf16_gemv call (model.rs:326)
@@ -29,7 +29,7 @@ constexpr uint32_t kSmallBatch = 16;                     // X3_ROWS: batches up 
 
 struct fe_bf16_kernels {
     fe_module_t module = nullptr;
-    fe_function_t gemm[4] = {}, reduce[3] = {}, swiglu[4] = {}, swiglu_reduce[3] = {};  // by form; by tile (fe_gemm_launch)
+    fe_function_t gemm[kFeGemmForms] = {}, reduce[kFeGemmTiles] = {}, swiglu[kFeGemmForms] = {}, swiglu_reduce[kFeGemmTiles] = {};  // by form; by tile (fe_gemm_launch)
     fe_function_t interleave = nullptr;
     fe_function_t gemv[5][7] = {};  // [kGemvRowForms][kGemvColForms]
     uint32_t cus = 0;
@@ -38,7 +38,7 @@ struct fe_bf16_kernels {
     int32_t nc = -1;           // columns a GEMV program takes, rounded up to 8, 16, .. 48, 72; -1 = by the shape (FE_BF16_NC)
     int32_t raster_group = -1; // raster group of the GEMM; -1 = by the shape (FE_BF16_GROUP)
     uint32_t gemm_splits = 8;  // most pieces a cut output tile takes (FE_GEMM_SPLITS; 1: never cut)
-    FeGemmTileOptions tile;    // "gemm_tile", "gemm_pieces"
+    FeGemmTileOptions tile{0, 0, true};  // "gemm_tile", "gemm_pieces"
 };
 
 // Which of kGemvColForms a GEMV takes. Time goes by the CU with the most columns, so the form is the one with the least of
@@ -96,9 +96,9 @@ int fe_bf16_kernels_load(fe_bf16_kernels **out) {
     if (!out) return fe_set_error(FE_ERR_ARG, "fe_bf16_kernels_load", "null out");
     auto *k = new fe_bf16_kernels;
     int c = fe_load_module(&k->module, "FE_BF16_HSACO", fe_k_bf16_hsaco, fe_k_bf16_hsaco_end);
-    for (int tile = 0; tile < 3 && !c; tile++) {
-        static const char *suffix[] = {"", "_s1", "_s2"};
-        const int form = tile ? tile + 1 : 0;
+    for (uint32_t tile = 0; tile < kFeGemmTiles && !c; tile++) {
+        static const char *suffix[] = {"", "_s1", "_s2", "_h7", "_h6", "_h5"};
+        const uint32_t form = tile ? tile + 1 : 0;
         const std::string s = suffix[tile];
         c = fe_hip_module_get_function(&k->gemm[form], k->module, ("fe_gemm_bf16" + s).c_str());
         if (!c) c = fe_hip_func_set_max_dyn_lds(k->gemm[form], kGemmLds[form]);

@@ -16,7 +16,8 @@ namespace {
 constexpr uint32_t kTile = 128;                 // crates/fe-fp4/src/lib.rs:28
 // dynamic LDS by form (256 x 256, its stream-K form, 128 x 256, 128 x 128): the k tiles in flight. Packed weights: three of A (128
 // bytes a row) and three of W (36 bytes; 64 in the fp16 form of FP8). FP8 codes: two or three of A, three of W, 128 bytes a row.
-constexpr uint32_t kGemmLds[4] = {144 * 1024, 144 * 1024, 136 * 1024, 68 * 1024}, kGemmLds8[4] = {160 * 1024, 160 * 1024, 144 * 1024, 80 * 1024};
+constexpr uint32_t kGemmLds[kFeGemmForms] = {144 * 1024, 144 * 1024, 136 * 1024, 68 * 1024, 144 * 1024, 120 * 1024, 120 * 1024};
+constexpr uint32_t kGemmLds8[kFeGemmForms] = {160 * 1024, 160 * 1024, 144 * 1024, 80 * 1024, 160 * 1024, 144 * 1024, 144 * 1024};
 // Forms of the GEMV over programs of 8 CO columns: rows / 2 and CO
 constexpr uint32_t kWideRowForms[4] = {1, 2, 4, 8}, kWideColForms[7] = {1, 2, 3, 4, 5, 6, 9};
 // Fp4Wide<XP, CO, Q>::LDS of k_fp4.hip; Q (rows m of k quantized by the program itself): with its four wavefronts' activations in the place of a stage's
@@ -33,7 +34,8 @@ struct fe_fp4_kernels {
     fe_module_t module = nullptr;
     fe_function_t quant4 = nullptr, gemv4[3] = {nullptr, nullptr, nullptr};
     // by form (256 x 256, stream-K, 128 x 256, 128 x 128) and by tile (fe_gemm_launch); gemm8: the fp16 form, 256 x 256 only
-    fe_function_t gemm4[4] = {}, swiglu4[4] = {}, gemm8c[4] = {}, gemm8[2] = {}, reduce4[3] = {}, swiglu_reduce4[3] = {}, reduce8c[3] = {};
+    fe_function_t gemm4[kFeGemmForms] = {}, swiglu4[kFeGemmForms] = {}, gemm8c[kFeGemmForms] = {}, gemm8[2] = {};
+    fe_function_t reduce4[kFeGemmTiles] = {}, swiglu_reduce4[kFeGemmTiles] = {}, reduce8c[kFeGemmTiles] = {};
     fe_function_t wide[4][7] = {};   // the GEMV over programs of 8 CO columns, [kWideRowForms][kWideColForms]
     fe_function_t wide_q[3][7] = {};  // the same, quantizing its activations itself
     fe_function_t quant8 = nullptr, expand8 = nullptr;
@@ -50,7 +52,7 @@ struct fe_fp4_kernels {
     uint32_t fp8_f16 = 0;      // FP8 linears as fp16 expansion on the 16-bit matrix instruction (FE_FP8_F16=1)
     uint32_t gemm_splits = 8;  // most pieces a cut output tile takes (FE_GEMM_SPLITS; 1: never cut)
     int32_t gemm_sk = 1;       // stream-K schedule of the GEMMs: 0 never, 1 where measured faster, 2 always (FE_GEMM_SK)
-    FeGemmTileOptions tile;    // "gemm_tile", "gemm_pieces"
+    FeGemmTileOptions tile{0, 0, true};  // "gemm_tile", "gemm_pieces"
 };
 
 struct fe_fp4_linear {
@@ -82,17 +84,17 @@ int fe_fp4_kernels_load(fe_fp4_kernels **out) {
         if (!c) c = fe_hip_module_get_function(f, k->module, nm.c_str());
         if (!c && lds) c = fe_hip_func_set_max_dyn_lds(*f, lds);
     };
-    static const char *form_sfx[] = {"", "_sk", "_s1", "_s2"}, *tile_sfx[] = {"", "_s1", "_s2"};
-    for (int i = 0; i < 4; i++) {
+    static const char *form_sfx[] = {"", "_sk", "_s1", "_s2", "_h7", "_h6", "_h5"}, *tile_sfx[] = {"", "_s1", "_s2", "_h7", "_h6", "_h5"};
+    for (uint32_t i = 0; i < kFeGemmForms; i++) {
         get(&k->gemm4[i], std::string("fe_gemm_nvfp4") + form_sfx[i], kGemmLds[i]);
         get(&k->swiglu4[i], std::string("fe_gemm_nvfp4_swiglu") + form_sfx[i], kGemmLds[i]);
         get(&k->gemm8c[i], std::string("fe_gemm_fp8_codes") + form_sfx[i], kGemmLds8[i]);
         if (i < 2) get(&k->gemm8[i], std::string("fe_gemm_fp8") + form_sfx[i], kGemmLds[i]);
     }
-    for (int i = 0; i < 3; i++) {
+    for (uint32_t i = 0; i < kFeGemmTiles; i++) {
         get(&k->reduce4[i], std::string("fe_gemm_nvfp4_reduce") + tile_sfx[i], 0);
         get(&k->swiglu_reduce4[i], std::string("fe_gemm_nvfp4_swiglu_reduce") + tile_sfx[i], 0);
-        get(&k->reduce8c[i], std::string("fe_gemm_fp8_codes_reduce") + tile_sfx[i], 0);
+        get(&k->reduce8c[i], std::string(i < 3 ? "fe_gemm_fp8_codes_reduce" : "fe_gemm_nvfp4_reduce") + tile_sfx[i], 0);  // (one layout of the lower tiles)
     }
     for (int xr = 1; xr <= 3 && !c; xr++) {
         char nm[32];
@@ -436,7 +438,7 @@ static int linear_gemm(const fe_fp4_linear *l, const fe_fp4_kernels *kern, fe_st
     // FP8 runs on the 8-bit matrix instruction over the codes of both operands, k tiles of 128 (FE_FP8_F16=1: the fp16
     // expansion on the 16-bit instruction, k tiles of 64; same products, another order of the f32 sums)
     const bool codes8 = l->fp8 && !kern->fp8_f16;
-    const FeGemmTileOptions f16_form{1, 0};  // (the fp16 form exists for 256 x 256 tiles only)
+    const FeGemmTileOptions f16_form{1, 0, false};  // (the fp16 form exists for 256 x 256 tiles only)
     const FeGemmPlan plan = fe_gemm_plan(m, n, codes8 ? k / 128 : k / 64, kern->cus, ws->part.p, ws->part.bytes, ws->counters.p, kGemvCounters,
                                          kern->gemm_splits, kern->gemm_sk, /*small_b=*/!l->fp8,
                                          l->fp8 ? kFeCostFp8 : kFeCostNvfp4, l->fp8 && !codes8 ? f16_form : kern->tile);

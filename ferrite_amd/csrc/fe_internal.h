@@ -262,11 +262,12 @@ inline FeGemmSchedule fe_gemm_schedule(uint32_t tiles, uint32_t ktiles, uint32_t
 
 // ---- which tiles a GEMM launch takes -------------------------------------------------------------------------------------------
 // Tile 0: 256 x 256, on one of the two schedules above. Tiles 1 (128 x 256) and 2 (128 x 128): a launch of small tiles, each cut
-// `splits` ways along K.
-constexpr uint32_t kFeGemmTileM[3] = {256, 128, 128}, kFeGemmTileN[3] = {256, 256, 128};
+// `splits` ways along K. Tiles 3, 4, 5 (224, 192, 160 x 256): as tile 0, one piece a program.
+constexpr uint32_t kFeGemmTiles = 6, kFeGemmTileM[kFeGemmTiles] = {256, 128, 128, 224, 192, 160}, kFeGemmTileN[kFeGemmTiles] = {256, 256, 128, 256, 256, 256};
+constexpr uint32_t kFeGemmForms = kFeGemmTiles + 1;  // kernels: tile 0 one piece a program and stream-K, then the other tiles
 
 struct FeGemmPlan {
-    FeGemmSchedule big;  // tile 0
+    FeGemmSchedule big;  // tiles 0 and 3..5
     uint32_t tile = 0, tiles = 0, splits = 1;
     float us = 0;  // the estimate (0: a tile was forced)
 };
@@ -274,6 +275,7 @@ struct FeGemmPlan {
 // with force_pieces pieces of K (0: one).
 struct FeGemmTileOptions {
     uint32_t force_tile = 0, force_pieces = 0;
+    bool low = false;  // the handle has kernels of tiles 3..5 (force_tile 4, 5, 6)
 };
 
 // What a program of each tile takes on one weight form: us a k tile (64; FP8: 128), `full` more of it when all CUs are busy (clock and
@@ -282,13 +284,15 @@ struct FeGemmTileOptions {
 // 10..13 % for bf16 and FP8, whose panels compete for memory). stream_k: what meeting through the workspace adds. again: what small
 // tiles in more than one round take more than their rounds add up to (trellis: the programs that come second decode alone; 528 tiles 128 x 128 of
 // 32 k tiles 80 us where the rounds add up to 67).
+// high: us a k tile of tiles of 256, 224, 192, 160 rows, and how much more of it when all CUs are busy, for the choice among them (fe_gemm_height): fitted to 112
+// timings a form and height (128..1900 rows, 2048 x 4096 .. 17408 x 5120) without a fixed part, half of them within 5 % (FP8 8 %).
 struct FeGemmCost {
-    float ktile[3], full[3], fixed[3], shared, stream_k, again;
+    float ktile[3], full[3], fixed[3], shared, stream_k, again, high[4][2];
 };
-constexpr FeGemmCost kFeCostTrellis = {{1.38f, 1.02f, 0.71f}, {0.12f, 0.07f, 0.08f}, {1.0f, 3.0f, 1.9f}, 1.63f, 48.7f, 1.12f};
-constexpr FeGemmCost kFeCostNvfp4 = {{1.32f, 0.73f, 0.44f}, {-0.07f, 0.05f, 0.09f}, {0.0f, 2.2f, 2.3f}, 1.59f, 44.0f, 1.0f};
-constexpr FeGemmCost kFeCostFp8 = {{1.20f, 0.58f, 0.66f}, {0.09f, 0.46f, 0.21f}, {0.0f, 2.5f, 0.4f}, 1.21f, 36.4f, 1.0f};
-constexpr FeGemmCost kFeCostBf16 = {{1.10f, 0.64f, 0.45f}, {0.22f, 0.43f, 0.41f}, {0.0f, 1.5f, 0.3f}, 1.53f, 53.2f, 1.0f};
+constexpr FeGemmCost kFeCostTrellis = {{1.38f, 1.02f, 0.71f}, {0.12f, 0.07f, 0.08f}, {1.0f, 3.0f, 1.9f}, 1.63f, 48.7f, 1.12f, {}};
+constexpr FeGemmCost kFeCostNvfp4 = {{1.32f, 0.73f, 0.44f}, {-0.07f, 0.05f, 0.09f}, {0.0f, 2.2f, 2.3f}, 1.59f, 44.0f, 1.0f, {{1.11f, 0.29f}, {1.16f, 0.16f}, {0.90f, 0.36f}, {0.57f, 1.03f}}};
+constexpr FeGemmCost kFeCostFp8 = {{1.20f, 0.58f, 0.66f}, {0.09f, 0.46f, 0.21f}, {0.0f, 2.5f, 0.4f}, 1.21f, 36.4f, 1.0f, {{1.81f, -0.29f}, {1.78f, -0.21f}, {1.68f, -0.20f}, {1.50f, -0.15f}}};
+constexpr FeGemmCost kFeCostBf16 = {{1.10f, 0.64f, 0.45f}, {0.22f, 0.43f, 0.41f}, {0.0f, 1.5f, 0.3f}, 1.53f, 53.2f, 1.0f, {{1.26f, 0.04f}, {1.24f, 0.01f}, {0.92f, 0.20f}, {0.77f, 0.34f}}};
 
 // `programs` programs of `ktiles` k tiles each, in rounds of all CUs (tile 2: two a CU).
 inline float fe_gemm_cost(const FeGemmCost &c, uint32_t tile, uint32_t programs, uint32_t ktiles, uint32_t cus) {
@@ -300,6 +304,18 @@ inline float fe_gemm_cost(const FeGemmCost &c, uint32_t tile, uint32_t programs,
 // The reduce launch: its start, and the partials written and read once.
 inline float fe_gemm_reduce_cost(uint32_t programs, uint32_t tile) {
     return 4.0f + (float)programs * (float)(kFeGemmTileM[tile] * kFeGemmTileN[tile]) * 8.0f / 5e6f;
+}
+
+// What a launch of tiles of one height (256, 224, 192, 160 rows: h 0..3) takes, for the choice among them: rounds of one program a CU, and the pieces' sums, which
+// travel twice.
+inline float fe_gemm_height(const FeGemmCost &c, uint32_t h, const FeGemmSplit &g, uint32_t ktiles, uint32_t cus, uint32_t rows_a_tile) {
+    auto rounds = [&](uint32_t programs, uint32_t k) {
+        const uint32_t last = programs % cus;
+        return (float)k * c.high[h][0] * ((float)(programs / cus) * (1.0f + c.high[h][1]) + (last ? 1.0f + c.high[h][1] * (float)last / (float)cus : 0.0f));
+    };
+    float t = rounds(g.full, ktiles);
+    if (g.cut()) t += rounds(g.cut() * g.splits, (ktiles + g.splits - 1) / g.splits) + 2.5f + (float)(g.cut() * g.splits * rows_a_tile) * 2048.0f / 5e6f;
+    return t;
 }
 
 // The rule: with fewer than a few rounds of 256 x 256 tiles, most of the time is CUs without a tile or pieces of K that meet;
@@ -324,11 +340,18 @@ inline FeGemmPlan fe_gemm_plan(uint32_t m, uint32_t n, uint32_t ktiles, uint32_t
         const size_t slots = part_bytes / (kFeGemmTileM[tile] * kFeGemmTileN[tile] * 4);
         return (uint32_t)std::max<size_t>(1, std::min<size_t>({want, ktiles, slots / tiles_of(tile)}));
     };
-    if (opt.force_tile >= 2) {
+    auto low = [&](uint32_t tile) {  // the one-piece schedule of tiles as high as kFeGemmTileM[tile]
+        return fe_gemm_schedule(tiles_of(tile), ktiles, cus, part, part_bytes, 0, 0, cap, 0, small_b);
+    };
+    if (opt.force_tile >= 4 && opt.low) {
+        p.tile = opt.force_tile - 1, p.big = low(p.tile);
+        return p;
+    }
+    if (opt.force_tile == 2 || opt.force_tile == 3) {
         take(opt.force_tile - 1, tiles_of(opt.force_tile - 1), most_pieces(opt.force_tile - 1, std::max(1u, opt.force_pieces)));
         return p;
     }
-    if (opt.force_tile == 1 || mode >= 2 || !cus) return p;
+    if (opt.force_tile || mode >= 2 || !cus) return p;
     float best;
     if (p.big.stream_k) {
         const FeGemmSchedArgs &a = p.big.args;
@@ -339,7 +362,26 @@ inline FeGemmPlan fe_gemm_plan(uint32_t m, uint32_t n, uint32_t ktiles, uint32_t
         if (g.cut())
             best += fe_gemm_cost(cost, 0, g.cut() * g.splits, (ktiles + g.splits - 1) / g.splits, cus) + fe_gemm_reduce_cost(g.cut() * g.splits, 0);
     }
+    // Lower tiles: as many row tiles of less waste, or another count of them that fills the rounds of the CUs better (rows that do not exist cost little power, but
+    // their time). By the ratio of the two estimates, which share most of their errors. Of 336 launches (8 layers, 14 row counts, NVFP4, FP8 and bf16) against 256 rows:
+    // 0.925, 0.93, 0.905 of the time (the best height each time: 0.92, 0.92, 0.90), four more than 2 % slower, at most 7 %. With the small tiles in the choice, 12 other layers
+    // of 144 launches a form against the rule without lower tiles: 0.93, 0.97, 0.93; 8 of 432 more than 3 % slower, at most 7 %.
+    if (opt.low && m <= 2048) {
+        const uint32_t tiles_n = (n + 255) / 256;
+        auto height = [&](uint32_t tile, uint32_t h, const FeGemmSplit &g) { return fe_gemm_height(cost, h, g, ktiles, cus, m / (tiles_of(tile) / tiles_n)); };
+        const float high = height(0, 0, p.big.split);
+        float ratio = p.big.stream_k ? 0.9f : 0.97f;
+        uint32_t pick = 0;
+        for (uint32_t tile = 3; tile < kFeGemmTiles; tile++) {
+            const FeGemmSplit g = low(tile).split;
+            float r = height(tile, tile - 2, g) / high;
+            if (2 * g.programs() < cus) r = std::max(r, 0.85f);  // (mostly idle CUs: a k tile takes the trip of its loads, at any height)
+            if (r < ratio) ratio = r, pick = tile;
+        }
+        if (pick) p.tile = pick, p.big = low(pick), best *= ratio;
+    }
     p.us = best;
+    const float margin = p.tile && !small_b ? 1.0f : 1.06f;  // (bf16 and FP8: what a lower tile gained is part of that margin)
     for (uint32_t tile = 1; tile <= 2 && m <= 2048; tile++) {
         const uint32_t tiles = tiles_of(tile), most = most_pieces(tile, std::min(cap, ktiles / 8));
         for (uint32_t pieces = 1; pieces <= most; pieces++) {
@@ -347,7 +389,7 @@ inline FeGemmPlan fe_gemm_plan(uint32_t m, uint32_t n, uint32_t ktiles, uint32_t
             float c = fe_gemm_cost(cost, tile, tiles * pieces, (ktiles + pieces - 1) / pieces, cus);
             if (pieces > 1) c += fe_gemm_reduce_cost(tiles * pieces, tile);
             if (tiles * pieces > cus * tile) c *= cost.again;
-            if (1.06f * c < best) take(tile, tiles, pieces), p.us = c, best = 1.06f * c;
+            if (margin * c < best) take(tile, tiles, pieces), p.us = c, best = margin * c;
         }
     }
     return p;
@@ -430,19 +472,19 @@ inline float fe_rgemm_other_us(const FeGemmPlan &p, uint32_t cus) {
 inline bool fe_rgemm_takes(const FeRgemmPlan &p, float other_us, uint32_t count) { return p.us <= other_us + 3.0f * (float)count; }
 
 // Launches a plan. gemm(form, programs, sched): form 0 = 256 x 256 one piece a program, 1 = stream-K, 2, 3 = tile 1, 2;
-// reduce(tile, grid, first, splits): the reduce kernel of a tile, for the tiles from `first` on.
+// 4, 5, 6 = tile 3, 4, 5; reduce(tile, grid, first, splits): the reduce kernel of a tile, for the tiles from `first` on.
 template <class Gemm, class Reduce>
 int fe_gemm_launch(const FeGemmPlan &p, Gemm gemm, Reduce reduce) {
     const uint32_t reduce_grid = kFeGemmTileM[p.tile] / 8 * (kFeGemmTileN[p.tile] / 128);  // workgroups a tile
-    if (p.tile) {
+    if (p.tile == 1 || p.tile == 2) {
         FeGemmSchedArgs a = p.big.args;
         a.full_tiles = 0, a.splits = p.splits, a.sk_base = a.sk_rem = 0;
         FE_TRY(gemm(p.tile + 1, p.tiles * p.splits, a));
         if (p.splits > 1) FE_TRY(reduce(p.tile, p.tiles * reduce_grid, 0u, p.splits));
         return 0;
     }
-    FE_TRY(gemm(p.big.stream_k ? 1u : 0u, p.big.programs, p.big.args));
+    FE_TRY(gemm(p.big.stream_k ? 1u : p.tile ? p.tile + 1 : 0u, p.big.programs, p.big.args));
     if (!p.big.stream_k && p.big.split.cut())
-        FE_TRY(reduce(0u, p.big.split.cut() * reduce_grid, p.big.split.full, p.big.split.splits));
+        FE_TRY(reduce(p.tile, p.big.split.cut() * reduce_grid, p.big.split.full, p.big.split.splits));
     return 0;
 }

@@ -32,7 +32,8 @@ struct G8Tile {
     static constexpr int WM = WM_, WN = WN_, TM = TM_, TN = TN_, NW = WM * WN, THREADS = 64 * NW;
     static constexpr int BM = 16 * TM * WM, BN = 16 * TN * WN;
     static constexpr int PART_FLOATS = BM * BN;
-    static constexpr int PARTS = 256 * 256 / (BM * BN);  // of a tile of 256 x 256: 1; 2, 4: the small tiles
+    static constexpr int PARTS = 256 * 256 / (BM * BN);  // of a tile of 256 x 256: 1 (also 224, 192, 160 x 256); 2, 4: the small tiles
+    static constexpr int LA = (BM + 63) / 64, A_STAGE = LA * 64 * 128;  // loads a wavefront, LDS bytes of a k tile of A (whole loads)
     static_assert(NW == 8, "eight wavefronts");
 };
 
@@ -82,9 +83,12 @@ __device__ __forceinline__ uint32_t g8_lds_addr(const void* p) {
 }
 // Byte offset of row `row` of an operand of m rows of `pitch` bytes. Rows past m lie out of the resource's range and read zero: what they would multiply is never
 // stored, and zeros take less of the board's power, which is what bounds the loop. (Operands of 2 GB and more, whose range such an offset could meet: row m - 1 again.)
-__device__ __forceinline__ uint32_t g8_row(uint32_t row, uint32_t m, uint32_t pitch) {
-    const uint32_t past = m * pitch <= 0x7fff0000u ? 0x80000000u : (m - 1) * pitch;
-    return row < m ? row * pitch : past;
+// ZERO false: row m - 1 again in any case (the stream-K forms, which meet few such rows: with the other offsets their loops of 256 registers are 1 % slower). at: byte
+// of the lane's piece in the row.
+template <bool ZERO>
+__device__ __forceinline__ uint32_t g8_row(uint32_t row, uint32_t m, uint32_t pitch, uint32_t at) {
+    const uint32_t off = (row < m ? row : m - 1) * pitch + at;
+    return ZERO && row >= m && m * pitch <= 0x7fff0000u ? 0x80000000u : off;
 }
 // chunk position <-> chunk (its own inverse): identity, or the two low bits swapped
 template <bool PERM>
@@ -143,10 +147,10 @@ struct G8Dense {
 // barrier sits between the slices: by then every wavefront has this tile's fragments in registers (this tile's LDS stages
 // are free for the k tiles NA / NW ahead) and the loads of tile kt + 1 have been waited for. Slice 0 issues the weight loads,
 // slice 1 those of A.
-template <class T, int NA, int NW, bool BF16, class W>
+template <class T, int NA, int NW, bool BF16, bool ZERO, class W>
 __device__ __forceinline__ void g8_mainloop(const void* a, uint32_t lda, uint32_t m, uint32_t kt0, uint32_t ktiles, uint32_t m0,
                                             const W& wo, unsigned char* lds, f32x4 (&acc)[T::TM][T::TN]) {
-    constexpr int TM = T::TM, TN = T::TN, LA = T::BM / 64, LB = W::LOADS, A_STAGE = T::BM * 128, W_AT = NA * A_STAGE;
+    constexpr int TM = T::TM, TN = T::TN, LA = T::LA, LB = W::LOADS, A_STAGE = T::A_STAGE, W_AT = NA * A_STAGE;
     static_assert(NA >= 2 && NW >= 2 && g8_flight0(LA, NA, LB, NW) < 64, "loads in flight");
     static_assert(W_AT + NW * W::STAGE <= 160 * 1024, "LDS");
     const uint32_t lane = threadIdx.x & 63, wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
@@ -156,7 +160,7 @@ __device__ __forceinline__ void g8_mainloop(const void* a, uint32_t lda, uint32_
 #pragma unroll
     for (int j = 0; j < LA; j++) {
         const uint32_t r = 8 * (wave + 8 * j) + (lane >> 3);
-        va[j] = g8_row(m0 + r, m, lda * 2) + (g8_perm<W::kPerm>((lane & 7) ^ (r & 7))) * 16;
+        va[j] = g8_row<ZERO>(r < T::BM ? m0 + r : m, m, lda * 2, (g8_perm<W::kPerm>((lane & 7) ^ (r & 7))) * 16);
     }
     const uint32_t base = g8_lds_addr(lds) + wave * 1024;
     auto ktc = [&](uint32_t kt) { return kt0 + (kt < ktiles ? kt : ktiles - 1); };  // past the end: the last tile again, never used
@@ -300,7 +304,7 @@ __device__ __forceinline__ void g8_reduce_rows(const float* __restrict__ part, u
         const uint32_t tiles_m = (m + T::BM - 1) / T::BM;
         tm = t % tiles_m, tn = t / tiles_m;
     } else {
-        gemm_raster(first + t, (m + 255) / 256, (n + 255) / 256, group, tm, tn);
+        gemm_raster(first + t, (m + T::BM - 1) / T::BM, (n + T::BN - 1) / T::BN, group, tm, tn);
     }
     const uint32_t m0 = tm * T::BM, n0 = tn * T::BN + cb * 128;
     if (m0 + (b / CB) * 8 >= m || n0 >= n) return;
@@ -332,10 +336,10 @@ __device__ __forceinline__ void g8_reduce_rows(const float* __restrict__ part, u
 // weights, double-buffered.
 // W: kPerm = true, STAGE bytes and LOADS loads a stage, issue(kt, dst of the stage, j, wave), Raw, read(stage in LDS, row of
 // the tile, lane group) -> Raw, expand(Raw, kk) -> values 8 kk .. + 7.
-template <class T, int NA, int NW, class W>
+template <class T, int NA, int NW, bool ZERO, class W>
 __device__ __forceinline__ void g8_mainloop_packed(const _Float16* a, uint32_t lda, uint32_t m, uint32_t kt0, uint32_t ktiles, uint32_t m0,
                                                    const W& wo, unsigned char* lds, f32x4 (&acc)[T::TM][T::TN]) {
-    constexpr int TM = T::TM, TN = T::TN, LA = T::BM / 64, LB = W::LOADS, A_STAGE = T::BM * 128, W_AT = NA * A_STAGE;
+    constexpr int TM = T::TM, TN = T::TN, LA = T::LA, LB = W::LOADS, A_STAGE = T::A_STAGE, W_AT = NA * A_STAGE;
     static_assert(NA >= 2 && NW >= 2 && g8_flight0(LA, NA, LB, NW) < 64, "loads in flight");
     static_assert(W_AT + NW * W::STAGE <= 160 * 1024, "LDS");
     static_assert(W::kPerm, "A's chunks");
@@ -346,7 +350,7 @@ __device__ __forceinline__ void g8_mainloop_packed(const _Float16* a, uint32_t l
 #pragma unroll
     for (int j = 0; j < LA; j++) {
         const uint32_t r = 8 * (wave + 8 * j) + (lane >> 3);
-        va[j] = g8_row(m0 + r, m, lda * 2) + (g8_perm<true>((lane & 7) ^ (r & 7))) * 16;
+        va[j] = g8_row<ZERO>(r < T::BM ? m0 + r : m, m, lda * 2, (g8_perm<true>((lane & 7) ^ (r & 7))) * 16);
     }
     const uint32_t base = g8_lds_addr(lds);
     auto ktc = [&](uint32_t kt) { return kt0 + (kt < ktiles ? kt : ktiles - 1); };
@@ -442,10 +446,10 @@ __device__ __forceinline__ void g8_mainloop_packed(const _Float16* a, uint32_t l
 // W: RAW_STAGE bytes and LOADS loads a packed stage, issue(kt, dst of the stage, j, wave), Words, read(stage in LDS) -> Words,
 // prepare(words), OPS 8-value chunks a thread, pair(words, chunk, p) -> values 2 p, 2 p + 1 of a chunk as packed fp16,
 // put(weight stage, chunk, 4 pairs).
-template <class T, int NA, int NR, class W>
+template <class T, int NA, int NR, bool ZERO, class W>
 __device__ __forceinline__ void g8_mainloop_decode(const _Float16* a, uint32_t lda, uint32_t m, uint32_t kt0, uint32_t ktiles, uint32_t m0,
                                                    const W& wo, unsigned char* lds, f32x4 (&acc)[T::TM][T::TN]) {
-    constexpr int TM = T::TM, TN = T::TN, LA = T::BM / 64, LR = W::LOADS, A_STAGE = T::BM * 128, W_STAGE = T::BN * 128;
+    constexpr int TM = T::TM, TN = T::TN, LA = T::LA, LR = W::LOADS, A_STAGE = T::A_STAGE, W_STAGE = T::BN * 128;
     constexpr int W_AT = NA * A_STAGE, R_AT = W_AT + 2 * W_STAGE;
     static_assert(R_AT + NR * W::RAW_STAGE <= 160 * 1024, "LDS");
     static_assert(NA >= 2 && NR >= 2 && NA <= NR + 1, "stages");
@@ -459,7 +463,7 @@ __device__ __forceinline__ void g8_mainloop_decode(const _Float16* a, uint32_t l
 #pragma unroll
     for (int j = 0; j < LA; j++) {
         const uint32_t r = 8 * (wave + 8 * j) + (lane >> 3);
-        va[j] = g8_row(m0 + r, m, lda * 2) + ((lane & 7) ^ (r & 7)) * 16;
+        va[j] = g8_row<ZERO>(r < T::BM ? m0 + r : m, m, lda * 2, ((lane & 7) ^ (r & 7)) * 16);
     }
     const uint32_t base = g8_lds_addr(lds);
     auto ktc = [&](uint32_t kt) { return kt0 + (kt < ktiles ? kt : ktiles - 1); };
@@ -576,10 +580,10 @@ __device__ __forceinline__ void g8_mainloop_decode(const _Float16* a, uint32_t l
 // place behind the last column. The barrier comes after the fifth column, the first that makes room for the next tile's.
 // a: codes [m][lda] (bytes).
 typedef int g8_i32x8 __attribute__((ext_vector_type(8)));
-template <class T, int NA, int NW>
+template <class T, int NA, int NW, bool ZERO>
 __device__ __forceinline__ void g8_mainloop_f8(const uint8_t* a, uint32_t lda, uint32_t m, uint32_t kt0, uint32_t ktiles, uint32_t m0,
                                                const G8Dense<T>& wo, unsigned char* lds, f32x4 (&acc)[T::TM][T::TN]) {
-    constexpr int TM = T::TM, TN = T::TN, R = 4, LA = T::BM / 64, LB = G8Dense<T>::LOADS, A_STAGE = T::BM * 128, W_AT = NA * A_STAGE;
+    constexpr int TM = T::TM, TN = T::TN, R = 4, LA = T::LA, LB = G8Dense<T>::LOADS, A_STAGE = T::A_STAGE, W_AT = NA * A_STAGE;
     constexpr int W_STAGE = G8Dense<T>::STAGE, BAR = TN - R;  // the barrier follows column BAR
     static_assert(TN == 2 * R || TN == R, "a ring of half or of all the columns");
     static_assert(NA >= 2 && NW >= 2 && g8_flight0(LA, NA, LB, NW) < 64, "loads in flight");
@@ -591,7 +595,7 @@ __device__ __forceinline__ void g8_mainloop_f8(const uint8_t* a, uint32_t lda, u
 #pragma unroll
     for (int j = 0; j < LA; j++) {
         const uint32_t r = 8 * (wave + 8 * j) + (lane >> 3);
-        va[j] = g8_row(m0 + r, m, lda) + ((lane & 7) ^ (r & 7)) * 16;
+        va[j] = g8_row<ZERO>(r < T::BM ? m0 + r : m, m, lda, ((lane & 7) ^ (r & 7)) * 16);
     }
     const uint32_t base = g8_lds_addr(lds) + wave * 1024;
     auto ktc = [&](uint32_t kt) { return kt0 + (kt < ktiles ? kt : ktiles - 1); };
@@ -755,7 +759,7 @@ __device__ __forceinline__ G8SmallWork g8_small_work(uint32_t pid, uint32_t grid
 template <class T, bool SK, class Main, class Finish>
 __device__ __forceinline__ void g8_schedule(const GemmSched& sc, uint32_t m, uint32_t n, uint32_t group, uint32_t ktiles,
                                             unsigned char* lds, Main main, Finish finish) {
-    const uint32_t p = blockIdx.x, tiles_m = (m + 255) / 256, tiles_n = (n + 255) / 256;
+    const uint32_t p = blockIdx.x, tiles_m = (m + T::BM - 1) / T::BM, tiles_n = (n + T::BN - 1) / T::BN;
     f32x4 acc[T::TM][T::TN];
     if constexpr (T::PARTS > 1) {
         const G8SmallWork wk = g8_small_work(p, gridDim.x, (m + T::BM - 1) / T::BM, sc.splits);

@@ -22,6 +22,9 @@ __device__ __forceinline__ void bf16_store4(uint16_t* c, const uint16_t* res, si
 typedef G8Tile<4, 2, 4, 8> Bf16Tile;    // 256 x 256
 typedef G8Tile<4, 2, 2, 8> Bf16TileS1;  // 128 x 256
 typedef G8Tile<4, 2, 2, 4> Bf16TileS2;  // 128 x 128, two programs a CU
+typedef G8Tile<2, 4, 7, 4> Bf16TileH7;  // 224 x 256
+typedef G8Tile<2, 4, 6, 4> Bf16TileH6;  // 192 x 256
+typedef G8Tile<2, 4, 5, 4> Bf16TileH5;  // 160 x 256
 // k tiles of A and of W in LDS: as many as the tile leaves room for
 template <class T>
 struct Bf16Stages {
@@ -40,7 +43,7 @@ __device__ __forceinline__ void bf16_gemm_program(const uint16_t* a, const uint1
         [&](uint32_t m0, uint32_t n0, uint32_t kt0, uint32_t ktn, f32x4(&acc)[T::TM][T::TN]) {
             G8Dense<T> wo;
             wo.rows(w, n, k, n0);
-            g8_mainloop<T, Bf16Stages<T>::NA, Bf16Stages<T>::NW, true>(a, lda, m, kt0, ktn, m0, wo, lds, acc);
+            g8_mainloop<T, Bf16Stages<T>::NA, Bf16Stages<T>::NW, true, true>(a, lda, m, kt0, ktn, m0, wo, lds, acc);
         },
         [&](uint32_t m0, uint32_t n0, f32x4(&acc)[T::TM][T::TN]) {
             const uint32_t row0 = m0 + wm * 16 * T::TM, col0 = n0 + wn * 16 * T::TN;
@@ -73,6 +76,9 @@ __device__ __forceinline__ void bf16_gemm_program(const uint16_t* a, const uint1
 BF16_GEMM_KERNELS(, Bf16Tile)
 BF16_GEMM_KERNELS(_s1, Bf16TileS1)
 BF16_GEMM_KERNELS(_s2, Bf16TileS2)
+BF16_GEMM_KERNELS(_h7, Bf16TileH7)
+BF16_GEMM_KERNELS(_h6, Bf16TileH6)
+BF16_GEMM_KERNELS(_h5, Bf16TileH5)
 
 // SwiGLU over a gate|up linear whose weight rows are interleaved in blocks of 8 ([gate 0..8, up 0..8, gate 8..16, ...],
 // fe_interleave_gu): of the 4 lanes that hold one 16-column block of a row, lanes 0, 1 have the 8 gate sums and lanes 2, 3
@@ -109,6 +115,9 @@ __device__ __forceinline__ void bf16_swiglu_store4(uint16_t* act, const float (&
 BF16_SWIGLU_KERNELS(, Bf16Tile)
 BF16_SWIGLU_KERNELS(_s1, Bf16TileS1)
 BF16_SWIGLU_KERNELS(_s2, Bf16TileS2)
+BF16_SWIGLU_KERNELS(_h7, Bf16TileH7)
+BF16_SWIGLU_KERNELS(_h6, Bf16TileH6)
+BF16_SWIGLU_KERNELS(_h5, Bf16TileH5)
 
 // dst row 16 b + i = gate row 8 b + i for i < 8, up row 8 b + i - 8 otherwise: the weight layout of fe_gemm_bf16_swiglu.
 // grid 2 inter, 256 threads; k % 8 == 0. (kernels/k-core/src/gemm.rs:281-296: fe_interleave_gu)

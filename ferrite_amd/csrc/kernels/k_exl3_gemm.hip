@@ -151,7 +151,7 @@ __device__ __forceinline__ void exl3_gemm_body(const _Float16* __restrict__ xh, 
                           [&](uint32_t m0, uint32_t n0, uint32_t kt0, uint32_t ktn, unsigned char* lds, f32x4(&acc)[T::TM][T::TN]) {
                               Exl3Packed<BITS, T> w;
                               w.setup(trellis, n, k, n0, stride_k, stride_nb);
-                              g8_mainloop_decode<T, Exl3Stages<BITS, T>::NA, Exl3Stages<BITS, T>::NR>(xh, k, m, kt0, ktn, m0, w, lds, acc);
+                              g8_mainloop_decode<T, Exl3Stages<BITS, T>::NA, Exl3Stages<BITS, T>::NR, !SK>(xh, k, m, kt0, ktn, m0, w, lds, acc);
                           });
 }
 
@@ -219,7 +219,7 @@ __device__ __forceinline__ void exl3_gemm_hat_kernel(HAT_GEMM_PARAMS) {
                                   const uint32_t r = n0 % 256 + 8 * (wave + 8 * j) + (lane >> 3);
                                   w.voff[j] = r * 128 + (((lane & 7) ^ ((r >> 3) & 1)) << 4);
                               }
-                              g8_mainloop<T, NA, NW, false>(xh, k, m, kt0, ktn, m0, w, lds, acc);
+                              g8_mainloop<T, NA, NW, false, !SK>(xh, k, m, kt0, ktn, m0, w, lds, acc);
                           });
 }
 // Finishes the tiles that a GEMM kernel cut along K: sums their partial slots and applies the output rotation and scale.

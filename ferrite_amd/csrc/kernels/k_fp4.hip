@@ -452,11 +452,14 @@ __device__ __forceinline__ void fp_store_piece(const FpOut& o, const float (&v)[
     }
 }
 
-// Tiles of 256 x 256, 128 x 256 (S1) and 128 x 128 (S2). Packed weights: a wavefront's columns are a quarter of the tile's, so
+// Tiles of 256 x 256, 128 x 256 (S1), 128 x 128 (S2) and 224, 192, 160 x 256 (H7, H6, H5). Packed weights: a wavefront's columns are a quarter of the tile's, so
 // that a weight is expanded by two wavefronts only. The GEMM over FP8 codes expands nothing.
 typedef G8Tile<2, 4, 8, 4> FpTile;
 typedef G8Tile<2, 4, 4, 4> FpTileS1;
 typedef G8Tile<2, 4, 4, 2> FpTileS2;
+typedef G8Tile<2, 4, 7, 4> FpTileH7;
+typedef G8Tile<2, 4, 6, 4> FpTileH6;
+typedef G8Tile<2, 4, 5, 4> FpTileH5;
 typedef G8Tile<4, 2, 4, 8> Fp8Tile;
 typedef G8Tile<4, 2, 2, 8> Fp8TileS1;
 typedef G8Tile<4, 2, 2, 4> Fp8TileS2;
@@ -480,7 +483,7 @@ __device__ __forceinline__ void fp_gemm_body(MakePacked make_packed, const FpOut
         sc, m, n, group_m, k / G8_BK, lds,
         [&](uint32_t m0, uint32_t n0, uint32_t kt0, uint32_t ktn, f32x4(&acc)[T::TM][T::TN]) {
             auto w = make_packed(n0);
-            g8_mainloop_packed<T, FpWaves<T>::NA, FpWaves<T>::NW>(aq, k, m, kt0, ktn, m0, w, lds, acc);
+            g8_mainloop_packed<T, FpWaves<T>::NA, FpWaves<T>::NW, !SK>(aq, k, m, kt0, ktn, m0, w, lds, acc);
         },
         [&](uint32_t m0, uint32_t n0, f32x4(&acc)[T::TM][T::TN]) {
             const uint32_t row0 = m0 + wm * 16 * T::TM, colb = n0 + wn * 16 * T::TN;
@@ -529,6 +532,9 @@ FP4_GEMM_KERNEL(, FpTile, false)
 FP4_GEMM_KERNEL(_sk, FpTile, true)
 FP4_GEMM_KERNEL(_s1, FpTileS1, false)
 FP4_GEMM_KERNEL(_s2, FpTileS2, false)
+FP4_GEMM_KERNEL(_h7, FpTileH7, false)
+FP4_GEMM_KERNEL(_h6, FpTileH6, false)
+FP4_GEMM_KERNEL(_h5, FpTileH5, false)
 
 #define FP_REDUCE_KERNEL(NAME, TILE)                                                                                       \
     extern "C" __global__ __launch_bounds__(256) void NAME(uint16_t* c, const float* part, const float* alpha,             \
@@ -540,6 +546,9 @@ FP4_GEMM_KERNEL(_s2, FpTileS2, false)
 FP_REDUCE_KERNEL(fe_gemm_nvfp4_reduce, FpTile)
 FP_REDUCE_KERNEL(fe_gemm_nvfp4_reduce_s1, FpTileS1)
 FP_REDUCE_KERNEL(fe_gemm_nvfp4_reduce_s2, FpTileS2)
+FP_REDUCE_KERNEL(fe_gemm_nvfp4_reduce_h7, FpTileH7)
+FP_REDUCE_KERNEL(fe_gemm_nvfp4_reduce_h6, FpTileH6)
+FP_REDUCE_KERNEL(fe_gemm_nvfp4_reduce_h5, FpTileH5)
 FP_REDUCE_KERNEL(fe_gemm_fp8_codes_reduce, Fp8Tile)
 FP_REDUCE_KERNEL(fe_gemm_fp8_codes_reduce_s1, Fp8TileS1)
 FP_REDUCE_KERNEL(fe_gemm_fp8_codes_reduce_s2, Fp8TileS2)
@@ -571,6 +580,9 @@ FP4_SWIGLU_KERNEL(, FpTile, false)
 FP4_SWIGLU_KERNEL(_sk, FpTile, true)
 FP4_SWIGLU_KERNEL(_s1, FpTileS1, false)
 FP4_SWIGLU_KERNEL(_s2, FpTileS2, false)
+FP4_SWIGLU_KERNEL(_h7, FpTileH7, false)
+FP4_SWIGLU_KERNEL(_h6, FpTileH6, false)
+FP4_SWIGLU_KERNEL(_h5, FpTileH5, false)
 #define FP4_SWIGLU_REDUCE_KERNEL(SUFFIX, TILE)                                                                             \
     extern "C" __global__ __launch_bounds__(256) void fe_gemm_nvfp4_swiglu_reduce##SUFFIX(                                 \
         const float* part, const float* alpha, uint32_t m, uint32_t n, uint32_t group_m, uint32_t first, uint32_t splits,  \
@@ -581,6 +593,9 @@ FP4_SWIGLU_KERNEL(_s2, FpTileS2, false)
 FP4_SWIGLU_REDUCE_KERNEL(, FpTile)
 FP4_SWIGLU_REDUCE_KERNEL(_s1, FpTileS1)
 FP4_SWIGLU_REDUCE_KERNEL(_s2, FpTileS2)
+FP4_SWIGLU_REDUCE_KERNEL(_h7, FpTileH7)
+FP4_SWIGLU_REDUCE_KERNEL(_h6, FpTileH6)
+FP4_SWIGLU_REDUCE_KERNEL(_h5, FpTileH5)
 
 // FP8: the 64 codes of row r = 128 nt + i, k tile kt are at w + nt * w_snt + kt * w_skt + i * w_sr; both fp16 expansions
 // are the values themselves. Finished by fe_gemm_nvfp4_reduce with scale 1. (kernels/k-fp4/src/lib.rs:472-484)
@@ -630,7 +645,7 @@ __device__ __forceinline__ void gemm_fp8_codes_kernel(FP8C_GEMM_PARAMS) {
                 nt = nt < nts ? nt : nts - 1;  // an odd count of 128-row tiles: the last program reads its first tile twice
                 wo.voff[j] = nt * w_snt + (ch >> 2) * w_skt + (r & 127) * w_sr + (ch & 3) * 16;
             }
-            g8_mainloop_f8<T, NA, 3>(aq, k, m, kt0, ktn, m0, wo, lds, acc);
+            g8_mainloop_f8<T, NA, 3, !SK>(aq, k, m, kt0, ktn, m0, wo, lds, acc);
         },
         [&](uint32_t m0, uint32_t n0, f32x4(&acc)[T::TM][T::TN]) {
             const uint32_t row0 = m0 + wm * 16 * T::TM, colb = n0 + wn * 16 * T::TN;
@@ -650,6 +665,9 @@ FP8C_GEMM_KERNEL(, Fp8Tile, false)
 FP8C_GEMM_KERNEL(_sk, Fp8Tile, true)
 FP8C_GEMM_KERNEL(_s1, Fp8TileS1, false)
 FP8C_GEMM_KERNEL(_s2, Fp8TileS2, false)
+FP8C_GEMM_KERNEL(_h7, FpTileH7, false)
+FP8C_GEMM_KERNEL(_h6, FpTileH6, false)
+FP8C_GEMM_KERNEL(_h5, FpTileH5, false)
 
 // ---- GEMV (1..48 rows) -------------------------------------------------------------------------------------------------
 
