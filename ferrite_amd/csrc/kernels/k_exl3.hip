@@ -379,7 +379,7 @@ __device__ __forceinline__ void gemvb_body(const GemvMember mb, uint32_t p0, uin
     constexpr int DEPTH = 4;  // load steps in flight per lane (5 and 6 measured 2..5 % slower, 8 10 %: 22.9 against 20.7 us)
     constexpr int GROUP = 8;  // steps of straight-line code per loop iteration (a multiple of DEPTH)
     const uint32_t tid = threadIdx.x, lane = tid & 63, wave = tid >> 6;
-    const uint32_t r = lane & 15, g = lane >> 4, q = r & 7, tau = r >> 3;
+    const uint32_t r = lane & 15, g = lane >> 4, q = r >> 1, tau = r & 1;
     const uint32_t n = mb.n, spb = k / 64, upb = spb / 2;  // load steps, units a column block
     const uint32_t base = mb.base, rem = mb.rem;
     // This workgroup runs the programs p0 .. p0 + np - 1 of the partition one after the other. Their runs are contiguous, so
@@ -497,14 +497,16 @@ __device__ __forceinline__ void gemvb_body(const GemvMember mb, uint32_t p0, uin
 
     auto one = [&](LaneWords<BITS>& slot, uint32_t t) {  // t: load step within the staged chunk
         f16x8 op[2][2];
+        // the inputs are asked for in front of the decode: behind it their way out of LDS holds the products up (with the word before a lane's run in one
+        // instruction instead of five: a layer of 5120 / 17408 at 1 row 68.4 -> 67.5 us, 1024 / 2816 26.7 -> 26.3)
+        const unsigned char* xp = xs + xrow + t * 128;
+        const f16x8 x0 = *(const f16x8*)xp, x1 = *(const f16x8*)(xp + 16);
         slot.w[0] = lane_prev_word(slot.w[BITS]);
         decode_lane<BITS>(slot, op);
         issue(slot);
         // keep the refill where it is issued: left alone, the scheduler sinks the loads to the end of the group, right in
         // front of the wait for them
         __builtin_amdgcn_sched_barrier(0);
-        const unsigned char* xp = xs + xrow + t * 128;
-        f16x8 x0 = *(const f16x8*)xp, x1 = *(const f16x8*)(xp + 16);
         acc[0] = __builtin_amdgcn_mfma_f32_16x16x32_f16(op[0][0], x0, acc[0], 0, 0, 0);
         acc[1] = __builtin_amdgcn_mfma_f32_16x16x32_f16(op[1][0], x0, acc[1], 0, 0, 0);
         acc[0] = __builtin_amdgcn_mfma_f32_16x16x32_f16(op[0][1], x1, acc[0], 0, 0, 0);
@@ -557,9 +559,9 @@ __device__ __forceinline__ void gemvb_body(const GemvMember mb, uint32_t p0, uin
     uint32_t pending = 0;
     auto flush = [&](uint32_t fnb, uint32_t p, bool keep) {
         __syncthreads();  // the previous segment's readers are done with `red`
-        // rows 4 g .. 4 g + 3 of A are columns 16 (g >> 1) + 4 (g & 1) + 8 h .. + 3 of the wavefront's 32 (tile g >> 1 of
-        // its pair, n = 4 (g & 1) + i + 8 h): a lane's four sums of either half are four neighbouring columns
-        float* rp = red + 32 * wave + 16 * (g >> 1) + 4 * (g & 1);
+        // a lane's four sums of either half: columns 16 (g & 1) + 4 (g >> 1) + 8 h .. + 3 of the wavefront's 32
+        acc[0] = lane_cols(acc[0]), acc[1] = lane_cols(acc[1]);
+        float* rp = red + 32 * wave + 16 * (g & 1) + 4 * (g >> 1);
         if (r < m) {  // accumulator column = input row
             f32x4 *r0 = (f32x4*)(rp + r * GEMV_RED_PITCH), *r1 = (f32x4*)(rp + r * GEMV_RED_PITCH + 8);
             if (PAIRS && pending) acc[0] = *r0 + acc[0], acc[1] = *r1 + acc[1];
@@ -914,7 +916,7 @@ __device__ __forceinline__ void gemv_wide_body(const GemvMember mb, uint32_t p, 
 #pragma unroll
                 for (int i = 0; i < BITS; i++) lw.w[i + 1] = words[i];
             }
-            lw.w[0] = lane_prev_word(lw.w[BITS]);
+            lw.w[0] = lane_prev_word_halves(lw.w[BITS]);
             f16x8 op[2][2];
             decode_lane<BITS>(lw, op);
             const unsigned char* xs = xp + slot * C::X_STAGE;

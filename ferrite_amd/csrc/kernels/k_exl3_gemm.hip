@@ -66,7 +66,7 @@ struct Exl3Packed {
     // The word before the run and the windows over the word boundaries. At 128 columns the threads of row half 1 shift their stream by
     // the 4 positions between the halves, so that both decode the same positions.
     __device__ __forceinline__ void prepare(Words& w) const {
-        w.w.w[0] = lane_prev_word(w.w.w[BITS]);
+        w.w.w[0] = lane_prev_word_halves(w.w.w[BITS]);
         if constexpr (BLOCKS == 1) {
             if (threadIdx.x >= 256) {
 #pragma unroll

@@ -111,7 +111,7 @@ __device__ __forceinline__ void rgemm_segment(const RgJob& job, uint32_t tile, u
         }
     };
     auto prepare = [&]() {
-        lw.w[0] = lane_prev_word(lw.w[BITS]);
+        lw.w[0] = lane_prev_word_halves(lw.w[BITS]);
         win = lane_windows<BITS>(lw);
     };
     u32x4 op[2][2][2];  // decoded weights of a k tile: [set][row half][k half], 8 values each
