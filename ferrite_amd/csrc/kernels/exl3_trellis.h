@@ -154,7 +154,31 @@ __device__ __forceinline__ uint32_t decode_lane_pair(const LaneWords<BITS>& lw, 
 }
 
 // Store 4 consecutive outputs. mode: 0 bf16, 1 f32, 2 bf16 y += v (f32 add, one rounding), 3 f32 y += v.
-// (kernels/k-exl3/src/gemv.rs:122-145)
+// (kernels/k-exl3/src/gemv.rs:122-145) old: what stands there, for the adding modes (store4_old), read ahead by the launches that only add sums: behind them
+// it is one more trip to memory (decode of 40 rows 112.8 -> 111.5 us; in the GEMV's own finish it gains nothing and costs registers).
+__device__ __forceinline__ u32x4 store4_old(const void* y, uint32_t mode, size_t i) {
+    u32x4 o = {0, 0, 0, 0};
+    if (mode == 3) o = *(const u32x4*)((const float*)y + i);
+    if (mode == 2) {
+        const u32x2 t = *(const u32x2*)((const uint16_t*)y + i);
+        o[0] = t[0], o[1] = t[1];
+    }
+    return o;
+}
+__device__ __forceinline__ void store4(void* y, uint32_t mode, size_t i, float (&v)[4], u32x4 old) {
+    if (mode & 1) {
+        f32x4 o = {v[0], v[1], v[2], v[3]};
+        if (mode & 2) o += __builtin_bit_cast(f32x4, old);
+        *(f32x4*)((float*)y + i) = o;
+    } else {
+        if (mode & 2) {
+            v[0] += __uint_as_float(old[0] << 16), v[1] += __uint_as_float(old[0] & 0xffff0000u);
+            v[2] += __uint_as_float(old[1] << 16), v[3] += __uint_as_float(old[1] & 0xffff0000u);
+        }
+        u32x2 o = {pack_bf16x2(v[0], v[1]), pack_bf16x2(v[2], v[3])};
+        *(u32x2*)((uint16_t*)y + i) = o;
+    }
+}
 __device__ __forceinline__ void store4(void* y, uint32_t mode, size_t i, float (&v)[4]) {
     if (mode & 1) {
         float* p = (float*)y + i;
@@ -173,16 +197,18 @@ __device__ __forceinline__ void store4(void* y, uint32_t mode, size_t i, float (
     }
 }
 
-// H over the 128 sums of a row (4 a lane of a half wavefront), * svh / sqrt(128), stored. (gemv.rs:172-180)
-__device__ __forceinline__ void finish_row(float (&v)[4], uint32_t l32, const uint16_t* svh, uint32_t col, void* y,
-                                           uint32_t mode, size_t at) {
+// H over the 128 sums of a row (4 a lane of a half wavefront), * svh / sqrt(128), stored. (gemv.rs:172-180) s: the lane's four output scales (fp16).
+__device__ __forceinline__ void finish_row(float (&v)[4], uint32_t l32, u32x2 s, void* y, uint32_t mode, size_t at, u32x4 old) {
     fwht128_half_wave(v, l32);
-    u32x2 s = *(const u32x2*)(svh + col);
     v[0] = v[0] * FE_HAD_SCALE * f16_bits_to_f32(s[0] & 0xffff);
     v[1] = v[1] * FE_HAD_SCALE * f16_bits_to_f32(s[0] >> 16);
     v[2] = v[2] * FE_HAD_SCALE * f16_bits_to_f32(s[1] & 0xffff);
     v[3] = v[3] * FE_HAD_SCALE * f16_bits_to_f32(s[1] >> 16);
-    store4(y, mode, at, v);
+    store4(y, mode, at, v, old);
+}
+__device__ __forceinline__ void finish_row(float (&v)[4], uint32_t l32, const uint16_t* svh, uint32_t col, void* y,
+                                           uint32_t mode, size_t at) {
+    finish_row(v, l32, *(const u32x2*)(svh + col), y, mode, at, store4_old(y, mode, at));
 }
 
 // The lane's four output scales as finish_row applies them, for callers that finish many rows of the same columns.

@@ -1041,9 +1041,13 @@ __device__ __forceinline__ void wide_finish_body(const GemvJob& job, uint32_t k,
     gemv_member_now(mb);
     const WideSpan sp = wide_span<PER>(mb, nb, k / 128);
     if (row >= m || ((y_mode & WIDE_WHOLE) && sp.first == sp.last)) return;
+    const uint32_t col = nb * 128 + 4 * l32;
+    const size_t at = (size_t)row * mb.n + col;
+    const u32x2 sv = *(const u32x2*)(mb.svh + col);  // (these two on their way beside the segments)
+    const u32x4 old = store4_old(mb.y, y_mode & 3, at);
     const f32x4 s = wide_row_sums<PER>(mb, nb, sp, m, row, l32);
     float v[4] = {s[0], s[1], s[2], s[3]};
-    finish_row(v, l32, mb.svh, nb * 128 + 4 * l32, mb.y, y_mode & 3, (size_t)row * mb.n + nb * 128 + 4 * l32);
+    finish_row(v, l32, sv, mb.y, y_mode & 3, at, old);
 }
 // The same for gate and up in front of down: both outputs (bf16), and down's rotated input of SwiGLU(gate, up), a 128-channel block of which
 // is a column block of the two. grid (column blocks of one of them, ceil(m / 8)).
@@ -1053,13 +1057,16 @@ __device__ __forceinline__ void wide_finish_mlp_body(const GemvJob& job, uint32_
     gemv_member_now(job.m[0]);
     if (row >= m) return;
     gemv_member_now(job.m[1]);
+    RotRaw raw = {};
+    raw.s = *(const u32x2*)(suh + c);
+    const u32x2 svs[2] = {*(const u32x2*)(job.m[0].svh + c), *(const u32x2*)(job.m[1].svh + c)};  // (on their way beside the segments)
     u32x2 y[2];
 #pragma unroll
     for (int i = 0; i < 2; i++) {
         const f32x4 s = wide_row_sums<PER>(job.m[i], nb, wide_span<PER>(job.m[i], nb, k / 128), m, row, l32);
         float v[4] = {s[0], s[1], s[2], s[3]};
         fwht128_half_wave(v, l32);
-        const u32x2 sv = *(const u32x2*)(job.m[i].svh + c);
+        const u32x2 sv = svs[i];
         v[0] = v[0] * FE_HAD_SCALE * f16_bits_to_f32(sv[0] & 0xffff);  // finish_row's products
         v[1] = v[1] * FE_HAD_SCALE * f16_bits_to_f32(sv[0] >> 16);
         v[2] = v[2] * FE_HAD_SCALE * f16_bits_to_f32(sv[1] & 0xffff);
@@ -1067,8 +1074,7 @@ __device__ __forceinline__ void wide_finish_mlp_body(const GemvJob& job, uint32_
         y[i] = (u32x2){pack_bf16x2(v[0], v[1]), pack_bf16x2(v[2], v[3])};
         *(u32x2*)((uint16_t*)job.m[i].y + (size_t)row * n + c) = y[i];
     }
-    RotRaw raw = {};
-    raw.xb = y[0], raw.ub = y[1], raw.s = *(const u32x2*)(suh + c);
+    raw.xb = y[0], raw.ub = y[1];
     *(u32x2*)(xh + (size_t)row * n + c) = rot_finish(raw, 2, l32);
 }
 #define WIDE_FINISH_KERNELS(SUFFIX, PER)                                                                                         \

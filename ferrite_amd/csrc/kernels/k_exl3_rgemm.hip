@@ -309,6 +309,10 @@ extern "C" __global__ __launch_bounds__(256) void exl3_rgemm_reduce(RgJob job, u
     if (first == last || nb >= mb.n / 128 || tm * bm + blockIdx.x % per * 8 >= job.rows) return;  // (one run's: finished there)
     const uint32_t slot = blocks * bm * 128;
     const float* p = job.part + (size_t)(first + t) * slot + ((size_t)b * bm + row) * 128 + 4 * l32;
+    const uint32_t col = nb * 128 + 4 * l32;
+    const size_t to = (size_t)at * mb.n + col;
+    const u32x2 sv = *(const u32x2*)(mb.svh + col);  // (these two on their way beside the pieces)
+    const u32x4 old = at < job.rows ? store4_old(mb.y, job.y_mode, to) : (u32x4){0, 0, 0, 0};
     constexpr uint32_t AT_ONCE = 8;  // loads in flight: one at a time the launch took 8.2 us on the 20 pieces of 5120 x 1024 at 128 rows (5.1 now)
     f32x4 sum = *(const f32x4*)p;
     for (uint32_t i0 = 1; i0 <= last - first; i0 += AT_ONCE) {
@@ -320,7 +324,7 @@ extern "C" __global__ __launch_bounds__(256) void exl3_rgemm_reduce(RgJob job, u
             if (first + i0 + i <= last) sum += piece[i];
     }
     float v[4] = {sum[0], sum[1], sum[2], sum[3]};
-    if (at < job.rows) finish_row(v, l32, mb.svh, nb * 128 + 4 * l32, mb.y, job.y_mode, (size_t)at * mb.n + nb * 128 + 4 * l32);
+    if (at < job.rows) finish_row(v, l32, sv, mb.y, job.y_mode, to, old);
 }
 
 #define RGEMM_KERNEL(BITS, RG, KG)                                                                                \
