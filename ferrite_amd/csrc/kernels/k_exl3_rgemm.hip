@@ -293,9 +293,17 @@ __device__ __forceinline__ void rgemm_body(const RgJob& job) {
     }
 }
 
+// Every line of the launch's arguments asked for at once, in front of the first use of any (as GEMV_JOB_LINES of k_exl3.hip): a trip to memory instead of five, one
+// behind the other.
+#define RG_JOB_LINES(job)                                                                                                                    \
+    "s"((job).m[0].first), "s"((job).m[1].first), "s"((job).m[2].first), "s"((job).m[3].first), "s"((job).count), "s"((job).k), "s"((job).rows), \
+        "s"((job).y_mode), "s"((job).tiles_m), "s"((job).tiles_n), "s"((job).group), "s"((job).full), "s"((job).runs), "s"((job).base),   \
+        "s"((job).rem), "s"((job).per), "s"((job).part)
+
 // Finishes the cut tiles: sums the pieces of a row in the order of K, then the output rotation and scale. grid: tiles after the full
 // ones x blocks x bm / 8, 256 threads, a half wavefront a row. all: steps of a tile.
 extern "C" __global__ __launch_bounds__(256) void exl3_rgemm_reduce(RgJob job, uint32_t bm, uint32_t blocks, uint32_t all) {
+    asm volatile("" ::RG_JOB_LINES(job), "s"(bm), "s"(blocks), "s"(all));
     const uint32_t per = bm / 8, l32 = threadIdx.x & 31, c = blockIdx.x / per, row = blockIdx.x % per * 8 + (threadIdx.x >> 5);
     const uint32_t t = c / blocks, b = c % blocks;
     uint32_t tm, tn;
@@ -329,6 +337,7 @@ extern "C" __global__ __launch_bounds__(256) void exl3_rgemm_reduce(RgJob job, u
 
 #define RGEMM_KERNEL(BITS, RG, KG)                                                                                \
     extern "C" __global__ __launch_bounds__(512, 2) void exl3_rgemm_b##BITS##_r##RG##_k##KG(RgJob job) {         \
+        asm volatile("" ::RG_JOB_LINES(job));                                                                     \
         rgemm_body<BITS, RG, KG>(job);                                                                            \
     }
 #define RGEMM_ROWS(BITS)                                                                                          \

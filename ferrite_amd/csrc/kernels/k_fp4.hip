@@ -515,6 +515,8 @@ __device__ __forceinline__ void fp_reduce_body(const FpOut& out, const float* pa
         uint32_t s_skt, uint32_t s_sr, GemmSched sc
 template <class T, bool SK>
 __device__ __forceinline__ void gemm_nvfp4_kernel(FP4_GEMM_PARAMS) {
+    asm volatile("" ::"s"(c), "s"(aq), "s"(w), "s"(sw), "s"(alpha), "s"(res), "s"(m), "s"(n), "s"(k), "s"(ldc), "s"(group_m), "s"(w_snt), "s"(w_skt), "s"(w_sr),
+                 "s"(s_snt), "s"(s_skt), "s"(s_sr), GEMM_SCHED_WORDS(sc));
     FpOut out = {c, res, ldc, nullptr, nullptr, nullptr, 0.f};
     fp_gemm_body<T, false, SK>(
         [&](uint32_t n0) {
@@ -562,6 +564,8 @@ FP_REDUCE_KERNEL(fe_gemm_fp8_codes_reduce_s2, Fp8TileS2)
         GemmSched sc, uint8_t *q_codes, uint8_t *q_sf, _Float16 *q_aq, float qg
 template <class T, bool SK>
 __device__ __forceinline__ void gemm_nvfp4_swiglu_kernel(FP4_SWIGLU_PARAMS) {
+    asm volatile("" ::"s"(aq), "s"(w), "s"(sw), "s"(alpha), "s"(m), "s"(n), "s"(k), "s"(group_m), "s"(w_snt), "s"(w_skt), "s"(w_sr), "s"(s_snt), "s"(s_skt),
+                 "s"(s_sr), GEMM_SCHED_WORDS(sc), "s"(q_codes), "s"(q_sf), "s"(q_aq), "s"(qg));
     FpOut out = {nullptr, nullptr, 0, q_codes, q_sf, q_aq, qg};
     fp_gemm_body<T, true, SK>(
         [&](uint32_t n0) {
