@@ -20,12 +20,14 @@ constexpr uint32_t kGemmLds[kFeGemmForms] = {144 * 1024, 144 * 1024, 136 * 1024,
 constexpr uint32_t kGemmLds8[kFeGemmForms] = {160 * 1024, 160 * 1024, 144 * 1024, 80 * 1024, 160 * 1024, 144 * 1024, 144 * 1024};
 // Forms of the GEMV over programs of 8 CO columns: rows / 2 and CO
 constexpr uint32_t kWideRowForms[4] = {1, 2, 4, 8}, kWideColForms[7] = {1, 2, 3, 4, 5, 6, 9};
-// Fp4Wide<XP, CO, Q>::LDS of k_fp4.hip; Q (rows m of k quantized by the program itself): with its four wavefronts' activations in the place of a stage's
-uint32_t wide_lds(uint32_t xp, uint32_t co, bool q = false, uint32_t m = 0, uint32_t k = 0) {
-    const uint32_t cg = (co + 1) / 2, stage = (co + (q ? 0 : xp)) * 1024 + cg * 256, x = q ? ((k / 256 + 3) / 4 * m + 1) / 2 * 4096 : 0;
-    return std::max(4 * std::max(2u, std::min((q ? 15 : 20) * 1024 / stage, 6u)) * stage + x, 256 * (16 * cg + 4));
+// Fp4Wide<XP, CO, Q, WV>::LDS of k_fp4.hip; Q (rows m of k quantized by the program itself): with its wavefronts' activations in the place of a stage's
+uint32_t wide_lds(uint32_t xp, uint32_t co, uint32_t waves, bool q = false, uint32_t m = 0, uint32_t k = 0) {
+    const uint32_t cg = (co + 1) / 2, stage = (co + (q ? 0 : xp)) * 1024 + cg * 256, x = q ? ((k / 256 + waves - 1) / waves * m + 1) / 2 * 1024 * waves : 0;
+    return std::max(waves * std::max(2u, std::min((q ? 60 : 80) * 1024 / (waves * stage), 6u)) * stage + x, 64 * waves * (16 * cg + 4));
 }
 constexpr uint32_t kCuLds = 160 * 1024;
+// The wavefronts of a form: eight where K is summed in eighths and two stages of eight wavefronts fit the LDS.
+uint32_t wide_waves(uint32_t xp, uint32_t co, bool eighths, bool q = false) { return eighths && co <= 6 && (q || xp <= 2 || (xp == 4 && co <= 4)) ? 8 : 4; }
 constexpr uint32_t kGemmThreads = 512;
 constexpr uint32_t kTileM = 256;                        // GM_BM
 }  // namespace
@@ -36,8 +38,8 @@ struct fe_fp4_kernels {
     // by form (256 x 256, stream-K, 128 x 256, 128 x 128) and by tile (fe_gemm_launch); gemm8: the fp16 form, 256 x 256 only
     fe_function_t gemm4[kFeGemmForms] = {}, swiglu4[kFeGemmForms] = {}, gemm8c[kFeGemmForms] = {}, gemm8[2] = {};
     fe_function_t reduce4[kFeGemmTiles] = {}, swiglu_reduce4[kFeGemmTiles] = {}, reduce8c[kFeGemmTiles] = {};
-    fe_function_t wide[4][7] = {};   // the GEMV over programs of 8 CO columns, [kWideRowForms][kWideColForms]
-    fe_function_t wide_q[3][7] = {};  // the same, quantizing its activations itself
+    fe_function_t wide[2][4][7] = {};    // the GEMV over programs of 8 CO columns, [quarters or eighths of K][kWideRowForms][kWideColForms]
+    fe_function_t wide_q[2][3][7] = {};  // the same, quantizing its activations itself
     fe_function_t quant8 = nullptr, expand8 = nullptr;
     uint32_t cus = 0;
     // Switches of the launch paths: read from the environment once, at load; fe_fp4_kernels_set_option changes them
@@ -46,7 +48,8 @@ struct fe_fp4_kernels {
     uint32_t gemv = 1;         // up to 64 rows run the GEMV (FE_FP4_NO_GEMV=1: the GEMM's single tile row)
     uint32_t gemv_sk = 0;      // K splits of the GEMV over weight tiles; 0 = two programs a CU (FE_FP4_GEMV_SK)
     uint32_t gemv_strips = 1;  // up to 16 rows run programs of some columns over all of K; 0: weight tiles and K splits, as more rows do (FE_FP4_NO_STRIPS=1)
-    uint32_t gemv_quant = 10240;  // most values (rows x k) that the GEMV for up to 16 rows quantizes itself, in every program (FE_FP4_GEMV_QUANT)
+    // most values (rows x k) that the four wavefronts of the GEMV for up to 16 rows quantize themselves, in every program; eight take twice as many (FE_FP4_GEMV_QUANT)
+    uint32_t gemv_quant = 10240;
     uint32_t gemv_cols = 0;    // columns a program of the GEMV for up to 16 rows takes, rounded up to 8, 16, .. 48, 72; 0 = by the shape (FE_FP4_GEMV_COLS)
     int32_t xcd = -1;          // column tiles dealt to the XCDs: -1 = where the weights are the larger operand (FE_FP4_XCD)
     uint32_t fp8_f16 = 0;      // FP8 linears as fp16 expansion on the 16-bit matrix instruction (FE_FP8_F16=1)
@@ -101,13 +104,13 @@ int fe_fp4_kernels_load(fe_fp4_kernels **out) {
         snprintf(nm, sizeof nm, "fe_gemv_nvfp4_x%d", xr);
         c = fe_hip_module_get_function(&k->gemv4[xr - 1], k->module, nm);
     }
-    for (uint32_t i = 0; i < 4; i++)
-        for (uint32_t j = 0; j < 7; j++)
-            get(&k->wide[i][j], "fe_gemv_nvfp4_r" + std::to_string(kWideRowForms[i]) + "_c" + std::to_string(kWideColForms[j]),
-                wide_lds(kWideRowForms[i], kWideColForms[j]));
-    for (uint32_t i = 0; i < 3; i++)
-        for (uint32_t j = 0; j < 7; j++)
-            get(&k->wide_q[i][j], "fe_gemv_nvfp4_q" + std::to_string(kWideRowForms[i]) + "_c" + std::to_string(kWideColForms[j]), kCuLds);
+    for (uint32_t i = 0; i < 8; i++)
+        for (uint32_t j = 0; j < 7; j++) {
+            const uint32_t xp = kWideRowForms[i % 4];
+            const std::string nm = std::to_string(xp) + "_c" + std::to_string(kWideColForms[j]) + (i / 4 ? "_e" : "");
+            get(&k->wide[i / 4][i % 4][j], "fe_gemv_nvfp4_r" + nm, wide_lds(xp, kWideColForms[j], wide_waves(xp, kWideColForms[j], i / 4)));
+            if (i % 4 < 3) get(&k->wide_q[i / 4][i % 4][j], "fe_gemv_nvfp4_q" + nm, kCuLds);
+        }
     if (!c) c = fe_hip_module_get_function(&k->quant8, k->module, "fe_fp8_quant");
     if (!c) c = fe_hip_module_get_function(&k->expand8, k->module, "fe_fp8_expand");
     int cus = 0;
@@ -364,7 +367,7 @@ static uint32_t wide_cols(uint32_t n, uint32_t xp, uint32_t cus, uint32_t forced
     uint32_t best = 0;
     uint64_t least = ~0ull;
     for (uint32_t i = 0; i < 7; i++) {
-        const uint32_t co = kWideColForms[i], programs = (n / 8 + co - 1) / co, room = wide_lds(xp, co, q, m, k) <= 80 * 1024 ? 2 : 1;
+        const uint32_t co = kWideColForms[i], programs = (n / 8 + co - 1) / co, room = wide_lds(xp, co, 4, q, m, k) <= 80 * 1024 ? 2 : 1;
         if (forced) {
             best = i;
             if (8 * co >= forced) break;
@@ -377,6 +380,27 @@ static uint32_t wide_cols(uint32_t n, uint32_t xp, uint32_t cus, uint32_t forced
         if (cost <= least) best = i, least = cost;
     }
     return best;
+}
+
+// The kernel of the GEMV of up to 16 rows; q: the one that quantizes its activations itself.
+// Linears that give no CU a second program sum eighths of K, with eight wavefronts up to 8 rows: a program's steps are a chain of LDS reads, scale products and matrix
+// instructions, which two wavefronts a SIMD overlap. (By the linear's shape alone: its rows' bits are the same at 1 to 16 rows.) us, quarters -> eighths:
+// 5120 x 5120 at 1 / 4 / 8 / 12 rows 7.2 -> 6.6, 8.2 -> 8.0, 9.0 -> 9.0, 9.8 -> 9.8; 5120 x 17408 15.1 -> 14.0, 14.8 -> 14.8, 18.3 -> 17.2, 19.7 -> 20.0; 5120 x 8704 9.9 -> 9.1,
+// 10.3 -> 10.4, 11.9 -> 11.4, 12.8 -> 12.9; 2048 x 11008 9.3 -> 7.2, 9.3 -> 8.7, 9.4 -> 9.4, 12.4 -> 12.4; 10240 x 4096 at 3 9.9 -> 8.0; 7168 x 2048 at 6 6.9 -> 5.2. With more
+// programs than CUs two of four wavefronts a CU are better (34816 x 5120 at 1 row 22.7 against 24.5), and of 1024 channels half of eight have no step (1024 x 1024 at 8
+// rows 4.3 -> 4.9).
+// Programs of eight that quantize take two octets rather than one: 1024 x 5120 at 1 row 5.3 -> 4.8, 2048 x 2048 at 8 rows 5.5 -> 4.9.
+struct WideForm {
+    uint32_t programs, waves, lds;
+    fe_function_t f;
+};
+static WideForm wide_form(const fe_fp4_linear *l, const fe_fp4_kernels *kern, uint32_t m, bool q) {
+    const uint32_t form = m <= 2 ? 0 : m <= 4 ? 1 : m <= 8 ? 2 : 3, xp = kWideRowForms[form], cus = std::max(kern->cus, 1u);
+    const bool eighths = l->k >= 2048 && l->n <= 48 * cus;
+    uint32_t cols = wide_cols(l->n, xp, cus, kern->gemv_cols, q, m, l->k);
+    if (q && eighths && !cols && !kern->gemv_cols) cols = 1;
+    const uint32_t co = kWideColForms[cols], waves = wide_waves(xp, co, eighths, q);
+    return {(l->n / 8 + co - 1) / co, waves, wide_lds(xp, co, waves, q, m, l->k), (q ? kern->wide_q[eighths][form] : kern->wide[eighths][form])[cols]};
 }
 
 // Whether fe_fp4_linear_gemm takes the GEMV of up to 16 rows over programs of some columns and all of K, nothing handed between them.
@@ -397,8 +421,7 @@ static int linear_gemm(const fe_fp4_linear *l, const fe_fp4_kernels *kern, fe_st
         // at once, not more (a second round of short programs costs more than idle CUs in the first).
         const uint32_t nts = n / kTile, kts = k / 64;
         if (takes_wide(l, kern, m)) {
-            const uint32_t form = m <= 2 ? 0 : m <= 4 ? 1 : m <= 8 ? 2 : 3, xp = kWideRowForms[form];
-            const uint32_t cols = wide_cols(n, xp, std::max(kern->cus, 1u), kern->gemv_cols, x != 0, m, k), co = kWideColForms[cols];
+            const WideForm wf = wide_form(l, kern, m, x != 0);
             struct {  // Fp4QuantTo
                 fe_devptr_t codes, sf, aq;
                 uint32_t ldx;
@@ -407,7 +430,7 @@ static int linear_gemm(const fe_fp4_linear *l, const fe_fp4_kernels *kern, fe_st
             fe_devptr_t aq = x ? x : ws->aq.p, w = l->w.p, sw = l->sw.p, alpha = l->alpha.p;
             uint32_t w_snt = l->w_snt, w_skt = l->w_skt, w_sr = l->w_sr, s_snt = l->s_snt, s_skt = l->s_skt, s_sr = l->s_sr;
             void *args[] = {&y, &aq, &w, &sw, &alpha, &res, &m, &n, &k, &ldy, &w_snt, &w_skt, &w_sr, &s_snt, &s_skt, &s_sr, &to};
-            return fe_hip_launch(x ? kern->wide_q[form][cols] : kern->wide[form][cols], (n / 8 + co - 1) / co, 1, 1, 256, 1, 1, wide_lds(xp, co, x != 0, m, k), s, args);
+            return fe_hip_launch(wf.f, wf.programs, 1, 1, 64 * wf.waves, 1, 1, wf.lds, s, args);
         }
         uint32_t sk = 2 * kern->cus / nts;
         if (kern->gemv_sk) sk = kern->gemv_sk;
@@ -484,11 +507,14 @@ int fe_fp4_linear_gemm(const fe_fp4_linear *l, const fe_fp4_kernels *kern, fe_st
 // Whether the GEMV's programs each quantize all of the activations: few values, since a program waits for all of them before its first product. us, with the
 // quantizer's launch -> without: 1024 x 1024 at 1 / 8 rows 6.9 -> 3.8, 7.1 -> 4.1; 5120 x 5120 at 1 / 2 rows 8.7 -> 7.3, 8.9 -> 8.0; 17408 x 5120 at 1 / 2 15.8 -> 14.0,
 // 16.2 -> 14.5; 34816 x 5120 at 2 24.7 -> 23.7; 16384 x 2560 at 4 9.3 -> 8.3; 5120 x 8704 at 1 11.5 -> 10.0. Beyond 10240 values it turns: 34816 x 5120 at 3 rows
-// 25.2 -> 27.0, 5120 x 8704 at 3 11.7 -> 12.6, 16384 x 2560 at 6 10.2 -> 14.3 (one program a CU). Up to 8 rows, what the LDS holds and 32 bits address. Not where the output or the
+// 25.2 -> 27.0, 16384 x 2560 at 6 10.2 -> 14.3 (one program a CU). Eight wavefronts quantize twice as many in that time: 5120 x 17408 at 1 row 17.2 -> 15.9, 4096 x 4096 at
+// 4 6.7 -> 5.8, 1024 x 5120 at 4 / 5 (25600 values) 6.7 -> 6.8, 7.1 -> 7.9. Up to 8 rows, what the LDS holds and 32 bits address. Not where the output or the
 // workspace lies in the activations' memory: programs that have finished would write over what others have yet to read.
 static bool fp4_quants_itself(const fe_fp4_linear *l, const fe_fp4_kernels *kern, const fe_fp4_workspace *ws, fe_devptr_t y, uint32_t ldy, fe_devptr_t x,
                               uint32_t lda, uint32_t m) {
-    if (!m || m > 8 || !takes_wide(l, kern, m) || (uint64_t)m * l->k > std::min(kern->gemv_quant, 32768u) || (uint64_t)m * lda >= (1u << 30)) return false;
+    if (!m || m > 8 || !takes_wide(l, kern, m) || (uint64_t)m * lda >= (1u << 30)) return false;
+    const WideForm f = wide_form(l, kern, m, true);
+    if ((uint64_t)m * l->k > std::min<uint64_t>((uint64_t)kern->gemv_quant * f.waves / 4, 32768) || f.lds > kCuLds) return false;
     const fe_devptr_t xe = x + ((size_t)(m - 1) * lda + l->k) * 2;
     auto apart = [&](fe_devptr_t p, size_t bytes) { return p + bytes <= x || p >= xe; };
     return apart(y, ((size_t)(m - 1) * ldy + l->n) * 2) && apart(ws->codes.p, ws->codes.bytes) && apart(ws->sf.p, ws->sf.bytes) && apart(ws->aq.p, ws->aq.bytes);

@@ -870,8 +870,9 @@ FP4_GEMV_KERNEL(3)  // (four groups of rows would not fit the registers of two p
 
 // ---- GEMV over programs of 8 CO columns (1..16 rows): no hand-off, every operand straight into LDS ---------------------------------
 //
-// y[r][n] for r < m <= 2 XP. grid ceil(N / 8 CO), 256 threads: a program takes 8 CO weight rows over all of K, its four wavefronts a
-// quarter of K's steps of 256 each (four k tiles); their sums are added in order. A row's bits depend on (k, W) only. K % 256 == 0.
+// y[r][n] for r < m <= 2 XP. grid ceil(N / 8 CO), 64 WV threads: a program takes 8 CO weight rows over all of K, its wavefronts (four or eight: wide_form of fe_fp4.cpp)
+// a quarter or an eighth of K's steps of 256 each (four k tiles). Sums of quarters are added in order; where wide_form sums eighths (EIGHTHS: all forms of such a linear
+// alike), two of them make a quarter. A row's bits depend on W's shape and values only. K % 256 == 0.
 // Lane L = 16 g + r multiplies, for 16 weight rows, row r's k tile 4 s + g (64 codes, four block scales) with the activations of the
 // same k; the order of k inside a step does not matter.
 // Stages belong to one wavefront (no barrier in the loop). Codes: 8 weight rows a load, [4 k tiles][8 rows][32 bytes]; lanes of
@@ -882,7 +883,8 @@ FP4_GEMV_KERNEL(3)  // (four groups of rows would not fit the registers of two p
 // staged whole (one and two rows: too many programs, each waiting for its own staging) and, up to 16 rows, weight tiles cut
 // along K (whose partial sums meet through memory; 17 rows and more still run there). us with the quantizer's launch, before -> now:
 // 5120 x 34816 at 1 / 4 / 8 / 16 rows 25.6 -> 22.1, 32.2 -> 22.1, 32.4 -> 25.7, 34.4 -> 28.8; 17408 x 5120 19.0 -> 14.3, 17.8 -> 14.9,
-// 18.0 -> 18.4, 19.3 -> 20.7; 5120 x 5120 9.6 -> 9.0, 10.3 -> 9.0, 12.2 -> 9.1, 12.5 -> 10.1.
+// 18.0 -> 18.4, 19.3 -> 20.7; 5120 x 5120 9.6 -> 9.0, 10.3 -> 9.0, 12.2 -> 9.1, 12.5 -> 10.1 (four wavefronts). Eight wavefronts against four: wide_form. Deeper
+// stages in place of more wavefronts lose: 5120 x 17408 at 1 row 17.3 -> 18.8 with eight steps in flight for three.
 //
 // Q: the program quantizes the activations itself, in front of its first step. aq is then bf16 rows [m][ldx]: a wavefront moves its quarter of K into LDS as
 // it is, in front of the first weights, makes fe_fp4_quant's values of it in their places (a block of 16 a lane) while the weights are on their way, and every
@@ -894,21 +896,21 @@ struct Fp4QuantTo {
     uint32_t ldx;
     float g;
 };
-template <int XP, int CO, bool Q>
+template <int XP, int CO, bool Q, int WV>
 struct Fp4Wide {
     static constexpr int CG = (CO + 1) / 2, XL = Q ? 0 : XP, L = CO + CG + XL;
     static constexpr int SC_AT = CO * 1024, X_AT = SC_AT + CG * 256, STAGE = X_AT + XL * 1024;
-    static constexpr int FIT = (Q ? 15 : 20) * 1024 / STAGE, DEPTH = FIT < 2 ? 2 : FIT < 6 ? FIT : 6;  // two programs a CU where two steps allow it
-    static constexpr int RED = 4 * 16 * (16 * CG + 4) * 4, LDS = 4 * DEPTH * STAGE > RED ? 4 * DEPTH * STAGE : RED;
+    static constexpr int FIT = (Q ? 60 : 80) * 1024 / (WV * STAGE), DEPTH = FIT < 2 ? 2 : FIT < 6 ? FIT : 6;  // two programs a CU where two steps allow it
+    static constexpr int RED = WV * 16 * (16 * CG + 4) * 4, LDS = WV * DEPTH * STAGE > RED ? WV * DEPTH * STAGE : RED;
     static_assert(DEPTH >= 2 && (DEPTH - 1) * L < (Q ? 48 : 64) && LDS <= 160 * 1024, "stages");
 };
 
-template <int XP, int CO, bool Q>
+template <int XP, int CO, bool Q, int WV, bool EIGHTHS>
 __device__ __forceinline__ void gemv_nvfp4_wide_body(uint16_t* c, const _Float16* aq, const uint8_t* w, const uint8_t* sw,
                                                      const float* alpha, const uint16_t* res, uint32_t m, uint32_t n, uint32_t k,
                                                      uint32_t ldc, uint32_t w_snt, uint32_t w_skt, uint32_t w_sr, uint32_t s_snt,
                                                      uint32_t s_skt, uint32_t s_sr, const Fp4QuantTo qt) {
-    typedef Fp4Wide<XP, CO, Q> C;
+    typedef Fp4Wide<XP, CO, Q, WV> C;
     constexpr int CG = C::CG, AHEAD = C::DEPTH - 1, PITCH = 16 * CG + 4;
     extern __shared__ __attribute__((aligned(1024))) unsigned char lds[];
     const uint32_t tid = threadIdx.x, lane = tid & 63, wave = __builtin_amdgcn_readfirstlane(tid >> 6), r = lane & 15, g = lane >> 4;
@@ -932,7 +934,9 @@ __device__ __forceinline__ void gemv_nvfp4_wide_body(uint16_t* c, const _Float16
     }
     unsigned char* stages = lds + wave * (C::DEPTH * C::STAGE);
     const uint32_t stages0 = g8_lds_addr(stages);
-    const uint32_t steps = k / 256, s0 = wave * steps / 4, count = (wave + 1) * steps / 4 - s0;
+    // EIGHTHS with four wavefronts: two eighths each, steps up to mid and from mid on, summed apart
+    constexpr bool TWO = EIGHTHS && WV == 4;
+    const uint32_t steps = k / 256, s0 = wave * steps / WV, count = (wave + 1) * steps / WV - s0, mid = TWO ? (2 * wave + 1) * steps / 8 - s0 : 0;
     auto issue = [&](uint32_t s, uint32_t slot) {
         const uint32_t to = stages0 + slot * C::STAGE;
 #pragma unroll
@@ -944,7 +948,7 @@ __device__ __forceinline__ void gemv_nvfp4_wide_body(uint16_t* c, const _Float16
     };
     const uint32_t odd = g & 1, xr = r < m ? r : m - 1;
     // Q: the wavefront's activations, [its steps][m rows][512 bytes] (a whole number of loads), chunks placed as in a stage
-    unsigned char* xq = lds + 4 * C::DEPTH * C::STAGE + wave * (((steps + 3) / 4 * m + 1) / 2 * 1024);
+    unsigned char* xq = lds + WV * C::DEPTH * C::STAGE + wave * (((steps + WV - 1) / WV * m + 1) / 2 * 1024);
     // half h of the lane's row and k tile; the 16-byte chunk of 8 activations that goes with code 32 (h ^ odd) + 8 e on
     uint32_t fw[CG], fx[8];
 #pragma unroll
@@ -959,7 +963,11 @@ __device__ __forceinline__ void gemv_nvfp4_wide_body(uint16_t* c, const _Float16
             const uint32_t chunk = 8 * g + 4 * (h ^ odd) + e;
             fx[4 * h + e] = (Q ? 0 : C::X_AT) + xr * 512 + (((chunk & 16) | ((chunk ^ xr) & 15)) << 4);
         }
-    f32x4 acc[CG] = {};
+    f32x4 acc[CG] = {}, low[CG] = {};
+    auto half = [&]() {
+#pragma unroll
+        for (int j = 0; j < CG; j++) low[j] = acc[j], acc[j] = f32x4{};
+    };
     uint32_t slot = 0;
     auto add = [&](uint32_t s) {
         const unsigned char *st = stages + slot * C::STAGE, *xst = Q ? xq + s * (m * 512) : st;
@@ -1007,7 +1015,16 @@ __device__ __forceinline__ void gemv_nvfp4_wide_body(uint16_t* c, const _Float16
             asm volatile("" ::: "memory");
         }
         uint32_t s = 0;
+        if constexpr (TWO && AHEAD == 1) {  // (with the sums taken apart inside one loop they would move between register files every step)
+            for (; s < mid; s++) {
+                g8_loads_wait<0>();
+                issue(s + 1, slot ? 0 : 1);  // (mid < count)
+                add(s);
+            }
+            half();
+        }
         for (; s + AHEAD < count; s++) {
+            if (TWO && AHEAD > 1 && s == mid) half();
             g8_loads_wait<(AHEAD - 1) * C::L>();  // (the stage in front of this one has been read, too)
             issue(s + AHEAD, slot ? slot - 1 : AHEAD);
             add(s);
@@ -1016,6 +1033,7 @@ __device__ __forceinline__ void gemv_nvfp4_wide_body(uint16_t* c, const _Float16
             constexpr int U = decltype(u_tag)::value;
             if constexpr (U < AHEAD)
                 if (s + U < count) {
+                    if (TWO && AHEAD > 1 && s + U == mid) half();
                     g8_loads_wait<(AHEAD - 1 - U) * C::L>();
                     add(s + U);
                 }
@@ -1030,34 +1048,36 @@ __device__ __forceinline__ void gemv_nvfp4_wide_body(uint16_t* c, const _Float16
     float(*red)[16][PITCH] = (float(*)[16][PITCH])lds;
     __syncthreads();
 #pragma unroll
-    for (int j = 0; j < CG; j++) *(f32x4*)&red[wave][r][16 * j + 4 * g] = acc[j];
+    for (int j = 0; j < CG; j++) *(f32x4*)&red[wave][r][16 * j + 4 * g] = TWO ? low[j] + acc[j] : acc[j];
     __syncthreads();
-    for (uint32_t i = tid; i < m * 2 * CO; i += 256) {
+    for (uint32_t i = tid; i < m * 2 * CO; i += 64 * WV) {
         const uint32_t row = i / (2 * CO), j = 4 * (i % (2 * CO)), col = col0 + j;
         if (col >= n) continue;
-        const f32x4 sum = ((*(const f32x4*)&red[0][row][j] + *(const f32x4*)&red[1][row][j]) + *(const f32x4*)&red[2][row][j]) +
-                          *(const f32x4*)&red[3][row][j];
+        auto quarter = [&](int p) { return WV == 8 ? *(const f32x4*)&red[2 * p][row][j] + *(const f32x4*)&red[2 * p + 1][row][j] : *(const f32x4*)&red[p][row][j]; };
+        const f32x4 sum = ((quarter(0) + quarter(1)) + quarter(2)) + quarter(3);
         const float v[4] = {sum[0], sum[1], sum[2], sum[3]};
         fp4_store4(c, res, (size_t)row * ldc + col, v, *(const f32x4*)(alpha + col) * FP4_GEMM_SCALE);
     }
 }
 
-#define FP4_WIDE_KERNEL(XP, CO)                                                                                           \
-    extern "C" __global__ __launch_bounds__(256) void fe_gemv_nvfp4_r##XP##_c##CO(                                        \
+#define FP4_WIDE_KERNEL(XP, CO, SUFFIX, WV, EIGHTHS)                                                                      \
+    extern "C" __global__ __launch_bounds__(64 * WV) void fe_gemv_nvfp4_r##XP##_c##CO##SUFFIX(                            \
         uint16_t* c, const _Float16* aq, const uint8_t* w, const uint8_t* sw, const float* alpha, const uint16_t* res,   \
         uint32_t m, uint32_t n, uint32_t k, uint32_t ldc, uint32_t w_snt, uint32_t w_skt, uint32_t w_sr, uint32_t s_snt, \
         uint32_t s_skt, uint32_t s_sr) {                                                                                  \
-        gemv_nvfp4_wide_body<XP, CO, false>(c, aq, w, sw, alpha, res, m, n, k, ldc, w_snt, w_skt, w_sr, s_snt, s_skt, s_sr, Fp4QuantTo{}); \
+        gemv_nvfp4_wide_body<XP, CO, false, WV, EIGHTHS>(c, aq, w, sw, alpha, res, m, n, k, ldc, w_snt, w_skt, w_sr, s_snt, s_skt, s_sr, Fp4QuantTo{}); \
     }
-#define FP4_WIDE_QUANT_KERNEL(XP, CO)                                                                                     \
-    extern "C" __global__ __launch_bounds__(256) void fe_gemv_nvfp4_q##XP##_c##CO(                                        \
+#define FP4_WIDE_QUANT_KERNEL(XP, CO, SUFFIX, WV, EIGHTHS)                                                                \
+    extern "C" __global__ __launch_bounds__(64 * WV) void fe_gemv_nvfp4_q##XP##_c##CO##SUFFIX(                            \
         uint16_t* c, const _Float16* x, const uint8_t* w, const uint8_t* sw, const float* alpha, const uint16_t* res,    \
         uint32_t m, uint32_t n, uint32_t k, uint32_t ldc, uint32_t w_snt, uint32_t w_skt, uint32_t w_sr, uint32_t s_snt, \
         uint32_t s_skt, uint32_t s_sr, Fp4QuantTo qt) {                                                                   \
-        gemv_nvfp4_wide_body<XP, CO, true>(c, x, w, sw, alpha, res, m, n, k, ldc, w_snt, w_skt, w_sr, s_snt, s_skt, s_sr, qt); \
+        gemv_nvfp4_wide_body<XP, CO, true, WV, EIGHTHS>(c, x, w, sw, alpha, res, m, n, k, ldc, w_snt, w_skt, w_sr, s_snt, s_skt, s_sr, qt); \
     }
-#define FP4_WIDE_FAMILY(KERNEL, XP) \
-    KERNEL(XP, 1) KERNEL(XP, 2) KERNEL(XP, 3) KERNEL(XP, 4) KERNEL(XP, 5) KERNEL(XP, 6) KERNEL(XP, 9)
+// "": quarters of K. "_e": eighths, by eight wavefronts where two stages of eight fit the LDS, else by four.
+#define FP4_WIDE_SIX(KERNEL, XP, SUFFIX, WV, EIGHTHS) \
+    KERNEL(XP, 1, SUFFIX, WV, EIGHTHS) KERNEL(XP, 2, SUFFIX, WV, EIGHTHS) KERNEL(XP, 3, SUFFIX, WV, EIGHTHS) KERNEL(XP, 4, SUFFIX, WV, EIGHTHS) KERNEL(XP, 5, SUFFIX, WV, EIGHTHS) KERNEL(XP, 6, SUFFIX, WV, EIGHTHS)
+#define FP4_WIDE_FAMILY(KERNEL, XP) FP4_WIDE_SIX(KERNEL, XP, , 4, false) KERNEL(XP, 9, , 4, false) KERNEL(XP, 9, _e, 4, true)
 FP4_WIDE_FAMILY(FP4_WIDE_KERNEL, 1)
 FP4_WIDE_FAMILY(FP4_WIDE_KERNEL, 2)
 FP4_WIDE_FAMILY(FP4_WIDE_KERNEL, 4)
@@ -1065,6 +1085,14 @@ FP4_WIDE_FAMILY(FP4_WIDE_KERNEL, 8)
 FP4_WIDE_FAMILY(FP4_WIDE_QUANT_KERNEL, 1)
 FP4_WIDE_FAMILY(FP4_WIDE_QUANT_KERNEL, 2)
 FP4_WIDE_FAMILY(FP4_WIDE_QUANT_KERNEL, 4)
+FP4_WIDE_SIX(FP4_WIDE_KERNEL, 1, _e, 8, true)
+FP4_WIDE_SIX(FP4_WIDE_KERNEL, 2, _e, 8, true)
+FP4_WIDE_KERNEL(4, 1, _e, 8, true) FP4_WIDE_KERNEL(4, 2, _e, 8, true) FP4_WIDE_KERNEL(4, 3, _e, 8, true) FP4_WIDE_KERNEL(4, 4, _e, 8, true)
+FP4_WIDE_KERNEL(4, 5, _e, 4, true) FP4_WIDE_KERNEL(4, 6, _e, 4, true)
+FP4_WIDE_SIX(FP4_WIDE_KERNEL, 8, _e, 4, true)
+FP4_WIDE_SIX(FP4_WIDE_QUANT_KERNEL, 1, _e, 8, true)
+FP4_WIDE_SIX(FP4_WIDE_QUANT_KERNEL, 2, _e, 8, true)
+FP4_WIDE_SIX(FP4_WIDE_QUANT_KERNEL, 4, _e, 8, true)
 
 // ---- matrix-unit peak probe ---------------------------------------------------------------------------------------------
 //
