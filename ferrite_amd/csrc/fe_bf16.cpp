@@ -31,7 +31,7 @@ struct fe_bf16_kernels {
     fe_module_t module = nullptr;
     fe_function_t gemm[kFeGemmForms] = {}, reduce[kFeGemmTiles] = {}, swiglu[kFeGemmForms] = {}, swiglu_reduce[kFeGemmTiles] = {};  // by form; by tile (fe_gemm_launch)
     fe_function_t interleave = nullptr;
-    fe_function_t gemv[5][7] = {};  // [kGemvRowForms][kGemvColForms]
+    fe_function_t gemv[5][7] = {}, gemv_swiglu[5][7] = {};  // [kGemvRowForms][kGemvColForms]
     uint32_t cus = 0;
     FeBuf part;
     // Switches, read from the environment once at load (fe_bf16_kernels_set_option changes them afterwards)
@@ -90,6 +90,23 @@ static int check(const char *fn, fe_devptr_t y, uint32_t ldy, fe_devptr_t x, uin
     return 0;
 }
 
+bool fe_bf16_gemv_swiglu_takes(const fe_bf16_kernels *kern, fe_devptr_t big, fe_devptr_t act, fe_devptr_t x, fe_devptr_t gate, fe_devptr_t up, uint32_t m, uint32_t inter,
+                               uint32_t k, uint32_t dec) {
+    if (!m || m > kGemvPass || (m > kSmallBatch && dec < m) || !inter || !k || inter % 8 || k % 256 || (uint64_t)m * k * 2 >= (1ull << 32)) return false;
+    if (check("", big, inter, x, k, gate, 0, inter, k) || check("", big, inter, x, k, up, 0, inter, k)) return false;
+    // programs that are done write act while others read x and the weights
+    const uint64_t bytes = (uint64_t)m * inter * 2, weights = (uint64_t)inter * k * 2;
+    auto apart = [&](fe_devptr_t p, uint64_t size) { return act + bytes <= p || p + size <= act; };
+    return kern && act % 4 == 0 && apart(x, (uint64_t)m * k * 2) && apart(gate, weights) && apart(up, weights);
+}
+
+int fe_bf16_gemv_swiglu(const fe_bf16_kernels *kern, fe_stream_t s, fe_devptr_t act, fe_devptr_t x, fe_devptr_t gate, fe_devptr_t up, uint32_t m, uint32_t inter, uint32_t k) {
+    const uint32_t form = m <= 8 ? 0 : (m + 15) / 16, xo = kGemvRowForms[form];
+    const uint32_t cols = gemv_cols(m, inter, k, xo, std::max(kern->cus, 1u), kern->nc), co = kGemvColForms[cols];
+    void *args[] = {&act, &x, &gate, &up, &m, &inter, &k, &k};
+    return fe_hip_launch(kern->gemv_swiglu[form][cols], (inter / 8 + co - 1) / co, 1, 1, 256, 1, 1, gemv_lds(xo, co), s, args);
+}
+
 extern "C" {
 
 int fe_bf16_kernels_load(fe_bf16_kernels **out) {
@@ -112,10 +129,13 @@ int fe_bf16_kernels_load(fe_bf16_kernels **out) {
         for (uint32_t j = 0; j < 7 && !c; j++) {
             const uint32_t xo = kGemvRowForms[i], co = kGemvColForms[j];
             if (!gemv_form(xo, co)) continue;
-            char nm[32];
-            snprintf(nm, sizeof nm, "fe_gemv_bf16_r%u_c%u", xo, co);
-            c = fe_hip_module_get_function(&k->gemv[i][j], k->module, nm);
-            if (!c) c = fe_hip_func_set_max_dyn_lds(k->gemv[i][j], gemv_lds(xo, co));
+            for (int pair = 0; pair < 2 && !c; pair++) {
+                char nm[40];
+                snprintf(nm, sizeof nm, "fe_gemv_bf16%s_r%u_c%u", pair ? "_swiglu" : "", xo, co);
+                fe_function_t &f = (pair ? k->gemv_swiglu : k->gemv)[i][j];
+                c = fe_hip_module_get_function(&f, k->module, nm);
+                if (!c) c = fe_hip_func_set_max_dyn_lds(f, gemv_lds(xo, co));
+            }
         }
     int cus = 0;
     if (!c) c = fe_hip_cu_count(&cus);

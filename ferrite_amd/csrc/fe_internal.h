@@ -488,3 +488,11 @@ int fe_gemm_launch(const FeGemmPlan &p, Gemm gemm, Reduce reduce) {
         FE_TRY(reduce(p.tile, p.big.split.cut() * reduce_grid, p.big.split.full, p.big.split.splits));
     return 0;
 }
+
+// ---- gate, up and SwiGLU of decode rows over plain bf16 weights (fe_bf16.cpp) ---------------------------------------------------
+// Whether fe_bf16_gemv_swiglu does what two fe_bf16_linear_forward into big ([m][inter] each) and fe_route_silu_mul into act do: all rows go through the GEMV in one pass,
+// the operands are what those take, and act lies apart from what other programs still read. (Two launches less: see gemv_bf16_body for both sides.)
+struct fe_bf16_kernels;
+bool fe_bf16_gemv_swiglu_takes(const fe_bf16_kernels *kern, fe_devptr_t big, fe_devptr_t act, fe_devptr_t x, fe_devptr_t gate, fe_devptr_t up, uint32_t m, uint32_t inter,
+                               uint32_t k, uint32_t dec);
+int fe_bf16_gemv_swiglu(const fe_bf16_kernels *kern, fe_stream_t s, fe_devptr_t act, fe_devptr_t x, fe_devptr_t gate, fe_devptr_t up, uint32_t m, uint32_t inter, uint32_t k);

@@ -401,6 +401,18 @@ int fe_route_mlp_forward_w(const fe_route_ctx *c, const fe_route_proj *gate_up, 
             return fe_exl3_mlp_forward(g->q, u->q, down->q, c->xk, c->s, xn, FE_DTYPE_BF16, big, big + (size_t)n_rest * inter * 2, x,
                                        FE_DTYPE_BF16_ADD, n_rest, c->xws);
     }
+    if (n_rest > 0 && gate_up->lins.size() == 2 && !(gate_up->prompt && c->fp4() && n_rest > FE_X3_ROWS) && c->bk) {
+        // decode rows through plain bf16 gate and up, each one part: one launch for both and SwiGLU (the bits of the launches below; big is not written)
+        const fe_route_linear *g = gate_up->lins[0].first, *u = gate_up->lins[1].first;
+        auto plain = [&](const fe_route_linear *l, size_t parts) {
+            return l->w && !(l->q && c->x3()) && !(l->p && c->fp4()) && l->k == hidden && l->n == inter && parts == 1;
+        };
+        if (plain(g, gate_up->lins[0].second.size()) && plain(u, gate_up->lins[1].second.size()) &&
+            fe_bf16_gemv_swiglu_takes(c->bk, big, act, xn, g->w, u->w, n_rest, inter, hidden, d) && !(down->q && c->x3())) {
+            FE_TRY(fe_bf16_gemv_swiglu(c->bk, c->s, act, xn, g->w, u->w, n_rest, inter, hidden));
+            return linear_forward(down, c, d, x, hidden, act, inter, n_rest, x);
+        }
+    }
     if (n_rest > 0) {
         fe_devptr_t ptr[8] = {};
         uint32_t ld[8] = {};
