@@ -34,7 +34,7 @@ constexpr uint32_t kTileM = 256;                        // GM_BM
 
 struct fe_fp4_kernels {
     fe_module_t module = nullptr;
-    fe_function_t quant4 = nullptr, gemv4[3] = {nullptr, nullptr, nullptr};
+    fe_function_t quant4 = nullptr, gemv4[2][3] = {};  // gemv4: [weight tiles, rows as they lie][rows / 16]
     // by form (256 x 256, stream-K, 128 x 256, 128 x 128) and by tile (fe_gemm_launch); gemm8: the fp16 form, 256 x 256 only
     fe_function_t gemm4[kFeGemmForms] = {}, swiglu4[kFeGemmForms] = {}, gemm8c[kFeGemmForms] = {}, gemm8[2] = {};
     fe_function_t reduce4[kFeGemmTiles] = {}, swiglu_reduce4[kFeGemmTiles] = {}, reduce8c[kFeGemmTiles] = {};
@@ -45,7 +45,7 @@ struct fe_fp4_kernels {
     // Switches of the launch paths: read from the environment once, at load; fe_fp4_kernels_set_option changes them
     // afterwards. No forward call reads the environment.
     uint32_t group_m = 8;      // raster group height in row tiles; 0 = all (FE_FP4_GROUP, lib.rs:31-32, 68)
-    uint32_t gemv = 1;         // up to 64 rows run the GEMV (FE_FP4_NO_GEMV=1: the GEMM's single tile row)
+    uint32_t gemv = 1;         // few rows run the GEMV (takes_gemv; FE_FP4_NO_GEMV=1: the GEMM's single tile row)
     uint32_t gemv_sk = 0;      // K splits of the GEMV over weight tiles; 0 = two programs a CU (FE_FP4_GEMV_SK)
     uint32_t gemv_strips = 1;  // up to 16 rows run programs of some columns over all of K; 0: weight tiles and K splits, as more rows do (FE_FP4_NO_STRIPS=1)
     // most values (rows x k) that the four wavefronts of the GEMV for up to 16 rows quantize themselves, in every program; eight take twice as many (FE_FP4_GEMV_QUANT)
@@ -73,7 +73,7 @@ struct fe_fp4_workspace {
     FeBuf codes, sf, aq, part, counters;  // part: partial sums of the GEMM (one slot a CU) or of the GEMV's splits
 };
 constexpr uint32_t kGemvRows = 48;      // rows of one fe_gemv_nvfp4 pass (three groups of 16)
-constexpr uint32_t kGemvMaxRows = 64;   // up to here the GEMV runs (two passes above 48 rows); above, the GEMM
+constexpr uint32_t kGemvMaxRows = 64;   // up to here the GEMV may run (two passes above 48 rows: takes_gemv); above, the GEMM
 constexpr uint32_t kGemvCounters = 8192;  // arrival counters: weight tiles of 128 rows (n <= 1 M)
 
 extern "C" {
@@ -99,11 +99,7 @@ int fe_fp4_kernels_load(fe_fp4_kernels **out) {
         get(&k->swiglu_reduce4[i], std::string("fe_gemm_nvfp4_swiglu_reduce") + tile_sfx[i], 0);
         get(&k->reduce8c[i], std::string(i < 3 ? "fe_gemm_fp8_codes_reduce" : "fe_gemm_nvfp4_reduce") + tile_sfx[i], 0);  // (one layout of the lower tiles)
     }
-    for (int xr = 1; xr <= 3 && !c; xr++) {
-        char nm[32];
-        snprintf(nm, sizeof nm, "fe_gemv_nvfp4_x%d", xr);
-        c = fe_hip_module_get_function(&k->gemv4[xr - 1], k->module, nm);
-    }
+    for (int i = 0; i < 6; i++) get(&k->gemv4[i / 3][i % 3], "fe_gemv_nvfp4_x" + std::to_string(i % 3 + 1) + (i / 3 ? "_v" : ""), 0);
     for (uint32_t i = 0; i < 8; i++)
         for (uint32_t j = 0; j < 7; j++) {
             const uint32_t xp = kWideRowForms[i % 4];
@@ -407,6 +403,13 @@ static WideForm wide_form(const fe_fp4_linear *l, const fe_fp4_kernels *kern, ui
 static bool takes_wide(const fe_fp4_linear *l, const fe_fp4_kernels *kern, uint32_t m) {
     return !l->fp8 && m <= 16 && l->n / kTile <= kGemvCounters && kern->gemv && kern->gemv_strips && !kern->gemv_sk && l->k % 256 == 0;
 }
+// Whether m rows go through a GEMV: all of one pass. 49..64 rows take two, which the GEMM beats everywhere (us at 64 rows, two passes -> GEMM: 34816 x 5120 83 -> 63, 17408 x
+// 5120 41 -> 32, 5120 x 17408 43 -> 30, 5120 x 5120 27 -> 17.5, 2048 x 6144 27 -> 14; 48 rows in one pass 51, 26, 27, 17, 17 against 62, 31, 30, 17, 14); they stay where
+// the caller asked for weight tiles (gemv_strips 0: a row's bits the same at every count up to 64) or their K splits, and with operands that the GEMM does not reach.
+static bool takes_gemv(const fe_fp4_kernels *kern, uint32_t m, bool gemm_reaches) {
+    return m <= kGemvRows || (m <= kGemvMaxRows && (!kern->gemv_strips || kern->gemv_sk || !gemm_reaches));
+}
+
 // x: null, or the activations (bf16 rows of lda) which that GEMV quantizes itself
 static int linear_gemm(const fe_fp4_linear *l, const fe_fp4_kernels *kern, fe_stream_t s, const fe_fp4_workspace *ws, fe_devptr_t y, uint32_t ldy,
                        uint32_t m, fe_devptr_t res, fe_devptr_t x, uint32_t lda) {
@@ -416,7 +419,8 @@ static int linear_gemm(const fe_fp4_linear *l, const fe_fp4_kernels *kern, fe_st
     if (!y || ldy % 8 || y % 16 || (res && res % 16) || ldy < l->n)
         return fe_set_error(FE_ERR_ARG, "fe_fp4_linear_gemm", "gemm: y/res must be 16-byte aligned rows");
     uint32_t n = l->n, k = l->k;
-    if (!l->fp8 && m <= kGemvMaxRows && n / kTile <= kGemvCounters && kern->gemv) {
+    const bool gemm_reaches = (uint64_t)m * k * 2 < (1ull << 32) && (uint64_t)n * k < (1ull << 32);
+    if (!l->fp8 && takes_gemv(kern, m, gemm_reaches) && n / kTile <= kGemvCounters && kern->gemv) {
         // decode-sized: the weight-read-bound GEMV, up to 48 rows a pass. Two programs fit a CU: as many programs as run
         // at once, not more (a second round of short programs costs more than idle CUs in the first).
         const uint32_t nts = n / kTile, kts = k / 64;
@@ -444,12 +448,11 @@ static int linear_gemm(const fe_fp4_linear *l, const fe_fp4_kernels *kern, fe_st
             uint32_t rows = m - r0 < kGemvRows ? m - r0 : kGemvRows;
             fe_devptr_t yy = y + (size_t)r0 * ldy * 2, aq = ws->aq.p + (size_t)r0 * k * 2, rr = res ? res + (size_t)r0 * ldy * 2 : 0;
             void *args[] = {&yy, &aq, &w, &sw, &alpha, &rr, &z, &cnt, &rows, &n, &k, &ldy, &sk, &w_snt, &w_skt, &w_sr, &s_snt, &s_skt, &s_sr};
-            FE_TRY(fe_hip_launch(kern->gemv4[(rows + 15) / 16 - 1], nts * sk, 1, 1, 256, 1, 1, 0, s, args));
+            FE_TRY(fe_hip_launch(kern->gemv4[w_sr != 32][(rows + 15) / 16 - 1], nts * sk, 1, 1, 256, 1, 1, 0, s, args));
         }
         return 0;
     }
-    if ((uint64_t)m * k * 2 >= (1ull << 32) || (uint64_t)n * k >= (1ull << 32))
-        return fe_set_error(FE_ERR_UNSUPPORTED, "fe_fp4_linear_gemm", "operand of 4 GB or more");
+    if (!gemm_reaches) return fe_set_error(FE_ERR_UNSUPPORTED, "fe_fp4_linear_gemm", "operand of 4 GB or more");
     const uint32_t tiles_m = (m + kTileM - 1) / kTileM;
     uint32_t group = kern->group_m == 0 || kern->group_m > tiles_m ? tiles_m : kern->group_m;  // lib.rs:148-151
     // FP8 codes: the weights are the larger operand from n >= m on, and at the 8-bit instruction's rate their traffic

@@ -698,7 +698,9 @@ struct Fp4GemvStage {
 // lanes hold them); the last to arrive (counters[tile]) adds them in split order, finishes the tile and re-arms the
 // counter, so the result does not depend on timing. A row's sums do not depend on XR. Weight
 // addressing as in fe_gemm_nvfp4.
-template <int XR>
+// NT: non-temporal loads of the weights. Not of rows as they lie in a checkpoint (_v): a wavefront's piece of such a row is a quarter of its cache line, which the next
+// wavefronts then read again from memory: 34816 x 5120 at 32 rows 131 us with, 102 without; 17408 x 5120 51 -> 39. (Weight tiles: 41.6 with, 42.2 without.)
+template <int XR, bool NT>
 __device__ __forceinline__ void gemv_nvfp4_body(uint16_t* c, const _Float16* aq, const uint8_t* w, const uint8_t* sw,
                                                 const float* alpha, const uint16_t* res, float* z, uint32_t* counters,
                                                 uint32_t m, uint32_t n, uint32_t k, uint32_t ldc, uint32_t sk,
@@ -723,8 +725,10 @@ __device__ __forceinline__ void gemv_nvfp4_body(uint16_t* c, const _Float16* aq,
         const uint8_t* sk_ = sp + (size_t)kt * s_skt;
 #pragma unroll
         for (int rg = 0; rg < FP4_GEMV_RG; rg++) {
-            st.cw[rg] = __builtin_nontemporal_load((const u32x2*)(wk + (size_t)(16 * rg) * w_sr));
-            st.sc[rg] = __builtin_nontemporal_load((const uint32_t*)(sk_ + (size_t)(16 * rg) * s_sr));
+            const u32x2* cw = (const u32x2*)(wk + (size_t)(16 * rg) * w_sr);
+            const uint32_t* sc = (const uint32_t*)(sk_ + (size_t)(16 * rg) * s_sr);
+            st.cw[rg] = NT ? __builtin_nontemporal_load(cw) : *cw;
+            st.sc[rg] = NT ? __builtin_nontemporal_load(sc) : *sc;
         }
 #pragma unroll
         for (int xr = 0; xr < XR; xr++) {
@@ -856,17 +860,17 @@ __device__ __forceinline__ void gemv_nvfp4_body(uint16_t* c, const _Float16* aq,
     }
 }
 
-#define FP4_GEMV_KERNEL(XR)                                                                                            \
-    extern "C" __global__ __launch_bounds__(256, 2) void fe_gemv_nvfp4_x##XR(                                          \
+#define FP4_GEMV_KERNEL(XR, SUFFIX, NT)                                                                                \
+    extern "C" __global__ __launch_bounds__(256, 2) void fe_gemv_nvfp4_x##XR##SUFFIX(                                  \
         uint16_t* c, const _Float16* aq, const uint8_t* w, const uint8_t* sw, const float* alpha, const uint16_t* res, \
         float* z, uint32_t* counters, uint32_t m, uint32_t n, uint32_t k, uint32_t ldc, uint32_t sk, uint32_t w_snt,   \
         uint32_t w_skt, uint32_t w_sr, uint32_t s_snt, uint32_t s_skt, uint32_t s_sr) {                                \
-        gemv_nvfp4_body<XR>(c, aq, w, sw, alpha, res, z, counters, m, n, k, ldc, sk, w_snt, w_skt, w_sr, s_snt, s_skt, \
-                            s_sr);                                                                                     \
+        gemv_nvfp4_body<XR, NT>(c, aq, w, sw, alpha, res, z, counters, m, n, k, ldc, sk, w_snt, w_skt, w_sr, s_snt,    \
+                                s_skt, s_sr);                                                                          \
     }
-FP4_GEMV_KERNEL(1)
-FP4_GEMV_KERNEL(2)
-FP4_GEMV_KERNEL(3)  // (four groups of rows would not fit the registers of two programs a CU)
+FP4_GEMV_KERNEL(1, , true) FP4_GEMV_KERNEL(1, _v, false)
+FP4_GEMV_KERNEL(2, , true) FP4_GEMV_KERNEL(2, _v, false)
+FP4_GEMV_KERNEL(3, , true) FP4_GEMV_KERNEL(3, _v, false)  // (four groups of rows would not fit the registers of two programs a CU)
 
 // ---- GEMV over programs of 8 CO columns (1..16 rows): no hand-off, every operand straight into LDS ---------------------------------
 //
