@@ -34,7 +34,7 @@ constexpr uint32_t kTileM = 256;                        // GM_BM
 
 struct fe_fp4_kernels {
     fe_module_t module = nullptr;
-    fe_function_t quant4 = nullptr, gemv4[2][3] = {};  // gemv4: [weight tiles, rows as they lie][rows / 16]
+    fe_function_t quant4 = nullptr, gemv4[2][3] = {}, gemv_swiglu4[2][3] = {};  // the GEMVs: [weight tiles, rows as they lie][rows / 16]
     // by form (256 x 256, stream-K, 128 x 256, 128 x 128) and by tile (fe_gemm_launch); gemm8: the fp16 form, 256 x 256 only
     fe_function_t gemm4[kFeGemmForms] = {}, swiglu4[kFeGemmForms] = {}, gemm8c[kFeGemmForms] = {}, gemm8[2] = {};
     fe_function_t reduce4[kFeGemmTiles] = {}, swiglu_reduce4[kFeGemmTiles] = {}, reduce8c[kFeGemmTiles] = {};
@@ -99,7 +99,11 @@ int fe_fp4_kernels_load(fe_fp4_kernels **out) {
         get(&k->swiglu_reduce4[i], std::string("fe_gemm_nvfp4_swiglu_reduce") + tile_sfx[i], 0);
         get(&k->reduce8c[i], std::string(i < 3 ? "fe_gemm_fp8_codes_reduce" : "fe_gemm_nvfp4_reduce") + tile_sfx[i], 0);  // (one layout of the lower tiles)
     }
-    for (int i = 0; i < 6; i++) get(&k->gemv4[i / 3][i % 3], "fe_gemv_nvfp4_x" + std::to_string(i % 3 + 1) + (i / 3 ? "_v" : ""), 0);
+    for (int i = 0; i < 6; i++) {
+        const std::string form = "x" + std::to_string(i % 3 + 1) + (i / 3 ? "_v" : "");
+        get(&k->gemv4[i / 3][i % 3], "fe_gemv_nvfp4_" + form, 0);
+        get(&k->gemv_swiglu4[i / 3][i % 3], "fe_gemv_nvfp4_swiglu_" + form, 0);
+    }
     for (uint32_t i = 0; i < 8; i++)
         for (uint32_t j = 0; j < 7; j++) {
             const uint32_t xp = kWideRowForms[i % 4];
@@ -406,8 +410,21 @@ static bool takes_wide(const fe_fp4_linear *l, const fe_fp4_kernels *kern, uint3
 // Whether m rows go through a GEMV: all of one pass. 49..64 rows take two, which the GEMM beats everywhere (us at 64 rows, two passes -> GEMM: 34816 x 5120 83 -> 63, 17408 x
 // 5120 41 -> 32, 5120 x 17408 43 -> 30, 5120 x 5120 27 -> 17.5, 2048 x 6144 27 -> 14; 48 rows in one pass 51, 26, 27, 17, 17 against 62, 31, 30, 17, 14); they stay where
 // the caller asked for weight tiles (gemv_strips 0: a row's bits the same at every count up to 64) or their K splits, and with operands that the GEMM does not reach.
-static bool takes_gemv(const fe_fp4_kernels *kern, uint32_t m, bool gemm_reaches) {
-    return m <= kGemvRows || (m <= kGemvMaxRows && (!kern->gemv_strips || kern->gemv_sk || !gemm_reaches));
+// From 33 rows on so do narrow linears of middling depth, whose tiles are cut along K either way (us at 48 rows, GEMV -> GEMM: 4096 x 4096 16.7 -> 14.1, 2048 x 6144 17.1 ->
+// 13.7, 1024 x 5120 15.0 -> 11.3, 1024 x 2816 12.3 -> 10.1, 128 x 8192 14.4 -> 13.1; beyond the lines 5120 x 5120 16.8 -> 16.9, 7168 x 2048 13.0 -> 13.7, 1024 x 1024 9.1 ->
+// 9.9, 512 x 14336 17.0 -> 18.9).
+static bool takes_gemv(const fe_fp4_linear *l, const fe_fp4_kernels *kern, uint32_t m, bool gemm_reaches) {
+    if (l->fp8 || m > kGemvMaxRows || l->n / kTile > kGemvCounters || !kern->gemv) return false;
+    if (!kern->gemv_strips || kern->gemv_sk || !gemm_reaches) return true;
+    return m <= 32 || (m <= kGemvRows && (l->n > 4096 || l->k < 2048 || l->k > 8192));
+}
+
+// K splits of the GEMV over weight tiles. Two programs fit a CU: as many programs as run at once, not more (a second round of short programs costs more than idle CUs in
+// the first).
+static uint32_t gemv_splits(const fe_fp4_kernels *kern, const fe_fp4_workspace *ws, uint32_t n, uint32_t k) {
+    uint32_t sk = std::min({kern->gemv_sk ? kern->gemv_sk : 2 * kern->cus / (n / kTile), 16u, k / 64 / 4});
+    while (sk > 1 && (size_t)sk * kGemvRows * n * 4 > ws->part.bytes) sk--;
+    return std::max(sk, 1u);
 }
 
 // x: null, or the activations (bf16 rows of lda) which that GEMV quantizes itself
@@ -420,10 +437,9 @@ static int linear_gemm(const fe_fp4_linear *l, const fe_fp4_kernels *kern, fe_st
         return fe_set_error(FE_ERR_ARG, "fe_fp4_linear_gemm", "gemm: y/res must be 16-byte aligned rows");
     uint32_t n = l->n, k = l->k;
     const bool gemm_reaches = (uint64_t)m * k * 2 < (1ull << 32) && (uint64_t)n * k < (1ull << 32);
-    if (!l->fp8 && takes_gemv(kern, m, gemm_reaches) && n / kTile <= kGemvCounters && kern->gemv) {
-        // decode-sized: the weight-read-bound GEMV, up to 48 rows a pass. Two programs fit a CU: as many programs as run
-        // at once, not more (a second round of short programs costs more than idle CUs in the first).
-        const uint32_t nts = n / kTile, kts = k / 64;
+    if (takes_gemv(l, kern, m, gemm_reaches)) {
+        // decode-sized: the weight-read-bound GEMV, up to 48 rows a pass
+        const uint32_t nts = n / kTile;
         if (takes_wide(l, kern, m)) {
             const WideForm wf = wide_form(l, kern, m, x != 0);
             struct {  // Fp4QuantTo
@@ -436,12 +452,7 @@ static int linear_gemm(const fe_fp4_linear *l, const fe_fp4_kernels *kern, fe_st
             void *args[] = {&y, &aq, &w, &sw, &alpha, &res, &m, &n, &k, &ldy, &w_snt, &w_skt, &w_sr, &s_snt, &s_skt, &s_sr, &to};
             return fe_hip_launch(wf.f, wf.programs, 1, 1, 64 * wf.waves, 1, 1, wf.lds, s, args);
         }
-        uint32_t sk = 2 * kern->cus / nts;
-        if (kern->gemv_sk) sk = kern->gemv_sk;
-        if (sk > 16) sk = 16;
-        if (sk > kts / 4) sk = kts / 4;
-        while (sk > 1 && (size_t)sk * kGemvRows * n * 4 > ws->part.bytes) sk--;
-        if (sk < 1) sk = 1;
+        uint32_t sk = gemv_splits(kern, ws, n, k);
         fe_devptr_t w = l->w.p, sw = l->sw.p, alpha = l->alpha.p, z = ws->part.p, cnt = ws->counters.p;
         uint32_t w_snt = l->w_snt, w_skt = l->w_skt, w_sr = l->w_sr, s_snt = l->s_snt, s_skt = l->s_skt, s_sr = l->s_sr;
         for (uint32_t r0 = 0; r0 < m; r0 += kGemvRows) {
@@ -554,6 +565,12 @@ int fe_fp4_linear_forward_swiglu(const fe_fp4_linear *l, const fe_fp4_kernels *k
     fe_devptr_t q_codes = act->codes.p, q_sf = act->sf.p, q_aq = act->aq.p;
     uint32_t w_snt = l->w_snt, w_skt = l->w_skt, w_sr = l->w_sr, s_snt = l->s_snt, s_skt = l->s_skt, s_sr = l->s_sr;
     // (stream-K only when forced: this kernel's stream-K form was slower wherever measured, 688 -> 714 us on 5120 x 34816)
+    if (m <= kGemvRows && takes_gemv(l, kern, m, true) && !kern->tile.force_tile && kern->gemm_sk < 2) {
+        uint32_t sk = gemv_splits(kern, ws, n, k);
+        fe_devptr_t cnt = ws->counters.p;
+        void *args[] = {&aq, &w, &sw, &alpha, &part, &cnt, &m, &n, &k, &sk, &w_snt, &w_skt, &w_sr, &s_snt, &s_skt, &s_sr, &q_codes, &q_sf, &q_aq, &down_g};
+        return fe_hip_launch(kern->gemv_swiglu4[w_sr != 32][(m + 15) / 16 - 1], n / kTile * sk, 1, 1, 256, 1, 1, 0, s, args);
+    }
     const FeGemmPlan plan = fe_gemm_plan(m, n, k / 64, kern->cus, ws->part.p, ws->part.bytes, ws->counters.p, kGemvCounters, kern->gemm_splits,
                                          kern->gemm_sk >= 2 ? kern->gemm_sk : 0, true, kFeCostNvfp4, kern->tile);
     if (!plan.tile && plan.big.stream_k && kern->xcd < 0) group = 1;

@@ -700,10 +700,12 @@ struct Fp4GemvStage {
 // addressing as in fe_gemm_nvfp4.
 // NT: non-temporal loads of the weights. Not of rows as they lie in a checkpoint (_v): a wavefront's piece of such a row is a quarter of its cache line, which the next
 // wavefronts then read again from memory: 34816 x 5120 at 32 rows 131 us with, 102 without; 17408 x 5120 51 -> 39. (Weight tiles: 41.6 with, 42.2 without.)
-template <int XR, bool NT>
-__device__ __forceinline__ void gemv_nvfp4_body(uint16_t* c, const _Float16* aq, const uint8_t* w, const uint8_t* sw,
-                                                const float* alpha, const uint16_t* res, float* z, uint32_t* counters,
-                                                uint32_t m, uint32_t n, uint32_t k, uint32_t ldc, uint32_t sk,
+// SWIGLU: a fused gate|up linear, whose finished tile goes through LDS to swiglu_quant_store (out), a row a half wavefront. 34816 x 5120 at 17 / 32 / 48 rows 37 / 42 / 51 us
+// against 63 in the GEMM (takes_gemv of fe_fp4.cpp).
+template <int XR, bool NT, bool SWIGLU>
+__device__ __forceinline__ void gemv_nvfp4_body(const FpOut out, const _Float16* aq, const uint8_t* w, const uint8_t* sw,
+                                                const float* alpha, float* z, uint32_t* counters,
+                                                uint32_t m, uint32_t n, uint32_t k, uint32_t sk,
                                                 uint32_t w_snt, uint32_t w_skt, uint32_t w_sr, uint32_t s_snt,
                                                 uint32_t s_skt, uint32_t s_sr) {
     __shared__ f32x4 red[4][FP4_GEMV_RG][64];
@@ -799,12 +801,34 @@ __device__ __forceinline__ void gemv_nvfp4_body(uint16_t* c, const _Float16* aq,
         for (int h = 0; h < 2; h++) {
             uint32_t cc = col + 16 * h;
             float o[4] = {v[h][0], v[h][1], v[h][2], v[h][3]};
-            fp4_store4(c, res, (size_t)row * ldc + cc, o, *(const f32x4*)(alpha + cc) * FP4_OPERAND_SCALE);
+            fp4_store4(out.c, out.res, (size_t)row * out.ldc + cc, o, *(const f32x4*)(alpha + cc) * FP4_OPERAND_SCALE);
+        }
+    };
+    constexpr uint32_t PITCH = 132;
+    float* tile = (float*)red;  // SWIGLU: [16 XR][PITCH] of the finished tile
+    static_assert(sizeof(red) >= 16 * XR * PITCH * 4, "tile");
+    auto finish_tile = [&](const f32x4 (&v)[XR][2]) {
+#pragma unroll
+        for (int xr = 0; xr < XR; xr++)
+#pragma unroll
+            for (int h = 0; h < 2; h++) *(f32x4*)(tile + (16 * xr + r) * PITCH + 32 * wave + 16 * h + 4 * g) = v[xr][h];
+        __syncthreads();
+        const uint32_t l32 = tid & 31, at = nt * 128 + 4 * l32;
+        const f32x4 al = *(const f32x4*)(alpha + at) * FP4_OPERAND_SCALE;
+        for (uint32_t row = tid >> 5; row < 16 * XR; row += 8) {
+            const f32x4 p = *(const f32x4*)(tile + row * PITCH + 4 * l32);
+            const float o[4] = {p[0], p[1], p[2], p[3]};
+            swiglu_quant_store(o, al, l32, row < m, row < m ? row : 0, at, n, out.q_codes, out.q_sf, out.q_aq, out.qg);
         }
     };
     if (sk == 1) {
+        if constexpr (SWIGLU) {
+            __syncthreads();  // (the last group's sums have been read)
+            finish_tile(sum);
+        } else {
 #pragma unroll
-        for (int xr = 0; xr < XR; xr++) finish(16 * xr + r, sum[xr]);
+            for (int xr = 0; xr < XR; xr++) finish(16 * xr + r, sum[xr]);
+        }
         return;
     }
     // Partials cross to another program, possibly on another XCD with its own L2: agent-scope accesses, ordered by the
@@ -834,7 +858,10 @@ __device__ __forceinline__ void gemv_nvfp4_body(uint16_t* c, const _Float16* aq,
 #pragma unroll
     for (int xr = 0; xr < XR; xr++) {
         const uint32_t row = 16 * xr + r;
-        if (row >= m) continue;
+        if (row >= m) {
+            if constexpr (SWIGLU) sum[xr][0] = sum[xr][1] = f32x4{};
+            continue;
+        }
         f32x4 tot[2] = {{0.f, 0.f, 0.f, 0.f}, {0.f, 0.f, 0.f, 0.f}};
         for (uint32_t s0 = 0; s0 < sk; s0 += 8) {
             f32x4 t[16];
@@ -856,8 +883,12 @@ __device__ __forceinline__ void gemv_nvfp4_body(uint16_t* c, const _Float16* aq,
                     for (int h = 0; h < 2; h++) tot[h] += t[2 * b + h];
                 }
         }
-        finish(row, tot);
+        if constexpr (SWIGLU)
+            sum[xr][0] = tot[0], sum[xr][1] = tot[1];
+        else
+            finish(row, tot);
     }
+    if constexpr (SWIGLU) finish_tile(sum);  // (two barriers since red was read)
 }
 
 #define FP4_GEMV_KERNEL(XR, SUFFIX, NT)                                                                                \
@@ -865,8 +896,15 @@ __device__ __forceinline__ void gemv_nvfp4_body(uint16_t* c, const _Float16* aq,
         uint16_t* c, const _Float16* aq, const uint8_t* w, const uint8_t* sw, const float* alpha, const uint16_t* res, \
         float* z, uint32_t* counters, uint32_t m, uint32_t n, uint32_t k, uint32_t ldc, uint32_t sk, uint32_t w_snt,   \
         uint32_t w_skt, uint32_t w_sr, uint32_t s_snt, uint32_t s_skt, uint32_t s_sr) {                                \
-        gemv_nvfp4_body<XR, NT>(c, aq, w, sw, alpha, res, z, counters, m, n, k, ldc, sk, w_snt, w_skt, w_sr, s_snt,    \
-                                s_skt, s_sr);                                                                          \
+        gemv_nvfp4_body<XR, NT, false>(FpOut{c, res, ldc, nullptr, nullptr, nullptr, 0.f}, aq, w, sw, alpha, z, counters, m, n, k, sk, \
+                                       w_snt, w_skt, w_sr, s_snt, s_skt, s_sr);                                        \
+    }                                                                                                                  \
+    extern "C" __global__ __launch_bounds__(256, 2) void fe_gemv_nvfp4_swiglu_x##XR##SUFFIX(                           \
+        const _Float16* aq, const uint8_t* w, const uint8_t* sw, const float* alpha, float* z, uint32_t* counters,     \
+        uint32_t m, uint32_t n, uint32_t k, uint32_t sk, uint32_t w_snt, uint32_t w_skt, uint32_t w_sr, uint32_t s_snt, \
+        uint32_t s_skt, uint32_t s_sr, uint8_t* q_codes, uint8_t* q_sf, _Float16* q_aq, float qg) {                    \
+        gemv_nvfp4_body<XR, NT, true>(FpOut{nullptr, nullptr, 0, q_codes, q_sf, q_aq, qg}, aq, w, sw, alpha, z, counters, m, n, k, sk, \
+                                      w_snt, w_skt, w_sr, s_snt, s_skt, s_sr);                                         \
     }
 FP4_GEMV_KERNEL(1, , true) FP4_GEMV_KERNEL(1, _v, false)
 FP4_GEMV_KERNEL(2, , true) FP4_GEMV_KERNEL(2, _v, false)
