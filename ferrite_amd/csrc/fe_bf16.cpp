@@ -90,9 +90,18 @@ static int check(const char *fn, fe_devptr_t y, uint32_t ldy, fe_devptr_t x, uin
     return 0;
 }
 
+// Whether all of a call's rows go through the GEMV: a batch of decode rows, or one so small that the GEMV's one read of the weights is ahead of the GEMM's tiles. us at 17 /
+// 24 / 32 rows, GEMM -> GEMV: 17408 x 5120 40 -> 31, 31, 32; 34816 x 5120 77 -> 58, 79 -> 60, 81 -> 62; 5120 x 5120 17 -> 13, 15, 16; 5120 x 8704 24 -> 19, 21, 23;
+// 8192 x 2048 12.6 -> 8; 1024 x 2816 8.7 -> 5.4, 5.7, 6.1. The line in rows times K is the activations' way from L2 once a program: 4096 x 14336 27 -> 24, 26, 29; 5120 x 17408
+// 38 -> 36, 39, 44; a block of 5120 x 8704 at 32 rows 68 -> 70. From 33 rows on (three groups of 16) the GEMM is ahead wherever K is 5120 and more.
+static bool rows_take_gemv(uint32_t m, uint32_t k, uint32_t dec) { return m <= kSmallBatch || dec >= m || (m <= 32 && (uint64_t)m * k <= (m <= 24 ? 350000 : 180000)); }
+
 bool fe_bf16_gemv_swiglu_takes(const fe_bf16_kernels *kern, fe_devptr_t big, fe_devptr_t act, fe_devptr_t x, fe_devptr_t gate, fe_devptr_t up, uint32_t m, uint32_t inter,
                                uint32_t k, uint32_t dec) {
-    if (!m || m > kGemvPass || (m > kSmallBatch && dec < m) || !inter || !k || inter % 8 || k % 256 || (uint64_t)m * k * 2 >= (1ull << 32)) return false;
+    // (against the GEMM with SwiGLU, where the caller has its weights, wider programs have to carry the activations: a block of 32 rows, GEMM -> GEMV, us: 5120 x 17408 133 ->
+    // 106, 5120 x 12288 98 -> 84, 4096 x 8192 60 -> 48, but 5120 x 8704 68 -> 71; of 24 rows 66 -> 60)
+    if (m > kSmallBatch && dec < m && inter < 12288 && (uint64_t)m * k > 131072) return false;
+    if (!m || m > kGemvPass || !rows_take_gemv(m, k, dec) || !inter || !k || inter % 8 || k % 256 || (uint64_t)m * k * 2 >= (1ull << 32)) return false;
     if (check("", big, inter, x, k, gate, 0, inter, k) || check("", big, inter, x, k, up, 0, inter, k)) return false;
     // programs that are done write act while others read x and the weights
     const uint64_t bytes = (uint64_t)m * inter * 2, weights = (uint64_t)inter * k * 2;
@@ -269,7 +278,7 @@ int fe_bf16_linear_forward(const fe_bf16_kernels *kern, fe_stream_t s, fe_devptr
     if (m == 0) return 0;
     FE_TRY(check(fn, y, ldy, x, lda, w, res, n, k));
     // decode / verify rows: the GEMV, so that a row's bits do not depend on the batch
-    uint32_t d = m <= kSmallBatch ? m : (dec < m ? dec : m);
+    uint32_t d = rows_take_gemv(m, k, dec) ? m : dec;
     if (k % 256) d = 0;
     for (uint32_t r = 0; r < d; r += kGemvPass) {
         const uint32_t mr = d - r < kGemvPass ? d - r : kGemvPass;

@@ -86,7 +86,8 @@ int fe_route_copy2d(fe_stream_t s, fe_devptr_t dst, uint32_t ldd, fe_devptr_t sr
  * GEMM on the quantized activation with the residual in place. The other rows: gate_up, fe_silu_mul, down with the
  * residual; where all of them go through down's trellis linear in one call (a decode batch, or a prompt when down has
  * no other form), SwiGLU is applied as its input rotation reads gate and up (fe_exl3_linear_forward_swiglu: the same bits, act is not written). Up to 64
- * decode rows through plain bf16 gate and up, each one part, take one launch for both and SwiGLU (the same bits, big is not written).
+ * decode rows (and small batches, as fe_bf16_linear_forward takes them) through plain bf16 gate and up, each one part, take one launch for both and SwiGLU (the
+ * same bits, big is not written).
  * big: scratch for gate_up's outputs ([rows][total n]); act: scratch [rows][inter]. */
 int fe_route_mlp_forward(const fe_route_ctx *c, const fe_route_proj *gate_up, const fe_route_linear *down,
                          const fe_fp4_linear *swiglu, const fe_fp4_workspace *act_ws, fe_devptr_t x, fe_devptr_t xn,

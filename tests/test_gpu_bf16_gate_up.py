@@ -6,7 +6,7 @@ pytestmark = pytest.mark.gpu
 
 
 # One step a wavefront (fewer than stages in flight), fewer steps in all than stages, as many as stages, many; the last program partly past the columns; every row form and
-# width of a program; rows by their count and as decode rows
+# width of a program; rows by their count and as decode rows, prompt rows that are few enough and one more
 @pytest.mark.parametrize("hidden,inter", [(256, 320), (512, 1216), (1792, 576), (2048, 1344), (5120, 192)])
 def test_one_launch_gives_the_bits_of_three(hidden, inter):
     import torch
@@ -22,7 +22,7 @@ def test_one_launch_gives_the_bits_of_three(hidden, inter):
     ctx.set_bf16(kern)
     gate_up = route.Proj([(route.Linear("gate", inter, hidden, w=g), [inter]), (route.Linear("up", inter, hidden, w=u), [inter])])
     down = route.Linear("down", hidden, inter, w=dn)
-    for m, dec in ((1, 0), (2, 0), (8, 0), (9, 0), (16, 0), (17, 17), (33, 40), (48, 48), (64, 64), (65, 65), (20, 4)):
+    for m, dec in ((1, 0), (2, 0), (8, 0), (9, 0), (16, 0), (17, 17), (20, 0), (32, 0), (33, 0), (33, 40), (48, 48), (64, 64), (65, 65), (20, 4)):
         xn = rand(m, hidden)
         xn[0, 3], xn[m - 1, hidden - 1] = float("inf"), float("nan")
         big, act = rand(m, 2 * inter), torch.zeros((m, inter), dtype=torch.bfloat16, device="cuda")
