@@ -331,7 +331,13 @@ inline FeGemmPlan fe_gemm_plan(uint32_t m, uint32_t n, uint32_t ktiles, uint32_t
                                fe_devptr_t counters, size_t counters_len, uint32_t cap, int mode, bool small_b,
                                const FeGemmCost &cost, const FeGemmTileOptions &opt) {
     FeGemmPlan p;
-    p.big = fe_gemm_schedule(((m + 255) / 256) * ((n + 255) / 256), ktiles, cus, part, part_bytes, counters, counters_len, cap, mode, small_b);
+    // Stream-K of the forms that have lower tiles, up to 2048 rows: only with fewer tiles than CUs. Behind or over whole rounds, rows that do not exist, the reduce launch and
+    // lower tiles cost the one-piece schedule less than the runs' meetings cost (NVFP4, us, stream-K -> one piece: 34816 x 5120 at 400 / 777 / 2048 rows 144 -> 130, 267 -> 242,
+    // 531 -> 521; 17408 x 5120 at 777 / 1800 138 -> 130, 273 -> 257; 16384 x 4096 at 1500 182 -> 154; at most 2 % the other way: 12288 x 2048 at 1500 69.0 -> 70.6). With
+    // fewer: 34816 x 5120 at 200 rows 94 against 102, 5120 x 17408 at 2048 265 against 277.
+    const uint32_t tiles256 = ((m + 255) / 256) * ((n + 255) / 256);
+    if (mode == 1 && opt.low && m <= 2048 && tiles256 > cus) mode = 0;
+    p.big = fe_gemm_schedule(tiles256, ktiles, cus, part, part_bytes, counters, counters_len, cap, mode, small_b);
     auto take = [&](uint32_t tile, uint32_t tiles, uint32_t pieces) { p.tile = tile, p.tiles = tiles, p.splits = pieces; };
     auto tiles_of = [&](uint32_t tile) {
         return ((m + kFeGemmTileM[tile] - 1) / kFeGemmTileM[tile]) * ((n + kFeGemmTileN[tile] - 1) / kFeGemmTileN[tile]);
