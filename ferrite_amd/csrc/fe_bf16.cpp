@@ -17,13 +17,6 @@ constexpr uint32_t kGemmThreads = 512;
 constexpr uint32_t kTileM = 256;                         // rows of the largest output tile
 constexpr uint32_t kGemvRows = 8;                        // rows of one fe_bf16_gemv call (model.rs:326)
 constexpr uint32_t kGemvPass = 64;                       // rows of one pass over the weights
-// The GEMV's forms: rows / 8, and columns / 8 of a program (those whose stages fit LDS)
-constexpr uint32_t kGemvRowForms[5] = {1, 2, 4, 6, 8}, kGemvColForms[7] = {1, 2, 3, 4, 5, 6, 9};
-constexpr bool gemv_form(uint32_t xo, uint32_t co) { return 12 * (co + xo) <= 160; }
-// Bf16Gemv<XO, CO>::LDS of k_bf16.hip
-uint32_t gemv_lds(uint32_t xo, uint32_t co) {
-    return 4 * std::max(3u, std::min(20 / (co + xo), 8u)) * (co + xo) * 1024;
-}
 constexpr uint32_t kSmallBatch = 16;                     // X3_ROWS: batches up to here are decode rows (model.rs:172)
 }  // namespace
 
@@ -40,33 +33,6 @@ struct fe_bf16_kernels {
     uint32_t gemm_splits = 8;  // most pieces a cut output tile takes (FE_GEMM_SPLITS; 1: never cut)
     FeGemmTileOptions tile{0, 0, true};  // "gemm_tile", "gemm_pieces"
 };
-
-// Which of kGemvColForms a GEMV takes. Time goes by the CU with the most columns, so the form is the one with the least of
-// rounds of one program a CU times a program's loads (columns, and half the weight for the x rows, which come from L2). us, 5120
-// columns of 17408 at 1 / 16 rows (640 octets of columns on 256 CUs): 2 octets 33.8 / 47.9, 3 octets 27.1 / 33.7, 4 octets
-// 30.0 / 39.4; 8704 columns of 5120 at 1 / 64 rows: 4 octets 20.9 / 43, 5 octets 15.2 / 27. With one or two rows a linear
-// of several octets a CU is better off with programs that start while others run: 17408 columns 27.1 us at 3 octets, 27.7 at 9.
-// (One and two rows as dot products on the vector ALUs would be up to 0.4 us faster at some widths: 5120 columns of 5120 9.7 / 10.1 us against
-// 10.0 / 10.2, 1024 of 5120 3.9 / 4.1 against 4.3 / 4.5; but a row's bits may not depend on the batch, and from three rows on the matrix
-// instruction is far ahead.)
-static uint32_t gemv_cols(uint32_t m, uint32_t n, uint32_t k, uint32_t xo, uint32_t cus, int32_t nc) {
-    const uint32_t octets = n / 8;
-    uint32_t best = 0;
-    uint64_t least = ~0ull;
-    for (uint32_t i = 0; i < 7; i++) {
-        const uint32_t co = kGemvColForms[i];
-        if (i && (!gemv_form(xo, co) || 16ull * co * k >= (1ull << 32))) break;
-        if (nc > 0) {
-            best = i;
-            if (8 * co >= (uint32_t)nc) break;
-            continue;
-        }
-        const uint64_t rounds = (octets + co * cus - 1) / (co * cus), cost = rounds * (2 * co + xo);
-        if (cost <= least) best = i, least = cost;
-    }
-    if (nc <= 0 && m <= 2 && best > 4) best = 2;
-    return best;
-}
 
 // Raster of the GEMM's output tiles (gemm_raster). Weights at least as large as the activations: column tiles are dealt
 // to the XCDs (group 0), each weight panel through one L2, the smaller activations through all of them; else row tiles
@@ -110,7 +76,7 @@ bool fe_bf16_gemv_swiglu_takes(const fe_bf16_kernels *kern, fe_devptr_t big, fe_
 }
 
 int fe_bf16_gemv_swiglu(const fe_bf16_kernels *kern, fe_stream_t s, fe_devptr_t act, fe_devptr_t x, fe_devptr_t gate, fe_devptr_t up, uint32_t m, uint32_t inter, uint32_t k) {
-    const uint32_t form = m <= 8 ? 0 : (m + 15) / 16, xo = kGemvRowForms[form];
+    const uint32_t form = gemv_row_form(m), xo = kGemvRowForms[form];
     const uint32_t cols = gemv_cols(m, inter, k, xo, std::max(kern->cus, 1u), kern->nc), co = kGemvColForms[cols];
     void *args[] = {&act, &x, &gate, &up, &m, &inter, &k, &k};
     return fe_hip_launch(kern->gemv_swiglu[form][cols], (inter / 8 + co - 1) / co, 1, 1, 256, 1, 1, gemv_lds(xo, co), s, args);
@@ -189,7 +155,7 @@ static int launch_gemv(const fe_bf16_kernels *kern, fe_stream_t s, fe_devptr_t y
             FE_TRY(launch_gemv(kern, s, y + (size_t)r * ldy * 2, ldy, x + (size_t)r * lda * 2, lda, w, res ? res + (size_t)r * ldy * 2 : 0, 1, n, k));
         return 0;
     }
-    const uint32_t form = m <= 8 ? 0 : (m + 15) / 16, xo = kGemvRowForms[form];
+    const uint32_t form = gemv_row_form(m), xo = kGemvRowForms[form];
     const uint32_t cols = gemv_cols(m, n, k, xo, std::max(kern->cus, 1u), kern->nc), co = kGemvColForms[cols];
     void *args[] = {&y, &x, &w, &res, &m, &n, &k, &lda, &ldy};
     return fe_hip_launch(kern->gemv[form][cols], (n / 8 + co - 1) / co, 1, 1, 256, 1, 1, gemv_lds(xo, co), s, args);

@@ -40,17 +40,18 @@ struct fe_fp4_kernels {
     fe_function_t reduce4[kFeGemmTiles] = {}, swiglu_reduce4[kFeGemmTiles] = {}, reduce8c[kFeGemmTiles] = {};
     fe_function_t wide[2][4][7] = {};    // the GEMV over programs of 8 CO columns, [quarters or eighths of K][kWideRowForms][kWideColForms]
     fe_function_t wide_q[2][3][7] = {};  // the same, quantizing its activations itself
+    fe_function_t gemv8[5][7] = {};  // the FP8 GEMV, [kGemvRowForms][kGemvColForms]
     fe_function_t quant8 = nullptr, expand8 = nullptr;
     uint32_t cus = 0;
     // Switches of the launch paths: read from the environment once, at load; fe_fp4_kernels_set_option changes them
     // afterwards. No forward call reads the environment.
     uint32_t group_m = 8;      // raster group height in row tiles; 0 = all (FE_FP4_GROUP, lib.rs:31-32, 68)
-    uint32_t gemv = 1;         // few rows run the GEMV (takes_gemv; FE_FP4_NO_GEMV=1: the GEMM's single tile row)
+    uint32_t gemv = 1;         // few rows run the GEMV (takes_gemv, fp8_gemv_rows; FE_FP4_NO_GEMV=1: the GEMM's single tile row)
     uint32_t gemv_sk = 0;      // K splits of the GEMV over weight tiles; 0 = two programs a CU (FE_FP4_GEMV_SK)
     uint32_t gemv_strips = 1;  // up to 16 rows run programs of some columns over all of K; 0: weight tiles and K splits, as more rows do (FE_FP4_NO_STRIPS=1)
     // most values (rows x k) that the four wavefronts of the GEMV for up to 16 rows quantize themselves, in every program; eight take twice as many (FE_FP4_GEMV_QUANT)
     uint32_t gemv_quant = 10240;
-    uint32_t gemv_cols = 0;    // columns a program of the GEMV for up to 16 rows takes, rounded up to 8, 16, .. 48, 72; 0 = by the shape (FE_FP4_GEMV_COLS)
+    uint32_t gemv_cols = 0;    // columns a program of the GEMV for up to 16 rows, or of the FP8 GEMV, takes, rounded up to 8, 16, .. 48, 72; 0 = by the shape (FE_FP4_GEMV_COLS)
     int32_t xcd = -1;          // column tiles dealt to the XCDs: -1 = where the weights are the larger operand (FE_FP4_XCD)
     uint32_t fp8_f16 = 0;      // FP8 linears as fp16 expansion on the 16-bit matrix instruction (FE_FP8_F16=1)
     uint32_t gemm_splits = 8;  // most pieces a cut output tile takes (FE_GEMM_SPLITS; 1: never cut)
@@ -110,6 +111,11 @@ int fe_fp4_kernels_load(fe_fp4_kernels **out) {
             const std::string nm = std::to_string(xp) + "_c" + std::to_string(kWideColForms[j]) + (i / 4 ? "_e" : "");
             get(&k->wide[i / 4][i % 4][j], "fe_gemv_nvfp4_r" + nm, wide_lds(xp, kWideColForms[j], wide_waves(xp, kWideColForms[j], i / 4)));
             if (i % 4 < 3) get(&k->wide_q[i / 4][i % 4][j], "fe_gemv_nvfp4_q" + nm, kCuLds);
+        }
+    for (uint32_t i = 0; i < 5; i++)
+        for (uint32_t j = 0; j < 7; j++) {
+            const uint32_t xo = kGemvRowForms[i], co = kGemvColForms[j];
+            if (gemv_form(xo, co)) get(&k->gemv8[i][j], "fe_gemv_fp8_r" + std::to_string(xo) + "_c" + std::to_string(co), gemv_lds(xo, co));
         }
     if (!c) c = fe_hip_module_get_function(&k->quant8, k->module, "fe_fp8_quant");
     if (!c) c = fe_hip_module_get_function(&k->expand8, k->module, "fe_fp8_expand");
@@ -427,6 +433,11 @@ static uint32_t gemv_splits(const fe_fp4_kernels *kern, const fe_fp4_workspace *
     return std::max(sk, 1u);
 }
 
+// Most rows that an FP8 linear takes through its GEMV. us, GEMM -> GEMV at 1 / 17 / 32 / 64 rows: 17408 x 5120 24.4 -> 15.1, 25.2 -> 16.1, 25.8 -> 17.4, 27.7 -> 27.1; 5120 x
+// 5120 12.0 -> 6.1, 12.5 -> 8.3, 12.7 -> 8.5, 13.3 -> 11.0; 1024 x 2816 9.7 -> 3.9, 10.2 -> 3.8, 10.2 -> 4.2, 10.7 -> 5.7; 4096 x 14336 21.2 -> 10.8, 19.8 -> 13.1, 20.0 -> 15.3,
+// 21.2 -> 21.1; 5120 x 17408 25.4 -> 15.8, 24.0 -> 18.2, 24.3 -> 22.1, but 25.2 -> 25.6 at 48 and 26.0 -> 28.2 at 64 (the activations' way from L2 once a program).
+static uint32_t fp8_gemv_rows(uint32_t k) { return k <= 14336 ? 64 : 40; }
+
 // x: null, or the activations (bf16 rows of lda) which that GEMV quantizes itself
 static int linear_gemm(const fe_fp4_linear *l, const fe_fp4_kernels *kern, fe_stream_t s, const fe_fp4_workspace *ws, fe_devptr_t y, uint32_t ldy,
                        uint32_t m, fe_devptr_t res, fe_devptr_t x, uint32_t lda) {
@@ -475,6 +486,12 @@ static int linear_gemm(const fe_fp4_linear *l, const fe_fp4_kernels *kern, fe_st
     // FP8 runs on the 8-bit matrix instruction over the codes of both operands, k tiles of 128 (FE_FP8_F16=1: the fp16
     // expansion on the 16-bit instruction, k tiles of 64; same products, another order of the f32 sums)
     const bool codes8 = l->fp8 && !kern->fp8_f16;
+    if (codes8 && kern->gemv && !kern->tile.force_tile && kern->gemm_sk < 2 && m <= fp8_gemv_rows(k)) {
+        const uint32_t form = gemv_row_form(m), xo = kGemvRowForms[form], cols = gemv_cols(std::max(m, 3u), n, k, xo, std::max(kern->cus, 1u), kern->gemv_cols ? (int32_t)kern->gemv_cols : -1), co = kGemvColForms[cols];
+        fe_devptr_t codes = ws->codes.p;
+        void *args[] = {&y, &codes, &w, &alpha, &res, &m, &n, &k, &ldy, &w_snt, &w_skt, &w_sr};
+        return fe_hip_launch(kern->gemv8[form][cols], (n / 8 + co - 1) / co, 1, 1, 256, 1, 1, gemv_lds(xo, co), s, args);
+    }
     const FeGemmTileOptions f16_form{1, 0, false};  // (the fp16 form exists for 256 x 256 tiles only)
     const FeGemmPlan plan = fe_gemm_plan(m, n, codes8 ? k / 128 : k / 64, kern->cus, ws->part.p, ws->part.bytes, ws->counters.p, kGemvCounters,
                                          kern->gemm_splits, kern->gemm_sk, /*small_b=*/!l->fp8,

@@ -673,6 +673,130 @@ FP8C_GEMM_KERNEL(_h7, FpTileH7, false)
 FP8C_GEMM_KERNEL(_h6, FpTileH6, false)
 FP8C_GEMM_KERNEL(_h5, FpTileH5, false)
 
+// ---- FP8 GEMV (few rows): the weights read once, no hand-off -----------------------------------------------------------
+//
+// c[m][ldc] = bf16((codes . W^T) * alpha[n]) (+ res) for m <= 8 XO rows of e4m3 codes [m][k], weights as in fe_gemm_fp8_codes. grid ceil(N / 8 CO), 256 threads: a program takes
+// 8 CO weight rows over all of K, its four wavefronts a quarter of K's steps of 128 codes each, DEPTH - 1 steps ahead in LDS stages of their own; a load is 8 rows x 128 bytes,
+// a row's 16-byte chunk c at position c ^ (row & 7). A wavefront adds its products in ascending k, the four sums are added in order: a row's bits depend on K and W only.
+// Bound by the weights' way from HBM up to 16 rows, by the activations' way from L2 as rows and K grow. It replaces the GEMM, whose tiles of 128 rows are mostly empty and whose
+// pieces of K need a reduce launch: fp8_gemv_rows of fe_fp4.cpp has both sides.
+template <int XO, int CO>
+struct Fp8Gemv {
+    static constexpr int L = CO + XO, STAGE = L * 1024;
+    static constexpr int FIT = 20 * 1024 / STAGE, DEPTH = FIT < 3 ? 3 : FIT < 8 ? FIT : 8;  // two programs a CU where three steps allow it
+    static_assert((DEPTH - 1) * L < 64 && 4 * DEPTH * STAGE <= 160 * 1024, "stages");
+};
+
+template <int XO, int CO>
+__device__ __forceinline__ void gemv_fp8_body(uint16_t* c, const uint8_t* x, const uint8_t* w, const float* alpha, const uint16_t* res, uint32_t m, uint32_t n, uint32_t k,
+                                              uint32_t ldc, uint32_t w_snt, uint32_t w_skt, uint32_t w_sr) {
+    typedef Fp8Gemv<XO, CO> C;
+    constexpr int RG = (XO + 1) / 2, CG = (CO + 1) / 2, AHEAD = C::DEPTH - 1, PITCH = 16 * CG + 4;
+    extern __shared__ __attribute__((aligned(1024))) unsigned char lds[];
+    const uint32_t tid = threadIdx.x, lane = tid & 63, wave = __builtin_amdgcn_readfirstlane(tid >> 6), r = lane & 15, g = lane >> 4;
+    const uint32_t col0 = blockIdx.x * 8 * CO, cols = n - col0 < 8 * CO ? n - col0 : 8 * CO, nt0 = col0 / 128, span = n / 128 - nt0 < 2 ? n / 128 - nt0 : 2;
+    const u32x4 wrs = g8_rsrc(w + (size_t)nt0 * w_snt, span * 128 * k), xrs = g8_rsrc(x, m * k);
+    // (columns and rows that do not exist repeat the last one; a step is two of the layout's k tiles: chunks 0..3 of a row from the first, 4..7 from the second)
+    const uint32_t lr = lane >> 3, ch = (lane & 7) ^ lr;
+    uint32_t vw[CO], vx[XO];
+#pragma unroll
+    for (int j = 0; j < CO; j++) {
+        const uint32_t i = col0 + (8 * j + lr < cols ? 8 * j + lr : cols - 1) - 128 * nt0;
+        vw[j] = (i >> 7) * w_snt + (ch >> 2) * w_skt + (i & 127) * w_sr + (ch & 3) * 16;
+    }
+#pragma unroll
+    for (int j = 0; j < XO; j++) vx[j] = (8 * j + lr < m ? 8 * j + lr : m - 1) * k + ch * 16;
+    unsigned char* stages = lds + wave * (C::DEPTH * C::STAGE);
+    const uint32_t stages0 = g8_lds_addr(stages);
+    const uint32_t steps = k / 128, s0 = wave * steps / 4, count = (wave + 1) * steps / 4 - s0;
+    auto issue = [&](uint32_t s, uint32_t slot) {
+        const uint32_t at = stages0 + slot * C::STAGE;
+#pragma unroll
+        for (int j = 0; j < CO; j++) g8_load_lds16_nt(wrs, at + j * 1024, vw[j], (s0 + s) * 2 * w_skt);
+#pragma unroll
+        for (int j = 0; j < XO; j++) g8_load_lds16(xrs, at + (CO + j) * 1024, vx[j], (s0 + s) * 128);
+    };
+    uint32_t fw[CG][2], fx[RG][2];
+    auto frag = [&](uint32_t row, int h) { return row * 128 + (((4 * h + g) ^ (row & 7)) << 4); };
+#pragma unroll
+    for (int h = 0; h < 2; h++) {
+#pragma unroll
+        for (int j = 0; j < CG; j++) fw[j][h] = frag(16 * j + r < 8 * CO ? 16 * j + r : 8 * CO - 1, h);
+#pragma unroll
+        for (int i = 0; i < RG; i++) fx[i][h] = CO * 1024 + frag(16 * i + r < m ? 16 * i + r : m - 1, h);
+    }
+    f32x4 acc[RG][CG] = {};
+    uint32_t slot = 0;
+    auto add = [&]() {
+        const unsigned char* st = stages + slot * C::STAGE;
+        auto read = [&](const uint32_t (&at)[2]) {
+            const u32x4 lo = *(const u32x4*)(st + at[0]), hi = *(const u32x4*)(st + at[1]);
+            return (g8_i32x8){(int)lo[0], (int)lo[1], (int)lo[2], (int)lo[3], (int)hi[0], (int)hi[1], (int)hi[2], (int)hi[3]};
+        };
+        g8_i32x8 wv[CG];
+#pragma unroll
+        for (int j = 0; j < CG; j++) wv[j] = read(fw[j]);
+#pragma unroll
+        for (int i = 0; i < RG; i++) {
+            const g8_i32x8 xv = read(fx[i]);
+#pragma unroll
+            for (int j = 0; j < CG; j++) acc[i][j] = __builtin_amdgcn_mfma_scale_f32_16x16x128_f8f6f4(wv[j], xv, acc[i][j], 0, 0, 0, 0, 0, 0);
+        }
+        slot = slot + 1 == C::DEPTH ? 0 : slot + 1;
+    };
+    if (count) {
+#pragma unroll
+        for (int u = 0; u < AHEAD; u++) issue((uint32_t)u < count ? u : count - 1, u);  // past the end: the last step again, not added
+        uint32_t s = 0;
+        for (; s + AHEAD < count; s++) {
+            g8_loads_wait<(AHEAD - 1) * C::L>();  // (the stage in front of this one has been read, too)
+            issue(s + AHEAD, slot ? slot - 1 : AHEAD);
+            add();
+        }
+        auto tail = [&](auto u_tag) {
+            constexpr int U = decltype(u_tag)::value;
+            if constexpr (U < AHEAD)
+                if (s + U < count) {
+                    g8_loads_wait<(AHEAD - 1 - U) * C::L>();
+                    add();
+                }
+        };
+        tail(std::integral_constant<int, 0>{});
+        tail(std::integral_constant<int, 1>{});
+        tail(std::integral_constant<int, 2>{});
+        tail(std::integral_constant<int, 3>{});
+        tail(std::integral_constant<int, 4>{});
+        tail(std::integral_constant<int, 5>{});
+        tail(std::integral_constant<int, 6>{});
+        g8_loads_wait<0>();
+    }
+    float(*red)[16][PITCH] = (float(*)[16][PITCH])lds;
+#pragma unroll
+    for (int i = 0; i < RG; i++) {
+        __syncthreads();
+#pragma unroll
+        for (int j = 0; j < CG; j++) *(f32x4*)&red[wave][r][16 * j + 4 * g] = acc[i][j];
+        __syncthreads();
+        for (uint32_t e = tid; e < 16 * 2 * CO; e += 256) {
+            const uint32_t row = e / (2 * CO), j = 4 * (e % (2 * CO));
+            if (16 * i + row >= m || j >= cols) continue;
+            const f32x4 sum = ((*(const f32x4*)&red[0][row][j] + *(const f32x4*)&red[1][row][j]) + *(const f32x4*)&red[2][row][j]) + *(const f32x4*)&red[3][row][j];
+            const float v[4] = {sum[0], sum[1], sum[2], sum[3]};
+            fp4_store4(c, res, (size_t)(16 * i + row) * ldc + col0 + j, v, *(const f32x4*)(alpha + col0 + j));
+        }
+    }
+}
+
+#define FP8_GEMV_KERNEL(XO, CO)                                                                                                                              \
+    extern "C" __global__ __launch_bounds__(256) void fe_gemv_fp8_r##XO##_c##CO(uint16_t* c, const uint8_t* x, const uint8_t* w, const float* alpha,          \
+        const uint16_t* res, uint32_t m, uint32_t n, uint32_t k, uint32_t ldc, uint32_t w_snt, uint32_t w_skt, uint32_t w_sr) {                               \
+        gemv_fp8_body<XO, CO>(c, x, w, alpha, res, m, n, k, ldc, w_snt, w_skt, w_sr);                                                                         \
+    }
+#define FP8_GEMV_ROWS(XO) FP8_GEMV_KERNEL(XO, 1) FP8_GEMV_KERNEL(XO, 2) FP8_GEMV_KERNEL(XO, 3) FP8_GEMV_KERNEL(XO, 4) FP8_GEMV_KERNEL(XO, 5)
+FP8_GEMV_ROWS(1) FP8_GEMV_ROWS(2) FP8_GEMV_ROWS(4) FP8_GEMV_ROWS(6) FP8_GEMV_ROWS(8)
+FP8_GEMV_KERNEL(1, 6) FP8_GEMV_KERNEL(2, 6) FP8_GEMV_KERNEL(4, 6) FP8_GEMV_KERNEL(6, 6)
+FP8_GEMV_KERNEL(1, 9) FP8_GEMV_KERNEL(2, 9) FP8_GEMV_KERNEL(4, 9)
+
 // ---- GEMV (1..48 rows) -------------------------------------------------------------------------------------------------
 
 #define FP4_GEMV_RG 8  // 16-row groups of a 128-row weight tile
