@@ -78,8 +78,9 @@ bool fe_bf16_gemv_swiglu_takes(const fe_bf16_kernels *kern, fe_devptr_t big, fe_
 int fe_bf16_gemv_swiglu(const fe_bf16_kernels *kern, fe_stream_t s, fe_devptr_t act, fe_devptr_t x, fe_devptr_t gate, fe_devptr_t up, uint32_t m, uint32_t inter, uint32_t k) {
     const uint32_t form = gemv_row_form(m), xo = kGemvRowForms[form];
     const uint32_t cols = gemv_cols(m, inter, k, xo, std::max(kern->cus, 1u), kern->nc), co = kGemvColForms[cols];
-    void *args[] = {&act, &x, &gate, &up, &m, &inter, &k, &k};
-    return fe_hip_launch(kern->gemv_swiglu[form][cols], (inter / 8 + co - 1) / co, 1, 1, 256, 1, 1, gemv_lds(xo, co), s, args);
+    uint32_t pc = gemv_even(inter, 8 * co, std::max(kern->cus, 1u), 2, kern->nc > 0 || m <= 2);
+    void *args[] = {&act, &x, &gate, &up, &m, &inter, &k, &k, &pc};
+    return fe_hip_launch(kern->gemv_swiglu[form][cols], (inter + pc - 1) / pc, 1, 1, 256, 1, 1, gemv_lds(xo, co), s, args);
 }
 
 extern "C" {
@@ -157,8 +158,9 @@ static int launch_gemv(const fe_bf16_kernels *kern, fe_stream_t s, fe_devptr_t y
     }
     const uint32_t form = gemv_row_form(m), xo = kGemvRowForms[form];
     const uint32_t cols = gemv_cols(m, n, k, xo, std::max(kern->cus, 1u), kern->nc), co = kGemvColForms[cols];
-    void *args[] = {&y, &x, &w, &res, &m, &n, &k, &lda, &ldy};
-    return fe_hip_launch(kern->gemv[form][cols], (n / 8 + co - 1) / co, 1, 1, 256, 1, 1, gemv_lds(xo, co), s, args);
+    uint32_t pc = gemv_even(n, 8 * co, std::max(kern->cus, 1u), 2, kern->nc > 0 || m <= 2);
+    void *args[] = {&y, &x, &w, &res, &m, &n, &k, &lda, &ldy, &pc};
+    return fe_hip_launch(kern->gemv[form][cols], (n + pc - 1) / pc, 1, 1, 256, 1, 1, gemv_lds(xo, co), s, args);
 }
 
 int fe_bf16_gemv(const fe_bf16_kernels *kern, fe_stream_t s, fe_devptr_t y, uint32_t ldy, fe_devptr_t x, uint32_t lda,

@@ -489,8 +489,9 @@ static int linear_gemm(const fe_fp4_linear *l, const fe_fp4_kernels *kern, fe_st
     if (codes8 && kern->gemv && !kern->tile.force_tile && kern->gemm_sk < 2 && m <= fp8_gemv_rows(k)) {
         const uint32_t form = gemv_row_form(m), xo = kGemvRowForms[form], cols = gemv_cols(std::max(m, 3u), n, k, xo, std::max(kern->cus, 1u), kern->gemv_cols ? (int32_t)kern->gemv_cols : -1), co = kGemvColForms[cols];
         fe_devptr_t codes = ws->codes.p;
-        void *args[] = {&y, &codes, &w, &alpha, &res, &m, &n, &k, &ldy, &w_snt, &w_skt, &w_sr};
-        return fe_hip_launch(kern->gemv8[form][cols], (n / 8 + co - 1) / co, 1, 1, 256, 1, 1, gemv_lds(xo, co), s, args);
+        uint32_t pc = gemv_even(n, 8 * co, std::max(kern->cus, 1u), 4, kern->gemv_cols != 0 || m <= 2);
+        void *args[] = {&y, &codes, &w, &alpha, &res, &m, &n, &k, &ldy, &w_snt, &w_skt, &w_sr, &pc};
+        return fe_hip_launch(kern->gemv8[form][cols], (n + pc - 1) / pc, 1, 1, 256, 1, 1, gemv_lds(xo, co), s, args);
     }
     const FeGemmTileOptions f16_form{1, 0, false};  // (the fp16 form exists for 256 x 256 tiles only)
     const FeGemmPlan plan = fe_gemm_plan(m, n, codes8 ? k / 128 : k / 64, kern->cus, ws->part.p, ws->part.bytes, ws->counters.p, kGemvCounters,

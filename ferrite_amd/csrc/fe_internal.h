@@ -510,6 +510,18 @@ constexpr bool gemv_form(uint32_t xo, uint32_t co) { return 12 * (co + xo) <= 16
 constexpr uint32_t gemv_row_form(uint32_t m) { return m <= 8 ? 0 : (m + 15) / 16; }
 // Bf16Gemv<XO, CO>::LDS of k_bf16.hip, and what Fp8Gemv of k_fp4.hip takes
 inline uint32_t gemv_lds(uint32_t xo, uint32_t co) { return 4 * std::max(3u, std::min(20 / (co + xo), 8u)) * (co + xo) * 1024; }
+// The columns that each program of a form of `most` columns takes (`whole`: those): as even as whole rounds of one program a CU allow, in steps of `step`; rows of a load
+// past them repeat the last one, which a cache holds. 5120 columns are 256 programs of 20 instead of 214 of 24, 17408 of 68 instead of 242 of 72. us, bf16 blocks (gate, up, down)
+// of 5120 x 17408 at 8 / 12 / 48 rows 83.9 -> 82.5, 87.5 -> 85.7, 142 -> 135, of 5120 x 8704 at 12 49.7 -> 47.1, of 1536 x 5120 at 12 15.2 -> 14.2; FP8 5120 x 17408 at 16
+// rows 17.3 -> 16.2, 5120 x 5120 7.6 -> 7.1. One and two rows, which are bound by the weights' way alone, gain nothing (bf16 3072 x 8192 27.7 -> 28.1: whole octets there), nor does NVFP4,
+// whose octets are pieces of 256 bytes (5120 x 17408 at 4 rows 14.6 -> 14.9: not done there).
+inline uint32_t gemv_even(uint32_t n, uint32_t most, uint32_t cus, uint32_t step, bool whole) {
+    const uint32_t programs = (n + most - 1) / most;
+    if (whole || 2 * programs <= cus) return most;
+    const uint32_t slots = (programs + cus - 1) / cus * cus;
+    return std::min(most, ((n + slots - 1) / slots + step - 1) / step * step);
+}
+
 // Which of kGemvColForms a GEMV takes. Time goes by the CU with the most columns, so the form is the one with the least of
 // rounds of one program a CU times a program's loads (columns, and half the weight for the x rows, which come from L2). us, 5120
 // columns of 17408 at 1 / 16 rows (640 octets of columns on 256 CUs): 2 octets 33.8 / 47.9, 3 octets 27.1 / 33.7, 4 octets

@@ -131,7 +131,7 @@ extern "C" __global__ __launch_bounds__(256) void fe_interleave_gu(uint16_t* dst
 
 // ---- GEMV (1..64 rows) -----------------------------------------------------------------------------------------------
 
-// y[r][n] = bf16(x[r][:] . W[n][:]) (+ res) for r < m <= 8 XO. grid ceil(N / 8 CO), 256 threads: a program takes 8 CO columns over
+// y[r][n] = bf16(x[r][:] . W[n][:]) (+ res) for r < m <= 8 XO. grid ceil(N / pc), 256 threads: a program takes pc <= 8 CO columns (gemv_even) over
 // all of K, its four wavefronts a quarter of K's steps of 64 each; a wavefront adds its products in v_mfma_f32_16x16x32_bf16 in
 // ascending k, the four sums are added in order. So a row's bits depend on K only, neither on the other rows nor on XO or
 // CO: the host picks them by the row count and the shape, where the reference picks between two kernels by the shape.
@@ -161,12 +161,12 @@ struct Bf16Gemv {
 // (gemv_cols): within 2 % of the best width of both launches on six layers at 1 to 64 rows.
 template <int XO, int CO, bool PAIR>
 __device__ __forceinline__ void gemv_bf16_body(uint16_t* c, const uint16_t* a, const uint16_t* w, const uint16_t* w2, const uint16_t* res,
-                                               uint32_t m, uint32_t n, uint32_t k, uint32_t lda, uint32_t ldc) {
+                                               uint32_t m, uint32_t n, uint32_t k, uint32_t lda, uint32_t ldc, uint32_t pc) {
     typedef Bf16Gemv<XO, CO> C;
     constexpr int RG = (XO + 1) / 2, CG = (CO + 1) / 2, AHEAD = C::DEPTH - 1, PITCH = 16 * CG + 4;
     extern __shared__ __attribute__((aligned(1024))) unsigned char lds[];
     const uint32_t tid = threadIdx.x, lane = tid & 63, wave = __builtin_amdgcn_readfirstlane(tid >> 6), r = lane & 15, g = lane >> 4;
-    const uint32_t col0 = blockIdx.x * 8 * CO, cols = n - col0 < 8 * CO ? n - col0 : 8 * CO;
+    const uint32_t col0 = blockIdx.x * pc, cols = n - col0 < pc ? n - col0 : pc;
     const u32x4 wrs = g8_rsrc(w + (size_t)col0 * k, cols * k * 2), w2rs = PAIR ? g8_rsrc(w2 + (size_t)col0 * k, cols * k * 2) : wrs, xrs = g8_rsrc(a, ((m - 1) * lda + k) * 2);
     // a row's 16-byte chunk c of a step lies at position c ^ (row & 7); rows that do not exist repeat the last one
     const uint32_t lr = lane >> 3, lc = ((lane & 7) ^ lr) << 4;
@@ -294,12 +294,12 @@ __device__ __forceinline__ void gemv_bf16_body(uint16_t* c, const uint16_t* a, c
 #define BF16_GEMV_KERNEL(XO, CO)                                                                                             \
     extern "C" __global__ __launch_bounds__(256) void fe_gemv_bf16_r##XO##_c##CO(                                            \
         uint16_t* c, const uint16_t* a, const uint16_t* w, const uint16_t* res, uint32_t m, uint32_t n, uint32_t k, uint32_t lda, \
-        uint32_t ldc) {                                                                                                    \
-        gemv_bf16_body<XO, CO, false>(c, a, w, w, res, m, n, k, lda, ldc);                                                 \
+        uint32_t ldc, uint32_t pc) {                                                                                       \
+        gemv_bf16_body<XO, CO, false>(c, a, w, w, res, m, n, k, lda, ldc, pc);                                             \
     }                                                                                                                      \
     extern "C" __global__ __launch_bounds__(256) void fe_gemv_bf16_swiglu_r##XO##_c##CO(                                   \
-        uint16_t* act, const uint16_t* a, const uint16_t* gate, const uint16_t* up, uint32_t m, uint32_t n, uint32_t k, uint32_t lda) { \
-        gemv_bf16_body<XO, CO, true>(act, a, gate, up, nullptr, m, n, k, lda, n);                                          \
+        uint16_t* act, const uint16_t* a, const uint16_t* gate, const uint16_t* up, uint32_t m, uint32_t n, uint32_t k, uint32_t lda, uint32_t pc) { \
+        gemv_bf16_body<XO, CO, true>(act, a, gate, up, nullptr, m, n, k, lda, n, pc);                                      \
     }
 #define BF16_GEMV_ROWS(XO)                                                                                                  \
     BF16_GEMV_KERNEL(XO, 1) BF16_GEMV_KERNEL(XO, 2) BF16_GEMV_KERNEL(XO, 3) BF16_GEMV_KERNEL(XO, 4) BF16_GEMV_KERNEL(XO, 5)

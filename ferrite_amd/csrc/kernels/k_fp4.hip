@@ -675,8 +675,8 @@ FP8C_GEMM_KERNEL(_h5, FpTileH5, false)
 
 // ---- FP8 GEMV (few rows): the weights read once, no hand-off -----------------------------------------------------------
 //
-// c[m][ldc] = bf16((codes . W^T) * alpha[n]) (+ res) for m <= 8 XO rows of e4m3 codes [m][k], weights as in fe_gemm_fp8_codes. grid ceil(N / 8 CO), 256 threads: a program takes
-// 8 CO weight rows over all of K, its four wavefronts a quarter of K's steps of 128 codes each, DEPTH - 1 steps ahead in LDS stages of their own; a load is 8 rows x 128 bytes,
+// c[m][ldc] = bf16((codes . W^T) * alpha[n]) (+ res) for m <= 8 XO rows of e4m3 codes [m][k], weights as in fe_gemm_fp8_codes. grid ceil(N / pc), 256 threads: a program takes
+// pc <= 8 CO weight rows (gemv_even) over all of K, its four wavefronts a quarter of K's steps of 128 codes each, DEPTH - 1 steps ahead in LDS stages of their own; a load is 8 rows x 128 bytes,
 // a row's 16-byte chunk c at position c ^ (row & 7). A wavefront adds its products in ascending k, the four sums are added in order: a row's bits depend on K and W only.
 // Bound by the weights' way from HBM up to 16 rows, by the activations' way from L2 as rows and K grow. It replaces the GEMM, whose tiles of 128 rows are mostly empty and whose
 // pieces of K need a reduce launch: fp8_gemv_rows of fe_fp4.cpp has both sides.
@@ -689,12 +689,12 @@ struct Fp8Gemv {
 
 template <int XO, int CO>
 __device__ __forceinline__ void gemv_fp8_body(uint16_t* c, const uint8_t* x, const uint8_t* w, const float* alpha, const uint16_t* res, uint32_t m, uint32_t n, uint32_t k,
-                                              uint32_t ldc, uint32_t w_snt, uint32_t w_skt, uint32_t w_sr) {
+                                              uint32_t ldc, uint32_t w_snt, uint32_t w_skt, uint32_t w_sr, uint32_t pc) {
     typedef Fp8Gemv<XO, CO> C;
     constexpr int RG = (XO + 1) / 2, CG = (CO + 1) / 2, AHEAD = C::DEPTH - 1, PITCH = 16 * CG + 4;
     extern __shared__ __attribute__((aligned(1024))) unsigned char lds[];
     const uint32_t tid = threadIdx.x, lane = tid & 63, wave = __builtin_amdgcn_readfirstlane(tid >> 6), r = lane & 15, g = lane >> 4;
-    const uint32_t col0 = blockIdx.x * 8 * CO, cols = n - col0 < 8 * CO ? n - col0 : 8 * CO, nt0 = col0 / 128, span = n / 128 - nt0 < 2 ? n / 128 - nt0 : 2;
+    const uint32_t col0 = blockIdx.x * pc, cols = n - col0 < pc ? n - col0 : pc, nt0 = col0 / 128, span = n / 128 - nt0 < 2 ? n / 128 - nt0 : 2;
     const u32x4 wrs = g8_rsrc(w + (size_t)nt0 * w_snt, span * 128 * k), xrs = g8_rsrc(x, m * k);
     // (columns and rows that do not exist repeat the last one; a step is two of the layout's k tiles: chunks 0..3 of a row from the first, 4..7 from the second)
     const uint32_t lr = lane >> 3, ch = (lane & 7) ^ lr;
@@ -789,8 +789,8 @@ __device__ __forceinline__ void gemv_fp8_body(uint16_t* c, const uint8_t* x, con
 
 #define FP8_GEMV_KERNEL(XO, CO)                                                                                                                              \
     extern "C" __global__ __launch_bounds__(256) void fe_gemv_fp8_r##XO##_c##CO(uint16_t* c, const uint8_t* x, const uint8_t* w, const float* alpha,          \
-        const uint16_t* res, uint32_t m, uint32_t n, uint32_t k, uint32_t ldc, uint32_t w_snt, uint32_t w_skt, uint32_t w_sr) {                               \
-        gemv_fp8_body<XO, CO>(c, x, w, alpha, res, m, n, k, ldc, w_snt, w_skt, w_sr);                                                                         \
+        const uint16_t* res, uint32_t m, uint32_t n, uint32_t k, uint32_t ldc, uint32_t w_snt, uint32_t w_skt, uint32_t w_sr, uint32_t pc) {                  \
+        gemv_fp8_body<XO, CO>(c, x, w, alpha, res, m, n, k, ldc, w_snt, w_skt, w_sr, pc);                                                                         \
     }
 #define FP8_GEMV_ROWS(XO) FP8_GEMV_KERNEL(XO, 1) FP8_GEMV_KERNEL(XO, 2) FP8_GEMV_KERNEL(XO, 3) FP8_GEMV_KERNEL(XO, 4) FP8_GEMV_KERNEL(XO, 5)
 FP8_GEMV_ROWS(1) FP8_GEMV_ROWS(2) FP8_GEMV_ROWS(4) FP8_GEMV_ROWS(6) FP8_GEMV_ROWS(8)

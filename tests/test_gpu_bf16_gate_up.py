@@ -6,8 +6,8 @@ pytestmark = pytest.mark.gpu
 
 
 # One step a wavefront (fewer than stages in flight), fewer steps in all than stages, as many as stages, many; the last program partly past the columns; every row form and
-# width of a program; rows by their count and as decode rows, prompt rows that are few enough and one more
-@pytest.mark.parametrize("hidden,inter", [(256, 320), (512, 1216), (1792, 576), (2048, 1344), (5120, 192)])
+# width of a program, also of fewer columns than its octets; rows by their count and as decode rows, prompt rows that are few enough and one more
+@pytest.mark.parametrize("hidden,inter", [(256, 320), (512, 1216), (1792, 576), (2048, 1344), (5120, 192), (256, 5184)])
 def test_one_launch_gives_the_bits_of_three(hidden, inter):
     import torch
     from ferrite_amd import bf16, route

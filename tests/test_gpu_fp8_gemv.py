@@ -6,8 +6,8 @@ pytestmark = pytest.mark.gpu
 
 
 # One step of K for one wavefront alone, quarters of unequal length, one step more than stages; the last program partly past n, columns of two weight tiles; K past the line
-# of 40 rows
-@pytest.mark.parametrize("n,k", [(128, 128), (384, 640), (640, 2944), (256, 17408)])
+# of 40 rows; programs of fewer columns than their octets
+@pytest.mark.parametrize("n,k", [(128, 128), (384, 640), (640, 2944), (256, 17408), (4992, 640)])
 def test_every_form_gives_the_same_bits(n, k):
     import torch
     from ferrite_amd import fp4
