@@ -24,8 +24,8 @@ typedef struct fe_bf16_kernels fe_bf16_kernels;
 int fe_bf16_kernels_load(fe_bf16_kernels **out);
 int fe_bf16_kernels_destroy(fe_bf16_kernels *k);
 /* Switches by name: "nc" columns a GEMV program takes (rounded up to 8, 16, .. 48, 72; FE_BF16_NC; -1 = by the shape), "raster_group" (FE_BF16_GROUP;
- * -1 = by the shape), "gemm_splits" (FE_GEMM_SPLITS); "gemm_tile" 0..3 (output tile of the GEMMs: by the shape,
- * 256 x 256, 128 x 256, 128 x 128) and "gemm_pieces" (pieces of K a forced small tile takes), both for tests. Read from the environment once, at load; no call reads it later. */
+ * -1 = by the shape), "gemm_splits" (FE_GEMM_SPLITS); "gemm_tile" 0..6 (output tile of the GEMMs: by the shape,
+ * 256 x 256, 128 x 256, 128 x 128, 224 x 256, 192 x 256, 160 x 256; other values FE_ERR_ARG) and "gemm_pieces" (pieces of K a forced small tile takes), both for tests. Read from the environment once, at load; no call reads it later. */
 int fe_bf16_kernels_set_option(fe_bf16_kernels *k, const char *name, int32_t value);
 
 /* fe_gemv_bf16 / fe_gemv_bf16_kw (gemm.rs:172-262): m <= 8 rows (fe_bf16_linear_forward takes up to 64 through

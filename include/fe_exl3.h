@@ -57,7 +57,7 @@ int fe_exl3_kernels_destroy(fe_exl3_kernels *k);
 /* Switches of the launch paths, by name (the environment variable that sets the same switch when the kernels are loaded):
  * "fused_rot" 0/1 (FE_EXL3_NO_FUSED_ROT), "fused_rot_pairs" (FE_EXL3_FUSED_ROT_PAIRS), "group" 0/1 (FE_EXL3_NO_GROUP),
  * "hat_rows" (FE_EXL3_HAT_ROWS; 0 = never), "lds_pad" 0/1 (FE_EXL3_NO_LDS_PAD), "fuse" 0/1 (FE_EXL3_NO_FUSE), "gemm_group_m" (FE_EXL3_GROUP),
- * "gemm_splits" (FE_GEMM_SPLITS), "gemm_tile" 0..3 (output tile of the prefill GEMM: by the shape, 256 x 256, 128 x 256, 128 x 128) and
+ * "gemm_splits" (FE_GEMM_SPLITS), "gemm_tile" 0..3 (output tile of the prefill GEMM: by the shape, 256 x 256, 128 x 256, 128 x 128; other values FE_ERR_ARG) and
  * "gemm_pieces" (pieces of K a forced small tile takes), both for tests, "rgemm" 0/1 (FE_EXL3_NO_RGEMM: prompts of 65..2303 rows through the
  * GEMM that decodes into registers, where its estimate is not above the other one's; a forced gemm_tile, another gemm_splits or gemm_sk than the default and kept tiles take the other one),
  * "rgemm_form" 0..2 and "rgemm_pieces" (its column blocks a program and pieces of K a tile, 0: by its plan; for tests), "gemv_pairs" 0..2 (two programs a workgroup of the decode GEMV for 17..64 rows

@@ -30,7 +30,7 @@ int fe_fp4_kernels_destroy(fe_fp4_kernels *k);
  * a program, or one of the FP8 GEMV (up to 64 rows, 40 where k > 14336), takes, rounded up to 8, 16, .. 48, 72; 0 = by the shape; same bits), "gemv_quant" (FE_FP4_GEMV_QUANT: most values, rows x k, that four wavefronts of such a program quantize themselves, eight
  * twice as many; default 10240; 0 = by a launch of its own; same bits), "gemv_once" and "gemv_waves" (accepted, without effect), "xcd" -1/0/1
  * (FE_FP4_XCD), "fp8_f16" 0/1 (FE_FP8_F16), "gemm_splits" (FE_GEMM_SPLITS), "gemm_tile" 0..6 (output tile of the GEMMs: by the shape, 256 x 256,
- * 128 x 256, 128 x 128, 224 x 256, 192 x 256, 160 x 256) and "gemm_pieces" (pieces of K a forced small tile takes), both for tests, "gemm_sk" 0..3 (FE_GEMM_SK: the stream-K schedule of the
+ * 128 x 256, 128 x 128, 224 x 256, 192 x 256, 160 x 256; other values FE_ERR_ARG) and "gemm_pieces" (pieces of K a forced small tile takes), both for tests, "gemm_sk" 0..3 (FE_GEMM_SK: the stream-K schedule of the
  * GEMM never / where it is the faster one / over all tiles / whole rounds then runs, the last two for tests). forward() reads no environment variable. No
  * counterpart in the reference (its FE_FP4_GROUP is read at load too, crates/fe-fp4/src/lib.rs:31-32, 68). */
 int fe_fp4_kernels_set_option(fe_fp4_kernels *k, const char *name, int32_t value);

@@ -1,0 +1,37 @@
+"""Host arithmetic of the handles' options and dispatch rules (no GPU): the sources compiled here against the built library, which serves what they call elsewhere."""
+import os
+import subprocess
+
+import pytest
+
+ROOT = os.path.dirname(os.path.dirname(os.path.abspath(__file__)))
+ROCM = os.environ.get("ROCM_PATH", "/opt/rocm")
+
+
+def run_host(tmp_path, source, main):
+    """The lines that `main` prints, compiled behind csrc/`source`."""
+    src, exe, lib = tmp_path / "main.cpp", str(tmp_path / "main"), os.path.join(ROOT, "ferrite_amd")
+    if not os.path.exists(os.path.join(lib, "libferrite_amd.so")):
+        from ferrite_amd import build
+        build.build()
+    src.write_text(f'#include <cstdio>\n#include "{source}"\n{main}')
+    subprocess.run(["g++", "-std=c++17", "-O1", "-fPIC", "-D__HIP_PLATFORM_AMD__", "-I", os.path.join(lib, "csrc"), "-I", os.path.join(ROOT, "include"), "-I", os.path.join(ROCM, "include"),
+                    str(src), "-o", exe, "-L", lib, "-lferrite_amd", "-L", os.path.join(ROCM, "lib"), "-lamdhip64", f"-Wl,-rpath,{lib}:{os.path.join(ROCM, 'lib')}"], check=True)
+    return subprocess.run([exe], stdout=subprocess.PIPE, text=True, check=True).stdout.splitlines()
+
+
+@pytest.mark.parametrize("handle,most", [("fp4", 6), ("bf16", 6), ("exl3", 3)])
+def test_a_tile_that_does_not_exist_is_refused(tmp_path, handle, most):
+    """gemm_tile picks a row of the tables of tiles and kernels: what lies past them is refused and changes nothing."""
+    lines = run_host(tmp_path, f"fe_{handle}.cpp", f"""
+int main() {{
+    fe_{handle}_kernels k;
+    auto set = [&](int v) {{
+        const int c = fe_{handle}_kernels_set_option(&k, "gemm_tile", v);
+        printf("%d %u\\n", c == FE_ERR_ARG ? 1 : c, k.tile.force_tile);
+    }};
+    for (int v = 0; v <= {most}; v++) set(v);
+    for (int v : {{-1, {most} + 1, 1000, (int)0x80000000}}) set(v);
+}}
+""")
+    assert lines == [f"0 {v}" for v in range(most + 1)] + [f"1 {most}"] * 4
