@@ -142,7 +142,7 @@ int fe_bf16_kernels_set_option(fe_bf16_kernels *k, const char *name, int32_t val
     if (nm == "nc") k->nc = value;
     else if (nm == "raster_group") k->raster_group = value;
     else if (nm == "gemm_splits") k->gemm_splits = (uint32_t)value;
-    else if (nm == "gemm_tile") return k->tile.set("fe_bf16_kernels_set_option", value);
+    else if (nm == "gemm_tile") return k->tile.set(value) ? 0 : fe_set_error(FE_ERR_ARG, "fe_bf16_kernels_set_option", "gemm_tile: 0..6");
     else if (nm == "gemm_pieces") k->tile.force_pieces = (uint32_t)value;
     else return fe_set_error(FE_ERR_ARG, "fe_bf16_kernels_set_option", name);
     return 0;

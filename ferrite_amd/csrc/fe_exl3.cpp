@@ -299,7 +299,7 @@ int fe_exl3_kernels_set_option(fe_exl3_kernels *k, const char *name, uint32_t va
     else if (nm == "gemm_group_m") o.gemm_group_m = value;
     else if (nm == "gemm_splits") o.gemm_splits = value;
     else if (nm == "gemm_sk") o.gemm_sk = value;
-    else if (nm == "gemm_tile") return k->tile.set("fe_exl3_kernels_set_option", value);
+    else if (nm == "gemm_tile") return k->tile.set(value) ? 0 : fe_set_error(FE_ERR_ARG, "fe_exl3_kernels_set_option", "gemm_tile: 0..3");
     else if (nm == "gemm_pieces") k->tile.force_pieces = value;
     else if (nm == "mlp_chain") o.mlp_chain = value;
     else if (nm == "rgemm") o.rgemm = value;

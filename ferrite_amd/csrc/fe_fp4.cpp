@@ -161,7 +161,7 @@ int fe_fp4_kernels_set_option(fe_fp4_kernels *k, const char *name, int32_t value
     else if (nm == "fp8_f16") k->fp8_f16 = value ? 1 : 0;
     else if (nm == "gemm_splits") k->gemm_splits = (uint32_t)value;
     else if (nm == "gemm_sk") k->gemm_sk = value;
-    else if (nm == "gemm_tile") return k->tile.set("fe_fp4_kernels_set_option", value);
+    else if (nm == "gemm_tile") return k->tile.set(value) ? 0 : fe_set_error(FE_ERR_ARG, "fe_fp4_kernels_set_option", "gemm_tile: 0..6");
     else if (nm == "gemm_pieces") k->tile.force_pieces = (uint32_t)value;
     else return fe_set_error(FE_ERR_ARG, "fe_fp4_kernels_set_option", name);
     return 0;

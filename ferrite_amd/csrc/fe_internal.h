@@ -277,10 +277,10 @@ struct FeGemmTileOptions {
     uint32_t force_tile = 0, force_pieces = 0;
     bool low = false;  // the handle has kernels of tiles 3..5 (force_tile 4, 5, 6)
     // option "gemm_tile": refused past the tiles that the handle has kernels of (fe_gemm_plan and the tables of kernels are indexed by it)
-    int set(const char *fn, int64_t value) {
-        if (value < 0 || value > (low ? kFeGemmTiles : 3u)) return fe_set_error(FE_ERR_ARG, fn, low ? "gemm_tile: 0..6" : "gemm_tile: 0..3");
+    bool set(int64_t value) {
+        if (value < 0 || value > (low ? kFeGemmTiles : 3u)) return false;
         force_tile = (uint32_t)value;
-        return 0;
+        return true;
     }
 };
 
