@@ -139,7 +139,8 @@ struct Fp4Block {
     u32x4 o[2];
 };
 // Without a NaN among the values: their magnitudes as bf16 bits are in order, so the largest is a maximum of 16-bit integers, and the conversions are the
-// hardware's; a block with a NaN (a magnitude above infinity's) goes through e2m1_nan_to_zero.
+// hardware's; a block with a NaN (a magnitude above infinity's) or an infinity, whose product with the multiplier may be one (g of 0, or so small that g / sf is 0), goes
+// through e2m1_nan_to_zero.
 __device__ __forceinline__ Fp4Block fp4_quant_block(u32x4 r0, u32x4 r1, float g) {
     typedef uint16_t u16x2 __attribute__((ext_vector_type(2)));
     u16x2 top = {0, 0};
@@ -149,8 +150,8 @@ __device__ __forceinline__ Fp4Block fp4_quant_block(u32x4 r0, u32x4 r1, float g)
         top = __builtin_elementwise_max(top, __builtin_bit_cast(u16x2, r1[j] & 0x7fff7fffu));
     }
     uint32_t amax = top[0] > top[1] ? top[0] : top[1];
-    const bool nan = amax > 0x7f80u;
-    if (nan) {  // the largest of the others
+    const bool special = amax >= 0x7f80u;
+    if (amax > 0x7f80u) {  // the largest of the others
         amax = 0;
 #pragma unroll
         for (int j = 0; j < 8; j++) {
@@ -164,7 +165,7 @@ __device__ __forceinline__ Fp4Block fp4_quant_block(u32x4 r0, u32x4 r1, float g)
     float sv = e4m3_to_f32(out.s8);
     float mul = sv > 0.f ? g / sv : 0.f;
     const f16x2 sc = e4m3_to_f16x2(out.s8);
-    const bool careful = nan || !(mul <= 3.402823466e38f);  // (0 times infinity)
+    const bool careful = special || !(mul <= 3.402823466e38f);  // (0 times infinity, on either side)
 #pragma unroll
     for (int w = 0; w < 2; w++) {
         float f[8];
