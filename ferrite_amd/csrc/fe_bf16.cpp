@@ -43,17 +43,22 @@ static uint32_t bf16_raster_group(uint32_t m, uint32_t n, uint32_t k, uint32_t t
     return n >= m ? 0 : tiles_m < 8 ? tiles_m : 8;
 }
 
+// Why a linear's operands are refused (0: they are not). Sets no error: rules of a dispatch ask it, too.
+static int refusal(fe_devptr_t y, uint32_t ldy, fe_devptr_t x, uint32_t lda, fe_devptr_t w, fe_devptr_t res, uint32_t n, uint32_t k, const char **why) {
+    if (!y || !x || !w) return *why = "null pointer", FE_ERR_ARG;
+    if (!n || !k || n % 8 || k % 64) return *why = "n % 8 == 0, k % 64 == 0", FE_ERR_SHAPE;
+    if (lda % 8 || lda < k || x % 16 || w % 16) return *why = "x / w rows must be 16-byte aligned, lda >= k", FE_ERR_ARG;
+    if (ldy % 4 || ldy < n || y % 8 || (res && res % 8)) return *why = "y / res rows must be 8-byte aligned, ldy >= n", FE_ERR_ARG;
+    return 0;
+}
 static int check(const char *fn, fe_devptr_t y, uint32_t ldy, fe_devptr_t x, uint32_t lda, fe_devptr_t w, fe_devptr_t res,
                  uint32_t n, uint32_t k) {
-    if (!y || !x || !w) return fe_set_error(FE_ERR_ARG, fn, "null pointer");
-    if (!n || !k || n % 8 || k % 64) {
-        char msg[120];
-        snprintf(msg, sizeof msg, "bf16 linear n %u k %u (n %% 8 == 0, k %% 64 == 0)", n, k);
-        return fe_set_error(FE_ERR_SHAPE, fn, msg);
-    }
-    if (lda % 8 || lda < k || x % 16 || w % 16) return fe_set_error(FE_ERR_ARG, fn, "x / w rows must be 16-byte aligned, lda >= k");
-    if (ldy % 4 || ldy < n || y % 8 || (res && res % 8)) return fe_set_error(FE_ERR_ARG, fn, "y / res rows must be 8-byte aligned, ldy >= n");
-    return 0;
+    const char *why = nullptr;
+    const int code = refusal(y, ldy, x, lda, w, res, n, k, &why);
+    if (!code) return 0;
+    char msg[120];
+    if (code == FE_ERR_SHAPE) snprintf(msg, sizeof msg, "bf16 linear n %u k %u (%s)", n, k, why);
+    return fe_set_error(code, fn, code == FE_ERR_SHAPE ? msg : why);
 }
 
 // Whether all of a call's rows go through the GEMV: a batch of decode rows, or one so small that the GEMV's one read of the weights is ahead of the GEMM's tiles. us at 17 /
@@ -68,7 +73,8 @@ bool fe_bf16_gemv_swiglu_takes(const fe_bf16_kernels *kern, fe_devptr_t big, fe_
     // 106, 5120 x 12288 98 -> 84, 4096 x 8192 60 -> 48, but 5120 x 8704 68 -> 71; of 24 rows 66 -> 60)
     if (m > kSmallBatch && dec < m && inter < 12288 && (uint64_t)m * k > 131072) return false;
     if (!m || m > kGemvPass || !rows_take_gemv(m, k, dec) || !inter || !k || inter % 8 || k % 256 || (uint64_t)m * k * 2 >= (1ull << 32)) return false;
-    if (check("", big, inter, x, k, gate, 0, inter, k) || check("", big, inter, x, k, up, 0, inter, k)) return false;
+    const char *why;
+    if (refusal(big, inter, x, k, gate, 0, inter, k, &why) || refusal(big, inter, x, k, up, 0, inter, k, &why)) return false;
     // programs that are done write act while others read x and the weights
     const uint64_t bytes = (uint64_t)m * inter * 2, weights = (uint64_t)inter * k * 2;
     auto apart = [&](fe_devptr_t p, uint64_t size) { return act + bytes <= p || p + size <= act; };
