@@ -68,10 +68,11 @@ static int check(const char *fn, fe_devptr_t y, uint32_t ldy, fe_devptr_t x, uin
 static bool rows_take_gemv(uint32_t m, uint32_t k, uint32_t dec) { return m <= kSmallBatch || dec >= m || (m <= 32 && (uint64_t)m * k <= (m <= 24 ? 350000 : 180000)); }
 
 bool fe_bf16_gemv_swiglu_takes(const fe_bf16_kernels *kern, fe_devptr_t big, fe_devptr_t act, fe_devptr_t x, fe_devptr_t gate, fe_devptr_t up, uint32_t m, uint32_t inter,
-                               uint32_t k, uint32_t dec) {
-    // (against the GEMM with SwiGLU, where the caller has its weights, wider programs have to carry the activations: a block of 32 rows, GEMM -> GEMV, us: 5120 x 17408 133 ->
-    // 106, 5120 x 12288 98 -> 84, 4096 x 8192 60 -> 48, but 5120 x 8704 68 -> 71; of 24 rows 66 -> 60)
-    if (m > kSmallBatch && dec < m && inter < 12288 && (uint64_t)m * k > 131072) return false;
+                               uint32_t k, uint32_t dec, bool over_gemm) {
+    // (against the GEMM with SwiGLU wider programs have to carry the activations: a block of 32 rows, GEMM -> GEMV, us: 5120 x 17408 133 ->
+    // 106, 5120 x 12288 98 -> 84, 4096 x 8192 60 -> 48, but 5120 x 8704 68 -> 71; of 24 rows 66 -> 60. Against gate, up and fe_silu_mul, where there are no such weights, it is ahead
+    // there too: 5120 x 8704 at 26 / 32 rows 63.0 -> 58.0, 63.9 -> 58.6, 5120 x 6144 at 30 53.0 -> 48.4, 7168 x 2048 at 25 32.7 -> 28.0)
+    if (over_gemm && m > kSmallBatch && dec < m && inter < 12288 && (uint64_t)m * k > 131072) return false;
     if (!m || m > kGemvPass || !rows_take_gemv(m, k, dec) || !inter || !k || inter % 8 || k % 256 || (uint64_t)m * k * 2 >= (1ull << 32)) return false;
     const char *why;
     if (refusal(big, inter, x, k, gate, 0, inter, k, &why) || refusal(big, inter, x, k, up, 0, inter, k, &why)) return false;

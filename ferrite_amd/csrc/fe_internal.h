@@ -503,10 +503,11 @@ int fe_gemm_launch(const FeGemmPlan &p, Gemm gemm, Reduce reduce) {
 
 // ---- gate, up and SwiGLU of decode rows over plain bf16 weights (fe_bf16.cpp) ---------------------------------------------------
 // Whether fe_bf16_gemv_swiglu does what two fe_bf16_linear_forward into big ([m][inter] each) and fe_route_silu_mul into act do: all rows go through the GEMV in one pass,
-// the operands are what those take, and act lies apart from what other programs still read. (Two launches less: see gemv_bf16_body for both sides.)
+// the operands are what those take, and act lies apart from what other programs still read. (Two launches less: see gemv_bf16_body for both sides.) over_gemm: the call would
+// otherwise take the GEMM with SwiGLU in its epilogue over interleaved weights, which is ahead of it at some row counts where gate, up and SwiGLU in three launches are not.
 struct fe_bf16_kernels;
 bool fe_bf16_gemv_swiglu_takes(const fe_bf16_kernels *kern, fe_devptr_t big, fe_devptr_t act, fe_devptr_t x, fe_devptr_t gate, fe_devptr_t up, uint32_t m, uint32_t inter,
-                               uint32_t k, uint32_t dec);
+                               uint32_t k, uint32_t dec, bool over_gemm);
 int fe_bf16_gemv_swiglu(const fe_bf16_kernels *kern, fe_stream_t s, fe_devptr_t act, fe_devptr_t x, fe_devptr_t gate, fe_devptr_t up, uint32_t m, uint32_t inter, uint32_t k);
 
 // ---- the GEMVs over programs of 8 CO columns and all of K, bf16 and FP8 ---------------------------------------------------------

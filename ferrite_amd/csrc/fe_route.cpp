@@ -371,11 +371,11 @@ int fe_route_mlp_forward_w(const fe_route_ctx *c, const fe_route_proj *gate_up, 
     const uint32_t pr_rows = rows - d;
     bool fused = false;
     // `n` rows through plain bf16 gate and up, each one part, in one launch with SwiGLU (the bits of two linears and fe_silu_mul; big is not written), down then not the trellis'
-    auto pair = [&](uint32_t n) {
+    auto pair = [&](uint32_t n, bool over_gemm) {
         if (!n || gate_up->lins.size() != 2 || (gate_up->prompt && c->fp4() && n > FE_X3_ROWS) || !c->bk || (down->q && c->x3())) return false;
         for (auto &l : gate_up->lins)
             if (!l.first->w || (l.first->q && c->x3()) || (l.first->p && c->fp4()) || l.first->k != hidden || l.first->n != inter || l.second.size() != 1) return false;
-        return fe_bf16_gemv_swiglu_takes(c->bk, big, act, xn, gate_up->lins[0].first->w, gate_up->lins[1].first->w, n, inter, hidden, d);
+        return fe_bf16_gemv_swiglu_takes(c->bk, big, act, xn, gate_up->lins[0].first->w, gate_up->lins[1].first->w, n, inter, hidden, d, over_gemm);
     };
     if (pr_rows > FE_X3_ROWS && swiglu && down->p && c->fp4() && act_ws) {
         const fe_devptr_t xn_p = xn + (size_t)d * hidden * 2, x_p = x + (size_t)d * hidden * 2;
@@ -386,7 +386,7 @@ int fe_route_mlp_forward_w(const fe_route_ctx *c, const fe_route_proj *gate_up, 
         FE_TRY(fe_fp4_linear_forward_swiglu(swiglu, c->fk, c->s, c->fws, act_ws, xn_p, hidden, pr_rows, down_g));
         FE_TRY(fe_fp4_linear_gemm(down->p, c->fk, c->s, act_ws, x_p, hidden, pr_rows, x_p));
         fused = true;
-    } else if (pr_rows > FE_X3_ROWS && swiglu_w && c->bk && !pair(rows)) {
+    } else if (pr_rows > FE_X3_ROWS && swiglu_w && c->bk && !pair(rows, true)) {
         // interleaved bf16 gate|up weights: one GEMM with SwiGLU in its epilogue, then down over the prompt rows with the
         // residual (model.rs:3179-3188)
         const fe_devptr_t xn_p = xn + (size_t)d * hidden * 2, x_p = x + (size_t)d * hidden * 2;
@@ -408,7 +408,7 @@ int fe_route_mlp_forward_w(const fe_route_ctx *c, const fe_route_proj *gate_up, 
             return fe_exl3_mlp_forward(g->q, u->q, down->q, c->xk, c->s, xn, FE_DTYPE_BF16, big, big + (size_t)n_rest * inter * 2, x,
                                        FE_DTYPE_BF16_ADD, n_rest, c->xws);
     }
-    if (pair(n_rest)) {
+    if (pair(n_rest, false)) {
         FE_TRY(fe_bf16_gemv_swiglu(c->bk, c->s, act, xn, gate_up->lins[0].first->w, gate_up->lins[1].first->w, n_rest, inter, hidden));
         return linear_forward(down, c, d, x, hidden, act, inter, n_rest, x);
     }

@@ -87,7 +87,7 @@ int fe_route_copy2d(fe_stream_t s, fe_devptr_t dst, uint32_t ldd, fe_devptr_t sr
  * residual; where all of them go through down's trellis linear in one call (a decode batch, or a prompt when down has
  * no other form), SwiGLU is applied as its input rotation reads gate and up (fe_exl3_linear_forward_swiglu: the same bits, act is not written). Up to 64
  * decode rows (and small batches, as fe_bf16_linear_forward takes them) through plain bf16 gate and up, each one part, take one launch for both and SwiGLU (the
- * same bits, big is not written).
+ * same bits, big is not written); a prompt of 17 to 32 rows for which swiglu_w is given (fe_route_mlp_forward_w) only where that launch is ahead of the GEMM over swiglu_w.
  * big: scratch for gate_up's outputs ([rows][total n]); act: scratch [rows][inter]. */
 int fe_route_mlp_forward(const fe_route_ctx *c, const fe_route_proj *gate_up, const fe_route_linear *down,
                          const fe_fp4_linear *swiglu, const fe_fp4_workspace *act_ws, fe_devptr_t x, fe_devptr_t xn,

@@ -44,8 +44,8 @@ int main() {
     const fe_bf16_kernels k;
     const fe_devptr_t big = 0x1000000, act = 0x2000000, x = 0x3000000, gate = 0x4000000, up = 0x5000000;
     fe_set_error(1, "kept", "");
-    for (uint32_t off : {0u, 4u, 16u}) printf("%d", fe_bf16_gemv_swiglu_takes(&k, big + off, act, x, gate, up, 4, 512, 256, 0));
-    printf("%d%d\\n", fe_bf16_gemv_swiglu_takes(&k, big, act, x + 8, gate, up, 4, 512, 256, 0), fe_bf16_gemv_swiglu_takes(&k, big, act, x, 0, up, 4, 512, 256, 0));
+    for (uint32_t off : {0u, 4u, 16u}) printf("%d", fe_bf16_gemv_swiglu_takes(&k, big + off, act, x, gate, up, 4, 512, 256, 0, false));
+    printf("%d%d\\n", fe_bf16_gemv_swiglu_takes(&k, big, act, x + 8, gate, up, 4, 512, 256, 0, false), fe_bf16_gemv_swiglu_takes(&k, big, act, x, 0, up, 4, 512, 256, 0, false));
     printf("%s\\n", fe_hip_last_error());
     const int code = fe_bf16_linear_forward(&k, nullptr, big, 12, x, 96, gate, 0, 1, 12, 96, 0);
     printf("%d %s\\n", code == FE_ERR_SHAPE, fe_hip_last_error());
