@@ -65,7 +65,11 @@ static int check(const char *fn, fe_devptr_t y, uint32_t ldy, fe_devptr_t x, uin
 // 24 / 32 rows, GEMM -> GEMV: 17408 x 5120 40 -> 31, 31, 32; 34816 x 5120 77 -> 58, 79 -> 60, 81 -> 62; 5120 x 5120 17 -> 13, 15, 16; 5120 x 8704 24 -> 19, 21, 23;
 // 8192 x 2048 12.6 -> 8; 1024 x 2816 8.7 -> 5.4, 5.7, 6.1. The line in rows times K is the activations' way from L2 once a program: 4096 x 14336 27 -> 24, 26, 29; 5120 x 17408
 // 38 -> 36, 39, 44; a block of 5120 x 8704 at 32 rows 68 -> 70. From 33 rows on (three groups of 16) the GEMM is ahead wherever K is 5120 and more.
-static bool rows_take_gemv(uint32_t m, uint32_t k, uint32_t dec) { return m <= kSmallBatch || dec >= m || (m <= 32 && (uint64_t)m * k <= (m <= 24 ? 350000 : 180000)); }
+// Operands of 4 GB and more, which the GEMM refuses, stay refused there.
+static bool gemm_reaches(uint32_t m, uint32_t n, uint32_t k, uint32_t lda) { return (uint64_t)m * lda * 2 < (1ull << 32) && (uint64_t)n * k * 2 < (1ull << 32); }
+static bool rows_take_gemv(uint32_t m, uint32_t n, uint32_t k, uint32_t lda, uint32_t dec) {
+    return m <= kSmallBatch || dec >= m || (m <= 32 && (uint64_t)m * k <= (m <= 24 ? 350000 : 180000) && gemm_reaches(k % 256 ? m : m - dec, n, k, lda));
+}
 
 bool fe_bf16_gemv_swiglu_takes(const fe_bf16_kernels *kern, fe_devptr_t big, fe_devptr_t act, fe_devptr_t x, fe_devptr_t gate, fe_devptr_t up, uint32_t m, uint32_t inter,
                                uint32_t k, uint32_t dec, bool over_gemm) {
@@ -73,7 +77,7 @@ bool fe_bf16_gemv_swiglu_takes(const fe_bf16_kernels *kern, fe_devptr_t big, fe_
     // 106, 5120 x 12288 98 -> 84, 4096 x 8192 60 -> 48, but 5120 x 8704 68 -> 71; of 24 rows 66 -> 60. Against gate, up and fe_silu_mul, where there are no such weights, it is ahead
     // there too: 5120 x 8704 at 26 / 32 rows 63.0 -> 58.0, 63.9 -> 58.6, 5120 x 6144 at 30 53.0 -> 48.4, 7168 x 2048 at 25 32.7 -> 28.0)
     if (over_gemm && m > kSmallBatch && dec < m && inter < 12288 && (uint64_t)m * k > 131072) return false;
-    if (!m || m > kGemvPass || !rows_take_gemv(m, k, dec) || !inter || !k || inter % 8 || k % 256 || (uint64_t)m * k * 2 >= (1ull << 32)) return false;
+    if (!m || m > kGemvPass || !rows_take_gemv(m, over_gemm ? 2 * inter : inter, k, k, dec) || !inter || !k || inter % 8 || k % 256 || (uint64_t)m * k * 2 >= (1ull << 32)) return false;
     const char *why;
     if (refusal(big, inter, x, k, gate, 0, inter, k, &why) || refusal(big, inter, x, k, up, 0, inter, k, &why)) return false;
     // programs that are done write act while others read x and the weights
@@ -186,8 +190,7 @@ int fe_bf16_gemm(const fe_bf16_kernels *kern, fe_stream_t s, fe_devptr_t y, uint
     if (!kern) return fe_set_error(FE_ERR_ARG, fn, "null kernels");
     if (m == 0) return 0;
     FE_TRY(check(fn, y, ldy, x, lda, w, res, n, k));
-    if ((uint64_t)m * lda * 2 >= (1ull << 32) || (uint64_t)n * k * 2 >= (1ull << 32))
-        return fe_set_error(FE_ERR_UNSUPPORTED, fn, "operand of 4 GB or more");
+    if (!gemm_reaches(m, n, k, lda)) return fe_set_error(FE_ERR_UNSUPPORTED, fn, "operand of 4 GB or more");
     const uint32_t tiles_m = (m + kTileM - 1) / kTileM;
     uint32_t group = bf16_raster_group(m, n, k, tiles_m);
     if (kern->raster_group >= 0) group = (uint32_t)kern->raster_group;
@@ -225,8 +228,7 @@ int fe_bf16_gemm_swiglu(const fe_bf16_kernels *kern, fe_stream_t s, fe_devptr_t 
     uint32_t n = 2 * inter;
     FE_TRY(check(fn, act, n, x, lda, w, 0, n, k));  // act rows have stride inter = n / 2, a multiple of 8
     if (n % 16) return fe_set_error(FE_ERR_SHAPE, fn, "inter % 8 == 0");
-    if ((uint64_t)m * lda * 2 >= (1ull << 32) || (uint64_t)n * k * 2 >= (1ull << 32))
-        return fe_set_error(FE_ERR_UNSUPPORTED, fn, "operand of 4 GB or more");
+    if (!gemm_reaches(m, n, k, lda)) return fe_set_error(FE_ERR_UNSUPPORTED, fn, "operand of 4 GB or more");
     const uint32_t tiles_m = (m + kTileM - 1) / kTileM;
     uint32_t group = bf16_raster_group(m, n, k, tiles_m);
     if (kern->raster_group >= 0) group = (uint32_t)kern->raster_group;
@@ -253,7 +255,7 @@ int fe_bf16_linear_forward(const fe_bf16_kernels *kern, fe_stream_t s, fe_devptr
     if (m == 0) return 0;
     FE_TRY(check(fn, y, ldy, x, lda, w, res, n, k));
     // decode / verify rows: the GEMV, so that a row's bits do not depend on the batch
-    uint32_t d = rows_take_gemv(m, k, dec) ? m : dec;
+    uint32_t d = rows_take_gemv(m, n, k, lda, dec) ? m : dec;
     if (k % 256) d = 0;
     for (uint32_t r = 0; r < d; r += kGemvPass) {
         const uint32_t mr = d - r < kGemvPass ? d - r : kGemvPass;

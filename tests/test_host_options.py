@@ -53,3 +53,22 @@ int main() {
 """)
     assert lines[:2] == ["10100", "kept:  (1)"]
     assert lines[2].startswith("1 fe_bf16_linear_forward: bf16 linear n 12 k 96 (n % 8 == 0, k % 64 == 0)")
+
+
+def test_what_the_gemm_refuses_stays_refused_at_few_rows(tmp_path):
+    """17 to 32 rows that are no decode rows may go through the GEMV, but not where the GEMM they went through before refuses the operands. (No case here reaches a launch.)"""
+    lines = run_host(tmp_path, "fe_bf16.cpp", """
+int main() {
+    const fe_bf16_kernels k;
+    const fe_devptr_t y = 0x1000000, x = 0x2000000, w = 0x3000000;
+    auto refused = [&](uint32_t n, uint32_t kk, uint32_t lda, uint32_t m, uint32_t dec) {
+        return fe_bf16_linear_forward(&k, nullptr, y, n, x, lda, w, 0, m, n, kk, dec) == FE_ERR_UNSUPPORTED;
+    };
+    printf("%d%d%d\\n", refused(262144, 8192, 8192, 17, 0), refused(524288, 4096, 4096, 32, 0), refused(512, 256, 1u << 27, 17, 0));
+    auto pair = [&](uint32_t m, uint32_t inter, uint32_t kk, uint32_t dec, bool over_gemm) {
+        return fe_bf16_gemv_swiglu_takes(&k, 0x1000, 0x7000000000000ull, x, w, w, m, inter, kk, dec, over_gemm);
+    };
+    printf("%d%d%d%d%d\\n", pair(17, 262144, 8192, 0, false), pair(17, 131072, 8192, 0, true), pair(17, 131072, 8192, 0, false), pair(17, 131064, 8192, 0, true), pair(17, 262144, 8192, 17, false));
+}
+""")
+    assert lines == ["111", "00111"]
