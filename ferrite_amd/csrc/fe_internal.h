@@ -178,6 +178,8 @@ struct FeGemmSchedule {
 // reduce launch and are 1..3 % faster: taken for a small weight operand, (c) below; (d) and (e) below are two more cases
 // of a small weight operand, runs over all tiles behind no whole round.
 // With decoded fp16 tiles or FP8 codes as the weight operand (32 KB a k tile) runs behind whole rounds lose 4..9 %.
+// (NVFP4 up to 2048 rows with more tiles than CUs asks with mode 0: fe_gemm_mode. Of what is said here about more tiles than CUs, the NVFP4 figures up to 2048 rows were taken
+// against a one-piece schedule without lower tiles and with rows that do not exist read again; the rules stand for NVFP4 over 2048 rows and for the trellis GEMM that decodes into LDS.)
 // Needs two partial slots a program and a zeroed counter a tile.
 constexpr uint32_t kFeXcds = 8;
 inline FeGemmSchedule fe_gemm_schedule(uint32_t tiles, uint32_t ktiles, uint32_t cus, fe_devptr_t part, size_t part_bytes,
@@ -324,6 +326,14 @@ inline float fe_gemm_height(const FeGemmCost &c, uint32_t h, const FeGemmSplit &
     return t;
 }
 
+// Stream-K of the forms that have lower tiles, up to 2048 rows: only with fewer tiles than CUs. Behind or over whole rounds, rows that do not exist, the reduce launch and
+// lower tiles cost the one-piece schedule less than the runs' meetings cost (NVFP4, us, stream-K -> one piece: 34816 x 5120 at 400 / 777 / 2048 rows 144 -> 130, 267 -> 242,
+// 531 -> 521; 17408 x 5120 at 777 / 1800 138 -> 130, 273 -> 257; 16384 x 4096 at 1500 182 -> 154; at most 2 % the other way: 12288 x 2048 at 1500 69.0 -> 70.6). With
+// fewer: 34816 x 5120 at 200 rows 94 against 102, 5120 x 17408 at 2048 265 against 277.
+inline int fe_gemm_mode(int mode, uint32_t m, uint32_t tiles256, uint32_t cus, const FeGemmTileOptions &opt) {
+    return mode == 1 && opt.low && m <= 2048 && tiles256 > cus ? 0 : mode;
+}
+
 // The rule: with fewer than a few rounds of 256 x 256 tiles, most of the time is CUs without a tile or pieces of K that meet;
 // tiles of half and a quarter the size fill the chip with fewer pieces. They read more operand bytes and run fewer matrix
 // instructions between two barriers (a k tile of them costs more than its share), so they pay only where the fill gains more:
@@ -337,12 +347,8 @@ inline FeGemmPlan fe_gemm_plan(uint32_t m, uint32_t n, uint32_t ktiles, uint32_t
                                fe_devptr_t counters, size_t counters_len, uint32_t cap, int mode, bool small_b,
                                const FeGemmCost &cost, const FeGemmTileOptions &opt) {
     FeGemmPlan p;
-    // Stream-K of the forms that have lower tiles, up to 2048 rows: only with fewer tiles than CUs. Behind or over whole rounds, rows that do not exist, the reduce launch and
-    // lower tiles cost the one-piece schedule less than the runs' meetings cost (NVFP4, us, stream-K -> one piece: 34816 x 5120 at 400 / 777 / 2048 rows 144 -> 130, 267 -> 242,
-    // 531 -> 521; 17408 x 5120 at 777 / 1800 138 -> 130, 273 -> 257; 16384 x 4096 at 1500 182 -> 154; at most 2 % the other way: 12288 x 2048 at 1500 69.0 -> 70.6). With
-    // fewer: 34816 x 5120 at 200 rows 94 against 102, 5120 x 17408 at 2048 265 against 277.
     const uint32_t tiles256 = ((m + 255) / 256) * ((n + 255) / 256);
-    if (mode == 1 && opt.low && m <= 2048 && tiles256 > cus) mode = 0;
+    mode = fe_gemm_mode(mode, m, tiles256, cus, opt);
     p.big = fe_gemm_schedule(tiles256, ktiles, cus, part, part_bytes, counters, counters_len, cap, mode, small_b);
     auto take = [&](uint32_t tile, uint32_t tiles, uint32_t pieces) { p.tile = tile, p.tiles = tiles, p.splits = pieces; };
     auto tiles_of = [&](uint32_t tile) {

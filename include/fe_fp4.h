@@ -39,7 +39,10 @@ int fe_fp4_kernels_set_option(fe_fp4_kernels *k, const char *name, int32_t value
  * workspace of two partial slots a CU and enough counters: stream_k 0 = one piece a program (whole = tiles computed
  * whole, splits = pieces of each remaining tile, added by a reduce launch), 1 = stream-K (whole = tiles computed whole in
  * rounds, then runs of run (+ 1 for the first run_rem programs) k tiles over the rest). Pure host arithmetic, no GPU
- * call. No counterpart in the reference; for tests and tuners. */
+ * call. No counterpart in the reference; for tests and tuners.
+ * A launch asks with its gemm_sk as mode, with two exceptions. NVFP4 launches of up to 2048 rows with more tiles than CUs ask with mode 0 in the place of 1, and the gate|up
+ * launches with SwiGLU with 0 in the place of 1 at any size. And up to 2048 rows a launch may take other tiles than 256 x 256 (128-row ones; NVFP4, FP8 and bf16 also of 224,
+ * 192 and 160 rows), which this call does not tell. */
 int fe_gemm_schedule_query(uint32_t tiles, uint32_t ktiles, uint32_t cus, int32_t mode, int32_t small_b, uint32_t *stream_k,
                            uint32_t *programs, uint32_t *whole, uint32_t *splits, uint32_t *run, uint32_t *run_rem);
 

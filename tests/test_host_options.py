@@ -72,3 +72,28 @@ int main() {
 }
 """)
     assert lines == ["111", "00111"]
+
+
+def test_the_schedule_query_tells_what_a_launch_asks(tmp_path):
+    """fe_gemm_schedule_query with the mode its comment names is the 256 x 256 schedule of an NVFP4 launch: mode 0 for up to 2048 rows and more tiles than CUs, else 1."""
+    lines = run_host(tmp_path, "fe_fp4.cpp", """
+int main() {
+    uint32_t asked = 0, differ = 0, stream_k[2] = {};
+    for (uint32_t m : {300u, 777u, 1024u, 1536u, 2048u, 2049u, 2304u, 4096u})
+        for (uint32_t n : {5120u, 16384u, 17408u, 34816u})
+            for (uint32_t k : {2048u, 5120u, 17408u}) {
+                const uint32_t tiles = (m + 255) / 256 * ((n + 255) / 256), cus = 256;
+                const int mode = m <= 2048 && tiles > cus ? 0 : 1;
+                FeGemmTileOptions whole{0, 0, true};
+                const FeGemmPlan p = fe_gemm_plan(m, n, k / 64, cus, 1, (size_t)cus * kFeGemmSlotsPerCu * kFeGemmPartBytes, 1, tiles, 8, 1, true, kFeCostNvfp4, whole);
+                if (p.tile) continue;
+                uint32_t sk, programs, full, splits, run, rem;
+                fe_gemm_schedule_query(tiles, k / 64, cus, mode, 1, &sk, &programs, &full, &splits, &run, &rem);
+                asked++, stream_k[mode] += sk;
+                differ += sk != p.big.stream_k || programs != p.big.programs || full != p.big.args.full_tiles || run != p.big.args.sk_base || rem != p.big.args.sk_rem ||
+                          splits != (sk ? 1 : p.big.split.splits);
+            }
+    printf("%d %u %d %d\\n", asked > 20, differ, stream_k[0] == 0, stream_k[1] > 4);
+}
+""")
+    assert lines == ["1 0 1 1"]
