@@ -28,6 +28,9 @@ uint32_t wide_lds(uint32_t xp, uint32_t co, uint32_t waves, bool q = false, uint
 constexpr uint32_t kCuLds = 160 * 1024;
 // The wavefronts of a form: eight where K is summed in eighths and two stages of eight wavefronts fit the LDS.
 uint32_t wide_waves(uint32_t xp, uint32_t co, bool eighths, bool q = false) { return eighths && co <= 6 && (q || xp <= 2 || (xp == 4 && co <= 4)) ? 8 : 4; }
+// Which widths exist: those that a rule or "gemv_cols" may pick. Nine octets pay with 9..16 rows of more columns than six octets a CU; a program of eight wavefronts that
+// quantizes takes two octets rather than one (wide_form).
+constexpr bool wide_built(uint32_t co, bool eighths, bool q) { return co == 9 ? !eighths && !q : co > 1 || !eighths || !q; }
 constexpr uint32_t kGemmThreads = 512;
 constexpr uint32_t kTileM = 256;                        // GM_BM
 }  // namespace
@@ -109,8 +112,9 @@ int fe_fp4_kernels_load(fe_fp4_kernels **out) {
         for (uint32_t j = 0; j < 7; j++) {
             const uint32_t xp = kWideRowForms[i % 4];
             const std::string nm = std::to_string(xp) + "_c" + std::to_string(kWideColForms[j]) + (i / 4 ? "_e" : "");
+            if (!wide_built(kWideColForms[j], i / 4, false)) continue;
             get(&k->wide[i / 4][i % 4][j], "fe_gemv_nvfp4_r" + nm, wide_lds(xp, kWideColForms[j], wide_waves(xp, kWideColForms[j], i / 4)));
-            if (i % 4 < 3) get(&k->wide_q[i / 4][i % 4][j], "fe_gemv_nvfp4_q" + nm, kCuLds);
+            if (i % 4 < 3 && wide_built(kWideColForms[j], i / 4, true)) get(&k->wide_q[i / 4][i % 4][j], "fe_gemv_nvfp4_q" + nm, kCuLds);
         }
     for (uint32_t i = 0; i < 5; i++)
         for (uint32_t j = 0; j < 7; j++) {
@@ -404,7 +408,8 @@ static WideForm wide_form(const fe_fp4_linear *l, const fe_fp4_kernels *kern, ui
     const uint32_t form = m <= 2 ? 0 : m <= 4 ? 1 : m <= 8 ? 2 : 3, xp = kWideRowForms[form], cus = std::max(kern->cus, 1u);
     const bool eighths = l->k >= 2048 && l->n <= 48 * cus;
     uint32_t cols = wide_cols(l->n, xp, cus, kern->gemv_cols, q, m, l->k);
-    if (q && eighths && !cols && !kern->gemv_cols) cols = 1;
+    if (cols == 6 && !wide_built(9, eighths, q)) cols = 5;  // (only where gemv_cols asks for 72)
+    if (cols == 0 && !wide_built(1, eighths, q)) cols = 1;
     const uint32_t co = kWideColForms[cols], waves = wide_waves(xp, co, eighths, q);
     return {(l->n / 8 + co - 1) / co, waves, wide_lds(xp, co, waves, q, m, l->k), (q ? kern->wide_q[eighths][form] : kern->wide[eighths][form])[cols]};
 }

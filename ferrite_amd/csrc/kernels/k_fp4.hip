@@ -1242,24 +1242,24 @@ __device__ __forceinline__ void gemv_nvfp4_wide_body(uint16_t* c, const _Float16
         gemv_nvfp4_wide_body<XP, CO, true, WV, EIGHTHS>(c, x, w, sw, alpha, res, m, n, k, ldc, w_snt, w_skt, w_sr, s_snt, s_skt, s_sr, qt); \
     }
 // "": quarters of K. "_e": eighths, by eight wavefronts where two stages of eight fit the LDS, else by four.
-#define FP4_WIDE_SIX(KERNEL, XP, SUFFIX, WV, EIGHTHS) \
-    KERNEL(XP, 1, SUFFIX, WV, EIGHTHS) KERNEL(XP, 2, SUFFIX, WV, EIGHTHS) KERNEL(XP, 3, SUFFIX, WV, EIGHTHS) KERNEL(XP, 4, SUFFIX, WV, EIGHTHS) KERNEL(XP, 5, SUFFIX, WV, EIGHTHS) KERNEL(XP, 6, SUFFIX, WV, EIGHTHS)
-#define FP4_WIDE_FAMILY(KERNEL, XP) FP4_WIDE_SIX(KERNEL, XP, , 4, false) KERNEL(XP, 9, , 4, false) KERNEL(XP, 9, _e, 4, true)
-FP4_WIDE_FAMILY(FP4_WIDE_KERNEL, 1)
-FP4_WIDE_FAMILY(FP4_WIDE_KERNEL, 2)
-FP4_WIDE_FAMILY(FP4_WIDE_KERNEL, 4)
-FP4_WIDE_FAMILY(FP4_WIDE_KERNEL, 8)
-FP4_WIDE_FAMILY(FP4_WIDE_QUANT_KERNEL, 1)
-FP4_WIDE_FAMILY(FP4_WIDE_QUANT_KERNEL, 2)
-FP4_WIDE_FAMILY(FP4_WIDE_QUANT_KERNEL, 4)
+#define FP4_WIDE_FIVE(KERNEL, XP, SUFFIX, WV, EIGHTHS) \
+    KERNEL(XP, 2, SUFFIX, WV, EIGHTHS) KERNEL(XP, 3, SUFFIX, WV, EIGHTHS) KERNEL(XP, 4, SUFFIX, WV, EIGHTHS) KERNEL(XP, 5, SUFFIX, WV, EIGHTHS) KERNEL(XP, 6, SUFFIX, WV, EIGHTHS)
+#define FP4_WIDE_SIX(KERNEL, XP, SUFFIX, WV, EIGHTHS) KERNEL(XP, 1, SUFFIX, WV, EIGHTHS) FP4_WIDE_FIVE(KERNEL, XP, SUFFIX, WV, EIGHTHS)
+FP4_WIDE_SIX(FP4_WIDE_KERNEL, 1, , 4, false) FP4_WIDE_KERNEL(1, 9, , 4, false)
+FP4_WIDE_SIX(FP4_WIDE_KERNEL, 2, , 4, false) FP4_WIDE_KERNEL(2, 9, , 4, false)
+FP4_WIDE_SIX(FP4_WIDE_KERNEL, 4, , 4, false) FP4_WIDE_KERNEL(4, 9, , 4, false)
+FP4_WIDE_SIX(FP4_WIDE_KERNEL, 8, , 4, false) FP4_WIDE_KERNEL(8, 9, , 4, false)
+FP4_WIDE_SIX(FP4_WIDE_QUANT_KERNEL, 1, , 4, false)
+FP4_WIDE_SIX(FP4_WIDE_QUANT_KERNEL, 2, , 4, false)
+FP4_WIDE_SIX(FP4_WIDE_QUANT_KERNEL, 4, , 4, false)
 FP4_WIDE_SIX(FP4_WIDE_KERNEL, 1, _e, 8, true)
 FP4_WIDE_SIX(FP4_WIDE_KERNEL, 2, _e, 8, true)
 FP4_WIDE_KERNEL(4, 1, _e, 8, true) FP4_WIDE_KERNEL(4, 2, _e, 8, true) FP4_WIDE_KERNEL(4, 3, _e, 8, true) FP4_WIDE_KERNEL(4, 4, _e, 8, true)
 FP4_WIDE_KERNEL(4, 5, _e, 4, true) FP4_WIDE_KERNEL(4, 6, _e, 4, true)
 FP4_WIDE_SIX(FP4_WIDE_KERNEL, 8, _e, 4, true)
-FP4_WIDE_SIX(FP4_WIDE_QUANT_KERNEL, 1, _e, 8, true)
-FP4_WIDE_SIX(FP4_WIDE_QUANT_KERNEL, 2, _e, 8, true)
-FP4_WIDE_SIX(FP4_WIDE_QUANT_KERNEL, 4, _e, 8, true)
+FP4_WIDE_FIVE(FP4_WIDE_QUANT_KERNEL, 1, _e, 8, true)
+FP4_WIDE_FIVE(FP4_WIDE_QUANT_KERNEL, 2, _e, 8, true)
+FP4_WIDE_FIVE(FP4_WIDE_QUANT_KERNEL, 4, _e, 8, true)
 
 // ---- matrix-unit peak probe ---------------------------------------------------------------------------------------------
 //

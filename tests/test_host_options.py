@@ -97,3 +97,33 @@ int main() {
 }
 """)
     assert lines == ["1 0 1 1"]
+
+
+def test_every_wide_form_of_nvfp4_is_one_that_a_rule_or_an_option_reaches(tmp_path):
+    """The GEMV of 1..16 rows: whatever the shape, the rows and gemv_cols, the form picked is one that is built, and each that is built is picked somewhere."""
+    lines = run_host(tmp_path, "fe_fp4.cpp", """
+int main() {
+    fe_fp4_kernels K;
+    K.cus = 256;
+    size_t built = 0, picked = 0, missing = 0;
+    bool seen[2][2][4][7] = {};
+    for (int q = 0; q < 2; q++)
+        for (int e = 0; e < 2; e++)
+            for (int i = 0; i < (q ? 3 : 4); i++)
+                for (int j = 0; j < 7; j++)
+                    if (wide_built(kWideColForms[j], e, q)) built++, (q ? K.wide_q[e][i] : K.wide[e][i])[j] = (fe_function_t)(size_t)(1 + ((q * 2 + e) * 4 + i) * 7 + j);
+    fe_fp4_linear l;
+    for (uint32_t cols : {0u, 8u, 16u, 24u, 32u, 40u, 48u, 72u, 1000u})
+        for (uint32_t n = 128; n < 120000; n += n < 20000 ? 256 : 8192)
+            for (uint32_t k : {256u, 1792u, 2048u, 5120u, 17408u})
+                for (uint32_t m = 1; m <= 16; m++)
+                    for (int q = 0; q < (m <= 8 ? 2 : 1); q++) {
+                        l.n = n, l.k = k, K.gemv_cols = cols;
+                        const size_t f = (size_t)wide_form(&l, &K, m, q).f;
+                        if (!f) missing++;
+                        else if (bool &s = (&seen[0][0][0][0])[f - 1]; !s) s = true, picked++;
+                    }
+    printf("%zu %d\\n", missing, picked == built);
+}
+""")
+    assert lines == ["0 1"]
