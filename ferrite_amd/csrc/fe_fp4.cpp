@@ -26,6 +26,7 @@ uint32_t wide_lds(uint32_t xp, uint32_t co, uint32_t waves, bool q = false, uint
     return std::max(waves * std::max(2u, std::min((q ? 60 : 80) * 1024 / (waves * stage), 6u)) * stage + x, 64 * waves * (16 * cg + 4));
 }
 constexpr uint32_t kCuLds = 160 * 1024;
+constexpr uint32_t kQuantValues = 10240;
 // The wavefronts of a form: eight where K is summed in eighths and two stages of eight wavefronts fit the LDS.
 uint32_t wide_waves(uint32_t xp, uint32_t co, bool eighths, bool q = false) { return eighths && co <= 6 && (q || xp <= 2 || (xp == 4 && co <= 4)) ? 8 : 4; }
 // Which widths exist: those that a rule or "gemv_cols" may pick. Nine octets pay with 9..16 rows of more columns than six octets a CU; a program of eight wavefronts that
@@ -52,8 +53,9 @@ struct fe_fp4_kernels {
     uint32_t gemv = 1;         // few rows run the GEMV (takes_gemv, fp8_gemv_rows; FE_FP4_NO_GEMV=1: the GEMM's single tile row)
     uint32_t gemv_sk = 0;      // K splits of the GEMV over weight tiles; 0 = two programs a CU (FE_FP4_GEMV_SK)
     uint32_t gemv_strips = 1;  // up to 16 rows run programs of some columns over all of K; 0: weight tiles and K splits, as more rows do (FE_FP4_NO_STRIPS=1)
-    // most values (rows x k) that the four wavefronts of the GEMV for up to 16 rows quantize themselves, in every program; eight take twice as many (FE_FP4_GEMV_QUANT)
-    uint32_t gemv_quant = 10240;
+    // most values (rows x k) that the four wavefronts of the GEMV for up to 16 rows quantize themselves, in every program; eight take twice as many; -1: by the shape, at most
+    // kQuantValues (FE_FP4_GEMV_QUANT)
+    int32_t gemv_quant = -1;
     uint32_t gemv_cols = 0;    // columns a program of the GEMV for up to 16 rows, or of the FP8 GEMV, takes, rounded up to 8, 16, .. 48, 72; 0 = by the shape (FE_FP4_GEMV_COLS)
     int32_t xcd = -1;          // column tiles dealt to the XCDs: -1 = where the weights are the larger operand (FE_FP4_XCD)
     uint32_t fp8_f16 = 0;      // FP8 linears as fp16 expansion on the 16-bit matrix instruction (FE_FP8_F16=1)
@@ -130,7 +132,7 @@ int fe_fp4_kernels_load(fe_fp4_kernels **out) {
     if (const char *e = getenv("FE_FP4_NO_GEMV")) k->gemv = atoi(e) ? 0 : 1;
     if (const char *e = getenv("FE_FP4_GEMV_SK")) k->gemv_sk = (uint32_t)atoi(e);
     if (const char *e = getenv("FE_FP4_NO_STRIPS")) k->gemv_strips = atoi(e) ? 0 : 1;
-    if (const char *e = getenv("FE_FP4_GEMV_QUANT")) k->gemv_quant = (uint32_t)atoi(e);
+    if (const char *e = getenv("FE_FP4_GEMV_QUANT")) k->gemv_quant = atoi(e);
     if (const char *e = getenv("FE_FP4_GEMV_COLS")) k->gemv_cols = (uint32_t)atoi(e);
     if (const char *e = getenv("FE_FP4_XCD")) k->xcd = atoi(e) ? 1 : 0;
     if (const char *e = getenv("FE_FP8_F16")) k->fp8_f16 = atoi(e) ? 1 : 0;
@@ -157,7 +159,7 @@ int fe_fp4_kernels_set_option(fe_fp4_kernels *k, const char *name, int32_t value
     if (nm == "group_m") k->group_m = (uint32_t)value;
     else if (nm == "gemv") k->gemv = value ? 1 : 0;
     else if (nm == "gemv_sk") k->gemv_sk = (uint32_t)value;
-    else if (nm == "gemv_quant") k->gemv_quant = (uint32_t)value;
+    else if (nm == "gemv_quant") k->gemv_quant = value;
     else if (nm == "gemv_cols") k->gemv_cols = value;
     else if (nm == "gemv_strips") k->gemv_strips = (uint32_t)value;
     else if (nm == "gemv_once" || nm == "gemv_waves") (void)value;  // of a kernel that is no more: accepted, without effect
@@ -545,13 +547,21 @@ int fe_fp4_linear_gemm(const fe_fp4_linear *l, const fe_fp4_kernels *kern, fe_st
 // quantizer's launch -> without: 1024 x 1024 at 1 / 8 rows 6.9 -> 3.8, 7.1 -> 4.1; 5120 x 5120 at 1 / 2 rows 8.7 -> 7.3, 8.9 -> 8.0; 17408 x 5120 at 1 / 2 15.8 -> 14.0,
 // 16.2 -> 14.5; 34816 x 5120 at 2 24.7 -> 23.7; 16384 x 2560 at 4 9.3 -> 8.3; 5120 x 8704 at 1 11.5 -> 10.0. Beyond 10240 values it turns: 34816 x 5120 at 3 rows
 // 25.2 -> 27.0, 16384 x 2560 at 6 10.2 -> 14.3 (one program a CU). Eight wavefronts quantize twice as many in that time: 5120 x 17408 at 1 row 17.2 -> 15.9, 4096 x 4096 at
-// 4 6.7 -> 5.8, 1024 x 5120 at 4 / 5 (25600 values) 6.7 -> 6.8, 7.1 -> 7.9. Up to 8 rows, what the LDS holds and 32 bits address. Not where the output or the
+// 4 6.7 -> 5.8, 1024 x 5120 at 4 / 5 (25600 values) 6.7 -> 6.8, 7.1 -> 7.9. What it costs is a wavefront's turns (64 blocks each) times the rounds of programs, each of which
+// quantizes again: of 268 shapes (1024 .. 152064 columns, 1 to 8 rows), by values alone 0.934 of the time, 51 more than 2 % slower, at most 36 % (152064 x 1280 at 8 rows 35.7 -> 48.4,
+// 152064 x 5120 at 1 74.6 -> 82.3, 16384 x 1280 at 8 7.8 -> 8.6); with at most three turns, five times the rounds, 0.918, three more than 2 %, at most 4 % (1024 columns; the better
+// of both 0.916). Inputs that no cache holds or that the last call read: the same within 2 %. Up to 8 rows, what the LDS holds and 32 bits address. Not where the output or the
 // workspace lies in the activations' memory: programs that have finished would write over what others have yet to read.
 static bool fp4_quants_itself(const fe_fp4_linear *l, const fe_fp4_kernels *kern, const fe_fp4_workspace *ws, fe_devptr_t y, uint32_t ldy, fe_devptr_t x,
                               uint32_t lda, uint32_t m) {
     if (!m || m > 8 || !takes_wide(l, kern, m) || (uint64_t)m * lda >= (1u << 30)) return false;
     const WideForm f = wide_form(l, kern, m, true);
-    if ((uint64_t)m * l->k > std::min<uint64_t>((uint64_t)kern->gemv_quant * f.waves / 4, 32768) || f.lds > kCuLds) return false;
+    const uint64_t most = kern->gemv_quant < 0 ? kQuantValues : (uint64_t)kern->gemv_quant;
+    if ((uint64_t)m * l->k > std::min<uint64_t>(most * f.waves / 4, 32768) || f.lds > kCuLds) return false;
+    if (kern->gemv_quant < 0) {
+        const uint32_t turns = ((l->k / 256 + f.waves - 1) / f.waves * m + 3) / 4, at_once = (f.lds <= kCuLds / 2 ? 2 : 1) * std::max(kern->cus, 1u);
+        if (turns > 3 || turns * std::max(at_once, f.programs) > 5 * at_once) return false;
+    }
     const fe_devptr_t xe = x + ((size_t)(m - 1) * lda + l->k) * 2;
     auto apart = [&](fe_devptr_t p, size_t bytes) { return p + bytes <= x || p >= xe; };
     return apart(y, ((size_t)(m - 1) * ldy + l->n) * 2) && apart(ws->codes.p, ws->codes.bytes) && apart(ws->sf.p, ws->sf.bytes) && apart(ws->aq.p, ws->aq.bytes);

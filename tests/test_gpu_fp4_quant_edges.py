@@ -30,3 +30,16 @@ def test_infinities_against_every_multiplier(oracle, g, inside):
     plain = lambda c: np.where(c & 7, c, 0)
     for a, b in ((codes & 15, want & 15), (codes >> 4, want >> 4)):
         assert np.array_equal(plain(a), plain(b))
+
+
+@pytest.mark.parametrize("n,k,m", [(128, 256, 1), (640, 2304, 3), (256, 17408, 1), (1152, 4096, 8)])
+def test_the_option_says_where_the_quantizer_runs(n, k, m):
+    """One kernel where the GEMV's programs quantize, two with the quantizer's own launch: the two sides that the comparisons of bits set against each other."""
+    import torch
+    from ferrite_amd import fp4, synth
+    from test_gpu_launch_counts import kernels_recorded
+    kern, ws, lin = fp4.Kernels.load(), fp4.Workspace(m, k), synth.fp4_linear(n, k, 1).upload()
+    x, y = torch.zeros((m, k), dtype=torch.bfloat16, device="cuda"), torch.zeros((m, n), dtype=torch.bfloat16, device="cuda")
+    for limit, kernels in ((32768, 1), (0, 2)):
+        kern.set_option("gemv_quant", limit)
+        assert kernels_recorded(torch, lambda: lin.forward(kern, ws, y, n, x, k, m)) == kernels

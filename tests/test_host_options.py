@@ -127,3 +127,28 @@ int main() {
 }
 """)
     assert lines == ["0 1"]
+
+
+# (columns, K, rows): us with the quantizer's launch and with every program quantizing all of the activations
+QUANT = {(152064, 1280, 8): (35.7, 48.4), (98304, 1280, 8): (25.4, 33.2), (65536, 2560, 4): (23.3, 27.5), (152064, 5120, 1): (74.6, 82.3), (65536, 5120, 2): (34.7, 38.6),
+         (16384, 1280, 8): (7.8, 8.6), (28672, 1280, 8): (11.8, 13.5), (24576, 1280, 8): (10.9, 13.7), (1024, 2560, 8): (6.4, 7.1), (5120, 2560, 8): (7.9, 8.5),
+         (5120, 5120, 1): (8.5, 6.7), (17408, 5120, 1): (13.9, 12.5), (34816, 5120, 2): (22.2, 21.1), (5120, 17408, 1): (14.6, 14.0), (24576, 512, 8): (8.4, 5.4),
+         (28672, 1024, 2): (9.6, 7.1), (4096, 4096, 5): (7.2, 6.9), (40960, 5120, 1): (26.2, 25.2), (1024, 1024, 8): (5.1, 4.1)}
+
+
+def test_programs_quantize_only_where_that_was_timed_faster(tmp_path):
+    calls = ", ".join("{%du, %du, %du}" % c for c in QUANT)
+    lines = run_host(tmp_path, "fe_fp4.cpp", f"""
+int main() {{
+    fe_fp4_kernels K;
+    K.cus = 256;
+    fe_fp4_linear l;
+    fe_fp4_workspace ws;
+    const uint32_t calls[][3] = {{{calls}}};
+    for (auto &c : calls) {{
+        l.n = c[0], l.k = c[1];
+        printf("%d\\n", fp4_quants_itself(&l, &K, &ws, 0x1000000, l.n, 0x2000000000ull, l.k, c[2]));
+    }}
+}}
+""")
+    assert [int(v) for v in lines] == [int(inside < launch) for launch, inside in QUANT.values()]
