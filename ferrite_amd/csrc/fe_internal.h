@@ -350,7 +350,7 @@ inline FeGemmPlan fe_gemm_plan(uint32_t m, uint32_t n, uint32_t ktiles, uint32_t
     const uint32_t tiles256 = ((m + 255) / 256) * ((n + 255) / 256);
     mode = fe_gemm_mode(mode, m, tiles256, cus, opt);
     p.big = fe_gemm_schedule(tiles256, ktiles, cus, part, part_bytes, counters, counters_len, cap, mode, small_b);
-    auto take = [&](uint32_t tile, uint32_t tiles, uint32_t pieces) { p.tile = tile, p.tiles = tiles, p.splits = pieces; };
+    auto take = [&](uint32_t tile, uint32_t tiles, uint32_t pieces) { p.tile = tile, p.tiles = tiles, p.splits = pieces, p.big.stream_k = false; };
     auto tiles_of = [&](uint32_t tile) {
         return ((m + kFeGemmTileM[tile] - 1) / kFeGemmTileM[tile]) * ((n + kFeGemmTileN[tile] - 1) / kFeGemmTileN[tile]);
     };
@@ -384,22 +384,21 @@ inline FeGemmPlan fe_gemm_plan(uint32_t m, uint32_t n, uint32_t ktiles, uint32_t
     // their time). By the ratio of the two estimates, which share most of their errors. Of 336 launches (8 layers, 14 row counts, NVFP4, FP8 and bf16) against 256 rows:
     // 0.925, 0.93, 0.905 of the time (the best height each time: 0.92, 0.92, 0.90), four more than 2 % slower, at most 7 %. With the small tiles in the choice, 12 other layers
     // of 144 launches a form against the rule without lower tiles: 0.93, 0.97, 0.93; 8 of 432 more than 3 % slower, at most 7 %.
+    uint32_t pick = 0;
+    float ratio = p.big.stream_k ? 0.9f : 0.97f;
     if (opt.low && m <= 2048) {
         const uint32_t tiles_n = (n + 255) / 256;
         auto height = [&](uint32_t tile, uint32_t h, const FeGemmSplit &g) { return fe_gemm_height(cost, h, g, ktiles, cus, m / (tiles_of(tile) / tiles_n)); };
         const float high = height(0, 0, p.big.split);
-        float ratio = p.big.stream_k ? 0.9f : 0.97f;
-        uint32_t pick = 0;
         for (uint32_t tile = 3; tile < kFeGemmTiles; tile++) {
             const FeGemmSplit g = low(tile).split;
             float r = height(tile, tile - 2, g) / high;
             if (2 * g.programs() < cus) r = std::max(r, 0.85f);  // (mostly idle CUs: a k tile takes the trip of its loads, at any height)
             if (r < ratio) ratio = r, pick = tile;
         }
-        if (pick) p.tile = pick, p.big = low(pick), best *= ratio;
     }
+    const float whole = best;
     p.us = best;
-    const float margin = p.tile && !small_b ? 1.0f : 1.06f;  // (bf16 and FP8: what a lower tile gained is part of that margin)
     for (uint32_t tile = 1; tile <= 2 && m <= 2048; tile++) {
         const uint32_t tiles = tiles_of(tile), most = most_pieces(tile, std::min(cap, ktiles / 8));
         for (uint32_t pieces = 1; pieces <= most; pieces++) {
@@ -407,9 +406,20 @@ inline FeGemmPlan fe_gemm_plan(uint32_t m, uint32_t n, uint32_t ktiles, uint32_t
             float c = fe_gemm_cost(cost, tile, tiles * pieces, (ktiles + pieces - 1) / pieces, cus);
             if (pieces > 1) c += fe_gemm_reduce_cost(tiles * pieces, tile);
             if (tiles * pieces > cus * tile) c *= cost.again;
-            if (margin * c < best) take(tile, tiles, pieces), p.us = c, best = margin * c;
+            if (1.06f * c < best) take(tile, tiles, pieces), p.us = c, best = 1.06f * c;
         }
     }
+    if (!pick) return p;
+    // In the place of a small tile a lower one is taken only with at least 12 k tiles and half of the CUs: the heights' estimate has no fixed part and was fitted on launches
+    // that fill the chip. Of 1499 launches (128 .. 40000 columns, K 256 .. 20000, 65 .. 2048 rows; NVFP4, its SwiGLU front, FP8, bf16) against the rule without lower tiles:
+    // with them wherever the estimate says so 68 more than 3 % slower (5248 x 256 at 636 rows 9.2 -> 13.1 us, 7168 x 256 SwiGLU at 140 13.4 -> 25.6, 256 x 1536 bf16 at
+    // 210 7.8 -> 10.3, 11136 x 256 FP8 at 315 9.1 -> 11.6) and 0.986 / 0.983 / 0.998 / 0.993 of the time in all; so 11, at most 6 %, and 0.980 / 0.979 / 0.991 / 0.989.
+    const FeGemmSchedule lower = low(pick);
+    if (p.tile) {
+        if (ktiles < 12 || 2 * lower.split.programs() < cus) return p;
+        if ((small_b ? 1.06f : 1.0f) * p.us < whole * ratio) return p;  // (bf16 and FP8: what a lower tile gained is part of that margin)
+    }
+    p.tile = pick, p.tiles = 0, p.splits = 1, p.big = lower, p.us = whole * ratio;
     return p;
 }
 

@@ -152,3 +152,27 @@ int main() {{
 }}
 """)
     assert [int(v) for v in lines] == [int(inside < launch) for launch, inside in QUANT.values()]
+
+
+# (form, rows, columns, K): us of a small tile (128 x 256 or 128 x 128) and of the lower one that the heights' estimate names in its place
+LOWER = {("nvfp4", 636, 5248, 256): (9.2, 13.1), ("nvfp4", 449, 768, 1536): (14.9, 18.3), ("nvfp4", 163, 256, 2560): (12.1, 14.7),
+         ("fp8", 315, 11136, 256): (9.1, 11.6), ("fp8", 584, 6784, 512): (11.2, 13.8), ("fp8", 180, 1024, 4864): (15.8, 18.5),
+         ("bf16", 210, 256, 1536): (7.8, 10.3), ("bf16", 228, 25984, 256): (9.4, 10.4), ("bf16", 79, 512, 1792): (8.2, 9.7),
+         ("nvfp4", 1686, 5888, 4096): (102.1, 83.7), ("nvfp4", 774, 37248, 2816): (188.2, 162.4), ("fp8", 868, 9856, 3584): (51.4, 43.4),
+         ("bf16", 1423, 5888, 2048): (47.3, 37.6), ("bf16", 721, 25984, 1280): (67.4, 57.7)}
+
+
+def test_a_lower_tile_takes_a_small_ones_place_where_that_was_timed_faster(tmp_path):
+    calls = ", ".join('{"%s", %d, %d, %d}' % c for c in LOWER)
+    lines = run_host(tmp_path, "fe_fp4.cpp", f"""
+int main() {{
+    struct {{ const char *form; uint32_t m, n, k; }} calls[] = {{{calls}}};
+    for (auto &c : calls) {{
+        const bool f8 = c.form[0] == 'f', bf = c.form[0] == 'b';
+        const FeGemmPlan p = fe_gemm_plan(c.m, c.n, c.k / (f8 ? 128 : 64), 256, 1, (size_t)512 * kFeGemmPartBytes, 1, 8192, 8, bf ? 0 : 1, !f8 && !bf,
+                                          f8 ? kFeCostFp8 : bf ? kFeCostBf16 : kFeCostNvfp4, FeGemmTileOptions{{0, 0, true}});
+        printf("%d\\n", p.tile >= 3 ? 1 : p.tile ? 0 : 2);
+    }}
+}}
+""")
+    assert [int(v) for v in lines] == [int(lower < small) for small, lower in LOWER.values()]
