@@ -50,7 +50,7 @@ struct fe_fp4_kernels {
     // Switches of the launch paths: read from the environment once, at load; fe_fp4_kernels_set_option changes them
     // afterwards. No forward call reads the environment.
     uint32_t group_m = 8;      // raster group height in row tiles; 0 = all (FE_FP4_GROUP, lib.rs:31-32, 68)
-    uint32_t gemv = 1;         // few rows run the GEMV (takes_gemv, fp8_gemv_rows; FE_FP4_NO_GEMV=1: the GEMM's single tile row)
+    uint32_t gemv = 1;         // few rows run the GEMV (takes_gemv, fe_gemv_ahead; FE_FP4_NO_GEMV=1: the GEMM's single tile row)
     uint32_t gemv_sk = 0;      // K splits of the GEMV over weight tiles; 0 = two programs a CU (FE_FP4_GEMV_SK)
     uint32_t gemv_strips = 1;  // up to 16 rows run programs of some columns over all of K; 0: weight tiles and K splits, as more rows do (FE_FP4_NO_STRIPS=1)
     // most values (rows x k) that the four wavefronts of the GEMV for up to 16 rows quantize themselves, in every program; eight take twice as many; -1: by the shape, at most
@@ -440,11 +440,6 @@ static uint32_t gemv_splits(const fe_fp4_kernels *kern, const fe_fp4_workspace *
     return std::max(sk, 1u);
 }
 
-// Most rows that an FP8 linear takes through its GEMV. us, GEMM -> GEMV at 1 / 17 / 32 / 64 rows: 17408 x 5120 24.4 -> 15.1, 25.2 -> 16.1, 25.8 -> 17.4, 27.7 -> 27.1; 5120 x
-// 5120 12.0 -> 6.1, 12.5 -> 8.3, 12.7 -> 8.5, 13.3 -> 11.0; 1024 x 2816 9.7 -> 3.9, 10.2 -> 3.8, 10.2 -> 4.2, 10.7 -> 5.7; 4096 x 14336 21.2 -> 10.8, 19.8 -> 13.1, 20.0 -> 15.3,
-// 21.2 -> 21.1; 5120 x 17408 25.4 -> 15.8, 24.0 -> 18.2, 24.3 -> 22.1, but 25.2 -> 25.6 at 48 and 26.0 -> 28.2 at 64 (the activations' way from L2 once a program).
-static uint32_t fp8_gemv_rows(uint32_t k) { return k <= 14336 ? 64 : 40; }
-
 // x: null, or the activations (bf16 rows of lda) which that GEMV quantizes itself
 static int linear_gemm(const fe_fp4_linear *l, const fe_fp4_kernels *kern, fe_stream_t s, const fe_fp4_workspace *ws, fe_devptr_t y, uint32_t ldy,
                        uint32_t m, fe_devptr_t res, fe_devptr_t x, uint32_t lda) {
@@ -493,17 +488,19 @@ static int linear_gemm(const fe_fp4_linear *l, const fe_fp4_kernels *kern, fe_st
     // FP8 runs on the 8-bit matrix instruction over the codes of both operands, k tiles of 128 (FE_FP8_F16=1: the fp16
     // expansion on the 16-bit instruction, k tiles of 64; same products, another order of the f32 sums)
     const bool codes8 = l->fp8 && !kern->fp8_f16;
-    if (codes8 && kern->gemv && !kern->tile.force_tile && kern->gemm_sk < 2 && m <= fp8_gemv_rows(k)) {
+    const FeGemmTileOptions f16_form{1, 0, false};  // (the fp16 form exists for 256 x 256 tiles only)
+    const bool few = codes8 && kern->gemv && !kern->tile.force_tile && kern->gemm_sk < 2 && m <= kGemvMaxRows;
+    FeGemmPlan plan;
+    if (!few || m > kFeGemvFp8.always)
+        plan = fe_gemm_plan(m, n, codes8 ? k / 128 : k / 64, kern->cus, ws->part.p, ws->part.bytes, ws->counters.p, kGemvCounters, kern->gemm_splits, kern->gemm_sk, /*small_b=*/!l->fp8,
+                            l->fp8 ? kFeCostFp8 : kFeCostNvfp4, l->fp8 && !codes8 ? f16_form : kern->tile);
+    if (few && fe_gemv_ahead(kFeGemvFp8, m, n, k, k / 128, std::max(kern->cus, 1u), 4, plan)) {
         const uint32_t form = gemv_row_form(m), xo = kGemvRowForms[form], cols = gemv_cols(std::max(m, 3u), n, k, xo, std::max(kern->cus, 1u), kern->gemv_cols ? (int32_t)kern->gemv_cols : -1), co = kGemvColForms[cols];
         fe_devptr_t codes = ws->codes.p;
         uint32_t pc = gemv_even(n, 8 * co, std::max(kern->cus, 1u), 4, kern->gemv_cols != 0 || m <= 2);
         void *args[] = {&y, &codes, &w, &alpha, &res, &m, &n, &k, &ldy, &w_snt, &w_skt, &w_sr, &pc};
         return fe_hip_launch(kern->gemv8[form][cols], (n + pc - 1) / pc, 1, 1, 256, 1, 1, gemv_lds(xo, co), s, args);
     }
-    const FeGemmTileOptions f16_form{1, 0, false};  // (the fp16 form exists for 256 x 256 tiles only)
-    const FeGemmPlan plan = fe_gemm_plan(m, n, codes8 ? k / 128 : k / 64, kern->cus, ws->part.p, ws->part.bytes, ws->counters.p, kGemvCounters,
-                                         kern->gemm_splits, kern->gemm_sk, /*small_b=*/!l->fp8,
-                                         l->fp8 ? kFeCostFp8 : kFeCostNvfp4, l->fp8 && !codes8 ? f16_form : kern->tile);
     if (l->fp8 && !codes8) {
         uint32_t count = m * k;
         fe_devptr_t codes = ws->codes.p;

@@ -571,3 +571,25 @@ inline uint32_t gemv_cols(uint32_t m, uint32_t n, uint32_t k, uint32_t xo, uint3
     if (nc <= 0 && m <= 2 && best > 4) best = 2;
     return best;
 }
+
+// Whether a GEMV over programs of columns is ahead of the GEMM that would run in its place, by an estimate of both (us). The GEMV's: a start, rounds of programs, the weights'
+// way from HBM, the activations' way from L2 once a program (the CU with the most) and the outputs. The GEMM's: its plan's estimate and what that leaves out at so few rows, the
+// weights' way; pieces of K cost less than it says. margin: on what the GEMM takes. Up to `always` rows the GEMV in any case.
+struct FeGemvLine {
+    uint32_t always;
+    float start, round, w, x, out, gemm_start, gemm_us, gemm_w, gemm_cut, gemm_pieces, margin;
+};
+inline bool fe_gemv_ahead(const FeGemvLine &c, uint32_t m, uint32_t n, uint32_t k, uint32_t steps, uint32_t cus, uint32_t even_step, const FeGemmPlan &gemm) {
+    if (m <= c.always) return true;
+    const uint32_t xo = kGemvRowForms[gemv_row_form(m)], co = kGemvColForms[gemv_cols(m, n, k, xo, cus, -1)], pc = gemv_even(n, 8 * co, cus, even_step, false);
+    const uint32_t programs = (n + pc - 1) / pc, at_once = (gemv_lds(xo, co) <= 80 * 1024 ? 2 : 1) * cus, a_cu = (programs + cus - 1) / cus;
+    const uint32_t pieces = gemm.tile == 1 || gemm.tile == 2 ? gemm.splits : gemm.big.split.splits;
+    const float weights = (float)n * (float)steps;
+    const float gemv = c.start + c.round * (float)((programs + at_once - 1) / at_once) + c.w * weights + c.x * (float)(a_cu * 8 * xo) * (float)steps + c.out * (float)m * (float)n;
+    return gemv <= c.margin * (c.gemm_start + c.gemm_us * gemm.us + c.gemm_w * weights - (pieces > 1 ? c.gemm_cut + c.gemm_pieces * (float)pieces * (float)n : 0.0f));
+}
+// FP8 (steps of 128 codes), up to 64 rows. Fitted to 2786 calls of 9..64 rows (128 .. 40000 columns, K 256 .. 20000), both estimates within 5 % for two thirds of them. Of the GEMM's
+// time in all, with lines by K alone (64 rows, 40 where K is past 14336) 0.689, 239 calls more than 3 % slower, at most 62 %; by this rule 0.679, 4, at most 9 % (the better one each time 0.678).
+// us, GEMM -> GEMV at 1 / 17 / 32 / 64 rows: 17408 x 5120 24.4 -> 15.1, 25.2 -> 16.1, 25.8 -> 17.4, 27.7 -> 27.1; 5120 x 5120 12.0 -> 6.1, 12.5 -> 8.3, 12.7 -> 8.5, 13.3 -> 11.0; 1024 x 2816
+// 9.7 -> 3.9, 10.2 -> 3.8, 10.2 -> 4.2, 10.7 -> 5.7; not taken: 38784 x 384 at 56 10.4 -> 16.5, 28672 x 640 at 60 10.6 -> 15.4, 11136 x 13952 at 61 40 -> 49, 29568 x 256 at 15 7.0 -> 7.9.
+constexpr FeGemvLine kFeGemvFp8{8, 3.38f, 0.94f, 15.1e-6f, 1.67e-3f, 2.7e-6f, 5.3f, 0.742f, 10.8e-6f, 0.62f, 0.127e-3f, 0.97f};

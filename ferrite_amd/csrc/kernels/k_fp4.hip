@@ -680,7 +680,7 @@ FP8C_GEMM_KERNEL(_h5, FpTileH5, false)
 // pc <= 8 CO weight rows (gemv_even) over all of K, its four wavefronts a quarter of K's steps of 128 codes each, DEPTH - 1 steps ahead in LDS stages of their own; a load is 8 rows x 128 bytes,
 // a row's 16-byte chunk c at position c ^ (row & 7). A wavefront adds its products in ascending k, the four sums are added in order: a row's bits depend on K and W only.
 // Bound by the weights' way from HBM up to 16 rows, by the activations' way from L2 as rows and K grow. It replaces the GEMM, whose tiles of 128 rows are mostly empty and whose
-// pieces of K need a reduce launch: fp8_gemv_rows of fe_fp4.cpp has both sides.
+// pieces of K need a reduce launch: kFeGemvFp8 of fe_internal.h has both sides.
 template <int XO, int CO>
 struct Fp8Gemv {
     static constexpr int L = CO + XO, STAGE = L * 1024;

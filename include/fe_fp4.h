@@ -27,7 +27,7 @@ int fe_fp4_kernels_destroy(fe_fp4_kernels *k);
 /* Switches of the launch paths, by name (the environment variable that sets the same switch when the kernels are loaded):
  * "group_m" (FE_FP4_GROUP), "gemv" 0/1 (FE_FP4_NO_GEMV), "gemv_sk" (FE_FP4_GEMV_SK; 0 = automatic), "gemv_strips" 0/1 (FE_FP4_NO_STRIPS: up to
  * 16 rows over weight tiles and K splits, as more rows run / in programs of some columns over all of K), "gemv_cols" (FE_FP4_GEMV_COLS: columns such
- * a program, or one of the FP8 GEMV (up to 64 rows, 40 where k > 14336), takes, rounded up to 8, 16, .. 48, 72, and to the nearest width that a form has (NVFP4: 48 at most where K is summed in eighths or the program quantizes, 16 at least where both); 0 = by the shape; same bits), "gemv_quant" (FE_FP4_GEMV_QUANT: most values, rows x k, that four wavefronts of such a program quantize themselves, eight
+ * a program, or one of the FP8 GEMV (up to 8 rows, up to 64 where it is ahead of the GEMM), takes, rounded up to 8, 16, .. 48, 72, and to the nearest width that a form has (NVFP4: 48 at most where K is summed in eighths or the program quantizes, 16 at least where both); 0 = by the shape; same bits), "gemv_quant" (FE_FP4_GEMV_QUANT: most values, rows x k, that four wavefronts of such a program quantize themselves, eight
  * twice as many; default -1 = by the shape, 10240 at most; 0 = by a launch of its own; same bits), "gemv_once" and "gemv_waves" (accepted, without effect), "xcd" -1/0/1
  * (FE_FP4_XCD), "fp8_f16" 0/1 (FE_FP8_F16), "gemm_splits" (FE_GEMM_SPLITS), "gemm_tile" 0..6 (output tile of the GEMMs: by the shape, 256 x 256,
  * 128 x 256, 128 x 128, 224 x 256, 192 x 256, 160 x 256; other values FE_ERR_ARG) and "gemm_pieces" (pieces of K a forced small tile takes), both for tests, "gemm_sk" 0..3 (FE_GEMM_SK: the stream-K schedule of the

@@ -176,3 +176,25 @@ int main() {{
 }}
 """)
     assert [int(v) for v in lines] == [int(lower < small) for small, lower in LOWER.values()]
+
+
+# (columns, K, rows): us of the FP8 GEMV and of the GEMM
+FP8 = {(11776, 12288, 58): (44.6, 36.7), (34176, 3840, 53): (40.2, 31.1), (21120, 512, 49): (12.5, 9.0), (35328, 2304, 61): (30.6, 25.4),
+       (26368, 512, 27): (10.7, 8.9), (37632, 384, 59): (16.6, 10.5), (27904, 256, 55): (12.0, 7.9), (2048, 19328, 58): (25.7, 22.0), (128, 2048, 52): (6.2, 11.5),
+       (1024, 1024, 43): (5.1, 10.2), (384, 640, 15): (4.5, 7.4), (1152, 10752, 17): (9.3, 14.8), (1024, 896, 20): (4.7, 8.8), (768, 1536, 53): (5.8, 12.4),
+       (768, 512, 53): (5.3, 8.0), (1920, 2432, 58): (7.3, 13.6)}
+
+
+def test_fp8_rows_take_the_gemv_where_that_was_timed_faster(tmp_path):
+    calls = ", ".join("{%du, %du, %du}" % c for c in FP8)
+    lines = run_host(tmp_path, "fe_fp4.cpp", f"""
+int main() {{
+    const uint32_t calls[][3] = {{{calls}}};
+    for (auto &c : calls) {{
+        const uint32_t n = c[0], k = c[1], m = c[2];
+        const FeGemmPlan p = fe_gemm_plan(m, n, k / 128, 256, 1, (size_t)512 * kFeGemmPartBytes, 1, 8192, 8, 1, false, kFeCostFp8, FeGemmTileOptions{{0, 0, true}});
+        printf("%d\\n", fe_gemv_ahead(kFeGemvFp8, m, n, k, k / 128, 256, 4, p));
+    }}
+}}
+""")
+    assert [int(v) for v in lines] == [int(gemv < gemm) for gemv, gemm in FP8.values()]
