@@ -11,7 +11,7 @@
 #include "fe_internal.h"
 
 namespace {
-// dynamic LDS by form (256 x 256, unused, 128 x 256, 128 x 128): the k tiles in flight, two or three of A and three of W
+// dynamic LDS by form (256 x 256, unused, 128 x 256, 128 x 128, 224, 192, 160 x 256): the k tiles in flight, three of W and two of A (128 x 256: three), A in whole loads of 64 rows
 constexpr uint32_t kGemmLds[kFeGemmForms] = {160 * 1024, 0, 144 * 1024, 80 * 1024, 160 * 1024, 144 * 1024, 144 * 1024};
 constexpr uint32_t kGemmThreads = 512;
 constexpr uint32_t kTileM = 256;                         // rows of the largest output tile

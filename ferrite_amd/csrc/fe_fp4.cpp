@@ -14,8 +14,9 @@
 
 namespace {
 constexpr uint32_t kTile = 128;                 // crates/fe-fp4/src/lib.rs:28
-// dynamic LDS by form (256 x 256, its stream-K form, 128 x 256, 128 x 128): the k tiles in flight. Packed weights: three of A (128
-// bytes a row) and three of W (36 bytes; 64 in the fp16 form of FP8). FP8 codes: two or three of A, three of W, 128 bytes a row.
+// dynamic LDS by form (256 x 256, its stream-K form, 128 x 256, 128 x 128, 224, 192, 160 x 256): the k tiles in flight, A in whole loads of 64 rows. Packed weights: three of
+// A (128 bytes a row; 128 x 256: five) and three of W (36 bytes, 64 in the fp16 form of FP8; 128 x 256: six, 128 x 128: four). FP8 codes: two of A (128 x 256: three), three of
+// W, 128 bytes a row.
 constexpr uint32_t kGemmLds[kFeGemmForms] = {144 * 1024, 144 * 1024, 136 * 1024, 68 * 1024, 144 * 1024, 120 * 1024, 120 * 1024};
 constexpr uint32_t kGemmLds8[kFeGemmForms] = {160 * 1024, 160 * 1024, 144 * 1024, 80 * 1024, 160 * 1024, 144 * 1024, 144 * 1024};
 // Forms of the GEMV over programs of 8 CO columns: rows / 2 and CO

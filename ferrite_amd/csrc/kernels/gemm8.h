@@ -140,7 +140,8 @@ struct G8Dense {
 };
 
 // acc[i][j]: weight rows (output columns) 16 (wn TN + j) + 4 (lane >> 4) + e, activation row 16 (wm TM + i) + (lane & 15).
-// k tiles kt0 .. kt0 + ktiles - 1. a: 16-bit values [m][lda]; rows past m repeat row m - 1. lds: the start of the dynamic LDS.
+// k tiles kt0 .. kt0 + ktiles - 1. a: 16-bit values [m][lda]; rows past m read zero (ZERO) or
+// repeat row m - 1 (g8_row). lds: the start of the dynamic LDS.
 //
 // One k tile is two slices of 32 k. A slice walks the TN columns of fragments (outer), TM MFMAs each; the outer fragment's
 // register is refilled for the next slice as soon as its MFMAs are issued, the TM inner fragments are double-buffered. The

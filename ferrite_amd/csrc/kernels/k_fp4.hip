@@ -1039,7 +1039,7 @@ FP4_GEMV_KERNEL(3, , true) FP4_GEMV_KERNEL(3, _v, false)  // (four groups of row
 //
 // y[r][n] for r < m <= 2 XP. grid ceil(N / 8 CO), 64 WV threads: a program takes 8 CO weight rows over all of K, its wavefronts (four or eight: wide_form of fe_fp4.cpp)
 // a quarter or an eighth of K's steps of 256 each (four k tiles). Sums of quarters are added in order; where wide_form sums eighths (EIGHTHS: all forms of such a linear
-// alike), two of them make a quarter. A row's bits depend on W's shape and values only. K % 256 == 0.
+// alike), two of them make a quarter. A row's bits depend on W's shape and values and, by wide_form's line, on the device's count of CUs only. K % 256 == 0.
 // Lane L = 16 g + r multiplies, for 16 weight rows, row r's k tile 4 s + g (64 codes, four block scales) with the activations of the
 // same k; the order of k inside a step does not matter.
 // Stages belong to one wavefront (no barrier in the loop). Codes: 8 weight rows a load, [4 k tiles][8 rows][32 bytes]; lanes of
