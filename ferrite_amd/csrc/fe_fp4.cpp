@@ -441,6 +441,22 @@ static uint32_t gemv_splits(const fe_fp4_kernels *kern, const fe_fp4_workspace *
     return std::max(sk, 1u);
 }
 
+// Whether a fused gate|up linear's rows go through the GEMV, by sk splits of K, and not through the GEMM that `plan` is of: up to 16 rows, and up to 48 where an estimate of both
+// (us) has it ahead. The GEMV's: a start, a wavefront's k tiles (less each where a CU has two programs), the weights' way, and the splits' sums, written and read. The
+// GEMM's: its plan's and what that leaves out at so few rows; pieces of K cost less than it says. Fitted to 11766 calls of 17..48 rows (256 .. 40960 columns, K 256 .. 19200, weight
+// tiles and, one in five, rows as they lie): half of either within 3 %. With the lines of takes_gemv 0.872 of the GEMM's time in all, 1798 calls more than 3 % slower than it, at most
+// 39 %; by this rule 0.867, 88, at most 23 % (the better one each time 0.856; of 3922 calls of 1..16 rows the GEMV is the slower one in 2). us, GEMM -> GEMV: 512 x 4992 at 45 rows 13.8 -> 18.4,
+// 1536 x 4480 at 38 14.6 -> 19.1, 4864 x 4224 at 40 18.7 -> 23.1, 1280 x 8832 at 35 18.5 -> 20.6 (not taken); 34816 x 5120 at 17 / 48 63 -> 37, 51, 40192 x 512 at 46 21.6 -> 15.0, 1536 x 1152 at 28 17.8 -> 11.2.
+static bool swiglu_takes_gemv(const fe_fp4_linear *l, const fe_fp4_kernels *kern, uint32_t m, uint32_t sk, const FeGemmPlan &plan) {
+    if (m > kGemvRows || l->n / kTile > kGemvCounters || !kern->gemv || kern->tile.force_tile || kern->gemm_sk >= 2) return false;
+    if (m <= 16 || !kern->gemv_strips || kern->gemv_sk) return true;
+    const uint32_t nts = l->n / kTile, steps = (l->k / 64 + 4 * sk - 1) / (4 * sk), pieces = plan.tile == 1 || plan.tile == 2 ? plan.splits : plan.big.split.splits;
+    const float groups = (float)((m + 15) / 16), weights = (float)l->n * (float)l->k, a_cu = std::max(1.0f, (float)(nts * sk) / (float)std::max(kern->cus, 1u));
+    const float gemv = 3.47f + groups * (1.6f + (0.513f - 0.142f * a_cu) * (float)steps + 0.124f * (float)sk) + (l->w_sr == 32 ? 0.102e-6f : 0.207e-6f) * weights +
+                       (sk > 1 ? 2.0f : 0.0f) + 0.96e-6f * (float)sk * (float)m * (float)l->n;
+    return gemv <= 0.95f * (7.95f + 1.007f * plan.us - 0.0174e-6f * weights - (pieces > 1 ? 6.08f : 0.0f));
+}
+
 // x: null, or the activations (bf16 rows of lda) which that GEMV quantizes itself
 static int linear_gemm(const fe_fp4_linear *l, const fe_fp4_kernels *kern, fe_stream_t s, const fe_fp4_workspace *ws, fe_devptr_t y, uint32_t ldy,
                        uint32_t m, fe_devptr_t res, fe_devptr_t x, uint32_t lda) {
@@ -596,14 +612,14 @@ int fe_fp4_linear_forward_swiglu(const fe_fp4_linear *l, const fe_fp4_kernels *k
     fe_devptr_t q_codes = act->codes.p, q_sf = act->sf.p, q_aq = act->aq.p;
     uint32_t w_snt = l->w_snt, w_skt = l->w_skt, w_sr = l->w_sr, s_snt = l->s_snt, s_skt = l->s_skt, s_sr = l->s_sr;
     // (stream-K only when forced: this kernel's stream-K form was slower wherever measured, 688 -> 714 us on 5120 x 34816)
-    if (m <= kGemvRows && takes_gemv(l, kern, m, true) && !kern->tile.force_tile && kern->gemm_sk < 2) {
-        uint32_t sk = gemv_splits(kern, ws, n, k);
-        fe_devptr_t cnt = ws->counters.p;
-        void *args[] = {&aq, &w, &sw, &alpha, &part, &cnt, &m, &n, &k, &sk, &w_snt, &w_skt, &w_sr, &s_snt, &s_skt, &s_sr, &q_codes, &q_sf, &q_aq, &down_g};
-        return fe_hip_launch(kern->gemv_swiglu4[w_sr != 32][(m + 15) / 16 - 1], n / kTile * sk, 1, 1, 256, 1, 1, 0, s, args);
-    }
     const FeGemmPlan plan = fe_gemm_plan(m, n, k / 64, kern->cus, ws->part.p, ws->part.bytes, ws->counters.p, kGemvCounters, kern->gemm_splits,
                                          kern->gemm_sk >= 2 ? kern->gemm_sk : 0, true, kFeCostNvfp4, kern->tile);
+    const uint32_t sk = gemv_splits(kern, ws, n, k);
+    if (swiglu_takes_gemv(l, kern, m, sk, plan)) {
+        fe_devptr_t cnt = ws->counters.p;
+        void *args[] = {&aq, &w, &sw, &alpha, &part, &cnt, &m, &n, &k, (void *)&sk, &w_snt, &w_skt, &w_sr, &s_snt, &s_skt, &s_sr, &q_codes, &q_sf, &q_aq, &down_g};
+        return fe_hip_launch(kern->gemv_swiglu4[w_sr != 32][(m + 15) / 16 - 1], n / kTile * sk, 1, 1, 256, 1, 1, 0, s, args);
+    }
     if (!plan.tile && plan.big.stream_k && kern->xcd < 0) group = 1;
     return fe_gemm_launch(
         plan,

@@ -826,7 +826,7 @@ struct Fp4GemvStage {
 // NT: non-temporal loads of the weights. Not of rows as they lie in a checkpoint (_v): a wavefront's piece of such a row is a quarter of its cache line, which the next
 // wavefronts then read again from memory: 34816 x 5120 at 32 rows 131 us with, 102 without; 17408 x 5120 51 -> 39. (Weight tiles: 41.6 with, 42.2 without.)
 // SWIGLU: a fused gate|up linear, whose finished tile goes through LDS to swiglu_quant_store (out), a row a half wavefront. 34816 x 5120 at 17 / 32 / 48 rows 37 / 42 / 51 us
-// against 63 in the GEMM (takes_gemv of fe_fp4.cpp).
+// against 63 in the GEMM (swiglu_takes_gemv of fe_fp4.cpp).
 template <int XR, bool NT, bool SWIGLU>
 __device__ __forceinline__ void gemv_nvfp4_body(const FpOut out, const _Float16* aq, const uint8_t* w, const uint8_t* sw,
                                                 const float* alpha, float* z, uint32_t* counters,

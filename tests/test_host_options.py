@@ -198,3 +198,30 @@ int main() {{
 }}
 """)
     assert [int(v) for v in lines] == [int(gemv < gemm) for gemv, gemm in FP8.values()]
+
+
+# SwiGLU fronts (columns of gate and up together, K, rows): us of the GEMV and of the GEMM
+SWIGLU = {(512, 4992, 45): (18.4, 13.8), (1536, 4480, 38): (19.1, 14.6), (4864, 4224, 40): (23.1, 18.7), (512, 2176, 38): (14.4, 12.4), (1280, 8832, 35): (20.6, 18.5),
+          (2304, 17536, 45): (30.5, 28.0), (6912, 3200, 48): (21.8, 19.3), (512, 3712, 33): (17.7, 12.8), (40192, 512, 46): (15.0, 21.6), (29184, 2688, 20): (19.7, 29.6),
+          (8704, 4096, 20): (15.4, 22.8), (1536, 1152, 28): (11.2, 17.8), (13824, 1024, 18): (12.1, 17.8), (35072, 9088, 24): (66.8, 114.9), (8960, 256, 20): (8.0, 11.7),
+          (512, 4992, 12): (10.4, 13.1)}  # up to 16 rows in any case
+
+
+def test_swiglu_fronts_take_the_gemv_where_that_was_timed_faster(tmp_path):
+    calls = ", ".join("{%du, %du, %du}" % c for c in SWIGLU)
+    lines = run_host(tmp_path, "fe_fp4.cpp", f"""
+int main() {{
+    fe_fp4_kernels K;
+    K.cus = 256;
+    fe_fp4_linear l;
+    fe_fp4_workspace ws;
+    ws.part.bytes = (size_t)512 * kFeGemmPartBytes;
+    const uint32_t calls[][3] = {{{calls}}};
+    for (auto &c : calls) {{
+        l.n = c[0], l.k = c[1], l.w_sr = 32;
+        const FeGemmPlan p = fe_gemm_plan(c[2], l.n, l.k / 64, 256, 1, ws.part.bytes, 1, 8192, 8, 0, true, kFeCostNvfp4, K.tile);
+        printf("%d\\n", swiglu_takes_gemv(&l, &K, c[2], gemv_splits(&K, &ws, l.n, l.k), p));
+    }}
+}}
+""")
+    assert [int(v) for v in lines] == [int(gemv < gemm) for gemv, gemm in SWIGLU.values()]
