@@ -61,29 +61,35 @@ static int check(const char *fn, fe_devptr_t y, uint32_t ldy, fe_devptr_t x, uin
     return fe_set_error(code, fn, code == FE_ERR_SHAPE ? msg : why);
 }
 
-// Whether all of a call's rows go through the GEMV: a batch of decode rows, or one so small that the GEMV's one read of the weights is ahead of the GEMM's tiles. us at 17 /
-// 24 / 32 rows, GEMM -> GEMV: 17408 x 5120 40 -> 31, 31, 32; 34816 x 5120 77 -> 58, 79 -> 60, 81 -> 62; 5120 x 5120 17 -> 13, 15, 16; 5120 x 8704 24 -> 19, 21, 23;
-// 8192 x 2048 12.6 -> 8; 1024 x 2816 8.7 -> 5.4, 5.7, 6.1. The line in rows times K is the activations' way from L2 once a program: 4096 x 14336 27 -> 24, 26, 29; 5120 x 17408
-// 38 -> 36, 39, 44; a block of 5120 x 8704 at 32 rows 68 -> 70. From 33 rows on (three groups of 16) the GEMM is ahead wherever K is 5120 and more.
-// Operands of 4 GB and more, which the GEMM refuses, stay refused there.
+// Operands of 4 GB and more the GEMM refuses, also where few rows could go another way.
 static bool gemm_reaches(uint32_t m, uint32_t n, uint32_t k, uint32_t lda) { return (uint64_t)m * lda * 2 < (1ull << 32) && (uint64_t)n * k * 2 < (1ull << 32); }
-static bool rows_take_gemv(uint32_t m, uint32_t n, uint32_t k, uint32_t lda, uint32_t dec) {
-    return m <= kSmallBatch || dec >= m || (m <= 32 && (uint64_t)m * k <= (m <= 24 ? 350000 : 180000) && gemm_reaches(k % 256 ? m : m - dec, n, k, lda));
+static FeGemmPlan gemm_plan(const fe_bf16_kernels *kern, uint32_t m, uint32_t n, uint32_t k) {
+    return fe_gemm_plan(m, n, k / 64, kern->cus, kern->part.p, kern->part.bytes, 0, 0, kern->gemm_splits, 0, false, kFeCostBf16, kern->tile);
+}
+// Whether all of a call's rows go through the GEMV: a batch of decode rows, or 17..32 rows where its one read of the weights is ahead of the GEMM's tiles (kFeGemvBf16).
+static bool rows_take_gemv(const fe_bf16_kernels *kern, uint32_t m, uint32_t n, uint32_t k, uint32_t lda, uint32_t dec) {
+    if (m <= kSmallBatch || dec >= m) return true;
+    if (m > 32 || k % 256 || !gemm_reaches(m - dec, n, k, lda)) return false;
+    return fe_gemv_ahead(kFeGemvBf16, m, n, k, k / 64, std::max(kern->cus, 1u), 2, gemm_plan(kern, m - dec, n, k), (float)n * (float)k * 2.0f, dec);
 }
 
 bool fe_bf16_gemv_swiglu_takes(const fe_bf16_kernels *kern, fe_devptr_t big, fe_devptr_t act, fe_devptr_t x, fe_devptr_t gate, fe_devptr_t up, uint32_t m, uint32_t inter,
                                uint32_t k, uint32_t dec, bool over_gemm) {
-    // (against the GEMM with SwiGLU wider programs have to carry the activations: a block of 32 rows, GEMM -> GEMV, us: 5120 x 17408 133 ->
-    // 106, 5120 x 12288 98 -> 84, 4096 x 8192 60 -> 48, but 5120 x 8704 68 -> 71; of 24 rows 66 -> 60. Against gate, up and fe_silu_mul, where there are no such weights, it is ahead
-    // there too: 5120 x 8704 at 26 / 32 rows 63.0 -> 58.0, 63.9 -> 58.6, 5120 x 6144 at 30 53.0 -> 48.4, 7168 x 2048 at 25 32.7 -> 28.0)
-    if (over_gemm && m > kSmallBatch && dec < m && inter < 12288 && (uint64_t)m * k > 131072) return false;
-    if (!m || m > kGemvPass || !rows_take_gemv(m, over_gemm ? 2 * inter : inter, k, k, dec) || !inter || !k || inter % 8 || k % 256 || (uint64_t)m * k * 2 >= (1ull << 32)) return false;
+    if (!kern || !m || m > kGemvPass || !inter || !k || inter % 8 || k % 256 || (uint64_t)m * k * 2 >= (1ull << 32)) return false;
+    // (against the GEMM with SwiGLU: kFeGemvBf16Pair. Against gate, up and fe_silu_mul, where there are no such weights, it is ahead wherever those go through the GEMV: 5120 x 8704 at
+    // 26 / 32 rows 63.0 -> 58.0, 63.9 -> 58.6, 5120 x 6144 at 30 53.0 -> 48.4, 7168 x 2048 at 25 32.7 -> 28.0)
+    if (over_gemm && m > kSmallBatch && dec < m) {
+        if (m > 32 || !gemm_reaches(m - dec, 2 * inter, k, k)) return false;
+        if (!fe_gemv_ahead(kFeGemvBf16Pair, m, inter, k, k / 64, std::max(kern->cus, 1u), 2, gemm_plan(kern, m - dec, 2 * inter, k), (float)inter * (float)k * 4.0f, dec)) return false;
+    } else if (!rows_take_gemv(kern, m, inter, k, k, dec)) {
+        return false;
+    }
     const char *why;
     if (refusal(big, inter, x, k, gate, 0, inter, k, &why) || refusal(big, inter, x, k, up, 0, inter, k, &why)) return false;
     // programs that are done write act while others read x and the weights
     const uint64_t bytes = (uint64_t)m * inter * 2, weights = (uint64_t)inter * k * 2;
     auto apart = [&](fe_devptr_t p, uint64_t size) { return act + bytes <= p || p + size <= act; };
-    return kern && act % 4 == 0 && apart(x, (uint64_t)m * k * 2) && apart(gate, weights) && apart(up, weights);
+    return act % 4 == 0 && apart(x, (uint64_t)m * k * 2) && apart(gate, weights) && apart(up, weights);
 }
 
 int fe_bf16_gemv_swiglu(const fe_bf16_kernels *kern, fe_stream_t s, fe_devptr_t act, fe_devptr_t x, fe_devptr_t gate, fe_devptr_t up, uint32_t m, uint32_t inter, uint32_t k) {
@@ -195,8 +201,7 @@ int fe_bf16_gemm(const fe_bf16_kernels *kern, fe_stream_t s, fe_devptr_t y, uint
     uint32_t group = bf16_raster_group(m, n, k, tiles_m);
     if (kern->raster_group >= 0) group = (uint32_t)kern->raster_group;
     if (group > tiles_m) group = tiles_m;
-    const FeGemmPlan plan = fe_gemm_plan(m, n, k / 64, kern->cus, kern->part.p, kern->part.bytes, 0, 0, kern->gemm_splits, 0, false,
-                                         kFeCostBf16, kern->tile);
+    const FeGemmPlan plan = gemm_plan(kern, m, n, k);
     return fe_gemm_launch(
         plan,
         [&](uint32_t form, uint32_t programs, FeGemmSchedArgs sched) {
@@ -233,8 +238,7 @@ int fe_bf16_gemm_swiglu(const fe_bf16_kernels *kern, fe_stream_t s, fe_devptr_t 
     uint32_t group = bf16_raster_group(m, n, k, tiles_m);
     if (kern->raster_group >= 0) group = (uint32_t)kern->raster_group;
     if (group > tiles_m) group = tiles_m;
-    const FeGemmPlan plan = fe_gemm_plan(m, n, k / 64, kern->cus, kern->part.p, kern->part.bytes, 0, 0, kern->gemm_splits, 0, false,
-                                         kFeCostBf16, kern->tile);
+    const FeGemmPlan plan = gemm_plan(kern, m, n, k);
     return fe_gemm_launch(
         plan,
         [&](uint32_t form, uint32_t programs, FeGemmSchedArgs sched) {
@@ -255,7 +259,7 @@ int fe_bf16_linear_forward(const fe_bf16_kernels *kern, fe_stream_t s, fe_devptr
     if (m == 0) return 0;
     FE_TRY(check(fn, y, ldy, x, lda, w, res, n, k));
     // decode / verify rows: the GEMV, so that a row's bits do not depend on the batch
-    uint32_t d = rows_take_gemv(m, n, k, lda, dec) ? m : dec;
+    uint32_t d = rows_take_gemv(kern, m, n, k, lda, dec) ? m : dec;
     if (k % 256) d = 0;
     for (uint32_t r = 0; r < d; r += kGemvPass) {
         const uint32_t mr = d - r < kGemvPass ? d - r : kGemvPass;

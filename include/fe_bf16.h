@@ -44,8 +44,9 @@ int fe_bf16_interleave_gu(const fe_bf16_kernels *kern, fe_stream_t s, fe_devptr_
  * interleaved weights W [2 inter][k]; act rows have stride inter. inter % 8 == 0. */
 int fe_bf16_gemm_swiglu(const fe_bf16_kernels *kern, fe_stream_t s, fe_devptr_t act, fe_devptr_t x, uint32_t lda,
                         fe_devptr_t w, uint32_t m, uint32_t inter, uint32_t k);
-/* The bf16 branch of Linear::forward (model.rs:310-345): all rows of a batch of <= 16 (of <= 24 where rows * k <= 350000 and of <= 32 where it is <= 180000, in which the
- * GEMV is ahead of the GEMM), else the leading `dec` rows, go through the GEMV in passes of up to 64 rows (when k % 256 == 0); the rows after them through the GEMM. */
+/* The bf16 branch of Linear::forward (model.rs:310-345): all rows of a batch of <= 16, and of <= 32 where an estimate
+ * of both has the GEMV ahead of the GEMM, else the leading `dec` rows, go through the GEMV in passes of up to 64 rows (when k % 256 == 0); the
+ * rows after them through the GEMM. */
 int fe_bf16_linear_forward(const fe_bf16_kernels *kern, fe_stream_t s, fe_devptr_t y, uint32_t ldy, fe_devptr_t x,
                            uint32_t lda, fe_devptr_t w, fe_devptr_t res, uint32_t m, uint32_t n, uint32_t k, uint32_t dec);
 

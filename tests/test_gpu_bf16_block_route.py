@@ -10,11 +10,11 @@ PAIR, GEMM, PARTS = "one GEMV", "GEMM with SwiGLU", "separate linears"
 # rows, decode rows, hidden, inter, interleaved weights given, what the decode rows (all rows where dec is None) and the prompt rows take
 @pytest.mark.parametrize("rows,dec,hidden,inter,fused,first,rest", [
     (1, None, 5120, 320, False, PAIR, PAIR), (16, None, 5120, 320, True, PAIR, PAIR),
-    (17, None, 5120, 320, True, PAIR, PAIR), (24, None, 5120, 320, True, PAIR, PAIR), (25, None, 5120, 320, True, PAIR, PAIR),  # 131072 values: the line against the GEMM
-    (32, None, 4096, 320, True, PAIR, PAIR), (26, None, 5120, 320, True, GEMM, GEMM), (32, None, 5120, 320, True, GEMM, GEMM),
+    (17, None, 2048, 320, True, PAIR, PAIR), (32, None, 2048, 1344, True, PAIR, PAIR), (32, None, 5120, 12288, True, PAIR, PAIR), (20, 4, 2048, 320, True, PAIR, PAIR),
+    (17, None, 5120, 320, True, GEMM, GEMM), (32, None, 5120, 320, True, GEMM, GEMM), (26, None, 7168, 320, True, GEMM, GEMM),  # the GEMM with SwiGLU is ahead of it
     (26, None, 5120, 320, False, PAIR, PAIR), (32, None, 5120, 320, False, PAIR, PAIR),  # no interleaved weights: against three launches
-    (32, None, 5120, 12288, True, PAIR, PAIR), (33, None, 5120, 320, True, GEMM, GEMM), (33, None, 5120, 320, False, PARTS, PARTS),
-    (23, None, 14848, 64, False, PAIR, PAIR), (23, None, 14848, 64, True, GEMM, GEMM), (24, None, 14848, 64, False, PARTS, PARTS),  # 350000 values: the linears' own line
+    (33, None, 5120, 320, True, GEMM, GEMM), (33, None, 5120, 320, False, PARTS, PARTS),
+    (23, None, 14848, 64, False, PARTS, PARTS), (23, None, 14848, 64, True, GEMM, GEMM),  # the linears' own line
     (64, 64, 5120, 320, True, PAIR, PAIR), (65, 65, 5120, 320, False, PARTS, PARTS), (40, 4, 5120, 320, True, PAIR, GEMM),
 ])
 def test_a_block_takes(rows, dec, hidden, inter, fused, first, rest):

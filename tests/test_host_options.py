@@ -59,7 +59,8 @@ def test_what_the_gemm_refuses_stays_refused_at_few_rows(tmp_path):
     """17 to 32 rows that are no decode rows may go through the GEMV, but not where the GEMM they went through before refuses the operands. (No case here reaches a launch.)"""
     lines = run_host(tmp_path, "fe_bf16.cpp", """
 int main() {
-    const fe_bf16_kernels k;
+    fe_bf16_kernels k;
+    k.cus = 256;
     const fe_devptr_t y = 0x1000000, x = 0x2000000, w = 0x3000000;
     auto refused = [&](uint32_t n, uint32_t kk, uint32_t lda, uint32_t m, uint32_t dec) {
         return fe_bf16_linear_forward(&k, nullptr, y, n, x, lda, w, 0, m, n, kk, dec) == FE_ERR_UNSUPPORTED;
@@ -225,3 +226,25 @@ int main() {{
 }}
 """)
     assert [int(v) for v in lines] == [int(gemv < gemm) for gemv, gemm in SWIGLU.values()]
+
+
+# bf16 linears and gate|up fronts (columns, K, rows): us of the GEMV and of the GEMM
+BF16 = {(61728, 256, 31): (15.8, 7.6), (55304, 256, 27): (14.5, 7.2), (24672, 512, 29): (9.8, 6.5), (53672, 1536, 31): (33.4, 27.7), (26952, 512, 17): (9.1, 6.6), (48152, 1280, 24): (26.2, 21.7),
+        (24936, 256, 22): (7.6, 4.9), (3520, 18432, 32): (33.7, 27.9), (104, 2304, 21): (3.8, 7.9), (12312, 768, 29): (5.8, 7.6), (264, 4608, 23): (6.3, 8.8), (8368, 512, 30): (4.0, 6.1),
+        (2488, 2816, 23): (6.0, 9.8), (144, 1280, 17): (3.2, 8.8), (5344, 1024, 20): (4.1, 8.5), (80048, 4096, 28): (114.0, 144.5), (28360, 6144, 22): (61.8, 84.9)}
+BF16_PAIR = {(28480, 256, 22): (18.8, 7.8), (15168, 256, 21): (9.8, 5.6), (27072, 1280, 20): (29.8, 24.1), (64, 18432, 26): (36.4, 17.4), (320, 10752, 20): (22.4, 12.9), (640, 14336, 22): (32.4, 19.2),
+             (384, 6400, 24): (15.0, 10.5), (640, 512, 20): (4.4, 6.2), (320, 1280, 21): (4.9, 8.1), (3072, 512, 30): (3.9, 6.8), (1280, 2560, 20): (7.0, 9.5), (2112, 1280, 20): (6.7, 10.3)}
+
+
+def test_bf16_rows_take_the_gemv_where_that_was_timed_faster(tmp_path):
+    calls = ", ".join("{%du, %du, %du, %d}" % (*c, pair) for t, pair in ((BF16, 0), (BF16_PAIR, 1)) for c in t)
+    lines = run_host(tmp_path, "fe_bf16.cpp", f"""
+int main() {{
+    struct {{ uint32_t n, k, m; int pair; }} calls[] = {{{calls}}};
+    for (auto &c : calls) {{
+        const FeGemmPlan p = fe_gemm_plan(c.m, c.pair ? 2 * c.n : c.n, c.k / 64, 256, 1, (size_t)512 * kFeGemmPartBytes, 0, 0, 8, 0, false, kFeCostBf16, FeGemmTileOptions{{0, 0, true}});
+        printf("%d\\n", fe_gemv_ahead(c.pair ? kFeGemvBf16Pair : kFeGemvBf16, c.m, c.n, c.k, c.k / 64, 256, 2, p, (c.pair ? 4.0f : 2.0f) * c.n * c.k));
+    }}
+}}
+""")
+    assert [int(v) for v in lines] == [int(gemv < gemm) for t in (BF16, BF16_PAIR) for gemv, gemm in t.values()]
