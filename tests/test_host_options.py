@@ -183,7 +183,8 @@ int main() {{
 FP8 = {(11776, 12288, 58): (44.6, 36.7), (34176, 3840, 53): (40.2, 31.1), (21120, 512, 49): (12.5, 9.0), (35328, 2304, 61): (30.6, 25.4),
        (26368, 512, 27): (10.7, 8.9), (37632, 384, 59): (16.6, 10.5), (27904, 256, 55): (12.0, 7.9), (2048, 19328, 58): (25.7, 22.0), (128, 2048, 52): (6.2, 11.5),
        (1024, 1024, 43): (5.1, 10.2), (384, 640, 15): (4.5, 7.4), (1152, 10752, 17): (9.3, 14.8), (1024, 896, 20): (4.7, 8.8), (768, 1536, 53): (5.8, 12.4),
-       (768, 512, 53): (5.3, 8.0), (1920, 2432, 58): (7.3, 13.6)}
+       (768, 512, 53): (5.3, 8.0), (1920, 2432, 58): (7.3, 13.6), (3328, 49664, 27): (42.3, 32.7), (46336, 5376, 28): (47.1, 39.5), (3200, 63744, 26): (51.0, 39.7),
+       (38272, 3840, 32): (31.0, 26.1), (4480, 17664, 18): (19.2, 23.4), (4480, 17664, 9): (16.4, 23.2)}
 
 
 def test_fp8_rows_take_the_gemv_where_that_was_timed_faster(tmp_path):
