@@ -421,16 +421,18 @@ static WideForm wide_form(const fe_fp4_linear *l, const fe_fp4_kernels *kern, ui
 static bool takes_wide(const fe_fp4_linear *l, const fe_fp4_kernels *kern, uint32_t m) {
     return !l->fp8 && m <= 16 && l->n / kTile <= kGemvCounters && kern->gemv && kern->gemv_strips && !kern->gemv_sk && l->k % 256 == 0;
 }
-// Whether m rows go through a GEMV: all of one pass. 49..64 rows take two, which the GEMM beats everywhere (us at 64 rows, two passes -> GEMM: 34816 x 5120 83 -> 63, 17408 x
+// Whether m rows go through a GEMV: all of one pass. 49..64 rows take two, which the GEMM beats (us at 64 rows, two passes -> GEMM: 34816 x 5120 83 -> 63, 17408 x
 // 5120 41 -> 32, 5120 x 17408 43 -> 30, 5120 x 5120 27 -> 17.5, 2048 x 6144 27 -> 14; 48 rows in one pass 51, 26, 27, 17, 17 against 62, 31, 30, 17, 14); they stay where
-// the caller asked for weight tiles (gemv_strips 0: a row's bits the same at every count up to 64) or their K splits, and with operands that the GEMM does not reach.
-// From 33 rows on so do narrow linears of middling depth, whose tiles are cut along K either way (us at 48 rows, GEMV -> GEMM: 4096 x 4096 16.7 -> 14.1, 2048 x 6144 17.1 ->
+// the caller asked for weight tiles (gemv_strips 0: a row's bits the same at every count up to 64) or their K splits, with operands that the GEMM does not reach, and where K is so deep
+// that the GEMM's eight pieces of a tile are longer than 16 splits (of 1907 linears of 49..64 rows the rule leaves 23 more than 3 % slower than the better one; without it 256 x 59136 at 53
+// 45 against 57).
+// From 33 rows on narrow linears of middling depth take it, too, whose tiles are cut along K either way (us at 48 rows, GEMV -> GEMM: 4096 x 4096 16.7 -> 14.1, 2048 x 6144 17.1 ->
 // 13.7, 1024 x 5120 15.0 -> 11.3, 1024 x 2816 12.3 -> 10.1, 128 x 8192 14.4 -> 13.1; beyond the lines 5120 x 5120 16.8 -> 16.9, 7168 x 2048 13.0 -> 13.7, 1024 x 1024 9.1 ->
 // 9.9, 512 x 14336 17.0 -> 18.9).
 static bool takes_gemv(const fe_fp4_linear *l, const fe_fp4_kernels *kern, uint32_t m, bool gemm_reaches) {
     if (l->fp8 || m > kGemvMaxRows || l->n / kTile > kGemvCounters || !kern->gemv) return false;
     if (!kern->gemv_strips || kern->gemv_sk || !gemm_reaches) return true;
-    return m <= 32 || (m <= kGemvRows && (l->n > 4096 || l->k < 2048 || l->k > 8192));
+    return m <= 32 || (m <= kGemvRows ? l->n > 4096 || l->k < 2048 || l->k > 8192 : l->k > 28000 + 12 * l->n);
 }
 
 // K splits of the GEMV over weight tiles. Two programs fit a CU: as many programs as run at once, not more (a second round of short programs costs more than idle CUs in

@@ -249,3 +249,24 @@ int main() {{
 }}
 """)
     assert [int(v) for v in lines] == [int(gemv < gemm) for t in (BF16, BF16_PAIR) for gemv, gemm in t.values()]
+
+
+# NVFP4 (columns, K, rows): us of the GEMV in two passes and of the GEMM
+NVFP4_PASSES = {(768, 68864, 62): (53.5, 66.4), (256, 74496, 58): (53.4, 70.0), (256, 59136, 53): (45.5, 56.7), (384, 53248, 51): (42.9, 51.9), (4736, 20224, 53): (45.5, 33.6),
+                (3712, 35328, 59): (55.5, 42.3), (34816, 5120, 64): (83.0, 63.0), (5120, 17408, 64): (43.0, 30.0), (2048, 6144, 64): (27.0, 14.0)}
+
+
+def test_nvfp4_takes_two_passes_where_that_was_timed_faster(tmp_path):
+    calls = ", ".join("{%du, %du, %du}" % c for c in NVFP4_PASSES)
+    lines = run_host(tmp_path, "fe_fp4.cpp", f"""
+int main() {{
+    fe_fp4_kernels K;
+    fe_fp4_linear l;
+    const uint32_t calls[][3] = {{{calls}}};
+    for (auto &c : calls) {{
+        l.n = c[0], l.k = c[1];
+        printf("%d\\n", takes_gemv(&l, &K, c[2], true));
+    }}
+}}
+""")
+    assert [int(v) for v in lines] == [int(gemv < gemm) for gemv, gemm in NVFP4_PASSES.values()]
