@@ -160,7 +160,11 @@ LOWER = {("nvfp4", 636, 5248, 256): (9.2, 13.1), ("nvfp4", 449, 768, 1536): (14.
          ("fp8", 315, 11136, 256): (9.1, 11.6), ("fp8", 584, 6784, 512): (11.2, 13.8), ("fp8", 180, 1024, 4864): (15.8, 18.5),
          ("bf16", 210, 256, 1536): (7.8, 10.3), ("bf16", 228, 25984, 256): (9.4, 10.4), ("bf16", 79, 512, 1792): (8.2, 9.7),
          ("nvfp4", 1686, 5888, 4096): (102.1, 83.7), ("nvfp4", 774, 37248, 2816): (188.2, 162.4), ("fp8", 868, 9856, 3584): (51.4, 43.4),
-         ("bf16", 1423, 5888, 2048): (47.3, 37.6), ("bf16", 721, 25984, 1280): (67.4, 57.7)}
+         ("bf16", 1423, 5888, 2048): (47.3, 37.6), ("bf16", 721, 25984, 1280): (67.4, 57.7),
+         ("bf16", 1231, 1024, 8960): (36.4, 43.2), ("bf16", 1303, 768, 15104): (41.9, 52.6), ("bf16", 864, 1792, 16384): (56.8, 89.7), ("bf16", 424, 1792, 7936): (27.2, 33.0),
+         ("bf16", 764, 2304, 8704): (40.8, 48.0), ("fp8", 711, 33536, 2048): (65.2, 70.8), ("fp8", 1516, 28672, 1792): (92.8, 102.6), ("nvfp4", 1313, 11008, 768): (33.5, 37.9),
+         ("bf16", 1035, 8192, 1792): (42.1, 33.1), ("bf16", 1041, 4608, 7680): (88.7, 73.5), ("bf16", 469, 16640, 1280): (33.7, 25.5), ("fp8", 1253, 7168, 2560): (38.2, 32.3),
+         ("nvfp4", 1159, 6912, 3328): (72.2, 58.6), ("nvfp4", 1528, 3840, 9216): (119.5, 98.4)}
 
 
 def test_a_lower_tile_takes_a_small_ones_place_where_that_was_timed_faster(tmp_path):
