@@ -415,17 +415,18 @@ inline FeGemmPlan fe_gemm_plan(uint32_t m, uint32_t n, uint32_t ktiles, uint32_t
     // with them wherever the estimate says so 68 more than 3 % slower (5248 x 256 at 636 rows 9.2 -> 13.1 us, 7168 x 256 SwiGLU at 140 13.4 -> 25.6, 256 x 1536 bf16 at
     // 210 7.8 -> 10.3, 11136 x 256 FP8 at 315 9.1 -> 11.6) and 0.986 / 0.983 / 0.998 / 0.993 of the time in all; so 11, at most 6 %, and 0.980 / 0.979 / 0.991 / 0.989. Of 52360 launches,
     // deep narrow and wide shallow ones among them, 807 were more than 3 % slower (bf16 1792 x 16384 at 864 rows 56.8 -> 89.7, 768 x 15104 at 1303
-    // 41.9 -> 52.6; at most 1.8 times); with the lines below 116 (41 of them bf16 in the
-    // place of 256 rows, at most 1.5 times: 35 and 49 tiles cut seven and five ways), 0.957 / 0.959 / 0.986 / 0.961 / 0.964 of the time (bf16, its SwiGLU front, FP8, NVFP4, its front; the best each time 0.949
+    // 41.9 -> 52.6; at most 1.8 times); with the lines below 139 (41 of them bf16 in the
+    // place of 256 rows, at most 1.5 times: 35 and 49 tiles cut seven and five ways), 0.957 / 0.959 / 0.986 / 0.960 / 0.964 of the time (bf16, its SwiGLU front, FP8, NVFP4, its front; the best each time 0.949
     // / 0.950 / 0.982 / 0.953 / 0.952).
     const FeGemmSchedule lower = low(pick);
     if (p.tile) {
         if (ktiles < 12 || 2 * lower.split.programs() < cus) return p;
         // Dense weights (bf16, FP8) in fewer lower tiles than a quarter of the CUs: deep narrow linears, which small tiles cut finer than eight pieces of a lower one (bf16:
-        // 826 launches 1.16 times the small tiles' time, from there on 0.90). More lower tiles than CUs: rounds of them want a clearer gain (48 of FP8 1.01, bf16 past 0.9 level).
+        // 826 launches 1.16 times the small tiles' time, from there on 0.90). More lower tiles than CUs and short K: rounds of them want a clearer gain (48 of FP8 1.01, bf16 past 0.9 level;
+        // not so from 24 k tiles on: 5120 x 17408 at 559 rows, NVFP4 block 290 us with them, 305 without).
         const uint32_t tiles = tiles_of(pick);
         if (!small_b && 4 * tiles < cus) return p;
-        const float margin = tiles > cus ? (small_b ? 0.97f : 0.9f) : small_b ? 1.06f : 1.0f;  // (bf16 and FP8: what a lower tile gained is part of that margin)
+        const float margin = tiles > cus && ktiles < 24 ? (small_b ? 0.97f : 0.9f) : small_b ? 1.06f : 1.0f;  // (bf16 and FP8: what a lower tile gained is part of that margin)
         if (margin * p.us < whole * ratio) return p;
     }
     p.tile = pick, p.tiles = 0, p.splits = 1, p.big = lower, p.us = whole * ratio;

@@ -164,7 +164,8 @@ LOWER = {("nvfp4", 636, 5248, 256): (9.2, 13.1), ("nvfp4", 449, 768, 1536): (14.
          ("bf16", 1231, 1024, 8960): (36.4, 43.2), ("bf16", 1303, 768, 15104): (41.9, 52.6), ("bf16", 864, 1792, 16384): (56.8, 89.7), ("bf16", 424, 1792, 7936): (27.2, 33.0),
          ("bf16", 764, 2304, 8704): (40.8, 48.0), ("fp8", 711, 33536, 2048): (65.2, 70.8), ("fp8", 1516, 28672, 1792): (92.8, 102.6), ("nvfp4", 1313, 11008, 768): (33.5, 37.9),
          ("bf16", 1035, 8192, 1792): (42.1, 33.1), ("bf16", 1041, 4608, 7680): (88.7, 73.5), ("bf16", 469, 16640, 1280): (33.7, 25.5), ("fp8", 1253, 7168, 2560): (38.2, 32.3),
-         ("nvfp4", 1159, 6912, 3328): (72.2, 58.6), ("nvfp4", 1528, 3840, 9216): (119.5, 98.4)}
+         ("nvfp4", 1159, 6912, 3328): (72.2, 58.6), ("nvfp4", 1528, 3840, 9216): (119.5, 98.4),
+         ("bf16", 365, 38400, 5632): (179.6, 162.4), ("bf16", 195, 33280, 3840): (80.6, 72.5), ("nvfp4", 839, 25600, 1792): (87.7, 74.5), ("nvfp4", 840, 25856, 3328): (148.2, 130.3)}
 
 
 def test_a_lower_tile_takes_a_small_ones_place_where_that_was_timed_faster(tmp_path):
