@@ -583,17 +583,17 @@ inline uint32_t gemv_cols(uint32_t m, uint32_t n, uint32_t k, uint32_t xo, uint3
 }
 
 // Whether a GEMV over programs of columns is ahead of the GEMM that would run in its place, by an estimate of both (us). The GEMV's: a start, rounds of programs, the weights'
-// way from HBM, the activations' way from L2 once a program (the CU with the most) and the outputs. The GEMM's: its plan's estimate and what that leaves out at so few rows, the
+// way from HBM, the activations' way from L2 once a program (the CU with the most; x: the form's rows, x_row: those that exist) and the outputs. The GEMM's: its plan's estimate and what that leaves out at so few rows, the
 // weights' way, of bytes past what the chip's last cache holds once more (far: us a byte), and the outputs; pieces of K cost less than it says. margin: on what the GEMM takes. Up to `always` rows
 // the GEMV in any case. beside: decode rows, which a GEMV of their own would take beside the GEMM.
 struct FeGemvLine {
     uint32_t always;
-    float start, round, w, x, out, gemm_start, gemm_us, gemm_w, gemm_cut, gemm_pieces, gemm_far, gemm_out, margin;
+    float start, round, w, x, x_row, out, gemm_start, gemm_us, gemm_w, gemm_cut, gemm_pieces, gemm_far, gemm_out, margin;
 };
 inline float fe_gemv_us(const FeGemvLine &c, uint32_t m, uint32_t n, uint32_t k, uint32_t steps, uint32_t cus, uint32_t even_step) {
     const uint32_t xo = kGemvRowForms[gemv_row_form(m)], co = kGemvColForms[gemv_cols(m, n, k, xo, cus, -1)], pc = gemv_even(n, 8 * co, cus, even_step, false);
     const uint32_t programs = (n + pc - 1) / pc, at_once = (gemv_lds(xo, co) <= 80 * 1024 ? 2 : 1) * cus, a_cu = (programs + cus - 1) / cus;
-    return c.start + c.round * (float)((programs + at_once - 1) / at_once) + c.w * (float)n * (float)steps + c.x * (float)(a_cu * 8 * xo) * (float)steps + c.out * (float)m * (float)n;
+    return c.start + c.round * (float)((programs + at_once - 1) / at_once) + c.w * (float)n * (float)steps + (float)a_cu * (c.x * (float)(8 * xo) + c.x_row * (float)m) * (float)steps + c.out * (float)m * (float)n;
 }
 inline bool fe_gemv_ahead(const FeGemvLine &c, uint32_t m, uint32_t n, uint32_t k, uint32_t steps, uint32_t cus, uint32_t even_step, const FeGemmPlan &gemm, float bytes = 0.0f,
                           uint32_t beside = 0) {
@@ -601,7 +601,7 @@ inline bool fe_gemv_ahead(const FeGemvLine &c, uint32_t m, uint32_t n, uint32_t 
     const uint32_t pieces = gemm.tile == 1 || gemm.tile == 2 ? gemm.splits : gemm.big.split.splits;
     const float weights = (float)n * (float)steps;
     const float t = c.gemm_start + c.gemm_us * gemm.us + c.gemm_w * weights + c.gemm_far * std::max(bytes - 250e6f, 0.0f) + c.gemm_out * (float)m * (float)n -
-                    (pieces > 1 ? c.gemm_cut + c.gemm_pieces * (float)pieces * (float)n : 0.0f);
+                    (pieces > 1 ? c.gemm_cut : 0.0f) - c.gemm_pieces * (float)pieces * (float)n;
     return fe_gemv_us(c, m, n, k, steps, cus, even_step) <= c.margin * t + (beside ? fe_gemv_us(c, beside, n, k, steps, cus, even_step) : 0.0f);
 }
 // FP8 (steps of 128 codes), up to 64 rows. Fitted to 17236 calls of 9..64 rows (128 .. 153600 columns, K 128 .. 76800, half of them past 40960 columns or K 20480), half of either
@@ -609,13 +609,13 @@ inline bool fe_gemv_ahead(const FeGemvLine &c, uint32_t m, uint32_t n, uint32_t 
 // better one each time 0.818). Fitted to those alone the rule took 0.829, 650 calls slower, at most 41 % (3328 x 49664 at 27 rows 32.7 -> 42.3 us, 46336 x 5376 at 28 39.5 -> 47.1); by K alone (64 rows, 40
 // where K is past 14336) wide linears of short K took up to 62 % more. us, GEMM -> GEMV at 1 / 17 / 32 / 64 rows: 17408 x 5120 24.4 -> 15.1, 25.2 -> 16.1, 25.8 -> 17.4, 27.7 -> 27.1; 5120 x 5120 12.0 -> 6.1,
 // 12.5 -> 8.3, 12.7 -> 8.5, 13.3 -> 11.0; 1024 x 2816 9.7 -> 3.9, 10.2 -> 3.8, 10.2 -> 4.2, 10.7 -> 5.7; not taken: 38784 x 384 at 56 10.4 -> 16.5, 28672 x 640 at 60 10.6 -> 15.4, 11136 x 13952 at 61 40 -> 49.
-constexpr FeGemvLine kFeGemvFp8{8, 3.47f, 0.835f, 14.4e-6f, 1.544e-3f, 2.39e-6f, 5.01f, 0.768f, 0.68e-6f, 1.64f, -17.5e-6f, 0.0f, 1.11e-6f, 0.95f};
-// bf16 (steps of 64), up to 32 rows that are no decode rows. Fitted to 18642 linears of 17..32 rows (64 .. 96000 columns, K 256 .. 19456), half of either estimate within 5 %. Of the
-// GEMM's time in all, with lines by rows times K alone (350000 up to 24 rows, 180000 up to 32) 0.862, 2207 calls more than 3 % slower than the GEMM, at most 2.1 times; by this rule
-// 0.833, 182, at most 25 % (the better one each time 0.822). us, GEMM -> GEMV at 17 / 24 / 32 rows: 17408 x 5120 40 -> 31, 31, 32; 34816 x 5120 77 -> 58, 79 -> 60, 81 -> 62; 5120 x 5120 17 -> 13,
-// 15, 16; 1024 x 2816 8.7 -> 5.4, 5.7, 6.1; not taken: 61728 x 256 at 31 7.6 -> 15.8, 55304 x 256 at 27 7.2 -> 14.5. From 33 rows on (three groups of 16) the GEMM is ahead wherever K is 5120 and more.
-constexpr FeGemvLine kFeGemvBf16{16, 0.97f, 1.17f, 14.96e-6f, 1.64e-3f, 1.8e-6f, 3.06f, 0.682f, 4.65e-6f, 1.06f, 0.0f, 0.0985e-6f, 0.0f, 0.95f};
-// bf16 gate and up (n each) in one launch against the GEMM with SwiGLU over their interleaved weights (its plan's): 2284 calls, by rows times K and inter 0.942 of the GEMM's time in
-// all, 410 more than 3 % slower, at most 2.4 times; by this rule 0.910, 47, at most 28 % (the better one 0.902). us, GEMM -> GEMV: 8512 x 3584 at 21 rows 29.2 -> 21.9, 1280 x 2560 at
-// 20 9.5 -> 7.0; not taken: 28480 x 256 at 22 7.8 -> 18.8, 15168 x 256 at 21 5.6 -> 9.8, 3840 x 3840 at 32 16.7 -> 20.6.
-constexpr FeGemvLine kFeGemvBf16Pair{16, 2.29f, 0.244f, 28.8e-6f, 3.31e-3f, 9.8e-6f, 3.78f, 0.651f, 11.9e-6f, 1.45f, 38e-6f, 0.0676e-6f, 0.0f, 0.95f};
+constexpr FeGemvLine kFeGemvFp8{8, 3.47f, 0.835f, 14.4e-6f, 1.544e-3f, 0.0f, 2.39e-6f, 5.01f, 0.768f, 0.68e-6f, 1.64f, -17.5e-6f, 0.0f, 1.11e-6f, 0.95f};
+// bf16 (steps of 64), up to 32 rows that are no decode rows. Fitted to 21244 linears of 17..32 rows (64 .. 96000 columns, K 256 .. 19456), half of either estimate within 5 %. By this rule
+// 0.832 of the GEMM's time in all, 194 more than 3 % slower than it, at most 25 % (the better one each time 0.824); with lines by rows times K alone (350000 up to 24 rows, 180000 up to 32) 0.862 of
+// 18642, 2207 slower, at most 2.1 times. us, GEMM -> GEMV at 17 / 24 / 32 rows: 17408 x 5120 40 -> 31, 31, 32; 34816 x 5120 77 -> 58, 79 -> 60, 81 -> 62; 5120 x 5120 17 -> 13, 15, 16; 1024 x 2816 8.7 -> 5.4,
+// 5.7, 6.1; not taken: 61728 x 256 at 31 7.6 -> 15.8, 55304 x 256 at 27 7.2 -> 14.5. From 33 rows on (three groups of 16) the GEMM is ahead wherever K is 5120 and more.
+constexpr FeGemvLine kFeGemvBf16{16, 0.91f, 1.236f, 15.0e-6f, 0.962e-3f, 0.894e-3f, 1.63e-6f, 3.05f, 0.681f, 4.69e-6f, 1.084f, -5.1e-6f, 0.0987e-6f, 0.0f, 0.97f};
+// bf16 gate and up (n each) in one launch against the GEMM with SwiGLU over their interleaved weights (its plan's): of 10529 calls 0.906 of the GEMM's time in all, 179 more than 3 %
+// slower, at most 28 % (the better one each time 0.901); by rows times K and inter 0.942 of 2284, 410 slower, at most 2.4 times. us, GEMM -> GEMV: 8512 x 3584 at 21 rows 29.2 -> 21.9, 1280 x 2560 at
+// 20 9.5 -> 7.0; not taken: 28480 x 256 at 22 7.8 -> 18.8, 15168 x 256 at 21 5.6 -> 9.8, 320 x 10752 at 20 12.9 -> 22.4.
+constexpr FeGemvLine kFeGemvBf16Pair{16, 2.19f, 0.371f, 28.7e-6f, 2.041e-3f, 1.674e-3f, 9.58e-6f, 3.55f, 0.689f, 11.0e-6f, 1.264f, 155e-6f, 0.0639e-6f, 5.86e-6f, 0.97f};
