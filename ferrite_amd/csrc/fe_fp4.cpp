@@ -614,14 +614,18 @@ int fe_fp4_linear_forward_swiglu(const fe_fp4_linear *l, const fe_fp4_kernels *k
     fe_devptr_t q_codes = act->codes.p, q_sf = act->sf.p, q_aq = act->aq.p;
     uint32_t w_snt = l->w_snt, w_skt = l->w_skt, w_sr = l->w_sr, s_snt = l->s_snt, s_skt = l->s_skt, s_sr = l->s_sr;
     // (stream-K only when forced: this kernel's stream-K form was slower wherever measured, 688 -> 714 us on 5120 x 34816)
-    const FeGemmPlan plan = fe_gemm_plan(m, n, k / 64, kern->cus, ws->part.p, ws->part.bytes, ws->counters.p, kGemvCounters, kern->gemm_splits,
-                                         kern->gemm_sk >= 2 ? kern->gemm_sk : 0, true, kFeCostNvfp4, kern->tile);
+    auto gemm_plan = [&](const FeGemmTileOptions &tile) {
+        return fe_gemm_plan(m, n, k / 64, kern->cus, ws->part.p, ws->part.bytes, ws->counters.p, kGemvCounters, kern->gemm_splits, kern->gemm_sk >= 2 ? kern->gemm_sk : 0, true, kFeCostNvfp4, tile);
+    };
     const uint32_t sk = gemv_splits(kern, ws, n, k);
-    if (swiglu_takes_gemv(l, kern, m, sk, plan)) {
+    if (m <= kGemvRows && swiglu_takes_gemv(l, kern, m, sk, gemm_plan(kern->tile))) {  // (fitted to the plans of a plain launch)
         fe_devptr_t cnt = ws->counters.p;
         void *args[] = {&aq, &w, &sw, &alpha, &part, &cnt, &m, &n, &k, (void *)&sk, &w_snt, &w_skt, &w_sr, &s_snt, &s_skt, &s_sr, &q_codes, &q_sf, &q_aq, &down_g};
         return fe_hip_launch(kern->gemv_swiglu4[w_sr != 32][(m + 15) / 16 - 1], n / kTile * sk, 1, 1, 256, 1, 1, 0, s, args);
     }
+    FeGemmTileOptions tile = kern->tile;
+    tile.nvfp4_front = true;
+    const FeGemmPlan plan = gemm_plan(tile);
     if (!plan.tile && plan.big.stream_k && kern->xcd < 0) group = 1;
     return fe_gemm_launch(
         plan,

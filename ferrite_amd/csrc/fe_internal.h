@@ -278,6 +278,7 @@ struct FeGemmPlan {
 struct FeGemmTileOptions {
     uint32_t force_tile = 0, force_pieces = 0;
     bool low = false;  // the handle has kernels of tiles 3..5 (force_tile 4, 5, 6)
+    bool nvfp4_front = false;  // an NVFP4 launch with SwiGLU and the quantizer behind it
     // option "gemm_tile": refused past the tiles that the handle has kernels of (fe_gemm_plan and the tables of kernels are indexed by it)
     bool set(int64_t value) {
         if (value < 0 || value > (low ? kFeGemmTiles : 3u)) return false;
@@ -420,7 +421,9 @@ inline FeGemmPlan fe_gemm_plan(uint32_t m, uint32_t n, uint32_t ktiles, uint32_t
     // / 0.950 / 0.982 / 0.953 / 0.952).
     const FeGemmSchedule lower = low(pick);
     if (p.tile) {
-        if (ktiles < 12 || 2 * lower.split.programs() < cus) return p;
+        // (Of an NVFP4 SwiGLU front with 16..23 k tiles, which small tiles may cut in two only, lower ones also with fewer programs: 45 launches of up to 16 tiles 0.82 of the small tiles' time;
+        // with 24..31, three pieces, 1.15, and of plain linears of 20..23 1.14.)
+        if (ktiles < 12 || (2 * lower.split.programs() < cus && !(opt.nvfp4_front && ktiles >= 16 && ktiles < 24))) return p;
         // Dense weights (bf16, FP8) in fewer lower tiles than a quarter of the CUs: deep narrow linears, which small tiles cut finer than eight pieces of a lower one (bf16:
         // 826 launches 1.16 times the small tiles' time, from there on 0.90). More lower tiles than CUs and short K: rounds of them want a clearer gain (48 of FP8 1.01, bf16 past 0.9 level;
         // not so from 24 k tiles on: 5120 x 17408 at 559 rows, NVFP4 block 290 us with them, 305 without).

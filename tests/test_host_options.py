@@ -165,7 +165,8 @@ LOWER = {("nvfp4", 636, 5248, 256): (9.2, 13.1), ("nvfp4", 449, 768, 1536): (14.
          ("bf16", 764, 2304, 8704): (40.8, 48.0), ("fp8", 711, 33536, 2048): (65.2, 70.8), ("fp8", 1516, 28672, 1792): (92.8, 102.6), ("nvfp4", 1313, 11008, 768): (33.5, 37.9),
          ("bf16", 1035, 8192, 1792): (42.1, 33.1), ("bf16", 1041, 4608, 7680): (88.7, 73.5), ("bf16", 469, 16640, 1280): (33.7, 25.5), ("fp8", 1253, 7168, 2560): (38.2, 32.3),
          ("nvfp4", 1159, 6912, 3328): (72.2, 58.6), ("nvfp4", 1528, 3840, 9216): (119.5, 98.4),
-         ("bf16", 365, 38400, 5632): (179.6, 162.4), ("bf16", 195, 33280, 3840): (80.6, 72.5), ("nvfp4", 839, 25600, 1792): (87.7, 74.5), ("nvfp4", 840, 25856, 3328): (148.2, 130.3)}
+         ("bf16", 365, 38400, 5632): (179.6, 162.4), ("bf16", 195, 33280, 3840): (80.6, 72.5), ("nvfp4", 839, 25600, 1792): (87.7, 74.5), ("nvfp4", 840, 25856, 3328): (148.2, 130.3),
+         ("front", 147, 512, 1024): (19.5, 15.0), ("front", 91, 768, 1024): (19.2, 14.5), ("front", 82, 1024, 1280): (16.7, 15.0), ("front", 165, 1024, 1024): (19.9, 16.2)}
 
 
 def test_a_lower_tile_takes_a_small_ones_place_where_that_was_timed_faster(tmp_path):
@@ -174,9 +175,9 @@ def test_a_lower_tile_takes_a_small_ones_place_where_that_was_timed_faster(tmp_p
 int main() {{
     struct {{ const char *form; uint32_t m, n, k; }} calls[] = {{{calls}}};
     for (auto &c : calls) {{
-        const bool f8 = c.form[0] == 'f', bf = c.form[0] == 'b';
-        const FeGemmPlan p = fe_gemm_plan(c.m, c.n, c.k / (f8 ? 128 : 64), 256, 1, (size_t)512 * kFeGemmPartBytes, 1, 8192, 8, bf ? 0 : 1, !f8 && !bf,
-                                          f8 ? kFeCostFp8 : bf ? kFeCostBf16 : kFeCostNvfp4, FeGemmTileOptions{{0, 0, true}});
+        const bool f8 = c.form[0] == 'f' && c.form[1] == 'p', front = c.form[0] == 'f' && !f8, bf = c.form[0] == 'b';
+        const FeGemmPlan p = fe_gemm_plan(c.m, c.n, c.k / (f8 ? 128 : 64), 256, 1, (size_t)512 * kFeGemmPartBytes, 1, 8192, 8, bf || front ? 0 : 1, !f8 && !bf,
+                                          f8 ? kFeCostFp8 : bf ? kFeCostBf16 : kFeCostNvfp4, FeGemmTileOptions{{0, 0, true, front}});
         printf("%d\\n", p.tile >= 3 ? 1 : p.tile ? 0 : 2);
     }}
 }}
