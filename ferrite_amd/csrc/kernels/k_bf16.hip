@@ -4,17 +4,19 @@
 
 #include "gemm8.h"
 
-// 4 sums of columns at.. of one row -> bf16; with res: bf16(bf16(sum) + res) (gemm.rs:152-158).
-__device__ __forceinline__ void bf16_store4(uint16_t* c, const uint16_t* res, size_t at, const float (&v)[4]) {
+// 4 sums of columns at.. of one row -> bf16; where a residual is added: bf16(bf16(sum) + old) (gemm.rs:152-158).
+__device__ __forceinline__ void bf16_store4(uint16_t* c, bool adds, u32x2 old, size_t at, const float (&v)[4]) {
     u32x2 o = {pack_bf16x2(v[0], v[1]), pack_bf16x2(v[2], v[3])};
-    if (res) {
-        u32x2 r = *(const u32x2*)(res + at);
+    if (adds) {
 #pragma unroll
         for (int e = 0; e < 2; e++)
-            o[e] = pack_bf16x2(bf16_bits_to_f32(o[e] & 0xffff) + bf16_bits_to_f32(r[e] & 0xffff),
-                               bf16_bits_to_f32(o[e] >> 16) + bf16_bits_to_f32(r[e] >> 16));
+            o[e] = pack_bf16x2(bf16_bits_to_f32(o[e] & 0xffff) + bf16_bits_to_f32(old[e] & 0xffff),
+                               bf16_bits_to_f32(o[e] >> 16) + bf16_bits_to_f32(old[e] >> 16));
     }
     *(u32x2*)(c + at) = o;
+}
+__device__ __forceinline__ void bf16_store4(uint16_t* c, const uint16_t* res, size_t at, const float (&v)[4]) {
+    bf16_store4(c, res != nullptr, res ? *(const u32x2*)(res + at) : (u32x2){0, 0}, at, v);
 }
 
 // ---- GEMM ------------------------------------------------------------------------------------------------------------
@@ -65,13 +67,19 @@ __device__ __forceinline__ void bf16_gemm_program(const uint16_t* a, const uint1
             if (row < m && col < n) bf16_store4(c, res, (size_t)row * ldc + col, v);                                       \
         });                                                                                                                \
     }                                                                                                                      \
-    extern "C" __global__ __launch_bounds__(256) void fe_gemm_bf16_reduce##SUFFIX(                                         \
+    extern "C" __global__ __launch_bounds__(512) void fe_gemm_bf16_reduce##SUFFIX(                                         \
         uint16_t* c, const float* part, const uint16_t* res, uint32_t m, uint32_t n, uint32_t ldc, uint32_t group_m,       \
         uint32_t first, uint32_t splits) {                                                                                 \
-        g8_reduce_rows<TILE>(part, m, n, group_m, first, splits, [&](uint32_t row, uint32_t n0, uint32_t l32, float (&v)[4]) { \
-            const uint32_t col = n0 + 4 * l32;                                                                             \
-            if (row < m && col < n) bf16_store4(c, res, (size_t)row * ldc + col, v);                                       \
-        });                                                                                                                \
+        g8_reduce_rows<TILE>(                                                                                              \
+            part, m, n, group_m, first, splits,                                                                            \
+            [&](uint32_t row, uint32_t n0, uint32_t l32) {                                                                 \
+                const uint32_t col = n0 + 4 * l32;                                                                         \
+                return res && row < m && col < n ? *(const u32x2*)(res + (size_t)row * ldc + col) : (u32x2){0, 0};         \
+            },                                                                                                             \
+            [&](uint32_t row, uint32_t n0, uint32_t l32, float (&v)[4], u32x2 old) {                                       \
+                const uint32_t col = n0 + 4 * l32;                                                                         \
+                if (row < m && col < n) bf16_store4(c, res != nullptr, old, (size_t)row * ldc + col, v);                   \
+            });                                                                                                            \
     }
 BF16_GEMM_KERNELS(, Bf16Tile)
 BF16_GEMM_KERNELS(_s1, Bf16TileS1)
@@ -106,11 +114,12 @@ __device__ __forceinline__ void bf16_swiglu_store4(uint16_t* act, const float (&
             bf16_swiglu_store4(act, v, lc, row < m, row, col, n);                                                          \
         });                                                                                                                \
     }                                                                                                                      \
-    extern "C" __global__ __launch_bounds__(256) void fe_gemm_bf16_swiglu_reduce##SUFFIX(                                  \
+    extern "C" __global__ __launch_bounds__(512) void fe_gemm_bf16_swiglu_reduce##SUFFIX(                                  \
         uint16_t* act, const float* part, uint32_t m, uint32_t n, uint32_t group_m, uint32_t first, uint32_t splits) {      \
-        g8_reduce_rows<TILE>(part, m, n, group_m, first, splits, [&](uint32_t row, uint32_t n0, uint32_t l32, float (&v)[4]) { \
-            bf16_swiglu_store4(act, v, l32, row < m, row, n0 + 4 * l32, n);                                                \
-        });                                                                                                                \
+        g8_reduce_rows<TILE>(part, m, n, group_m, first, splits, [](uint32_t, uint32_t, uint32_t) { return 0u; },          \
+                             [&](uint32_t row, uint32_t n0, uint32_t l32, float (&v)[4], uint32_t) {                       \
+                                 bf16_swiglu_store4(act, v, l32, row < m, row, n0 + 4 * l32, n);                           \
+                             });                                                                                           \
     }
 BF16_SWIGLU_KERNELS(, Bf16Tile)
 BF16_SWIGLU_KERNELS(_s1, Bf16TileS1)

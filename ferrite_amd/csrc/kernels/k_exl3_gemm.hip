@@ -223,13 +223,23 @@ __device__ __forceinline__ void exl3_gemm_hat_kernel(HAT_GEMM_PARAMS) {
                           });
 }
 // Finishes the tiles that a GEMM kernel cut along K: sums their partial slots and applies the output rotation and scale.
-// grid: cut tiles * (BM / 8) * (BN / 128), 256 threads.
+// grid: cut tiles * (BM / 16) * (BN / 128), 512 threads.
 template <class T>
 __device__ __forceinline__ void exl3_reduce_body(const float* part, const uint16_t* svh, void* y, uint32_t n, uint32_t m, uint32_t y_mode,
                                                  uint32_t group_m, uint32_t first, uint32_t splits) {
-    g8_reduce_rows<T>(part, m, n, group_m, first, splits, [&](uint32_t row, uint32_t n0, uint32_t l32, float (&v)[4]) {
-        if (row < m) finish_row(v, l32, svh, n0 + 4 * l32, y, y_mode, (size_t)row * n + n0 + 4 * l32);
-    });
+    struct Ahead {
+        u32x2 sv;
+        u32x4 old;
+    };
+    g8_reduce_rows<T>(
+        part, m, n, group_m, first, splits,
+        [&](uint32_t row, uint32_t n0, uint32_t l32) {
+            const uint32_t col = n0 + 4 * l32;
+            return Ahead{*(const u32x2*)(svh + col), row < m ? store4_old(y, y_mode, (size_t)row * n + col) : (u32x4){0, 0, 0, 0}};
+        },
+        [&](uint32_t row, uint32_t n0, uint32_t l32, float (&v)[4], Ahead a) {
+            if (row < m) finish_row(v, l32, a.sv, y, y_mode, (size_t)row * n + n0 + 4 * l32, a.old);
+        });
 }
 #define HAT_GEMM_KERNEL(SUFFIX, TILE, SK)                                                                                  \
     extern "C" __global__ __launch_bounds__(512, Exl3Waves<TILE>::MIN) void exl3_gemm_hat##SUFFIX(HAT_GEMM_PARAMS) {       \
@@ -240,7 +250,7 @@ HAT_GEMM_KERNEL(_sk, Exl3Tile, true)
 HAT_GEMM_KERNEL(_s1, Exl3TileS1, false)
 HAT_GEMM_KERNEL(_s2, Exl3TileS2, false)
 #define REDUCE_KERNEL(SUFFIX, TILE)                                                                                        \
-    extern "C" __global__ __launch_bounds__(256) void exl3_gemm_reduce##SUFFIX(                                            \
+    extern "C" __global__ __launch_bounds__(512) void exl3_gemm_reduce##SUFFIX(                                            \
         const float* part, const uint16_t* svh, void* y, uint32_t n, uint32_t m, uint32_t y_mode, uint32_t group_m,        \
         uint32_t first, uint32_t splits) {                                                                                 \
         exl3_reduce_body<TILE>(part, svh, y, n, m, y_mode, group_m, first, splits);                                        \

@@ -274,16 +274,19 @@ struct Fp4Packed {
 #define FP4_OPERAND_SCALE 0.0625f
 
 // One row piece of the output: 4 columns from `col` of row `grow`, bf16((sum) * alpha) (+ res: bf16(bf16(.) + res)).
-__device__ __forceinline__ void fp4_store4(uint16_t* c, const uint16_t* res, size_t at, const float (&v)[4], f32x4 al) {
+// (adds, old: whether a residual is added, and its four values)
+__device__ __forceinline__ void fp4_store4(uint16_t* c, bool adds, u32x2 old, size_t at, const float (&v)[4], f32x4 al) {
     u32x2 o = {pack_bf16x2(v[0] * al[0], v[1] * al[1]), pack_bf16x2(v[2] * al[2], v[3] * al[3])};
-    if (res) {
-        u32x2 r = *(const u32x2*)(res + at);
+    if (adds) {
 #pragma unroll
         for (int e = 0; e < 2; e++)
-            o[e] = pack_bf16x2(bf16_bits_to_f32(o[e] & 0xffff) + bf16_bits_to_f32(r[e] & 0xffff),
-                               bf16_bits_to_f32(o[e] >> 16) + bf16_bits_to_f32(r[e] >> 16));
+            o[e] = pack_bf16x2(bf16_bits_to_f32(o[e] & 0xffff) + bf16_bits_to_f32(old[e] & 0xffff),
+                               bf16_bits_to_f32(o[e] >> 16) + bf16_bits_to_f32(old[e] >> 16));
     }
     *(u32x2*)(c + at) = o;
+}
+__device__ __forceinline__ void fp4_store4(uint16_t* c, const uint16_t* res, size_t at, const float (&v)[4], f32x4 al) {
+    fp4_store4(c, res != nullptr, res ? *(const u32x2*)(res + at) : (u32x2){0, 0}, at, v, al);
 }
 
 // ---- FP8 (e4m3, one scale per tensor) -------------------------------------------------------------------------------------
@@ -497,14 +500,29 @@ __device__ __forceinline__ void fp_gemm_body(MakePacked make_packed, const FpOut
         });
 }
 
-// Finishes the tiles that a GEMM kernel cut along K. grid: cut tiles * (BM / 8) * (BN / 128), 256 threads.
+// Finishes the tiles that a GEMM kernel cut along K. grid: cut tiles * (BM / 16) * (BN / 128), 512 threads.
 template <class T, bool SWIGLU>
 __device__ __forceinline__ void fp_reduce_body(const FpOut& out, const float* part, const float* alpha, float scale,
                                                uint32_t m, uint32_t n, uint32_t group_m, uint32_t first, uint32_t splits) {
-    g8_reduce_rows<T>(part, m, n, group_m, first, splits, [&](uint32_t row, uint32_t n0, uint32_t l32, float (&v)[4]) {
-        const uint32_t col = n0 + 4 * l32;
-        fp_store_piece<SWIGLU>(out, v, *(const f32x4*)(alpha + col) * scale, l32, row, m, col, n);
-    });
+    struct Ahead {
+        f32x4 al;
+        u32x2 old;
+    };
+    g8_reduce_rows<T>(
+        part, m, n, group_m, first, splits,
+        [&](uint32_t row, uint32_t n0, uint32_t l32) {
+            const uint32_t col = n0 + 4 * l32;
+            Ahead a = {*(const f32x4*)(alpha + col) * scale, {0, 0}};
+            if (!SWIGLU && out.res && row < m) a.old = *(const u32x2*)(out.res + (size_t)row * out.ldc + col);
+            return a;
+        },
+        [&](uint32_t row, uint32_t n0, uint32_t l32, float (&v)[4], const Ahead& a) {
+            const uint32_t col = n0 + 4 * l32;
+            if constexpr (SWIGLU)
+                fp_store_piece<true>(out, v, a.al, l32, row, m, col, n);
+            else if (row < m)
+                fp4_store4(out.c, out.res != nullptr, a.old, (size_t)row * out.ldc + col, v, a.al);
+        });
 }
 
 // NVFP4: the codes of row r = 128 nt + i, k tile kt are 32 bytes at w + nt * w_snt + kt * w_skt + i * w_sr, its 4 scales
@@ -540,7 +558,7 @@ FP4_GEMM_KERNEL(_h6, FpTileH6, false)
 FP4_GEMM_KERNEL(_h5, FpTileH5, false)
 
 #define FP_REDUCE_KERNEL(NAME, TILE)                                                                                       \
-    extern "C" __global__ __launch_bounds__(256) void NAME(uint16_t* c, const float* part, const float* alpha,             \
+    extern "C" __global__ __launch_bounds__(512) void NAME(uint16_t* c, const float* part, const float* alpha,             \
                                                            const uint16_t* res, uint32_t m, uint32_t n, uint32_t ldc,      \
                                                            uint32_t group_m, uint32_t first, uint32_t splits, float scale) { \
         FpOut out = {c, res, ldc, nullptr, nullptr, nullptr, 0.f};                                                         \
@@ -589,7 +607,7 @@ FP4_SWIGLU_KERNEL(_h7, FpTileH7, false)
 FP4_SWIGLU_KERNEL(_h6, FpTileH6, false)
 FP4_SWIGLU_KERNEL(_h5, FpTileH5, false)
 #define FP4_SWIGLU_REDUCE_KERNEL(SUFFIX, TILE)                                                                             \
-    extern "C" __global__ __launch_bounds__(256) void fe_gemm_nvfp4_swiglu_reduce##SUFFIX(                                 \
+    extern "C" __global__ __launch_bounds__(512) void fe_gemm_nvfp4_swiglu_reduce##SUFFIX(                                 \
         const float* part, const float* alpha, uint32_t m, uint32_t n, uint32_t group_m, uint32_t first, uint32_t splits,  \
         uint8_t* q_codes, uint8_t* q_sf, _Float16* q_aq, float qg) {                                                       \
         FpOut out = {nullptr, nullptr, 0, q_codes, q_sf, q_aq, qg};                                                        \
