@@ -882,28 +882,30 @@ __device__ __forceinline__ void gemv_wide_body(const GemvMember mb, uint32_t p, 
     uint32_t u = run_start(PER * p);
     const uint32_t uend = run_start(PER * p + PER < mb.programs ? PER * p + PER : mb.programs), mid = run_start(PER * p + 1);
     while (u < uend) {
-        const uint32_t nb = u / upb, in = u - nb * upb, units = uend - u < upb - in ? uend - u : upb - in, steps = 2 * units;
+        // A step's offsets and stages are running scalars: the quotient comes from the vector unit, and left there it takes the loads' offsets, a 32-bit multiply among them,
+        // and the stages along, 133..139 vector instructions a step where the decode takes 119; 123 so. A layer of 5120 / 17408 at 3 bits, 17 / 32 / 40 / 64 rows 90.3 / 94.5 / 104.8 /
+        // 122.5 -> 86.3 / 90.5 / 102.4 / 120.7 us, at 4 bits 88.9 / 93.3 / 105.6 / 125.9 -> 86.5 / 90.9 / 102.9 / 122.7, 9 rows 86.8 -> 84.7.
+        const uint32_t nb = __builtin_amdgcn_readfirstlane(u / upb), in = u - nb * upb, units = uend - u < upb - in ? uend - u : upb - in, steps = 2 * units;
         const uint32_t aside = mid > u && mid < u + units ? 2 * (mid - u) : steps;  // the step at which the second program's run starts
         u += units;
-        const uint32_t w0 = nb * mb.stride_nb * 4 + 2 * in * step_bytes, x0 = 2 * in * 128;
-        auto issue = [&](uint32_t s, uint32_t slot) {  // past the end: the last step again, never used
-            s = s < steps ? s : steps - 1;
+        uint32_t w_at = nb * mb.stride_nb * 4 + 2 * in * step_bytes, x_at = 2 * in * 128, left = steps;  // the next step to ask for
+        auto issue = [&](uint32_t x_to, uint32_t w_to) {
 #pragma unroll
-            for (int j = 0; j < C::LX; j++)
-                g8_load_lds16(xrs, lds0 + slot * C::X_STAGE + (wave + 4 * j) % (2 * RG) * 1024, vx[j], x0 + s * 128);
+            for (int j = 0; j < C::LX; j++) g8_load_lds16(xrs, x_to + (wave + 4 * j) % (2 * RG) * 1024, vx[j], x_at);
 #pragma unroll
-            for (int j = 0; j < C::LW; j++)
-                g8_load_lds16(wrs, lds0 + C::W_AT + slot * C::W_STAGE + (wave + 4 * j) % BITS * 1024, vw[j], w0 + s * step_bytes);
+            for (int j = 0; j < C::LW; j++) g8_load_lds16(wrs, w_to + (wave + 4 * j) % BITS * 1024, vw[j], w_at);
+            const bool more = --left != 0;  // past the end: the last step again, never used
+            x_at += more ? 128 : 0, w_at += more ? step_bytes : 0, left += more ? 0 : 1;
         };
 #pragma unroll
-        for (int s = 0; s < C::DEPTH - 1; s++) issue(s, s);
+        for (int s = 0; s < C::DEPTH - 1; s++) issue(lds0 + s * C::X_STAGE, lds0 + C::W_AT + s * C::W_STAGE);
 #pragma unroll
         for (int rg = 0; rg < RG; rg++) acc[rg][0] = acc[rg][1] = (f32x4){0.f, 0.f, 0.f, 0.f};
-        uint32_t slot = 0;
-        auto step = [&](uint32_t s) {
+        uint32_t slot = 0, to = C::DEPTH - 1;  // the stage of this step, the one that is free
+        auto step = [&]() {
             g8_loads_wait<(C::DEPTH - 2) * (C::LX + C::LW)>();
             g8_barrier();
-            issue(s + C::DEPTH - 1, slot ? slot - 1 : C::DEPTH - 1);
+            issue(lds0 + to * C::X_STAGE, lds0 + C::W_AT + to * C::W_STAGE);
             LaneWords<BITS> lw;
             const uint32_t* words = (const uint32_t*)(wp + slot * C::W_STAGE);
             if constexpr (BITS % 4 == 0) {
@@ -928,15 +930,15 @@ __device__ __forceinline__ void gemv_wide_body(const GemvMember mb, uint32_t p, 
                 acc[rg][0] = __builtin_amdgcn_mfma_f32_16x16x32_f16(op[0][1], b1, acc[rg][0], 0, 0, 0);
                 acc[rg][1] = __builtin_amdgcn_mfma_f32_16x16x32_f16(op[1][1], b1, acc[rg][1], 0, 0, 0);
             }
-            slot = slot + 1 == C::DEPTH ? 0 : slot + 1;
+            to = slot, slot = slot + 1 == C::DEPTH ? 0 : slot + 1;
         };
         if constexpr (PER == 1) {
-            for (uint32_t s = 0; s < steps; s++) step(s);
+            for (uint32_t s = 0; s < steps; s++) step();
         } else {
             f32x4 hold[RG][2] = {};
             uint32_t s = 0, stop = aside;
             for (;;) {
-                do step(s);
+                do step();
                 while (++s < stop);
                 if (s == steps) break;
 #pragma unroll
