@@ -414,7 +414,7 @@ __device__ __forceinline__ void gemvb_body(const GemvMember mb, uint32_t p0, uin
     // Rotating here: (row, 128-channel block) pairs of a chunk go to the half wavefronts: half wavefront hw takes blocks hw,
     // hw + 8, ... of every row. The first pair's loads go out ahead of the trellis loads (loads return in order), so
     // that the rotation runs while the first trellis words are still on their way.
-    const bool rotating = src.x != nullptr;
+    const bool rotating = CHAIN != 0 || src.x != nullptr;
     struct RotAt {
         size_t at, xat;
         uint32_t c, off;
@@ -660,7 +660,7 @@ __device__ __forceinline__ void gemvb_body(const GemvMember mb, uint32_t p0, uin
                     }
                 }
             };
-            if (m <= 8)
+            if (CHAIN != 0 || m <= 8)
                 rows_of(std::integral_constant<int, 1>{});
             else
                 rows_of(std::integral_constant<int, 2>{});
