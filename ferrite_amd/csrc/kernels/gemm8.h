@@ -251,44 +251,111 @@ __device__ __forceinline__ void g8_mainloop(const void* a, uint32_t lda, uint32_
 // Hands the wavefront's accumulators out row by row: 16 rows at a time pass through the wavefront's own LDS slab so that
 // LPR = 4 TN consecutive lanes hold the wavefront's 16 TN columns of one row, 4 a lane. U passes of 64 / LPR rows are in
 // flight together: transform(v[U][4], lane in row) works on all of them at once (no branches), then
-// store(row in 0 .. 16 TM - 1, lane in row, v[4]) is called for each. No workgroup barrier: a slab belongs to its wavefront.
-template <class T, class Transform, class Store>
-__device__ __forceinline__ void g8_epilogue(f32x4 (&acc)[T::TM][T::TN], unsigned char* lds, Transform transform, Store store) {
-    constexpr int LPR = 4 * T::TN, RP = 64 / LPR, PITCH = 16 * T::TN + 4, U = 16 / RP < 4 ? 16 / RP : 4;
+// store(row in 0 .. 16 TM - 1, lane in row, v[4], what ahead(row, lane in row) returned) is called for each. ahead: what store needs of memory, asked for 16 rows at a
+// time in front of the first of them: behind a store the next load waits for it (NVFP4 stream-K, 2048 rows of 5120 x 17408 with a residual 310 -> 300 us, FP8 185 -> 177.5). No workgroup barrier: a slab belongs to its wavefront.
+template <class T, class Transform, class Ahead, class Store>
+__device__ __forceinline__ void g8_epilogue(f32x4 (&acc)[T::TM][T::TN], unsigned char* lds, Transform transform, Ahead ahead, Store store) {
+    constexpr int LPR = 4 * T::TN, RP = 64 / LPR, PITCH = 16 * T::TN + 4, U = 16 / RP < 4 ? 16 / RP : 4, PASSES = 16 / RP;
     const uint32_t lane = threadIdx.x & 63, wave = threadIdx.x >> 6, fr = lane & 15, fc = lane >> 4;
     float* slab = (float*)(lds + wave * (16 * PITCH * 4));
     const uint32_t lr = lane / LPR, lc = lane % LPR;
+    typedef decltype(ahead(0u, 0u)) Old;
+    Old old[PASSES];
 #pragma unroll
     for (int i = 0; i < T::TM; i++) {
+#pragma unroll
+        for (int q = 0; q < PASSES; q++) old[q] = ahead(16 * i + RP * q + lr, lc);
 #pragma unroll
         for (int j = 0; j < T::TN; j++) *(f32x4*)(slab + fr * PITCH + 16 * j + 4 * fc) = acc[i][j];
         gm_slab_sync();
 #pragma unroll
-        for (int r0 = 0; r0 < 16; r0 += RP * U) {
+        for (int q0 = 0; q0 < PASSES; q0 += U) {
             float v[U][4];
 #pragma unroll
             for (int u = 0; u < U; u++) {
-                const f32x4 t = *(const f32x4*)(slab + (r0 + RP * u + lr) * PITCH + 4 * lc);
+                const f32x4 t = *(const f32x4*)(slab + (RP * (q0 + u) + lr) * PITCH + 4 * lc);
                 v[u][0] = t[0], v[u][1] = t[1], v[u][2] = t[2], v[u][3] = t[3];
             }
             transform(v, lc);
+            // All of them have arrived from here on, also those of rows that are not stored: a load left in flight would have the next segment of a stream-K form wait for
+            // everything at its start, its own first k tiles too (FP8, 2048 rows of 5120 x 17408 without a residual 169 -> 172.5 us).
+            if constexpr (!std::is_empty<Old>::value) {
 #pragma unroll
-            for (int u = 0; u < U; u++) store(16 * i + r0 + RP * u + lr, lc, v[u]);
+                for (int u = 0; u < U; u++) asm volatile("" : "+v"(old[q0 + u]));
+            }
+#pragma unroll
+            for (int u = 0; u < U; u++) store(16 * i + RP * (q0 + u) + lr, lc, v[u], old[q0 + u]);
         }
         gm_slab_sync();
     }
+}
+struct G8Nothing {};  // for epilogues that ask for nothing ahead
+__device__ __forceinline__ auto g8_ask_nothing() {
+    return [](uint32_t, uint32_t) { return G8Nothing{}; };
+}
+
+// a: its rows of 16 lanes 0, 2 and those of b, alternating; b: rows 1, 3 likewise.
+__device__ __forceinline__ void g8_swap16(uint32_t& a, uint32_t& b) {
+    const auto r = __builtin_amdgcn_permlane16_swap(a, b, false, false);
+    a = r[0], b = r[1];
+}
+typedef uint32_t u32x4_a8 __attribute__((ext_vector_type(4), aligned(8)));
+
+// The wavefront's accumulators as bf16 rows added to a residual: c = bf16(bf16(sum) + res), row stride ldc, both pointers at its first row and column; pack(sums, column tile)
+// -> two words of bf16. A lane holds 4 columns of a row in every column tile and trades the half of two tiles with the lane 16 away: 8 neighbouring columns a lane, without
+// LDS. rows, cols: those that exist from there on (cols a multiple of 8). What a residual costs is the trip to memory: asked for where it is added, row piece by row piece, each
+// load waits behind the store before it, 10 us a launch. Asked for 16 rows ahead, us, launches without / with one before -> now: bf16, 2048 rows of 8192 x 256 15.0 / 25.3 ->
+// 14.5 / 19.8, of 8192 x 4096 95 / 105 -> 95 / 99.5; FP8, 1000 rows of 5120 x 5120 34.2 / 40.9 -> 33.9 / 34.4, 512 of 17408 x 5120 55 / 65 -> 55 / 56; NVFP4, 2048 of 8192 x 512
+// 23.6 / 33.1 -> 23.4 / 27.5. Through the slab (g8_epilogue, asked for ahead as well) the first takes 21.8; without a residual the slab's whole lines are ahead (14.5 against 15.2).
+template <class T, class Pack>
+__device__ __forceinline__ void g8_add_bf16(f32x4 (&acc)[T::TM][T::TN], uint16_t* c, const uint16_t* res, uint32_t ldc, uint32_t rows, uint32_t cols, Pack pack) {
+    constexpr int TM = T::TM, TN = T::TN, P = TN / 2;
+    const uint32_t lane = threadIdx.x & 63, fr = lane & 15, fc = lane >> 4, cc = 16 * (fc & 1) + 8 * (fc >> 1);
+    auto run = [&](auto whole_tag) {
+        constexpr bool WHOLE = decltype(whole_tag)::value;
+        uint16_t* p = c + (size_t)fr * ldc + cc;
+        const uint16_t* r = res + (size_t)fr * ldc + cc;
+        auto in = [&](int i, int j) { return WHOLE || (16 * i + fr < rows && 32 * j + cc < cols); };
+        u32x4 old[2][P];
+        auto ask = [&](int i) {
+#pragma unroll
+            for (int j = 0; j < P; j++)
+                if (in(i, j)) old[i & 1][j] = *(const u32x4_a8*)(r + 32 * j);
+            r += (size_t)16 * ldc;
+        };
+        ask(0);
+#pragma unroll
+        for (int i = 0; i < TM; i++) {
+            if (!WHOLE && 16 * i >= rows) break;
+            if (i + 1 < TM) ask(i + 1);
+#pragma unroll
+            for (int j = 0; j < P; j++) {
+                const u32x2 a = pack(acc[i][2 * j], 2 * j), b = pack(acc[i][2 * j + 1], 2 * j + 1);
+                uint32_t a0 = a[0], a1 = a[1], b0 = b[0], b1 = b[1];
+                g8_swap16(a0, b0), g8_swap16(a1, b1);
+                if (in(i, j)) *(u32x4_a8*)(p + 32 * j) = add_bf16x8((u32x4){a0, a1, b0, b1}, old[i & 1][j]);
+            }
+            p += (size_t)16 * ldc;
+        }
+    };
+    if (rows >= 16 * TM && cols >= 16 * TN)
+        run(std::true_type{});
+    else
+        run(std::false_type{});
 }
 
 // A program's accumulators in its partial slot, as the lanes hold them: piece (i, j) of thread t at ((i TN + j) 512 + t) 16. rows: those of the tile that
 // exist; groups of 16 past them are left out.
 template <class T>
 __device__ __forceinline__ void g8_store_partial(f32x4 (&acc)[T::TM][T::TN], float* slot, uint32_t rows) {
-    const uint32_t row0 = (threadIdx.x >> 6) / T::WN * (16 * T::TM);
+    const uint32_t row0 = (threadIdx.x >> 6) / T::WN * (16 * T::TM), tid = threadIdx.x;
+    const __amdgpu_buffer_rsrc_t rs = __builtin_amdgcn_make_buffer_rsrc((void*)slot, 0, T::PART_FLOATS * 4, 0x00020000);  // (pieces by a scalar offset)
 #pragma unroll
     for (int i = 0; i < T::TM; i++)
         if (row0 + 16 * i < rows)
 #pragma unroll
-            for (int j = 0; j < T::TN; j++) *(f32x4*)(slot + ((i * T::TN + j) * T::THREADS + threadIdx.x) * 4) = acc[i][j];
+            for (int j = 0; j < T::TN; j++)
+                __builtin_amdgcn_raw_buffer_store_b128(__builtin_bit_cast(u32x4, acc[i][j]), rs, tid * 16, (i * T::TN + j) * T::THREADS * 16, 0);
 }
 
 // Body of a reduce kernel: grid = cut tiles * (BM / 16) * (BN / 128), 512 threads for 16 rows x 128 columns. A wavefront sums the `splits` slots of 16 of

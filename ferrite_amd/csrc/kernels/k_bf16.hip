@@ -15,9 +15,6 @@ __device__ __forceinline__ void bf16_store4(uint16_t* c, bool adds, u32x2 old, s
     }
     *(u32x2*)(c + at) = o;
 }
-__device__ __forceinline__ void bf16_store4(uint16_t* c, const uint16_t* res, size_t at, const float (&v)[4]) {
-    bf16_store4(c, res != nullptr, res ? *(const u32x2*)(res + at) : (u32x2){0, 0}, at, v);
-}
 
 // ---- GEMM ------------------------------------------------------------------------------------------------------------
 
@@ -33,13 +30,12 @@ struct Bf16Stages {
     static constexpr int NA = T::PARTS == 2 ? 3 : 2, NW = 3, MIN_WAVES = T::PARTS == 4 ? 4 : 2;
 };
 
-// One program's share of A . W^T: main loop, then the partial slot (a tile cut along K) or done(row, col, lane in row, v[4]) for
-// every row piece of the tile, all lanes of a row calling (row >= m and col >= n included).
-template <class T, class Done>
+// One program's share of A . W^T: main loop, then the partial slot (a tile cut along K) or finish(acc, lds, the wavefront's first row and column).
+template <class T, class Finish>
 __device__ __forceinline__ void bf16_gemm_program(const uint16_t* a, const uint16_t* w, uint32_t m, uint32_t n, uint32_t k, uint32_t lda,
-                                                  uint32_t group_m, const GemmSched& sc, Done done) {
+                                                  uint32_t group_m, const GemmSched& sc, Finish finish) {
     extern __shared__ __attribute__((aligned(1024))) unsigned char lds[];
-    const uint32_t wave = threadIdx.x >> 6, wm = wave / T::WN, wn = wave % T::WN;
+    const uint32_t wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6), wm = wave / T::WN, wn = wave % T::WN;
     g8_schedule<T, false>(
         sc, m, n, group_m, k / G8_BK, lds,
         [&](uint32_t m0, uint32_t n0, uint32_t kt0, uint32_t ktn, f32x4(&acc)[T::TM][T::TN]) {
@@ -48,10 +44,21 @@ __device__ __forceinline__ void bf16_gemm_program(const uint16_t* a, const uint1
             g8_mainloop<T, Bf16Stages<T>::NA, Bf16Stages<T>::NW, true, true>(a, lda, m, kt0, ktn, m0, wo, lds, acc);
         },
         [&](uint32_t m0, uint32_t n0, f32x4(&acc)[T::TM][T::TN]) {
-            const uint32_t row0 = m0 + wm * 16 * T::TM, col0 = n0 + wn * 16 * T::TN;
-            g8_epilogue<T>(
-                acc, lds, [](auto&, uint32_t) {},
-                [&](uint32_t row, uint32_t lc, float (&v)[4]) { done(row0 + row, col0 + 4 * lc, lc, v); });
+            finish(acc, lds, m0 + wm * 16 * T::TM, n0 + wn * 16 * T::TN);
+        });
+}
+
+// The wavefront's rows of a finished tile, from row0, col0 on.
+template <class T>
+__device__ __forceinline__ void bf16_tile_store(f32x4 (&acc)[T::TM][T::TN], unsigned char* lds, uint16_t* c, const uint16_t* res, uint32_t m, uint32_t n, uint32_t ldc,
+                                                uint32_t row0, uint32_t col0) {
+    if (row0 >= m || col0 >= n) return;
+    const size_t first = (size_t)row0 * ldc + col0;
+    if (res)
+        g8_add_bf16<T>(acc, c + first, res + first, ldc, m - row0, n - col0, [](f32x4 v, int) { return (u32x2){pack_bf16x2(v[0], v[1]), pack_bf16x2(v[2], v[3])}; });
+    else
+        g8_epilogue<T>(acc, lds, [](auto&, uint32_t) {}, g8_ask_nothing(), [&](uint32_t row, uint32_t lc, float (&v)[4], G8Nothing) {
+            if (row < m - row0 && 4 * lc < n - col0) bf16_store4(c, false, (u32x2){0, 0}, first + (size_t)row * ldc + 4 * lc, v);
         });
 }
 
@@ -63,8 +70,8 @@ __device__ __forceinline__ void bf16_gemm_program(const uint16_t* a, const uint1
     extern "C" __global__ __launch_bounds__(512, Bf16Stages<TILE>::MIN_WAVES) void fe_gemm_bf16##SUFFIX(                   \
         uint16_t* c, const uint16_t* a, const uint16_t* w, const uint16_t* res, uint32_t m, uint32_t n, uint32_t k,        \
         uint32_t lda, uint32_t ldc, uint32_t group_m, GemmSched sc) {                                                      \
-        bf16_gemm_program<TILE>(a, w, m, n, k, lda, group_m, sc, [&](uint32_t row, uint32_t col, uint32_t, float (&v)[4]) { \
-            if (row < m && col < n) bf16_store4(c, res, (size_t)row * ldc + col, v);                                       \
+        bf16_gemm_program<TILE>(a, w, m, n, k, lda, group_m, sc, [&](auto& acc, unsigned char* lds, uint32_t row0, uint32_t col0) { \
+            bf16_tile_store<TILE>(acc, lds, c, res, m, n, ldc, row0, col0);                                                \
         });                                                                                                                \
     }                                                                                                                      \
     extern "C" __global__ __launch_bounds__(512) void fe_gemm_bf16_reduce##SUFFIX(                                         \
@@ -110,8 +117,11 @@ __device__ __forceinline__ void bf16_swiglu_store4(uint16_t* act, const float (&
     extern "C" __global__ __launch_bounds__(512, Bf16Stages<TILE>::MIN_WAVES) void fe_gemm_bf16_swiglu##SUFFIX(            \
         uint16_t* act, const uint16_t* a, const uint16_t* w, uint32_t m, uint32_t n, uint32_t k, uint32_t lda,             \
         uint32_t group_m, GemmSched sc) {                                                                                  \
-        bf16_gemm_program<TILE>(a, w, m, n, k, lda, group_m, sc, [&](uint32_t row, uint32_t col, uint32_t lc, float (&v)[4]) { \
-            bf16_swiglu_store4(act, v, lc, row < m, row, col, n);                                                          \
+        bf16_gemm_program<TILE>(a, w, m, n, k, lda, group_m, sc, [&](auto& acc, unsigned char* lds, uint32_t row0, uint32_t col0) { \
+            g8_epilogue<TILE>(                                                                                             \
+                acc, lds, [](auto&, uint32_t) {}, g8_ask_nothing(), [&](uint32_t row, uint32_t lc, float (&v)[4], G8Nothing) { \
+                    bf16_swiglu_store4(act, v, lc, row0 + row < m, row0 + row, col0 + 4 * lc, n);                          \
+                });                                                                                                        \
         });                                                                                                                \
     }                                                                                                                      \
     extern "C" __global__ __launch_bounds__(512) void fe_gemm_bf16_swiglu_reduce##SUFFIX(                                  \

@@ -414,6 +414,8 @@ __device__ __forceinline__ void gemvb_body(const GemvMember mb, uint32_t p0, uin
     // Rotating here: (row, 128-channel block) pairs of a chunk go to the half wavefronts: half wavefront hw takes blocks hw,
     // hw + 8, ... of every row. The first pair's loads go out ahead of the trellis loads (loads return in order), so
     // that the rotation runs while the first trellis words are still on their way.
+    // (CHAIN: always, and up to 8 rows only, mlp_chain_fits. Code for what never comes is not free: with it the kernel is 47 KB, which with the 23 KB of the GEMV is more than the 64 KB of
+    // instructions that two CUs cache, and a layer's launches displace each other's: 5120 / 17408 at 4 bits, 1 row, two layers 135.1 -> 134.1 us, 1024 / 2816 26.28 -> 26.01.)
     const bool rotating = CHAIN != 0 || src.x != nullptr;
     struct RotAt {
         size_t at, xat;

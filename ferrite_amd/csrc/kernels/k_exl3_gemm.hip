@@ -105,7 +105,7 @@ template <class T, bool SK, class Loop>
 __device__ __forceinline__ void exl3_gemm_tile(const uint16_t* __restrict__ svh, void* y, uint32_t n, uint32_t k, uint32_t m,
                                                uint32_t y_mode, uint32_t group_m, const GemmSched& sched, Loop loop) {
     extern __shared__ __attribute__((aligned(1024))) unsigned char lds[];
-    const uint32_t lane = threadIdx.x & 63, wave = threadIdx.x >> 6, wm = wave / T::WN, wn = wave % T::WN;
+    const uint32_t lane = threadIdx.x & 63, wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6), wm = wave / T::WN, wn = wave % T::WN;
     g8_schedule<T, SK>(
         sched, m, n, group_m, k / G8_BK, lds,
         [&](uint32_t m0, uint32_t n0, uint32_t kt0, uint32_t ktn, f32x4(&acc)[T::TM][T::TN]) { loop(m0, n0, kt0, ktn, lds, acc); },
@@ -126,8 +126,18 @@ __device__ __forceinline__ void exl3_gemm_tile(const uint16_t* __restrict__ svh,
 #pragma unroll
                             for (int e = 0; e < 4; e++) v[u][e] = v[u][e] * FE_HAD_SCALE * sc[e];  // finish_row's products
                     },
-                    [&](uint32_t row, uint32_t, float (&v)[4]) {
-                        if (row0 + row < m) store4(y, MODE, (size_t)(row0 + row) * n + col, v);
+                    [&](uint32_t row, uint32_t) {
+                        if constexpr (MODE >= 2)
+                            return row0 + row < m ? store4_old(y, MODE, (size_t)(row0 + row) * n + col) : (u32x4){0, 0, 0, 0};
+                        else
+                            return G8Nothing{};
+                    },
+                    [&](uint32_t row, uint32_t, float (&v)[4], auto old) {
+                        if (row0 + row >= m) return;
+                        if constexpr (MODE >= 2)
+                            store4(y, MODE, (size_t)(row0 + row) * n + col, v, old);
+                        else
+                            store4(y, MODE, (size_t)(row0 + row) * n + col, v);
                     });
             };
             if (y_mode == 0)

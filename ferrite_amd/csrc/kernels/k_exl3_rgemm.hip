@@ -253,13 +253,20 @@ __device__ __forceinline__ void rgemm_segment(const RgJob& job, uint32_t tile, u
                     const f32x4 s = *(const f32x4*)(red + row * PITCH + b * 132 + 4 * l32);
                     v[u][0] = s[0], v[u][1] = s[1], v[u][2] = s[2], v[u][3] = s[3];
                 }
+                // (the old outputs of all four asked for together: behind a store the next load waits for it)
+                u32x4 old[4];
+#pragma unroll
+                for (int u = 0; u < 4; u++) {
+                    const uint32_t row = q0 + u * step_rows;
+                    old[u] = live && row < here ? store4_old(mb.y, MODE, (size_t)(m0 + row0 + row) * n + col) : (u32x4){0, 0, 0, 0};
+                }
                 fwht128_half_wave_rows(v, l32);
 #pragma unroll
                 for (int u = 0; u < 4; u++) {
 #pragma unroll
                     for (int e = 0; e < 4; e++) v[u][e] = v[u][e] * FE_HAD_SCALE * sc[e];
                     const uint32_t row = q0 + u * step_rows;
-                    if (live && row < here) store4(mb.y, MODE, (size_t)(m0 + row0 + row) * n + col, v[u]);
+                    if (live && row < here) store4(mb.y, MODE, (size_t)(m0 + row0 + row) * n + col, v[u], old[u]);
                 }
             }
         });

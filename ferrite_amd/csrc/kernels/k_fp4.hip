@@ -445,15 +445,50 @@ struct FpOut {
     float qg;
 };
 
-// One row piece: 4 sums of columns col.. of row grow. SWIGLU: every lane of the half wavefront takes part.
-template <bool SWIGLU>
-__device__ __forceinline__ void fp_store_piece(const FpOut& o, const float (&v)[4], f32x4 al, uint32_t l32, uint32_t grow,
-                                               uint32_t m, uint32_t col, uint32_t n) {
-    if constexpr (SWIGLU) {
-        swiglu_quant_store(v, al, l32, grow < m, grow < m ? grow : 0, col, n, o.q_codes, o.q_sf, o.q_aq, o.qg);
-    } else {
-        if (grow < m) fp4_store4(o.c, o.res, (size_t)grow * o.ldc + col, v, al);
+// The wavefront's rows of a finished tile, from row0, colb (inside n) on: sums times alpha * scale. (The stream-K forms add a residual row piece by row piece, too: g8_add_bf16's
+// registers, beside what their loop over segments keeps, would cost 30 spilled ones.)
+template <class T, bool SWIGLU, bool SK>
+__device__ __forceinline__ void fp_tile_store(f32x4 (&acc)[T::TM][T::TN], unsigned char* lds, const FpOut& o, const float* alpha, float scale, uint32_t m, uint32_t n,
+                                              uint32_t row0, uint32_t colb) {
+    const uint32_t lane = threadIdx.x & 63, col = colb + 4 * (lane % (4 * T::TN));
+    if constexpr (!SWIGLU && !SK) {
+        if (o.res) {
+            if (row0 >= m) return;
+            f32x4 al[T::TN];
+#pragma unroll
+            for (int j = 0; j < T::TN; j++) al[j] = *(const f32x4*)(alpha + colb + 16 * j + 4 * (lane >> 4)) * scale;
+            const size_t first = (size_t)row0 * o.ldc + colb;
+            g8_add_bf16<T>(acc, o.c + first, o.res + first, o.ldc, m - row0, n - colb, [&](f32x4 v, int j) {
+                return (u32x2){pack_bf16x2(v[0] * al[j][0], v[1] * al[j][1]), pack_bf16x2(v[2] * al[j][2], v[3] * al[j][3])};
+            });
+            return;
+        }
     }
+    const f32x4 al = *(const f32x4*)(alpha + col) * scale;
+    auto rows = [&](auto adds_tag) {
+        constexpr bool ADDS = decltype(adds_tag)::value;
+        g8_epilogue<T>(
+            acc, lds, [](auto&, uint32_t) {},
+            [&](uint32_t r, uint32_t) {
+                if constexpr (ADDS)
+                    return row0 + r < m ? *(const u32x2*)(o.res + (size_t)(row0 + r) * o.ldc + col) : (u32x2){0, 0};
+                else
+                    return G8Nothing{};
+            },
+            [&](uint32_t r, uint32_t lc, float (&v)[4], auto old) {
+                const uint32_t row = row0 + r;
+                if constexpr (SWIGLU)
+                    swiglu_quant_store(v, al, lc, row < m, row < m ? row : 0, col, n, o.q_codes, o.q_sf, o.q_aq, o.qg);
+                else if constexpr (ADDS) {
+                    if (row < m) fp4_store4(o.c, true, old, (size_t)row * o.ldc + col, v, al);
+                } else if (row < m)
+                    fp4_store4(o.c, false, (u32x2){0, 0}, (size_t)row * o.ldc + col, v, al);
+            });
+    };
+    if (SK && !SWIGLU && o.res)
+        rows(std::bool_constant<SK && !SWIGLU>{});
+    else
+        rows(std::false_type{});
 }
 
 // Tiles of 256 x 256, 128 x 256 (S1), 128 x 128 (S2) and 224, 192, 160 x 256 (H7, H6, H5). Packed weights: a wavefront's columns are a quarter of the tile's, so
@@ -482,7 +517,7 @@ __device__ __forceinline__ void fp_gemm_body(MakePacked make_packed, const FpOut
                                              float scale, uint32_t m, uint32_t n, uint32_t k, uint32_t group_m,
                                              const GemmSched& sc) {
     extern __shared__ __attribute__((aligned(1024))) unsigned char lds[];
-    const uint32_t lane = threadIdx.x & 63, wave = threadIdx.x >> 6, wm = wave / T::WN, wn = wave % T::WN;
+    const uint32_t wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6), wm = wave / T::WN, wn = wave % T::WN;
     g8_schedule<T, SK>(
         sc, m, n, group_m, k / G8_BK, lds,
         [&](uint32_t m0, uint32_t n0, uint32_t kt0, uint32_t ktn, f32x4(&acc)[T::TM][T::TN]) {
@@ -492,11 +527,7 @@ __device__ __forceinline__ void fp_gemm_body(MakePacked make_packed, const FpOut
         [&](uint32_t m0, uint32_t n0, f32x4(&acc)[T::TM][T::TN]) {
             const uint32_t row0 = m0 + wm * 16 * T::TM, colb = n0 + wn * 16 * T::TN;
             if (colb >= n) return;
-            const uint32_t col = colb + 4 * (lane % (4 * T::TN));
-            const f32x4 al = *(const f32x4*)(alpha + col) * scale;
-            g8_epilogue<T>(
-                acc, lds, [](auto&, uint32_t) {},
-                [&](uint32_t row, uint32_t lc, float (&v)[4]) { fp_store_piece<SWIGLU>(out, v, al, lc, row0 + row, m, col, n); });
+            fp_tile_store<T, SWIGLU, SK>(acc, lds, out, alpha, scale, m, n, row0, colb);
         });
 }
 
@@ -519,7 +550,7 @@ __device__ __forceinline__ void fp_reduce_body(const FpOut& out, const float* pa
         [&](uint32_t row, uint32_t n0, uint32_t l32, float (&v)[4], const Ahead& a) {
             const uint32_t col = n0 + 4 * l32;
             if constexpr (SWIGLU)
-                fp_store_piece<true>(out, v, a.al, l32, row, m, col, n);
+                swiglu_quant_store(v, a.al, l32, row < m, row < m ? row : 0, col, n, out.q_codes, out.q_sf, out.q_aq, out.qg);
             else if (row < m)
                 fp4_store4(out.c, out.res != nullptr, a.old, (size_t)row * out.ldc + col, v, a.al);
         });
@@ -653,7 +684,7 @@ template <class T, bool SK>
 __device__ __forceinline__ void gemm_fp8_codes_kernel(FP8C_GEMM_PARAMS) {
     constexpr int NA = T::PARTS == 2 ? 3 : 2;
     extern __shared__ __attribute__((aligned(1024))) unsigned char lds[];
-    const uint32_t nts = n / 128, lane = threadIdx.x & 63, wave = threadIdx.x >> 6, wm = wave / T::WN, wn = wave % T::WN;
+    const uint32_t nts = n / 128, lane = threadIdx.x & 63, wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6), wm = wave / T::WN, wn = wave % T::WN;
     FpOut out = {c, res, ldc, nullptr, nullptr, nullptr, 0.f};
     g8_schedule<T, SK>(
         sc, m, n, group_m, k / 128, lds,
@@ -673,11 +704,7 @@ __device__ __forceinline__ void gemm_fp8_codes_kernel(FP8C_GEMM_PARAMS) {
         [&](uint32_t m0, uint32_t n0, f32x4(&acc)[T::TM][T::TN]) {
             const uint32_t row0 = m0 + wm * 16 * T::TM, colb = n0 + wn * 16 * T::TN;
             if (colb >= n) return;
-            const uint32_t col = colb + 4 * (lane % (4 * T::TN));
-            const f32x4 al = *(const f32x4*)(alpha + col);
-            g8_epilogue<T>(
-                acc, lds, [](auto&, uint32_t) {},
-                [&](uint32_t r, uint32_t lc, float (&v)[4]) { fp_store_piece<false>(out, v, al, lc, row0 + r, m, col, n); });
+            fp_tile_store<T, false, SK>(acc, lds, out, alpha, 1.0f, m, n, row0, colb);
         });
 }
 #define FP8C_GEMM_KERNEL(SUFFIX, TILE, SK)                                                                                 \

@@ -31,6 +31,13 @@ __device__ __forceinline__ uint32_t pack_bf16x2(float lo, float hi) {
     f32x2 v = {lo, hi};
     return __builtin_bit_cast(uint32_t, __builtin_convertvector(v, bf16x2));
 }
+// bf16(a + b) of 4 pairs
+__device__ __forceinline__ u32x4 add_bf16x8(u32x4 a, u32x4 b) {
+#pragma unroll
+    for (int e = 0; e < 4; e++)
+        a[e] = pack_bf16x2(bf16_bits_to_f32(a[e] & 0xffff) + bf16_bits_to_f32(b[e] & 0xffff), bf16_bits_to_f32(a[e] >> 16) + bf16_bits_to_f32(b[e] >> 16));
+    return a;
+}
 
 __device__ __forceinline__ float f16_bits_to_f32(uint32_t h) {
     return (float)__builtin_bit_cast(_Float16, (uint16_t)h);
