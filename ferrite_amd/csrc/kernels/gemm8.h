@@ -294,9 +294,13 @@ __device__ __forceinline__ auto g8_ask_nothing() {
     return [](uint32_t, uint32_t) { return G8Nothing{}; };
 }
 
-// a: its rows of 16 lanes 0, 2 and those of b, alternating; b: rows 1, 3 likewise.
+// a: its rows of 16 lanes 0, 2 and those of b, alternating; b: rows 1, 3 likewise. And the same with halves of the wavefront.
 __device__ __forceinline__ void g8_swap16(uint32_t& a, uint32_t& b) {
     const auto r = __builtin_amdgcn_permlane16_swap(a, b, false, false);
+    a = r[0], b = r[1];
+}
+__device__ __forceinline__ void g8_swap32(uint32_t& a, uint32_t& b) {
+    const auto r = __builtin_amdgcn_permlane32_swap(a, b, false, false);
     a = r[0], b = r[1];
 }
 typedef uint32_t u32x4_a8 __attribute__((ext_vector_type(4), aligned(8)));

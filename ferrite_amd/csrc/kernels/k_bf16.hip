@@ -111,6 +111,34 @@ __device__ __forceinline__ void bf16_swiglu_store4(uint16_t* act, const float (&
     *(u32x2*)(act + (size_t)grow * (n >> 1) + (col >> 4) * 8 + 4 * (l32 & 1)) = o;
 }
 
+// The same for a finished tile, without LDS: the gate sums of a column tile lie in the wavefront's lower half and the up sums in its upper half, so two tiles trade halves, after
+// which every lane has gate and up of 4 features; and two such pairs trade rows of 16 lanes, after which it has 8 features of a row. (Through the slab half of the lanes
+// computed what they did not store: an MLP block of 1000 rows of 5120 / 17408 465.7 -> 456.0 us.)
+template <class T>
+__device__ __forceinline__ void bf16_tile_swiglu(f32x4 (&acc)[T::TM][T::TN], uint16_t* act, uint32_t m, uint32_t n, uint32_t row0, uint32_t col0) {
+    static_assert(T::TN % 4 == 0, "two pairs of column tiles");
+    if (row0 >= m || col0 >= n) return;
+    const uint32_t lane = threadIdx.x & 63, fr = lane & 15, fc = lane >> 4, ct = (fc >> 1) + 2 * (fc & 1);  // of four column tiles the one whose features the lane stores
+    auto pair = [](f32x4 a, f32x4 b) {
+        uint32_t g0 = pack_bf16x2(a[0], a[1]), g1 = pack_bf16x2(a[2], a[3]), u0 = pack_bf16x2(b[0], b[1]), u1 = pack_bf16x2(b[2], b[3]);
+        g8_swap32(g0, u0), g8_swap32(g1, u1);
+        return (u32x2){silu_mul_bf16x2(g0, u0), silu_mul_bf16x2(g1, u1)};
+    };
+    uint16_t* p = act + (size_t)(row0 + fr) * (n >> 1) + (col0 >> 1) + 8 * ct;
+#pragma unroll
+    for (int i = 0; i < T::TM; i++) {
+        if (16 * i >= m - row0) break;
+#pragma unroll
+        for (int j = 0; j < T::TN; j += 4) {
+            const u32x2 x = pair(acc[i][j], acc[i][j + 1]), y = pair(acc[i][j + 2], acc[i][j + 3]);
+            uint32_t x0 = x[0], x1 = x[1], y0 = y[0], y1 = y[1];
+            g8_swap16(x0, y0), g8_swap16(x1, y1);
+            if (16 * i + fr < m - row0 && 16 * (j + ct) < n - col0) *(u32x4_a8*)(p + 8 * j) = (u32x4){x0, x1, y0, y1};
+        }
+        p += (size_t)8 * n;
+    }
+}
+
 // act[M][N / 2] = SwiGLU(A . W^T) for interleaved gate|up weights W [N][K], N % 16 == 0: fe_gemm_bf16 with the epilogue
 // above, and its reduce kernels. (kernels/k-core/src/gemm.rs:264-279: fe_gemm_swiglu)
 #define BF16_SWIGLU_KERNELS(SUFFIX, TILE)                                                                                  \
@@ -118,10 +146,7 @@ __device__ __forceinline__ void bf16_swiglu_store4(uint16_t* act, const float (&
         uint16_t* act, const uint16_t* a, const uint16_t* w, uint32_t m, uint32_t n, uint32_t k, uint32_t lda,             \
         uint32_t group_m, GemmSched sc) {                                                                                  \
         bf16_gemm_program<TILE>(a, w, m, n, k, lda, group_m, sc, [&](auto& acc, unsigned char* lds, uint32_t row0, uint32_t col0) { \
-            g8_epilogue<TILE>(                                                                                             \
-                acc, lds, [](auto&, uint32_t) {}, g8_ask_nothing(), [&](uint32_t row, uint32_t lc, float (&v)[4], G8Nothing) { \
-                    bf16_swiglu_store4(act, v, lc, row0 + row < m, row0 + row, col0 + 4 * lc, n);                          \
-                });                                                                                                        \
+            bf16_tile_swiglu<TILE>(acc, act, m, n, row0, col0);                                                            \
         });                                                                                                                \
     }                                                                                                                      \
     extern "C" __global__ __launch_bounds__(512) void fe_gemm_bf16_swiglu_reduce##SUFFIX(                                  \

@@ -432,6 +432,79 @@ __device__ __forceinline__ void swiglu_quant_store(const float (&v)[4], f32x4 al
     if (j == 0) q_sf[sf_tiled(row, blk, kb)] = (uint8_t)s8;
 }
 
+// The same for a finished tile of the GEMM, without LDS and with every lane at work (through the slab the lanes with up sums computed what they did not store): the gate sums
+// of a column tile lie in the wavefront's lower half and the up sums in its upper half, so the two tiles of a 16-feature block trade halves, after which lane group fc has gate and up
+// of the block's features 4 fc .. + 3; the block's maximum comes from the lanes 16 and 32 away; and two blocks trade rows of 16 lanes, so that a lane stores 8 features of one
+// (a tile with one block a wavefront: 4). rows: those that exist from row0 on.
+// Bound by its vector instructions, which no matrix instruction hides (a program has its CU alone): about 10 us a program through the slab, half of that now. Launch, us: 2048
+// rows of 34816 x 5120 558 -> 535, 390 rows 144 -> 132; MLP blocks of 2048 / 5 + 390 rows 888 -> 841, 287.5 -> 273.7 with the residual's loads ahead.
+template <class T>
+__device__ __forceinline__ void fp4_tile_swiglu(f32x4 (&acc)[T::TM][T::TN], const float* alpha, float scale, uint32_t row0, uint32_t rows, uint32_t colb, uint32_t n, uint8_t* q_codes,
+                                                uint8_t* q_sf, _Float16* q_aq, float qg) {
+    constexpr int TN = T::TN, STEP = TN % 4 == 0 ? 4 : 2;  // column tiles that are stored together
+    const uint32_t lane = threadIdx.x & 63, fr = lane & 15, fc = lane >> 4, inter = n >> 1, kb = inter >> 4;
+    f32x4 al[TN];
+#pragma unroll
+    for (int j = 0; j < TN; j++) al[j] = *(const f32x4*)(alpha + colb + 16 * j + 4 * fc) * scale;
+    struct Part {
+        uint32_t q, s8, o0, o1;  // 4 codes, the block's scale, the 4 values as the GEMM's operand
+    };
+    auto block = [&](f32x4 a, f32x4 b, f32x4 ala, f32x4 alb) {
+        a *= ala, b *= alb;
+        uint32_t g[2] = {pack_bf16x2(a[0], a[1]), pack_bf16x2(a[2], a[3])}, u[2] = {pack_bf16x2(b[0], b[1]), pack_bf16x2(b[2], b[3])};
+        g8_swap32(g[0], u[0]), g8_swap32(g[1], u[1]);
+        float act[4], amax = 0.f;
+#pragma unroll
+        for (int e = 0; e < 4; e++) {
+            const uint32_t gw = g[e >> 1], uw = u[e >> 1];
+            act[e] = swiglu(__uint_as_float(e & 1 ? gw & 0xffff0000u : gw << 16), __uint_as_float(e & 1 ? uw & 0xffff0000u : uw << 16));
+            amax = __builtin_fmaxf(amax, __builtin_fabsf(act[e]));
+        }
+        uint32_t x = __float_as_uint(amax), y = x;
+        g8_swap16(x, y);
+        x = y = __float_as_uint(__builtin_fmaxf(__uint_as_float(x), __uint_as_float(y)));
+        g8_swap32(x, y);
+        amax = __builtin_fmaxf(__uint_as_float(x), __uint_as_float(y));
+        Part r;
+        r.s8 = f32_to_e4m3_pos(amax * (1.0f / 6.0f) * qg);
+        const float sv = e4m3_to_f32(r.s8);
+        const float mul = sv > 0.f ? qg / sv : 0.f;
+        r.q = f32x2_to_e2m1_byte<0>(0u, act[0] * mul, act[1] * mul);
+        r.q = f32x2_to_e2m1_byte<1>(r.q, act[2] * mul, act[3] * mul);
+        uint32_t t[4];
+        e2m1x8_to_f16(r.q, t);
+        const f16x2 sc = e4m3_to_f16x2(r.s8);
+        r.o0 = __builtin_bit_cast(uint32_t, (f16x2)(__builtin_bit_cast(f16x2, t[0]) * sc));
+        r.o1 = __builtin_bit_cast(uint32_t, (f16x2)(__builtin_bit_cast(f16x2, t[1]) * sc));
+        return r;
+    };
+#pragma unroll
+    for (int i = 0; i < T::TM; i++) {
+        if (16 * i >= rows) break;
+        const uint32_t row = row0 + 16 * i + fr;
+#pragma unroll
+        for (int j = 0; j < TN; j += STEP) {
+            Part x = block(acc[i][j], acc[i][j + 1], al[j], al[j + 1]);
+            const uint32_t blk = (colb >> 5) + j / 2;
+            if constexpr (STEP == 4) {
+                Part y = block(acc[i][j + 2], acc[i][j + 3], al[j + 2], al[j + 3]);
+                g8_swap16(x.o0, y.o0), g8_swap16(x.o1, y.o1), g8_swap16(x.q, y.q);
+                // lane groups 0, 2 store block blk's features 0..7, 8..15, groups 1, 3 the next block's
+                const uint32_t my = blk + (fc & 1), half = fc >> 1;
+                if (16 * i + fr < rows) {
+                    *(u32x4*)(q_aq + (size_t)row * inter + my * 16 + 8 * half) = (u32x4){x.o0, x.o1, y.o0, y.o1};
+                    *(uint32_t*)(q_codes + (size_t)row * (inter >> 1) + my * 8 + 4 * half) = (x.q & 0xffff) | (y.q << 16);
+                    if (fc < 2) q_sf[sf_tiled(row, my, kb)] = (uint8_t)(fc ? y.s8 : x.s8);
+                }
+            } else if (16 * i + fr < rows) {
+                *(u32x2*)(q_aq + (size_t)row * inter + blk * 16 + 4 * fc) = (u32x2){x.o0, x.o1};
+                *(uint16_t*)(q_codes + (size_t)row * (inter >> 1) + blk * 8 + 2 * fc) = (uint16_t)x.q;
+                if (fc == 0) q_sf[sf_tiled(row, blk, kb)] = (uint8_t)x.s8;
+            }
+        }
+    }
+}
+
 // ---- GEMM kernels ------------------------------------------------------------------------------------------------------------
 
 // Where the output of a GEMM goes: C (bf16, + residual) or, for a fused gate|up linear, the NVFP4-quantized SwiGLU.
@@ -445,13 +518,17 @@ struct FpOut {
     float qg;
 };
 
-// The wavefront's rows of a finished tile, from row0, colb (inside n) on: sums times alpha * scale. (The stream-K forms add a residual row piece by row piece, too: g8_add_bf16's
+// The wavefront's rows of a finished tile, from row0, colb (inside n) on: sums times alpha * scale. (The stream-K forms add a residual through the slab: g8_add_bf16's
 // registers, beside what their loop over segments keeps, would cost 30 spilled ones.)
 template <class T, bool SWIGLU, bool SK>
 __device__ __forceinline__ void fp_tile_store(f32x4 (&acc)[T::TM][T::TN], unsigned char* lds, const FpOut& o, const float* alpha, float scale, uint32_t m, uint32_t n,
                                               uint32_t row0, uint32_t colb) {
+    if constexpr (SWIGLU) {
+        if (row0 < m) fp4_tile_swiglu<T>(acc, alpha, scale, row0, m - row0, colb, n, o.q_codes, o.q_sf, o.q_aq, o.qg);
+        return;
+    }
     const uint32_t lane = threadIdx.x & 63, col = colb + 4 * (lane % (4 * T::TN));
-    if constexpr (!SWIGLU && !SK) {
+    if constexpr (!SK) {
         if (o.res) {
             if (row0 >= m) return;
             f32x4 al[T::TN];
@@ -475,18 +552,17 @@ __device__ __forceinline__ void fp_tile_store(f32x4 (&acc)[T::TM][T::TN], unsign
                 else
                     return G8Nothing{};
             },
-            [&](uint32_t r, uint32_t lc, float (&v)[4], auto old) {
+            [&](uint32_t r, uint32_t, float (&v)[4], auto old) {
                 const uint32_t row = row0 + r;
-                if constexpr (SWIGLU)
-                    swiglu_quant_store(v, al, lc, row < m, row < m ? row : 0, col, n, o.q_codes, o.q_sf, o.q_aq, o.qg);
-                else if constexpr (ADDS) {
-                    if (row < m) fp4_store4(o.c, true, old, (size_t)row * o.ldc + col, v, al);
-                } else if (row < m)
+                if (row >= m) return;
+                if constexpr (ADDS)
+                    fp4_store4(o.c, true, old, (size_t)row * o.ldc + col, v, al);
+                else
                     fp4_store4(o.c, false, (u32x2){0, 0}, (size_t)row * o.ldc + col, v, al);
             });
     };
-    if (SK && !SWIGLU && o.res)
-        rows(std::bool_constant<SK && !SWIGLU>{});
+    if (SK && o.res)
+        rows(std::bool_constant<SK>{});
     else
         rows(std::false_type{});
 }

@@ -1,4 +1,4 @@
-"""The GEMMs' epilogues with a residual: bf16(bf16(sum) + res) of the very sums that the call without one rounds, bit for bit, in every tile (whole ones, rows and columns that
+"""The epilogues of the prompt GEMMs. With a residual: bf16(bf16(sum) + res) of the very sums that the call without one rounds, bit for bit, in every tile (whole ones, rows and columns that
 end inside one), in place and from another buffer, with rows that lie further apart than they are wide; nothing is written past a row's columns or past the last row."""
 import numpy as np
 import pytest
@@ -58,3 +58,44 @@ def test_residual(form, m, n, k, gap):
         kern.set_option("gemm_pieces", 0)
         if form != "bf16":
             kern.set_option("gemm_sk", 1)
+
+
+@pytest.mark.parametrize("inter,k,m", [(128, 512, 70), (640, 256, 300), (384, 512, 256)])
+def test_nvfp4_swiglu_of_exact_sums(inter, k, m):
+    """The NVFP4 SwiGLU front on operands whose sums are exact in f32 in any order: the tiles' epilogue (registers, lane by lane) and the reduce launch of cut tiles (rows through
+    LDS) leave the same codes, scales and fp16 operand, the last seen through the linear that reads it."""
+    import torch
+    from ferrite_amd import fp4, synth
+    kern = fp4.Kernels.load()
+    rng = np.random.default_rng(11)
+    part = lambda n, kk: (rng.integers(0, 256, (n, kk // 2), dtype=np.uint8), np.full((n, kk // 16), 0x38, np.uint8))  # any codes, scales of 1
+    g, u, d = part(inter, k), part(inter, k), part(256, inter)
+    fused = fp4.HostLinear.fuse([("gate", *g, 2.0 ** -7, 1.0), ("up", *u, 2.0 ** -7, 1.0)])
+    sw = fused.into_swiglu().upload()
+    down = fp4.HostLinear.fuse([("down", *d, 2.0 ** -5, 1.0)]).upload()
+    x = rng.choice([0.0, 0.5, 1.0, 1.5, 2.0, 3.0, 4.0, 6.0], (m, k)) * rng.choice([-1.0, 1.0], (m, k))
+    x[:, ::16] = 6.0  # (every block's scale is 1)
+    x = torch.from_numpy(x).to(torch.bfloat16).cuda()
+    ws, act = fp4.Workspace(m, k), fp4.Workspace(m, inter)
+
+    def call(tile, pieces):
+        kern.set_option("gemm_tile", tile)
+        kern.set_option("gemm_pieces", pieces)
+        sw.forward_swiglu(kern, ws, act, x, k, m, 0.5)
+        kern.set_option("gemm_tile", 1)
+        y = torch.zeros((m, 256), dtype=torch.bfloat16, device="cuda")
+        down.gemm(kern, act, y, 256, m)
+        torch.cuda.synchronize()
+        return [a.copy() for a in act.read(m, inter)] + [y.view(torch.int16).cpu().numpy()]
+
+    try:
+        kern.set_option("gemm_splits", 1)
+        want = call(2, 2)  # cut: the reduce launch
+        assert np.unique(want[0]).size > 64 and np.unique(want[1]).size > 4
+        for tile, pieces in [(1, 1), (2, 1), (3, 1), (3, 2), (4, 1), (5, 1), (6, 1)]:
+            for a, b in zip(call(tile, pieces), want):
+                assert np.array_equal(a, b), (tile, pieces)
+    finally:
+        kern.set_option("gemm_splits", 8)
+        kern.set_option("gemm_tile", 0)
+        kern.set_option("gemm_pieces", 0)
