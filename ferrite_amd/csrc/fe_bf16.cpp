@@ -211,7 +211,7 @@ int fe_bf16_gemm(const fe_bf16_kernels *kern, fe_stream_t s, fe_devptr_t y, uint
         [&](uint32_t tile, uint32_t grid, uint32_t first, uint32_t splits) {
             fe_devptr_t part = kern->part.p;
             void *args[] = {&y, &part, &res, &m, &n, &ldy, &group, &first, &splits};
-            return fe_hip_launch(kern->reduce[tile], grid, 1, 1, kReduceThreads, 1, 1, 0, s, args);
+            return fe_hip_launch(kern->reduce[tile], grid, 1, 1, fe_reduce_threads(tile), 1, 1, 0, s, args);
         });
 }
 
@@ -248,7 +248,7 @@ int fe_bf16_gemm_swiglu(const fe_bf16_kernels *kern, fe_stream_t s, fe_devptr_t 
         [&](uint32_t tile, uint32_t grid, uint32_t first, uint32_t splits) {
             fe_devptr_t part = kern->part.p;
             void *args[] = {&act, &part, &m, &n, &group, &first, &splits};
-            return fe_hip_launch(kern->swiglu_reduce[tile], grid, 1, 1, kReduceThreads, 1, 1, 0, s, args);
+            return fe_hip_launch(kern->swiglu_reduce[tile], grid, 1, 1, fe_reduce_threads(tile), 1, 1, 0, s, args);
         });
 }
 

@@ -730,7 +730,7 @@ static int launch_gemm(const fe_exl3_linear *l, fe_stream_t s, fe_devptr_t xh, f
         },
         [&](uint32_t tile, uint32_t grid, uint32_t first, uint32_t splits) {
             void *args[] = {&part, &svh, &y, &n, &rows, &mode, &group, &first, &splits};
-            return fe_hip_launch(kern->gemm_reduce[tile], grid, 1, 1, kReduceThreads, 1, 1, 0, s, args);
+            return fe_hip_launch(kern->gemm_reduce[tile], grid, 1, 1, fe_reduce_threads(tile), 1, 1, 0, s, args);
         });
 }
 

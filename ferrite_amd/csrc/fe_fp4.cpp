@@ -549,7 +549,7 @@ static int linear_gemm(const fe_fp4_linear *l, const fe_fp4_kernels *kern, fe_st
             fe_devptr_t part = ws->part.p;
             float scale = l->fp8 ? 1.0f : 0.5f;  // 1 / what the fp16 operands carry (FP4_GEMM_SCALE)
             void *args[] = {&y, &part, &alpha, &res, &m, &n, &ldy, &group, &first, &splits, &scale};
-            return fe_hip_launch(codes8 ? kern->reduce8c[tile] : kern->reduce4[tile], grid, 1, 1, kReduceThreads, 1, 1, 0, s, args);
+            return fe_hip_launch(codes8 ? kern->reduce8c[tile] : kern->reduce4[tile], grid, 1, 1, fe_reduce_threads(tile), 1, 1, 0, s, args);
         });
 }
 
@@ -636,7 +636,7 @@ int fe_fp4_linear_forward_swiglu(const fe_fp4_linear *l, const fe_fp4_kernels *k
         },
         [&](uint32_t tile, uint32_t grid, uint32_t first, uint32_t splits) {
             void *args[] = {&part, &alpha, &m, &n, &group, &first, &splits, &q_codes, &q_sf, &q_aq, &down_g};
-            return fe_hip_launch(kern->swiglu_reduce4[tile], grid, 1, 1, kReduceThreads, 1, 1, 0, s, args);
+            return fe_hip_launch(kern->swiglu_reduce4[tile], grid, 1, 1, fe_reduce_threads(tile), 1, 1, 0, s, args);
         });
 }
 

@@ -512,12 +512,12 @@ inline float fe_rgemm_other_us(const FeGemmPlan &p, uint32_t cus) {
 }
 inline bool fe_rgemm_takes(const FeRgemmPlan &p, float other_us, uint32_t count) { return p.us <= other_us + 3.0f * (float)count; }
 
-constexpr uint32_t kReduceThreads = 512;  // of the reduce kernels (g8_reduce_rows of gemm8.h)
+constexpr uint32_t fe_reduce_threads(uint32_t tile) { return tile == 2 ? 256 : 512; }  // of the reduce kernels, half a wavefront a row (g8_reduce_rows of gemm8.h)
 // Launches a plan. gemm(form, programs, sched): form 0 = 256 x 256 one piece a program, 1 = stream-K, 2, 3 = tile 1, 2;
 // 4, 5, 6 = tile 3, 4, 5; reduce(tile, grid, first, splits): the reduce kernel of a tile, for the tiles from `first` on.
 template <class Gemm, class Reduce>
 int fe_gemm_launch(const FeGemmPlan &p, Gemm gemm, Reduce reduce) {
-    const uint32_t reduce_grid = kFeGemmTileM[p.tile] / 16 * (kFeGemmTileN[p.tile] / 128);  // workgroups a tile (of kReduceThreads)
+    const uint32_t reduce_grid = kFeGemmTileM[p.tile] / (fe_reduce_threads(p.tile) / 32) * (kFeGemmTileN[p.tile] / 128);  // workgroups a tile
     if (p.tile == 1 || p.tile == 2) {
         FeGemmSchedArgs a = p.big.args;
         a.full_tiles = 0, a.splits = p.splits, a.sk_base = a.sk_rem = 0;

@@ -367,12 +367,15 @@ __device__ __forceinline__ void g8_store_partial(f32x4 (&acc)[T::TM][T::TN], flo
 // lane, to fn(row, first column of the block, l32, v[4], ahead(row, first column, l32)); blocks outside n are left out, rows are not. `ahead` reads what fn
 // needs besides the sums.
 // What it costs is trips to memory, not bytes: so every load of a workgroup is asked for before the first is waited for (up to eight slots, and what `ahead` reads).
+// Tiles of 128 x 128: 8 rows and 256 threads a workgroup, a half wavefront reads its row's pieces, the first slot, then four, two, one. Their launches are small (64 tiles for 215
+// rows of 4096 columns), and more and smaller workgroups are ahead there (all slots at once are not: 5120 x 5120 at 300 rows 22.1 -> 23.5): us, GEMM and reduce, 16 -> 8 rows: FP8 4096 x 4096 at 130 / 215 rows 16.7 / 18.1 -> 14.9 / 15.7, 2048 x 8192 at 130 17.0 -> 14.2,
+// 1024 x 5120 at 512 15.4 -> 13.8, NVFP4 4096 x 4096 at 215 21.9 -> 19.7; bf16 level (1024 x 5120 at 512 17.4 -> 18.5).
 template <class T, class Ahead, class RowFn>
 __device__ __forceinline__ void g8_reduce_rows(const float* __restrict__ part, uint32_t m, uint32_t n, uint32_t group, uint32_t first,
                                                uint32_t splits, Ahead ahead, RowFn fn) {
-    constexpr uint32_t CB = T::BN / 128, PER_TILE = T::BM / 16 * CB, PITCH = 132;
-    __shared__ __attribute__((aligned(16))) float red[16 * PITCH];
-    const uint32_t t = blockIdx.x / PER_TILE, b = blockIdx.x % PER_TILE, rg = b / CB, cb = b % CB;
+    constexpr bool WHOLE = T::PARTS < 4;  // 1 KB of a slot a wavefront
+    constexpr uint32_t ROWS = WHOLE ? 16 : 8, CB = T::BN / 128, PER_TILE = T::BM / ROWS * CB, PITCH = 132;
+    const uint32_t t = blockIdx.x / PER_TILE, b = blockIdx.x % PER_TILE, cb = b % CB;
     const uint32_t lane = threadIdx.x & 63, wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6), l32 = threadIdx.x & 31, hw = threadIdx.x >> 5;
     uint32_t tm, tn;
     if constexpr (T::PARTS > 1) {
@@ -381,29 +384,52 @@ __device__ __forceinline__ void g8_reduce_rows(const float* __restrict__ part, u
     } else {
         gemm_raster(first + t, (m + T::BM - 1) / T::BM, (n + T::BN - 1) / T::BN, group, tm, tn);
     }
-    const uint32_t row0 = tm * T::BM + 16 * rg, n0 = tn * T::BN + cb * 128;
+    const uint32_t in = b / CB * ROWS, row0 = tm * T::BM + in, n0 = tn * T::BN + cb * 128;  // in: the workgroup's first row of the tile
     if (row0 >= m || n0 >= n) return;
-    const uint32_t c16 = 8 * cb + wave, piece = (rg % T::TM * T::TN + c16 % T::TN) * T::THREADS + (rg / T::TM * T::WN + c16 / T::TN) * 64 + lane;
-    const float* p = part + (size_t)t * splits * T::PART_FLOATS + piece * 4;
-    auto slot = [&](uint32_t sp) { return *(const f32x4*)(p + (size_t)(sp < splits ? sp : splits - 1) * T::PART_FLOATS); };  // (past the last: that one again, not added)
-    f32x4 q[8];
+    if constexpr (WHOLE) {
+        __shared__ __attribute__((aligned(16))) float red[16 * PITCH];
+        const uint32_t rg = in / 16, c16 = 8 * cb + wave, piece = (rg % T::TM * T::TN + c16 % T::TN) * T::THREADS + (rg / T::TM * T::WN + c16 / T::TN) * 64 + lane;
+        const float* p = part + (size_t)t * splits * T::PART_FLOATS + piece * 4;
+        auto slot = [&](uint32_t sp) { return *(const f32x4*)(p + (size_t)(sp < splits ? sp : splits - 1) * T::PART_FLOATS); };  // (past the last: that one again, not added)
+        f32x4 q[8];
 #pragma unroll
-    for (uint32_t i = 0; i < 4; i++) q[i] = slot(i);
-    if (splits > 4) {
+        for (uint32_t i = 0; i < 4; i++) q[i] = slot(i);
+        if (splits > 4) {
 #pragma unroll
-        for (uint32_t i = 4; i < 8; i++) q[i] = slot(i);
+            for (uint32_t i = 4; i < 8; i++) q[i] = slot(i);
+        }
+        const auto st = ahead(row0 + hw, n0, l32);
+        f32x4 sum = q[0];
+#pragma unroll
+        for (uint32_t i = 1; i < 8; i++)
+            if (i < splits) sum += q[i];
+        for (uint32_t sp = 8; sp < splits; sp++) sum += slot(sp);
+        *(f32x4*)(red + (lane & 15) * PITCH + 16 * wave + 4 * (lane >> 4)) = sum;
+        __syncthreads();
+        const f32x4 r = *(const f32x4*)(red + hw * PITCH + 4 * l32);
+        float v[4] = {r[0], r[1], r[2], r[3]};
+        fn(row0 + hw, n0, l32, v, st);
+    } else {
+        const uint32_t row = in + hw, c4 = cb * 32 + l32, wn = c4 / (4 * T::TN), j = (c4 / 4) % T::TN, fc = c4 % 4;
+        const uint32_t wm = row / (16 * T::TM), i = (row / 16) % T::TM, fr = row % 16;
+        const float* p = part + (size_t)t * splits * T::PART_FLOATS + ((i * T::TN + j) * T::THREADS + (wm * T::WN + wn) * 64 + fc * 16 + fr) * 4;
+        const auto st = ahead(row0 + hw, n0, l32);
+        f32x4 sum = *(const f32x4*)p;
+        auto add = [&](auto n_tag, uint32_t sp) {  // so many pieces in flight a lane
+            constexpr uint32_t N = decltype(n_tag)::value;
+            f32x4 piece[N];
+#pragma unroll
+            for (uint32_t q = 0; q < N; q++) piece[q] = *(const f32x4*)(p + (size_t)(sp + q) * T::PART_FLOATS);
+#pragma unroll
+            for (uint32_t q = 0; q < N; q++) sum += piece[q];
+        };
+        uint32_t sp = 1;
+        for (; sp + 4 <= splits; sp += 4) add(std::integral_constant<uint32_t, 4>{}, sp);
+        if (sp + 2 <= splits) add(std::integral_constant<uint32_t, 2>{}, sp), sp += 2;
+        if (sp < splits) add(std::integral_constant<uint32_t, 1>{}, sp);
+        float v[4] = {sum[0], sum[1], sum[2], sum[3]};
+        fn(row0 + hw, n0, l32, v, st);
     }
-    const auto st = ahead(row0 + hw, n0, l32);
-    f32x4 sum = q[0];
-#pragma unroll
-    for (uint32_t i = 1; i < 8; i++)
-        if (i < splits) sum += q[i];
-    for (uint32_t sp = 8; sp < splits; sp++) sum += slot(sp);
-    *(f32x4*)(red + (lane & 15) * PITCH + 16 * wave + 4 * (lane >> 4)) = sum;
-    __syncthreads();
-    const f32x4 r = *(const f32x4*)(red + hw * PITCH + 4 * l32);
-    float v[4] = {r[0], r[1], r[2], r[3]};
-    fn(row0 + hw, n0, l32, v, st);
 }
 
 // The same loop for a weight operand that is packed in memory and expanded to 16-bit values as it becomes a fragment: the

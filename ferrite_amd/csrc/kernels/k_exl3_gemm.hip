@@ -233,7 +233,7 @@ __device__ __forceinline__ void exl3_gemm_hat_kernel(HAT_GEMM_PARAMS) {
                           });
 }
 // Finishes the tiles that a GEMM kernel cut along K: sums their partial slots and applies the output rotation and scale.
-// grid: cut tiles * (BM / 16) * (BN / 128), 512 threads.
+// Grid and threads: g8_reduce_rows.
 template <class T>
 __device__ __forceinline__ void exl3_reduce_body(const float* part, const uint16_t* svh, void* y, uint32_t n, uint32_t m, uint32_t y_mode,
                                                  uint32_t group_m, uint32_t first, uint32_t splits) {

@@ -607,7 +607,7 @@ __device__ __forceinline__ void fp_gemm_body(MakePacked make_packed, const FpOut
         });
 }
 
-// Finishes the tiles that a GEMM kernel cut along K. grid: cut tiles * (BM / 16) * (BN / 128), 512 threads.
+// Finishes the tiles that a GEMM kernel cut along K. Grid and threads: g8_reduce_rows.
 template <class T, bool SWIGLU>
 __device__ __forceinline__ void fp_reduce_body(const FpOut& out, const float* part, const float* alpha, float scale,
                                                uint32_t m, uint32_t n, uint32_t group_m, uint32_t first, uint32_t splits) {
