@@ -294,13 +294,14 @@ struct FeGemmTileOptions {
 // tiles in more than one round take more than their rounds add up to (trellis: the programs that come second decode alone; 528 tiles 128 x 128 of
 // 32 k tiles 80 us where the rounds add up to 67).
 // high: us a k tile of tiles of 256, 224, 192, 160 rows, and how much more of it when all CUs are busy, for the choice among them (fe_gemm_height): fitted to 112
-// timings a form and height (128..1900 rows, 2048 x 4096 .. 17408 x 5120) without a fixed part, half of them within 5 % (FP8 8 %).
+// timings a form and height (128..1900 rows, 2048 x 4096 .. 17408 x 5120) without a fixed part, half of them within 5 % (FP8: to 60, half within 5 %, nine tenths within 11..15 %; 220 launches, 13
+// linears: 0.969 of the time with the tiles picked by the loop and the figures before, 2048 x 8192 at 1536 rows 34.9 -> 36.5, 34816 x 5120 at 130 71.7 -> 73.5, no other twice more than 3 % slower).
 struct FeGemmCost {
     float ktile[3], full[3], fixed[3], shared, stream_k, again, high[4][2];
 };
 constexpr FeGemmCost kFeCostTrellis = {{1.38f, 1.02f, 0.71f}, {0.12f, 0.07f, 0.08f}, {1.0f, 3.0f, 1.9f}, 1.63f, 48.7f, 1.12f, {}};
 constexpr FeGemmCost kFeCostNvfp4 = {{1.32f, 0.73f, 0.44f}, {-0.07f, 0.05f, 0.09f}, {0.0f, 2.2f, 2.3f}, 1.59f, 44.0f, 1.0f, {{1.11f, 0.29f}, {1.16f, 0.16f}, {0.90f, 0.36f}, {0.57f, 1.03f}}};
-constexpr FeGemmCost kFeCostFp8 = {{1.20f, 0.58f, 0.66f}, {0.09f, 0.46f, 0.21f}, {0.0f, 2.5f, 0.4f}, 1.21f, 36.4f, 1.0f, {{1.81f, -0.29f}, {1.78f, -0.21f}, {1.68f, -0.20f}, {1.50f, -0.15f}}};
+constexpr FeGemmCost kFeCostFp8 = {{1.20f, 0.58f, 0.66f}, {0.09f, 0.46f, 0.21f}, {0.0f, 2.5f, 0.4f}, 1.21f, 36.4f, 1.0f, {{1.04f, 0.13f}, {1.07f, 0.03f}, {0.93f, 0.10f}, {0.88f, 0.05f}}};
 constexpr FeGemmCost kFeCostBf16 = {{1.10f, 0.64f, 0.45f}, {0.22f, 0.43f, 0.41f}, {0.0f, 1.5f, 0.3f}, 1.53f, 53.2f, 1.0f, {{1.26f, 0.04f}, {1.24f, 0.01f}, {0.92f, 0.20f}, {0.77f, 0.34f}}};
 
 // `programs` programs of `ktiles` k tiles each, in rounds of all CUs (tile 2: two a CU).

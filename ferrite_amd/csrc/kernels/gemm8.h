@@ -680,14 +680,16 @@ __device__ __forceinline__ void g8_mainloop_decode(const _Float16* a, uint32_t l
 // The loop for 8-bit operands (e4m3 codes on both sides) on v_mfma_f32_16x16x128_f8f6f4: a k tile is 128 codes, so rows are again
 // 128 bytes and stages, chunk positions and loads are those of g8_mainloop; a lane's operand of the one MFMA step of a k
 // tile is chunks fc and 4 + fc of its row (both operands alike: k is a summation index only). A fragment takes 8 registers,
-// so the weight fragments pass through a ring of four, each refilled four columns ahead, and the A fragments are refilled in
-// place behind the last column. The barrier comes after the fifth column, the first that makes room for the next tile's.
+// so the weight fragments pass through a ring of half the columns, each refilled as many ahead, and the A fragments are refilled in
+// place behind the last column. The barrier comes after the first column of the second half, the first that makes room for the next tile's. (The lower tiles' four columns with a
+// ring of four, the barrier behind the first and the weights' loads in a lump in front of it: a k tile of 160 rows took as long as one of 256. Ring of four -> of two, us: 380 rows of 17408 x
+// 5120 in tiles of 160 rows 46.5 -> 40.0, 777 in tiles of 224 77.9 -> 71.5, 600 of 5120 x 17408 in tiles of 160 62.0 -> 56.0. 128 x 128, two programs a CU: level, kept at four.)
 // a: codes [m][lda] (bytes).
 typedef int g8_i32x8 __attribute__((ext_vector_type(8)));
 template <class T, int NA, int NW, bool ZERO>
 __device__ __forceinline__ void g8_mainloop_f8(const uint8_t* a, uint32_t lda, uint32_t m, uint32_t kt0, uint32_t ktiles, uint32_t m0,
                                                const G8Dense<T>& wo, unsigned char* lds, f32x4 (&acc)[T::TM][T::TN]) {
-    constexpr int TM = T::TM, TN = T::TN, R = 4, LA = T::LA, LB = G8Dense<T>::LOADS, A_STAGE = T::A_STAGE, W_AT = NA * A_STAGE;
+    constexpr int TM = T::TM, TN = T::TN, R = T::PARTS == 1 ? TN / 2 : 4, LA = T::LA, LB = G8Dense<T>::LOADS, A_STAGE = T::A_STAGE, W_AT = NA * A_STAGE;
     constexpr int W_STAGE = G8Dense<T>::STAGE, BAR = TN - R;  // the barrier follows column BAR
     static_assert(TN == 2 * R || TN == R, "a ring of half or of all the columns");
     static_assert(NA >= 2 && NW >= 2 && g8_flight0(LA, NA, LB, NW) < 64, "loads in flight");
