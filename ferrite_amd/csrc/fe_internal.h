@@ -293,16 +293,17 @@ struct FeGemmTileOptions {
 // 10..13 % for bf16 and FP8, whose panels compete for memory). stream_k: what meeting through the workspace adds. again: what small
 // tiles in more than one round take more than their rounds add up to (trellis: the programs that come second decode alone; 528 tiles 128 x 128 of
 // 32 k tiles 80 us where the rounds add up to 67).
+// short_k: how much of the small tiles' estimate a lower tile may take with more tiles than CUs and fewer than 24 k tiles (fe_gemm_plan).
 // high: us a k tile of tiles of 256, 224, 192, 160 rows, and how much more of it when all CUs are busy, for the choice among them (fe_gemm_height): fitted to 112
 // timings a form and height (128..1900 rows, 2048 x 4096 .. 17408 x 5120) without a fixed part, half of them within 5 % (FP8: to 60, half within 5 %, nine tenths within 11..15 %; 220 launches, 13
-// linears: 0.969 of the time with the tiles picked by the loop and the figures before, 2048 x 8192 at 1536 rows 34.9 -> 36.5, 34816 x 5120 at 130 71.7 -> 73.5, no other twice more than 3 % slower).
+// linears: 0.965 of the time with the tiles picked by the loop and the figures before; 5120 x 17408 at 1100 rows 91.4 -> 96.5, 2048 x 8192 at 1536 35.0 -> 36.6, no other more than 3.2 % slower).
 struct FeGemmCost {
-    float ktile[3], full[3], fixed[3], shared, stream_k, again, high[4][2];
+    float ktile[3], full[3], fixed[3], shared, stream_k, again, high[4][2], short_k;
 };
-constexpr FeGemmCost kFeCostTrellis = {{1.38f, 1.02f, 0.71f}, {0.12f, 0.07f, 0.08f}, {1.0f, 3.0f, 1.9f}, 1.63f, 48.7f, 1.12f, {}};
-constexpr FeGemmCost kFeCostNvfp4 = {{1.32f, 0.73f, 0.44f}, {-0.07f, 0.05f, 0.09f}, {0.0f, 2.2f, 2.3f}, 1.59f, 44.0f, 1.0f, {{1.11f, 0.29f}, {1.16f, 0.16f}, {0.90f, 0.36f}, {0.57f, 1.03f}}};
-constexpr FeGemmCost kFeCostFp8 = {{1.20f, 0.58f, 0.66f}, {0.09f, 0.46f, 0.21f}, {0.0f, 2.5f, 0.4f}, 1.21f, 36.4f, 1.0f, {{1.04f, 0.13f}, {1.07f, 0.03f}, {0.93f, 0.10f}, {0.88f, 0.05f}}};
-constexpr FeGemmCost kFeCostBf16 = {{1.10f, 0.64f, 0.45f}, {0.22f, 0.43f, 0.41f}, {0.0f, 1.5f, 0.3f}, 1.53f, 53.2f, 1.0f, {{1.26f, 0.04f}, {1.24f, 0.01f}, {0.92f, 0.20f}, {0.77f, 0.34f}}};
+constexpr FeGemmCost kFeCostTrellis = {{1.38f, 1.02f, 0.71f}, {0.12f, 0.07f, 0.08f}, {1.0f, 3.0f, 1.9f}, 1.63f, 48.7f, 1.12f, {}, 0.0f};
+constexpr FeGemmCost kFeCostNvfp4 = {{1.32f, 0.73f, 0.44f}, {-0.07f, 0.05f, 0.09f}, {0.0f, 2.2f, 2.3f}, 1.59f, 44.0f, 1.0f, {{1.11f, 0.29f}, {1.16f, 0.16f}, {0.90f, 0.36f}, {0.57f, 1.03f}}, 0.97f};
+constexpr FeGemmCost kFeCostFp8 = {{1.20f, 0.58f, 0.66f}, {0.09f, 0.46f, 0.21f}, {0.0f, 2.5f, 0.4f}, 1.21f, 36.4f, 1.0f, {{1.04f, 0.13f}, {1.07f, 0.03f}, {0.93f, 0.10f}, {0.88f, 0.05f}}, 0.77f};
+constexpr FeGemmCost kFeCostBf16 = {{1.10f, 0.64f, 0.45f}, {0.22f, 0.43f, 0.41f}, {0.0f, 1.5f, 0.3f}, 1.53f, 53.2f, 1.0f, {{1.26f, 0.04f}, {1.24f, 0.01f}, {0.92f, 0.20f}, {0.77f, 0.34f}}, 0.9f};
 
 // `programs` programs of `ktiles` k tiles each, in rounds of all CUs (tile 2: two a CU).
 inline float fe_gemm_cost(const FeGemmCost &c, uint32_t tile, uint32_t programs, uint32_t ktiles, uint32_t cus) {
@@ -428,9 +429,10 @@ inline FeGemmPlan fe_gemm_plan(uint32_t m, uint32_t n, uint32_t ktiles, uint32_t
         // Dense weights (bf16, FP8) in fewer lower tiles than a quarter of the CUs: deep narrow linears, which small tiles cut finer than eight pieces of a lower one (bf16:
         // 826 launches 1.16 times the small tiles' time, from there on 0.90). More lower tiles than CUs and short K: rounds of them want a clearer gain (48 of FP8 1.01, bf16 past 0.9 level;
         // not so from 24 k tiles on: 5120 x 17408 at 559 rows, NVFP4 block 290 us with them, 305 without).
+        // (FP8 0.77: its lower tiles' estimate leaves out what short K costs; 33536 x 2048 at 711 rows, 65.2 in small tiles, would be 0.80, 7168 x 2560 at 1253, 38.2 against 32.3, is 0.58.)
         const uint32_t tiles = tiles_of(pick);
         if (!small_b && 4 * tiles < cus) return p;
-        const float margin = tiles > cus && ktiles < 24 ? (small_b ? 0.97f : 0.9f) : small_b ? 1.06f : 1.0f;  // (bf16 and FP8: what a lower tile gained is part of that margin)
+        const float margin = tiles > cus && ktiles < 24 ? cost.short_k : small_b ? 1.06f : 1.0f;  // (bf16 and FP8: what a lower tile gained is part of that margin)
         if (margin * p.us < whole * ratio) return p;
     }
     p.tile = pick, p.tiles = 0, p.splits = 1, p.big = lower, p.us = whole * ratio;
