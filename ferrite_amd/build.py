@@ -22,7 +22,7 @@ DEVICE_FLAGS = ["--offload-arch=gfx950", "-O3", "-std=c++17", "-mcode-object-ver
                 "-Xclang", "-target-feature", "-Xclang", "-packed-fp32-ops"]
 # code objects: name, source, defines; the ones that take longest first
 # ALIGNED: loops that start a line of the instruction cache. Where a tile loop of 1.4 KB happens to start moves a GEMM by 2 % (NVFP4, 512 rows of 17408 x 5120: 85.5 us at the start of a
-# line, 87.4 twelve bytes into one). Not the decode kernels: each is a few hundred instructions long-lived and the padding costs more (1024 / 2816 at 1 row 26.0 -> 26.35 us).
+# line, 87.4 twelve bytes into one). Not the decode kernels, whose groups of load steps are straight code of 8 KB: there the padding costs more (1024 / 2816 at 1 row 26.0 -> 26.35 us).
 ALIGNED = ["-falign-loops=128"]
 KERNELS = [("k_exl3_gemm", "k_exl3_gemm.hip", ALIGNED)]
 KERNELS += [(f"k_exl3_rgemm_b{b}", "k_exl3_rgemm.hip", ALIGNED + [f"-DRG_BITS={b}"]) for b in (8, 6, 5, 4, 3, 2)]
