@@ -299,10 +299,11 @@ struct FeGemmTileOptions {
 // linears: 0.965 of the time with the tiles picked by the loop and the figures before; 5120 x 17408 at 1100 rows 91.4 -> 96.5, 2048 x 8192 at 1536 35.0 -> 36.6, no other more than 3.2 % slower).
 struct FeGemmCost {
     float ktile[3], full[3], fixed[3], shared, stream_k, again, high[4][2], short_k;
+    bool f8 = false;
 };
 constexpr FeGemmCost kFeCostTrellis = {{1.38f, 1.02f, 0.71f}, {0.12f, 0.07f, 0.08f}, {1.0f, 3.0f, 1.9f}, 1.63f, 48.7f, 1.12f, {}, 0.0f};
 constexpr FeGemmCost kFeCostNvfp4 = {{1.32f, 0.73f, 0.44f}, {-0.07f, 0.05f, 0.09f}, {0.0f, 2.2f, 2.3f}, 1.59f, 44.0f, 1.0f, {{1.11f, 0.29f}, {1.16f, 0.16f}, {0.90f, 0.36f}, {0.57f, 1.03f}}, 0.97f};
-constexpr FeGemmCost kFeCostFp8 = {{1.20f, 0.58f, 0.66f}, {0.09f, 0.46f, 0.21f}, {0.0f, 2.5f, 0.4f}, 1.21f, 36.4f, 1.0f, {{1.04f, 0.13f}, {1.07f, 0.03f}, {0.93f, 0.10f}, {0.88f, 0.05f}}, 0.77f};
+constexpr FeGemmCost kFeCostFp8 = {{1.20f, 0.58f, 0.66f}, {0.09f, 0.46f, 0.21f}, {0.0f, 2.5f, 0.4f}, 1.21f, 36.4f, 1.0f, {{1.04f, 0.13f}, {1.07f, 0.03f}, {0.93f, 0.10f}, {0.88f, 0.05f}}, 0.77f, true};
 constexpr FeGemmCost kFeCostBf16 = {{1.10f, 0.64f, 0.45f}, {0.22f, 0.43f, 0.41f}, {0.0f, 1.5f, 0.3f}, 1.53f, 53.2f, 1.0f, {{1.26f, 0.04f}, {1.24f, 0.01f}, {0.92f, 0.20f}, {0.77f, 0.34f}}, 0.9f};
 
 // `programs` programs of `ktiles` k tiles each, in rounds of all CUs (tile 2: two a CU).
@@ -429,10 +430,14 @@ inline FeGemmPlan fe_gemm_plan(uint32_t m, uint32_t n, uint32_t ktiles, uint32_t
         // Dense weights (bf16, FP8) in fewer lower tiles than a quarter of the CUs: deep narrow linears, which small tiles cut finer than eight pieces of a lower one (bf16:
         // 826 launches 1.16 times the small tiles' time, from there on 0.90). More lower tiles than CUs and short K: rounds of them want a clearer gain (48 of FP8 1.01, bf16 past 0.9 level;
         // not so from 24 k tiles on: 5120 x 17408 at 559 rows, NVFP4 block 290 us with them, 305 without).
-        // (FP8 0.77: its lower tiles' estimate leaves out what short K costs; 33536 x 2048 at 711 rows, 65.2 in small tiles, would be 0.80, 7168 x 2560 at 1253, 38.2 against 32.3, is 0.58.)
         const uint32_t tiles = tiles_of(pick);
         if (!small_b && 4 * tiles < cus) return p;
-        const float margin = tiles > cus && ktiles < 24 ? cost.short_k : small_b ? 1.06f : 1.0f;  // (bf16 and FP8: what a lower tile gained is part of that margin)
+        // FP8, whose heights leave out what a cut and short K cost: not where every lower tile is cut (29 launches of 7 linears 0.97 to 1.14 of the small tiles' time, two of them ahead by more
+        // than 1 %, none by more than 3: 5120 x 17408 at 1100 / 1216 rows 88.6 -> 91.7, 92.7 -> 103.6, 5120 x 6144 at 512 25.0 -> 28.5, 2048 x 8192 at 1536 32.9 -> 35.4); a few cut tiles behind a
+        // whole round are ahead (34816 x 5120 at 250 82.8 -> 66.5). And the clearer gain for short K at any count: with fewer tiles than CUs 8192 x 2048 at 1024 rows takes 19.7 -> 20.7
+        // where the ratio is 0.99, at 1100 rows 23.7 -> 20.9 where it is 0.46 (ten launches between 0.46 and 0.77: 0.71 to 0.96 of the time).
+        if (cost.f8 && !lower.split.full && m > kFeGemmTileM[pick]) return p;
+        const float margin = ktiles < 24 && (tiles > cus || cost.f8) ? cost.short_k : small_b ? 1.06f : 1.0f;  // (bf16 and FP8: what a lower tile gained is part of that margin)
         if (margin * p.us < whole * ratio) return p;
     }
     p.tile = pick, p.tiles = 0, p.splits = 1, p.big = lower, p.us = whole * ratio;

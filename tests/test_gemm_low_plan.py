@@ -43,6 +43,20 @@ TIMED = {
     ("nvfp4", 160, 34816, 5120): (5, 0),   # 76, 256 rows 93
     ("nvfp4", 320, 34816, 5120): (5, 0),   # 102, 256 rows 126
     ("nvfp4", 1024, 34816, 5120): (0, 0),  # 267, stream-K 277
+    # FP8: where every lower tile would be cut, and with short K and a ratio near 1, the small tiles
+    ("fp8", 1100, 5120, 17408): (1, 0),   # 88.6, 192 rows cut in two 91.7
+    ("fp8", 1216, 5120, 17408): (1, 0),   # 92.7, 224 rows cut in two 103.6
+    ("fp8", 1216, 2048, 8192): (1, 0),    # 28.8, 160 rows cut in four 30.5
+    ("fp8", 1536, 2048, 8192): (1, 0),    # 32.9, 160 rows cut in three 35.4
+    ("fp8", 512, 5120, 6144): (1, 0),     # 25.0, 160 rows cut in three 28.5
+    ("fp8", 1024, 3072, 9216): (1, 0),    # 35.0, 160 rows cut in three 38.0
+    ("fp8", 1024, 8192, 2048): (2, 0),    # 19.7, 160 rows whole 20.7
+    # and the lower tiles where they are ahead
+    ("fp8", 420, 17408, 5120): (5, 0),    # 38.6, 128 rows 46.7
+    ("fp8", 250, 34816, 5120): (5, 0),    # a round and 16 tiles cut in seven 66.5, 128 rows 82.8
+    ("fp8", 1100, 8192, 2048): (5, 0),    # 21.0, 128 x 128 23.7
+    ("fp8", 1300, 17408, 5120): (4, 0),   # 93.4, 128 rows 103.3
+    ("fp8", 777, 5120, 17408): (3, 0),    # each cut in three 74.2, 256 rows so 76.4
 }
 
 
