@@ -93,18 +93,19 @@ def main(argv):
                 print(json.dumps(mfma_peak(fk, kind, cus, seed=seed, timed_s=1.0)), flush=True)
     elif what == "valu":
         kern = exl3.Kernels.load()
-        grid, iters = 4 * cus, 4096
-        base = None
-        for op in exl3.Kernels.PROBE_OPS:
-            kern.probe_op(op, grid, iters, 20)
-            with Smi() as s:
-                ms = kern.probe_op(op, grid, iters, 200)
-            ops = grid * 256 * 8 * iters / (ms * 1e-3)
-            base = base or ops
-            clk = s.summary()["sclk_MHz_median"]
-            print(json.dumps({"probe": f"valu_{op}", "Tlane_ops_per_s": round(ops / 1e12, 2), "relative_to_add": round(ops / base, 3),
-                              "cycles_per_wave_instruction_per_simd": round(4 * cus * 64 * clk * 1e6 / ops, 2) if clk else None,
-                              "sclk_MHz_median": clk}), flush=True)
+        for waves in (2, 4, 8):  # a SIMD; the decode GEMV: 4
+            grid, iters, base = waves * cus, 4096, None
+            for op in exl3.Kernels.PROBE_OPS:
+                kern.probe_op(op, grid, iters, 20)
+                with Smi() as s:
+                    ms = kern.probe_op(op, grid, iters, 200)
+                ops = grid * 256 * 8 * iters / (ms * 1e-3)
+                base = base or ops
+                clk = s.summary()["sclk_MHz_median"]
+                print(json.dumps({"probe": f"valu_{op}", "wavefronts_per_simd": waves, "us": round(ms * 1e3, 1),
+                                  "Tlane_ops_per_s": round(ops / 1e12, 2), "relative_to_add": round(ops / base, 3),
+                                  "cycles_per_wave_instruction_per_simd": round(4 * cus * 64 * clk * 1e6 / ops, 2) if clk else None,
+                                  "sclk_MHz_median": clk}), flush=True)
     elif what == "decode":
         kern = exl3.Kernels.load()
         grid, iters = 4 * cus, 256
