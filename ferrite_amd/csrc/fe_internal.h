@@ -295,8 +295,9 @@ struct FeGemmTileOptions {
 // 32 k tiles 80 us where the rounds add up to 67).
 // short_k: how much of the small tiles' estimate a lower tile may take with more tiles than CUs and fewer than 24 k tiles (fe_gemm_plan).
 // high: us a k tile of tiles of 256, 224, 192, 160 rows, and how much more of it when all CUs are busy, for the choice among them (fe_gemm_height): fitted to 112
-// timings a form and height (128..1900 rows, 2048 x 4096 .. 17408 x 5120) without a fixed part, half of them within 5 % (FP8: to 60, half within 5 %, nine tenths within 11..15 %; 220 launches, 13
-// linears: 0.965 of the time with the tiles picked by the loop and the figures before; 5120 x 17408 at 1100 rows 91.4 -> 96.5, 2048 x 8192 at 1536 35.0 -> 36.6, no other more than 3.2 % slower).
+// timings a form and height (128..1900 rows, 2048 x 4096 .. 17408 x 5120) without a fixed part, half of them within 5 % (FP8: to 60, half within 5 %, nine tenths within 11..15 %; 962 launches against the tree before its lower tiles'
+// loop of today, 647 of them with another tile: those 0.910 of the time, one more than 3 % slower, 1792 x 19072 at 1263 rows 69.0 -> 73.3; the others 0.985, 8704 x 5120 at 129 rows 20.5 -> 21.1).
+// f8: FP8 weights, for two lines of fe_gemm_plan.
 struct FeGemmCost {
     float ktile[3], full[3], fixed[3], shared, stream_k, again, high[4][2], short_k;
     bool f8 = false;
@@ -387,7 +388,8 @@ inline FeGemmPlan fe_gemm_plan(uint32_t m, uint32_t n, uint32_t ktiles, uint32_t
     // Lower tiles: as many row tiles of less waste, or another count of them that fills the rounds of the CUs better (rows that do not exist cost little power, but
     // their time). By the ratio of the two estimates, which share most of their errors. Of 336 launches (8 layers, 14 row counts, NVFP4, FP8 and bf16) against 256 rows:
     // 0.925, 0.93, 0.905 of the time (the best height each time: 0.92, 0.92, 0.90), four more than 2 % slower, at most 7 %. With the small tiles in the choice, 12 other layers
-    // of 144 launches a form against the rule without lower tiles: 0.93, 0.97, 0.93; 8 of 432 more than 3 % slower, at most 7 %.
+    // of 144 launches a form against the rule without lower tiles: 0.93, 0.97, 0.93; 8 of 432 more than 3 % slower, at most 7 %. (With FP8's loop and heights, the reduce launches and the
+    // epilogues of before; FP8's figures since are at FeGemmCost.)
     uint32_t pick = 0;
     float ratio = p.big.stream_k ? 0.9f : 0.97f;
     if (opt.low && m <= 2048) {
@@ -421,7 +423,7 @@ inline FeGemmPlan fe_gemm_plan(uint32_t m, uint32_t n, uint32_t ktiles, uint32_t
     // deep narrow and wide shallow ones among them, 807 were more than 3 % slower (bf16 1792 x 16384 at 864 rows 56.8 -> 89.7, 768 x 15104 at 1303
     // 41.9 -> 52.6; at most 1.8 times); with the lines below 139 (41 of them bf16 in the
     // place of 256 rows, at most 1.5 times: 35 and 49 tiles cut seven and five ways), 0.957 / 0.959 / 0.986 / 0.960 / 0.964 of the time (bf16, its SwiGLU front, FP8, NVFP4, its front; the best each time 0.949
-    // / 0.950 / 0.982 / 0.953 / 0.952).
+    // / 0.950 / 0.982 / 0.953 / 0.952). All of these with FP8's loop and heights, the reduce launches and the epilogues of before, and FP8 with a margin of 0.9 for short K.
     const FeGemmSchedule lower = low(pick);
     if (p.tile) {
         // (Of an NVFP4 SwiGLU front with 16..23 k tiles, which small tiles may cut in two only, lower ones also with fewer programs: 45 launches of up to 16 tiles 0.82 of the small tiles' time;
@@ -432,10 +434,10 @@ inline FeGemmPlan fe_gemm_plan(uint32_t m, uint32_t n, uint32_t ktiles, uint32_t
         // not so from 24 k tiles on: 5120 x 17408 at 559 rows, NVFP4 block 290 us with them, 305 without).
         const uint32_t tiles = tiles_of(pick);
         if (!small_b && 4 * tiles < cus) return p;
-        // FP8, whose heights leave out what a cut and short K cost: not where every lower tile is cut (29 launches of 7 linears 0.97 to 1.14 of the small tiles' time, two of them ahead by more
-        // than 1 %, none by more than 3: 5120 x 17408 at 1100 / 1216 rows 88.6 -> 91.7, 92.7 -> 103.6, 5120 x 6144 at 512 25.0 -> 28.5, 2048 x 8192 at 1536 32.9 -> 35.4); a few cut tiles behind a
-        // whole round are ahead (34816 x 5120 at 250 82.8 -> 66.5). And the clearer gain for short K at any count: with fewer tiles than CUs 8192 x 2048 at 1024 rows takes 19.7 -> 20.7
-        // where the ratio is 0.99, at 1100 rows 23.7 -> 20.9 where it is 0.46 (ten launches between 0.46 and 0.77: 0.71 to 0.96 of the time).
+        // FP8, whose heights leave out what a cut and short K cost: not where every lower tile is cut, unless one is as high as the rows (small tiles, us -> lower ones: 5120 x 17408 at
+        // 1100 / 1216 rows 88.6 -> 91.7, 92.7 -> 103.6, 5120 x 6144 at 512 25.0 -> 28.5, 2048 x 8192 at 1536 32.9 -> 35.4; 70 launches 0.95 to 1.14 of the small tiles' time; one row tile:
+        // 18944 x 8448 at 155 53.5 -> 45.9). A few cut tiles behind a whole round are ahead (34816 x 5120 at 250 82.8 -> 66.5). And the clearer gain for short K at any count: with fewer
+        // tiles than CUs 8192 x 2048 at 1024 rows takes 19.7 -> 20.7 where the ratio is 0.99, at 1100 rows 23.7 -> 20.9 where it is 0.46 (ten launches between 0.46 and 0.77: 0.71 to 0.96).
         if (cost.f8 && !lower.split.full && m > kFeGemmTileM[pick]) return p;
         const float margin = ktiles < 24 && (tiles > cus || cost.f8) ? cost.short_k : small_b ? 1.06f : 1.0f;  // (bf16 and FP8: what a lower tile gained is part of that margin)
         if (margin * p.us < whole * ratio) return p;

@@ -415,7 +415,7 @@ __device__ __forceinline__ void gemvb_body(const GemvMember mb, uint32_t p0, uin
     // hw + 8, ... of every row. The first pair's loads go out ahead of the trellis loads (loads return in order), so
     // that the rotation runs while the first trellis words are still on their way.
     // (CHAIN: always, and up to 8 rows only, mlp_chain_fits. Code for what never comes is not free: with it the kernel is 47 KB, which with the 23 KB of the GEMV is more than the 64 KB of
-    // instructions that two CUs cache, and a layer's launches displace each other's: 5120 / 17408 at 4 bits, 1 row, two layers 135.1 -> 134.1 us, 1024 / 2816 26.28 -> 26.01.)
+    // instructions that two CUs cache, and a layer's launches displace each other's: 5120 / 17408 at 4 bits, 1 row, two layers 134.6 -> 133.5 us, 1024 / 2816 26.11 -> 25.84.)
     const bool rotating = CHAIN != 0 || src.x != nullptr;
     struct RotAt {
         size_t at, xat;
@@ -838,8 +838,9 @@ GEMVB_FAMILY(8)
 // 5120 / 17408 layer, 8.0 of 17.6 for o, 7.6 of 42.8 for gate and up, 14.2 of 34.9 for down; now 13.7 + 4.6, 11.3 + 4.7, 36.4 + 6.1, 21.8 + 5, and the launch
 // behind gate and up leaves down's rotated input as well, which took a launch of 5 us.) A layer at 17 / 40 / 64 rows 107 / 138 / 173 -> 99 / 116 / 140 us. Written through
 // (a plain store leaves the launch's end to write 14 MB back: 1 to 2 us more). Registers stay under 128, so that four programs share a
-// CU. Bound by the decode (gate and up: 22 us at the vector ALUs' rate), each program's start, and the products; decoding the next step between the
-// products of this one was measured and changes nothing, the other programs of the CU already fill that time.
+// CU. Bound by the decode and each program's start and end: at 40 rows and 4 bits gate and up issue vector instructions for 20 us, 70 % of the time between the first wavefront and
+// the last, in a launch of 37 (matrix pipe busy in 23 %, LDS bank conflicts 12 % of the cycles). Decoding the next step between the products of this one was measured and changes
+// nothing.
 template <int BITS, int RG>
 struct GemvWide {
     static constexpr int X_STAGE = RG * 2048, W_STAGE = 1024 * BITS;
@@ -885,8 +886,9 @@ __device__ __forceinline__ void gemv_wide_body(const GemvMember mb, uint32_t p, 
     const uint32_t uend = run_start(PER * p + PER < mb.programs ? PER * p + PER : mb.programs), mid = run_start(PER * p + 1);
     while (u < uend) {
         // A step's offsets and stages are running scalars: the quotient comes from the vector unit, and left there it takes the loads' offsets, a 32-bit multiply among them,
-        // and the stages along, 133..139 vector instructions a step where the decode takes 119; 123 so. A layer of 5120 / 17408 at 3 bits, 17 / 32 / 40 / 64 rows 90.3 / 94.5 / 104.8 /
-        // 122.5 -> 86.3 / 90.5 / 102.4 / 120.7 us, at 4 bits 88.9 / 93.3 / 105.6 / 125.9 -> 86.5 / 90.9 / 102.9 / 122.7, 9 rows 86.8 -> 84.7.
+        // and the stages along, 133..139 vector instructions a step where the decode takes 119; 123 so. A layer of 5120 / 17408 again and again, 17 / 32 / 40 / 64 rows at 3 bits 88.6 / 92.9 /
+        // 101.5 / 118.3 -> 83.7 / 87.9 / 99.2 / 116.5 us, at 4 bits 87.2 / 91.4 / 101.6 / 120.9 -> 84.8 / 88.7 / 99.8 / 117.4, 9 rows 86.6 -> 84.2; three layers in turn, whose weights
+        // no cache holds: 94.8 / 98.0 / 106.6 / 125.6 -> 90.1 / 93.4 / 104.2 / 124.0, 94.8 / 98.6 / 108.0 / 130.0 -> 93.4 / 96.0 / 106.3 / 125.4, 88.2 -> 86.8.
         const uint32_t nb = __builtin_amdgcn_readfirstlane(u / upb), in = u - nb * upb, units = uend - u < upb - in ? uend - u : upb - in, steps = 2 * units;
         const uint32_t aside = mid > u && mid < u + units ? 2 * (mid - u) : steps;  // the step at which the second program's run starts
         u += units;

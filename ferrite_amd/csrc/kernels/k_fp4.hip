@@ -437,7 +437,7 @@ __device__ __forceinline__ void swiglu_quant_store(const float (&v)[4], f32x4 al
 // of the block's features 4 fc .. + 3; the block's maximum comes from the lanes 16 and 32 away; and two blocks trade rows of 16 lanes, so that a lane stores 8 features of one
 // (a tile with one block a wavefront: 4). rows: those that exist from row0 on.
 // Bound by its vector instructions, which no matrix instruction hides (a program has its CU alone): about 10 us a program through the slab, half of that now. Launch, us: 2048
-// rows of 34816 x 5120 558 -> 535, 390 rows 144 -> 132; MLP blocks of 2048 / 5 + 390 rows 888 -> 841, 287.5 -> 273.7 with the residual's loads ahead.
+// rows of 34816 x 5120 558 -> 535, 390 rows 144 -> 132; MLP blocks of 2048 / 5 + 390 rows 865 -> 816, 279 -> 269.
 template <class T>
 __device__ __forceinline__ void fp4_tile_swiglu(f32x4 (&acc)[T::TM][T::TN], const float* alpha, float scale, uint32_t row0, uint32_t rows, uint32_t colb, uint32_t n, uint8_t* q_codes,
                                                 uint8_t* q_sf, _Float16* q_aq, float qg) {
