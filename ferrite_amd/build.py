@@ -21,10 +21,11 @@ HIPCC = os.path.join(ROCM, "bin", "hipcc")
 DEVICE_FLAGS = ["--offload-arch=gfx950", "-O3", "-std=c++17", "-mcode-object-version=5",
                 "-Xclang", "-target-feature", "-Xclang", "-packed-fp32-ops"]
 # code objects: name, source, defines; the ones that take longest first
-# ALIGNED: loops that start a line of the instruction cache. Where a tile loop of 1.4 KB happens to start moves a GEMM by 2 % (NVFP4, 512 rows of 17408 x 5120: 85.5 us at the start of a
-# line, 87.4 twelve bytes into one). Not the trellis decode's object, whose groups of load steps are straight code of 8 KB: there the padding costs more (1024 / 2816 at 1 row 26.0 -> 26.35 us).
-# The GEMVs of NVFP4, FP8 and bf16 share the GEMMs' objects and are padded with them, which costs them nothing: 260 calls of 1..48 rows from a graph, 512 x 2048 .. 17408 x 5120, 1.000 of the
-# time without, at most 2.6 % more (bf16 512 x 2048 at 8 rows 2.68 -> 2.75 us) or 5 % less.
+# ALIGNED: loops that start a line of the instruction cache. Where a tile loop of 1.4 KB happens to start moves a GEMM by 2 % (NVFP4, 512 rows of
+# 17408 x 5120: 85.5 us at the start of a line, 87.4 twelve bytes into one). Not the trellis decode's object, whose groups of load steps are straight
+# code of 8 KB: there the padding costs more (1024 / 2816 at 1 row 26.0 -> 26.35 us). The GEMVs of NVFP4, FP8 and bf16 share the GEMMs' objects and
+# are padded with them, which costs them nothing: 260 calls of 1..48 rows from a graph, 512 x 2048 .. 17408 x 5120, 1.000 of the time without, at most
+# 2.6 % more (bf16 512 x 2048 at 8 rows 2.68 -> 2.75 us) or 5 % less.
 ALIGNED = ["-falign-loops=128"]
 KERNELS = [("k_exl3_gemm", "k_exl3_gemm.hip", ALIGNED)]
 KERNELS += [(f"k_exl3_rgemm_b{b}", "k_exl3_rgemm.hip", ALIGNED + [f"-DRG_BITS={b}"]) for b in (8, 6, 5, 4, 3, 2)]

@@ -11,7 +11,8 @@
 #include "fe_internal.h"
 
 namespace {
-// dynamic LDS by form (256 x 256, unused, 128 x 256, 128 x 128, 224, 192, 160 x 256): the k tiles in flight, three of W and two of A (128 x 256: three), A in whole loads of 64 rows
+// dynamic LDS by form (256 x 256, unused, 128 x 256, 128 x 128, 224, 192, 160 x 256): the k tiles in flight, three of W and two of A (128 x 256:
+// three), A in whole loads of 64 rows
 constexpr uint32_t kGemmLds[kFeGemmForms] = {160 * 1024, 0, 144 * 1024, 80 * 1024, 160 * 1024, 144 * 1024, 144 * 1024};
 constexpr uint32_t kGemmThreads = 512;
 constexpr uint32_t kTileM = 256;                         // rows of the largest output tile
@@ -66,7 +67,8 @@ static bool gemm_reaches(uint32_t m, uint32_t n, uint32_t k, uint32_t lda) { ret
 static FeGemmPlan gemm_plan(const fe_bf16_kernels *kern, uint32_t m, uint32_t n, uint32_t k) {
     return fe_gemm_plan(m, n, k / 64, kern->cus, kern->part.p, kern->part.bytes, 0, 0, kern->gemm_splits, 0, false, kFeCostBf16, kern->tile);
 }
-// Whether all of a call's rows go through the GEMV: a batch of decode rows, or 17..32 rows where its one read of the weights is ahead of the GEMM's tiles (kFeGemvBf16).
+// Whether all of a call's rows go through the GEMV: a batch of decode rows, or 17..32 rows where its one read of the weights is ahead of the GEMM's
+// tiles (kFeGemvBf16).
 static bool rows_take_gemv(const fe_bf16_kernels *kern, uint32_t m, uint32_t n, uint32_t k, uint32_t lda, uint32_t dec) {
     if (m <= kSmallBatch || dec >= m) return true;
     if (m > 32 || k % 256 || !gemm_reaches(m - dec, n, k, lda)) return false;
@@ -76,8 +78,8 @@ static bool rows_take_gemv(const fe_bf16_kernels *kern, uint32_t m, uint32_t n, 
 bool fe_bf16_gemv_swiglu_takes(const fe_bf16_kernels *kern, fe_devptr_t big, fe_devptr_t act, fe_devptr_t x, fe_devptr_t gate, fe_devptr_t up, uint32_t m, uint32_t inter,
                                uint32_t k, uint32_t dec, bool over_gemm) {
     if (!kern || !m || m > kGemvPass || !inter || !k || inter % 8 || k % 256 || (uint64_t)m * k * 2 >= (1ull << 32)) return false;
-    // (against the GEMM with SwiGLU: kFeGemvBf16Pair. Against gate, up and fe_silu_mul, where there are no such weights, it is ahead wherever those go through the GEMV: 5120 x 8704 at
-    // 26 / 32 rows 63.0 -> 58.0, 63.9 -> 58.6, 5120 x 6144 at 30 53.0 -> 48.4, 7168 x 2048 at 25 32.7 -> 28.0)
+    // (against the GEMM with SwiGLU: kFeGemvBf16Pair. Against gate, up and fe_silu_mul, where there are no such weights, it is ahead wherever those
+    // go through the GEMV: 5120 x 8704 at 26 / 32 rows 63.0 -> 58.0, 63.9 -> 58.6, 5120 x 6144 at 30 53.0 -> 48.4, 7168 x 2048 at 25 32.7 -> 28.0)
     if (over_gemm && m > kSmallBatch && dec < m) {
         if (m > 32 || !gemm_reaches(m - dec, 2 * inter, k, k)) return false;
         if (!fe_gemv_ahead(kFeGemvBf16Pair, m, inter, k, k / 64, std::max(kern->cus, 1u), 2, gemm_plan(kern, m - dec, 2 * inter, k), (float)inter * (float)k * 4.0f, dec)) return false;

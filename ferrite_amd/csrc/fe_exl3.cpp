@@ -17,11 +17,12 @@
 namespace {
 
 constexpr uint32_t kMaxRowsPerPass = 64;       // 4 row groups of 16
-// Rows from which the prefill decodes once into fp16 tiles (9 output tile rows). Decoding in the registers (exl3_rgemm_b*) against once, us, at 2048 (or 2100) / 2304 / 2560 (2600) /
-// 3072 / 4096 rows, 4 bits: 5120 x 17408 345 / 388 / 431 / 507 / 667 against 341 / 400 / 434 / 484 / 638, 17408 x 5120 353 / 401 / 449 / 497 / 663 against 374 / 406 / 435 / 479 / 646, 5120 x 5120 126 /
-// 136 / 141 / 158 / 220 against 139 / 132 / 138 / 152 / 210, 4096 x 14336 244 / 251 / 315 / 355 / 461 against 241 / 244 / 308 / 357 / 432, 11008 x 4096 203 / 211 / 248 / 275 / 335 against 243 / 245 / 258 / 272 /
-// 327; at 2 and 8 bits alike. So they meet between 2304 and 2600 rows. Linears below about 16 million weights stay faster in the registers up to 4000 rows (2048 x 2048 39 / 42 / 42 / 47 / 50 against
-// 47 / 50 / 74 / 79 / 64), which this line does not tell apart.
+// Rows from which the prefill decodes once into fp16 tiles (9 output tile rows). Decoding in the registers (exl3_rgemm_b*) against once, us, at 2048
+// (or 2100) / 2304 / 2560 (2600) / 3072 / 4096 rows, 4 bits: 5120 x 17408 345 / 388 / 431 / 507 / 667 against 341 / 400 / 434 / 484 / 638, 17408 x
+// 5120 353 / 401 / 449 / 497 / 663 against 374 / 406 / 435 / 479 / 646, 5120 x 5120 126 / 136 / 141 / 158 / 220 against 139 / 132 / 138 / 152 / 210,
+// 4096 x 14336 244 / 251 / 315 / 355 / 461 against 241 / 244 / 308 / 357 / 432, 11008 x 4096 203 / 211 / 248 / 275 / 335 against 243 / 245 / 258 /
+// 272 / 327; at 2 and 8 bits alike. So they meet between 2304 and 2600 rows. Linears below about 16 million weights stay faster in the registers up
+// to 4000 rows (2048 x 2048 39 / 42 / 42 / 47 / 50 against 47 / 50 / 74 / 79 / 64), which this line does not tell apart.
 constexpr uint32_t kHatRows = 2304;
 constexpr uint32_t kChainRows = 8;             // most rows of the one-launch MLP (mlp_chain_fits)
 constexpr uint32_t kWideWhole = 4;             // WIDE_WHOLE of k_exl3.hip
@@ -342,11 +343,11 @@ int fe_exl3_plan_for(uint32_t k, uint32_t n, uint32_t bits, uint32_t blocks, fe_
         if (!tuned && units < (uint32_t)cus) wk = 2;
         // Wider than deep (gate, up) with more than two but fewer than four programs a CU: two. Such linears come in pairs, whose
         // programs then fill the CUs once. us, 4 bits, one linear / gate and up at 1 and at 40 rows: 5120 x 8704, 680 programs 13.3 / 20.5, 25.0 / 36.3,
-        // 512 programs 12.5 / 18.3, 22.2 / 34.3; 5120 x 7168, 560: 12.8 / 20.2, 25.2 / 33.4, 512: 12.0 / 16.4, 22.6 / 32.1; 4096 x 11008, 688: 13.2 / 20.5, 23.8 / 36.4, 512:
-        // 13.8 / 19.6, 23.4 / 33.7 (one such linear alone is the loser, 0.6 us up to 8 rows). Of four programs a CU and more all four, which
-        // hide each other's loads where one linear runs alone (5120 x 17408, 512 -> 1024 programs: 1, 2, 16 rows 20.5 -> 18.2, 21.9 -> 19.1, 26.9 -> 25.0; gate
-        // and up 30.9 -> 30.7, 33.3 -> 32.3, 42.2 -> 41.8) and from 17 rows on run in pairs (programs_per); at 8 bits, with twice the bytes in flight,
-        // they gain nothing: 1, 5, 16 rows 23.9 -> 24.3, 26.6 -> 28.8, 32.4 -> 32.8.
+        // 512 programs 12.5 / 18.3, 22.2 / 34.3; 5120 x 7168, 560: 12.8 / 20.2, 25.2 / 33.4, 512: 12.0 / 16.4, 22.6 / 32.1; 4096 x 11008, 688: 13.2 /
+        // 20.5, 23.8 / 36.4, 512: 13.8 / 19.6, 23.4 / 33.7 (one such linear alone is the loser, 0.6 us up to 8 rows). Of four programs a CU and more
+        // all four, which hide each other's loads where one linear runs alone (5120 x 17408, 512 -> 1024 programs: 1, 2, 16 rows 20.5 -> 18.2, 21.9
+        // -> 19.1, 26.9 -> 25.0; gate and up 30.9 -> 30.7, 33.3 -> 32.3, 42.2 -> 41.8) and from 17 rows on run in pairs (programs_per); at 8 bits,
+        // with twice the bytes in flight, they gain nothing: 1, 5, 16 rows 23.9 -> 24.3, 26.6 -> 28.8, 32.4 -> 32.8.
         if (!tuned && n > k && occ == 4 && units / wk > 2 * (uint32_t)cus && (bits == 8 || units / wk < 4 * (uint32_t)cus)) occ = 2;
     }
     occ = env_u32("FE_EXL3_OCC", occ), wk = std::max(1u, env_u32("FE_EXL3_MIN_UNITS", wk));  // tuning runs
@@ -645,10 +646,10 @@ static bool rgemm_reaches(const fe_exl3_linear *l, uint32_t rows) {
 }
 
 // ... and whether they do, by the estimates of both (fe_rgemm_takes): the other one is the faster on some narrow linears, where its smaller tiles
-// need fewer pieces of K. us with the rotation, 4 bits, LDS / the registers alone, by the plan before this estimate / by this rule: 16896 x 1920 at 1501 rows 131 / 136 /
-// 131, 3328 x 1024 at 387 rows 23.1 / 27.7 / 23.0, 2816 x 1024 at 512 rows 22.8 / 27.8 / 23.1 (through LDS), 5120 x 1024 at 128 rows 21.1 / 23.6 / 17.3, 17408 x 5120 at 203, 512
-// and 2048 rows 69.5 / 61.9 / 55.4, 110 / 118 / 105, 370 / 355 / 354, 5120 x 17408 at 203 rows 65.8 / 64.2 / 60.9. MLP blocks: 110 drawn ones take 0.77 of their time through LDS and 0.97 of
-// their time by the plan before (slowest: 1.00 and 1.05).
+// need fewer pieces of K. us with the rotation, 4 bits, LDS / the registers alone, by the plan before this estimate / by this rule: 16896 x 1920 at
+// 1501 rows 131 / 136 / 131, 3328 x 1024 at 387 rows 23.1 / 27.7 / 23.0, 2816 x 1024 at 512 rows 22.8 / 27.8 / 23.1 (through LDS), 5120 x 1024 at 128
+// rows 21.1 / 23.6 / 17.3, 17408 x 5120 at 203, 512 and 2048 rows 69.5 / 61.9 / 55.4, 110 / 118 / 105, 370 / 355 / 354, 5120 x 17408 at 203 rows 65.8
+// / 64.2 / 60.9. MLP blocks: 110 drawn ones take 0.77 of their time through LDS and 0.97 of their time by the plan before (slowest: 1.00 and 1.05).
 static bool rgemm_takes(const fe_exl3_linear *const *ls, size_t count, uint32_t rows, const fe_exl3_workspace *ws, FeRgemmPlan *p) {
     const fe_exl3_kernels *kern = ls[0]->kern;
     const fe_exl3_options &o = kern->opt;
@@ -790,9 +791,9 @@ static bool gemv_reaches(const fe_exl3_linear *l) { return fe_exl3_linear_weight
 
 // Programs that a workgroup of the GEMV for 17..64 rows runs as one: two where every linear of the launch has four programs a CU. Every
 // segment leaves its sums of all rows in memory, so from 17 rows on half as many segments pay, while up to 16 rows the programs as
-// they are hide each other's loads (the bits are the same). 5120 x 17408 at 4 bits (1024 programs, 2 x 20 KB of sums each at 40 rows), one linear / gate and up,
-// us, single programs -> pairs: 17 rows 25.6 / 41.2 -> 25.5 / 39.2, 40 rows 29.9 / 50.6 -> 28.8 / 45.6, 64 rows 35.0 / 57.9 -> 32.8 / 53.2; 17408 x 5120 at 6 bits 40 / 64
-// rows 34.2 / 43.2 -> 33.4 / 37.9.
+// they are hide each other's loads (the bits are the same). 5120 x 17408 at 4 bits (1024 programs, 2 x 20 KB of sums each at 40 rows), one linear /
+// gate and up, us, single programs -> pairs: 17 rows 25.6 / 41.2 -> 25.5 / 39.2, 40 rows 29.9 / 50.6 -> 28.8 / 45.6, 64 rows 35.0 / 57.9 -> 32.8 /
+// 53.2; 17408 x 5120 at 6 bits 40 / 64 rows 34.2 / 43.2 -> 33.4 / 37.9.
 static uint32_t programs_per(const fe_exl3_linear *const *ls, size_t count) {
     const uint32_t opt = ls[0]->kern->opt.gemv_pairs;
     for (size_t i = 0; i < count; i++)
@@ -802,9 +803,11 @@ static uint32_t programs_per(const fe_exl3_linear *const *ls, size_t count) {
 
 // Who finishes the column blocks of 17..64 rows: the GEMV's programs, where no block is cut (wide linears of a short K: the launch behind would only carry
 // sums to memory and back); from 33 rows on the programs and the launch each their own, where half the blocks are whole and there are programs enough
-// to finish them side by side; else the launch all of them. us, 4 bits, all by the launch -> by this rule, 17 / 33 / 64 rows: whole: 512 x 65536 15.1 / - / 21.4 -> 12.4 / - / 15.7,
-// 768 x 65536 18.4 / 21.3 / 25.1 -> 15.4 / 17.4 / 19.8, 2560 x 131072 66.5 / 77.8 / 89.6 -> 63.8 / 71.4 / 82.7, 5120 x 131072 124.7 / 145.0 / 162.3 -> 121.0 / 137.4 / 157.4;
-// both: 512 x 99968 25.3 / 32.3 -> 24.1 / 29.3 at 33 / 64, 1024 x 151936 50.3 / 59.6 -> 48.6 / 56.9 (at 17 rows both lose 0 to 4 % to the launch). Few programs finish
+// to finish them side by side; else the launch all of them. us, 4 bits, all by the launch -> by this rule, 17 / 33 / 64 rows: whole: 512 x 65536 15.1
+// / - / 21.4 -> 12.4 / - / 15.7, 768 x 65536 18.4 / 21.3 / 25.1 -> 15.4 / 17.4 / 19.8, 2560 x 131072 66.5 / 77.8 / 89.6 -> 63.8 / 71.4 / 82.7, 5120 x
+// 131072 124.7 / 145.0 / 162.3 -> 121.0 / 137.4 / 157.4;
+// both: 512 x 99968 25.3 / 32.3 -> 24.1 / 29.3 at 33 / 64, 1024 x 151936 50.3 / 59.6 -> 48.6 / 56.9 (at 17 rows both lose 0 to 4 % to the launch).
+// Few programs finish
 // slowly: 256 x 32896, 128 of them, 40 / 64 rows 16.0 / 18.9 by the launch, 17.4 / 20.5 by both.
 enum class WideEnd { Launch, Both, Programs };
 static WideEnd wide_end(const fe_exl3_linear *const *ls, size_t count, uint32_t per, uint32_t rows) {
@@ -1143,9 +1146,9 @@ static bool mlp_chain_fits(const fe_exl3_linear *g, const fe_exl3_linear *u, con
     if (rows < 1 || rows > 16 || rows > ws->max_rows || y_dtype < 0 || y_dtype > 3) return false;
     // every stage rotates its own input inside the launch, (row, 128-channel block) pairs a program and round of the front stage (as
     // fused_rotation_fits, but there are two rotations' launches to save). One launch against several, us: 5120 x 17408 at 4 bits (6 units, two rounds) 4 / 5 /
-    // 6 / 8 rows 52.6 / 56.3 / 58.9 / 64.4 against 55.5 / 57.2 / 57.6 / 59.8; 5120 x 8704 (6 units, one round) 6 / 8 / 10 rows 37.6 / 41.1 / 46.2 against 39.7 / 41.3 /
-    // 43.2; 2048 x 5632 (4 units) 6 / 8 / 10 / 12 rows 24.0 / 26.5 / 30.1 / 32.0 against 25.7 / 26.1 / 27.5 / 27.5; 1024 x 2816 (2 units) 8 / 10 rows 21.2 / 24.3 against
-    // 23.2 / 21.6. So up to 8 rows and 48 pairs.
+    // 6 / 8 rows 52.6 / 56.3 / 58.9 / 64.4 against 55.5 / 57.2 / 57.6 / 59.8; 5120 x 8704 (6 units, one round) 6 / 8 / 10 rows 37.6 / 41.1 / 46.2
+    // against 39.7 / 41.3 / 43.2; 2048 x 5632 (4 units) 6 / 8 / 10 / 12 rows 24.0 / 26.5 / 30.1 / 32.0 against 25.7 / 26.1 / 27.5 / 27.5; 1024 x 2816
+    // (2 units) 8 / 10 rows 21.2 / 24.3 against 23.2 / 21.6. So up to 8 rows and 48 pairs.
     const fe_exl3_options &o = g->kern->opt;
     const uint32_t d_units = units_per_program(d, chain_part(d)->programs), rounds = launch_rounds(g->kern, g->programs + u->programs);
     const uint32_t f_units = std::max(units_per_program(g, g->programs), units_per_program(u, u->programs));
@@ -1236,9 +1239,10 @@ int fe_exl3_mlp_forward(const fe_exl3_linear *gate, const fe_exl3_linear *up, co
     }
     bool fused = false;
     // From 9 rows on gate and up leave their sums to a launch that finishes them with all CUs and rotates down's input too, in the place of the
-    // rotation's launch. A layer, 4 / 5 / 8 bits, at 5 / 8 / 11 / 16 rows, with the finisher inside the GEMV and a rotation / this way: 5120 x 17408 84.7 / 96.4 /
-    // 96.9 / 130.0 us against 85.9 / 97.0 / 93.1 / 123.8, 2560 x 6912 59.3 / 67.6 against 57.5 / 64.8 at 11 / 16. Over 271 MLP blocks of 9..16 rows (2 to 8 bits, 512 .. 6144 wide) 0.95 of the
-    // time (geometric mean; slowest 1.03: 2560 x 6912 at 9 rows and 2 bits, 31.5 against 32.5 us).
+    // rotation's launch. A layer, 4 / 5 / 8 bits, at 5 / 8 / 11 / 16 rows, with the finisher inside the GEMV and a rotation / this way: 5120 x 17408
+    // 84.7 / 96.4 / 96.9 / 130.0 us against 85.9 / 97.0 / 93.1 / 123.8, 2560 x 6912 59.3 / 67.6 against 57.5 / 64.8 at 11 / 16. Over 271 MLP blocks
+    // of 9..16 rows (2 to 8 bits, 512 .. 6144 wide) 0.95 of the time (geometric mean; slowest 1.03: 2560 x 6912 at 9 rows and 2 bits, 31.5 against
+    // 32.5 us).
     if (rows > 8 && group_fits(front, 2, rows, ws, &fused) && !fused && down->k <= ws->max_k && (rows > 16 || !kern->opt.handoff_fenced)) {
         FE_TRY(forward_group(front, 2, kern, s, x, x_dtype, ys, FE_DTYPE_BF16, rows, ws, false, dl, fn));
         return launch_rows(dl, s, ws->xh.p, y, y_dtype, rows, ws, RotInput{});

@@ -14,9 +14,9 @@
 
 namespace {
 constexpr uint32_t kTile = 128;                 // crates/fe-fp4/src/lib.rs:28
-// dynamic LDS by form (256 x 256, its stream-K form, 128 x 256, 128 x 128, 224, 192, 160 x 256): the k tiles in flight, A in whole loads of 64 rows. Packed weights: three of
-// A (128 bytes a row; 128 x 256: five) and three of W (36 bytes, 64 in the fp16 form of FP8; 128 x 256: six, 128 x 128: four). FP8 codes: two of A (128 x 256: three), three of
-// W, 128 bytes a row.
+// dynamic LDS by form (256 x 256, its stream-K form, 128 x 256, 128 x 128, 224, 192, 160 x 256): the k tiles in flight, A in whole loads of 64 rows.
+// Packed weights: three of A (128 bytes a row; 128 x 256: five) and three of W (36 bytes, 64 in the fp16 form of FP8; 128 x 256: six, 128 x 128:
+// four). FP8 codes: two of A (128 x 256: three), three of W, 128 bytes a row.
 constexpr uint32_t kGemmLds[kFeGemmForms] = {144 * 1024, 144 * 1024, 136 * 1024, 68 * 1024, 144 * 1024, 120 * 1024, 120 * 1024};
 constexpr uint32_t kGemmLds8[kFeGemmForms] = {160 * 1024, 160 * 1024, 144 * 1024, 80 * 1024, 160 * 1024, 144 * 1024, 144 * 1024};
 // Forms of the GEMV over programs of 8 CO columns: rows / 2 and CO
@@ -30,8 +30,8 @@ constexpr uint32_t kCuLds = 160 * 1024;
 constexpr uint32_t kQuantValues = 10240;
 // The wavefronts of a form: eight where K is summed in eighths and two stages of eight wavefronts fit the LDS.
 uint32_t wide_waves(uint32_t xp, uint32_t co, bool eighths, bool q = false) { return eighths && co <= 6 && (q || xp <= 2 || (xp == 4 && co <= 4)) ? 8 : 4; }
-// Which widths exist: those that a rule or "gemv_cols" may pick. Nine octets pay with 9..16 rows of more columns than six octets a CU; a program of eight wavefronts that
-// quantizes takes two octets rather than one (wide_form).
+// Which widths exist: those that a rule or "gemv_cols" may pick. Nine octets pay with 9..16 rows of more columns than six octets a CU; a program of
+// eight wavefronts that quantizes takes two octets rather than one (wide_form).
 constexpr bool wide_built(uint32_t co, bool eighths, bool q) { return co == 9 ? !eighths && !q : co > 1 || !eighths || !q; }
 constexpr uint32_t kGemmThreads = 512;
 constexpr uint32_t kTileM = 256;                        // GM_BM
@@ -54,8 +54,8 @@ struct fe_fp4_kernels {
     uint32_t gemv = 1;         // few rows run the GEMV (takes_gemv, fe_gemv_ahead; FE_FP4_NO_GEMV=1: the GEMM's single tile row)
     uint32_t gemv_sk = 0;      // K splits of the GEMV over weight tiles; 0 = two programs a CU (FE_FP4_GEMV_SK)
     uint32_t gemv_strips = 1;  // up to 16 rows run programs of some columns over all of K; 0: weight tiles and K splits, as more rows do (FE_FP4_NO_STRIPS=1)
-    // most values (rows x k) that the four wavefronts of the GEMV for up to 16 rows quantize themselves, in every program; eight take twice as many; -1: by the shape, at most
-    // kQuantValues (FE_FP4_GEMV_QUANT)
+    // most values (rows x k) that the four wavefronts of the GEMV for up to 16 rows quantize themselves, in every program; eight take twice as many;
+    // -1: by the shape, at most kQuantValues (FE_FP4_GEMV_QUANT)
     int32_t gemv_quant = -1;
     uint32_t gemv_cols = 0;    // columns a program of the GEMV for up to 16 rows, or of the FP8 GEMV, takes, rounded up to 8, 16, .. 48, 72; 0 = by the shape (FE_FP4_GEMV_COLS)
     int32_t xcd = -1;          // column tiles dealt to the XCDs: -1 = where the weights are the larger operand (FE_FP4_XCD)
@@ -396,13 +396,13 @@ static uint32_t wide_cols(uint32_t n, uint32_t xp, uint32_t cus, uint32_t forced
 }
 
 // The kernel of the GEMV of up to 16 rows; q: the one that quantizes its activations itself.
-// Linears that give no CU a second program sum eighths of K, with eight wavefronts up to 8 rows: a program's steps are a chain of LDS reads, scale products and matrix
-// instructions, which two wavefronts a SIMD overlap. (By the linear's shape alone: its rows' bits are the same at 1 to 16 rows.) us, quarters -> eighths:
-// 5120 x 5120 at 1 / 4 / 8 / 12 rows 7.2 -> 6.6, 8.2 -> 8.0, 9.0 -> 9.0, 9.8 -> 9.8; 5120 x 17408 15.1 -> 14.0, 14.8 -> 14.8, 18.3 -> 17.2, 19.7 -> 20.0; 5120 x 8704 9.9 -> 9.1,
-// 10.3 -> 10.4, 11.9 -> 11.4, 12.8 -> 12.9; 2048 x 11008 9.3 -> 7.2, 9.3 -> 8.7, 9.4 -> 9.4, 12.4 -> 12.4; 10240 x 4096 at 3 9.9 -> 8.0; 7168 x 2048 at 6 6.9 -> 5.2. With more
-// programs than CUs two of four wavefronts a CU are better (34816 x 5120 at 1 row 22.7 against 24.5), and of 1024 channels half of eight have no step (1024 x 1024 at 8
-// rows 4.3 -> 4.9).
-// Programs of eight that quantize take two octets rather than one: 1024 x 5120 at 1 row 5.3 -> 4.8, 2048 x 2048 at 8 rows 5.5 -> 4.9.
+// Linears that give no CU a second program sum eighths of K, with eight wavefronts up to 8 rows: a program's steps are a chain of LDS reads, scale
+// products and matrix instructions, which two wavefronts a SIMD overlap. (By the linear's shape alone: its rows' bits are the same at 1 to 16 rows.)
+// us, quarters -> eighths: 5120 x 5120 at 1 / 4 / 8 / 12 rows 7.2 -> 6.6, 8.2 -> 8.0, 9.0 -> 9.0, 9.8 -> 9.8; 5120 x 17408 15.1 -> 14.0, 14.8 ->
+// 14.8, 18.3 -> 17.2, 19.7 -> 20.0; 5120 x 8704 9.9 -> 9.1, 10.3 -> 10.4, 11.9 -> 11.4, 12.8 -> 12.9; 2048 x 11008 9.3 -> 7.2, 9.3 -> 8.7, 9.4 ->
+// 9.4, 12.4 -> 12.4; 10240 x 4096 at 3 9.9 -> 8.0; 7168 x 2048 at 6 6.9 -> 5.2. With more programs than CUs two of four wavefronts a CU are better
+// (34816 x 5120 at 1 row 22.7 against 24.5), and of 1024 channels half of eight have no step (1024 x 1024 at 8 rows 4.3 -> 4.9). Programs of eight
+// that quantize take two octets rather than one: 1024 x 5120 at 1 row 5.3 -> 4.8, 2048 x 2048 at 8 rows 5.5 -> 4.9.
 struct WideForm {
     uint32_t programs, waves, lds;
     fe_function_t f;
@@ -421,34 +421,37 @@ static WideForm wide_form(const fe_fp4_linear *l, const fe_fp4_kernels *kern, ui
 static bool takes_wide(const fe_fp4_linear *l, const fe_fp4_kernels *kern, uint32_t m) {
     return !l->fp8 && m <= 16 && l->n / kTile <= kGemvCounters && kern->gemv && kern->gemv_strips && !kern->gemv_sk && l->k % 256 == 0;
 }
-// Whether m rows go through a GEMV: all of one pass. 49..64 rows take two, which the GEMM beats (us at 64 rows, two passes -> GEMM: 34816 x 5120 83 -> 63, 17408 x
-// 5120 41 -> 32, 5120 x 17408 43 -> 30, 5120 x 5120 27 -> 17.5, 2048 x 6144 27 -> 14; 48 rows in one pass 51, 26, 27, 17, 17 against 62, 31, 30, 17, 14); they stay where
-// the caller asked for weight tiles (gemv_strips 0: a row's bits the same at every count up to 64) or their K splits, with operands that the GEMM does not reach, and where K is so deep
-// that the GEMM's eight pieces of a tile are longer than 16 splits (of 1907 linears of 49..64 rows the rule leaves 23 more than 3 % slower than the better one; without it 256 x 59136 at 53
-// 45 against 57).
-// From 33 rows on narrow linears of middling depth take it, too, whose tiles are cut along K either way (us at 48 rows, GEMV -> GEMM: 4096 x 4096 16.7 -> 14.1, 2048 x 6144 17.1 ->
-// 13.7, 1024 x 5120 15.0 -> 11.3, 1024 x 2816 12.3 -> 10.1, 128 x 8192 14.4 -> 13.1; beyond the lines 5120 x 5120 16.8 -> 16.9, 7168 x 2048 13.0 -> 13.7, 1024 x 1024 9.1 ->
-// 9.9, 512 x 14336 17.0 -> 18.9).
+// Whether m rows go through a GEMV: all of one pass. 49..64 rows take two, which the GEMM beats (us at 64 rows, two passes -> GEMM: 34816 x 5120 83
+// -> 63, 17408 x 5120 41 -> 32, 5120 x 17408 43 -> 30, 5120 x 5120 27 -> 17.5, 2048 x 6144 27 -> 14; 48 rows in one pass 51, 26, 27, 17, 17 against
+// 62, 31, 30, 17, 14); they stay where the caller asked for weight tiles (gemv_strips 0: a row's bits the same at every count up to 64) or their K
+// splits, with operands that the GEMM does not reach, and where K is so deep that the GEMM's eight pieces of a tile are longer than 16 splits (of
+// 1907 linears of 49..64 rows the rule leaves 23 more than 3 % slower than the better one; without it 256 x 59136 at 53 45 against 57). From 33 rows
+// on narrow linears of middling depth take it, too, whose tiles are cut along K either way (us at 48 rows, GEMV -> GEMM: 4096 x 4096 16.7 -> 14.1,
+// 2048 x 6144 17.1 -> 13.7, 1024 x 5120 15.0 -> 11.3, 1024 x 2816 12.3 -> 10.1, 128 x 8192 14.4 -> 13.1; beyond the lines 5120 x 5120 16.8 -> 16.9,
+// 7168 x 2048 13.0 -> 13.7, 1024 x 1024 9.1 -> 9.9, 512 x 14336 17.0 -> 18.9).
 static bool takes_gemv(const fe_fp4_linear *l, const fe_fp4_kernels *kern, uint32_t m, bool gemm_reaches) {
     if (l->fp8 || m > kGemvMaxRows || l->n / kTile > kGemvCounters || !kern->gemv) return false;
     if (!kern->gemv_strips || kern->gemv_sk || !gemm_reaches) return true;
     return m <= 32 || (m <= kGemvRows ? l->n > 4096 || l->k < 2048 || l->k > 8192 : l->k > 28000 + 12 * l->n);
 }
 
-// K splits of the GEMV over weight tiles. Two programs fit a CU: as many programs as run at once, not more (a second round of short programs costs more than idle CUs in
-// the first).
+// K splits of the GEMV over weight tiles. Two programs fit a CU: as many programs as run at once, not more (a second round of short programs costs
+// more than idle CUs in the first).
 static uint32_t gemv_splits(const fe_fp4_kernels *kern, const fe_fp4_workspace *ws, uint32_t n, uint32_t k) {
     uint32_t sk = std::min({kern->gemv_sk ? kern->gemv_sk : 2 * kern->cus / (n / kTile), 16u, k / 64 / 4});
     while (sk > 1 && (size_t)sk * kGemvRows * n * 4 > ws->part.bytes) sk--;
     return std::max(sk, 1u);
 }
 
-// Whether a fused gate|up linear's rows go through the GEMV, by sk splits of K, and not through the GEMM that `plan` is of: up to 16 rows, and up to 48 where an estimate of both
-// (us) has it ahead. The GEMV's: a start, a wavefront's k tiles (less each where a CU has two programs), the weights' way, and the splits' sums, written and read. The
-// GEMM's: its plan's and what that leaves out at so few rows; pieces of K cost less than it says. Fitted to 11766 calls of 17..48 rows (256 .. 40960 columns, K 256 .. 19200, weight
-// tiles and, one in five, rows as they lie): half of either within 3 %. With the lines of takes_gemv 0.872 of the GEMM's time in all, 1798 calls more than 3 % slower than it, at most
-// 39 %; by this rule 0.867, 88, at most 23 % (the better one each time 0.856; of 3922 calls of 1..16 rows the GEMV is the slower one in 2). us, GEMM -> GEMV: 512 x 4992 at 45 rows 13.8 -> 18.4,
-// 1536 x 4480 at 38 14.6 -> 19.1, 4864 x 4224 at 40 18.7 -> 23.1, 1280 x 8832 at 35 18.5 -> 20.6 (not taken); 34816 x 5120 at 17 / 48 63 -> 37, 51, 40192 x 512 at 46 21.6 -> 15.0, 1536 x 1152 at 28 17.8 -> 11.2.
+// Whether a fused gate|up linear's rows go through the GEMV, by sk splits of K, and not through the GEMM that `plan` is of: up to 16 rows, and up to
+// 48 where an estimate of both
+// (us) has it ahead. The GEMV's: a start, a wavefront's k tiles (less each where a CU has two programs), the weights' way, and the splits' sums,
+// written and read. The GEMM's: its plan's and what that leaves out at so few rows; pieces of K cost less than it says. Fitted to 11766 calls of
+// 17..48 rows (256 .. 40960 columns, K 256 .. 19200, weight tiles and, one in five, rows as they lie): half of either within 3 %. With the lines of
+// takes_gemv 0.872 of the GEMM's time in all, 1798 calls more than 3 % slower than it, at most 39 %; by this rule 0.867, 88, at most 23 % (the better
+// one each time 0.856; of 3922 calls of 1..16 rows the GEMV is the slower one in 2). us, GEMM -> GEMV: 512 x 4992 at 45 rows 13.8 -> 18.4, 1536 x
+// 4480 at 38 14.6 -> 19.1, 4864 x 4224 at 40 18.7 -> 23.1, 1280 x 8832 at 35 18.5 -> 20.6 (not taken); 34816 x 5120 at 17 / 48 63 -> 37, 51, 40192 x
+// 512 at 46 21.6 -> 15.0, 1536 x 1152 at 28 17.8 -> 11.2.
 static bool swiglu_takes_gemv(const fe_fp4_linear *l, const fe_fp4_kernels *kern, uint32_t m, uint32_t sk, const FeGemmPlan &plan) {
     if (m > kGemvRows || l->n / kTile > kGemvCounters || !kern->gemv || kern->tile.force_tile || kern->gemm_sk >= 2) return false;
     if (m <= 16 || !kern->gemv_strips || kern->gemv_sk) return true;
@@ -560,14 +563,16 @@ int fe_fp4_linear_gemm(const fe_fp4_linear *l, const fe_fp4_kernels *kern, fe_st
 }
 
 // Whether the GEMV's programs each quantize all of the activations: few values, since a program waits for all of them before its first product. us, with the
-// quantizer's launch -> without: 1024 x 1024 at 1 / 8 rows 6.9 -> 3.8, 7.1 -> 4.1; 5120 x 5120 at 1 / 2 rows 8.7 -> 7.3, 8.9 -> 8.0; 17408 x 5120 at 1 / 2 15.8 -> 14.0,
-// 16.2 -> 14.5; 34816 x 5120 at 2 24.7 -> 23.7; 16384 x 2560 at 4 9.3 -> 8.3; 5120 x 8704 at 1 11.5 -> 10.0. Beyond 10240 values it turns: 34816 x 5120 at 3 rows
-// 25.2 -> 27.0, 16384 x 2560 at 6 10.2 -> 14.3 (one program a CU). Eight wavefronts quantize twice as many in that time: 5120 x 17408 at 1 row 17.2 -> 15.9, 4096 x 4096 at
-// 4 6.7 -> 5.8, 1024 x 5120 at 4 / 5 (25600 values) 6.7 -> 6.8, 7.1 -> 7.9. What it costs is a wavefront's turns (64 blocks each) times the rounds of programs, each of which
-// quantizes again: of 268 shapes (1024 .. 152064 columns, 1 to 8 rows), by values alone 0.934 of the time, 51 more than 2 % slower, at most 36 % (152064 x 1280 at 8 rows 35.7 -> 48.4,
-// 152064 x 5120 at 1 74.6 -> 82.3, 16384 x 1280 at 8 7.8 -> 8.6); with at most three turns, five times the rounds, 0.918, three more than 2 %, at most 4 % (1024 columns; the better
-// of both 0.916). Inputs that no cache holds or that the last call read: the same within 2 %. Up to 8 rows, what the LDS holds and 32 bits address. Not where the output or the
-// workspace lies in the activations' memory: programs that have finished would write over what others have yet to read.
+// quantizer's launch -> without: 1024 x 1024 at 1 / 8 rows 6.9 -> 3.8, 7.1 -> 4.1; 5120 x 5120 at 1 / 2 rows 8.7 -> 7.3, 8.9 -> 8.0; 17408 x 5120 at
+// 1 / 2 15.8 -> 14.0, 16.2 -> 14.5; 34816 x 5120 at 2 24.7 -> 23.7; 16384 x 2560 at 4 9.3 -> 8.3; 5120 x 8704 at 1 11.5 -> 10.0. Beyond 10240 values
+// it turns: 34816 x 5120 at 3 rows 25.2 -> 27.0, 16384 x 2560 at 6 10.2 -> 14.3 (one program a CU). Eight wavefronts quantize twice as many in that
+// time: 5120 x 17408 at 1 row 17.2 -> 15.9, 4096 x 4096 at 4 6.7 -> 5.8, 1024 x 5120 at 4 / 5 (25600 values) 6.7 -> 6.8, 7.1 -> 7.9. What it costs is
+// a wavefront's turns (64 blocks each) times the rounds of programs, each of which quantizes again: of 268 shapes (1024 .. 152064 columns, 1 to 8
+// rows), by values alone 0.934 of the time, 51 more than 2 % slower, at most 36 % (152064 x 1280 at 8 rows 35.7 -> 48.4, 152064 x 5120 at 1 74.6 ->
+// 82.3, 16384 x 1280 at 8 7.8 -> 8.6); with at most three turns, five times the rounds, 0.918, three more than 2 %, at most 4 % (1024 columns; the
+// better of both 0.916). Inputs that no cache holds or that the last call read: the same within 2 %. Up to 8 rows, what the LDS holds and 32 bits
+// address. Not where the output or the workspace lies in the activations' memory: programs that have finished would write over what others have yet
+// to read.
 static bool fp4_quants_itself(const fe_fp4_linear *l, const fe_fp4_kernels *kern, const fe_fp4_workspace *ws, fe_devptr_t y, uint32_t ldy, fe_devptr_t x,
                               uint32_t lda, uint32_t m) {
     if (!m || m > 8 || !takes_wide(l, kern, m) || (uint64_t)m * lda >= (1u << 30)) return false;

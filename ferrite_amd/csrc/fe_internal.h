@@ -178,9 +178,9 @@ struct FeGemmSchedule {
 // reduce launch and are 1..3 % faster: taken for a small weight operand, (c) below; (d) and (e) below are two more cases
 // of a small weight operand, runs over all tiles behind no whole round.
 // With decoded fp16 tiles or FP8 codes as the weight operand (32 KB a k tile) runs behind whole rounds lose 4..9 %.
-// (NVFP4 up to 2048 rows with more tiles than CUs asks with mode 0: fe_gemm_mode. Of what is said here about more tiles than CUs, the NVFP4 figures up to 2048 rows were taken
-// against a one-piece schedule without lower tiles and with rows that do not exist read again; the rules stand for NVFP4 over 2048 rows and for the trellis GEMM that decodes into LDS.)
-// Needs two partial slots a program and a zeroed counter a tile.
+// (NVFP4 up to 2048 rows with more tiles than CUs asks with mode 0: fe_gemm_mode. Of what is said here about more tiles than CUs, the NVFP4 figures
+// up to 2048 rows were taken against a one-piece schedule without lower tiles and with rows that do not exist read again; the rules stand for NVFP4
+// over 2048 rows and for the trellis GEMM that decodes into LDS.) Needs two partial slots a program and a zeroed counter a tile.
 constexpr uint32_t kFeXcds = 8;
 inline FeGemmSchedule fe_gemm_schedule(uint32_t tiles, uint32_t ktiles, uint32_t cus, fe_devptr_t part, size_t part_bytes,
                                        fe_devptr_t counters, size_t counters_len, uint32_t cap, int mode, bool small_b) {
@@ -294,9 +294,10 @@ struct FeGemmTileOptions {
 // tiles in more than one round take more than their rounds add up to (trellis: the programs that come second decode alone; 528 tiles 128 x 128 of
 // 32 k tiles 80 us where the rounds add up to 67).
 // short_k: how much of the small tiles' estimate a lower tile may take with more tiles than CUs and fewer than 24 k tiles (fe_gemm_plan).
-// high: us a k tile of tiles of 256, 224, 192, 160 rows, and how much more of it when all CUs are busy, for the choice among them (fe_gemm_height): fitted to 112
-// timings a form and height (128..1900 rows, 2048 x 4096 .. 17408 x 5120) without a fixed part, half of them within 5 % (FP8: to 60, half within 5 %, nine tenths within 11..15 %; 962 launches against the tree before its lower tiles'
-// loop of today, 647 of them with another tile: those 0.910 of the time, one more than 3 % slower, 1792 x 19072 at 1263 rows 69.0 -> 73.3; the others 0.985, 8704 x 5120 at 129 rows 20.5 -> 21.1).
+// high: us a k tile of tiles of 256, 224, 192, 160 rows, and how much more of it when all CUs are busy, for the choice among them (fe_gemm_height):
+// fitted to 112 timings a form and height (128..1900 rows, 2048 x 4096 .. 17408 x 5120) without a fixed part, half of them within 5 % (FP8: to 60,
+// half within 5 %, nine tenths within 11..15 %; 962 launches against the tree before its lower tiles' loop of today, 647 of them with another tile:
+// those 0.910 of the time, one more than 3 % slower, 1792 x 19072 at 1263 rows 69.0 -> 73.3; the others 0.985, 8704 x 5120 at 129 rows 20.5 -> 21.1).
 // f8: FP8 weights, for two lines of fe_gemm_plan.
 struct FeGemmCost {
     float ktile[3], full[3], fixed[3], shared, stream_k, again, high[4][2], short_k;
@@ -319,8 +320,8 @@ inline float fe_gemm_reduce_cost(uint32_t programs, uint32_t tile) {
     return 4.0f + (float)programs * (float)(kFeGemmTileM[tile] * kFeGemmTileN[tile]) * 8.0f / 5e6f;
 }
 
-// What a launch of tiles of one height (256, 224, 192, 160 rows: h 0..3) takes, for the choice among them: rounds of one program a CU, and the pieces' sums, which
-// travel twice.
+// What a launch of tiles of one height (256, 224, 192, 160 rows: h 0..3) takes, for the choice among them: rounds of one program a CU, and the
+// pieces' sums, which travel twice.
 inline float fe_gemm_height(const FeGemmCost &c, uint32_t h, const FeGemmSplit &g, uint32_t ktiles, uint32_t cus, uint32_t rows_a_tile) {
     auto rounds = [&](uint32_t programs, uint32_t k) {
         const uint32_t last = programs % cus;
@@ -331,9 +332,10 @@ inline float fe_gemm_height(const FeGemmCost &c, uint32_t h, const FeGemmSplit &
     return t;
 }
 
-// Stream-K of the forms that have lower tiles, up to 2048 rows: only with fewer tiles than CUs. Behind or over whole rounds, rows that do not exist, the reduce launch and
-// lower tiles cost the one-piece schedule less than the runs' meetings cost (NVFP4, us, stream-K -> one piece: 34816 x 5120 at 400 / 777 / 2048 rows 144 -> 130, 267 -> 242,
-// 531 -> 521; 17408 x 5120 at 777 / 1800 138 -> 130, 273 -> 257; 16384 x 4096 at 1500 182 -> 154; at most 2 % the other way: 12288 x 2048 at 1500 69.0 -> 70.6). With
+// Stream-K of the forms that have lower tiles, up to 2048 rows: only with fewer tiles than CUs. Behind or over whole rounds, rows that do not exist,
+// the reduce launch and lower tiles cost the one-piece schedule less than the runs' meetings cost (NVFP4, us, stream-K -> one piece: 34816 x 5120 at
+// 400 / 777 / 2048 rows 144 -> 130, 267 -> 242, 531 -> 521; 17408 x 5120 at 777 / 1800 138 -> 130, 273 -> 257; 16384 x 4096 at 1500 182 -> 154; at
+// most 2 % the other way: 12288 x 2048 at 1500 69.0 -> 70.6). With
 // fewer: 34816 x 5120 at 200 rows 94 against 102, 5120 x 17408 at 2048 265 against 277.
 inline int fe_gemm_mode(int mode, uint32_t m, uint32_t tiles256, uint32_t cus, const FeGemmTileOptions &opt) {
     return mode == 1 && opt.low && m <= 2048 && tiles256 > cus ? 0 : mode;
@@ -385,11 +387,12 @@ inline FeGemmPlan fe_gemm_plan(uint32_t m, uint32_t n, uint32_t ktiles, uint32_t
         if (g.cut())
             best += fe_gemm_cost(cost, 0, g.cut() * g.splits, (ktiles + g.splits - 1) / g.splits, cus) + fe_gemm_reduce_cost(g.cut() * g.splits, 0);
     }
-    // Lower tiles: as many row tiles of less waste, or another count of them that fills the rounds of the CUs better (rows that do not exist cost little power, but
-    // their time). By the ratio of the two estimates, which share most of their errors. Of 336 launches (8 layers, 14 row counts, NVFP4, FP8 and bf16) against 256 rows:
-    // 0.925, 0.93, 0.905 of the time (the best height each time: 0.92, 0.92, 0.90), four more than 2 % slower, at most 7 %. With the small tiles in the choice, 12 other layers
-    // of 144 launches a form against the rule without lower tiles: 0.93, 0.97, 0.93; 8 of 432 more than 3 % slower, at most 7 %. (With FP8's loop and heights, the reduce launches and the
-    // epilogues of before; FP8's figures since are at FeGemmCost.)
+    // Lower tiles: as many row tiles of less waste, or another count of them that fills the rounds of the CUs better (rows that do not exist cost
+    // little power, but their time). By the ratio of the two estimates, which share most of their errors. Of 336 launches (8 layers, 14 row counts,
+    // NVFP4, FP8 and bf16) against 256 rows: 0.925, 0.93, 0.905 of the time (the best height each time: 0.92, 0.92, 0.90), four more than 2 % slower,
+    // at most 7 %. With the small tiles in the choice, 12 other layers of 144 launches a form against the rule without lower tiles: 0.93, 0.97, 0.93;
+    // 8 of 432 more than 3 % slower, at most 7 %. (With FP8's loop and heights, the reduce launches and the epilogues of before; FP8's figures since
+    // are at FeGemmCost.)
     uint32_t pick = 0;
     float ratio = p.big.stream_k ? 0.9f : 0.97f;
     if (opt.low && m <= 2048) {
@@ -416,28 +419,33 @@ inline FeGemmPlan fe_gemm_plan(uint32_t m, uint32_t n, uint32_t ktiles, uint32_t
         }
     }
     if (!pick) return p;
-    // In the place of a small tile a lower one is taken only with at least 12 k tiles and half of the CUs: the heights' estimate has no fixed part and was fitted on launches
-    // that fill the chip. Of 1499 launches (128 .. 40000 columns, K 256 .. 20000, 65 .. 2048 rows; NVFP4, its SwiGLU front, FP8, bf16) against the rule without lower tiles:
-    // with them wherever the estimate says so 68 more than 3 % slower (5248 x 256 at 636 rows 9.2 -> 13.1 us, 7168 x 256 SwiGLU at 140 13.4 -> 25.6, 256 x 1536 bf16 at
-    // 210 7.8 -> 10.3, 11136 x 256 FP8 at 315 9.1 -> 11.6) and 0.986 / 0.983 / 0.998 / 0.993 of the time in all; so 11, at most 6 %, and 0.980 / 0.979 / 0.991 / 0.989. Of 52360 launches,
-    // deep narrow and wide shallow ones among them, 807 were more than 3 % slower (bf16 1792 x 16384 at 864 rows 56.8 -> 89.7, 768 x 15104 at 1303
-    // 41.9 -> 52.6; at most 1.8 times); with the lines below 139 (41 of them bf16 in the
-    // place of 256 rows, at most 1.5 times: 35 and 49 tiles cut seven and five ways), 0.957 / 0.959 / 0.986 / 0.960 / 0.964 of the time (bf16, its SwiGLU front, FP8, NVFP4, its front; the best each time 0.949
-    // / 0.950 / 0.982 / 0.953 / 0.952). All of these with FP8's loop and heights, the reduce launches and the epilogues of before, and FP8 with a margin of 0.9 for short K.
+    // In the place of a small tile a lower one is taken only with at least 12 k tiles and half of the CUs: the heights' estimate has no fixed part
+    // and was fitted on launches that fill the chip. Of 1499 launches (128 .. 40000 columns, K 256 .. 20000, 65 .. 2048 rows; NVFP4, its SwiGLU
+    // front, FP8, bf16) against the rule without lower tiles: with them wherever the estimate says so 68 more than 3 % slower (5248 x 256 at 636 rows
+    // 9.2 -> 13.1 us, 7168 x 256 SwiGLU at 140 13.4 -> 25.6, 256 x 1536 bf16 at 210 7.8 -> 10.3, 11136 x 256 FP8 at 315 9.1 -> 11.6) and 0.986 /
+    // 0.983 / 0.998 / 0.993 of the time in all; so 11, at most 6 %, and 0.980 / 0.979 / 0.991 / 0.989. Of 52360 launches, deep narrow and wide
+    // shallow ones among them, 807 were more than 3 % slower (bf16 1792 x 16384 at 864 rows 56.8 -> 89.7, 768 x 15104 at 1303 41.9 -> 52.6; at most
+    // 1.8 times); with the lines below 139 (41 of them bf16 in the place of 256 rows, at most 1.5 times: 35 and 49 tiles cut seven and five ways),
+    // 0.957 / 0.959 / 0.986 / 0.960 / 0.964 of the time (bf16, its SwiGLU front, FP8, NVFP4, its front; the best each time 0.949 / 0.950 / 0.982 /
+    // 0.953 / 0.952). All of these with FP8's loop and heights, the reduce launches and the epilogues of before, and FP8 with a margin of 0.9 for
+    // short K.
     const FeGemmSchedule lower = low(pick);
     if (p.tile) {
-        // (Of an NVFP4 SwiGLU front with 16..23 k tiles, which small tiles may cut in two only, lower ones also with fewer programs: 45 launches of up to 16 tiles 0.82 of the small tiles' time;
-        // with 24..31, three pieces, 1.15, and of plain linears of 20..23 1.14.)
+        // (Of an NVFP4 SwiGLU front with 16..23 k tiles, which small tiles may cut in two only, lower ones also with fewer programs: 45 launches of
+        // up to 16 tiles 0.82 of the small tiles' time; with 24..31, three pieces, 1.15, and of plain linears of 20..23 1.14.)
         if (ktiles < 12 || (2 * lower.split.programs() < cus && !(opt.nvfp4_front && ktiles >= 16 && ktiles < 24))) return p;
-        // Dense weights (bf16, FP8) in fewer lower tiles than a quarter of the CUs: deep narrow linears, which small tiles cut finer than eight pieces of a lower one (bf16:
-        // 826 launches 1.16 times the small tiles' time, from there on 0.90). More lower tiles than CUs and short K: rounds of them want a clearer gain (48 of FP8 1.01, bf16 past 0.9 level;
-        // not so from 24 k tiles on: 5120 x 17408 at 559 rows, NVFP4 block 290 us with them, 305 without).
+        // Dense weights (bf16, FP8) in fewer lower tiles than a quarter of the CUs: deep narrow linears, which small tiles cut finer than eight
+        // pieces of a lower one (bf16: 826 launches 1.16 times the small tiles' time, from there on 0.90). More lower tiles than CUs and short K:
+        // rounds of them want a clearer gain (48 of FP8 1.01, bf16 past 0.9 level; not so from 24 k tiles on: 5120 x 17408 at 559 rows, NVFP4 block
+        // 290 us with them, 305 without).
         const uint32_t tiles = tiles_of(pick);
         if (!small_b && 4 * tiles < cus) return p;
-        // FP8, whose heights leave out what a cut and short K cost: not where every lower tile is cut, unless one is as high as the rows (small tiles, us -> lower ones: 5120 x 17408 at
-        // 1100 / 1216 rows 88.6 -> 91.7, 92.7 -> 103.6, 5120 x 6144 at 512 25.0 -> 28.5, 2048 x 8192 at 1536 32.9 -> 35.4; 70 launches 0.95 to 1.14 of the small tiles' time; one row tile:
-        // 18944 x 8448 at 155 53.5 -> 45.9). A few cut tiles behind a whole round are ahead (34816 x 5120 at 250 82.8 -> 66.5). And the clearer gain for short K at any count: with fewer
-        // tiles than CUs 8192 x 2048 at 1024 rows takes 19.7 -> 20.7 where the ratio is 0.99, at 1100 rows 23.7 -> 20.9 where it is 0.46 (ten launches between 0.46 and 0.77: 0.71 to 0.96).
+        // FP8, whose heights leave out what a cut and short K cost: not where every lower tile is cut, unless one is as high as the rows (small
+        // tiles, us -> lower ones: 5120 x 17408 at 1100 / 1216 rows 88.6 -> 91.7, 92.7 -> 103.6, 5120 x 6144 at 512 25.0 -> 28.5, 2048 x 8192 at 1536
+        // 32.9 -> 35.4; 70 launches 0.95 to 1.14 of the small tiles' time; one row tile: 18944 x 8448 at 155 53.5 -> 45.9). A few cut tiles behind a
+        // whole round are ahead (34816 x 5120 at 250 82.8 -> 66.5). And the clearer gain for short K at any count: with fewer tiles than CUs 8192 x
+        // 2048 at 1024 rows takes 19.7 -> 20.7 where the ratio is 0.99, at 1100 rows 23.7 -> 20.9 where it is 0.46 (ten launches between 0.46 and
+        // 0.77: 0.71 to 0.96).
         if (cost.f8 && !lower.split.full && m > kFeGemmTileM[pick]) return p;
         const float margin = ktiles < 24 && (tiles > cus || cost.f8) ? cost.short_k : small_b ? 1.06f : 1.0f;  // (bf16 and FP8: what a lower tile gained is part of that margin)
         if (margin * p.us < whole * ratio) return p;
@@ -542,9 +550,10 @@ int fe_gemm_launch(const FeGemmPlan &p, Gemm gemm, Reduce reduce) {
 }
 
 // ---- gate, up and SwiGLU of decode rows over plain bf16 weights (fe_bf16.cpp) ---------------------------------------------------
-// Whether fe_bf16_gemv_swiglu does what two fe_bf16_linear_forward into big ([m][inter] each) and fe_route_silu_mul into act do: all rows go through the GEMV in one pass,
-// the operands are what those take, and act lies apart from what other programs still read. (Two launches less: see gemv_bf16_body for both sides.) over_gemm: the call would
-// otherwise take the GEMM with SwiGLU in its epilogue over interleaved weights, which is ahead of it at some row counts where gate, up and SwiGLU in three launches are not.
+// Whether fe_bf16_gemv_swiglu does what two fe_bf16_linear_forward into big ([m][inter] each) and fe_route_silu_mul into act do: all rows go through
+// the GEMV in one pass, the operands are what those take, and act lies apart from what other programs still read. (Two launches less: see
+// gemv_bf16_body for both sides.) over_gemm: the call would otherwise take the GEMM with SwiGLU in its epilogue over interleaved weights, which is
+// ahead of it at some row counts where gate, up and SwiGLU in three launches are not.
 struct fe_bf16_kernels;
 bool fe_bf16_gemv_swiglu_takes(const fe_bf16_kernels *kern, fe_devptr_t big, fe_devptr_t act, fe_devptr_t x, fe_devptr_t gate, fe_devptr_t up, uint32_t m, uint32_t inter,
                                uint32_t k, uint32_t dec, bool over_gemm);
@@ -557,11 +566,12 @@ constexpr bool gemv_form(uint32_t xo, uint32_t co) { return 12 * (co + xo) <= 16
 constexpr uint32_t gemv_row_form(uint32_t m) { return m <= 8 ? 0 : (m + 15) / 16; }
 // Bf16Gemv<XO, CO>::LDS of k_bf16.hip, and what Fp8Gemv of k_fp4.hip takes
 inline uint32_t gemv_lds(uint32_t xo, uint32_t co) { return 4 * std::max(3u, std::min(20 / (co + xo), 8u)) * (co + xo) * 1024; }
-// The columns that each program of a form of `most` columns takes (`whole`: those): as even as whole rounds of one program a CU allow, in steps of `step`; rows of a load
-// past them repeat the last one, which a cache holds. 5120 columns are 256 programs of 20 instead of 214 of 24, 17408 of 68 instead of 242 of 72. us, bf16 blocks (gate, up, down)
-// of 5120 x 17408 at 8 / 12 / 48 rows 83.9 -> 82.5, 87.5 -> 85.7, 142 -> 135, of 5120 x 8704 at 12 49.7 -> 47.1, of 1536 x 5120 at 12 15.2 -> 14.2; FP8 5120 x 17408 at 16
-// rows 17.3 -> 16.2, 5120 x 5120 7.6 -> 7.1. One and two rows, which are bound by the weights' way alone, gain nothing (bf16 3072 x 8192 27.7 -> 28.1: whole octets there), nor does NVFP4,
-// whose octets are pieces of 256 bytes (5120 x 17408 at 4 rows 14.6 -> 14.9: not done there).
+// The columns that each program of a form of `most` columns takes (`whole`: those): as even as whole rounds of one program a CU allow, in steps of
+// `step`; rows of a load past them repeat the last one, which a cache holds. 5120 columns are 256 programs of 20 instead of 214 of 24, 17408 of 68
+// instead of 242 of 72. us, bf16 blocks (gate, up, down) of 5120 x 17408 at 8 / 12 / 48 rows 83.9 -> 82.5, 87.5 -> 85.7, 142 -> 135, of 5120 x 8704
+// at 12 49.7 -> 47.1, of 1536 x 5120 at 12 15.2 -> 14.2; FP8 5120 x 17408 at 16 rows 17.3 -> 16.2, 5120 x 5120 7.6 -> 7.1. One and two rows, which
+// are bound by the weights' way alone, gain nothing (bf16 3072 x 8192 27.7 -> 28.1: whole octets there), nor does NVFP4, whose octets are pieces of
+// 256 bytes (5120 x 17408 at 4 rows 14.6 -> 14.9: not done there).
 inline uint32_t gemv_even(uint32_t n, uint32_t most, uint32_t cus, uint32_t step, bool whole) {
     const uint32_t programs = (n + most - 1) / most;
     if (whole || 2 * programs <= cus) return most;
@@ -596,10 +606,11 @@ inline uint32_t gemv_cols(uint32_t m, uint32_t n, uint32_t k, uint32_t xo, uint3
     return best;
 }
 
-// Whether a GEMV over programs of columns is ahead of the GEMM that would run in its place, by an estimate of both (us). The GEMV's: a start, rounds of programs, the weights'
-// way from HBM, the activations' way from L2 once a program (the CU with the most; x: the form's rows, x_row: those that exist) and the outputs. The GEMM's: its plan's estimate and what that leaves out at so few rows, the
-// weights' way, of bytes past what the chip's last cache holds once more (far: us a byte), and the outputs; pieces of K cost less than it says. margin: on what the GEMM takes. Up to `always` rows
-// the GEMV in any case. beside: decode rows, which a GEMV of their own would take beside the GEMM.
+// Whether a GEMV over programs of columns is ahead of the GEMM that would run in its place, by an estimate of both (us). The GEMV's: a start, rounds
+// of programs, the weights' way from HBM, the activations' way from L2 once a program (the CU with the most; x: the form's rows, x_row: those that
+// exist) and the outputs. The GEMM's: its plan's estimate and what that leaves out at so few rows, the weights' way, of bytes past what the chip's
+// last cache holds once more (far: us a byte), and the outputs; pieces of K cost less than it says. margin: on what the GEMM takes. Up to `always`
+// rows the GEMV in any case. beside: decode rows, which a GEMV of their own would take beside the GEMM.
 struct FeGemvLine {
     uint32_t always;
     float start, round, w, x, x_row, out, gemm_start, gemm_us, gemm_w, gemm_cut, gemm_pieces, gemm_far, gemm_out, margin;
@@ -618,18 +629,23 @@ inline bool fe_gemv_ahead(const FeGemvLine &c, uint32_t m, uint32_t n, uint32_t 
                     (pieces > 1 ? c.gemm_cut : 0.0f) - c.gemm_pieces * (float)pieces * (float)n;
     return fe_gemv_us(c, m, n, k, steps, cus, even_step) <= c.margin * t + (beside ? fe_gemv_us(c, beside, n, k, steps, cus, even_step) : 0.0f);
 }
-// FP8 (steps of 128 codes), up to 64 rows. Fitted to 17236 calls of 9..64 rows (128 .. 153600 columns, K 128 .. 76800, half of them past 40960 columns or K 20480), half of either
-// estimate within 5 %. Of the GEMM's time in all 0.824, 180 calls more than 3 % slower than it, at most 21 %, 30 of them among the 11408 of up to 40960 columns and K 20480, at most 15 % (the
-// better one each time 0.818). Fitted to those alone the rule took 0.829, 650 calls slower, at most 41 % (3328 x 49664 at 27 rows 32.7 -> 42.3 us, 46336 x 5376 at 28 39.5 -> 47.1); by K alone (64 rows, 40
-// where K is past 14336) wide linears of short K took up to 62 % more. us, GEMM -> GEMV at 1 / 17 / 32 / 64 rows: 17408 x 5120 24.4 -> 15.1, 25.2 -> 16.1, 25.8 -> 17.4, 27.7 -> 27.1; 5120 x 5120 12.0 -> 6.1,
-// 12.5 -> 8.3, 12.7 -> 8.5, 13.3 -> 11.0; 1024 x 2816 9.7 -> 3.9, 10.2 -> 3.8, 10.2 -> 4.2, 10.7 -> 5.7; not taken: 38784 x 384 at 56 10.4 -> 16.5, 28672 x 640 at 60 10.6 -> 15.4, 11136 x 13952 at 61 40 -> 49.
+// FP8 (steps of 128 codes), up to 64 rows. Fitted to 17236 calls of 9..64 rows (128 .. 153600 columns, K 128 .. 76800, half of them past 40960
+// columns or K 20480), half of either estimate within 5 %. Of the GEMM's time in all 0.824, 180 calls more than 3 % slower than it, at most 21 %, 30
+// of them among the 11408 of up to 40960 columns and K 20480, at most 15 % (the better one each time 0.818). Fitted to those alone the rule took
+// 0.829, 650 calls slower, at most 41 % (3328 x 49664 at 27 rows 32.7 -> 42.3 us, 46336 x 5376 at 28 39.5 -> 47.1); by K alone (64 rows, 40 where K
+// is past 14336) wide linears of short K took up to 62 % more. us, GEMM -> GEMV at 1 / 17 / 32 / 64 rows: 17408 x 5120 24.4 -> 15.1, 25.2 -> 16.1,
+// 25.8 -> 17.4, 27.7 -> 27.1; 5120 x 5120 12.0 -> 6.1, 12.5 -> 8.3, 12.7 -> 8.5, 13.3 -> 11.0; 1024 x 2816 9.7 -> 3.9, 10.2 -> 3.8, 10.2 -> 4.2, 10.7
+// -> 5.7; not taken: 38784 x 384 at 56 10.4 -> 16.5, 28672 x 640 at 60 10.6 -> 15.4, 11136 x 13952 at 61 40 -> 49.
 constexpr FeGemvLine kFeGemvFp8{8, 3.47f, 0.835f, 14.4e-6f, 1.544e-3f, 0.0f, 2.39e-6f, 5.01f, 0.768f, 0.68e-6f, 1.64f, -17.5e-6f, 0.0f, 1.11e-6f, 0.95f};
-// bf16 (steps of 64), up to 32 rows that are no decode rows. Fitted to 21244 linears of 17..32 rows (64 .. 96000 columns, K 256 .. 19456), half of either estimate within 5 %. By this rule
-// 0.832 of the GEMM's time in all, 194 more than 3 % slower than it, at most 25 % (the better one each time 0.824); with lines by rows times K alone (350000 up to 24 rows, 180000 up to 32) 0.862 of
-// 18642, 2207 slower, at most 2.1 times. us, GEMM -> GEMV at 17 / 24 / 32 rows: 17408 x 5120 40 -> 31, 31, 32; 34816 x 5120 77 -> 58, 79 -> 60, 81 -> 62; 5120 x 5120 17 -> 13, 15, 16; 1024 x 2816 8.7 -> 5.4,
-// 5.7, 6.1; not taken: 61728 x 256 at 31 7.6 -> 15.8, 55304 x 256 at 27 7.2 -> 14.5. From 33 rows on (three groups of 16) the GEMM is ahead wherever K is 5120 and more.
+// bf16 (steps of 64), up to 32 rows that are no decode rows. Fitted to 21244 linears of 17..32 rows (64 .. 96000 columns, K 256 .. 19456), half of
+// either estimate within 5 %. By this rule 0.832 of the GEMM's time in all, 194 more than 3 % slower than it, at most 25 % (the better one each time
+// 0.824); with lines by rows times K alone (350000 up to 24 rows, 180000 up to 32) 0.862 of 18642, 2207 slower, at most 2.1 times. us, GEMM -> GEMV
+// at 17 / 24 / 32 rows: 17408 x 5120 40 -> 31, 31, 32; 34816 x 5120 77 -> 58, 79 -> 60, 81 -> 62; 5120 x 5120 17 -> 13, 15, 16; 1024 x 2816 8.7 ->
+// 5.4, 5.7, 6.1; not taken: 61728 x 256 at 31 7.6 -> 15.8, 55304 x 256 at 27 7.2 -> 14.5. From 33 rows on (three groups of 16) the GEMM is ahead
+// wherever K is 5120 and more.
 constexpr FeGemvLine kFeGemvBf16{16, 0.91f, 1.236f, 15.0e-6f, 0.962e-3f, 0.894e-3f, 1.63e-6f, 3.05f, 0.681f, 4.69e-6f, 1.084f, -5.1e-6f, 0.0987e-6f, 0.0f, 0.97f};
-// bf16 gate and up (n each) in one launch against the GEMM with SwiGLU over their interleaved weights (its plan's): of 10529 calls 0.906 of the GEMM's time in all, 179 more than 3 %
-// slower, at most 28 % (the better one each time 0.901); by rows times K and inter 0.942 of 2284, 410 slower, at most 2.4 times. us, GEMM -> GEMV: 8512 x 3584 at 21 rows 29.2 -> 21.9, 1280 x 2560 at
-// 20 9.5 -> 7.0; not taken: 28480 x 256 at 22 7.8 -> 18.8, 15168 x 256 at 21 5.6 -> 9.8, 320 x 10752 at 20 12.9 -> 22.4.
+// bf16 gate and up (n each) in one launch against the GEMM with SwiGLU over their interleaved weights (its plan's): of 10529 calls 0.906 of the
+// GEMM's time in all, 179 more than 3 % slower, at most 28 % (the better one each time 0.901); by rows times K and inter 0.942 of 2284, 410 slower,
+// at most 2.4 times. us, GEMM -> GEMV: 8512 x 3584 at 21 rows 29.2 -> 21.9, 1280 x 2560 at 20 9.5 -> 7.0; not taken: 28480 x 256 at 22 7.8 -> 18.8,
+// 15168 x 256 at 21 5.6 -> 9.8, 320 x 10752 at 20 12.9 -> 22.4.
 constexpr FeGemvLine kFeGemvBf16Pair{16, 2.19f, 0.371f, 28.7e-6f, 2.041e-3f, 1.674e-3f, 9.58e-6f, 3.55f, 0.689f, 11.0e-6f, 1.264f, 155e-6f, 0.0639e-6f, 5.86e-6f, 0.97f};

@@ -43,10 +43,11 @@ __device__ __forceinline__ uint32_t decode2_mul1(uint32_t s0, uint32_t s1) {
 // tile r & 1, the BITS words of fragment lanes 4q .. 4q + 3 (q = r >> 1) plus the word before them, which is all its 32
 // states need. (The tiles alternate over the lanes, so that the word before, the last one of lane q - 1 of the same tile, is two lanes away
 // in the 16, also at q = 0: lane_prev_word, one instruction where tiles in the two halves of the 16 lanes take three. The kernels whose words come
-// through LDS keep tile r >> 3, q = r & 7: alternating they read them 2 % slower, prompts of 203 rows.) Those states are rows n = q and n = q + 8 of the tile over all 16 k, so after decoding the lane holds, for
-// each of the two, the 16 values as two 8-value MFMA operands (k 0..7 and k 8..15) in k order. v_mfma_f32_16x16x32_f16
-// then sums over the 4 k steps: A = decoded weights (row r), B = 16 rotated input rows (column = input row), and the
-// accumulators of lane L are rows 4 g .. 4 g + 3 of A (columns q = 2 g, 2 g + 1 of both tiles), input row r; lane_cols makes four neighbouring columns of them.
+// through LDS keep tile r >> 3, q = r & 7: alternating they read them 2 % slower, prompts of 203 rows.) Those states are rows n = q and n = q + 8 of
+// the tile over all 16 k, so after decoding the lane holds, for each of the two, the 16 values as two 8-value MFMA operands (k 0..7 and k 8..15) in k
+// order. v_mfma_f32_16x16x32_f16 then sums over the 4 k steps: A = decoded weights (row r), B = 16 rotated input rows (column = input row), and the
+// accumulators of lane L are rows 4 g .. 4 g + 3 of A (columns q = 2 g, 2 g + 1 of both tiles), input row r; lane_cols makes four neighbouring
+// columns of them.
 
 template <int BITS>
 struct LaneWords {
@@ -218,7 +219,8 @@ __device__ __forceinline__ f32x4 row_scales(const uint16_t* svh, uint32_t col) {
                    f16_bits_to_f32(s[1] >> 16)};
 }
 // (Moves that leave no lane out and read no old value: with one, each cost a move of zero in front, five instructions a step instead of three or one.)
-// The last word of the lane two before, around the 16 lanes of a DPP row: the word before the lane's run where the two tiles of a k step alternate over the lanes.
+// The last word of the lane two before, around the 16 lanes of a DPP row: the word before the lane's run where the two tiles of a k step alternate
+// over the lanes.
 __device__ __forceinline__ uint32_t lane_prev_word(uint32_t last) { return (uint32_t)__builtin_amdgcn_mov_dpp((int)last, 0x122, 0xf, 0xf, true); }
 // The same where lanes 0..7 have the one tile and lanes 8..15 the other: lane i takes lane i - 1 (row_shr:1) or, at q = 0, lane i + 7 (row_ror:9).
 __device__ __forceinline__ uint32_t lane_prev_word_halves(uint32_t last) {
@@ -226,8 +228,8 @@ __device__ __forceinline__ uint32_t lane_prev_word_halves(uint32_t last) {
     const uint32_t ror = (uint32_t)__builtin_amdgcn_mov_dpp((int)last, 0x129, 0xf, 0xf, true);
     return (threadIdx.x & 7) ? shr : ror;
 }
-// A lane's accumulators (rows 4 g .. 4 g + 3 of A: columns 2 g, 2 g + 1 of tiles 0 and 1, the tiles alternating) as four neighbouring columns: 16 (g & 1) + 4 (g >> 1) .. + 3 of
-// the wavefront's 32 (+ 8 h). Lanes of even g give their tile 1 to the lanes 16 further on for those lanes' tile 0.
+// A lane's accumulators (rows 4 g .. 4 g + 3 of A: columns 2 g, 2 g + 1 of tiles 0 and 1, the tiles alternating) as four neighbouring columns: 16 (g
+// & 1) + 4 (g >> 1) .. + 3 of the wavefront's 32 (+ 8 h). Lanes of even g give their tile 1 to the lanes 16 further on for those lanes' tile 0.
 __device__ __forceinline__ f32x4 lane_cols(f32x4 a) {
     typedef uint32_t pair_t __attribute__((ext_vector_type(2)));
     const pair_t lo = __builtin_bit_cast(pair_t, __builtin_amdgcn_permlane16_swap(__float_as_uint(a[0]), __float_as_uint(a[1]), false, false));

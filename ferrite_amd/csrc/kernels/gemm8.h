@@ -81,10 +81,10 @@ __device__ __forceinline__ u32x4 g8_rsrc(const void* p, uint32_t bytes) {
 __device__ __forceinline__ uint32_t g8_lds_addr(const void* p) {
     return (uint32_t)(uintptr_t)(const __attribute__((address_space(3))) void*)p;
 }
-// Byte offset of row `row` of an operand of m rows of `pitch` bytes. Rows past m lie out of the resource's range and read zero: what they would multiply is never
-// stored, and zeros take less of the board's power, which is what bounds the loop. (Operands of 2 GB and more, whose range such an offset could meet: row m - 1 again.)
-// ZERO false: row m - 1 again in any case (the stream-K forms, which meet few such rows: with the other offsets their loops of 256 registers are 1 % slower). at: byte
-// of the lane's piece in the row.
+// Byte offset of row `row` of an operand of m rows of `pitch` bytes. Rows past m lie out of the resource's range and read zero: what they would
+// multiply is never stored, and zeros take less of the board's power, which is what bounds the loop. (Operands of 2 GB and more, whose range such an
+// offset could meet: row m - 1 again.) ZERO false: row m - 1 again in any case (the stream-K forms, which meet few such rows: with the other offsets
+// their loops of 256 registers are 1 % slower). at: byte of the lane's piece in the row.
 template <bool ZERO>
 __device__ __forceinline__ uint32_t g8_row(uint32_t row, uint32_t m, uint32_t pitch, uint32_t at) {
     const uint32_t off = (row < m ? row : m - 1) * pitch + at;
@@ -251,8 +251,9 @@ __device__ __forceinline__ void g8_mainloop(const void* a, uint32_t lda, uint32_
 // Hands the wavefront's accumulators out row by row: 16 rows at a time pass through the wavefront's own LDS slab so that
 // LPR = 4 TN consecutive lanes hold the wavefront's 16 TN columns of one row, 4 a lane. U passes of 64 / LPR rows are in
 // flight together: transform(v[U][4], lane in row) works on all of them at once (no branches), then
-// store(row in 0 .. 16 TM - 1, lane in row, v[4], what ahead(row, lane in row) returned) is called for each. ahead: what store needs of memory, asked for 16 rows at a
-// time in front of the first of them: behind a store the next load waits for it (NVFP4 stream-K, 2048 rows of 5120 x 17408 with a residual 310 -> 300 us, FP8 185 -> 177.5). No workgroup barrier: a slab belongs to its wavefront.
+// store(row in 0 .. 16 TM - 1, lane in row, v[4], what ahead(row, lane in row) returned) is called for each. ahead: what store needs of memory, asked
+// for 16 rows at a time in front of the first of them: behind a store the next load waits for it (NVFP4 stream-K, 2048 rows of 5120 x 17408 with a
+// residual 310 -> 300 us, FP8 185 -> 177.5). No workgroup barrier: a slab belongs to its wavefront.
 template <class T, class Transform, class Ahead, class Store>
 __device__ __forceinline__ void g8_epilogue(f32x4 (&acc)[T::TM][T::TN], unsigned char* lds, Transform transform, Ahead ahead, Store store) {
     constexpr int LPR = 4 * T::TN, RP = 64 / LPR, PITCH = 16 * T::TN + 4, U = 16 / RP < 4 ? 16 / RP : 4, PASSES = 16 / RP;
@@ -277,8 +278,9 @@ __device__ __forceinline__ void g8_epilogue(f32x4 (&acc)[T::TM][T::TN], unsigned
                 v[u][0] = t[0], v[u][1] = t[1], v[u][2] = t[2], v[u][3] = t[3];
             }
             transform(v, lc);
-            // All of them have arrived from here on, also those of rows that are not stored: a load left in flight would have the next segment of a stream-K form wait for
-            // everything at its start, its own first k tiles too (FP8, 2048 rows of 5120 x 17408 without a residual 169 -> 172.5 us).
+            // All of them have arrived from here on, also those of rows that are not stored: a load left in flight would have the next segment of a
+            // stream-K form wait for everything at its start, its own first k tiles too (FP8, 2048 rows of 5120 x 17408 without a residual 169 ->
+            // 172.5 us).
             if constexpr (!std::is_empty<Old>::value) {
 #pragma unroll
                 for (int u = 0; u < U; u++) asm volatile("" : "+v"(old[q0 + u]));
@@ -305,12 +307,13 @@ __device__ __forceinline__ void g8_swap32(uint32_t& a, uint32_t& b) {
 }
 typedef uint32_t u32x4_a8 __attribute__((ext_vector_type(4), aligned(8)));
 
-// The wavefront's accumulators as bf16 rows added to a residual: c = bf16(bf16(sum) + res), row stride ldc, both pointers at its first row and column; pack(sums, column tile)
-// -> two words of bf16. A lane holds 4 columns of a row in every column tile and trades the half of two tiles with the lane 16 away: 8 neighbouring columns a lane, without
-// LDS. rows, cols: those that exist from there on (cols a multiple of 8). What a residual costs is the trip to memory: asked for where it is added, row piece by row piece, each
-// load waits behind the store before it, 10 us a launch. Asked for 16 rows ahead, us, launches without / with one before -> now: bf16, 2048 rows of 8192 x 256 15.0 / 25.3 ->
-// 14.5 / 19.8, of 8192 x 4096 95 / 105 -> 95 / 99.5; FP8, 1000 rows of 5120 x 5120 34.2 / 40.9 -> 33.9 / 34.4, 512 of 17408 x 5120 55 / 65 -> 55 / 56; NVFP4, 2048 of 8192 x 512
-// 23.6 / 33.1 -> 23.4 / 27.5. Through the slab (g8_epilogue, asked for ahead as well) the first takes 21.8; without a residual the slab's whole lines are ahead (14.5 against 15.2).
+// The wavefront's accumulators as bf16 rows added to a residual: c = bf16(bf16(sum) + res), row stride ldc, both pointers at its first row and
+// column; pack(sums, column tile) -> two words of bf16. A lane holds 4 columns of a row in every column tile and trades the half of two tiles with
+// the lane 16 away: 8 neighbouring columns a lane, without LDS. rows, cols: those that exist from there on (cols a multiple of 8). What a residual costs is the trip to memory: asked
+// for where it is added, row piece by row piece, each load waits behind the store before it, 10 us a launch. Asked for 16 rows ahead, us, launches
+// without / with one before -> now: bf16, 2048 rows of 8192 x 256 15.0 / 25.3 -> 14.5 / 19.8, of 8192 x 4096 95 / 105 -> 95 / 99.5; FP8, 1000 rows of
+// 5120 x 5120 34.2 / 40.9 -> 33.9 / 34.4, 512 of 17408 x 5120 55 / 65 -> 55 / 56; NVFP4, 2048 of 8192 x 512 23.6 / 33.1 -> 23.4 / 27.5. Through the
+// slab (g8_epilogue, asked for ahead as well) the first takes 21.8; without a residual the slab's whole lines are ahead (14.5 against 15.2).
 template <class T, class Pack>
 __device__ __forceinline__ void g8_add_bf16(f32x4 (&acc)[T::TM][T::TN], uint16_t* c, const uint16_t* res, uint32_t ldc, uint32_t rows, uint32_t cols, Pack pack) {
     constexpr int TM = T::TM, TN = T::TN, P = TN / 2;
@@ -363,13 +366,14 @@ __device__ __forceinline__ void g8_store_partial(f32x4 (&acc)[T::TM][T::TN], flo
 }
 
 // Body of a reduce kernel: grid = cut tiles * (BM / 16) * (BN / 128), 512 threads for 16 rows x 128 columns. A wavefront sums the `splits` slots of 16 of
-// the columns as g8_store_partial left them, 1 KB a slot, in split order; the sums change hands through LDS, and each half wavefront passes one row, 4 columns a
-// lane, to fn(row, first column of the block, l32, v[4], ahead(row, first column, l32)); blocks outside n are left out, rows are not. `ahead` reads what fn
-// needs besides the sums.
-// What it costs is trips to memory, not bytes: so every load of a workgroup is asked for before the first is waited for (up to eight slots, and what `ahead` reads).
-// Tiles of 128 x 128: 8 rows and 256 threads a workgroup, a half wavefront reads its row's pieces, the first slot, then four, two, one. Their launches are small (64 tiles for 215
-// rows of 4096 columns), and more and smaller workgroups are ahead there (all slots at once are not: 5120 x 5120 at 300 rows 22.1 -> 23.5): us, GEMM and reduce, 16 -> 8 rows: FP8 4096 x 4096 at 130 / 215 rows 16.7 / 18.1 -> 14.9 / 15.7, 2048 x 8192 at 130 17.0 -> 14.2,
-// 1024 x 5120 at 512 15.4 -> 13.8, NVFP4 4096 x 4096 at 215 21.9 -> 19.7; bf16 level (1024 x 5120 at 512 17.4 -> 18.5).
+// the columns as g8_store_partial left them, 1 KB a slot, in split order; the sums change hands through LDS, and each half wavefront passes one row,
+// 4 columns a lane, to fn(row, first column of the block, l32, v[4], ahead(row, first column, l32)); blocks outside n are left out, rows are not.
+// `ahead` reads what fn needs besides the sums. What it costs is trips to memory, not bytes: so every load of a workgroup is asked for before the
+// first is waited for (up to eight slots, and what `ahead` reads). Tiles of 128 x 128: 8 rows and 256 threads a workgroup, a half wavefront reads its
+// row's pieces, the first slot, then four, two, one. Their launches are small (64 tiles for 215 rows of 4096 columns), and more and smaller
+// workgroups are ahead there (all slots at once are not: 5120 x 5120 at 300 rows 22.1 -> 23.5): us, GEMM and reduce, 16 -> 8 rows: FP8 4096 x 4096 at
+// 130 / 215 rows 16.7 / 18.1 -> 14.9 / 15.7, 2048 x 8192 at 130 17.0 -> 14.2, 1024 x 5120 at 512 15.4 -> 13.8, NVFP4 4096 x 4096 at 215 21.9 -> 19.7;
+// bf16 level (1024 x 5120 at 512 17.4 -> 18.5).
 template <class T, class Ahead, class RowFn>
 __device__ __forceinline__ void g8_reduce_rows(const float* __restrict__ part, uint32_t m, uint32_t n, uint32_t group, uint32_t first,
                                                uint32_t splits, Ahead ahead, RowFn fn) {
@@ -681,9 +685,10 @@ __device__ __forceinline__ void g8_mainloop_decode(const _Float16* a, uint32_t l
 // 128 bytes and stages, chunk positions and loads are those of g8_mainloop; a lane's operand of the one MFMA step of a k
 // tile is chunks fc and 4 + fc of its row (both operands alike: k is a summation index only). A fragment takes 8 registers,
 // so the weight fragments pass through a ring of half the columns, each refilled as many ahead, and the A fragments are refilled in
-// place behind the last column. The barrier comes after the first column of the second half, the first that makes room for the next tile's. (The lower tiles' four columns with a
-// ring of four, the barrier behind the first and the weights' loads in a lump in front of it: a k tile of 160 rows took as long as one of 256. Ring of four -> of two, us: 380 rows of 17408 x
-// 5120 in tiles of 160 rows 46.5 -> 40.0, 777 in tiles of 224 77.9 -> 71.5, 600 of 5120 x 17408 in tiles of 160 62.0 -> 56.0. 128 x 128, two programs a CU: level, kept at four.)
+// place behind the last column. The barrier comes after the first column of the second half, the first that makes room for the next tile's. (The
+// lower tiles' four columns with a ring of four, the barrier behind the first and the weights' loads in a lump in front of it: a k tile of 160 rows
+// took as long as one of 256. Ring of four -> of two, us: 380 rows of 17408 x 5120 in tiles of 160 rows 46.5 -> 40.0, 777 in tiles of 224 77.9 ->
+// 71.5, 600 of 5120 x 17408 in tiles of 160 62.0 -> 56.0. 128 x 128, two programs a CU: level, kept at four.)
 // a: codes [m][lda] (bytes).
 typedef int g8_i32x8 __attribute__((ext_vector_type(8)));
 template <class T, int NA, int NW, bool ZERO>

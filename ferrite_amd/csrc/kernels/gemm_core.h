@@ -105,6 +105,6 @@ struct GemmSched {
     uint32_t part_bytes;
     uint32_t* counters;
 };
-// A schedule's words as inputs of an empty statement at a kernel's start, with its other arguments: all asked for at once (a launch's arguments come from memory that no
-// cache holds: left where they are first used, three to five trips one behind the other).
+// A schedule's words as inputs of an empty statement at a kernel's start, with its other arguments: all asked for at once (a launch's arguments come
+// from memory that no cache holds: left where they are first used, three to five trips one behind the other).
 #define GEMM_SCHED_WORDS(s) "s"((s).full_tiles), "s"((s).splits), "s"((s).sk_base), "s"((s).sk_rem), "s"((s).part), "s"((s).part_bytes), "s"((s).counters)

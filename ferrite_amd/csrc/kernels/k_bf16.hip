@@ -111,9 +111,9 @@ __device__ __forceinline__ void bf16_swiglu_store4(uint16_t* act, const float (&
     *(u32x2*)(act + (size_t)grow * (n >> 1) + (col >> 4) * 8 + 4 * (l32 & 1)) = o;
 }
 
-// The same for a finished tile, without LDS: the gate sums of a column tile lie in the wavefront's lower half and the up sums in its upper half, so two tiles trade halves, after
-// which every lane has gate and up of 4 features; and two such pairs trade rows of 16 lanes, after which it has 8 features of a row. (Through the slab half of the lanes
-// computed what they did not store: an MLP block of 1000 rows of 5120 / 17408 451 -> 444 us.)
+// The same for a finished tile, without LDS: the gate sums of a column tile lie in the wavefront's lower half and the up sums in its upper half, so
+// two tiles trade halves, after which every lane has gate and up of 4 features; and two such pairs trade rows of 16 lanes, after which it has 8
+// features of a row. (Through the slab half of the lanes computed what they did not store: an MLP block of 1000 rows of 5120 / 17408 451 -> 444 us.)
 template <class T>
 __device__ __forceinline__ void bf16_tile_swiglu(f32x4 (&acc)[T::TM][T::TN], uint16_t* act, uint32_t m, uint32_t n, uint32_t row0, uint32_t col0) {
     static_assert(T::TN % 4 == 0, "two pairs of column tiles");
@@ -187,8 +187,9 @@ extern "C" __global__ __launch_bounds__(256) void fe_interleave_gu(uint16_t* dst
 // lines, which fragments loaded straight into registers (16 rows x 64 bytes) are not, at 42 us instead of 28. The weight loads
 // are non-temporal (31.5 -> 28.3 us at 1 row). x comes from L2 once a program, so wide programs (CO) matter with the rows.
 // 5120 x 17408, us, before -> now: 1 row 26.6 -> 27.1, 4 rows 29.6 -> 27.8, 8 rows 40.6 -> 28.1, 16 rows 80.8 -> 29.2, 40 rows
-// 202 -> 43, 64 rows 321 -> 52 (one or two rows on a few widths 2 to 5 % slower: 5120 x 5120 9.4 -> 9.8); 17408 x 5120: 27.3 -> 27.1, 32.3 -> 27.8, 41.7 -> 29.3, 83.3 -> 33.7, 209 -> 48, 334 -> 57.
-// Distance of the bf16 results from 64-bit sums: 1.66e-3 of their norm, the same to seven digits before and now.
+// 202 -> 43, 64 rows 321 -> 52 (one or two rows on a few widths 2 to 5 % slower: 5120 x 5120 9.4 -> 9.8); 17408 x 5120: 27.3 -> 27.1, 32.3 -> 27.8,
+// 41.7 -> 29.3, 83.3 -> 33.7, 209 -> 48, 334 -> 57. Distance of the bf16 results from 64-bit sums: 1.66e-3 of their norm, the same to seven digits
+// before and now.
 template <int XO, int CO>
 struct Bf16Gemv {
     static constexpr int L = CO + XO, STAGE = L * 1024;  // loads of a step
@@ -198,10 +199,12 @@ struct Bf16Gemv {
     static_assert((DEPTH - 1) * L < 64 && LDS <= 160 * 1024, "stages");
 };
 
-// PAIR: c[r][n] = bf16(bf16(silu(bf16(x . W[n]))) * bf16(x . W2[n])), gate and up of an MLP block at once: a program runs its columns of W, then those of W2, in one chain of
-// steps (the loads run across), and keeps the gate's sums in registers meanwhile. The bits of two GEMVs and fe_silu_mul behind them; res is not read. An MLP block
-// (gate, up, SwiGLU, down) in two launches for four, us: 5120 x 17408 at 1 / 12 / 32 / 64 rows 84 -> 80, 93 -> 88, 117 -> 108, 171 -> 160; 2048 x 5632 19.0 -> 14.9,
-// 21.8 -> 16.5, 27.9 -> 23.0, 39.4 -> 34.0; 1024 x 2816 12.1 -> 7.9, 13.6 -> 9.5, 17.2 -> 13.1, 23.1 -> 18.7. The columns of a program are those of the single linear
+// PAIR: c[r][n] = bf16(bf16(silu(bf16(x . W[n]))) * bf16(x . W2[n])), gate and up of an MLP block at once: a program runs its columns of W, then
+// those of W2, in one chain of steps (the loads run across), and keeps the gate's sums in registers meanwhile. The bits of two GEMVs and fe_silu_mul
+// behind them; res is not read. An MLP block
+// (gate, up, SwiGLU, down) in two launches for four, us: 5120 x 17408 at 1 / 12 / 32 / 64 rows 84 -> 80, 93 -> 88, 117 -> 108, 171 -> 160; 2048 x
+// 5632 19.0 -> 14.9, 21.8 -> 16.5, 27.9 -> 23.0, 39.4 -> 34.0; 1024 x 2816 12.1 -> 7.9, 13.6 -> 9.5, 17.2 -> 13.1, 23.1 -> 18.7. The columns of a
+// program are those of the single linear
 // (gemv_cols): within 2 % of the best width of both launches on six layers at 1 to 64 rows.
 template <int XO, int CO, bool PAIR>
 __device__ __forceinline__ void gemv_bf16_body(uint16_t* c, const uint16_t* a, const uint16_t* w, const uint16_t* w2, const uint16_t* res,

@@ -206,14 +206,15 @@ extern "C" __global__ __launch_bounds__(128) void exl3_rot_in_group(RotGroup g, 
 // by column block and the member's `programs` programs each take one contiguous run of them, base + 1 units for the first
 // rem programs and base for the rest, whatever the shape: with a multiple of the CU count of programs, which the CUs take
 // round by round, the CUs' shares differ by at most one unit. (Spreading the longer runs evenly over the program numbers
-// is worse: their period can divide the CU count, and then a CU gets only long runs or only short ones.) A run may start and end inside a column block, so a block's sum is assembled from segments: each program
-// leaves the partial sums of its segment of block nb in z[program + nb] and bumps the block's arrival counter; the
-// program that arrives last adds the segments, those of programs 2 j and 2 j + 1 to each other first and the pairs in program order
-// (so that gemv_wide_body can run a pair as one workgroup; the order does not depend on who is last: deterministic), applies the output rotation and re-arms the counter. The partition depends on (k, n, programs) only, never on the
-// row count: row r of a batch has the bits of the single-row call. Inside a program: 4 wavefronts owning 2 of the
-// block's 8 tiles each, the rotated inputs of the run staged in LDS (rotated here when src.x is set), four load steps in
-// flight per lane. Several linears of one input share a launch: each member's programs are exactly those of its own
-// launch (same runs, same sums, same bits). (kernels/k-exl3/src/gemv.rs:412-587 is the reference's split-K form.)
+// is worse: their period can divide the CU count, and then a CU gets only long runs or only short ones.) A run may start and end inside a column
+// block, so a block's sum is assembled from segments: each program leaves the partial sums of its segment of block nb in z[program + nb] and bumps
+// the block's arrival counter; the program that arrives last adds the segments, those of programs 2 j and 2 j + 1 to each other first and the pairs
+// in program order
+// (so that gemv_wide_body can run a pair as one workgroup; the order does not depend on who is last: deterministic), applies the output rotation and
+// re-arms the counter. The partition depends on (k, n, programs) only, never on the row count: row r of a batch has the bits of the single-row call.
+// Inside a program: 4 wavefronts owning 2 of the block's 8 tiles each, the rotated inputs of the run staged in LDS (rotated here when src.x is set),
+// four load steps in flight per lane. Several linears of one input share a launch: each member's programs are exactly those of its own launch (same
+// runs, same sums, same bits). (kernels/k-exl3/src/gemv.rs:412-587 is the reference's split-K form.)
 struct GemvMember {
     const uint32_t* trellis;
     const uint16_t *svh, *suh;
@@ -233,8 +234,9 @@ struct GemvJob {
 // A launch's arguments lie in memory that no cache of the XCD holds when the launch begins, so the first scalar load of each of their lines is a trip to
 // memory, and left to itself the compiler loads an argument where it is first used: seven such waits, one behind the other, in front of a program's
 // first weights. As inputs of one empty statement (which needs them in registers) every scalar and a word of every line of the members are asked for at
-// once, and then the program's member whole, out of the cache that now holds it. 0.4 us a launch (nothing in launches of few arguments, the rotations): a decode layer of the 5120 / 17408 model at 1 row 69.7 ->
-// 68.5 us, of 7 rows at 5 bits 97.0 -> 94.4, of 40 rows 113.1 -> 109.2; 1024 / 2816 at 1 row (three launches) 27.9 -> 26.7.
+// once, and then the program's member whole, out of the cache that now holds it. 0.4 us a launch (nothing in launches of few arguments, the
+// rotations): a decode layer of the 5120 / 17408 model at 1 row 69.7 -> 68.5 us, of 7 rows at 5 bits 97.0 -> 94.4, of 40 rows 113.1 -> 109.2; 1024 /
+// 2816 at 1 row (three launches) 27.9 -> 26.7.
 #define GEMV_JOB_LINES(job)                                                                                                              \
     "s"((job).count), "s"((job).first[1]), "s"((job).first[2]), "s"((job).first[3]), "s"((job).first[4]), "s"((job).m[0].n), "s"((job).m[1].n), \
         "s"((job).m[2].trellis), "s"((job).m[2].n), "s"((job).m[3].n)
@@ -414,8 +416,9 @@ __device__ __forceinline__ void gemvb_body(const GemvMember mb, uint32_t p0, uin
     // Rotating here: (row, 128-channel block) pairs of a chunk go to the half wavefronts: half wavefront hw takes blocks hw,
     // hw + 8, ... of every row. The first pair's loads go out ahead of the trellis loads (loads return in order), so
     // that the rotation runs while the first trellis words are still on their way.
-    // (CHAIN: always, and up to 8 rows only, mlp_chain_fits. Code for what never comes is not free: with it the kernel is 47 KB, which with the 23 KB of the GEMV is more than the 64 KB of
-    // instructions that two CUs cache, and a layer's launches displace each other's: 5120 / 17408 at 4 bits, 1 row, two layers 134.6 -> 133.5 us, 1024 / 2816 26.11 -> 25.84.)
+    // (CHAIN: always, and up to 8 rows only, mlp_chain_fits. Code for what never comes is not free: with it the kernel is 47 KB, which with the 23 KB
+    // of the GEMV is more than the 64 KB of instructions that two CUs cache, and a layer's launches displace each other's: 5120 / 17408 at 4 bits, 1
+    // row, two layers 134.6 -> 133.5 us, 1024 / 2816 26.11 -> 25.84.)
     const bool rotating = CHAIN != 0 || src.x != nullptr;
     struct RotAt {
         size_t at, xat;
@@ -836,11 +839,12 @@ GEMVB_FAMILY(8)
 // the column blocks that lie in one run (wide_end). (In gemvb_body's hand-off the
 // program that arrives last at a block reads its segments alone, 12 loads in flight: at 40 rows and 4 bits 10.4 of 22.2 us for q + k + v of the
 // 5120 / 17408 layer, 8.0 of 17.6 for o, 7.6 of 42.8 for gate and up, 14.2 of 34.9 for down; now 13.7 + 4.6, 11.3 + 4.7, 36.4 + 6.1, 21.8 + 5, and the launch
-// behind gate and up leaves down's rotated input as well, which took a launch of 5 us.) A layer at 17 / 40 / 64 rows 107 / 138 / 173 -> 99 / 116 / 140 us. Written through
+// behind gate and up leaves down's rotated input as well, which took a launch of 5 us.) A layer at 17 / 40 / 64 rows 107 / 138 / 173 -> 99 / 116 /
+// 140 us. Written through
 // (a plain store leaves the launch's end to write 14 MB back: 1 to 2 us more). Registers stay under 128, so that four programs share a
-// CU. Bound by the decode and each program's start and end: at 40 rows and 4 bits gate and up issue vector instructions for 20 us, 70 % of the time between the first wavefront and
-// the last, in a launch of 37 (matrix pipe busy in 23 %, LDS bank conflicts 12 % of the cycles). Decoding the next step between the products of this one was measured and changes
-// nothing.
+// CU. Bound by the decode and each program's start and end: at 40 rows and 4 bits gate and up issue vector instructions for 20 us, 70 % of the time
+// between the first wavefront and the last, in a launch of 37 (matrix pipe busy in 23 %, LDS bank conflicts 12 % of the cycles). Decoding the next
+// step between the products of this one was measured and changes nothing.
 template <int BITS, int RG>
 struct GemvWide {
     static constexpr int X_STAGE = RG * 2048, W_STAGE = 1024 * BITS;
@@ -885,10 +889,11 @@ __device__ __forceinline__ void gemv_wide_body(const GemvMember mb, uint32_t p, 
     uint32_t u = run_start(PER * p);
     const uint32_t uend = run_start(PER * p + PER < mb.programs ? PER * p + PER : mb.programs), mid = run_start(PER * p + 1);
     while (u < uend) {
-        // A step's offsets and stages are running scalars: the quotient comes from the vector unit, and left there it takes the loads' offsets, a 32-bit multiply among them,
-        // and the stages along, 133..139 vector instructions a step where the decode takes 119; 123 so. A layer of 5120 / 17408 again and again, 17 / 32 / 40 / 64 rows at 3 bits 88.6 / 92.9 /
-        // 101.5 / 118.3 -> 83.7 / 87.9 / 99.2 / 116.5 us, at 4 bits 87.2 / 91.4 / 101.6 / 120.9 -> 84.8 / 88.7 / 99.8 / 117.4, 9 rows 86.6 -> 84.2; three layers in turn, whose weights
-        // no cache holds: 94.8 / 98.0 / 106.6 / 125.6 -> 90.1 / 93.4 / 104.2 / 124.0, 94.8 / 98.6 / 108.0 / 130.0 -> 93.4 / 96.0 / 106.3 / 125.4, 88.2 -> 86.8.
+        // A step's offsets and stages are running scalars: the quotient comes from the vector unit, and left there it takes the loads' offsets, a
+        // 32-bit multiply among them, and the stages along, 133..139 vector instructions a step where the decode takes 119; 123 so. A layer of 5120 /
+        // 17408 again and again, 17 / 32 / 40 / 64 rows at 3 bits 88.6 / 92.9 / 101.5 / 118.3 -> 83.7 / 87.9 / 99.2 / 116.5 us, at 4 bits 87.2 / 91.4
+        // / 101.6 / 120.9 -> 84.8 / 88.7 / 99.8 / 117.4, 9 rows 86.6 -> 84.2; three layers in turn, whose weights no cache holds: 94.8 / 98.0 / 106.6
+        // / 125.6 -> 90.1 / 93.4 / 104.2 / 124.0, 94.8 / 98.6 / 108.0 / 130.0 -> 93.4 / 96.0 / 106.3 / 125.4, 88.2 -> 86.8.
         const uint32_t nb = __builtin_amdgcn_readfirstlane(u / upb), in = u - nb * upb, units = uend - u < upb - in ? uend - u : upb - in, steps = 2 * units;
         const uint32_t aside = mid > u && mid < u + units ? 2 * (mid - u) : steps;  // the step at which the second program's run starts
         u += units;

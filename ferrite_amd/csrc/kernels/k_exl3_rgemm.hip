@@ -11,13 +11,14 @@
 // front of the loop, where it runs with the matrix pipe idle.
 //
 // What bounds it: with few rows the decode (96 rows: 156 vector instructions a wavefront and step, 24 of them products; a step of the two wavefronts of a SIMD
-// takes 1980 cycles, the matrix pipe busy 38 %), from 160 rows on the board's power: 208 rows of 17408 x 5120 run at 1.76 GHz with the matrix pipe 47 % busy, and
-// 256 programs of whole tiles take the cycles of 130 of them (399 000) and 22 % more time, 1.73 GHz against 2.14. So what counts beside the balance of the
-// programs is to move and multiply little: row tiles as even and as low as the rows
-// need (203 rows: 224, not 256), rows that do not exist read as zeros, tiles whole where possible (the sums of a cut one travel twice), gate
-// and up in one launch. Loads are issued early in a step (at two stages the wait at the next step's start has to find them done: 17408 x
-// 5120, 224 rows 47.5 -> 43.0 us), words a step earlier than A. us, the GEMM that goes through LDS -> this one, 4 bits, with rotation and reduce
-// launches: 5120 x 17408 at 203 / 512 / 2048 rows 65.8 / 112 / 350 -> 60.9 / 107 / 347, 17408 x 5120 69.5 / 110 / 370 -> 55.4 / 105 / 354, 5120 x 1024 at 128 rows 21.1 -> 17.3.
+// takes 1980 cycles, the matrix pipe busy 38 %), from 160 rows on the board's power: 208 rows of 17408 x 5120 run at 1.76 GHz with the matrix pipe 47
+// % busy, and 256 programs of whole tiles take the cycles of 130 of them (399 000) and 22 % more time, 1.73 GHz against 2.14. So what counts beside
+// the balance of the programs is to move and multiply little: row tiles as even and as low as the rows need (203 rows: 224, not 256), rows that do
+// not exist read as zeros, tiles whole where possible (the sums of a cut one travel twice), gate and up in one launch. Loads are issued early in a
+// step (at two stages the wait at the next step's start has to find them done: 17408 x 5120, 224 rows 47.5 -> 43.0 us), words a step earlier than A.
+// us, the GEMM that goes through LDS -> this one, 4 bits, with rotation and reduce
+// launches: 5120 x 17408 at 203 / 512 / 2048 rows 65.8 / 112 / 350 -> 60.9 / 107 / 347, 17408 x 5120 69.5 / 110 / 370 -> 55.4 / 105 / 354, 5120 x
+// 1024 at 128 rows 21.1 -> 17.3.
 #include "exl3_trellis.h"
 #include "gemm8.h"
 
@@ -32,8 +33,8 @@ struct RgMember {
 // The tiles: the members' column tiles, one member after the other, times tiles_m row tiles of BM rows. Programs 0 .. full - 1 take
 // one tile each over all of K. The tiles after them are dealt to `runs` programs: `per` a tile, each a per-th of its steps, or (per 0) the tiles' steps laid
 // end to end in equal runs (base steps, the first rem programs one more). Runs that end inside a tile start the next one's products over, and meet
-// the other programs' inputs at another depth of K: where pieces come out even a tile, 3 % of the time of the best plan (589 linears). A tile that is cut leaves the sums of its pieces, the one of run q in slot
-// q + (tile - full), for the reduce kernel, which adds them in the order of K.
+// the other programs' inputs at another depth of K: where pieces come out even a tile, 3 % of the time of the best plan (589 linears). A tile that is
+// cut leaves the sums of its pieces, the one of run q in slot q + (tile - full), for the reduce kernel, which adds them in the order of K.
 struct RgJob {
     RgMember m[RG_MEMBERS];
     uint32_t count, k, rows, y_mode, tiles_m, tiles_n, group, full, runs, base, rem, per;
@@ -300,8 +301,8 @@ __device__ __forceinline__ void rgemm_body(const RgJob& job) {
     }
 }
 
-// Every line of the launch's arguments asked for at once, in front of the first use of any (as GEMV_JOB_LINES of k_exl3.hip): a trip to memory instead of five, one
-// behind the other.
+// Every line of the launch's arguments asked for at once, in front of the first use of any (as GEMV_JOB_LINES of k_exl3.hip): a trip to memory
+// instead of five, one behind the other.
 #define RG_JOB_LINES(job)                                                                                                                    \
     "s"((job).m[0].first), "s"((job).m[1].first), "s"((job).m[2].first), "s"((job).m[3].first), "s"((job).count), "s"((job).k), "s"((job).rows), \
         "s"((job).y_mode), "s"((job).tiles_m), "s"((job).tiles_n), "s"((job).group), "s"((job).full), "s"((job).runs), "s"((job).base),   \

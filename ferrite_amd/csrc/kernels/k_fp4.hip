@@ -139,8 +139,8 @@ struct Fp4Block {
     u32x4 o[2];
 };
 // Without a NaN among the values: their magnitudes as bf16 bits are in order, so the largest is a maximum of 16-bit integers, and the conversions are the
-// hardware's; a block with a NaN (a magnitude above infinity's) or an infinity, whose product with the multiplier may be one (g of 0, or so small that g / sf is 0), goes
-// through e2m1_nan_to_zero.
+// hardware's; a block with a NaN (a magnitude above infinity's) or an infinity, whose product with the multiplier may be one (g of 0, or so small
+// that g / sf is 0), goes through e2m1_nan_to_zero.
 __device__ __forceinline__ Fp4Block fp4_quant_block(u32x4 r0, u32x4 r1, float g) {
     typedef uint16_t u16x2 __attribute__((ext_vector_type(2)));
     u16x2 top = {0, 0};
@@ -432,12 +432,13 @@ __device__ __forceinline__ void swiglu_quant_store(const float (&v)[4], f32x4 al
     if (j == 0) q_sf[sf_tiled(row, blk, kb)] = (uint8_t)s8;
 }
 
-// The same for a finished tile of the GEMM, without LDS and with every lane at work (through the slab the lanes with up sums computed what they did not store): the gate sums
-// of a column tile lie in the wavefront's lower half and the up sums in its upper half, so the two tiles of a 16-feature block trade halves, after which lane group fc has gate and up
-// of the block's features 4 fc .. + 3; the block's maximum comes from the lanes 16 and 32 away; and two blocks trade rows of 16 lanes, so that a lane stores 8 features of one
+// The same for a finished tile of the GEMM, without LDS and with every lane at work (through the slab the lanes with up sums computed what they did
+// not store): the gate sums of a column tile lie in the wavefront's lower half and the up sums in its upper half, so the two tiles of a 16-feature
+// block trade halves, after which lane group fc has gate and up of the block's features 4 fc .. + 3; the block's maximum comes from the lanes 16 and
+// 32 away; and two blocks trade rows of 16 lanes, so that a lane stores 8 features of one
 // (a tile with one block a wavefront: 4). rows: those that exist from row0 on.
-// Bound by its vector instructions, which no matrix instruction hides (a program has its CU alone): about 10 us a program through the slab, half of that now. Launch, us: 2048
-// rows of 34816 x 5120 558 -> 535, 390 rows 144 -> 132; MLP blocks of 2048 / 5 + 390 rows 865 -> 816, 279 -> 269.
+// Bound by its vector instructions, which no matrix instruction hides (a program has its CU alone): about 10 us a program through the slab, half of
+// that now. Launch, us: 2048 rows of 34816 x 5120 558 -> 535, 390 rows 144 -> 132; MLP blocks of 2048 / 5 + 390 rows 865 -> 816, 279 -> 269.
 template <class T>
 __device__ __forceinline__ void fp4_tile_swiglu(f32x4 (&acc)[T::TM][T::TN], const float* alpha, float scale, uint32_t row0, uint32_t rows, uint32_t colb, uint32_t n, uint8_t* q_codes,
                                                 uint8_t* q_sf, _Float16* q_aq, float qg) {
@@ -518,8 +519,8 @@ struct FpOut {
     float qg;
 };
 
-// The wavefront's rows of a finished tile, from row0, colb (inside n) on: sums times alpha * scale. (The stream-K forms add a residual through the slab: g8_add_bf16's
-// registers, beside what their loop over segments keeps, would cost 30 spilled ones.)
+// The wavefront's rows of a finished tile, from row0, colb (inside n) on: sums times alpha * scale. (The stream-K forms add a residual through the
+// slab: g8_add_bf16's registers, beside what their loop over segments keeps, would cost 30 spilled ones.)
 template <class T, bool SWIGLU, bool SK>
 __device__ __forceinline__ void fp_tile_store(f32x4 (&acc)[T::TM][T::TN], unsigned char* lds, const FpOut& o, const float* alpha, float scale, uint32_t m, uint32_t n,
                                               uint32_t row0, uint32_t colb) {
@@ -567,8 +568,8 @@ __device__ __forceinline__ void fp_tile_store(f32x4 (&acc)[T::TM][T::TN], unsign
         rows(std::false_type{});
 }
 
-// Tiles of 256 x 256, 128 x 256 (S1), 128 x 128 (S2) and 224, 192, 160 x 256 (H7, H6, H5). Packed weights: a wavefront's columns are a quarter of the tile's, so
-// that a weight is expanded by two wavefronts only. The GEMM over FP8 codes expands nothing.
+// Tiles of 256 x 256, 128 x 256 (S1), 128 x 128 (S2) and 224, 192, 160 x 256 (H7, H6, H5). Packed weights: a wavefront's columns are a quarter of the
+// tile's, so that a weight is expanded by two wavefronts only. The GEMM over FP8 codes expands nothing.
 typedef G8Tile<2, 4, 8, 4> FpTile;
 typedef G8Tile<2, 4, 4, 4> FpTileS1;
 typedef G8Tile<2, 4, 4, 2> FpTileS2;
@@ -797,11 +798,12 @@ FP8C_GEMM_KERNEL(_h5, FpTileH5, false)
 
 // ---- FP8 GEMV (few rows): the weights read once, no hand-off -----------------------------------------------------------
 //
-// c[m][ldc] = bf16((codes . W^T) * alpha[n]) (+ res) for m <= 8 XO rows of e4m3 codes [m][k], weights as in fe_gemm_fp8_codes. grid ceil(N / pc), 256 threads: a program takes
-// pc <= 8 CO weight rows (gemv_even) over all of K, its four wavefronts a quarter of K's steps of 128 codes each, DEPTH - 1 steps ahead in LDS stages of their own; a load is 8 rows x 128 bytes,
-// a row's 16-byte chunk c at position c ^ (row & 7). A wavefront adds its products in ascending k, the four sums are added in order: a row's bits depend on K and W only.
-// Bound by the weights' way from HBM up to 16 rows, by the activations' way from L2 as rows and K grow. It replaces the GEMM, whose tiles of 128 rows are mostly empty and whose
-// pieces of K need a reduce launch: kFeGemvFp8 of fe_internal.h has both sides.
+// c[m][ldc] = bf16((codes . W^T) * alpha[n]) (+ res) for m <= 8 XO rows of e4m3 codes [m][k], weights as in fe_gemm_fp8_codes. grid ceil(N / pc), 256
+// threads: a program takes pc <= 8 CO weight rows (gemv_even) over all of K, its four wavefronts a quarter of K's steps of 128 codes each, DEPTH - 1
+// steps ahead in LDS stages of their own; a load is 8 rows x 128 bytes, a row's 16-byte chunk c at position c ^ (row & 7). A wavefront adds its
+// products in ascending k, the four sums are added in order: a row's bits depend on K and W only. Bound by the weights' way from HBM up to 16 rows,
+// by the activations' way from L2 as rows and K grow. It replaces the GEMM, whose tiles of 128 rows are mostly empty and whose pieces of K need a
+// reduce launch: kFeGemvFp8 of fe_internal.h has both sides.
 template <int XO, int CO>
 struct Fp8Gemv {
     static constexpr int L = CO + XO, STAGE = L * 1024;
@@ -818,7 +820,8 @@ __device__ __forceinline__ void gemv_fp8_body(uint16_t* c, const uint8_t* x, con
     const uint32_t tid = threadIdx.x, lane = tid & 63, wave = __builtin_amdgcn_readfirstlane(tid >> 6), r = lane & 15, g = lane >> 4;
     const uint32_t col0 = blockIdx.x * pc, cols = n - col0 < pc ? n - col0 : pc, nt0 = col0 / 128, span = n / 128 - nt0 < 2 ? n / 128 - nt0 : 2;
     const u32x4 wrs = g8_rsrc(w + (size_t)nt0 * w_snt, span * 128 * k), xrs = g8_rsrc(x, m * k);
-    // (columns and rows that do not exist repeat the last one; a step is two of the layout's k tiles: chunks 0..3 of a row from the first, 4..7 from the second)
+    // (columns and rows that do not exist repeat the last one; a step is two of the layout's k tiles: chunks 0..3 of a row from the first, 4..7 from
+    // the second)
     const uint32_t lr = lane >> 3, ch = (lane & 7) ^ lr;
     uint32_t vw[CO], vx[XO];
 #pragma unroll
@@ -944,10 +947,10 @@ struct Fp4GemvStage {
 // lanes hold them); the last to arrive (counters[tile]) adds them in split order, finishes the tile and re-arms the
 // counter, so the result does not depend on timing. A row's sums do not depend on XR. Weight
 // addressing as in fe_gemm_nvfp4.
-// NT: non-temporal loads of the weights. Not of rows as they lie in a checkpoint (_v): a wavefront's piece of such a row is a quarter of its cache line, which the next
-// wavefronts then read again from memory: 34816 x 5120 at 32 rows 131 us with, 102 without; 17408 x 5120 51 -> 39. (Weight tiles: 41.6 with, 42.2 without.)
-// SWIGLU: a fused gate|up linear, whose finished tile goes through LDS to swiglu_quant_store (out), a row a half wavefront. 34816 x 5120 at 17 / 32 / 48 rows 37 / 42 / 51 us
-// against 63 in the GEMM (swiglu_takes_gemv of fe_fp4.cpp).
+// NT: non-temporal loads of the weights. Not of rows as they lie in a checkpoint (_v): a wavefront's piece of such a row is a quarter of its cache
+// line, which the next wavefronts then read again from memory: 34816 x 5120 at 32 rows 131 us with, 102 without; 17408 x 5120 51 -> 39. (Weight
+// tiles: 41.6 with, 42.2 without.) SWIGLU: a fused gate|up linear, whose finished tile goes through LDS to swiglu_quant_store (out), a row a half
+// wavefront. 34816 x 5120 at 17 / 32 / 48 rows 37 / 42 / 51 us against 63 in the GEMM (swiglu_takes_gemv of fe_fp4.cpp).
 template <int XR, bool NT, bool SWIGLU>
 __device__ __forceinline__ void gemv_nvfp4_body(const FpOut out, const _Float16* aq, const uint8_t* w, const uint8_t* sw,
                                                 const float* alpha, float* z, uint32_t* counters,
@@ -1158,21 +1161,21 @@ FP4_GEMV_KERNEL(3, , true) FP4_GEMV_KERNEL(3, _v, false)  // (four groups of row
 
 // ---- GEMV over programs of 8 CO columns (1..16 rows): no hand-off, every operand straight into LDS ---------------------------------
 //
-// y[r][n] for r < m <= 2 XP. grid ceil(N / 8 CO), 64 WV threads: a program takes 8 CO weight rows over all of K, its wavefronts (four or eight: wide_form of fe_fp4.cpp)
-// a quarter or an eighth of K's steps of 256 each (four k tiles). Sums of quarters are added in order; where wide_form sums eighths (EIGHTHS: all forms of such a linear
-// alike), two of them make a quarter. A row's bits depend on W's shape and values and, by wide_form's line, on the device's count of CUs only. K % 256 == 0.
-// Lane L = 16 g + r multiplies, for 16 weight rows, row r's k tile 4 s + g (64 codes, four block scales) with the activations of the
-// same k; the order of k inside a step does not matter.
-// Stages belong to one wavefront (no barrier in the loop). Codes: 8 weight rows a load, [4 k tiles][8 rows][32 bytes]; lanes of
-// odd g read the second half of a row's k tile first, so that 16 lanes that read together cover the 64 banks. Scales: 16 rows a load,
-// [4 k tiles][16 rows][4]. Activations: 2 rows a load, 512 bytes each, chunk c at position c ^ (row & 15) in its half.
+// y[r][n] for r < m <= 2 XP. grid ceil(N / 8 CO), 64 WV threads: a program takes 8 CO weight rows over all of K, its wavefronts (four or eight:
+// wide_form of fe_fp4.cpp) a quarter or an eighth of K's steps of 256 each (four k tiles). Sums of quarters are added in order; where wide_form sums
+// eighths (EIGHTHS: all forms of such a linear alike), two of them make a quarter. A row's bits depend on W's shape and values and, by wide_form's
+// line, on the device's count of CUs only. K % 256 == 0. Lane L = 16 g + r multiplies, for 16 weight rows, row r's k tile 4 s + g (64 codes, four
+// block scales) with the activations of the same k; the order of k inside a step does not matter. Stages belong to one wavefront (no barrier in the
+// loop). Codes: 8 weight rows a load, [4 k tiles][8 rows][32 bytes]; lanes of odd g read the second half of a row's k tile first, so that 16 lanes
+// that read together cover the 64 banks. Scales: 16 rows a load, [4 k tiles][16 rows][4]. Activations: 2 rows a load, 512 bytes each, chunk c at
+// position c ^ (row & 15) in its half.
 //
-// Bound by the codes' way from HBM and the start of a launch at one row, by the activations' way from L2 from 8 rows on. It replaces programs of 16 weight rows with the activations
-// staged whole (one and two rows: too many programs, each waiting for its own staging) and, up to 16 rows, weight tiles cut
-// along K (whose partial sums meet through memory; 17 rows and more still run there). us with the quantizer's launch, before -> now:
-// 5120 x 34816 at 1 / 4 / 8 / 16 rows 25.6 -> 22.1, 32.2 -> 22.1, 32.4 -> 25.7, 34.4 -> 28.8; 17408 x 5120 19.0 -> 14.3, 17.8 -> 14.9,
-// 18.0 -> 18.4, 19.3 -> 20.7; 5120 x 5120 9.6 -> 9.0, 10.3 -> 9.0, 12.2 -> 9.1, 12.5 -> 10.1 (four wavefronts). Eight wavefronts against four: wide_form. Deeper
-// stages in place of more wavefronts lose: 5120 x 17408 at 1 row 17.3 -> 18.8 with eight steps in flight for three.
+// Bound by the codes' way from HBM and the start of a launch at one row, by the activations' way from L2 from 8 rows on. It replaces programs of 16
+// weight rows with the activations staged whole (one and two rows: too many programs, each waiting for its own staging) and, up to 16 rows, weight
+// tiles cut along K (whose partial sums meet through memory; 17 rows and more still run there). us with the quantizer's launch, before -> now: 5120 x
+// 34816 at 1 / 4 / 8 / 16 rows 25.6 -> 22.1, 32.2 -> 22.1, 32.4 -> 25.7, 34.4 -> 28.8; 17408 x 5120 19.0 -> 14.3, 17.8 -> 14.9, 18.0 -> 18.4, 19.3 ->
+// 20.7; 5120 x 5120 9.6 -> 9.0, 10.3 -> 9.0, 12.2 -> 9.1, 12.5 -> 10.1 (four wavefronts). Eight wavefronts against four: wide_form. Deeper stages in
+// place of more wavefronts lose: 5120 x 17408 at 1 row 17.3 -> 18.8 with eight steps in flight for three.
 //
 // Q: the program quantizes the activations itself, in front of its first step. aq is then bf16 rows [m][ldx]: a wavefront moves its quarter of K into LDS as
 // it is, in front of the first weights, makes fe_fp4_quant's values of it in their places (a block of 16 a lane) while the weights are on their way, and every
@@ -1389,8 +1392,9 @@ FP4_WIDE_FIVE(FP4_WIDE_QUANT_KERNEL, 4, _e, 8, true)
 // fe_fp4_peak). KIND 0: v_mfma_f32_32x32x16_f16, 1: v_mfma_f32_32x32x16_bf16, 2: v_mfma_f32_32x32x64_f8f6f4 on e4m3
 // codes (the unscaled form). seed == 0: every operand element is 0.5 or 1 (few bits toggle from one instruction to the
 // next, the reference's kind of pattern); otherwise signs and mantissas are random bits of the seed (an even seed:
-// only the top five mantissa bits of the 16-bit kinds), magnitudes in [0.5, 2), as the operands of a GEMM on real data toggle: the clock the board holds under its power limit depends on
-// it. One float a lane is written so that nothing is dead code. Flops of a launch: wavefronts x iters x 16 x 2 x 32 x 32 x
+// only the top five mantissa bits of the 16-bit kinds), magnitudes in [0.5, 2), as the operands of a GEMM on real data toggle: the clock the board
+// holds under its power limit depends on it. One float a lane is written so that nothing is dead code. Flops of a launch: wavefronts x iters x 16 x 2
+// x 32 x 32 x
 // (16 or 64).
 template <int KIND>
 __device__ __forceinline__ void mfma_peak_body(float* out, uint32_t iters, uint32_t seed) {
