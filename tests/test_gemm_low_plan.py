@@ -54,6 +54,7 @@ TIMED = {
     # and the lower tiles where they are ahead
     ("fp8", 420, 17408, 5120): (5, 0),    # 38.6, 128 rows 46.7
     ("fp8", 250, 34816, 5120): (5, 0),    # a round and 16 tiles cut in seven 66.5, 128 rows 82.8
+    ("fp8", 155, 18944, 8448): (5, 0),    # one row tile, cut in three 45.9, 128 rows 53.5
     ("fp8", 1100, 8192, 2048): (5, 0),    # 21.0, 128 x 128 23.7
     ("fp8", 1300, 17408, 5120): (4, 0),   # 93.4, 128 rows 103.3
     ("fp8", 777, 5120, 17408): (3, 0),    # each cut in three 74.2, 256 rows so 76.4
